@@ -1,0 +1,79 @@
+"""Prompt attention at the edges of its tiles: 32 rows a wave, 32 to 128 rows
+a workgroup, 32 or 64 keys a staged tile, 16 tokens a cache block.
+
+Bound: weights are rounded to bf16 before the second product (2^-9 of the
+weighted sum of |v|, so 2^-9 max|v|), the output once more (2^-9 of itself);
+the rest is fp32. Twice that is allowed."""
+import pytest
+import torch
+
+import kubeai_amd.ops as ops
+from kubeai_amd.ops import ref
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _run(lens, ctxs, nq, nkv, hd, scale, window=0, softcap=0.0, fp8=False, spare_blocks=0):
+    torch.manual_seed(len(lens) * 1000 + sum(lens) + hd)
+    need = [(n + c + 15) // 16 for n, c in zip(lens, ctxs)]
+    nb = sum(need) + 1
+    order = torch.randperm(nb - 1) + 1
+    bt = torch.zeros(len(lens), max(need) + spare_blocks, dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(need):
+        bt[i, :n] = order[at : at + n]
+        at += n
+    kc = torch.randn(nb, nkv, 16, hd, device=DEV, dtype=torch.bfloat16)
+    vc = torch.randn_like(kc)
+    # rows that no query sees must not reach the result
+    for i, (n, c) in enumerate(zip(lens, ctxs)):
+        if (n + c) % 16:
+            kc[bt[i, need[i] - 1], :, (n + c) % 16 :] = float("nan")
+            vc[bt[i, need[i] - 1], :, (n + c) % 16 :] = float("nan")
+    if fp8:
+        kc, vc = kc.to(torch.float8_e5m2), vc.to(torch.float8_e5m2)
+    qkv = torch.randn(sum(lens), (nq + 2) * hd, device=DEV, dtype=torch.bfloat16)
+    q = qkv[:, : nq * hd].unflatten(-1, (nq, hd))  # strided rows, as in the model
+    start = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32, device=DEV)
+    total = torch.tensor([n + c for n, c in zip(lens, ctxs)], dtype=torch.int32, device=DEV)
+    got = ops.paged_attention_prefill(q, kc, vc, bt.to(DEV), start, total, scale,
+                                      window=window, softcap=softcap)
+    want = ref.paged_attention_prefill(q.float(), kc.float(), vc.float(), bt.to(DEV), start,
+                                       total, scale, window=window, softcap=softcap)
+    vmax = torch.nan_to_num(vc.float()).abs().max().item()
+    torch.testing.assert_close(got.float(), want, atol=2 * 2.0 ** -9 * vmax, rtol=2 * 2.0 ** -9)
+
+
+@pytest.mark.parametrize("group", [1, 2, 4, 8])
+@pytest.mark.parametrize("hd", [128, 256])
+def test_row_and_key_remainders(group, hd):
+    _run([1, 31, 32, 33, 65, 127, 128, 129], [0, 1, 32, 63, 64, 65, 15, 200],
+         2 * group, 2, hd, hd ** -0.5)
+
+
+@pytest.mark.parametrize("hd", [128, 256])
+@pytest.mark.parametrize("window", [1, 31, 64, 65])
+@pytest.mark.parametrize("softcap", [0.0, 20.0])
+def test_windows(hd, window, softcap):
+    _run([3, 100, 40], [130, 0, 64], 4, 2, hd, hd ** -0.5, window=window, softcap=softcap)
+
+
+@pytest.mark.parametrize("hd", [128, 256])
+def test_eight_bit_cache(hd):
+    _run([70, 5], [33, 100], 8, 2, hd, hd ** -0.5, fp8=True)
+
+
+def test_softcap_small_and_large_scores():
+    _run([80], [40], 4, 1, 256, 1e-4, softcap=50.0)
+    _run([80], [40], 4, 1, 256, 2.0, softcap=30.0)
+
+
+def test_negative_and_zero_scale():
+    _run([50, 17], [20, 0], 4, 1, 128, -0.05)
+    _run([50, 17], [20, 0], 4, 1, 128, 0.0)
+
+
+def test_wide_block_tables_and_many_short_runs():
+    _run([16] * 70 + [200] + [1] * 30, [0] * 70 + [5] + [40] * 30, 8, 2, 128, 0.09,
+         spare_blocks=40)
