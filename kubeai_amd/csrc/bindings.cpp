@@ -31,6 +31,8 @@ void gumbel_sample(torch::Tensor out, torch::Tensor logits,
                    int64_t step);
 void sgmv(torch::Tensor y, torch::Tensor x, torch::Tensor A, torch::Tensor B,
           torch::Tensor idx, double scale);
+void lora_apply(torch::Tensor y, torch::Tensor x, torch::Tensor table,
+                torch::Tensor ids, int64_t max_rank);
 void register_chwbl(pybind11::module_& m);
 // one-shot fused all-reduce over xGMI (allreduce.hip)
 pybind11::bytes xgmi_alloc();
@@ -89,5 +91,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("xgmi_max_elems", &xgmi_max_elems, "one-shot capacity (bf16 elems)");
   m.def("xgmi_shutdown", &xgmi_shutdown, "free/close comm buffers");
   m.def("sgmv", &sgmv, "segmented gather LoRA apply (one adapter segment)");
+  m.def("lora_apply", &lora_apply,
+        "LoRA apply over a batch of tokens with mixed adapters");
   register_chwbl(m);
 }

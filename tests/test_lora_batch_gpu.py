@@ -1,0 +1,90 @@
+"""The batched LoRA kernels at the edges of their tiles: 16 tokens, 1024
+inputs and 16 ranks a workgroup of the first, 512 outputs of the second.
+
+y is rounded to bf16 once (2^-9 of itself); the sums before are fp32 over at
+most 1100 + 64 terms (1100 * 2^-24 of the sum of magnitudes, far below)."""
+import pytest
+import torch
+
+from kubeai_amd.engine.lora import LoRAManager, _float_word, _two_words
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _apply(T, H, out, ranks, ids, y_pad=0):
+    from kubeai_amd import _C
+
+    torch.manual_seed(T + H + out)
+    x = torch.randn(T, H, device=DEV, dtype=torch.bfloat16)
+    wide = torch.randn(T, out + y_pad, device=DEV, dtype=torch.bfloat16)
+    y = wide[:, :out]
+    sets = {lid: (torch.randn(r, H, device=DEV, dtype=torch.bfloat16) * 0.1,
+                  torch.randn(out, r, device=DEV, dtype=torch.bfloat16), 2.0 / r)
+            for lid, r in ranks.items()}
+    table = torch.tensor([[A.data_ptr(), B.data_ptr(), _two_words(A.shape[0], lid), _float_word(s)]
+                          for lid, (A, B, s) in sets.items()], dtype=torch.int64, device=DEV)
+    want, rest = y.double(), wide[:, out:].clone()
+    for t, lid in enumerate(ids):
+        if lid in sets:
+            A, B, s = sets[lid]
+            want[t] += (B.double() @ (A.double() @ x[t].double())) * s
+    _C.lora_apply(y, x, table, torch.tensor(ids, dtype=torch.int32, device=DEV),
+                  max(ranks.values()))
+    torch.testing.assert_close(y.double(), want, atol=1e-4, rtol=2.0 ** -8)
+    assert torch.equal(wide[:, out:], rest)
+
+
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 50])
+@pytest.mark.parametrize("H,out", [(1024, 512), (1032, 514), (40, 6), (2048, 511)])
+def test_sizes(T, H, out):
+    _apply(T, H, out, {3: 16, 9: 8}, [(0, 3, 9, 5)[t * 7 % 4] for t in range(T)])
+
+
+@pytest.mark.parametrize("rank", [1, 7, 8, 17, 48, 64])
+def test_ranks_beside_each_other(rank):
+    _apply(33, 1024, 520, {1: rank, 2: 16, 3: 3}, [1, 2, 3] * 11)
+
+
+def test_sixteen_adapters_in_a_tile_and_strided_rows():
+    _apply(32, 256, 300, {k + 1: 8 + k % 9 for k in range(16)}, list(range(1, 17)) * 2, y_pad=5)
+    _apply(20, 256, 300, {1: 16}, [0] * 20)
+
+
+class _Cfg:
+    hidden_size, intermediate_size, num_hidden_layers = 128, 256, 2
+    num_attention_heads, num_key_value_heads, head_dim = 2, 1, 64
+    num_local_experts = 0
+
+
+class _Model(torch.nn.Module):
+    cfg = _Cfg()
+
+
+def test_manager_batched_equals_one_by_one():
+    """The table's route against the per-adapter one, and what it leaves to it:
+    ranks above the table's and tensors of another type."""
+    m = LoRAManager(_Model(), DEV, torch.bfloat16)
+    for lid in (4, 7):
+        m.load(lid, None)
+    ids = torch.tensor([4, 0, 7, 7, 4, 1], dtype=torch.int32, device=DEV)
+    assert set(m._tables) == set(m.TARGETS)
+    for target, din, dout in (("qkv", 128, 256), ("o", 128, 128), ("gate_up", 128, 512),
+                              ("down", 256, 128)):
+        x = torch.randn(6, din, device=DEV, dtype=torch.bfloat16)
+        y = torch.randn(6, dout, device=DEV, dtype=torch.bfloat16)
+        one, many = y.clone(), y.clone()
+        m.apply(1, target, x, many, ids)
+        tables, m._tables = m._tables, {}
+        m.apply(1, target, x, one, ids)
+        m._tables = tables
+        torch.testing.assert_close(many, one, atol=1e-4, rtol=2.0 ** -7)
+        assert torch.equal(many[1], y[1]) and torch.equal(many[5], y[5])
+    m.unload(4)
+    y2 = y.clone()
+    m.apply(0, "down", x, y2, ids)
+    assert torch.equal(y2[0], y[0]) and not torch.equal(y2[2], y[2])
+    m.adapters[7]["qkv"][0] = (torch.zeros(65, 128, device=DEV, dtype=torch.bfloat16),
+                               torch.zeros(256, 65, device=DEV, dtype=torch.bfloat16), 1.0)
+    m._build_tables()
+    assert "qkv" not in m._tables and "o" in m._tables
