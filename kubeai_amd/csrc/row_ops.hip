@@ -1,0 +1,284 @@
+// Row kernels of the decoder layers for gfx950: RMSNorm (with the residual
+// add) in bf16 or straight to fp8 (OCP e4m3) with a scale per row, SwiGLU to
+// fp8, and plain fp8 row quantization.
+//
+// Semantics: kubeai_amd/ops/ref.py (fp32 inside, bf16 in). fp8: per row,
+// scale = max|v| / 448, out = v / scale rounded to nearest even — what
+// torch._scaled_mm's rowwise scale_a expects.
+//
+// One workgroup per row, bound by reading and writing the rows. A row stays
+// in registers between the passes over it (sum of squares, maximum, output):
+// the values per thread are a template parameter, since a register array
+// that is indexed by a runtime trip count lives in scratch memory. With many
+// rows 256 threads each hold more of a row; with few rows as many threads as
+// the row has 16-byte units (up to 1024) shorten the chain of loads.
+// Measured, us (runtime trip count, 256 threads -> this):
+//   8192 rows: residual add + norm to fp8, 4096 wide     116 ->  39 (5.9 TB/s)
+//              SwiGLU to fp8, 14336 wide                 229 -> 124 (4.7 TB/s)
+//              quantization, 4096 wide                    61 ->  18
+//   2048 rows: residual add + norm, 4096 wide              25 ->  11
+//   40 rows:   SwiGLU to fp8                               11 ->   5
+//              residual add + norm to fp8                   6 ->   5
+// With few rows what is left is the launch.
+#include <torch/extension.h>
+
+#include <type_traits>
+
+#include "common.h"
+
+namespace {
+
+constexpr int kMaxH = 16384;     // bf16 norms
+constexpr int kMaxHFp8 = 32768;  // fp8 outputs
+
+typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
+
+DEV_INLINE float block_max(float v, float* smem) {
+  const int wave = threadIdx.x / WAVE_SIZE, lane = threadIdx.x % WAVE_SIZE;
+  const int n_waves = blockDim.x / WAVE_SIZE;
+  v = wave_reduce_max(v);
+  if (lane == 0) smem[wave] = v;
+  __syncthreads();
+  float m = 0.f;
+#pragma unroll
+  for (int w = 0; w < 16; ++w)
+    if (w < n_waves) m = fmaxf(m, smem[w]);
+  return m;
+}
+
+// 8 values -> 8 bytes of e4m3, round to nearest even; |v| <= 448 up to
+// rounding, so nothing overflows
+DEV_INLINE u32x2 to_fp8x8(const float* v, float inv_scale) {
+  u32x2 o;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    int w = __builtin_amdgcn_cvt_pk_fp8_f32(v[4 * h] * inv_scale,
+                                            v[4 * h + 1] * inv_scale, 0, false);
+    w = __builtin_amdgcn_cvt_pk_fp8_f32(v[4 * h + 2] * inv_scale,
+                                        v[4 * h + 3] * inv_scale, w, true);
+    o[h] = (uint32_t)w;
+  }
+  return o;
+}
+
+// scale a row held in registers (VPT units of 8 per thread) to fp8
+template <int VPT>
+DEV_INLINE void write_fp8_row(unsigned char* out, float* out_scale, int64_t row,
+                              const float (&vals)[VPT][8], float amax, int H,
+                              float* smem) {
+  const float gmax = fmaxf(block_max(amax, smem), 1e-6f);
+  if (threadIdx.x == 0) out_scale[row] = gmax / 448.0f;
+  const float inv_scale = 448.0f / gmax;
+#pragma unroll
+  for (int k = 0; k < VPT; ++k) {
+    const int i = threadIdx.x + k * blockDim.x;
+    if (i < H / 8)
+      *reinterpret_cast<u32x2*>(out + row * H + i * 8) =
+          to_fp8x8(vals[k], inv_scale);
+  }
+}
+
+// ADD: residual += x, norm of the sum. FP8: fp8 output with a row scale.
+template <bool ADD, bool FP8, int VPT>
+__launch_bounds__(VPT == 8 ? 512 : 1024) __global__ void rmsnorm_kernel(
+    void* __restrict__ out, float* __restrict__ out_scale,
+    const ushort* x,        // [T, H]; may be `out`
+    ushort* __restrict__ residual,
+    const ushort* __restrict__ w, const float eps, const int H) {
+  const int64_t row = blockIdx.x;
+  const int nvec = H / 8;
+  __shared__ float red[2][16];
+  float vals[VPT][8];
+  float ssum = 0.f;
+#pragma unroll
+  for (int k = 0; k < VPT; ++k) {
+    const int i = threadIdx.x + k * blockDim.x;
+    if (i < nvec) {
+      const ushort8 xv = reinterpret_cast<const ushort8*>(x + row * H)[i];
+      if constexpr (ADD) {
+        ushort8* rp = reinterpret_cast<ushort8*>(residual + row * H) + i;
+        const ushort8 rin = *rp;
+        ushort8 rv;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          vals[k][j] = bf16_to_f32(xv[j]) + bf16_to_f32(rin[j]);
+          rv[j] = f32_to_bf16(vals[k][j]);
+        }
+        *rp = rv;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) vals[k][j] = bf16_to_f32(xv[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ssum += vals[k][j] * vals[k][j];
+    }
+  }
+  const float total = block_reduce_sum(ssum, red[0]);
+  const float inv_rms = rsqrtf(total / (float)H + eps);
+  float amax = 0.f;
+#pragma unroll
+  for (int k = 0; k < VPT; ++k) {
+    const int i = threadIdx.x + k * blockDim.x;
+    if (i < nvec) {
+      const ushort8 wv = reinterpret_cast<const ushort8*>(w)[i];
+      if constexpr (FP8) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          vals[k][j] *= inv_rms * bf16_to_f32(wv[j]);
+          amax = fmaxf(amax, fabsf(vals[k][j]));
+        }
+      } else {
+        ushort8 o;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          o[j] = f32_to_bf16(vals[k][j] * inv_rms * bf16_to_f32(wv[j]));
+        reinterpret_cast<ushort8*>((ushort*)out + row * H)[i] = o;
+      }
+    }
+  }
+  if constexpr (FP8)
+    write_fp8_row<VPT>((unsigned char*)out, out_scale, row, vals, amax, H, red[1]);
+}
+
+// SILU: silu(gate) * up of packed [T, 2H] rows, else the rows as they are
+template <bool SILU, int VPT>
+__launch_bounds__(VPT == 8 ? 512 : 1024) __global__ void to_fp8_kernel(
+    unsigned char* __restrict__ out, float* __restrict__ out_scale,
+    const ushort* __restrict__ xin, const int H) {
+  const int64_t row = blockIdx.x;
+  const int nvec = H / 8;
+  const ushort8* xr =
+      reinterpret_cast<const ushort8*>(xin + row * (SILU ? 2 : 1) * H);
+  __shared__ float red[16];
+  float vals[VPT][8];
+  float amax = 0.f;
+#pragma unroll
+  for (int k = 0; k < VPT; ++k) {
+    const int i = threadIdx.x + k * blockDim.x;
+    if (i < nvec) {
+      const ushort8 g = xr[i];
+      if constexpr (SILU) {
+        const ushort8 u = xr[nvec + i];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float gf = bf16_to_f32(g[j]);
+          vals[k][j] = gf / (1.0f + __expf(-gf)) * bf16_to_f32(u[j]);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) vals[k][j] = bf16_to_f32(g[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(vals[k][j]));
+    }
+  }
+  write_fp8_row<VPT>(out, out_scale, row, vals, amax, H, red);
+}
+
+// threads per row and units per thread for T rows of H values
+struct Split {
+  int threads, vpt;
+};
+Split split_for(int64_t T, int H) {
+  const int nvec = H / 8;
+  // from about four rows a CU on the chip is full with 256 threads a row;
+  // longer rows take 512, so that a thread's registers do not limit the waves
+  const int threads = T >= 1024 ? (nvec <= 1024 ? 256 : 512)
+                                : std::min(1024, (nvec + 63) / 64 * 64);
+  return {threads, (nvec + threads - 1) / threads};
+}
+
+// call f with the smallest instantiated number of units; 8 units come with at
+// most 512 threads (32768 values: 8 x 512 or 4 x 1024)
+template <typename F>
+void with_vpt(int vpt, F&& f) {
+  if (vpt <= 1) f(std::integral_constant<int, 1>{});
+  else if (vpt <= 2) f(std::integral_constant<int, 2>{});
+  else if (vpt <= 4) f(std::integral_constant<int, 4>{});
+  else f(std::integral_constant<int, 8>{});
+}
+
+void check_row_op(const torch::Tensor& x, int max_h) {
+  TORCH_CHECK(x.is_contiguous());
+  TORCH_CHECK(x.scalar_type() == torch::kBFloat16);
+  TORCH_CHECK(x.size(-1) % 8 == 0 && x.size(-1) <= max_h);
+}
+
+template <bool ADD, bool FP8>
+void launch_norm(void* out, float* out_scale, const torch::Tensor& x,
+                 ushort* residual, const torch::Tensor& weight, double eps) {
+  const int H = x.size(-1);
+  const int64_t T = x.numel() / H;
+  const Split s = split_for(T, H);
+  with_vpt(s.vpt, [&](auto vpt) {
+    hipLaunchKernelGGL((rmsnorm_kernel<ADD, FP8, decltype(vpt)::value>),
+                       dim3((uint32_t)T), dim3(s.threads), 0,
+                       c10::hip::getCurrentHIPStream().stream(), out, out_scale,
+                       (const ushort*)x.data_ptr(), residual,
+                       (const ushort*)weight.data_ptr(), (float)eps, H);
+  });
+  HIP_CHECK_KERNEL();
+}
+
+template <bool SILU>
+void launch_to_fp8(torch::Tensor& out, torch::Tensor& out_scale,
+                   const torch::Tensor& x, int64_t T, int H) {
+  if (T == 0) return;
+  const Split s = split_for(T, H);
+  with_vpt(s.vpt, [&](auto vpt) {
+    hipLaunchKernelGGL((to_fp8_kernel<SILU, decltype(vpt)::value>),
+                       dim3((uint32_t)T), dim3(s.threads), 0,
+                       c10::hip::getCurrentHIPStream().stream(),
+                       (unsigned char*)out.data_ptr(),
+                       out_scale.data_ptr<float>(),
+                       (const ushort*)x.data_ptr(), H);
+  });
+  HIP_CHECK_KERNEL();
+}
+
+}  // namespace
+
+void rmsnorm(torch::Tensor out, torch::Tensor x, torch::Tensor weight,
+             double eps) {
+  check_row_op(x, kMaxH);
+  TORCH_CHECK(out.is_contiguous());
+  launch_norm<false, false>(out.data_ptr(), nullptr, x, nullptr, weight, eps);
+}
+
+void fused_add_rmsnorm(torch::Tensor x, torch::Tensor residual,
+                       torch::Tensor weight, double eps) {
+  check_row_op(x, kMaxH);
+  TORCH_CHECK(residual.is_contiguous());
+  launch_norm<true, false>(x.data_ptr(), nullptr, x,
+                           (ushort*)residual.data_ptr(), weight, eps);
+}
+
+void rmsnorm_fp8(torch::Tensor out, torch::Tensor out_scale, torch::Tensor x,
+                 torch::Tensor weight, double eps) {
+  check_row_op(x, kMaxHFp8);
+  launch_norm<false, true>(out.data_ptr(), out_scale.data_ptr<float>(), x,
+                           nullptr, weight, eps);
+}
+
+void fused_add_rmsnorm_fp8(torch::Tensor out, torch::Tensor out_scale,
+                           torch::Tensor x, torch::Tensor residual,
+                           torch::Tensor weight, double eps) {
+  check_row_op(x, kMaxHFp8);
+  TORCH_CHECK(residual.is_contiguous());
+  launch_norm<true, true>(out.data_ptr(), out_scale.data_ptr<float>(), x,
+                          (ushort*)residual.data_ptr(), weight, eps);
+}
+
+void silu_and_mul_fp8(torch::Tensor out, torch::Tensor out_scale,
+                      torch::Tensor x) {
+  check_row_op(x, 2 * kMaxHFp8);
+  const int I = x.size(1) / 2;
+  TORCH_CHECK(I % 8 == 0 && I <= kMaxHFp8);
+  launch_to_fp8<true>(out, out_scale, x, x.size(0), I);
+}
+
+void quant_fp8(torch::Tensor out, torch::Tensor out_scale, torch::Tensor x) {
+  check_row_op(x, kMaxHFp8);
+  const int H = x.size(-1);
+  launch_to_fp8<false>(out, out_scale, x, x.numel() / H, H);
+}

@@ -107,27 +107,32 @@ class Attention(nn.Module):
             lm = getattr(self, "_lora_manager", None)
             if lm is not None and lm.active and fb.lora_ids is not None:
                 lm.apply(self.layer_idx, "qkv", x, qkv, fb.lora_ids)
-        q, k, v = qkv.split(
-            [self.n_q * self.hd, self.n_kv * self.hd, self.n_kv * self.hd], dim=-1
-        )
-        # strided views into the qkv buffer — the HIP kernels take a row
-        # stride, so no .contiguous() copies (saves 3 HBM round trips/layer)
-        q = q.unflatten(-1, (self.n_q, self.hd))
-        k = k.unflatten(-1, (self.n_kv, self.hd))
-        v = v.unflatten(-1, (self.n_kv, self.hd))
+        if isinstance(cos_sin, tuple):
+            # (global, local) caches — gemma3 dual rope bases
+            cos_sin = cos_sin[0] if self.is_global else cos_sin[1]
+        k_cache, v_cache = kv_cache
         if self.qk_norm:
             # gemma3: per-head RMSNorm ((1+w) stored as w) before rope;
             # fp32 math, contiguous bf16 out. v follows to contiguous —
             # the cache-write kernel wants k/v with one shared row stride
-            q = _rms_head(q, self.q_norm, self.norm_eps)
-            k = _rms_head(k, self.k_norm, self.norm_eps)
-            v = v.contiguous()
-        if isinstance(cos_sin, tuple):
-            # (global, local) caches — gemma3 dual rope bases
-            cos_sin = cos_sin[0] if self.is_global else cos_sin[1]
-        q, k = ops.rope(q, k, fb.positions, cos_sin)
-        k_cache, v_cache = kv_cache
-        ops.reshape_and_cache(k, v, k_cache, v_cache, fb.slot_mapping)
+            q, k, v = qkv.split(
+                [self.n_q * self.hd, self.n_kv * self.hd, self.n_kv * self.hd],
+                dim=-1,
+            )
+            q = _rms_head(
+                q.unflatten(-1, (self.n_q, self.hd)), self.q_norm, self.norm_eps
+            )
+            k = _rms_head(
+                k.unflatten(-1, (self.n_kv, self.hd)), self.k_norm, self.norm_eps
+            )
+            v = v.unflatten(-1, (self.n_kv, self.hd)).contiguous()
+            q, k = ops.rope(q, k, fb.positions, cos_sin)
+            ops.reshape_and_cache(k, v, k_cache, v_cache, fb.slot_mapping)
+        else:
+            q = ops.rope_and_cache(
+                qkv, self.n_q, fb.positions, cos_sin, k_cache, v_cache,
+                fb.slot_mapping,
+            )
 
         out = torch.empty(
             (T, self.n_q, self.hd), dtype=qkv.dtype, device=qkv.device
@@ -312,7 +317,7 @@ class DecoderLayer(nn.Module):
             and fb.lora_ids is None
         ):
             # fp8 serving: norms/activations emit fp8 + per-row scales
-            # directly (quant_fp8.hip), so activation quantization costs
+            # directly (row_ops.hip), so activation quantization costs
             # nothing extra; residual stays bf16
             if residual is None:
                 residual = x

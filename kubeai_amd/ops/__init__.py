@@ -71,6 +71,32 @@ def reshape_and_cache(k, v, k_cache, v_cache, slot_mapping) -> None:
     ref.reshape_and_cache(k, v, k_cache, v_cache, slot_mapping)
 
 
+def rope_and_cache(qkv, n_q: int, positions, cos_sin, k_cache, v_cache, slot_mapping):
+    """q | k | v rows of the fused projection: q is rotated (in place on GPU) and
+    returned as [T, n_q, hd], k is rotated and written to the paged cache with
+    v. One launch on GPU where heads split into 16-byte units."""
+    n_kv, hd = k_cache.shape[1], k_cache.shape[3]
+    q, k, v = qkv.split([n_q * hd, n_kv * hd, n_kv * hd], dim=-1)
+    q = q.unflatten(-1, (n_q, hd))
+    if (
+        qkv.is_cuda
+        and hd % 16 == 0
+        and qkv.dtype == torch.bfloat16
+        and qkv.stride(1) == 1
+        and qkv.stride(0) % 8 == 0
+        and qkv.data_ptr() % 16 == 0
+        and k_cache.dtype in (torch.bfloat16, torch.float8_e5m2)
+        and v_cache.dtype == k_cache.dtype
+        and v_cache.shape == k_cache.shape
+    ):
+        _require_ext()
+        _C.rope_cache(qkv, positions, cos_sin, k_cache, v_cache, slot_mapping, n_q)
+        return q
+    q, k = rope(q, k.unflatten(-1, (n_kv, hd)), positions, cos_sin)
+    reshape_and_cache(k, v.unflatten(-1, (n_kv, hd)), k_cache, v_cache, slot_mapping)
+    return q
+
+
 def paged_attention_decode(
     q, k_cache, v_cache, block_tables, seq_lens, scale: float, out=None,
     window: int = 0, softcap: float = 0.0,

@@ -1,0 +1,98 @@
+"""Row kernels at the edges of their splits (256, 512 and up to 1024 threads
+a row, 1 to 8 units of 8 values a thread, rows below and above 1024) and the
+fused rotation and cache write against the two-kernel route.
+
+Bounds: bf16 outputs are rounded once (2^-9 of themselves; the norm's fp32
+sum adds below 1e-5). fp8 outputs: a value may land on the neighbouring
+eight-bit number where the fp32 quotient differs in its last bits, 2^-3 of
+itself, in less than one value in 500; the scale is fp32."""
+import pytest
+import torch
+
+import kubeai_amd.ops as ops
+from kubeai_amd.ops import ref
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+WIDTHS = [8, 504, 512, 2048, 4096, 4104, 8192, 16384]
+
+
+def _x(T, H):
+    torch.manual_seed(T * 7 + H)
+    return torch.randn(T, H, device=DEV, dtype=torch.bfloat16)
+
+
+def _close_fp8(q, s, want):
+    """q * s against want [T, H] fp32."""
+    amax = want.abs().amax(-1).clamp_min(1e-6)
+    torch.testing.assert_close(s, amax / 448.0, atol=0, rtol=1e-5)
+    exact = (want / (amax / 448.0)[:, None]).to(torch.float8_e4m3fn).float()
+    off = q.float() != exact
+    assert off.float().mean().item() < 2e-3
+    torch.testing.assert_close(q.float(), exact, atol=2.0 ** -9, rtol=2.0 ** -3 + 1e-6)
+
+
+@pytest.mark.parametrize("H", WIDTHS)
+@pytest.mark.parametrize("T", [1, 3, 1023, 1024])
+def test_norms(T, H):
+    x, r = _x(T, H), _x(T + 1, H)[1:].contiguous()
+    w = torch.randn(H, device=DEV, dtype=torch.bfloat16)
+    want = ref.rmsnorm(x.float(), w.float(), 1e-5)
+    torch.testing.assert_close(ops.rmsnorm(x, w, 1e-5).float(), want, atol=1e-5, rtol=2.0 ** -8)
+    _close_fp8(*ops.rmsnorm_fp8(x, w, 1e-5), want)
+    want, total = ref.fused_add_rmsnorm(x.float(), r.float(), w.float(), 1e-5)
+    r2 = r.clone()
+    _close_fp8(*ops.fused_add_rmsnorm_fp8(x, r2, w, 1e-5), want)
+    assert torch.equal(r2, total.bfloat16())
+    got, r3 = ops.fused_add_rmsnorm(x.clone(), r.clone(), w, 1e-5)
+    torch.testing.assert_close(got.float(), want, atol=1e-5, rtol=2.0 ** -8)
+    assert torch.equal(r3, r2)
+
+
+@pytest.mark.parametrize("H", WIDTHS + [14336, 28672, 32768])
+@pytest.mark.parametrize("T", [1, 1024])
+def test_to_fp8(T, H):
+    x = _x(T, H)
+    _close_fp8(*ops.quant_fp8(x), x.float())
+    gu = _x(T, 2 * H)
+    g, u = gu.float().chunk(2, -1)
+    q, s = ops.silu_and_mul_fp8(gu)
+    # __expf: 2 ulp around 1 + e^-g
+    _close_fp8(q, s, torch.nn.functional.silu(g) * u)
+
+
+def test_zero_and_huge_rows():
+    x = torch.zeros(4, 512, device=DEV, dtype=torch.bfloat16)
+    x[1] = 3e38
+    x[2, 5] = 1e-30
+    q, s = ops.quant_fp8(x)
+    assert (q[0].float() == 0).all() and (q[1].float() == 448).all()
+    torch.testing.assert_close(s[:1], torch.full((1,), 1e-6 / 448, device=DEV))
+
+
+@pytest.mark.parametrize("nq,nkv,hd", [(32, 8, 128), (3, 1, 16), (8, 4, 256), (5, 5, 80)])
+@pytest.mark.parametrize("cache", [torch.bfloat16, torch.float8_e5m2])
+@pytest.mark.parametrize("pad", [0, 8])
+def test_rope_and_cache_equals_two_kernels(nq, nkv, hd, cache, pad):
+    T, width = 21, (nq + 2 * nkv) * hd
+    qkv = _x(T, width + pad)[:, :width]
+    pos = torch.randint(0, 900, (T,), device=DEV, dtype=torch.int32)
+    slots = torch.randperm(5 * 16, device=DEV)[:T]
+    slots[3] = -1
+    cs = ref.make_cos_sin_cache(hd, 1000).to(DEV)
+    one = [torch.zeros(5, nkv, 16, hd, device=DEV).to(cache) for _ in range(2)]
+    two = [c.clone() for c in one]
+    other = qkv.clone()
+    q = ops.rope_and_cache(qkv, nq, pos, cs, *one, slots)
+    q2, k2, v2 = other.split([nq * hd, nkv * hd, nkv * hd], -1)
+    q2, k2 = ops.rope(q2.unflatten(-1, (nq, hd)), k2.unflatten(-1, (nkv, hd)), pos, cs)
+    ops.reshape_and_cache(k2, v2.unflatten(-1, (nkv, hd)), *two, slots)
+    # the compiler may contract x1 c - x2 s either way: the fp32 values differ in
+    # their last bit and fall to different sides of a rounding tie about once in
+    # 2^15 values (bf16); then by one step of the result's type
+    step = 2.0 ** -7 if cache == torch.bfloat16 else 2.0 ** -2
+    for a, b, rtol in [(q, q2, 2.0 ** -7)] + [(a, b, step) for a, b in zip(one, two)]:
+        a, b = a.float(), b.float()
+        assert (a != b).sum().item() <= 2 + a.numel() // 1000
+        torch.testing.assert_close(a, b, atol=1e-6, rtol=rtol)
+    assert torch.equal(one[1].view(torch.uint8), two[1].view(torch.uint8))
