@@ -2,21 +2,37 @@
 //
 // Semantics: kubeai_amd/ops/ref.py::paged_attention_decode.
 //
-// Design (MI355X-first, memory-bound regime — see guide Appendix B):
-//  - workgroup = (seq, kv_head); 4 waves; GQA group of G = n_q/n_kv query
-//    heads computed together so each KV byte is read from HBM exactly once.
-//  - waves process DISJOINT cache blocks (flash-decoding split): wave w takes
-//    blocks w, w+4, ... with per-wave online-softmax state, merged at the end
-//    through LDS (m*, l*, o* combine). This keeps the chip busy at small
-//    decode batches (B*n_kv*4 waves in flight).
-//  - each wave stages its 16-token KV tile into its own LDS buffer with
-//    ushort8 (16 B) vector loads (rows padded 16 B for bank spread).
-//  - scoring is token-parallel: 4 lanes per token, each covering a 32-elem
-//    head_dim slice, 2-step part reduction — one pass scores the whole tile
-//    (v1's 16 serial 64-lane butterflies were the VALU bottleneck).
-//  - tile-level online softmax with defer-max (rescale only when the
-//    running max grows); PV accumulates per-lane head_dim pairs with the
-//    per-token p reaching lanes via one __shfl broadcast.
+// Structure:
+//  - workgroup = (sequence, kv head, split of the keys); 4 waves take tiles of
+//    NB cache blocks in turn (32 keys at head size 128, 16 at 256), each with
+//    its own softmax state; the G query heads of the group share every key.
+//  - S^T = K.Q^T on v_mfma_f32_16x16x32_bf16: a lane reads 16 bytes of one
+//    key straight into the operand (16 keys x 64 contiguous bytes per load,
+//    no LDS), the query heads are columns (lane & 15; those past G repeat the
+//    last head). Scores of 4 keys per block lie in the lane, a maximum is two
+//    lane swaps, the sum stays per lane until the end.
+//  - O^T += V^T.P^T: the score registers are the second product's operand as
+//    they stand. V needs its keys along a lane: it goes through a
+//    wave-private LDS tile (row-major, 16-byte units XOR-swizzled, no
+//    barriers) and comes back through ds_read_b64_tr_b16.
+//  - the weights keep their 24 bits: they are split into three bf16 parts
+//    (each the rounded rest of the one before) that are multiplied one after
+//    the other into the same fp32 sum.
+//  - the next tile's K and V are in flight while this one is computed (two
+//    register sets).
+// Bound by reading the cache. The form before this (scores and weighted sum
+// on the vector ALUs) issued about 150 LDS operations per 16 keys, most of
+// them the lane permutes that passed a weight to every lane; here it is 12.
+// Measured, kernel + merge of the splits, us (before -> this):
+//   heads 32/8 x 128, 40 rows of 100-700 keys         41 ->  23
+//   96 rows of 1500-4000                             364 -> 228 (5.0 TB/s)
+//   64 rows of 1536                                  137 ->  80 (5.1 TB/s)
+//     the same, e5m2 cache                           128 ->  51
+//   8 rows of 3584                                    48 ->  31
+//   1 row of 3000 and 7 idle ones                     32 ->  14
+//   heads 64/8 x 128, 32 rows of 1000-3000           165 ->  60
+//   heads 8/4 x 256, cap, 40 rows of 300-900          55 ->  45
+// At head size 256 a tile is one block (two would need 512 registers).
 #include <torch/extension.h>
 
 #include <type_traits>
@@ -25,29 +41,33 @@
 
 namespace {
 
-constexpr int kWaves = 2;  // 2 waves/workgroup: fits double-buffered tiles
+constexpr int kWaves = 4;
 constexpr int kBlockThreads = kWaves * WAVE_SIZE;
-constexpr int kBS = 16;   // cache block size (tokens)
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2v;  // v_dot2 operand
-// +8 ushorts (16 B) row padding: keeps 16 B staging alignment and breaks
-// the power-of-two row stride so the (token, part) score reads spread
-// over banks (4-way residual aliasing ~= 1.6x on the LDS op, vs 32-way
-// unpadded)
-constexpr int kPad = 8;
+constexpr int kBS = 16;      // cache block size (tokens)
+constexpr int kMaxSplits = 16;
+constexpr int kMaxG = 8;
+
+typedef __attribute__((ext_vector_type(8))) short bf16x8;
+typedef __attribute__((ext_vector_type(4))) short bf16x4;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+
+// combine a value over the four 16-lane groups that hold the same column
+template <typename F>
+DEV_INLINE float over_groups(float v, F&& f) {
+  const auto a = __builtin_amdgcn_permlane32_swap(
+      __float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane16_swap(
+      __float_as_uint(v), __float_as_uint(v), false, false);
+  return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
 
 // CT = cache element type: ushort (bf16) or unsigned char (fp8 e5m2,
-// converted to bf16 in-register while staging — same LDS layout/compute)
-// HD = head dim: 128 (llama family) or 256 (gemma2). A lane always
-// covers a 32-element slice, so HD sets PARTS = HD/32 lanes per token
-// and TOKP = 64/PARTS tokens scored per pass (two passes per 16-token
-// tile at HD=256).
-// SOFTCAP > 0 applies gemma2-style attention-logit soft capping,
-// s = cap * tanh(s / cap), after scaling and before masking.
-// CAP: compile-time softcap enable — a runtime branch in the score
-// loop measured -13% on the capless hot path (194.6 vs 169.0 us at
-// B=64 L=2048), so capped models get their own instantiation.
-template <int G, typename CT = ushort, int HD = 128, bool CAP = false>
-__launch_bounds__(kBlockThreads) __global__ void paged_decode_kernel(
+// converted to bf16 on the way in, exactly). CAP: s = cap * tanh(s / cap)
+// after scaling and before masking.
+template <int HD, typename CT, bool CAP>
+__launch_bounds__(kBlockThreads, 2) __global__ void paged_decode_kernel(
     ushort* __restrict__ out,            // [B, n_q, hd] bf16
     const ushort* __restrict__ q,        // [B, n_q, hd] bf16
     const CT* __restrict__ k_cache,      // [nb, n_kv, bs, hd]
@@ -55,329 +75,285 @@ __launch_bounds__(kBlockThreads) __global__ void paged_decode_kernel(
     const int32_t* __restrict__ block_tables,  // [B, max_blocks]
     const int32_t* __restrict__ seq_lens,      // [B]
     const float scale, const float softcap, const int window,
-    const int n_kv, const int max_blocks,
+    const int n_kv, const int G, const int max_blocks,
     const int64_t q_stride, const int n_splits,
     float* __restrict__ part_o,    // [B, n_q, n_splits, hd]
     float* __restrict__ part_ml) { // [B, n_q, n_splits, 2]
+  constexpr int NB = HD == 128 ? 2 : 1;  // cache blocks per tile
+  constexpr int NC = HD / 32;            // contraction steps of S
+  constexpr int ND = HD / 16;            // row blocks of O^T
+  constexpr int NV = HD / 32;            // 16-byte V units per lane and block
   const int b = blockIdx.x / (n_kv * n_splits);
   const int rem = blockIdx.x % (n_kv * n_splits);
   const int kh = rem / n_splits;
   const int split = rem % n_splits;
   const int n_q = n_kv * G;
-  const int wave = threadIdx.x / WAVE_SIZE;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
   const int lane = threadIdx.x % WAVE_SIZE;
+  const int col = lane & 15, grp = lane >> 4;
   const int L = seq_lens[b];
   const int n_blocks = (L + kBS - 1) / kBS;
   // sliding window: the query (position L-1) attends keys in
-  // (L-1-window, L-1] -> global positions >= w0; whole blocks below w0
-  // are skipped, the straddling block is masked per token
+  // (L-1-window, L-1]; splits divide the visible blocks only
   const int w0 = (window > 0) ? max(0, L - window) : 0;
-  // flash-decoding splits divide the WINDOWED block range — splitting
-  // the full range would leave every split below w0 empty for long
-  // sequences (mistral at L >> window would use a fraction of the
-  // launched workgroups)
   const int blk_base = w0 / kBS;
-  const int n_eff = n_blocks - blk_base;
-  const int chunk = (n_eff + n_splits - 1) / n_splits;
-  const int blk_lo = blk_base + split * chunk;
-  const int blk_hi = min(n_blocks, blk_lo + chunk);
+  const int n_units = (n_blocks - blk_base + NB - 1) / NB;  // tiles
+  const int chunk = (n_units + n_splits - 1) / n_splits;
+  const int t_lo = split * chunk;
+  const int t_hi = min(n_units, t_lo + chunk);
 
-  // LDS: per-wave double-buffered KV tiles + merge scratch. Element type
-  // follows the cache: bf16 stages bf16; fp8 stages the RAW e5m2 bytes
-  // (half the LDS footprint/traffic) and converts during compute with the
-  // native packed bf8->f32 instruction (v_cvt_pk_f32_bf8). 8-element row
-  // pad keeps 8 B staging alignment and breaks bank aliasing for both
-  // element widths (bf16: 68-dword stride, gcd 4; fp8: 34-dword, gcd 2).
-  constexpr int PARTS = HD / 32;    // lanes per token in scoring
-  constexpr int TOKP = 64 / PARTS;  // tokens scored per pass
-  constexpr int EPL = HD / 64;      // output elems owned per lane
-  __shared__ CT k_lds[kWaves][2][kBS][HD + kPad];
-  __shared__ CT v_lds[kWaves][2][kBS][HD + kPad];
-  __shared__ float merge_o[kWaves][G][HD];
-  __shared__ float merge_ml[kWaves][G][2];
+  constexpr int kVTile = NB * kBS * HD;  // elements of a wave's V tile
+  constexpr size_t kSmem = sizeof(ushort) * kWaves * kVTile >
+                                   sizeof(float) * kWaves * kMaxG * HD
+                               ? sizeof(ushort) * kWaves * kVTile
+                               : sizeof(float) * kWaves * kMaxG * HD;
+  __shared__ __attribute__((aligned(16))) char smem[kSmem];
+  __shared__ float merge_ml[kWaves][kMaxG][2];
+  char* vt = smem + wave * kVTile * 2;
 
-  // --- lane roles -----------------------------------------------------
-  // scoring: PARTS lanes per token, each covering a 32-elem slice of
-  //   head_dim — TOKP tile tokens score in parallel with a log2(PARTS)-
-  //   step part reduction (replaces v1's serial 64-lane butterflies)
-  // PV/output: lane owns head_dim elems [EPL*lane, EPL*lane+EPL);
-  //   per-token p reaches every lane via one __shfl broadcast
-  const int tok_of = lane / PARTS;
-  const int part = lane % PARTS;
-
-  // q slice for this lane's part, packed bf16 pairs (16 u32 per head)
-  uint32_t q_pack[G][16];
+  bf16x8 q_frag[NC];
+  {
+    const ushort* qp = q + (int64_t)b * q_stride +
+                       (int64_t)(kh * G + min(col, G - 1)) * HD + grp * 8;
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-    const uint32_t* qp = reinterpret_cast<const uint32_t*>(
-        q + (int64_t)b * q_stride + (int64_t)(kh * G + g) * HD + part * 32);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) q_pack[g][i] = qp[i];
+    for (int c = 0; c < NC; ++c)
+      q_frag[c] = *reinterpret_cast<const bf16x8*>(qp + c * 32);
   }
+  const float c2 = CAP ? scale : scale * kLog2e;
+  const float inv_cap = CAP ? 1.0f / softcap : 0.f;
 
-  float m[G], l[G], o[G][EPL];
+  f32x4 o_acc[ND];
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-    m[g] = -INFINITY;
-    l[g] = 0.f;
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) o[g][e] = 0.f;
-  }
+  for (int d = 0; d < ND; ++d) o_acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;  // l_run: this lane's keys
 
   const int32_t* bt = block_tables + (int64_t)b * max_blocks;
-
-  // T14 async-stage: global loads for block n+1 issue before block n's
-  // compute (their latency hides under it); the register payload lands in
-  // the other LDS buffer just before it is needed. Per-wave buffers ->
-  // no barriers anywhere in the loop.
-  // staging vector = 8 elements: 16 B (bf16) or 8 B (raw fp8 bytes)
-  using StageVec = std::conditional_t<sizeof(CT) == 2, ushort8, uint64_t>;
-  constexpr int NS = (kBS * HD / 8) / WAVE_SIZE;
-  StageVec stage_k[NS], stage_v[NS];  // this lane's vectors of each tile
-
-  auto issue_loads = [&](int blk_i) {
-    const int64_t blk = bt[blk_i];
-    const CT* base_k = k_cache + ((blk * n_kv + kh) * kBS) * HD;
-    const CT* base_v = v_cache + ((blk * n_kv + kh) * kBS) * HD;
-    const StageVec* src_k = reinterpret_cast<const StageVec*>(base_k);
-    const StageVec* src_v = reinterpret_cast<const StageVec*>(base_v);
-#pragma unroll
-    for (int i = 0; i < NS; ++i) {
-      stage_k[i] = src_k[lane + i * WAVE_SIZE];
-      stage_v[i] = src_v[lane + i * WAVE_SIZE];
-    }
+  using Unit = std::conditional_t<sizeof(CT) == 2, bf16x8, uint64_t>;
+  Unit kf[2][NB][NC], vf[2][NB][NV];
+  auto to_bf16 = [](const Unit& u) -> bf16x8 {
+    if constexpr (sizeof(CT) == 2) return u;
+    else return __builtin_bit_cast(bf16x8, e5m2x8_to_bf16x8(u));
   };
-  auto write_tile = [&](int buf) {
+  auto load_tile = [&](int set, int t) {
 #pragma unroll
-    for (int i = 0; i < NS; ++i) {
-      const int vec = lane + i * WAVE_SIZE;  // 8-element vector index
-      const int row = vec / (HD / 8);
-      const int col = vec % (HD / 8);
-      *reinterpret_cast<StageVec*>(&k_lds[wave][buf][row][col * 8]) =
-          stage_k[i];
-      *reinterpret_cast<StageVec*>(&v_lds[wave][buf][row][col * 8]) =
-          stage_v[i];
+    for (int j = 0; j < NB; ++j) {
+      const int64_t blk = bt[min(blk_base + t * NB + j, n_blocks - 1)];
+      const int64_t base = (blk * n_kv + kh) * (kBS * HD);
+      const CT* kp = k_cache + base + col * HD + grp * 8;
+      const CT* vp = v_cache + base + lane * 8;
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        kf[set][j][c] = *reinterpret_cast<const Unit*>(kp + c * 32);
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        vf[set][j][i] =
+            *reinterpret_cast<const Unit*>(vp + i * WAVE_SIZE * 8);
     }
   };
 
-  const int first = blk_lo + wave;
-  int cur = 0;
-  if (first < blk_hi) {
-    issue_loads(first);
-    write_tile(0);
-  }
+  // LDS offsets of the transposing reads: keys 4 grp + (lane >> 2 & 3) of a
+  // block, columns 16 d + 4 (lane & 3); units of rows r are XORed with
+  // 2 (r & 3), which spreads the four rows of a 16-lane read over the banks
+  const int tr_row = 4 * grp + ((lane >> 2) & 3);
+  const int tr_x = ((lane >> 2) & 3) << 1;
+  const int tr_u = (lane & 3) >> 1;  // unit within the 32 bytes
+  const char* tr_base = vt + tr_row * HD * 2 + (lane & 1) * 8;
 
-  for (int blk_i = first; blk_i < blk_hi; blk_i += kWaves) {
-    const int tile_start = blk_i * kBS;
-    const int tile_len = min(kBS, L - tile_start);
-    if (blk_i + kWaves < blk_hi) issue_loads(blk_i + kWaves);
-
-    // TOKP tokens score per pass; kBS/TOKP passes cover the tile (one
-    // pass at HD=128, two at HD=256)
+  auto compute = [&](int set, int t) {
+    const int tok0 = (blk_base + t * NB) * kBS;
+    const bool whole = tok0 >= w0 && tok0 + NB * kBS <= L;
+    // ---- V to LDS ------------------------------------------------------
 #pragma unroll
-    for (int tp = 0; tp < kBS; tp += TOKP) {
-      const int tok = tp + tok_of;
-      // ---- scores: lane computes its (token, part-slice) partial ------
-      float s[G];
+    for (int j = 0; j < NB; ++j)
 #pragma unroll
-      for (int g = 0; g < G; ++g) s[g] = 0.f;
-      if constexpr (sizeof(CT) == 2) {
-        // v_dot2c_f32_bf16: one instruction per bf16 pair-dot-accumulate
-        // (replaces 2 unpacks + 2 fma per (g, j) — a 3x VALU cut in the
-        // score phase)
-        const uint32_t* krow = reinterpret_cast<const uint32_t*>(
-            &k_lds[wave][cur][tok][part * 32]);
+      for (int i = 0; i < NV; ++i) {
+        const int e = lane + i * WAVE_SIZE;  // 16-byte unit of the block
+        const int row = e / (HD / 8), un = e % (HD / 8);
+        bf16x8 v = to_bf16(vf[set][j][i]);
+        // rows past the end: their weight is 0, but 0 * stale NaN is not
+        if (!whole && tok0 + j * kBS + row >= L) v = bf16x8{};
+        *reinterpret_cast<bf16x8*>(
+            vt + (j * kBS + row) * HD * 2 + ((un ^ ((row & 3) << 1)) << 4)) = v;
+      }
+    // ---- scores ----------------------------------------------------------
+    f32x4 s[NB];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const bf16x2v kk = __builtin_bit_cast(bf16x2v, krow[j]);
+    for (int j = 0; j < NB; ++j) {
+      s[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int g = 0; g < G; ++g)
-            s[g] = __builtin_amdgcn_fdot2_f32_bf16(
-                kk, __builtin_bit_cast(bf16x2v, q_pack[g][j]), s[g], false);
+      for (int c = 0; c < NC; ++c)
+        s[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            to_bf16(kf[set][j][c]), q_frag[c], s[j], 0, 0, 0);
+    }
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float x = s[j][i] * c2;
+        if constexpr (CAP) x = soft_cap(x, softcap, inv_cap) * kLog2e;
+        const int tok = tok0 + j * kBS + grp * 4 + i;
+        if (!whole && (tok >= L || tok < w0)) x = -INFINITY;
+        s[j][i] = x;
+        tmax = fmaxf(tmax, x);
+      }
+    tmax = over_groups(tmax, [](float a, float c) { return fmaxf(a, c); });
+    // the maximum may lag by 2^11 before everything is rescaled
+    if (!__all(tmax <= m_run + 11.0f)) {
+      const float m_new = fmaxf(m_run, tmax);
+      const float corr =
+          __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.f : m_new));
+      l_run *= corr;
+#pragma unroll
+      for (int d = 0; d < ND; ++d) o_acc[d] *= corr;
+      m_run = m_new;
+    }
+    const float m_use = (m_run == -INFINITY) ? 0.f : m_run;
+    // ---- weights, in three bf16 parts --------------------------------------
+    short p_part[3][NB * 4];
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float p = __builtin_amdgcn_exp2f(s[j][i] - m_use);
+        l_run += p;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const __bf16 r = (__bf16)p;
+          p_part[k][j * 4 + i] = __builtin_bit_cast(short, r);
+          p -= (float)r;
+        }
+      }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // ---- O^T += V^T . P^T ------------------------------------------------
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+      const char* a = tr_base + (((2 * d + tr_u) ^ tr_x) << 4);
+      const bf16x4 v0 =
+          __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4*)(a));
+      if constexpr (NB == 2) {
+        const bf16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_bf16x4*)(a + kBS * HD * 2));
+        const bf16x8 v =
+            __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          bf16x8 p;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) p[i] = p_part[k][i];
+          o_acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, p, o_acc[d],
+                                                             0, 0, 0);
         }
       } else {
-        // raw e5m2 slice: each uint32 holds 4 bytes -> 4 elements; the
-        // packed bf8->f32 convert does 2 per instruction
-        const uint32_t* krow = reinterpret_cast<const uint32_t*>(
-            &k_lds[wave][cur][tok][part * 32]);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const uint32_t kk = krow[j];
-          const floatx2 k01 = __builtin_amdgcn_cvt_pk_f32_bf8(kk, false);
-          const floatx2 k23 = __builtin_amdgcn_cvt_pk_f32_bf8(kk, true);
+        for (int k = 0; k < 3; ++k) {
+          bf16x4 p;
 #pragma unroll
-          for (int g = 0; g < G; ++g) {
-            const uint32_t qa = q_pack[g][2 * j];
-            const uint32_t qb = q_pack[g][2 * j + 1];
-            s[g] = fmaf(k01.x, bf16_to_f32((ushort)(qa & 0xffff)), s[g]);
-            s[g] = fmaf(k01.y, bf16_to_f32((ushort)(qa >> 16)), s[g]);
-            s[g] = fmaf(k23.x, bf16_to_f32((ushort)(qb & 0xffff)), s[g]);
-            s[g] = fmaf(k23.y, bf16_to_f32((ushort)(qb >> 16)), s[g]);
-          }
-        }
-      }
-      float p[G];
-      float rsum[G];
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        // reduce across the part-slices -> full dot in all PARTS lanes
-#pragma unroll
-        for (int off = 1; off < PARTS; off <<= 1)
-          s[g] += __shfl_xor(s[g], off, 64);
-        s[g] = (tok < tile_len && tile_start + tok >= w0) ? s[g] * scale
-                                                          : -INFINITY;
-        if constexpr (CAP) {
-          if (s[g] != -INFINITY) s[g] = softcap * tanhf(s[g] / softcap);
-        }
-        // pass max across tokens (lane bits above the part bits)
-        float tmax = s[g];
-#pragma unroll
-        for (int off = PARTS; off < 64; off <<= 1)
-          tmax = fmaxf(tmax, __shfl_xor(tmax, off, 64));
-        const float m_new = fmaxf(m[g], tmax);
-        if (m_new != m[g]) {  // defer-max: wave-uniform rescale on growth
-          const float corr = __expf(m[g] - m_new);
-          l[g] *= corr;
-#pragma unroll
-          for (int e = 0; e < EPL; ++e) o[g][e] *= corr;
-          m[g] = m_new;
-        }
-        p[g] = (s[g] == -INFINITY) ? 0.f : __expf(s[g] - m_new);
-        rsum[g] = p[g];
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1)
-          rsum[g] += __shfl_xor(rsum[g], off, 64);
-        l[g] += rsum[g] * (1.0f / PARTS);  // each token counted PARTS x
-      }
-
-      // ---- PV: lane accumulates its EPL output elems ------------------
-#pragma unroll
-      for (int t = tp; t < tp + TOKP; ++t) {
-        if (t >= tile_len) break;
-        float vv[EPL];
-        if constexpr (sizeof(CT) == 2) {
-#pragma unroll
-          for (int e = 0; e < EPL; e += 2) {
-            const uint32_t vr = *reinterpret_cast<const uint32_t*>(
-                &v_lds[wave][cur][t][EPL * lane + e]);
-            vv[e] = bf16_to_f32((ushort)(vr & 0xffff));
-            vv[e + 1] = bf16_to_f32((ushort)(vr >> 16));
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < EPL; e += 2) {
-            const uint32_t vr = *reinterpret_cast<const ushort*>(
-                &v_lds[wave][cur][t][EPL * lane + e]);
-            const floatx2 vf = __builtin_amdgcn_cvt_pk_f32_bf8(vr, false);
-            vv[e] = vf.x;
-            vv[e + 1] = vf.y;
-          }
-        }
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-          const float pt = __shfl(p[g], (t - tp) * PARTS, 64);
-#pragma unroll
-          for (int e = 0; e < EPL; ++e)
-            o[g][e] = fmaf(pt, vv[e], o[g][e]);
+          for (int i = 0; i < 4; ++i) p[i] = p_part[k][i];
+          o_acc[d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v0, p, o_acc[d],
+                                                               0, 0, 0);
         }
       }
     }
+    // the next tile's V is stored after these reads (LDS operations of a
+    // wave run in order)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
 
-    // land the prefetched tile in the other buffer (waits only on vmcnt)
-    if (blk_i + kWaves < blk_hi) write_tile(cur ^ 1);
-    cur ^= 1;
+  const int first = t_lo + wave;
+  if (first < t_hi) load_tile(0, first);
+  for (int t = first; t < t_hi; t += 2 * kWaves) {
+    if (t + kWaves < t_hi) load_tile(1, t + kWaves);
+    compute(0, t);
+    if (t + kWaves < t_hi) {
+      if (t + 2 * kWaves < t_hi) load_tile(0, t + 2 * kWaves);
+      compute(1, t + kWaves);
+    }
   }
 
-  // cross-wave merge through LDS
+  // ---- merge the waves -----------------------------------------------------
+  l_run = over_groups(l_run, [](float a, float c) { return a + c; });
+  __syncthreads();  // the V tiles are free
+  float* merge_o = reinterpret_cast<float*>(smem);  // [wave][G][HD]
+  if (col < G) {
+    float* mo = merge_o + (wave * G + col) * HD + grp * 4;
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) merge_o[wave][g][EPL * lane + e] = o[g][e];
-    if (lane == 0) {
-      merge_ml[wave][g][0] = m[g];
-      merge_ml[wave][g][1] = l[g];
+    for (int d = 0; d < ND; ++d)
+      *reinterpret_cast<f32x4*>(mo + d * 16) = o_acc[d];
+    if (grp == 0) {
+      merge_ml[wave][col][0] = m_run;
+      merge_ml[wave][col][1] = l_run;
     }
   }
   __syncthreads();
-
-  // wave w finalizes heads g = w, w+2, ... (for G<2, wave 1 idles here)
-  for (int g = wave; g < G; g += kWaves) {
+  for (int i = threadIdx.x; i < G * (HD / 4); i += kBlockThreads) {
+    const int g = i / (HD / 4), e = i % (HD / 4) * 4;
     float m_star = -INFINITY;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) m_star = fmaxf(m_star, merge_ml[w][g][0]);
-    float l_star = 0.f, oo[EPL];
+    const float m_use = (m_star == -INFINITY) ? 0.f : m_star;
+    float l_star = 0.f;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) oo[e] = 0.f;
-    if (m_star != -INFINITY) {
-#pragma unroll
-      for (int w = 0; w < kWaves; ++w) {
-        const float c = __expf(merge_ml[w][g][0] - m_star);
-        l_star += merge_ml[w][g][1] * c;
-#pragma unroll
-        for (int e = 0; e < EPL; ++e)
-          oo[e] += merge_o[w][g][EPL * lane + e] * c;
-      }
+    for (int w = 0; w < kWaves; ++w) {
+      const float c = __builtin_amdgcn_exp2f(merge_ml[w][g][0] - m_use);
+      l_star += merge_ml[w][g][1] * c;
+      o += *reinterpret_cast<const f32x4*>(merge_o + (w * G + g) * HD + e) * c;
     }
-    const int head = kh * G + g;
+    const int64_t head = (int64_t)b * n_q + kh * G + g;
     if (n_splits == 1) {
       const float inv_l = 1.0f / l_star;
-      ushort* oh = out + ((int64_t)b * n_q + head) * HD;
+      ushort4_t r;
 #pragma unroll
-      for (int e = 0; e < EPL; e += 2) {
-        uint32_t packed =
-            ((uint32_t)f32_to_bf16(oo[e + 1] * inv_l) << 16) |
-            f32_to_bf16(oo[e] * inv_l);
-        *reinterpret_cast<uint32_t*>(&oh[EPL * lane + e]) = packed;
-      }
+      for (int k = 0; k < 4; ++k) r[k] = f32_to_bf16(o[k] * inv_l);
+      *reinterpret_cast<ushort4_t*>(out + head * HD + e) = r;
     } else {
-      // flash-decoding partials (empty splits write m=-inf, l=0, o=0)
-      float* po = part_o + (((int64_t)b * n_q + head) * n_splits + split) * HD;
-#pragma unroll
-      for (int e = 0; e < EPL; ++e) po[EPL * lane + e] = oo[e];
-      if (lane == 0) {
-        float* pm = part_ml + (((int64_t)b * n_q + head) * n_splits + split) * 2;
-        pm[0] = m_star;
-        pm[1] = l_star;
+      // partial results (an empty split writes m = -inf, l = 0, o = 0)
+      *reinterpret_cast<f32x4*>(part_o + (head * n_splits + split) * HD + e) = o;
+      if (e == 0) {
+        part_ml[(head * n_splits + split) * 2] = m_star;
+        part_ml[(head * n_splits + split) * 2 + 1] = l_star;
       }
     }
   }
 }
 
-// Merge flash-decoding partials: one wave per (seq, q_head).
-template <int HD = 128>
+// Merge the splits' results: one wave per (sequence, query head). The lanes
+// read all splits' (m, l) at once and the rows of O are independent loads.
+template <int HD>
 __global__ void decode_merge_kernel(
     ushort* __restrict__ out,             // [B, n_q, hd]
     const float* __restrict__ part_o,     // [B, n_q, n_splits, hd]
     const float* __restrict__ part_ml,    // [B, n_q, n_splits, 2]
-    const int n_q, const int n_splits, const int64_t n_bh) {
+    const int n_splits, const int64_t n_bh) {
   constexpr int EPL = HD / 64;
+  typedef __attribute__((ext_vector_type(EPL))) float vec;
   const int64_t bh = (int64_t)blockIdx.x * (blockDim.x / WAVE_SIZE) +
                      threadIdx.x / WAVE_SIZE;
   if (bh >= n_bh) return;
   const int lane = threadIdx.x % WAVE_SIZE;
   const float* pml = part_ml + bh * n_splits * 2;
-  const float* po = part_o + bh * n_splits * HD;
-  float m_star = -INFINITY;
-  for (int s = 0; s < n_splits; ++s) m_star = fmaxf(m_star, pml[2 * s]);
-  float l_star = 0.f, oo[EPL];
+  const vec* po = reinterpret_cast<const vec*>(part_o + bh * n_splits * HD) + lane;
+  const int s = min(lane, n_splits - 1);
+  const float ms = pml[2 * s], ls = lane < n_splits ? pml[2 * s + 1] : 0.f;
+  const float m_star = wave_reduce_max(ms);
+  const float c = __builtin_amdgcn_exp2f(ms - (m_star == -INFINITY ? 0.f : m_star));
+  const float l_star = wave_reduce_sum(ls * c);
+  vec o;
 #pragma unroll
-  for (int e = 0; e < EPL; ++e) oo[e] = 0.f;
-  for (int s = 0; s < n_splits; ++s) {
-    const float ms = pml[2 * s];
-    if (ms == -INFINITY) continue;
-    const float c = __expf(ms - m_star);
-    l_star += pml[2 * s + 1] * c;
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) oo[e] += po[s * HD + EPL * lane + e] * c;
-  }
+  for (int e = 0; e < EPL; ++e) o[e] = 0.f;
+#pragma unroll 4
+  for (int k = 0; k < n_splits; ++k)
+    o += po[k * 64] * __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(c), k));
   const float inv_l = 1.0f / l_star;
-  ushort* oh = out + bh * HD;
+  ushort* oh = out + bh * HD + EPL * lane;
 #pragma unroll
-  for (int e = 0; e < EPL; e += 2) {
-    uint32_t packed = ((uint32_t)f32_to_bf16(oo[e + 1] * inv_l) << 16) |
-                      f32_to_bf16(oo[e] * inv_l);
-    *reinterpret_cast<uint32_t*>(&oh[EPL * lane + e]) = packed;
-  }
+  for (int e = 0; e < EPL; e += 2)
+    *reinterpret_cast<uint32_t*>(oh + e) =
+        ((uint32_t)f32_to_bf16(o[e + 1] * inv_l) << 16) |
+        f32_to_bf16(o[e] * inv_l);
 }
 
 }  // namespace
@@ -403,33 +379,20 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
   const int G = n_q / n_kv;
   TORCH_CHECK(n_q % n_kv == 0);
   if (B == 0) return;
-  // flash-decoding split: target 2048 workgroups, cap 16. Fixed-shape
-  // microbenches (scripts/sweep_decode_splits.py) mildly favor 4096, but
-  // the live bench's length mix loses ~4.5% end-to-end at 4096 (extra
-  // fp32 partial traffic + merge work inside graph replay) — same-box
-  // A/B in profiles/r01_results.md. KUBEAI_DECODE_SPLIT_TARGET overrides
-  // for tuning sweeps.
+  TORCH_CHECK(G == 1 || G == 2 || G == 4 || G == 5 || G == 6 || G == 8,
+              "unsupported GQA group size ", G);
+  // The keys are split until 512 workgroups (two a CU) are there; the lengths
+  // are not known here, and more splits cost in the merge: 40 rows of 100-700
+  // keys, 8 kv heads 23.0 us at 512, 25.6 at 1536; one row of 3000 among 7 idle
+  // ones 13.6 at 512, 17.0 at 1536, 16.7 at 256. KUBEAI_DECODE_SPLIT_TARGET overrides for tuning sweeps.
   static const int split_target = []() {
     const char* e = getenv("KUBEAI_DECODE_SPLIT_TARGET");
-    const int v = e ? atoi(e) : 2048;
-    return v > 0 ? v : 2048;
+    const int v = e ? atoi(e) : 512;
+    return v > 0 ? v : 512;
   }();
-  // optional length-aware bound: >=N cache blocks per split, so short
-  // sequences don't launch mostly-empty splits (max_blocks is the widest
-  // block table this step — host-side, no device sync)
-  static const int min_blocks_per_split = []() {
-    const char* e = getenv("KUBEAI_DECODE_MIN_BLOCKS_PER_SPLIT");
-    return e ? atoi(e) : 0;
-  }();
-  int n_splits = 1;
-  const int base_wgs = B * n_kv;
-  if (base_wgs < split_target) {
-    n_splits = std::min<int>(16, (split_target + base_wgs - 1) / base_wgs);
-    if (min_blocks_per_split > 0) {
-      const int cap = std::max(1, max_blocks / min_blocks_per_split);
-      n_splits = std::min(n_splits, cap);
-    }
-  }
+  const int64_t base_wgs = (int64_t)B * n_kv;
+  const int n_splits = (int)std::max<int64_t>(
+      1, std::min<int64_t>(kMaxSplits, (split_target + base_wgs - 1) / base_wgs));
   torch::Tensor part_o, part_ml;
   float *part_o_ptr = nullptr, *part_ml_ptr = nullptr;
   if (n_splits > 1) {
@@ -440,68 +403,42 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
     part_o_ptr = part_o.data_ptr<float>();
     part_ml_ptr = part_ml.data_ptr<float>();
   }
-  dim3 grid(B * n_kv * n_splits), block(kBlockThreads);
+  const dim3 grid((uint32_t)(base_wgs * n_splits)), block(kBlockThreads);
   auto stream = c10::hip::getCurrentHIPStream().stream();
-  const bool fp8_cache = k_cache.scalar_type() == torch::kFloat8_e5m2;
-#define LAUNCH_CT_HD(GG, CT, HDV)                                         \
-  do {                                                                    \
-    if (softcap > 0.0)                                                    \
-      LAUNCH_IMPL(GG, CT, HDV, true);                                     \
-    else                                                                  \
-      LAUNCH_IMPL(GG, CT, HDV, false);                                    \
-  } while (0)
-#define LAUNCH_IMPL(GG, CT, HDV, CAPV)                                    \
-  hipLaunchKernelGGL((paged_decode_kernel<GG, CT, HDV, CAPV>), grid,      \
-                     block, 0,                                            \
-                     stream, (ushort*)out.data_ptr(),                     \
-                     (const ushort*)q.data_ptr(),                         \
-                     (const CT*)k_cache.data_ptr(),                       \
-                     (const CT*)v_cache.data_ptr(),                       \
-                     block_tables.data_ptr<int32_t>(),                    \
-                     seq_lens.data_ptr<int32_t>(), (float)scale,          \
-                     (float)softcap, (int)window, n_kv,                   \
-                     max_blocks, q.stride(0), n_splits, part_o_ptr,       \
-                     part_ml_ptr)
-#define LAUNCH(GG)                                                        \
-  do {                                                                    \
-    if (hd == 256) {                                                      \
-      /* gemma2 shapes: G <= 2 in practice, fp8 cache supported */        \
-      if (fp8_cache) LAUNCH_CT_HD(GG, unsigned char, 256);                \
-      else LAUNCH_CT_HD(GG, ushort, 256);                                 \
-    } else if (fp8_cache) {                                               \
-      LAUNCH_CT_HD(GG, unsigned char, 128);                               \
-    } else {                                                              \
-      LAUNCH_CT_HD(GG, ushort, 128);                                      \
-    }                                                                     \
-  } while (0)
-  switch (G) {
-    case 1: LAUNCH(1); break;
-    case 2: LAUNCH(2); break;
-    case 4: LAUNCH(4); break;
-    case 5: LAUNCH(5); break;
-    case 6: LAUNCH(6); break;
-    case 8: LAUNCH(8); break;
-    default: TORCH_CHECK(false, "unsupported GQA group size ", G);
-  }
-#undef LAUNCH
-#undef LAUNCH_CT_HD
-#undef LAUNCH_IMPL
+  auto launch = [&](auto hdv, auto ct, auto cap) {
+    using CT = decltype(ct);
+    hipLaunchKernelGGL(
+        (paged_decode_kernel<decltype(hdv)::value, CT, decltype(cap)::value>),
+        grid, block, 0, stream, (ushort*)out.data_ptr(),
+        (const ushort*)q.data_ptr(), (const CT*)k_cache.data_ptr(),
+        (const CT*)v_cache.data_ptr(), block_tables.data_ptr<int32_t>(),
+        seq_lens.data_ptr<int32_t>(), (float)scale, (float)softcap,
+        (int)window, n_kv, G, max_blocks, q.stride(0), n_splits, part_o_ptr,
+        part_ml_ptr);
+  };
+  auto with_cap = [&](auto hdv, auto ct) {
+    if (softcap > 0.0) launch(hdv, ct, std::true_type{});
+    else launch(hdv, ct, std::false_type{});
+  };
+  auto with_hd = [&](auto ct) {
+    if (hd == 256) with_cap(std::integral_constant<int, 256>{}, ct);
+    else with_cap(std::integral_constant<int, 128>{}, ct);
+  };
+  if (k_cache.scalar_type() == torch::kFloat8_e5m2) with_hd((unsigned char)0);
+  else with_hd((ushort)0);
   HIP_CHECK_KERNEL();
   if (n_splits > 1) {
     const int64_t n_bh = (int64_t)B * n_q;
     const int wpb = 4;
+    const dim3 mgrid((uint32_t)((n_bh + wpb - 1) / wpb)), mblock(wpb * WAVE_SIZE);
     if (hd == 256)
-      hipLaunchKernelGGL((decode_merge_kernel<256>),
-                         dim3((uint32_t)((n_bh + wpb - 1) / wpb)),
-                         dim3(wpb * WAVE_SIZE), 0, stream,
+      hipLaunchKernelGGL((decode_merge_kernel<256>), mgrid, mblock, 0, stream,
                          (ushort*)out.data_ptr(), part_o_ptr, part_ml_ptr,
-                         n_q, n_splits, n_bh);
+                         n_splits, n_bh);
     else
-      hipLaunchKernelGGL((decode_merge_kernel<128>),
-                         dim3((uint32_t)((n_bh + wpb - 1) / wpb)),
-                         dim3(wpb * WAVE_SIZE), 0, stream,
+      hipLaunchKernelGGL((decode_merge_kernel<128>), mgrid, mblock, 0, stream,
                          (ushort*)out.data_ptr(), part_o_ptr, part_ml_ptr,
-                         n_q, n_splits, n_bh);
+                         n_splits, n_bh);
     HIP_CHECK_KERNEL();
   }
 }

@@ -63,7 +63,6 @@ namespace {
 constexpr int kBS = 16;  // cache block size (tokens)
 constexpr int kQB = 32;  // query rows per wave
 constexpr int kNW = 4;   // waves per workgroup
-constexpr float kLog2e = 1.4426950408889634f;
 
 typedef __attribute__((ext_vector_type(8))) short bf16x8;
 typedef __attribute__((ext_vector_type(4))) short bf16x4;
@@ -72,19 +71,6 @@ typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
-
-// cap * tanh(x / cap): odd polynomial near zero (the quotient below would
-// cancel), 1 - 2 / (1 + e^2y) elsewhere; within 2e-7 of tanhf
-DEV_INLINE float soft_cap(float x, float cap, float inv_cap) {
-  const float y = x * inv_cap;
-  const float y2 = y * y;
-  const float small =
-      y * fmaf(y2, fmaf(y2, fmaf(y2, -0.05396825397f, 0.13333333333f),
-                        -0.33333333333f), 1.0f);
-  const float e = __builtin_amdgcn_exp2f(fminf(y, 20.f) * (2.f * kLog2e));
-  const float big = 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + e);
-  return cap * (fabsf(y) < 0.2f ? small : big);
-}
 
 // run s of the packed stream owns the tile numbers from start[s] / size + s
 // on (never fewer than it needs): T / size + n_seq numbers cover every batch

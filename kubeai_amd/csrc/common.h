@@ -110,6 +110,21 @@ DEV_INLINE unsigned char f32_to_e5m2(float x) {
   return (unsigned char)__hip_cvt_float_to_fp8(x, __HIP_SATFINITE, __HIP_E5M2);
 }
 
+constexpr float kLog2e = 1.4426950408889634f;
+
+// cap * tanh(x / cap): odd polynomial near zero (the quotient below would
+// cancel), 1 - 2 / (1 + e^2y) elsewhere; within 2e-7 of tanhf
+DEV_INLINE float soft_cap(float x, float cap, float inv_cap) {
+  const float y = x * inv_cap;
+  const float y2 = y * y;
+  const float small =
+      y * fmaf(y2, fmaf(y2, fmaf(y2, -0.05396825397f, 0.13333333333f),
+                        -0.33333333333f), 1.0f);
+  const float e = __builtin_amdgcn_exp2f(fminf(y, 20.f) * (2.f * kLog2e));
+  const float big = 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + e);
+  return cap * (fabsf(y) < 0.2f ? small : big);
+}
+
 // ---------------- wave reductions (64-wide) ----------------
 
 DEV_INLINE float wave_reduce_sum(float v) {

@@ -3,7 +3,7 @@
 The split target is read once per process (static), so run this script
 once per value:
 
-    for t in 512 1024 2048 4096 8192; do
+    for t in 192 256 512 1024 2048; do
         KUBEAI_DECODE_SPLIT_TARGET=$t python scripts/sweep_decode_splits.py
     done
 
@@ -25,7 +25,7 @@ sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
 from bench_ops import timeit  # noqa: E402
 
 dev = "cuda"
-target = os.environ.get("KUBEAI_DECODE_SPLIT_TARGET", "2048")
+target = os.environ.get("KUBEAI_DECODE_SPLIT_TARGET", "512")
 print(f"== split target {target} ==", flush=True)
 torch.manual_seed(0)
 for B, L in ((40, 1536), (8, 8192), (256, 2048)):

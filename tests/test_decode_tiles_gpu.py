@@ -1,0 +1,74 @@
+"""Decode attention at the edges of its tiles (16-key blocks, tiles of 32 keys
+at head size 128, 4 waves, splits) and of its group sizes.
+
+The weights keep fp32 accuracy, so the bound is the output's own rounding to
+bf16 (2^-9 of itself) plus fp32 sums and exponentials (1e-5 of max|v| ~ 5);
+twice that is allowed."""
+import pytest
+import torch
+
+import kubeai_amd.ops as ops
+from kubeai_amd.ops import ref
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _run(lens, nq, nkv, hd, scale, window=0, softcap=0.0, fp8=False, spare=0):
+    torch.manual_seed(sum(lens) + nq * hd)
+    need = [(n + 15) // 16 for n in lens]
+    nb = sum(need) + 1
+    order = torch.randperm(nb - 1) + 1
+    bt = torch.zeros(len(lens), max(need) + spare, dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(need):
+        bt[i, :n] = order[at : at + n]
+        at += n
+    kc = torch.randn(nb, nkv, 16, hd, device=DEV, dtype=torch.bfloat16)
+    vc = torch.randn_like(kc)
+    for i, n in enumerate(lens):  # rows behind the last key hold anything
+        if n % 16:
+            kc[bt[i, need[i] - 1], :, n % 16 :] = float("nan")
+            vc[bt[i, need[i] - 1], :, n % 16 :] = float("nan")
+    if fp8:
+        kc, vc = kc.to(torch.float8_e5m2), vc.to(torch.float8_e5m2)
+    q = torch.randn(len(lens), nq + 2, hd, device=DEV, dtype=torch.bfloat16)[:, :nq]
+    total = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    got = ops.paged_attention_decode(q, kc, vc, bt.to(DEV), total, scale, window=window,
+                                     softcap=softcap)
+    want = ref.paged_attention_decode(q.float(), kc.float(), vc.float(), bt.to(DEV), total,
+                                      scale, window=window, softcap=softcap)
+    torch.testing.assert_close(got.float(), want, atol=1e-4, rtol=2.0 ** -8)
+
+
+EDGES = [1, 15, 16, 17, 31, 32, 33, 64, 127, 128, 129, 161, 700, 2049]
+
+
+@pytest.mark.parametrize("group", [1, 2, 4, 5, 6, 8])
+@pytest.mark.parametrize("hd", [128, 256])
+def test_lengths_and_groups(group, hd):
+    _run(EDGES, 2 * group, 2, hd, hd ** -0.5)
+
+
+@pytest.mark.parametrize("rows", [1, 3, 600])
+def test_one_split_and_many(rows):
+    # 600 rows of one kv head are not split, one row is split sixteen times
+    _run([5 + 37 * i % 300 for i in range(rows)], 4, 1, 128, 0.09, spare=50)
+
+
+@pytest.mark.parametrize("hd", [128, 256])
+@pytest.mark.parametrize("window", [1, 16, 31, 33, 500])
+@pytest.mark.parametrize("softcap", [0.0, 20.0])
+def test_windows(hd, window, softcap):
+    _run(EDGES, 4, 2, hd, hd ** -0.5, window=window, softcap=softcap)
+
+
+@pytest.mark.parametrize("hd", [128, 256])
+def test_eight_bit_cache(hd):
+    _run(EDGES, 8, 2, hd, hd ** -0.5, fp8=True)
+
+
+def test_peaked_flat_and_negative_scales():
+    _run(EDGES, 8, 2, 128, 3.0)
+    _run(EDGES, 8, 2, 128, 0.0)
+    _run(EDGES, 8, 2, 128, -0.2)
