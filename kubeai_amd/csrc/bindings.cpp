@@ -28,6 +28,19 @@ void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
                              int64_t window, double softcap);
 void silu_and_mul(torch::Tensor out, torch::Tensor x);
 void gelu_and_mul(torch::Tensor out, torch::Tensor x);
+void skinny_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
+                   c10::optional<torch::Tensor> sx,
+                   c10::optional<torch::Tensor> sw,
+                   c10::optional<torch::Tensor> bias);
+void skinny_experts(torch::Tensor y, torch::Tensor x, torch::Tensor w,
+                    c10::optional<torch::Tensor> sx,
+                    c10::optional<torch::Tensor> sw, torch::Tensor begin,
+                    c10::optional<torch::Tensor> src);
+void moe_route(torch::Tensor index, torch::Tensor weight, torch::Tensor begin,
+               torch::Tensor src, torch::Tensor place, torch::Tensor x,
+               torch::Tensor w);
+void moe_combine(torch::Tensor out, torch::Tensor y, torch::Tensor place,
+                 torch::Tensor weight);
 void skinny_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w);
 void greedy_sample(torch::Tensor out, torch::Tensor logits);
 void gumbel_sample(torch::Tensor out, torch::Tensor logits,
@@ -78,7 +91,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "paged causal flash attention over cached KV");
   m.def("gelu_and_mul", &gelu_and_mul, "GeGLU tanh-gelu(gate)*up");
   m.def("silu_and_mul", &silu_and_mul, "SwiGLU activation");
-  m.def("skinny_gemm", &skinny_gemm, "weight-streaming GEMM for M<=64");
+  m.def("skinny_gemm", &skinny_gemm, "weight-streaming product, bf16");
+  m.def("skinny_experts", &skinny_experts,
+        "weight-streaming product of each expert's rows");
+  m.def("moe_route", &moe_route,
+        "router scores, top-k weights and tokens in expert order");
+  m.def("moe_combine", &moe_combine, "weighted sum of the experts' rows");
+  m.def("skinny_linear", &skinny_linear,
+        "weight-streaming product of up to 96 rows, bf16 or scaled fp8");
   m.def("greedy_sample", &greedy_sample, "argmax sampling");
   m.def("gumbel_sample", &gumbel_sample, "temperature sampling (hash RNG)");
   m.def("rmsnorm_fp8", &rmsnorm_fp8, "rmsnorm with fused fp8 row quant");

@@ -112,4 +112,6 @@ def convert_to_fp8(model: nn.Module) -> int:
             # MoE: attention runs the fused-fp8 path; the MLP input stays
             # bf16 (router needs it) and MoEMLP quantizes once itself
             layer._fp8_fused = True
+            if hasattr(mlp, "stack_experts"):
+                mlp.stack_experts()
     return n

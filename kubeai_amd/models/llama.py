@@ -208,9 +208,19 @@ class MLP(nn.Module):
 class MoEMLP(nn.Module):
     """Mixtral-style sparse MoE block (token-level top-k routing).
 
-    Expert GEMMs are grouped per expert (sort tokens by expert) so each
-    expert runs one hipBLASLt GEMM over its token group.
-    """
+    On GPU, steps of up to GROUPED_MAX_TOKENS tokens route on the device
+    (csrc/moe.hip) and run all experts' rows in one weight-streaming product
+    per projection (csrc/skinny_gemm.hip): shapes do not depend on the routing,
+    so decode steps can be recorded in a graph, and every expert's weights are
+    read once, for its own rows only. The experts' weights lie behind one
+    another in one tensor for that; the modules' parameters are views of it.
+    Larger steps gather each expert's rows and run its library GEMMs."""
+
+    #: one pass of 8 experts of 14336 (us, grouped / every expert through the
+    #: library): fp8 1 token 137/540, 40 297/542, 256 450/764, 512 831/1274;
+    #: bf16 40 561/822, 512 1403/1537, 768 1810/1699 (an expert's weights are
+    #: read again for every 96 of its rows)
+    GROUPED_MAX_TOKENS = 512
 
     def __init__(self, cfg: ModelArchConfig):
         super().__init__()
@@ -218,8 +228,80 @@ class MoEMLP(nn.Module):
         self.top_k = cfg.num_experts_per_tok
         self.gate = nn.Linear(cfg.hidden_size, self.n_experts, bias=False)
         self.experts = nn.ModuleList([MLP(cfg) for _ in range(self.n_experts)])
+        self.gelu = cfg.hidden_act == "gelu_pytorch_tanh"
+        self._stacks: dict = {}
+        self.stack_experts()
+
+    def stack_experts(self) -> None:
+        """Put the experts' weights (and fp8 scales) behind one another and
+        leave views of them in the modules. Called again when the modules
+        have been replaced (fp8 conversion)."""
+        self._stacks = {}
+        for proj in ("gate_up_proj", "down_proj"):
+            mods = [getattr(e, proj) for e in self.experts]
+            if any(getattr(m, "bias", None) is not None for m in mods):
+                self._stacks = {}
+                return
+            for name in ("weight_fp8", "weight_scale"):
+                if name in mods[0]._buffers:
+                    self._stacks[proj, name] = torch.stack(
+                        [m._buffers[name] for m in mods]
+                    )
+                    for m, v in zip(mods, self._stacks[proj, name]):
+                        m._buffers[name] = v
+            if "weight" in mods[0]._parameters:
+                stack = torch.stack([m.weight.data for m in mods])
+                self._stacks[proj, "weight"] = stack
+                for m, v in zip(mods, stack):
+                    m.weight = nn.Parameter(v, requires_grad=m.weight.requires_grad)
+
+    def _stack(self, proj: str, name: str):
+        """The stacked tensor, or None where a module's own tensor has been
+        moved out of it since."""
+        stack = self._stacks.get((proj, name))
+        if stack is None:
+            return None
+        at, step = stack.data_ptr(), stack.stride(0) * stack.element_size()
+        for e in self.experts:
+            m = getattr(e, proj)
+            t = m._parameters.get(name) if name == "weight" else m._buffers.get(name)
+            if t is None or t.data_ptr() != at or t.shape != stack.shape[1:]:
+                return None
+            at += step
+        return stack
+
+    def _grouped(self, x: torch.Tensor):
+        """All experts' rows at once; None where the kernels do not take it."""
+        if not (
+            x.is_cuda
+            and x.dtype == self.gate.weight.dtype == torch.bfloat16
+            and x.is_contiguous()
+            and 1 <= x.shape[0] <= self.GROUPED_MAX_TOKENS
+            and self.n_experts <= 32
+            and self.top_k <= 8
+            and not torch.is_grad_enabled()
+        ):
+            return None
+        fp8 = ("down_proj", "weight_fp8") in self._stacks
+        name = "weight_fp8" if fp8 else "weight"
+        gu, dn = self._stack("gate_up_proj", name), self._stack("down_proj", name)
+        if gu is None or dn is None or (
+            gu.shape[2] * gu.element_size() % 64 or dn.shape[2] * dn.element_size() % 64
+            or gu.shape[1] % 16 or dn.shape[1] % 8
+        ):
+            return None
+        if not fp8:
+            return ops.moe_mlp(x, self.gate.weight, self.top_k, gu, dn, gelu=self.gelu)
+        gs = self._stack("gate_up_proj", "weight_scale")
+        ds = self._stack("down_proj", "weight_scale")
+        if gs is None or ds is None or self.gelu:
+            return None
+        return ops.moe_mlp(x, self.gate.weight, self.top_k, gu, dn, gs, ds)
 
     def forward(self, x: torch.Tensor, fb: ForwardBatch | None = None) -> torch.Tensor:
+        out = self._grouped(x)
+        if out is not None:
+            return out
         T, H = x.shape
         router = F.linear(x.float(), self.gate.weight.float())  # [T, E]
         weights, selected = torch.topk(router, self.top_k, dim=-1)

@@ -237,6 +237,39 @@ def quant_fp8(x):
     return out, scale
 
 
+def moe_mlp(x, router, top_k: int, gate_up, down, gate_up_scale=None, down_scale=None,
+            gelu: bool = False):
+    """GPU-only: sparse mixture of gated experts. x [T, H], router [E, H] (both
+    bf16), gate_up [E, 2I, H] and down [E, H, I] in bf16, or fp8 with scales per
+    output column (x is then quantized once, every expert's activations once).
+    Router scores, weights and the sum over a token's experts are fp32."""
+    _require_ext()
+    T, H = x.shape
+    E, n = router.shape[0], T * top_k
+    i32 = torch.empty(3 * n + E + 1, dtype=torch.int32, device=x.device)
+    index, src, place, begin = i32.split([n, n, n, E + 1])
+    index = index.view(T, top_k)
+    weight = torch.empty((T, top_k), dtype=torch.float32, device=x.device)
+    _C.moe_route(index, weight, begin, src, place, x, router.detach())
+    h = torch.empty((n, gate_up.shape[1]), dtype=torch.bfloat16, device=x.device)
+    y = torch.empty((n, H), dtype=torch.bfloat16, device=x.device)
+    if gate_up_scale is not None:
+        _C.skinny_experts(h, *_with_scale(quant_fp8(x), gate_up, gate_up_scale), begin, src)
+        _C.skinny_experts(y, *_with_scale(silu_and_mul_fp8(h), down, down_scale), begin, None)
+    else:
+        _C.skinny_experts(h, x, gate_up, None, None, begin, src)
+        a = gelu_and_mul(h) if gelu else silu_and_mul(h)
+        _C.skinny_experts(y, a, down, None, None, begin, None)
+    out = torch.empty_like(x)
+    _C.moe_combine(out, y, place, weight)
+    return out
+
+
+def _with_scale(quantized, weight, weight_scale):
+    xq, xs = quantized
+    return xq, weight, xs, weight_scale
+
+
 def greedy_sample(logits):
     if logits.is_cuda:
         _require_ext()

@@ -1,0 +1,127 @@
+"""Device-side routing and grouped expert products at the edges of their tiles
+(16-row tiles, 64 columns a workgroup, 256/512-byte steps of K, several passes
+for an expert with many rows) and skinny products at theirs.
+
+The reference rounds where the kernels do (each product and the activation to
+bf16), so what is left is fp32 sums in another order, which moves a rounded
+intermediate by one bf16 step (2^-8) now and then: bounded as 2^-7 of the
+largest value of a row, and 1e-3 in the norm."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+import kubeai_amd.ops as ops
+from kubeai_amd.engine.quant import Fp8Linear
+from kubeai_amd.models.config import PRESETS, ModelArchConfig
+from kubeai_amd.models.llama import MoEMLP
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _close(got, want):
+    got, want = got.float(), want.float()
+    assert (got - want).norm() <= 2e-3 * want.norm() + 1e-6
+    big = want.abs().amax(-1, keepdim=True)
+    assert ((got - want).abs() <= 2.0 ** -7 * big + 1e-6).all()
+
+
+def _mm(x, w):
+    return (x.double() @ w.double().T).float()
+
+
+@pytest.mark.parametrize("M", [1, 15, 16, 17, 33, 64, 65, 96])
+@pytest.mark.parametrize("N,K", [(4, 32), (60, 64), (64, 96), (100, 544), (4100, 1312),
+                                 (16640, 256)])
+def test_skinny_linear(M, N, K):
+    from kubeai_amd import _C
+
+    torch.manual_seed(M + N + K)
+    wide = torch.randn(M, K + 16, device=DEV, dtype=torch.bfloat16)
+    x, w = wide[:, :K], torch.randn(N, K, device=DEV, dtype=torch.bfloat16)
+    y = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    b = torch.randn(N, device=DEV, dtype=torch.bfloat16)
+    _C.skinny_linear(y, x, w, None, None, None)
+    _close(y, _mm(x, w))
+    _C.skinny_linear(y, x, w, None, None, b)
+    _close(y, _mm(x, w) + b.float())
+    if K % 64:
+        return
+    x8, w8 = x.contiguous().to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn)
+    sx, sw = torch.rand(M, device=DEV) + 0.1, torch.rand(N, device=DEV) + 0.1
+    _C.skinny_linear(y, x8, w8, sx, sw, b)
+    _close(y, _mm(x8.float(), w8.float()) * sx[:, None] * sw + b.float())
+
+
+def _experts(E, I, H):
+    gu = torch.randn(E, 2 * I, H, device=DEV, dtype=torch.bfloat16) * H ** -0.5
+    dn = torch.randn(E, H, I, device=DEV, dtype=torch.bfloat16) * I ** -0.5
+    return gu, dn
+
+
+@pytest.mark.parametrize("T,E,top", [(1, 8, 2), (3, 1, 1), (17, 5, 3), (40, 8, 2), (97, 32, 8),
+                                     (300, 4, 2)])
+@pytest.mark.parametrize("one_expert", [False, True])
+def test_moe(T, E, top, one_expert):
+    torch.manual_seed(T * E)
+    H, I = 256, 160
+    x = torch.randn(T, H, device=DEV, dtype=torch.bfloat16)
+    router = torch.randn(E, H, device=DEV, dtype=torch.bfloat16)
+    if one_expert:  # every token's first choice is the last expert
+        x[:, 0] = 100.0
+        router[:, 0] = 0.0
+        router[E - 1, 0] = 5.0
+    gu, dn = _experts(E, I, H)
+    got = ops.moe_mlp(x, router, top, gu, dn)
+    z = _mm(x, router)
+    v, idx = z.topk(top, -1)
+    w = torch.softmax(v, -1)
+    want = torch.zeros(T, H, device=DEV)
+    for e in range(E):
+        h = _mm(x, gu[e]).bfloat16().float()
+        g, u = h.chunk(2, -1)
+        a = (F.silu(g) * u).bfloat16()
+        y = _mm(a, dn[e]).bfloat16().float()
+        want += (w * (idx == e)).sum(-1, keepdim=True) * y
+    _close(got, want)
+
+
+def test_module_routes():
+    """fp8 and bf16 modules against their per-expert route, weights copied in
+    after construction, and a module whose tensor has left the stack."""
+    cfg = ModelArchConfig(architecture="mixtral", hidden_size=256, intermediate_size=192,
+                          num_local_experts=4, num_experts_per_tok=2)
+    torch.manual_seed(5)
+    prev = torch.get_default_dtype()
+    torch.set_default_dtype(torch.bfloat16)
+    try:
+        with torch.device(DEV):
+            m = MoEMLP(cfg)
+    finally:
+        torch.set_default_dtype(prev)
+    x = torch.randn(37, 256, device=DEV, dtype=torch.bfloat16)
+
+    def both():
+        grouped = m._grouped(x)
+        assert grouped is not None
+        m.GROUPED_MAX_TOKENS = 0
+        one_by_one = m(x)
+        del m.GROUPED_MAX_TOKENS
+        # the per-expert route rounds weights and partial sums to bf16
+        assert (grouped - one_by_one).float().norm() < 0.02 * one_by_one.float().norm()
+        return grouped
+
+    with torch.inference_mode():
+        both()
+        for e in m.experts:
+            e.down_proj.weight.copy_(torch.randn_like(e.down_proj.weight))
+        both()
+        for e in m.experts:
+            e.gate_up_proj = Fp8Linear(e.gate_up_proj.weight)
+            e.down_proj = Fp8Linear(e.down_proj.weight)
+        assert m._grouped(x) is None  # the modules' tensors are not the stack's
+        m.stack_experts()
+        both()
+        m.experts[1].down_proj.weight_fp8 = m.experts[1].down_proj.weight_fp8.clone()
+        assert m._grouped(x) is None
+    assert PRESETS["mixtral-8x7b"].num_local_experts <= 32
