@@ -9,8 +9,16 @@ void rope(torch::Tensor q, torch::Tensor k, torch::Tensor positions,
           torch::Tensor cos_sin);
 void rope_cache(torch::Tensor qkv, torch::Tensor positions,
                 torch::Tensor cos_sin, torch::Tensor k_cache,
-                torch::Tensor v_cache, torch::Tensor slot_mapping,
-                int64_t n_q);
+                torch::Tensor v_cache, torch::Tensor slot_mapping, int64_t n_q,
+                c10::optional<torch::Tensor> part,
+                c10::optional<torch::Tensor> sx,
+                c10::optional<torch::Tensor> sw);
+torch::Tensor skinny_sums(torch::Tensor x, torch::Tensor w);
+void rmsnorm_sums(torch::Tensor out, c10::optional<torch::Tensor> out_scale,
+                  torch::Tensor part, c10::optional<torch::Tensor> sx,
+                  c10::optional<torch::Tensor> sw,
+                  c10::optional<torch::Tensor> residual, torch::Tensor weight,
+                  double eps);
 void reshape_and_cache_fp8(torch::Tensor k, torch::Tensor v,
                            torch::Tensor k_cache, torch::Tensor v_cache,
                            torch::Tensor slot_mapping);
@@ -94,6 +102,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_gemm", &skinny_gemm, "weight-streaming product, bf16");
   m.def("skinny_experts", &skinny_experts,
         "weight-streaming product of each expert's rows");
+  m.def("skinny_sums", &skinny_sums, "fp32 part sums of a skinny product");
+  m.def("rmsnorm_sums", &rmsnorm_sums, "norm of a product's part sums");
   m.def("moe_route", &moe_route,
         "router scores, top-k weights and tokens in expert order");
   m.def("moe_combine", &moe_combine, "weighted sum of the experts' rows");

@@ -125,6 +125,59 @@ DEV_INLINE float soft_cap(float x, float cap, float inv_cap) {
   return cap * (fabsf(y) < 0.2f ? small : big);
 }
 
+// The result of a matrix product that was cut along K: fp32 sums of every
+// part, [parts, M, N], to be added, scaled (fp8 operands) and rounded to bf16
+// by whoever reads it.
+struct ProductSums {
+  const float* part;
+  const float* sx;  // per row, or null
+  const float* sw;  // per column
+  int parts;
+  int64_t stride;   // M * N
+  int N;
+};
+
+// Sum of PARTS parts of 8 neighbouring columns; every load is issued before
+// the first addition (a chain of eight would cost eight latencies).
+template <int PARTS>
+DEV_INLINE void add_parts8(const float* a, int64_t stride, float4_t* v) {
+  float4_t t[PARTS][2];
+#pragma unroll
+  for (int s = 0; s < PARTS; ++s) {
+    const float4_t* b = reinterpret_cast<const float4_t*>(a + s * stride);
+    t[s][0] = b[0];
+    t[s][1] = b[1];
+  }
+#pragma unroll
+  for (int s = 0; s < PARTS; ++s) {
+    v[0] += t[s][0];
+    v[1] += t[s][1];
+  }
+}
+
+// 8 neighbouring columns n.. of row m, as the bf16 values a stored product
+// would have (the parts are added in order, whatever their number)
+DEV_INLINE ushort8 read_sums8(const ProductSums& p, int64_t m, int n) {
+  const float* a = p.part + m * p.N + n;
+  float4_t v[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  int s = 0;
+  for (; s + 8 <= p.parts; s += 8) add_parts8<8>(a + s * p.stride, p.stride, v);
+  if (s + 4 <= p.parts) {
+    add_parts8<4>(a + s * p.stride, p.stride, v);
+    s += 4;
+  }
+  for (; s < p.parts; ++s) add_parts8<1>(a + s * p.stride, p.stride, v);
+  ushort8 o;
+  const float sx = p.sx ? p.sx[m] : 1.0f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    float f = v[j / 4][j % 4];
+    if (p.sx) f = f * sx * p.sw[n + j];
+    o[j] = f32_to_bf16(f);
+  }
+  return o;
+}
+
 // ---------------- wave reductions (64-wide) ----------------
 
 DEV_INLINE float wave_reduce_sum(float v) {

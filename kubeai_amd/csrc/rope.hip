@@ -8,6 +8,8 @@
 // (i, i + hd/2) for hd=128 (one pair per lane), generic loop otherwise.
 #include <torch/extension.h>
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -63,9 +65,12 @@ DEV_INLINE void put_row8(CT* dst, const ushort8& v) {
   }
 }
 
-template <typename CT>
+// SUMS: the projection is a product's parts; q goes to its own rows.
+template <typename CT, bool SUMS>
 __launch_bounds__(256) __global__ void rope_cache_kernel(
-    ushort* __restrict__ qkv,  // [T, (n_q + 2 n_kv) hd], rows strided
+    ushort* __restrict__ qkv,  // [T, (n_q + 2 n_kv) hd], rows strided; SUMS:
+                               // q out [T, n_q hd]
+    const ProductSums sums,
     const int32_t* __restrict__ positions,
     const float* __restrict__ cos_sin,   // [max_pos, hd]
     CT* __restrict__ k_cache,            // [nb, n_kv, bs, hd]
@@ -87,8 +92,14 @@ __launch_bounds__(256) __global__ void rope_cache_kernel(
     const int64_t slot = head < n_q ? 0 : slot_mapping[tok];
     if (slot < 0) return;  // a padding token's key goes nowhere
     const float* cs = cos_sin + (int64_t)positions[tok] * hd + p;
-    const ushort8 a = *reinterpret_cast<const ushort8*>(base);
-    const ushort8 b = *reinterpret_cast<const ushort8*>(base + half);
+    ushort8 a, b;
+    if constexpr (SUMS) {
+      a = read_sums8(sums, tok, head * hd + p);
+      b = read_sums8(sums, tok, head * hd + p + half);
+    } else {
+      a = *reinterpret_cast<const ushort8*>(base);
+      b = *reinterpret_cast<const ushort8*>(base + half);
+    }
     ushort8 oa, ob;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -111,18 +122,26 @@ __launch_bounds__(256) __global__ void rope_cache_kernel(
     if (slot < 0) return;
     const int upr = hd / 8;
     const int head = (item - n_rot) / upr, u = (item - n_rot) % upr * 8;
-    put_row8(v_cache + (((slot / bs) * n_kv + head) * bs + slot % bs) * hd + u,
-             *reinterpret_cast<const ushort8*>(
-                 row + (int64_t)(n_q + n_kv + head) * hd + u));
+    ushort8 v;
+    if constexpr (SUMS)
+      v = read_sums8(sums, tok, (n_q + n_kv + head) * hd + u);
+    else
+      v = *reinterpret_cast<const ushort8*>(
+          row + (int64_t)(n_q + n_kv + head) * hd + u);
+    put_row8(v_cache + (((slot / bs) * n_kv + head) * bs + slot % bs) * hd + u, v);
   }
 }
 
 }  // namespace
 
+// qkv: the bf16 projection (q is rotated in place), or with `part` its sums
+// (fp32 [parts, T, width], sx and sw for fp8 operands), and q's rows out
 void rope_cache(torch::Tensor qkv, torch::Tensor positions,
                 torch::Tensor cos_sin, torch::Tensor k_cache,
-                torch::Tensor v_cache, torch::Tensor slot_mapping,
-                int64_t n_q) {
+                torch::Tensor v_cache, torch::Tensor slot_mapping, int64_t n_q,
+                c10::optional<torch::Tensor> part,
+                c10::optional<torch::Tensor> sx,
+                c10::optional<torch::Tensor> sw) {
   TORCH_CHECK(qkv.scalar_type() == torch::kBFloat16 && qkv.dim() == 2 &&
               qkv.stride(1) == 1 && qkv.stride(0) % 8 == 0 &&
               ((uintptr_t)qkv.data_ptr() & 15) == 0);
@@ -135,30 +154,46 @@ void rope_cache(torch::Tensor qkv, torch::Tensor positions,
                k_cache.scalar_type() == torch::kFloat8_e5m2));
   const int n_kv = k_cache.size(1), bs = k_cache.size(2), hd = k_cache.size(3);
   const int64_t T = qkv.size(0);
+  const int width = (int)(n_q + 2 * n_kv) * hd;
   TORCH_CHECK(hd % 16 == 0 && cos_sin.size(1) == hd &&
               v_cache.sizes() == k_cache.sizes() &&
-              qkv.size(1) == (n_q + 2 * n_kv) * hd);
+              qkv.size(1) == (part.has_value() ? n_q * hd : width));
   TORCH_CHECK(positions.numel() >= T && slot_mapping.numel() >= T);
+  ProductSums p{};
+  if (part.has_value()) {
+    TORCH_CHECK(part->scalar_type() == torch::kFloat32 && part->is_contiguous() &&
+                part->dim() == 3 && part->size(1) == T && part->size(2) == width);
+    TORCH_CHECK(sx.has_value() == sw.has_value());
+    p = {part->data_ptr<float>(), nullptr, nullptr, (int)part->size(0), T * width,
+         width};
+    if (sx.has_value()) {
+      TORCH_CHECK(sx->scalar_type() == torch::kFloat32 && sx->is_contiguous() &&
+                  sx->numel() == T && sw->scalar_type() == torch::kFloat32 &&
+                  sw->is_contiguous() && sw->numel() == width);
+      p.sx = sx->data_ptr<float>();
+      p.sw = sw->data_ptr<float>();
+    }
+  }
   if (T == 0) return;
   const int64_t items = T * ((n_q + n_kv) * (hd / 16) + n_kv * (hd / 8));
   const dim3 grid((uint32_t)((items + 255) / 256));
-  auto stream = c10::hip::getCurrentHIPStream().stream();
-  if (k_cache.scalar_type() == torch::kBFloat16)
-    hipLaunchKernelGGL((rope_cache_kernel<ushort>), grid, dim3(256), 0, stream,
-                       (ushort*)qkv.data_ptr(), positions.data_ptr<int32_t>(),
-                       cos_sin.data_ptr<float>(), (ushort*)k_cache.data_ptr(),
-                       (ushort*)v_cache.data_ptr(),
-                       slot_mapping.data_ptr<int64_t>(), (int)n_q, n_kv, hd, bs,
-                       T, qkv.stride(0));
-  else
-    hipLaunchKernelGGL((rope_cache_kernel<unsigned char>), grid, dim3(256), 0,
-                       stream, (ushort*)qkv.data_ptr(),
+  auto go = [&](auto ct, auto sums) {
+    using CT = decltype(ct);
+    hipLaunchKernelGGL((rope_cache_kernel<CT, decltype(sums)::value>), grid,
+                       dim3(256), 0, c10::hip::getCurrentHIPStream().stream(),
+                       (ushort*)qkv.data_ptr(), p,
                        positions.data_ptr<int32_t>(),
-                       cos_sin.data_ptr<float>(),
-                       (unsigned char*)k_cache.data_ptr(),
-                       (unsigned char*)v_cache.data_ptr(),
+                       cos_sin.data_ptr<float>(), (CT*)k_cache.data_ptr(),
+                       (CT*)v_cache.data_ptr(),
                        slot_mapping.data_ptr<int64_t>(), (int)n_q, n_kv, hd, bs,
                        T, qkv.stride(0));
+  };
+  auto with_ct = [&](auto sums) {
+    if (k_cache.scalar_type() == torch::kBFloat16) go((ushort)0, sums);
+    else go((unsigned char)0, sums);
+  };
+  if (part.has_value()) with_ct(std::true_type{});
+  else with_ct(std::false_type{});
   HIP_CHECK_KERNEL();
 }
 

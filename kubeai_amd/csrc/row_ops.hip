@@ -78,13 +78,15 @@ DEV_INLINE void write_fp8_row(unsigned char* out, float* out_scale, int64_t row,
   }
 }
 
-// ADD: residual += x, norm of the sum. FP8: fp8 output with a row scale.
-template <bool ADD, bool FP8, int VPT>
+// ADD: residual += x, norm of the sum. FP8: fp8 output with a row scale. SUMS:
+// x is a product's parts (added here instead of in a launch of their own).
+template <bool ADD, bool FP8, bool SUMS, int VPT>
 __launch_bounds__(VPT == 8 ? 512 : 1024) __global__ void rmsnorm_kernel(
     void* __restrict__ out, float* __restrict__ out_scale,
     const ushort* x,        // [T, H]; may be `out`
     ushort* __restrict__ residual,
-    const ushort* __restrict__ w, const float eps, const int H) {
+    const ushort* __restrict__ w, const float eps, const int H,
+    const ProductSums sums) {
   const int64_t row = blockIdx.x;
   const int nvec = H / 8;
   __shared__ float red[2][16];
@@ -94,7 +96,9 @@ __launch_bounds__(VPT == 8 ? 512 : 1024) __global__ void rmsnorm_kernel(
   for (int k = 0; k < VPT; ++k) {
     const int i = threadIdx.x + k * blockDim.x;
     if (i < nvec) {
-      const ushort8 xv = reinterpret_cast<const ushort8*>(x + row * H)[i];
+      ushort8 xv;
+      if constexpr (SUMS) xv = read_sums8(sums, row, i * 8);
+      else xv = reinterpret_cast<const ushort8*>(x + row * H)[i];
       if constexpr (ADD) {
         ushort8* rp = reinterpret_cast<ushort8*>(residual + row * H) + i;
         const ushort8 rin = *rp;
@@ -204,18 +208,17 @@ void check_row_op(const torch::Tensor& x, int max_h) {
   TORCH_CHECK(x.size(-1) % 8 == 0 && x.size(-1) <= max_h);
 }
 
-template <bool ADD, bool FP8>
-void launch_norm(void* out, float* out_scale, const torch::Tensor& x,
-                 ushort* residual, const torch::Tensor& weight, double eps) {
-  const int H = x.size(-1);
-  const int64_t T = x.numel() / H;
+template <bool ADD, bool FP8, bool SUMS = false>
+void launch_norm(void* out, float* out_scale, const ushort* x, int64_t T, int H,
+                 ushort* residual, const torch::Tensor& weight, double eps,
+                 const ProductSums& sums = {}) {
   const Split s = split_for(T, H);
   with_vpt(s.vpt, [&](auto vpt) {
-    hipLaunchKernelGGL((rmsnorm_kernel<ADD, FP8, decltype(vpt)::value>),
+    hipLaunchKernelGGL((rmsnorm_kernel<ADD, FP8, SUMS, decltype(vpt)::value>),
                        dim3((uint32_t)T), dim3(s.threads), 0,
                        c10::hip::getCurrentHIPStream().stream(), out, out_scale,
-                       (const ushort*)x.data_ptr(), residual,
-                       (const ushort*)weight.data_ptr(), (float)eps, H);
+                       x, residual, (const ushort*)weight.data_ptr(), (float)eps,
+                       H, sums);
   });
   HIP_CHECK_KERNEL();
 }
@@ -242,22 +245,23 @@ void rmsnorm(torch::Tensor out, torch::Tensor x, torch::Tensor weight,
              double eps) {
   check_row_op(x, kMaxH);
   TORCH_CHECK(out.is_contiguous());
-  launch_norm<false, false>(out.data_ptr(), nullptr, x, nullptr, weight, eps);
+  launch_norm<false, false>(out.data_ptr(), nullptr, (const ushort*)x.data_ptr(),
+      x.numel() / x.size(-1), x.size(-1), nullptr, weight, eps);
 }
 
 void fused_add_rmsnorm(torch::Tensor x, torch::Tensor residual,
                        torch::Tensor weight, double eps) {
   check_row_op(x, kMaxH);
   TORCH_CHECK(residual.is_contiguous());
-  launch_norm<true, false>(x.data_ptr(), nullptr, x,
-                           (ushort*)residual.data_ptr(), weight, eps);
+  launch_norm<true, false>(x.data_ptr(), nullptr, (const ushort*)x.data_ptr(),
+      x.numel() / x.size(-1), x.size(-1), (ushort*)residual.data_ptr(), weight, eps);
 }
 
 void rmsnorm_fp8(torch::Tensor out, torch::Tensor out_scale, torch::Tensor x,
                  torch::Tensor weight, double eps) {
   check_row_op(x, kMaxHFp8);
-  launch_norm<false, true>(out.data_ptr(), out_scale.data_ptr<float>(), x,
-                           nullptr, weight, eps);
+  launch_norm<false, true>(out.data_ptr(), out_scale.data_ptr<float>(), (const ushort*)x.data_ptr(),
+      x.numel() / x.size(-1), x.size(-1), nullptr, weight, eps);
 }
 
 void fused_add_rmsnorm_fp8(torch::Tensor out, torch::Tensor out_scale,
@@ -265,8 +269,8 @@ void fused_add_rmsnorm_fp8(torch::Tensor out, torch::Tensor out_scale,
                            torch::Tensor weight, double eps) {
   check_row_op(x, kMaxHFp8);
   TORCH_CHECK(residual.is_contiguous());
-  launch_norm<true, true>(out.data_ptr(), out_scale.data_ptr<float>(), x,
-                          (ushort*)residual.data_ptr(), weight, eps);
+  launch_norm<true, true>(out.data_ptr(), out_scale.data_ptr<float>(), (const ushort*)x.data_ptr(),
+      x.numel() / x.size(-1), x.size(-1), (ushort*)residual.data_ptr(), weight, eps);
 }
 
 void silu_and_mul_fp8(torch::Tensor out, torch::Tensor out_scale,
@@ -281,4 +285,48 @@ void quant_fp8(torch::Tensor out, torch::Tensor out_scale, torch::Tensor x) {
   check_row_op(x, kMaxHFp8);
   const int H = x.size(-1);
   launch_to_fp8<false>(out, out_scale, x, x.numel() / H, H);
+}
+
+// the norms of a row that is still a product's parts: part fp32 [parts, T, H],
+// sx [T] and sw [H] for fp8 operands. residual: added and updated, or none.
+// out_scale given: out is fp8, else bf16.
+void rmsnorm_sums(torch::Tensor out, c10::optional<torch::Tensor> out_scale,
+                  torch::Tensor part, c10::optional<torch::Tensor> sx,
+                  c10::optional<torch::Tensor> sw,
+                  c10::optional<torch::Tensor> residual, torch::Tensor weight,
+                  double eps) {
+  TORCH_CHECK(part.scalar_type() == torch::kFloat32 && part.is_contiguous() &&
+              part.is_cuda() && part.dim() == 3);
+  const int64_t T = part.size(1);
+  const int H = part.size(2);
+  TORCH_CHECK(H % 8 == 0 && H <= (out_scale.has_value() ? kMaxHFp8 : kMaxH));
+  TORCH_CHECK(sx.has_value() == sw.has_value());
+  if (sx.has_value())
+    TORCH_CHECK(sx->scalar_type() == torch::kFloat32 && sx->is_contiguous() &&
+                sx->numel() == T && sw->scalar_type() == torch::kFloat32 &&
+                sw->is_contiguous() && sw->numel() == H);
+  TORCH_CHECK(out.is_contiguous() && out.numel() == T * H &&
+              out.element_size() == (out_scale.has_value() ? 1 : 2));
+  TORCH_CHECK(weight.scalar_type() == torch::kBFloat16 && weight.numel() == H);
+  ushort* res = nullptr;
+  if (residual.has_value()) {
+    TORCH_CHECK(residual->is_contiguous() && residual->numel() == T * H &&
+                residual->scalar_type() == torch::kBFloat16);
+    res = (ushort*)residual->data_ptr();
+  }
+  float* scale = nullptr;
+  if (out_scale.has_value()) {
+    TORCH_CHECK(out_scale->scalar_type() == torch::kFloat32 &&
+                out_scale->is_contiguous() && out_scale->numel() == T);
+    scale = out_scale->data_ptr<float>();
+  }
+  const ProductSums p{part.data_ptr<float>(),
+                      sx.has_value() ? sx->data_ptr<float>() : nullptr,
+                      sw.has_value() ? sw->data_ptr<float>() : nullptr,
+                      (int)part.size(0), T * H, H};
+  void* o = out.data_ptr();
+  if (res && scale) launch_norm<true, true, true>(o, scale, nullptr, T, H, res, weight, eps, p);
+  else if (res) launch_norm<true, false, true>(o, nullptr, nullptr, T, H, res, weight, eps, p);
+  else if (scale) launch_norm<false, true, true>(o, scale, nullptr, T, H, nullptr, weight, eps, p);
+  else launch_norm<false, false, true>(o, nullptr, nullptr, T, H, nullptr, weight, eps, p);
 }

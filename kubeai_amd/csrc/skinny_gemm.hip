@@ -20,6 +20,18 @@
 // that about 768 result (N = 6144, 40 rows fp8: 8.8 us with 768, 9.7 with
 // 384); from 256 on the second pass costs more than the parts give (28672:
 // 28.2 us whole, 29.8 in two parts).
+// Where a consumer can add the parts itself (skinny_sums; the norm after an
+// attention or feed-forward block, the rotation of q and k) that second pass,
+// about 5 us of launch and drain, is gone.
+// Measured in the decode step, W out of cache, us (library product + what
+// reads it -> this + that):
+//   fp8, 40 rows  4096 -> 6144 and rotation   13.5 + 4.9 ->  9.6 + 6.9
+//                 14336 -> 4096 and norm      23.0 + 5.1 -> 16.4 + 7.4
+//                 4096 -> 4096 and norm       11.8 + 5.1 ->  8.0 + 7.4
+//   bf16, 8 rows  4096 -> 6144 and rotation   15.5 + 4.9 -> 12.1 + 4.8
+//                 14336 -> 4096 and norm      25.6 + 5.2 -> 23.0 + 4.8
+//                 4096 -> 28672               62.9       -> 49.6 (4.7 TB/s)
+//   bf16, 96 rows 14336 -> 4096 and norm      54.1 + 5.5 -> 36.0 + 5.8
 // The grouped form multiplies every expert's rows of a mixture in one launch,
 // x rows gathered by index. 8 experts of 4096 x 14336, 40 tokens of 2 experts
 // each, both products with routing and activation: fp8 297 us (4.8 TB/s over
@@ -253,7 +265,7 @@ struct Shape {
 Shape check(const torch::Tensor& x, const torch::Tensor& w,
             const c10::optional<torch::Tensor>& sx,
             const c10::optional<torch::Tensor>& sw,
-            const c10::optional<torch::Tensor>& bias) {
+            const c10::optional<torch::Tensor>& bias, bool raw = false) {
   const bool fp8 = w.scalar_type() == torch::kFloat8_e4m3fn;
   TORCH_CHECK(fp8 || w.scalar_type() == torch::kBFloat16,
               "bf16 or fp8 e4m3 weights");
@@ -269,9 +281,9 @@ Shape check(const torch::Tensor& x, const torch::Tensor& w,
               ((uintptr_t)x.data_ptr() & 15) == 0 &&
               ((uintptr_t)w.data_ptr() & 15) == 0,
               "16-byte aligned rows");
-  TORCH_CHECK(fp8 == (sx.has_value() && sw.has_value()),
+  TORCH_CHECK(raw || fp8 == (sx.has_value() && sw.has_value()),
               "fp8 operands come with their scales, bf16 ones without");
-  if (fp8) {
+  if (fp8 && !raw) {
     TORCH_CHECK(sx->scalar_type() == torch::kFloat32 && sx->is_contiguous() &&
                 sx->numel() == s.M && sw->scalar_type() == torch::kFloat32 &&
                 sw->is_contiguous() && sw->numel() == s.N);
@@ -334,6 +346,17 @@ void skinny_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                      dim3(256), 0, c10::hip::getCurrentHIPStream().stream(), yp,
                      part.data_ptr<float>(), sxp, swp, bp, s.M, s.N, cut.parts);
   HIP_CHECK_KERNEL();
+}
+
+// the fp32 sums of x w^T alone, [parts, M, N], for a consumer that adds the
+// parts itself (and applies an fp8 product's scales)
+torch::Tensor skinny_sums(torch::Tensor x, torch::Tensor w) {
+  c10::optional<torch::Tensor> none;
+  const Shape s = check(x, w, none, none, none, true);
+  const Cut cut = cut_for(s.N, s.KB);
+  auto part = torch::empty({cut.parts, s.M, s.N}, x.options().dtype(torch::kFloat32));
+  launch(nullptr, part.data_ptr<float>(), x, w, nullptr, nullptr, nullptr, s, cut);
+  return part;
 }
 
 // y[i] = x[src[i]] w[e]^T for the rows i of expert e, scaled as above; w

@@ -54,13 +54,16 @@ class Fp8Linear(nn.Module):
             w = self.weight_fp8.float() * self.weight_scale.reshape(-1, 1)
             y = (x @ w.t()).to(torch.bfloat16)
             return y + self.bias if self.bias is not None else y
-        return torch._scaled_mm(
-            xq,
-            self.weight_fp8.t(),
-            scale_a=x_scale.view(-1, 1),
-            scale_b=self.weight_scale,
-            bias=self.bias,
-            out_dtype=torch.bfloat16,
+        return ops.linear_fp8(
+            xq, x_scale, self.weight_fp8, self.weight_scale, self.bias
+        )
+
+    def sums_quantized(self, xq: torch.Tensor, x_scale: torch.Tensor):
+        """forward_quantized as ops.ProductSums, or None (library product)."""
+        if self.bias is not None:
+            return None
+        return ops.product_sums(
+            xq, self.weight_fp8, x_scale, self.weight_scale.view(-1)
         )
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:

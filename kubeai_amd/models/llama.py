@@ -26,15 +26,28 @@ from .config import ModelArchConfig
 
 
 class EngineLinear(nn.Linear):
-    """nn.Linear routed through ops.linear: the hand-written weight-
-    streaming GEMM takes skinny decode batches (M<=64); hipBLASLt keeps
-    the rest. Bias (Qwen2 qkv) is added outside the skinny path."""
+    """nn.Linear routed through ops.linear. Bias (Qwen2 qkv) is added outside
+    the product."""
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         y = ops.linear(x, self.weight)
         if self.bias is not None:
             y = y + self.bias
         return y
+
+    def sums(self, x: torch.Tensor):
+        """The product as ops.ProductSums, or None (library product, bias)."""
+        return None if self.bias is not None else ops.product_sums(x, self.weight)
+
+
+def _project(linear, x, as_sums: bool):
+    """linear(x), x a tensor or an (fp8 rows, scales) pair. as_sums: what reads
+    the result takes ops.ProductSums, so it may be that."""
+    if isinstance(x, tuple):
+        y = linear.sums_quantized(*x) if as_sums else None
+        return linear.forward_quantized(*x) if y is None else y
+    y = linear.sums(x) if as_sums and isinstance(linear, EngineLinear) else None
+    return linear(x) if y is None else y
 
 
 def _rms_head(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
@@ -93,24 +106,25 @@ class Attention(nn.Module):
         fb: ForwardBatch,
         kv_cache: tuple[torch.Tensor, torch.Tensor],
         cos_sin: torch.Tensor,
+        as_sums: bool = False,
     ) -> torch.Tensor:
+        """as_sums: the caller takes the result as ops.ProductSums too."""
         fp8_in = isinstance(x, tuple)  # (fp8 tensor, row scales) from a
         # fused producer kernel (DecoderLayer fp8 path)
-        if fp8_in:
-            xq, xs = x
-            T = xq.shape[0]
-            qkv = self.qkv_proj.forward_quantized(xq, xs)
-            lm = None
-        else:
-            T = x.shape[0]
-            qkv = self.qkv_proj(x)
-            lm = getattr(self, "_lora_manager", None)
-            if lm is not None and lm.active and fb.lora_ids is not None:
-                lm.apply(self.layer_idx, "qkv", x, qkv, fb.lora_ids)
+        k_cache, v_cache = kv_cache
+        T = (x[0] if fp8_in else x).shape[0]
+        lm = None if fp8_in else getattr(self, "_lora_manager", None)
+        lora_live = lm is not None and lm.active and fb.lora_ids is not None
+        qkv = _project(
+            self.qkv_proj, x,
+            not lora_live and not self.qk_norm
+            and ops.rope_takes_sums(k_cache, v_cache),
+        )
+        if lora_live:
+            lm.apply(self.layer_idx, "qkv", x, qkv, fb.lora_ids)
         if isinstance(cos_sin, tuple):
             # (global, local) caches — gemma3 dual rope bases
             cos_sin = cos_sin[0] if self.is_global else cos_sin[1]
-        k_cache, v_cache = kv_cache
         if self.qk_norm:
             # gemma3: per-head RMSNorm ((1+w) stored as w) before rope;
             # fp32 math, contiguous bf16 out. v follows to contiguous —
@@ -135,7 +149,7 @@ class Attention(nn.Module):
             )
 
         out = torch.empty(
-            (T, self.n_q, self.hd), dtype=qkv.dtype, device=qkv.device
+            (T, self.n_q, self.hd), dtype=q.dtype, device=q.device
         )
         nd = fb.n_decode
         if nd > 0:
@@ -165,10 +179,9 @@ class Attention(nn.Module):
             )
         attn_flat = out.view(T, -1)
         if fp8_in:
-            a8, ascale = ops.quant_fp8(attn_flat)
-            return self.o_proj.forward_quantized(a8, ascale)
-        result = self.o_proj(attn_flat)
-        if lm is not None and lm.active and fb.lora_ids is not None:
+            return _project(self.o_proj, ops.quant_fp8(attn_flat), as_sums)
+        result = _project(self.o_proj, attn_flat, as_sums and not lora_live)
+        if lora_live:
             lm.apply(self.layer_idx, "o", attn_flat, result, fb.lora_ids)
         return result
 
@@ -185,11 +198,13 @@ class MLP(nn.Module):
         self.down_proj = EngineLinear(cfg.intermediate_size, cfg.hidden_size, bias=False)
         self.gelu = cfg.hidden_act == "gelu_pytorch_tanh"
 
-    def forward(self, x, fb: ForwardBatch | None = None) -> torch.Tensor:
+    def forward(
+        self, x, fb: ForwardBatch | None = None, as_sums: bool = False
+    ) -> torch.Tensor:
+        """as_sums: the caller takes the result as ops.ProductSums too."""
         if isinstance(x, tuple):  # fused fp8 path (never active with LoRA)
             h = self.gate_up_proj.forward_quantized(*x)
-            a8, ascale = ops.silu_and_mul_fp8(h)
-            return self.down_proj.forward_quantized(a8, ascale)
+            return _project(self.down_proj, ops.silu_and_mul_fp8(h), as_sums)
         h = self.gate_up_proj(x)
         lm = getattr(self, "_lora_manager", None)
         lora_live = (
@@ -199,7 +214,7 @@ class MLP(nn.Module):
         if lora_live:
             lm.apply(self.layer_idx, "gate_up", x, h, fb.lora_ids)
         a = ops.gelu_and_mul(h) if self.gelu else ops.silu_and_mul(h)
-        y = self.down_proj(a)
+        y = _project(self.down_proj, a, as_sums and not lora_live)
         if lora_live:
             lm.apply(self.layer_idx, "down", a, y, fb.lora_ids)
         return y
@@ -298,7 +313,9 @@ class MoEMLP(nn.Module):
             return None
         return ops.moe_mlp(x, self.gate.weight, self.top_k, gu, dn, gs, ds)
 
-    def forward(self, x: torch.Tensor, fb: ForwardBatch | None = None) -> torch.Tensor:
+    def forward(
+        self, x: torch.Tensor, fb: ForwardBatch | None = None, as_sums: bool = False
+    ) -> torch.Tensor:
         out = self._grouped(x)
         if out is not None:
             return out
@@ -384,12 +401,13 @@ class DecoderLayer(nn.Module):
             hidden = x if residual is None else x + residual
             a = self.self_attn(
                 ops.rmsnorm(hidden, self.input_layernorm, self.eps),
-                fb, kv_cache, cos_sin,
+                fb, kv_cache, cos_sin, as_sums=True,
             )
             a = ops.rmsnorm(a, self.post_attention_layernorm, self.eps)
             h2 = hidden + a
             mm = self.mlp(
-                ops.rmsnorm(h2, self.pre_feedforward_layernorm, self.eps), fb
+                ops.rmsnorm(h2, self.pre_feedforward_layernorm, self.eps), fb,
+                as_sums=True,
             )
             mm = ops.rmsnorm(mm, self.post_feedforward_layernorm, self.eps)
             return mm, h2
@@ -408,7 +426,7 @@ class DecoderLayer(nn.Module):
                 xq, xs = ops.fused_add_rmsnorm_fp8(
                     x, residual, self.input_layernorm, self.eps
                 )
-            x = self.self_attn((xq, xs), fb, kv_cache, cos_sin)
+            x = self.self_attn((xq, xs), fb, kv_cache, cos_sin, as_sums=True)
             if isinstance(self.mlp, MoEMLP):
                 # router consumes bf16; MoEMLP quantizes once internally
                 x, residual = ops.fused_add_rmsnorm(
@@ -419,7 +437,7 @@ class DecoderLayer(nn.Module):
                 xq, xs = ops.fused_add_rmsnorm_fp8(
                     x, residual, self.post_attention_layernorm, self.eps
                 )
-                x = self.mlp((xq, xs))
+                x = self.mlp((xq, xs), as_sums=True)
             return x, residual
         if residual is None:
             residual = x
@@ -428,13 +446,14 @@ class DecoderLayer(nn.Module):
             x, residual = ops.fused_add_rmsnorm(
                 x, residual, self.input_layernorm, self.eps
             )
-        x = self.self_attn(x, fb, kv_cache, cos_sin)
+        plain = self.res_mult == 1.0  # the next norm reads the branch as it is
+        x = self.self_attn(x, fb, kv_cache, cos_sin, as_sums=plain)
         if self.res_mult != 1.0:
             x = x * self.res_mult
         x, residual = ops.fused_add_rmsnorm(
             x, residual, self.post_attention_layernorm, self.eps
         )
-        x = self.mlp(x, fb)
+        x = self.mlp(x, fb, as_sums=plain)
         if self.res_mult != 1.0:
             x = x * self.res_mult
         return x, residual

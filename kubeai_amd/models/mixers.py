@@ -18,6 +18,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from kubeai_amd import ops
 from kubeai_amd.ops import seq as sops
 
 
@@ -34,7 +35,7 @@ class Proj(nn.Module):
         nn.init.normal_(self.weight, std=n_in ** -0.5)
 
     def forward(self, x):
-        return F.linear(x, self.weight)
+        return ops.linear(x, self.weight)
 
 
 class CausalConvTails(nn.Module):

@@ -34,6 +34,8 @@ def _require_ext() -> None:
 
 
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
+    if isinstance(x, ProductSums):
+        return _norm_sums(x, None, weight, eps, fp8=False)
     if x.is_cuda:
         _require_ext()
         out = torch.empty_like(x)
@@ -43,7 +45,10 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
 
 
 def fused_add_rmsnorm(x, residual, weight, eps: float):
-    """In-place on GPU: x <- rmsnorm(x + residual), residual <- x + residual."""
+    """In-place on GPU: x <- rmsnorm(x + residual), residual <- x + residual
+    (x as ProductSums: a new tensor takes the norm)."""
+    if isinstance(x, ProductSums):
+        return _norm_sums(x, residual, weight, eps, fp8=False), residual
     if x.is_cuda:
         _require_ext()
         _C.fused_add_rmsnorm(x, residual, weight, eps)
@@ -71,11 +76,30 @@ def reshape_and_cache(k, v, k_cache, v_cache, slot_mapping) -> None:
     ref.reshape_and_cache(k, v, k_cache, v_cache, slot_mapping)
 
 
+def rope_takes_sums(k_cache, v_cache) -> bool:
+    return (
+        k_cache.is_cuda
+        and k_cache.shape[3] % 16 == 0
+        and k_cache.dtype in (torch.bfloat16, torch.float8_e5m2)
+        and v_cache.dtype == k_cache.dtype
+        and v_cache.shape == k_cache.shape
+        and k_cache.is_contiguous()
+        and v_cache.is_contiguous()
+    )
+
+
 def rope_and_cache(qkv, n_q: int, positions, cos_sin, k_cache, v_cache, slot_mapping):
     """q | k | v rows of the fused projection: q is rotated (in place on GPU) and
     returned as [T, n_q, hd], k is rotated and written to the paged cache with
-    v. One launch on GPU where heads split into 16-byte units."""
+    v. One launch on GPU where heads split into 16-byte units; qkv may be a
+    product's sums there (rope_takes_sums)."""
     n_kv, hd = k_cache.shape[1], k_cache.shape[3]
+    if isinstance(qkv, ProductSums):
+        q = torch.empty((qkv.shape[0], n_q * hd), dtype=torch.bfloat16,
+                        device=qkv.part.device)
+        _C.rope_cache(q, positions, cos_sin, k_cache, v_cache, slot_mapping, n_q,
+                      *qkv.args())
+        return q.unflatten(-1, (n_q, hd))
     q, k, v = qkv.split([n_q * hd, n_kv * hd, n_kv * hd], dim=-1)
     q = q.unflatten(-1, (n_q, hd))
     if (
@@ -90,7 +114,8 @@ def rope_and_cache(qkv, n_q: int, positions, cos_sin, k_cache, v_cache, slot_map
         and v_cache.shape == k_cache.shape
     ):
         _require_ext()
-        _C.rope_cache(qkv, positions, cos_sin, k_cache, v_cache, slot_mapping, n_q)
+        _C.rope_cache(qkv, positions, cos_sin, k_cache, v_cache, slot_mapping, n_q,
+                      None, None, None)
         return q
     q, k = rope(q, k.unflatten(-1, (n_kv, hd)), positions, cos_sin)
     reshape_and_cache(k, v.unflatten(-1, (n_kv, hd)), k_cache, v_cache, slot_mapping)
@@ -168,39 +193,109 @@ def gelu_and_mul(x):
     return ref.gelu_and_mul(x)
 
 
-import os
+class ProductSums:
+    """A matrix product of few rows whose parts along K are not added yet: fp32
+    [parts, M, N], with the scales of fp8 operands. What reads it next adds,
+    scales and rounds it to bf16 on the way (fused_add_rmsnorm, rmsnorm and
+    their fp8 forms, rope_and_cache)."""
 
-_USE_SKINNY = os.environ.get("KUBEAI_SKINNY_GEMM", "0") == "1"
+    is_cuda = True
+
+    def __init__(self, part, x_scale=None, w_scale=None):
+        self.part, self.x_scale, self.w_scale = part, x_scale, w_scale
+        self.shape = part.shape[1:]
+
+    def args(self):
+        return self.part, self.x_scale, self.w_scale
+
+
+def _skinny_operands(x, weight) -> bool:
+    """Operands that the weight-streaming product takes."""
+    return (
+        _C is not None
+        and x.is_cuda
+        and x.dtype == weight.dtype
+        and x.dtype in (torch.bfloat16, torch.float8_e4m3fn)
+        and x.dim() == 2
+        and 1 <= x.shape[0] <= 96
+        and x.is_contiguous()
+        and weight.is_contiguous()
+        # (the library refuses fp8 columns that are no multiple of 16)
+        and weight.shape[0] % (8 if x.dtype == torch.bfloat16 else 16) == 0
+        and weight.shape[1] * weight.element_size() % 64 == 0
+        and weight.device == x.device
+        and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
+    )
+
+
+def product_sums(x, weight, x_scale=None, w_scale=None):
+    """x weight^T as ProductSums for a consumer that takes them, or None where
+    the library's product is the better one: from 16384 columns on the product
+    fills the chip without being cut, and above 96 rows it is no longer the
+    weights that bound it. (Per product and consumer, us, library -> this: 40
+    rows fp8 4096 -> 6144 18.4 -> 16.5, 14336 -> 4096 28.1 -> 23.8; 96 rows bf16
+    14336 -> 4096 59.6 -> 41.8, 4096 -> 4096 27.5 -> 22.)"""
+    if not (
+        x.shape[0] <= 96 and weight.shape[0] < 16384 and _skinny_operands(x, weight)
+    ):
+        return None
+    return ProductSums(_C.skinny_sums(x, weight), x_scale, w_scale)
+
+
+def _streams_better(M: int, N: int, K: int) -> bool:
+    """Whether the weight-streaming product beats the library's where it has to
+    add its parts itself. Few rows and a width that fills the chip uncut (us,
+    library / this): 8 rows bf16 4096 -> 28672 65 / 50, 2304 -> 18432 51 / 24,
+    2048 -> 32256 33 / 30, fp8 4096 -> 28672 34 / 29; at 32 rows 57 / 56 and
+    21 / 31, at 128256 columns 192 / 198. Very long rows, which the library does
+    not cut: 32256 -> 2048 83 / 36 at 8 rows, 127 / 61 at 96; 14336 -> 4096 at 8
+    rows 27 / 29."""
+    return (M <= 16 and 16384 <= N <= 65536) or (K >= 8 * N and K >= 16384)
 
 
 def linear(x, weight):
-    """GEMM dispatch. The hand-written weight-streaming kernel (skinny_gemm)
-    currently loses to hipBLASLt on MI355X (direct 16 B row gathers do not
-    coalesce; measured 0.3-0.65x — profiles/r01_results.md), so it is
-    opt-in via KUBEAI_SKINNY_GEMM=1 until the LDS-staged variant lands."""
+    """x weight^T. Few rows against a wide or a very long weight go through the
+    weight-streaming kernel (csrc/skinny_gemm.hip), the rest to the library."""
     if (
-        _USE_SKINNY
-        and x.is_cuda
+        x.is_cuda
+        and x.dim() == weight.dim() == 2
+        and x.shape[0] <= 96
+        and _streams_better(x.shape[0], *weight.shape)
         and x.dtype == torch.bfloat16
-        and x.dim() == 2
-        and 1 <= x.shape[0] <= 64
-        and weight.shape[1] % 64 == 0
-        and weight.shape[0] % 64 == 0
-        and x.is_contiguous()
-        and weight.is_contiguous()
+        and _skinny_operands(x, weight)
     ):
-        _require_ext()
         y = torch.empty(
             (x.shape[0], weight.shape[0]), dtype=x.dtype, device=x.device
         )
-        _C.skinny_gemm(y, x, weight)
+        _C.skinny_linear(y, x, weight, None, None, None)
         return y
     return torch.nn.functional.linear(x, weight)
+
+
+def linear_fp8(xq, x_scale, weight, w_scale, bias=None):
+    """(xq * x_scale) (weight * w_scale)^T + bias in bf16; xq [M, K] and weight
+    [N, K] e4m3, x_scale [M], w_scale [1, N]."""
+    if (
+        xq.shape[0] <= 96
+        and _streams_better(xq.shape[0], *weight.shape)
+        and _skinny_operands(xq, weight)
+    ):
+        y = torch.empty(
+            (xq.shape[0], weight.shape[0]), dtype=torch.bfloat16, device=xq.device
+        )
+        _C.skinny_linear(y, xq, weight, x_scale.reshape(-1), w_scale.reshape(-1), bias)
+        return y
+    return torch._scaled_mm(
+        xq, weight.t(), scale_a=x_scale.view(-1, 1), scale_b=w_scale, bias=bias,
+        out_dtype=torch.bfloat16,
+    )
 
 
 def rmsnorm_fp8(x, weight, eps: float):
     """GPU-only: rmsnorm with fused per-row fp8 quantization."""
     _require_ext()
+    if isinstance(x, ProductSums):
+        return _norm_sums(x, None, weight, eps, fp8=True)
     out = torch.empty(x.shape, dtype=torch.float8_e4m3fn, device=x.device)
     scale = torch.empty(x.shape[0], dtype=torch.float32, device=x.device)
     _C.rmsnorm_fp8(out, scale, x, weight, eps)
@@ -210,10 +305,23 @@ def rmsnorm_fp8(x, weight, eps: float):
 def fused_add_rmsnorm_fp8(x, residual, weight, eps: float):
     """GPU-only, in-place residual update; returns (fp8 out, row scales)."""
     _require_ext()
+    if isinstance(x, ProductSums):
+        return _norm_sums(x, residual, weight, eps, fp8=True)
     out = torch.empty(x.shape, dtype=torch.float8_e4m3fn, device=x.device)
     scale = torch.empty(x.shape[0], dtype=torch.float32, device=x.device)
     _C.fused_add_rmsnorm_fp8(out, scale, x, residual, weight, eps)
     return out, scale
+
+
+def _norm_sums(x: ProductSums, residual, weight, eps: float, fp8: bool):
+    """bf16 rows, or (fp8 rows, scales), of the norm of a product's sums."""
+    dev = x.part.device
+    out = torch.empty(
+        x.shape, dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16, device=dev
+    )
+    scale = torch.empty(x.shape[0], dtype=torch.float32, device=dev) if fp8 else None
+    _C.rmsnorm_sums(out, scale, *x.args(), residual, weight, eps)
+    return (out, scale) if fp8 else out
 
 
 def silu_and_mul_fp8(x):

@@ -96,3 +96,95 @@ def test_rope_and_cache_equals_two_kernels(nq, nkv, hd, cache, pad):
         assert (a != b).sum().item() <= 2 + a.numel() // 1000
         torch.testing.assert_close(a, b, atol=1e-6, rtol=rtol)
     assert torch.equal(one[1].view(torch.uint8), two[1].view(torch.uint8))
+
+
+@pytest.mark.parametrize("M", [1, 17, 96])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("N,K", [(512, 1024), (4112, 512), (1008, 9216)])
+def test_norms_of_product_sums(M, fp8, N, K):
+    """Added on the way in, the parts give the same bf16 row as added first; the
+    norms of the two may contract their fp32 products either way, which moves
+    one output in some hundreds by one step of its type."""
+    from kubeai_amd import _C
+
+    def near(a, b, step):
+        a, b = a.float(), b.float()
+        assert (a != b).sum().item() <= 2 + a.numel() // 100
+        torch.testing.assert_close(a, b, atol=1e-6, rtol=step)
+
+    x, w = _x(M, K), _x(N, K) * 0.05
+    sx = sw = None
+    if fp8:
+        x, w = x.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn)
+        sx, sw = torch.rand(M, device=DEV) + 0.5, torch.rand(N, device=DEV) + 0.5
+    y = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    _C.skinny_linear(y, x, w, sx, sw, None)
+    weight = torch.randn(N, device=DEV, dtype=torch.bfloat16)
+    r = _x(M, N)
+
+    def sums():
+        p = ops.product_sums(x, w, sx, sw)
+        assert isinstance(p, ops.ProductSums)
+        return p
+
+    near(ops.rmsnorm(sums(), weight, 1e-5), ops.rmsnorm(y, weight, 1e-5), 2.0 ** -7)
+    (a, sa), (b, sb) = ops.rmsnorm_fp8(sums(), weight, 1e-5), ops.rmsnorm_fp8(y, weight, 1e-5)
+    near(a, b, 2.0 ** -3)
+    torch.testing.assert_close(sa, sb, atol=0, rtol=1e-6)
+    r1, r2 = r.clone(), r.clone()
+    got, res = ops.fused_add_rmsnorm(sums(), r1, weight, 1e-5)
+    want, _ = ops.fused_add_rmsnorm(y.clone(), r2, weight, 1e-5)
+    assert res is r1 and torch.equal(r1, r2)
+    near(got, want, 2.0 ** -7)
+    r1, r2 = r.clone(), r.clone()
+    (a, sa), (b, sb) = (ops.fused_add_rmsnorm_fp8(sums(), r1, weight, 1e-5),
+                        ops.fused_add_rmsnorm_fp8(y, r2, weight, 1e-5))
+    near(a, b, 2.0 ** -3)
+    torch.testing.assert_close(sa, sb, atol=0, rtol=1e-6)
+    assert torch.equal(r1, r2)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("cache", [torch.bfloat16, torch.float8_e5m2])
+def test_rope_of_product_sums(fp8, cache):
+    from kubeai_amd import _C
+
+    T, nq, nkv, hd, K = 21, 6, 2, 64, 1024
+    width = (nq + 2 * nkv) * hd
+    x, w = _x(T, K), _x(width, K) * 0.05
+    sx = sw = None
+    if fp8:
+        x, w = x.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn)
+        sx, sw = torch.rand(T, device=DEV) + 0.5, torch.rand(width, device=DEV) + 0.5
+    y = torch.empty(T, width, device=DEV, dtype=torch.bfloat16)
+    _C.skinny_linear(y, x, w, sx, sw, None)
+    pos = torch.randint(0, 900, (T,), device=DEV, dtype=torch.int32)
+    slots = torch.randperm(32, device=DEV)[:T]
+    slots[2] = -1
+    cs = ref.make_cos_sin_cache(hd, 1000).to(DEV)
+    one = [torch.zeros(2, nkv, 16, hd, device=DEV).to(cache) for _ in range(2)]
+    two = [c.clone() for c in one]
+    q = ops.rope_and_cache(ops.product_sums(x, w, sx, sw), nq, pos, cs, *one, slots)
+    q2 = ops.rope_and_cache(y, nq, pos, cs, *two, slots)
+    assert q.is_contiguous()
+    step = 2.0 ** -7 if cache == torch.bfloat16 else 2.0 ** -2  # see above
+    for a, b, rtol in [(q, q2, 2.0 ** -7)] + [(a, b, step) for a, b in zip(one, two)]:
+        a, b = a.float(), b.float()
+        assert (a != b).sum().item() <= 2 + a.numel() // 1000
+        torch.testing.assert_close(a, b, atol=1e-6, rtol=rtol)
+
+
+def test_linear_routes_agree():
+    """Shapes on both sides of every rule, against the library's product."""
+    for M, N, K in [(1, 16384, 64), (16, 16384, 64), (17, 16384, 64), (3, 16368, 64),
+                    (96, 1024, 16384), (97, 1024, 16384), (5, 2048, 16384), (8, 65552, 64)]:
+        x, w = _x(M, K), _x(N, K) * K ** -0.5
+        want = torch.nn.functional.linear(x.float(), w.float())
+        torch.testing.assert_close(ops.linear(x, w).float(), want, atol=2e-3, rtol=2.0 ** -7)
+        x8, w8 = x.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn)
+        sx, sw = torch.rand(M, device=DEV) + 0.5, torch.rand(1, N, device=DEV) + 0.5
+        b = torch.randn(N, device=DEV, dtype=torch.bfloat16)
+        want = torch.nn.functional.linear(x8.float(), w8.float()) * sx[:, None] * sw + b.float()
+        got = ops.linear_fp8(x8, sx, w8, sw, b)
+        # the library adds the bias in fp32 or after rounding, as it likes
+        torch.testing.assert_close(got.float(), want, atol=2e-2, rtol=2.0 ** -7)
