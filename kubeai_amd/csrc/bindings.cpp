@@ -14,6 +14,8 @@ void rope_cache(torch::Tensor qkv, torch::Tensor positions,
                 c10::optional<torch::Tensor> sx,
                 c10::optional<torch::Tensor> sw);
 torch::Tensor skinny_sums(torch::Tensor x, torch::Tensor w);
+void quant_fp8_rows(torch::Tensor out, torch::Tensor out_scale, torch::Tensor x,
+                    torch::Tensor src);
 void rmsnorm_sums(torch::Tensor out, c10::optional<torch::Tensor> out_scale,
                   torch::Tensor part, c10::optional<torch::Tensor> sx,
                   c10::optional<torch::Tensor> sw,
@@ -103,6 +105,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_experts", &skinny_experts,
         "weight-streaming product of each expert's rows");
   m.def("skinny_sums", &skinny_sums, "fp32 part sums of a skinny product");
+  m.def("quant_fp8_rows", &quant_fp8_rows, "gathered bf16 rows -> fp8");
   m.def("rmsnorm_sums", &rmsnorm_sums, "norm of a product's part sums");
   m.def("moe_route", &moe_route,
         "router scores, top-k weights and tokens in expert order");

@@ -144,15 +144,18 @@ __launch_bounds__(VPT == 8 ? 512 : 1024) __global__ void rmsnorm_kernel(
     write_fp8_row<VPT>((unsigned char*)out, out_scale, row, vals, amax, H, red[1]);
 }
 
-// SILU: silu(gate) * up of packed [T, 2H] rows, else the rows as they are
+// SILU: silu(gate) * up of packed [T, 2H] rows, else the rows as they are.
+// src: row i is row src[i] of the input.
 template <bool SILU, int VPT>
 __launch_bounds__(VPT == 8 ? 512 : 1024) __global__ void to_fp8_kernel(
     unsigned char* __restrict__ out, float* __restrict__ out_scale,
-    const ushort* __restrict__ xin, const int H) {
+    const ushort* __restrict__ xin, const int32_t* __restrict__ src,
+    const int H) {
   const int64_t row = blockIdx.x;
   const int nvec = H / 8;
+  const int64_t from = src ? src[row] : row;
   const ushort8* xr =
-      reinterpret_cast<const ushort8*>(xin + row * (SILU ? 2 : 1) * H);
+      reinterpret_cast<const ushort8*>(xin + from * (SILU ? 2 : 1) * H);
   __shared__ float red[16];
   float vals[VPT][8];
   float amax = 0.f;
@@ -225,7 +228,8 @@ void launch_norm(void* out, float* out_scale, const ushort* x, int64_t T, int H,
 
 template <bool SILU>
 void launch_to_fp8(torch::Tensor& out, torch::Tensor& out_scale,
-                   const torch::Tensor& x, int64_t T, int H) {
+                   const torch::Tensor& x, int64_t T, int H,
+                   const int32_t* src = nullptr) {
   if (T == 0) return;
   const Split s = split_for(T, H);
   with_vpt(s.vpt, [&](auto vpt) {
@@ -234,7 +238,7 @@ void launch_to_fp8(torch::Tensor& out, torch::Tensor& out_scale,
                        c10::hip::getCurrentHIPStream().stream(),
                        (unsigned char*)out.data_ptr(),
                        out_scale.data_ptr<float>(),
-                       (const ushort*)x.data_ptr(), H);
+                       (const ushort*)x.data_ptr(), src, H);
   });
   HIP_CHECK_KERNEL();
 }
@@ -285,6 +289,19 @@ void quant_fp8(torch::Tensor out, torch::Tensor out_scale, torch::Tensor x) {
   check_row_op(x, kMaxHFp8);
   const int H = x.size(-1);
   launch_to_fp8<false>(out, out_scale, x, x.numel() / H, H);
+}
+
+// rows of x in the order of src (int32, entries are rows of x), quantized
+void quant_fp8_rows(torch::Tensor out, torch::Tensor out_scale, torch::Tensor x,
+                    torch::Tensor src) {
+  check_row_op(x, kMaxHFp8);
+  TORCH_CHECK(x.dim() == 2 && src.scalar_type() == torch::kInt32 &&
+              src.is_contiguous() && src.is_cuda());
+  const int64_t n = src.numel();
+  TORCH_CHECK(out.is_contiguous() && out.numel() == n * x.size(1) &&
+              out.element_size() == 1 && out_scale.is_contiguous() &&
+              out_scale.numel() == n);
+  launch_to_fp8<false>(out, out_scale, x, n, x.size(1), src.data_ptr<int32_t>());
 }
 
 // the norms of a row that is still a product's parts: part fp32 [parts, T, H],

@@ -229,23 +229,35 @@ class MoEMLP(nn.Module):
     so decode steps can be recorded in a graph, and every expert's weights are
     read once, for its own rows only. The experts' weights lie behind one
     another in one tensor for that; the modules' parameters are views of it.
-    Larger steps gather each expert's rows and run its library GEMMs."""
+    Larger steps sort the rows by expert on the device, read the experts' row
+    counts once and run each expert's library products on its slice."""
 
-    #: one pass of 8 experts of 14336 (us, grouped / every expert through the
-    #: library): fp8 1 token 137/540, 40 297/542, 256 450/764, 512 831/1274;
-    #: bf16 40 561/822, 512 1403/1537, 768 1810/1699 (an expert's weights are
-    #: read again for every 96 of its rows)
-    GROUPED_MAX_TOKENS = 512
+    #: one pass of 8 experts of 14336, us, grouped / sorted / every expert's
+    #: tokens asked for one after the other: fp8 256 tokens 498/532/794, 320
+    #: 507/555/1378, 512 839/637/1301, 2048 2447/1274/2021; bf16 320
+    #: 802/914/1503, 512 1360/982/1558, 2048 4193/1893/2570 (grouped reads an
+    #: expert's weights again for every 96 of its rows)
+    GROUPED_MAX_TOKENS = 320
 
     def __init__(self, cfg: ModelArchConfig):
         super().__init__()
         self.n_experts = cfg.num_local_experts
         self.top_k = cfg.num_experts_per_tok
         self.gate = nn.Linear(cfg.hidden_size, self.n_experts, bias=False)
-        self.experts = nn.ModuleList([MLP(cfg) for _ in range(self.n_experts)])
+        with torch.device("meta"):  # their weights are views, made below
+            self.experts = nn.ModuleList([MLP(cfg) for _ in range(self.n_experts)])
         self.gelu = cfg.hidden_act == "gelu_pytorch_tanh"
-        self._stacks: dict = {}
-        self.stack_experts()
+        self._stacks = {
+            (proj, "weight"): torch.empty(
+                (self.n_experts,) + getattr(self.experts[0], proj).weight.shape
+            )
+            for proj in ("gate_up_proj", "down_proj")
+        }
+        for e, expert in enumerate(self.experts):
+            for proj in ("gate_up_proj", "down_proj"):
+                lin = getattr(expert, proj)
+                lin.weight = nn.Parameter(self._stacks[proj, "weight"][e])
+                lin.reset_parameters()
 
     def stack_experts(self) -> None:
         """Put the experts' weights (and fp8 scales) behind one another and
@@ -285,17 +297,54 @@ class MoEMLP(nn.Module):
             at += step
         return stack
 
-    def _grouped(self, x: torch.Tensor):
-        """All experts' rows at once; None where the kernels do not take it."""
-        if not (
+    def _on_device(self, x: torch.Tensor) -> bool:
+        """Whether csrc/moe.hip takes the routing of x."""
+        return (
             x.is_cuda
             and x.dtype == self.gate.weight.dtype == torch.bfloat16
             and x.is_contiguous()
-            and 1 <= x.shape[0] <= self.GROUPED_MAX_TOKENS
+            and x.shape[0] >= 1
+            and x.shape[1] % 8 == 0
             and self.n_experts <= 32
             and self.top_k <= 8
             and not torch.is_grad_enabled()
-        ):
+        )
+
+    def _sorted(self, x: torch.Tensor) -> torch.Tensor:
+        """Rows in expert order, a library product per expert and projection."""
+        weight, begin, src, place = ops.moe_route(x, self.gate.weight, self.top_k)
+        n = src.shape[0]
+        first = self.experts[0]
+        fp8 = hasattr(first.gate_up_proj, "forward_quantized")
+        rows = ops.quant_fp8_rows(x, src) if fp8 else x.index_select(0, src)
+        ends = begin.tolist()  # the step's one look at the routing per layer
+
+        def products(rows, proj, width):
+            y = torch.empty((n, width), dtype=x.dtype, device=x.device)
+            for e, expert in enumerate(self.experts):
+                lo, hi = ends[e], ends[e + 1]
+                if lo == hi:
+                    continue
+                lin = getattr(expert, proj)
+                if fp8:
+                    ops.linear_fp8(
+                        rows[0][lo:hi], rows[1][lo:hi], lin.weight_fp8,
+                        lin.weight_scale, lin.bias, out=y[lo:hi],
+                    )
+                else:
+                    torch.mm(rows[lo:hi], lin.weight.t(), out=y[lo:hi])
+            return y
+
+        h = products(rows, "gate_up_proj", 2 * first.down_proj.in_features)
+        if fp8:
+            a = ops.silu_and_mul_fp8(h)
+        else:
+            a = ops.gelu_and_mul(h) if self.gelu else ops.silu_and_mul(h)
+        return ops.moe_combine(products(a, "down_proj", x.shape[1]), place, weight)
+
+    def _grouped(self, x: torch.Tensor):
+        """All experts' rows at once; None where the kernels do not take it."""
+        if not (self._on_device(x) and x.shape[0] <= self.GROUPED_MAX_TOKENS):
             return None
         fp8 = ("down_proj", "weight_fp8") in self._stacks
         name = "weight_fp8" if fp8 else "weight"
@@ -319,6 +368,8 @@ class MoEMLP(nn.Module):
         out = self._grouped(x)
         if out is not None:
             return out
+        if x.shape[0] > 256 and self._on_device(x):
+            return self._sorted(x)
         T, H = x.shape
         router = F.linear(x.float(), self.gate.weight.float())  # [T, E]
         weights, selected = torch.topk(router, self.top_k, dim=-1)

@@ -272,22 +272,24 @@ def linear(x, weight):
     return torch.nn.functional.linear(x, weight)
 
 
-def linear_fp8(xq, x_scale, weight, w_scale, bias=None):
+def linear_fp8(xq, x_scale, weight, w_scale, bias=None, out=None):
     """(xq * x_scale) (weight * w_scale)^T + bias in bf16; xq [M, K] and weight
-    [N, K] e4m3, x_scale [M], w_scale [1, N]."""
+    [N, K] e4m3, x_scale [M], w_scale [1, N]; into `out` (dense rows) if given."""
     if (
         xq.shape[0] <= 96
         and _streams_better(xq.shape[0], *weight.shape)
         and _skinny_operands(xq, weight)
     ):
-        y = torch.empty(
-            (xq.shape[0], weight.shape[0]), dtype=torch.bfloat16, device=xq.device
-        )
-        _C.skinny_linear(y, xq, weight, x_scale.reshape(-1), w_scale.reshape(-1), bias)
-        return y
+        if out is None:
+            out = torch.empty(
+                (xq.shape[0], weight.shape[0]), dtype=torch.bfloat16, device=xq.device
+            )
+        _C.skinny_linear(out, xq, weight, x_scale.reshape(-1), w_scale.reshape(-1), bias)
+        return out
+    kw = {} if out is None else {"out": out}
     return torch._scaled_mm(
         xq, weight.t(), scale_a=x_scale.view(-1, 1), scale_b=w_scale, bias=bias,
-        out_dtype=torch.bfloat16,
+        out_dtype=torch.bfloat16, **kw,
     )
 
 
@@ -345,22 +347,48 @@ def quant_fp8(x):
     return out, scale
 
 
+def moe_route(x, router, top_k: int):
+    """GPU-only: fp32 router scores of x [T, H] (router [E, H], both bf16) and
+    the softmax over every token's top_k experts. Returns (weight fp32 [T, k],
+    begin int32 [E + 1], src, place int32 [T k]): rows begin[e]..begin[e + 1] of
+    the expert order are token src[row]'s, pair (t, j) is row place[t k + j]."""
+    _require_ext()
+    T, E, n = x.shape[0], router.shape[0], x.shape[0] * top_k
+    i32 = torch.empty(3 * n + E + 1, dtype=torch.int32, device=x.device)
+    index, src, place, begin = i32.split([n, n, n, E + 1])
+    weight = torch.empty((T, top_k), dtype=torch.float32, device=x.device)
+    _C.moe_route(index.view(T, top_k), weight, begin, src, place, x, router.detach())
+    return weight, begin, src, place
+
+
+def moe_combine(y, place, weight):
+    """GPU-only: sum over every token's experts of weight * row (expert order)."""
+    out = torch.empty((weight.shape[0], y.shape[1]), dtype=y.dtype, device=y.device)
+    _C.moe_combine(out, y, place, weight)
+    return out
+
+
+def quant_fp8_rows(x, src):
+    """GPU-only: quant_fp8 of the rows src (int32) of x."""
+    _require_ext()
+    out = torch.empty(
+        (src.shape[0], x.shape[1]), dtype=torch.float8_e4m3fn, device=x.device
+    )
+    scale = torch.empty(src.shape[0], dtype=torch.float32, device=x.device)
+    _C.quant_fp8_rows(out, scale, x, src)
+    return out, scale
+
+
 def moe_mlp(x, router, top_k: int, gate_up, down, gate_up_scale=None, down_scale=None,
             gelu: bool = False):
     """GPU-only: sparse mixture of gated experts. x [T, H], router [E, H] (both
     bf16), gate_up [E, 2I, H] and down [E, H, I] in bf16, or fp8 with scales per
     output column (x is then quantized once, every expert's activations once).
     Router scores, weights and the sum over a token's experts are fp32."""
-    _require_ext()
-    T, H = x.shape
-    E, n = router.shape[0], T * top_k
-    i32 = torch.empty(3 * n + E + 1, dtype=torch.int32, device=x.device)
-    index, src, place, begin = i32.split([n, n, n, E + 1])
-    index = index.view(T, top_k)
-    weight = torch.empty((T, top_k), dtype=torch.float32, device=x.device)
-    _C.moe_route(index, weight, begin, src, place, x, router.detach())
+    weight, begin, src, place = moe_route(x, router, top_k)
+    n = src.shape[0]
     h = torch.empty((n, gate_up.shape[1]), dtype=torch.bfloat16, device=x.device)
-    y = torch.empty((n, H), dtype=torch.bfloat16, device=x.device)
+    y = torch.empty((n, x.shape[1]), dtype=torch.bfloat16, device=x.device)
     if gate_up_scale is not None:
         _C.skinny_experts(h, *_with_scale(quant_fp8(x), gate_up, gate_up_scale), begin, src)
         _C.skinny_experts(y, *_with_scale(silu_and_mul_fp8(h), down, down_scale), begin, None)
@@ -368,9 +396,7 @@ def moe_mlp(x, router, top_k: int, gate_up, down, gate_up_scale=None, down_scale
         _C.skinny_experts(h, x, gate_up, None, None, begin, src)
         a = gelu_and_mul(h) if gelu else silu_and_mul(h)
         _C.skinny_experts(y, a, down, None, None, begin, None)
-    out = torch.empty_like(x)
-    _C.moe_combine(out, y, place, weight)
-    return out
+    return moe_combine(y, place, weight)
 
 
 def _with_scale(quantized, weight, weight_scale):

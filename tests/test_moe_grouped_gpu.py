@@ -104,11 +104,12 @@ def test_module_routes():
     def both():
         grouped = m._grouped(x)
         assert grouped is not None
-        m.GROUPED_MAX_TOKENS = 0
+        m._on_device = lambda x: False
         one_by_one = m(x)
-        del m.GROUPED_MAX_TOKENS
+        del m._on_device
         # the per-expert route rounds weights and partial sums to bf16
         assert (grouped - one_by_one).float().norm() < 0.02 * one_by_one.float().norm()
+        _close(m._sorted(x), grouped)  # the same roundings, library products
         return grouped
 
     with torch.inference_mode():
@@ -124,4 +125,7 @@ def test_module_routes():
         both()
         m.experts[1].down_proj.weight_fp8 = m.experts[1].down_proj.weight_fp8.clone()
         assert m._grouped(x) is None
+        big = torch.randn(700, 256, device=DEV, dtype=torch.bfloat16)
+        many, few = m(big)[:37].float(), m(big[:37].contiguous()).float()
+        assert (many - few).norm() < 0.02 * few.norm()  # sorted, and per expert
     assert PRESETS["mixtral-8x7b"].num_local_experts <= 32
