@@ -46,6 +46,11 @@ void skinny_experts(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                     c10::optional<torch::Tensor> sx,
                     c10::optional<torch::Tensor> sw, torch::Tensor begin,
                     c10::optional<torch::Tensor> src);
+void grouped_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
+                    c10::optional<torch::Tensor> sx,
+                    c10::optional<torch::Tensor> sw, torch::Tensor bounds,
+                    c10::optional<torch::Tensor> src,
+                    c10::optional<torch::Tensor> square);
 void moe_route(torch::Tensor index, torch::Tensor weight, torch::Tensor begin,
                torch::Tensor src, torch::Tensor place, torch::Tensor x,
                torch::Tensor w);
@@ -104,6 +109,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_gemm", &skinny_gemm, "weight-streaming product, bf16");
   m.def("skinny_experts", &skinny_experts,
         "weight-streaming product of each expert's rows");
+  m.def("grouped_linear", &grouped_linear,
+        "all experts' products of a large step, bf16 or fp8 e4m3");
   m.def("skinny_sums", &skinny_sums, "fp32 part sums of a skinny product");
   m.def("quant_fp8_rows", &quant_fp8_rows, "gathered bf16 rows -> fp8");
   m.def("rmsnorm_sums", &rmsnorm_sums, "norm of a product's part sums");

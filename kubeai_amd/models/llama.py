@@ -229,15 +229,18 @@ class MoEMLP(nn.Module):
     so decode steps can be recorded in a graph, and every expert's weights are
     read once, for its own rows only. The experts' weights lie behind one
     another in one tensor for that; the modules' parameters are views of it.
-    Larger steps sort the rows by expert on the device, read the experts' row
-    counts once and run each expert's library products on its slice."""
+    Larger steps sort the rows by expert on the device; a projection is one
+    tiled product for all experts (csrc/grouped_gemm.hip) or, where that is the
+    slower one, the library's on each expert's slice, after one look at the
+    experts' row counts."""
 
-    #: one pass of 8 experts of 14336, us, grouped / sorted / every expert's
-    #: tokens asked for one after the other: fp8 256 tokens 498/532/794, 320
-    #: 507/555/1378, 512 839/637/1301, 2048 2447/1274/2021; bf16 320
-    #: 802/914/1503, 512 1360/982/1558, 2048 4193/1893/2570 (grouped reads an
-    #: expert's weights again for every 96 of its rows)
-    GROUPED_MAX_TOKENS = 320
+    #: one pass of 8 experts of 14336, us, weight-streaming / tiled / every
+    #: expert's tokens asked for one after the other: fp8 128 tokens
+    #: 358/387/722, 256 447/411/743, 512 819/470/1361, 2048 2413/1015/2006;
+    #: bf16 128 617/690/1159, 256 734/731/1221, 512 1397/871/1614, 2048
+    #: 4223/1708/2488 (streaming reads an expert's weights again for every 96
+    #: of its rows). Up to 256 tokens any routing may be recorded in a graph.
+    GROUPED_MAX_TOKENS = 256
 
     def __init__(self, cfg: ModelArchConfig):
         super().__init__()
@@ -311,15 +314,30 @@ class MoEMLP(nn.Module):
         )
 
     def _sorted(self, x: torch.Tensor) -> torch.Tensor:
-        """Rows in expert order, a library product per expert and projection."""
+        """Rows in expert order, one product per projection for all experts, or
+        the library's for one after the other."""
         weight, begin, src, place = ops.moe_route(x, self.gate.weight, self.top_k)
         n = src.shape[0]
         first = self.experts[0]
         fp8 = hasattr(first.gate_up_proj, "forward_quantized")
-        rows = ops.quant_fp8_rows(x, src) if fp8 else x.index_select(0, src)
-        ends = begin.tolist()  # the step's one look at the routing per layer
+        ends = None
 
-        def products(rows, proj, width):
+        def products(rows, proj, width, src=None):
+            nonlocal ends
+            rows, scale = rows if fp8 else (rows, None)
+            w = self._stack(proj, "weight_fp8" if fp8 else "weight")
+            ws = self._stack(proj, "weight_scale") if fp8 else None
+            if (
+                w is not None and (ws is not None) == fp8
+                and ops.grouped_linear_takes(rows, w) and ops.grouped_linear_better(n, w)
+            ):
+                return ops.grouped_linear(
+                    rows, w, begin, src=src, scales=(scale, ws) if fp8 else None
+                )
+            if src is not None:
+                rows = rows.index_select(0, src)
+            if ends is None:
+                ends = begin.tolist()
             y = torch.empty((n, width), dtype=x.dtype, device=x.device)
             for e, expert in enumerate(self.experts):
                 lo, hi = ends[e], ends[e + 1]
@@ -328,17 +346,19 @@ class MoEMLP(nn.Module):
                 lin = getattr(expert, proj)
                 if fp8:
                     ops.linear_fp8(
-                        rows[0][lo:hi], rows[1][lo:hi], lin.weight_fp8,
+                        rows[lo:hi], scale[lo:hi], lin.weight_fp8,
                         lin.weight_scale, lin.bias, out=y[lo:hi],
                     )
                 else:
                     torch.mm(rows[lo:hi], lin.weight.t(), out=y[lo:hi])
             return y
 
-        h = products(rows, "gate_up_proj", 2 * first.down_proj.in_features)
+        width = 2 * first.down_proj.in_features
         if fp8:
+            h = products(ops.quant_fp8_rows(x, src), "gate_up_proj", width)
             a = ops.silu_and_mul_fp8(h)
         else:
+            h = products(x, "gate_up_proj", width, src)
             a = ops.gelu_and_mul(h) if self.gelu else ops.silu_and_mul(h)
         return ops.moe_combine(products(a, "down_proj", x.shape[1]), place, weight)
 

@@ -651,24 +651,35 @@ class GeluMLP(nn.Module):
 
 
 class ExpertRows:
-    """The tokens of a large step gathered by expert: rows of one buffer, so
-    that everything but the products themselves is one launch for all
-    experts. The row counts come to the host (the products need shapes)."""
+    """The tokens of a large step in expert order: rows of one buffer, so that
+    each product and each pass between them is one launch for all experts, and
+    the row counts stay on the device. Where the products are the library's
+    (types and sizes that csrc/grouped_gemm.hip does not take or is slower for)
+    there is one per expert, and the counts come to the host: they need shapes."""
 
     def __init__(self, h, index, weights, experts: int):
-        tok, self.weight, self.place, counts = sops.expert_order(index, weights, experts)
-        self.h = h.index_select(0, tok)
-        self.counts = counts.tolist()
+        self.h = h
+        self.token, self.weight, self.place, self.counts = sops.expert_order(
+            index, weights, experts)
 
-    def products(self, x, weight_of, n_out: int):
-        """x's rows of expert e times weight_of(e) ([n_out, in]), for all e."""
-        y = torch.empty((x.shape[0], n_out), dtype=x.dtype, device=x.device)
+    def products(self, x, w, square: bool = False):
+        """Every expert's rows (of the tokens if x is None, else of x) times its
+        matrix in w [experts, out, in]; square: then relu(.)^2 * weight."""
+        src = self.token if x is None else None
+        rows = self.h if x is None else x
+        if ops.grouped_linear_takes(rows, w) and ops.grouped_linear_better(
+                self.token.shape[0], w):
+            return ops.grouped_linear(rows, w, self.counts, src=src,
+                                      square=self.weight if square else None)
+        if x is None:
+            rows = rows.index_select(0, src)
+        y = torch.empty((rows.shape[0], w.shape[1]), dtype=rows.dtype, device=rows.device)
         s = 0
-        for e, n in enumerate(self.counts):
+        for e, n in enumerate(self.counts.tolist()):
             if n:
-                torch.mm(x[s : s + n], weight_of(e).t(), out=y[s : s + n])
+                torch.mm(rows[s : s + n], w[e].t(), out=y[s : s + n])
                 s += n
-        return y
+        return sops.relu_squared_weighted(y, self.weight, w.shape[1]) if square else y
 
 
 class RoutedSquaredReluMoE(nn.Module):
@@ -681,8 +692,8 @@ class RoutedSquaredReluMoE(nn.Module):
     run them as two GEMMs over every expert with the routing weight (0 for
     experts a token did not choose) folded into the activation, so the sum
     over experts happens inside the second GEMM's fp32 accumulation and the
-    step has no data-dependent shapes. Large steps gather each expert's
-    tokens and run its slice of the stacked matrices."""
+    step has no data-dependent shapes. Large steps put the tokens in expert
+    order and multiply each expert's by its slice of the stacked matrices."""
 
     DENSE_MAX_TOKENS = 256
 
@@ -705,9 +716,8 @@ class RoutedSquaredReluMoE(nn.Module):
             a = sops.relu_squared_weighted(self.up(h), dense, ff)
             return self.down(a)
         rows = ExpertRows(h, idx, w, E)
-        u = rows.products(rows.h, lambda e: self.up.weight[e * ff : (e + 1) * ff], ff)
-        a = sops.relu_squared_weighted(u, rows.weight, ff)
-        y = rows.products(a, lambda e: self.down.weight[:, e * ff : (e + 1) * ff], h.shape[1])
+        a = rows.products(None, self.up.weight[: E * ff].unflatten(0, (E, ff)), square=True)
+        y = rows.products(a, self.down.weight[:, : E * ff].unflatten(1, (E, ff)).transpose(0, 1))
         shared = None
         if self.shared_ff:
             u = F.linear(h, self.up.weight[E * ff :])
@@ -787,10 +797,9 @@ class RoutedGatedMoE(nn.Module):
             y = self.down(a)
             return (y, gu[:, at:]) if self.extra_out else y
         rows = ExpertRows(h, idx, w, E)
-        gu = rows.products(rows.h, lambda e: self.gate_up.weight[e * 2 * ff : (e + 1) * 2 * ff],
-                           2 * ff)
+        gu = rows.products(None, self.gate_up.weight[: E * 2 * ff].unflatten(0, (E, 2 * ff)))
         a = sops.glu_weighted(gu, rows.weight, ff, w_input=self.w_input, **self.act)
-        y = rows.products(a, lambda e: self.down.weight[:, e * ff : (e + 1) * ff], h.shape[1])
+        y = rows.products(a, self.down.weight[:, : E * ff].unflatten(1, (E, ff)).transpose(0, 1))
         shared = None
         extra = None
         if sff or self.extra_out:

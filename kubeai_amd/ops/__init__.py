@@ -399,6 +399,52 @@ def moe_mlp(x, router, top_k: int, gate_up, down, gate_up_scale=None, down_scale
     return moe_combine(y, place, weight)
 
 
+def grouped_linear_takes(x, w) -> bool:
+    """Whether grouped_linear multiplies rows like x by w [E, N, K] of x's type."""
+    es = x.element_size()
+    return (
+        x.is_cuda
+        and _C is not None
+        and x.dtype == w.dtype
+        and x.dtype in (torch.bfloat16, torch.float8_e4m3fn)
+        and x.stride(1) == w.stride(2) == 1
+        and w.shape[2] * es % 128 == 0
+        and w.shape[1] % 4 == 0
+        and 0 < w.shape[0] < 65536
+        and x.stride(0) * es % 16 == w.stride(0) * es % 16 == w.stride(1) * es % 16 == 0
+        and x.stride(0) >= w.shape[2] <= w.stride(1)
+        and x.data_ptr() % 16 == w.data_ptr() % 16 == 0
+        and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
+    )
+
+
+def grouped_linear_better(n: int, w) -> bool:
+    """Whether n rows of w's experts are better multiplied by grouped_linear than
+    by a library product per expert. fp8: always (8 experts, 512 rows each, us,
+    grouped / library: 28672 x 4096 609/686, 4096 x 14336 354/474; 2048 rows
+    1963/1892 and 1016/1127, without the look at the routing from the host). bf16: unless
+    every expert's product fills the chip by itself (3584 x 2048, 768 rows
+    107/171, 2048 rows 260/283; 4096 x 14336, 1024 rows 1063/1106, 2048 rows
+    2144/1857; 28672 x 4096, 64 rows 398/428, 128 rows 551/468, 512 1139/955)."""
+    mean, cols = n / w.shape[0], w.shape[1] / 256
+    return w.element_size() == 1 or mean <= 96 or (
+        cols <= 64 and (mean / 256) * cols < 120
+    )
+
+
+def grouped_linear(x, w, bounds, src=None, scales=None, square=None):
+    """GPU-only: rows of x [*, K] in expert order times their expert's matrix,
+    w [E, N, K] (any strides of e and n), all experts in one launch. bounds int32:
+    the experts' row counts [E] or offsets [E + 1]; src int32: the rows of x
+    (all, in order). fp8 x and w: scales = (fp32 per row of x, [E, N]). square
+    (fp32 per row): relu(product)^2 * square instead of the product."""
+    _require_ext()
+    n = x.shape[0] if src is None else src.shape[0]
+    y = torch.empty((n, w.shape[1]), dtype=torch.bfloat16, device=x.device)
+    _C.grouped_linear(y, x, w, *(scales or (None, None)), bounds, src, square)
+    return y
+
+
 def _with_scale(quantized, weight, weight_scale):
     xq, xs = quantized
     return xq, weight, xs, weight_scale
