@@ -13,15 +13,19 @@
 //    tokens are kept, as fp32 partial sums per input range. 16 tokens share
 //    each A byte; splitting the inputs gives 14336-wide inputs 14 workgroups
 //    per 16 tokens.
-//  - lora_expand: workgroup = 16 tokens x 512 outputs (2 a thread). B rows
-//    are held in registers and used for the adapter's tokens; the products
-//    stay fp32 x fp32 on the vector ALUs (v is not rounded; 2 R flops per
-//    element of y, which is read and written once, is below the memory time).
-// It is bound by reading and writing y, and at decode sizes by the launches.
+//  - lora_expand: workgroup = 16 tokens x 256 outputs, on the matrix cores:
+//    B rows are bf16 as they are, v (fp32) is cut into three bf16 parts that
+//    add up to it exactly, and a token keeps its own adapter's result. A lane
+//    holds 16 neighbouring outputs of one token (32: 27 us for 28672 outputs
+//    instead of 22, too few waves in flight).
+// Both are bound by latency: a few dependent loads (ids and table, entry, v, B)
+// and a launch each. So the table is searched in registers, one load for all
+// its ids, and x and y are asked for before anything is known about them.
 // 4 adapters of rank 16, 28 decode rows and 304 prompt tokens (384 padded),
-// us for shrink + expand: 4096 -> 4096 9 + 16, 4096 -> 28672 9 + 22, 14336 ->
-// 4096 11 + 16; one launch per adapter took 4 x 59 each, and finding the
-// adapters present four synchronisations.
+// us for shrink + expand: 4096 -> 4096 9 + 9.5, 4096 -> 28672 9 + 22, 14336 ->
+// 4096 10 + 9 (expand 16, 22 and 16 with a search per thread, the vector ALUs
+// and y read last); one launch per adapter took 4 x 59 each, and finding the adapters
+// present four synchronisations.
 //
 // sgmv applies one adapter to the rows that `idx` names (the form for
 // adapters that the table does not take, see engine/lora.py). Design:
@@ -85,6 +89,7 @@ __global__ void sgmv_kernel(
 // ---- the whole batch ---------------------------------------------------
 constexpr int kTok = 16;      // tokens per workgroup
 constexpr int kShrinkK = 1024;  // inputs per shrink workgroup
+constexpr int kLaneOut = 16;    // outputs per expand lane
 
 typedef __attribute__((ext_vector_type(8))) short bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -99,15 +104,17 @@ struct LoraEntry {
 };
 static_assert(sizeof(LoraEntry) == 32, "the host builds rows of 4 int64");
 
-// table row of every token's adapter (-1: base model or not loaded)
-DEV_INLINE int lora_slot(const LoraEntry* tab, int n, const int32_t* ids,
-                         int64_t t, int64_t T) {
-  if (t >= T) return -1;
-  const int id = ids[t];
-  if (id == 0) return -1;
-  for (int i = 0; i < n; ++i)
-    if (tab[i].id == id) return i;
-  return -1;
+// table row of the adapter id of every lane (-1: base model or not loaded);
+// all lanes take part
+DEV_INLINE int lora_slot(const LoraEntry* tab, int n, int id) {
+  const int lane = threadIdx.x % WAVE_SIZE;
+  int slot = -1;
+  for (int base = 0; base < n; base += WAVE_SIZE) {
+    const int here = base + lane < n ? tab[base + lane].id : 0;
+    for (int i = 0; i < min(n - base, WAVE_SIZE); ++i)
+      if (__builtin_amdgcn_readlane(here, i) == id && slot < 0) slot = base + i;
+  }
+  return id == 0 ? -1 : slot;
 }
 
 __global__ __launch_bounds__(kBlock) void lora_shrink_kernel(
@@ -124,10 +131,7 @@ __global__ __launch_bounds__(kBlock) void lora_shrink_kernel(
   const int m = lane & 15, kg = lane >> 4;
   __shared__ float red[NW][kTok][kTok + 1];
 
-  const int slot = lora_slot(tab, n, ids, t0 + m, T);
-  uint64_t todo = __ballot(slot >= 0) & 0xffffull;
-  if (todo == 0) return;  // the same in every wave
-
+  const int id = t0 + m < T ? ids[t0 + m] : 0;
   const int k0 = split * kShrinkK + wave * (kShrinkK / NW) + kg * 8;
   const ushort* xr = x + min(t0 + m, T - 1) * x_stride;
   bf16x8 xf[STEPS];
@@ -136,6 +140,9 @@ __global__ __launch_bounds__(kBlock) void lora_shrink_kernel(
     const int k = k0 + i * 32;  // H is a multiple of 8
     xf[i] = k < H ? *reinterpret_cast<const bf16x8*>(xr + k) : bf16x8{};
   }
+  const int slot = lora_slot(tab, n, id);
+  uint64_t todo = __ballot(slot >= 0) & 0xffffull;
+  if (todo == 0) return;  // the same in every wave
   while (todo) {
     const int cur = __builtin_amdgcn_readlane(slot, __builtin_ctzll(todo));
     todo &= (todo - 1) & ~__ballot(slot == cur);  // shrinks in any case
@@ -171,89 +178,120 @@ __global__ __launch_bounds__(kBlock) void lora_shrink_kernel(
   }
 }
 
-// COLS: outputs per thread (2 where rows of y are 4-byte aligned)
-template <int COLS>
+// VEC: rows of y are whole 16-byte units
+template <bool VEC>
 __global__ __launch_bounds__(kBlock) void lora_expand_kernel(
     ushort* __restrict__ y,          // [T, out] +=, rows strided
     const float* __restrict__ part,  // [splits, T, r_pad]
     const LoraEntry* __restrict__ tab, const int n,
     const int32_t* __restrict__ ids, const int64_t T, const int out,
     const int64_t y_stride, const int r_pad, const int splits) {
+  constexpr int kTiles = kLaneOut / 4;
   const int64_t t0 = (int64_t)blockIdx.x * kTok;
-  const int lane = threadIdx.x % WAVE_SIZE;
-  __shared__ float v[kTok][kMaxR];
+  const int wave = threadIdx.x / WAVE_SIZE, lane = threadIdx.x % WAVE_SIZE;
+  const int m = lane & 15, kg = lane >> 4;
+  __shared__ __attribute__((aligned(16))) float v[kTok][kMaxR + 4];
 
-  const int slot = lora_slot(tab, n, ids, t0 + (lane & 15), T);
-  uint64_t todo = __ballot(slot >= 0) & 0xffffull;
-  const uint32_t active = (uint32_t)todo;
-  if (todo == 0) return;
-
-  for (int i = threadIdx.x; i < kTok * r_pad; i += kBlock) {
-    const int tok = i / r_pad, r = i % r_pad;
-    const int own = lora_slot(tab, n, ids, t0 + tok, T);
-    float s = 0.f;
-    if (own >= 0 && r < tab[own].rank) {
-      for (int k = 0; k < splits; ++k)
-        s += part[((int64_t)k * T + t0 + tok) * r_pad + r];
-      s *= tab[own].scale;
+  const int id = t0 + m < T ? ids[t0 + m] : 0;
+  // this lane's outputs of token m
+  const int wave_out = (blockIdx.y * (kBlock / WAVE_SIZE) + wave) * 4 * kLaneOut;
+  const int o0 = wave_out + kg * kLaneOut;
+  ushort* yr = y + min(t0 + m, T - 1) * y_stride + o0;
+  ushort8 old[kLaneOut / 8];
+  if constexpr (VEC) {
+#pragma unroll
+    for (int q = 0; q < kLaneOut / 8; ++q) {
+      old[q] = ushort8{};
+      if (id != 0 && o0 + 8 * q < out) old[q] = *reinterpret_cast<ushort8*>(yr + 8 * q);
     }
-    v[tok][r] = s;
+  }
+  const int slot = lora_slot(tab, n, id);
+  uint64_t todo = __ballot(slot >= 0) & 0xffffull;
+  if (todo == 0) return;  // the same in every wave
+  const int rank = slot >= 0 ? tab[slot].rank : 0;
+  const float scale = slot >= 0 ? tab[slot].scale : 0.f;
+
+  const int cols = r_pad <= 32 ? 32 : kMaxR;  // whole steps of K
+  for (int i = threadIdx.x; i < kTok * cols; i += kBlock) {
+    const int tok = i / cols, r = i % cols;
+    const bool own = r < __shfl(rank, tok);
+    const float* from = part + (t0 + tok) * r_pad + r;
+    float s = 0.f;
+#pragma unroll 4
+    for (int k = 0; k < splits; ++k)
+      s += own ? from[(int64_t)k * T * r_pad] : 0.f;
+    v[tok][r] = s * __shfl(scale, tok);
   }
   __syncthreads();
 
-  // lanes past the last output stay: the ballots below need every token's lane
-  const int o_own = (blockIdx.y * kBlock + threadIdx.x) * COLS;
-  const bool live = o_own < out;
-  const int o = live ? o_own : 0;
-  float acc[kTok][COLS];
+  f32x4 acc[kTiles];
 #pragma unroll
-  for (int i = 0; i < kTok; ++i)
-#pragma unroll
-    for (int c = 0; c < COLS; ++c) acc[i][c] = 0.f;
+  for (int j = 0; j < kTiles; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
   while (todo) {
     const int cur = __builtin_amdgcn_readlane(slot, __builtin_ctzll(todo));
-    const uint32_t mine = (uint32_t)(__ballot(slot == cur) & todo);
-    todo &= (todo - 1) & ~(uint64_t)mine;  // shrinks in any case
+    todo &= (todo - 1) & ~__ballot(slot == cur);  // shrinks in any case
     const ushort* B = tab[cur].B;
     const int R = tab[cur].rank;
-    for (int r0 = 0; r0 < R; r0 += 8) {
-      float b[COLS][8];
+    f32x4 sum[kTiles];  // of all tokens; kept for the adapter's own
 #pragma unroll
-      for (int c = 0; c < COLS; ++c) {
-        const ushort* br = B + (int64_t)(o + c) * R + r0;
+    for (int j = 0; j < kTiles; ++j) sum[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < R; k0 += 32) {
+      const int k = k0 + kg * 8;
+      bf16x8 b[kTiles];
+#pragma unroll
+      for (int j = 0; j < kTiles; ++j) {
+        // row m of tile j: outputs 4 j .. 4 j + 3 of every lane's 16
+        const int o = wave_out + (m >> 2) * kLaneOut + j * 4 + (m & 3);
+        const ushort* br = B + (int64_t)min(o, out - 1) * R + k;
+        b[j] = bf16x8{};
         if ((R & 7) == 0) {
-          const ushort8 bv = *reinterpret_cast<const ushort8*>(br);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) b[c][j] = bf16_to_f32(bv[j]);
+          if (k < R) b[j] = *reinterpret_cast<const bf16x8*>(br);
         } else {
 #pragma unroll
-          for (int j = 0; j < 8; ++j)
-            b[c][j] = r0 + j < R ? bf16_to_f32(br[j]) : 0.f;
+          for (int e = 0; e < 8; ++e)
+            if (k + e < R) b[j][e] = (short)br[e];
+        }
+      }
+      // v in three parts of 8 bits each, cut off: their sum is v
+      bf16x8 part3[3];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float rest = v[m][k + e];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+          const uint32_t top = __float_as_uint(rest) & 0xffff0000u;
+          part3[p][e] = (short)(top >> 16);
+          // nothing is left of infinities and NaN
+          rest = (top & 0x7f800000u) == 0x7f800000u ? 0.f : rest - __uint_as_float(top);
         }
       }
 #pragma unroll
-      for (int i = 0; i < kTok; ++i) {
-        if (!(mine >> i & 1)) continue;  // the same in every lane
+      for (int j = 0; j < kTiles; ++j)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float vj = v[i][r0 + j];
-#pragma unroll
-          for (int c = 0; c < COLS; ++c) acc[i][c] = fmaf(b[c][j], vj, acc[i][c]);
-        }
-      }
+        for (int p = 2; p >= 0; --p)
+          sum[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], part3[p], sum[j], 0, 0, 0);
     }
-  }
 #pragma unroll
-  for (int i = 0; i < kTok; ++i) {
-    if (!live || !(active >> i & 1)) continue;
-    ushort* yp = y + (t0 + i) * y_stride + o;
-    if constexpr (COLS == 2) {
-      const uint32_t old = *reinterpret_cast<uint32_t*>(yp);
-      const uint32_t lo = f32_to_bf16(bf16_to_f32((ushort)old) + acc[i][0]);
-      const uint32_t hi = f32_to_bf16(bf16_to_f32((ushort)(old >> 16)) + acc[i][1]);
-      *reinterpret_cast<uint32_t*>(yp) = lo | (hi << 16);
+    for (int j = 0; j < kTiles; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[j][e] = slot == cur ? sum[j][e] : acc[j][e];
+  }
+  if (slot < 0) return;
+#pragma unroll
+  for (int q = 0; q < kLaneOut / 8; ++q) {
+    if constexpr (VEC) {
+      if (o0 + 8 * q >= out) continue;
+      ushort8 to;
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        to[e] = f32_to_bf16(bf16_to_f32(old[q][e]) + acc[2 * q + e / 4][e % 4]);
+      *reinterpret_cast<ushort8*>(yr + 8 * q) = to;
     } else {
-      *yp = f32_to_bf16(bf16_to_f32(*yp) + acc[i][0]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (o0 + 8 * q + e < out)
+          yr[8 * q + e] =
+              f32_to_bf16(bf16_to_f32(yr[8 * q + e]) + acc[2 * q + e / 4][e % 4]);
     }
   }
 }
@@ -289,20 +327,18 @@ void lora_apply(torch::Tensor y, torch::Tensor x, torch::Tensor table,
                      (const ushort*)x.data_ptr(), tab, n,
                      ids.data_ptr<int32_t>(), T, H, x.stride(0), r_pad);
   HIP_CHECK_KERNEL();
-  const bool pair = out % 2 == 0 && y.stride(0) % 2 == 0 &&
-                    ((uintptr_t)y.data_ptr() & 3) == 0;
-  const int cols = pair ? 2 : 1;
-  const dim3 grid(tiles, (out + kBlock * cols - 1) / (kBlock * cols));
-  if (pair)
-    hipLaunchKernelGGL((lora_expand_kernel<2>), grid, dim3(kBlock), 0, stream,
+  constexpr int kOut = kBlock / 16 * kLaneOut;  // outputs per workgroup
+  const dim3 grid(tiles, (out + kOut - 1) / kOut);
+  auto expand = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, stream,
                        (ushort*)y.data_ptr(), part.data_ptr<float>(), tab, n,
                        ids.data_ptr<int32_t>(), T, out, y.stride(0), r_pad,
                        splits);
+  };
+  if (out % 8 == 0 && y.stride(0) % 8 == 0 && ((uintptr_t)y.data_ptr() & 15) == 0)
+    expand(lora_expand_kernel<true>);
   else
-    hipLaunchKernelGGL((lora_expand_kernel<1>), grid, dim3(kBlock), 0, stream,
-                       (ushort*)y.data_ptr(), part.data_ptr<float>(), tab, n,
-                       ids.data_ptr<int32_t>(), T, out, y.stride(0), r_pad,
-                       splits);
+    expand(lora_expand_kernel<false>);
   HIP_CHECK_KERNEL();
 }
 

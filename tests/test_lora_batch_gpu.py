@@ -1,5 +1,5 @@
 """The batched LoRA kernels at the edges of their tiles: 16 tokens, 1024
-inputs and 16 ranks a workgroup of the first, 512 outputs of the second.
+inputs and 16 ranks a workgroup of the first, 256 outputs of the second.
 
 y is rounded to bf16 once (2^-9 of itself); the sums before are fp32 over at
 most 1100 + 64 terms (1100 * 2^-24 of the sum of magnitudes, far below)."""
@@ -49,6 +49,25 @@ def test_ranks_beside_each_other(rank):
 def test_sixteen_adapters_in_a_tile_and_strided_rows():
     _apply(32, 256, 300, {k + 1: 8 + k % 9 for k in range(16)}, list(range(1, 17)) * 2, y_pad=5)
     _apply(20, 256, 300, {1: 16}, [0] * 20)
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+def test_an_adapter_without_finite_weights_keeps_to_its_tokens(bad):
+    from kubeai_amd import _C
+
+    torch.manual_seed(1)
+    x = torch.randn(16, 64, device=DEV, dtype=torch.bfloat16)
+    A = torch.randn(2, 8, 64, device=DEV, dtype=torch.bfloat16)
+    B = torch.randn(2, 40, 8, device=DEV, dtype=torch.bfloat16)
+    A[1, 3, 5] = B[1, 7, 2] = bad
+    table = torch.tensor([[A[i].data_ptr(), B[i].data_ptr(), _two_words(8, i + 1),
+                           _float_word(1.0)] for i in range(2)], dtype=torch.int64, device=DEV)
+    ids = torch.tensor([1, 2] * 8, dtype=torch.int32, device=DEV)
+    y = torch.zeros(16, 40, device=DEV, dtype=torch.bfloat16)
+    _C.lora_apply(y, x, table, ids, 8)
+    want = (x[::2].double() @ A[0].double().T) @ B[0].double().T
+    torch.testing.assert_close(y[::2].double(), want, atol=1e-4, rtol=2.0 ** -8)
+    assert not y[1::2].isfinite().any()
 
 
 class _Cfg:
