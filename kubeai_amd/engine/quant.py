@@ -29,10 +29,12 @@ class Fp8Linear(nn.Module):
             self.register_buffer("bias", bias.detach().to(torch.bfloat16))
         else:
             self.bias = None
-        w = weight_bf16.detach().float()
-        w_amax = w.abs().amax(dim=1, keepdim=True).clamp_min(1e-6)  # [out,1]
+        w = weight_bf16.detach()
+        # the largest magnitude is exact in the weight's own type: half the
+        # bytes of a pass over fp32 copies
+        w_amax = w.abs().amax(dim=1, keepdim=True).float().clamp_min(1e-6)  # [out,1]
         w_scale = w_amax / FP8_MAX
-        wq = (w / w_scale).clamp(-FP8_MAX, FP8_MAX).to(FP8_DTYPE)
+        wq = (w.float() / w_scale).clamp_(-FP8_MAX, FP8_MAX).to(FP8_DTYPE)
         # scaled_mm wants mat2 column-major: keep [out, in] row-major and
         # pass .t() (a column-major view) at call time
         self.register_buffer("weight_fp8", wq.contiguous())
