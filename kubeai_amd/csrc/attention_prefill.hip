@@ -72,17 +72,19 @@ typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
 
-// run s of the packed stream owns the tile numbers from start[s] / size + s
-// on (never fewer than it needs): T / size + n_seq numbers cover every batch
+// run s of the packed stream owns the tile numbers from (start[s] - start[0])
+// / size + s on (never fewer than it needs): T / size + n_seq numbers cover
+// every batch. The runs may be a part of a longer stream (start[0] > 0).
 DEV_INLINE int find_tile(const int32_t* start, int n_seq, int size, int n,
                          int* tile) {
+  const int base = start[0];
   int lo = 0, hi = n_seq - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (start[mid] / size + mid <= n) lo = mid;
+    if ((start[mid] - base) / size + mid <= n) lo = mid;
     else hi = mid - 1;
   }
-  *tile = n - (start[lo] / size + lo);
+  *tile = n - ((start[lo] - base) / size + lo);
   return lo;
 }
 

@@ -77,3 +77,29 @@ def test_negative_and_zero_scale():
 def test_wide_block_tables_and_many_short_runs():
     _run([16] * 70 + [200] + [1] * 30, [0] * 70 + [5] + [40] * 30, 8, 2, 128, 0.09,
          spare_blocks=40)
+
+
+@pytest.mark.parametrize("first,lens", [(100, [200]), (1, [40, 33, 0, 129]), (255, [1, 31, 300])])
+def test_runs_of_a_longer_stream(first, lens):
+    """Offsets that do not begin at 0: the rows before them are not touched."""
+    torch.manual_seed(first)
+    nq, nkv, hd, ctx = 8, 2, 128, 20
+    need = [(n + ctx + 15) // 16 for n in lens]
+    bt = torch.zeros(len(lens), max(need), dtype=torch.int32)
+    at = 1
+    for i, n in enumerate(need):
+        bt[i, :n] = torch.arange(at, at + n)
+        at += n
+    kc = torch.randn(at, nkv, 16, hd, device=DEV, dtype=torch.bfloat16)
+    vc = torch.randn_like(kc)
+    q = torch.randn(first + sum(lens), nq, hd, device=DEV, dtype=torch.bfloat16)
+    ends = [first + sum(lens[:i]) for i in range(len(lens) + 1)]
+    start = torch.tensor(ends, dtype=torch.int32, device=DEV)
+    total = torch.tensor([n + ctx for n in lens], dtype=torch.int32, device=DEV)
+    got = torch.full_like(q, 7.0)
+    ops.paged_attention_prefill(q, kc, vc, bt.to(DEV), start, total, 0.09, out=got)
+    want = ref.paged_attention_prefill(q[first:].float(), kc.float(), vc.float(), bt.to(DEV),
+                                       start - first, total, 0.09)
+    assert (got[:first] == 7.0).all()
+    torch.testing.assert_close(got[first:].float(), want, rtol=2 * 2.0 ** -9,
+                               atol=2 * 2.0 ** -9 * vc.float().abs().max().item())
