@@ -71,7 +71,8 @@ class Fp8Linear(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if (
             x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16
-            and x.is_contiguous() and x.shape[1] % 8 == 0 and x.shape[1] <= 32768
+            and x.is_contiguous() and ops.aligned(x)
+            and x.shape[1] % 8 == 0 and x.shape[1] <= 32768
         ):
             return self.forward_quantized(*ops.quant_fp8(x))
         a_amax = x.float().abs().amax(dim=-1, keepdim=True).clamp_min(1e-6)

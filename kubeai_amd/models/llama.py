@@ -307,9 +307,12 @@ class MoEMLP(nn.Module):
             and x.dtype == self.gate.weight.dtype == torch.bfloat16
             and x.is_contiguous()
             and x.shape[0] >= 1
+            and x.stride(0) == x.shape[1]  # (of a single row it may be anything)
             and x.shape[1] % 8 == 0
+            and self.gate.weight.is_contiguous()
+            and ops.aligned(x, self.gate.weight)
             and self.n_experts <= 32
-            and self.top_k <= 8
+            and self.top_k <= min(8, self.n_experts)
             and not torch.is_grad_enabled()
         )
 

@@ -209,6 +209,12 @@ class ProductSums:
         return self.part, self.x_scale, self.w_scale
 
 
+def aligned(*tensors) -> bool:
+    """Whether kernels may read the tensors' storage 16 bytes at a time. (A slice
+    that counts as contiguous can begin anywhere.)"""
+    return all(t.data_ptr() % 16 == 0 for t in tensors)
+
+
 def _skinny_operands(x, weight) -> bool:
     """Operands that the weight-streaming product takes."""
     return (
@@ -220,6 +226,9 @@ def _skinny_operands(x, weight) -> bool:
         and 1 <= x.shape[0] <= 96
         and x.is_contiguous()
         and weight.is_contiguous()
+        # (the stride of a single row may be anything)
+        and x.stride(0) == x.shape[1]
+        and aligned(x, weight)
         # (the library refuses fp8 columns that are no multiple of 16)
         and weight.shape[0] % (8 if x.dtype == torch.bfloat16 else 16) == 0
         and weight.shape[1] * weight.element_size() % 64 == 0
@@ -279,6 +288,7 @@ def linear_fp8(xq, x_scale, weight, w_scale, bias=None, out=None):
         xq.shape[0] <= 96
         and _streams_better(xq.shape[0], *weight.shape)
         and _skinny_operands(xq, weight)
+        and (out is None or out.is_contiguous())
     ):
         if out is None:
             out = torch.empty(
@@ -413,7 +423,7 @@ def grouped_linear_takes(x, w) -> bool:
         and 0 < w.shape[0] < 65536
         and x.stride(0) * es % 16 == w.stride(0) * es % 16 == w.stride(1) * es % 16 == 0
         and x.stride(0) >= w.shape[2] <= w.stride(1)
-        and x.data_ptr() % 16 == w.data_ptr() % 16 == 0
+        and aligned(x, w)
         and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
     )
 

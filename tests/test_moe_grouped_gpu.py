@@ -129,3 +129,18 @@ def test_module_routes():
         many, few = m(big)[:37].float(), m(big[:37].contiguous()).float()
         assert (many - few).norm() < 0.02 * few.norm()  # sorted, and per expert
     assert PRESETS["mixtral-8x7b"].num_local_experts <= 32
+
+
+def test_rows_that_begin_anywhere():
+    """Hidden rows that are not on a 16-byte boundary take the per-expert route."""
+    cfg = ModelArchConfig(architecture="mixtral", hidden_size=128, intermediate_size=64,
+                          num_local_experts=4, num_experts_per_tok=2)
+    with torch.device(DEV):
+        m = MoEMLP(cfg).bfloat16()
+    m.stack_experts()
+    for T in (5, 300):
+        odd = torch.randn(T * 128 + 1, device=DEV, dtype=torch.bfloat16)[1:].view(T, 128)
+        with torch.inference_mode():
+            got, want = m(odd).float(), m(odd.clone()).float()
+        # the per-expert route rounds weights and partial sums to bf16
+        assert (got - want).norm() < 0.02 * want.norm()

@@ -10,6 +10,7 @@ import pytest
 import torch
 
 import kubeai_amd.ops as ops
+from kubeai_amd.engine.quant import Fp8Linear
 from kubeai_amd.ops import ref
 
 pytestmark = pytest.mark.gpu
@@ -188,3 +189,20 @@ def test_linear_routes_agree():
         got = ops.linear_fp8(x8, sx, w8, sw, b)
         # the library adds the bias in fp32 or after rounding, as it likes
         torch.testing.assert_close(got.float(), want, atol=2e-2, rtol=2.0 ** -7)
+
+
+def test_products_of_operands_that_begin_anywhere():
+    """A slice of one row counts as contiguous whatever its address and stride;
+    the kernels that read 16 bytes at a time leave it to the library."""
+    torch.manual_seed(3)
+    N, K = 512, 17408
+    w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) * K ** -0.5
+    odd = torch.empty(N * K + 1, device=DEV, dtype=torch.bfloat16)[1:].view(N, K).copy_(w)
+    wide = torch.randn(3, K + 9, device=DEV, dtype=torch.bfloat16)
+    for x, m in ((wide[:1, 1 : K + 1], w), (wide[:1, :K], w), (wide[:, :K].contiguous(), odd)):
+        want = torch.nn.functional.linear(x.float(), m.float())
+        torch.testing.assert_close(ops.linear(x, m).float(), want, atol=2e-3, rtol=2.0 ** -7)
+        assert ops.product_sums(x, m) is None
+    x = wide[:1, 1 : K + 1]
+    lin = Fp8Linear(w)
+    torch.testing.assert_close(lin(x).float(), lin(x.clone()).float(), atol=2e-2, rtol=2.0 ** -6)
