@@ -107,3 +107,19 @@ def test_manager_batched_equals_one_by_one():
                                torch.zeros(256, 65, device=DEV, dtype=torch.bfloat16), 1.0)
     m._build_tables()
     assert "qkv" not in m._tables and "o" in m._tables
+
+
+@pytest.mark.parametrize("pad,first", [(1, 0), (4, 0), (8, 3), (9, 1)])
+@pytest.mark.parametrize("T", [1, 20])
+def test_rows_that_begin_anywhere(T, pad, first):
+    """x as a slice of wider rows, at any offset and stride."""
+    m = LoRAManager(_Model(), DEV, torch.bfloat16)
+    m.load(4, None)
+    ids = torch.full((T,), 4, dtype=torch.int32, device=DEV)
+    wide = torch.randn(T, 128 + pad, device=DEV, dtype=torch.bfloat16)
+    x = wide[:, first : first + 128]
+    y = torch.randn(T, 256, device=DEV, dtype=torch.bfloat16)
+    A, B, s = m.adapters[4]["qkv"][1]
+    want = y.double() + (x.double() @ A.double().T @ B.double().T) * s
+    m.apply(1, "qkv", x, y, ids)
+    torch.testing.assert_close(y.double(), want, atol=1e-4, rtol=2.0 ** -8)
