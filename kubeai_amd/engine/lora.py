@@ -33,8 +33,8 @@ class LoRAManager:
         # adapters[lora_id][target] = list over layers of (A [r,in], B [out,r], scale)
         self.adapters: dict[int, dict[str, list[tuple[torch.Tensor, torch.Tensor, float]]]] = {}
         # target -> (device table rows by layer, widest rank, (in, out), the
-        # tensors the rows point to) for the batched kernel; targets it does not
-        # take are absent
+        # adapters in it, the tensors the rows point to) for the batched kernel;
+        # targets it does not take are absent
         self._tables: dict[str, tuple] = {}
         model.lora_manager = self
         for m in model.modules():
@@ -64,7 +64,8 @@ class LoRAManager:
         form where any adapter's tensors are not what the batched kernel reads
         (bf16, dense, rank up to 64, the same sizes in every layer). The new
         tables take the old ones' place in one assignment, and a table keeps its
-        tensors: a step on another thread finishes with what it began with."""
+        tensors, whatever becomes of the adapters' lists: a step on another
+        thread finishes with what it began with."""
         tables = {}
         adapters = {lid: a for lid, a in self.adapters.items() if lid != 0}
         on_gpu = torch.device(self.device).type == "cuda"
@@ -89,7 +90,8 @@ class LoRAManager:
             ]
             table = torch.tensor(rows, dtype=torch.int64).to(self.device)
             rank = max(A.shape[0] for _, s in sets for A, _, _ in s[:layers])
-            tables[target] = (list(table.unbind(0)), rank, (din, dout), sets)
+            kept = [t.detach() for _, s in sets for A, B, _ in s[:layers] for t in (A, B)]
+            tables[target] = (list(table.unbind(0)), rank, (din, dout), adapters.keys(), kept)
         self._tables = tables
 
     @property
@@ -240,6 +242,7 @@ class LoRAManager:
         tab = self._tables.get(target)
         if (
             tab is not None
+            and tab[3] == self.adapters.keys()  # nothing came or went beside load()
             and layer_idx < len(tab[0])
             and x.dtype == y.dtype == torch.bfloat16
             and (x.shape[1], y.shape[1]) == tab[2]

@@ -123,3 +123,22 @@ def test_rows_that_begin_anywhere(T, pad, first):
     want = y.double() + (x.double() @ A.double().T @ B.double().T) * s
     m.apply(1, "qkv", x, y, ids)
     torch.testing.assert_close(y.double(), want, atol=1e-4, rtol=2.0 ** -8)
+
+
+def test_an_adapter_that_is_not_in_the_table_yet():
+    """Put into the manager beside load() (as load() itself does before the table
+    is rebuilt), and tensors that are let go: the table holds its own."""
+    m = LoRAManager(_Model(), DEV, torch.bfloat16)
+    m.load(4, None)
+    kept = {t.data_ptr() for t in m._tables["qkv"][4]}
+    assert kept == {t.data_ptr() for s in m.adapters[4]["qkv"] for t in s[:2]}
+    m.adapters[9] = m._random_adapter(9)
+    ids = torch.tensor([4, 9, 0], dtype=torch.int32, device=DEV)
+    x = torch.randn(3, 128, device=DEV, dtype=torch.bfloat16)
+    y = torch.zeros(3, 256, device=DEV, dtype=torch.bfloat16)
+    m.apply(0, "qkv", x, y, ids)
+    for t in (0, 1):
+        A, B, s = m.adapters[int(ids[t])]["qkv"][0]
+        want = (x[t].double() @ A.double().T @ B.double().T) * s
+        torch.testing.assert_close(y[t].double(), want, atol=1e-4, rtol=2.0 ** -8)
+    assert (y[2] == 0).all()
