@@ -72,3 +72,25 @@ def test_peaked_flat_and_negative_scales():
     _run(EDGES, 8, 2, 128, 3.0)
     _run(EDGES, 8, 2, 128, 0.0)
     _run(EDGES, 8, 2, 128, -0.2)
+
+
+@pytest.mark.parametrize("hd", [128, 256])
+@pytest.mark.parametrize("softcap", [0.0, 20.0])
+def test_keys_that_are_not_finite(hd, softcap):
+    """A NaN score reaches the output; a capped infinite one is the cap."""
+    torch.manual_seed(hd)
+    kc = torch.randn(9, 1, 16, hd, device=DEV, dtype=torch.bfloat16)
+    vc = torch.randn_like(kc)
+    kc[2, 0, 5, 7] = float("nan")
+    kc[4, 0, 3, 1], kc[6, 0, 3, 1] = float("inf"), -float("inf")
+    bt = torch.tensor([[1, 2], [3, 4], [5, 6], [7, 8]], dtype=torch.int32, device=DEV)
+    total = torch.full((4,), 30, dtype=torch.int32, device=DEV)
+    q = torch.randn(4, 2, hd, device=DEV, dtype=torch.bfloat16)
+    args = (bt, total, hd ** -0.5)
+    got = ops.paged_attention_decode(q, kc, vc, *args, softcap=softcap).float()
+    want = ref.paged_attention_decode(q.float(), kc.float(), vc.float(), *args, softcap=softcap)
+    assert want[0].isnan().all() and want[3].isfinite().all()
+    if softcap:
+        torch.testing.assert_close(got, want, atol=1e-4, rtol=2.0 ** -8, equal_nan=True)
+    else:  # an infinite score outweighs all others or is outweighed
+        assert torch.equal(got.isnan(), want.isnan())

@@ -103,3 +103,27 @@ def test_runs_of_a_longer_stream(first, lens):
     assert (got[:first] == 7.0).all()
     torch.testing.assert_close(got[first:].float(), want, rtol=2 * 2.0 ** -9,
                                atol=2 * 2.0 ** -9 * vc.float().abs().max().item())
+
+
+@pytest.mark.parametrize("hd", [128, 256])
+@pytest.mark.parametrize("softcap", [0.0, 20.0])
+def test_keys_that_are_not_finite(hd, softcap):
+    """A NaN score reaches the rows that see it; a capped infinite one is the cap."""
+    torch.manual_seed(hd)
+    kc = torch.randn(10, 1, 16, hd, device=DEV, dtype=torch.bfloat16)
+    vc = torch.randn_like(kc)
+    kc[2, 0, 5, 7] = float("nan")
+    kc[5, 0, 3, 1], kc[8, 0, 3, 1] = float("inf"), -float("inf")
+    bt = torch.tensor([[1, 2, 3], [4, 5, 6], [7, 8, 9]], dtype=torch.int32, device=DEV)
+    total = torch.full((3,), 40, dtype=torch.int32, device=DEV)
+    start = torch.tensor([0, 40, 80, 120], dtype=torch.int32, device=DEV)
+    q = torch.randn(120, 2, hd, device=DEV, dtype=torch.bfloat16)
+    args = (bt, start, total, hd ** -0.5)
+    got = ops.paged_attention_prefill(q, kc, vc, *args, softcap=softcap).float()
+    want = ref.paged_attention_prefill(q.float(), kc.float(), vc.float(), *args, softcap=softcap)
+    assert want[21:40].isnan().all() and want[:21].isfinite().all()
+    if softcap:
+        bound = 2 * 2.0 ** -9 * vc.float().abs().max().item()
+        torch.testing.assert_close(got, want, atol=bound, rtol=2 * 2.0 ** -9, equal_nan=True)
+    else:  # an infinite score outweighs all others or is outweighed
+        assert torch.equal(got.isnan(), want.isnan())
