@@ -15,9 +15,10 @@
 //    they stand. V needs its keys along a lane: it goes through a
 //    wave-private LDS tile (row-major, 16-byte units XOR-swizzled, no
 //    barriers) and comes back through ds_read_b64_tr_b16.
-//  - the weights keep their 24 bits: they are split into three bf16 parts
-//    (each the rounded rest of the one before) that are multiplied one after
-//    the other into the same fp32 sum.
+//  - the weights keep their 24 bits: they are cut into three bf16 parts of 8
+//    bits that are multiplied one after the other into the same fp32 sum. A
+//    part that would be 0 is 2^-100 (or the weight, if that is less): times an
+//    infinite value 0 would be NaN.
 //  - the next tile's K and V are in flight while this one is computed (two
 //    register sets).
 // Bound by reading the cache. The form before this (scores and weighted sum
@@ -217,11 +218,12 @@ __launch_bounds__(kBlockThreads, 2) __global__ void paged_decode_kernel(
       for (int i = 0; i < 4; ++i) {
         float p = __builtin_amdgcn_exp2f(s[j][i] - m_use);
         l_run += p;
+        const float least = fminf(p, 0x1p-100f);
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-          const __bf16 r = (__bf16)p;
-          p_part[k][j * 4 + i] = __builtin_bit_cast(short, r);
-          p -= (float)r;
+          const uint32_t top = __float_as_uint(p) & 0xffff0000u;
+          p_part[k][j * 4 + i] = (short)(top >> 16);
+          p = fmaxf(p - __uint_as_float(top), least);
         }
       }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");

@@ -94,3 +94,29 @@ def test_keys_that_are_not_finite(hd, softcap):
         torch.testing.assert_close(got, want, atol=1e-4, rtol=2.0 ** -8, equal_nan=True)
     else:  # an infinite score outweighs all others or is outweighed
         assert torch.equal(got.isnan(), want.isnan())
+
+
+@pytest.mark.parametrize("hd", [128, 256])
+@pytest.mark.parametrize("cache", [torch.bfloat16, torch.float8_e5m2])
+@pytest.mark.parametrize("L", [1, 20, 300])
+def test_values_that_are_not_finite(hd, cache, L):
+    """An infinite value is infinite in the output, also behind a weight that bf16
+    holds exactly (1 key: weight 1; equal scores: a power of two)."""
+    torch.manual_seed(L)
+    nb = (L + 15) // 16
+    kc = torch.randn(3 * nb, 2, 16, hd, device=DEV, dtype=torch.bfloat16)
+    vc = torch.randn_like(kc)
+    at = min(L - 1, 9)
+    vc[0, 0, at, 3], vc[0, 0, at, 9], vc[0, 1, at, hd - 1] = float("inf"), -float("inf"), float("nan")
+    vc[nb, 1, 0, 0] = float("inf")
+    kc, vc = kc.to(cache), vc.to(cache)
+    if cache != torch.bfloat16:  # (the conversion keeps infinities)
+        assert vc[0, 0, at, 3].float().isinf()
+    bt = torch.arange(3 * nb, dtype=torch.int32, device=DEV).view(3, nb)
+    total = torch.full((3,), L, dtype=torch.int32, device=DEV)
+    for scale in (hd ** -0.5, 0.0):
+        q = torch.randn(3, 4, hd, device=DEV, dtype=torch.bfloat16)
+        got = ops.paged_attention_decode(q, kc, vc, bt, total, scale).float()
+        want = ref.paged_attention_decode(q.float(), kc.float(), vc.float(), bt, total, scale)
+        assert want[0, 0, 3] == float("inf") and want[0, 1, 9] == -float("inf")
+        torch.testing.assert_close(got, want, atol=1e-4, rtol=2.0 ** -8, equal_nan=True)
