@@ -252,17 +252,22 @@ __global__ __launch_bounds__(kBlock) void lora_expand_kernel(
             if (k + e < R) b[j][e] = (short)br[e];
         }
       }
-      // v in three parts of 8 bits each, cut off: their sum is v
+      // v in three parts of 8 bits each, cut off: their sum is v. A part that
+      // would be 0 is 2^-100 with v's sign (or v, if that is less): 0 times an
+      // infinite B would be NaN. Nothing else is left of infinities and NaN.
       bf16x8 part3[3];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         float rest = v[m][k + e];
+        const uint32_t sign = __float_as_uint(rest) & 0x80000000u;
+        const float least = fminf(fabsf(rest), 0x1p-100f);
 #pragma unroll
         for (int p = 0; p < 3; ++p) {
           const uint32_t top = __float_as_uint(rest) & 0xffff0000u;
           part3[p][e] = (short)(top >> 16);
-          // nothing is left of infinities and NaN
-          rest = (top & 0x7f800000u) == 0x7f800000u ? 0.f : rest - __uint_as_float(top);
+          // (inf - inf is NaN, which the maximum passes over)
+          const float left = fmaxf(fabsf(rest - __uint_as_float(top)), least);
+          rest = __uint_as_float(__float_as_uint(left) | sign);
         }
       }
 #pragma unroll

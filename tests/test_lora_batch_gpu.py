@@ -142,3 +142,26 @@ def test_an_adapter_that_is_not_in_the_table_yet():
         want = (x[t].double() @ A.double().T @ B.double().T) * s
         torch.testing.assert_close(y[t].double(), want, atol=1e-4, rtol=2.0 ** -8)
     assert (y[2] == 0).all()
+
+
+@pytest.mark.parametrize("rank", [1, 8, 33])
+def test_infinite_weights_reach_the_output(rank):
+    """An infinite B is infinite in y, with the sign of the product, also where
+    the rank's value is one that bf16 holds exactly; NaN and 0 times it are NaN."""
+    from kubeai_amd import _C
+
+    x = torch.zeros(4, 64, device=DEV, dtype=torch.bfloat16)
+    x[0, 0], x[1, 0], x[2, 0] = 1.0, -3.0, 0.0
+    x[3] = torch.randn(64, device=DEV)
+    A = torch.zeros(rank, 64, device=DEV, dtype=torch.bfloat16)
+    A[0] = torch.randn(64, device=DEV)
+    A[0, 0] = 0.5
+    B = torch.randn(40, rank, device=DEV, dtype=torch.bfloat16)
+    B[3, 0], B[5, 0], B[17, 0] = float("inf"), -float("inf"), float("nan")
+    table = torch.tensor([[A.data_ptr(), B.data_ptr(), _two_words(rank, 1), _float_word(2.0)]],
+                         dtype=torch.int64, device=DEV)
+    y = torch.ones(4, 40, device=DEV, dtype=torch.bfloat16)
+    want = y.double() + 2.0 * (x.double() @ A.double().T) @ B.double().T
+    _C.lora_apply(y, x, table, torch.ones(4, dtype=torch.int32, device=DEV), rank)
+    assert want[0, 3] == float("inf") and want[1, 3] == -float("inf") and want[2, 3].isnan()
+    torch.testing.assert_close(y.double(), want, atol=1e-4, rtol=2.0 ** -8, equal_nan=True)
