@@ -316,9 +316,9 @@ void lora_apply(torch::Tensor y, torch::Tensor x, torch::Tensor table,
   TORCH_CHECK(table.scalar_type() == torch::kInt64 && table.is_contiguous() &&
               table.dim() == 2 && table.size(1) == 4);
   TORCH_CHECK(table.is_cuda() && ids.is_cuda() && x.is_cuda() && y.is_cuda());
-  TORCH_CHECK((x.stride(0) % 8 == 0 || x.size(0) == 1) &&
-                  ((uintptr_t)x.data_ptr() & 15) == 0,
-              "16-byte aligned rows");
+  // its rows are read 16 bytes at a time
+  if ((x.stride(0) % 8 != 0 && x.size(0) > 1) || ((uintptr_t)x.data_ptr() & 15) != 0)
+    x = x.clone(at::MemoryFormat::Contiguous);
   TORCH_CHECK(max_rank >= 1 && max_rank <= kMaxR);
   const int64_t T = x.size(0);
   const int H = x.size(1), out = y.size(1), n = table.size(0);

@@ -251,9 +251,6 @@ class LoRAManager:
         ):
             from kubeai_amd import _C
 
-            if x.stride(0) % 8 or x.data_ptr() % 16:
-                # its rows are read 16 bytes at a time
-                x = x.clone(memory_format=torch.contiguous_format)
             _C.lora_apply(y, x, tab[0][layer_idx], lora_ids, tab[1])
             return
         present = torch.unique(lora_ids)
