@@ -5,7 +5,9 @@
 //
 //  - moe_route: workgroup = token; a wave per expert in turn, the products of
 //    the bf16 hidden row and router rows summed in fp32; the largest top_k
-//    (ties: the lower expert) and the softmax over them in fp32.
+//    (ties: the lower expert) and the softmax over them in fp32. NaN is the
+//    largest score, and infinite scores make the weights NaN, as in the library
+//    calls that this stands for: a token whose scores are not finite shows it.
 //  - moe_order: one workgroup sorts the T * top_k (token, choice) pairs by
 //    expert, tokens ascending: every thread counts a run of pairs per expert
 //    (LDS [expert][thread]), the counts are scanned, every thread places its
@@ -50,14 +52,15 @@ __launch_bounds__(256) __global__ void moe_route_kernel(
   }
   __syncthreads();
   if (wave != 0) return;
-  // lane e holds expert e; NaN scores lose to every number
-  float v = lane < E ? logit[lane] : -INFINITY;
-  if (!(v == v)) v = -INFINITY;
+  // lane e holds expert e; the order of the scores, lanes past E below all
+  const float v = lane < E ? logit[lane] : -INFINITY;
+  const bool nan = v != v;
   bool taken = lane >= E;
   float first = 0.f, total = 0.f, mine = 0.f;
   for (int k = 0; k < top; ++k) {
-    float best = taken ? -INFINITY : v;
-    int at = taken ? kMaxExperts : lane;
+    float best = taken ? -INFINITY : nan ? INFINITY : v;
+    // among equals: NaN, then the lower expert; one that is left before the rest
+    int at = lane + (taken ? 2 * WAVE_SIZE : nan ? 0 : WAVE_SIZE);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
       const float ov = __shfl_xor(best, off, 64);
@@ -67,8 +70,10 @@ __launch_bounds__(256) __global__ void moe_route_kernel(
         at = oa;
       }
     }
+    if (at < WAVE_SIZE) best = NAN;
+    at %= WAVE_SIZE;
     if (k == 0) first = best;
-    const float p = best == first ? 1.0f : __expf(best - first);
+    const float p = __expf(best - first);
     total += p;
     if (lane == k) {
       mine = p;

@@ -144,3 +144,41 @@ def test_rows_that_begin_anywhere():
             got, want = m(odd).float(), m(odd.clone()).float()
         # the per-expert route rounds weights and partial sums to bf16
         assert (got - want).norm() < 0.02 * want.norm()
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("E,top", [(4, 2), (5, 5), (32, 8), (1, 1)])
+def test_scores_that_are_not_finite(bad, E, top):
+    """The same weights as topk and softmax give, NaN among them, and every
+    token's experts differ and are in range."""
+    torch.manual_seed(E)
+    x = torch.randn(9, 64, device=DEV, dtype=torch.bfloat16)
+    router = torch.randn(E, 64, device=DEV, dtype=torch.bfloat16)
+    x[0, 3] = x[4, 7] = bad
+    x[6, :] = bad
+    router[E // 2, 5] = bad  # an infinite or NaN score of every other token
+    x[8] = 0.0  # (0 times infinity)
+    z = x.float() @ router.float().T
+    v = z.topk(top, -1).values
+    want = torch.softmax(v, -1)
+    weight, begin, src, place = ops.moe_route(x, router, top)
+    torch.testing.assert_close(weight, want, atol=1e-5, rtol=1e-4, equal_nan=True)
+    b, s, p = begin.tolist(), src.tolist(), place.tolist()
+    assert b[0] == 0 and b[-1] == 9 * top and sorted(p) == list(range(9 * top))
+    for e in range(E):  # a token is at an expert once
+        rows = s[b[e] : b[e + 1]]
+        assert rows == sorted(set(rows))
+
+
+def test_a_router_that_is_not_finite_reaches_the_output():
+    cfg = ModelArchConfig(architecture="mixtral", hidden_size=128, intermediate_size=64,
+                          num_local_experts=4, num_experts_per_tok=2)
+    with torch.device(DEV):
+        m = MoEMLP(cfg).bfloat16()
+    m.stack_experts()
+    with torch.inference_mode():
+        m.gate.weight[2, 0] = float("nan")
+        for T in (5, 300):
+            x = torch.randn(T, 128, device=DEV, dtype=torch.bfloat16)
+            assert m._grouped(x) is not None or T > m.GROUPED_MAX_TOKENS
+            assert m(x).isnan().all()
