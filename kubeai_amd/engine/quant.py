@@ -100,13 +100,7 @@ def convert_to_fp8(model: nn.Module) -> int:
     (llama.DecoderLayer checks _fp8_fused): producer kernels emit fp8 +
     per-row scales, so per-linear dynamic quantization disappears.
     """
-    n = 0
-    for mod in model.modules():
-        for name in _TARGETS:
-            child = getattr(mod, name, None)
-            if isinstance(child, nn.Linear):
-                setattr(mod, name, Fp8Linear(child.weight, child.bias))
-                n += 1
+    n = _swap_linears(model)
     for layer in getattr(model, "layers", []):
         attn = getattr(layer, "self_attn", None)
         mlp = getattr(layer, "mlp", None)
@@ -118,6 +112,22 @@ def convert_to_fp8(model: nn.Module) -> int:
             # MoE: attention runs the fused-fp8 path; the MLP input stays
             # bf16 (router needs it) and MoEMLP quantizes once itself
             layer._fp8_fused = True
-            if hasattr(mlp, "stack_experts"):
-                mlp.stack_experts()
+    return n
+
+
+def _swap_linears(mod: nn.Module) -> int:
+    """The target modules below mod, a mixture's experts stacked again before
+    the next mixture is begun: its bf16 weights lie in one tensor, which is
+    freed by that, so one layer's at most are there twice."""
+    n = 0
+    for name in _TARGETS:
+        child = getattr(mod, name, None)
+        if isinstance(child, nn.Linear):
+            setattr(mod, name, Fp8Linear(child.weight, child.bias))
+            n += 1
+    del child
+    for sub in mod.children():
+        n += _swap_linears(sub)
+    if hasattr(mod, "stack_experts"):
+        mod.stack_experts()
     return n

@@ -289,6 +289,8 @@ class ModelRunner:
             if spec is not None
         )
         if self.device.type == "cuda" and per_block_bytes > 0:
+            # what loading and conversion left in torch's cache counts as free
+            torch.cuda.empty_cache()
             free, total = torch.cuda.mem_get_info(self.device)
             budget = total * gpu_memory_utilization - (total - free)
             # reserve activation headroom: 4% of total
