@@ -220,6 +220,15 @@ class MLP(nn.Module):
         return y
 
 
+def _own_tensor(module: nn.Module, name: str):
+    t = module._parameters.get(name)
+    return module._buffers.get(name) if t is None else t
+
+
+def _restack_after_load(module: "MoEMLP", _) -> None:
+    module._restack()
+
+
 class MoEMLP(nn.Module):
     """Mixtral-style sparse MoE block (token-level top-k routing).
 
@@ -261,44 +270,67 @@ class MoEMLP(nn.Module):
                 lin = getattr(expert, proj)
                 lin.weight = nn.Parameter(self._stacks[proj, "weight"][e])
                 lin.reset_parameters()
+        self.register_load_state_dict_post_hook(_restack_after_load)
 
     def stack_experts(self) -> None:
         """Put the experts' weights (and fp8 scales) behind one another and
         leave views of them in the modules. Called again when the modules
-        have been replaced (fp8 conversion)."""
+        or their tensors have been replaced (fp8 conversion)."""
         self._stacks = {}
         for proj in ("gate_up_proj", "down_proj"):
             mods = [getattr(e, proj) for e in self.experts]
             if any(getattr(m, "bias", None) is not None for m in mods):
                 self._stacks = {}
                 return
-            for name in ("weight_fp8", "weight_scale"):
-                if name in mods[0]._buffers:
-                    self._stacks[proj, name] = torch.stack(
-                        [m._buffers[name] for m in mods]
-                    )
-                    for m, v in zip(mods, self._stacks[proj, name]):
+            for name in ("weight_fp8", "weight_scale", "weight"):
+                parts = [_own_tensor(m, name) for m in mods]
+                if any(t is None for t in parts) or len(
+                    {(t.shape, t.dtype, t.device) for t in parts}
+                ) != 1:
+                    continue
+                with torch.inference_mode(False), torch.no_grad():
+                    stack = torch.stack(parts)
+                self._stacks[proj, name] = stack
+                for m, t, v in zip(mods, parts, stack):
+                    if isinstance(t, nn.Parameter):
+                        t.data = v
+                    else:
                         m._buffers[name] = v
-            if "weight" in mods[0]._parameters:
-                stack = torch.stack([m.weight.data for m in mods])
-                self._stacks[proj, "weight"] = stack
-                for m, v in zip(mods, stack):
-                    m.weight = nn.Parameter(v, requires_grad=m.weight.requires_grad)
+                del parts, t
 
     def _stack(self, proj: str, name: str):
         """The stacked tensor, or None where a module's own tensor has been
-        moved out of it since."""
+        moved out of it since (it is let go then)."""
         stack = self._stacks.get((proj, name))
         if stack is None:
             return None
         at, step = stack.data_ptr(), stack.stride(0) * stack.element_size()
         for e in self.experts:
-            m = getattr(e, proj)
-            t = m._parameters.get(name) if name == "weight" else m._buffers.get(name)
+            t = _own_tensor(getattr(e, proj), name)
             if t is None or t.data_ptr() != at or t.shape != stack.shape[1:]:
+                self._stacks.pop((proj, name), None)
                 return None
             at += step
         return stack
+
+    # The stacks go where the modules' tensors go: to another device or type,
+    # into a copy or a pickle, to the tensors that a state dict assigns.
+    def _restack(self) -> None:
+        kinds = list(self._stacks)
+        if any(self._stack(*k) is None for k in kinds):
+            self.stack_experts()
+
+    def _apply(self, fn, recurse=True):
+        super()._apply(fn, recurse)
+        self._restack()
+        return self
+
+    def __getstate__(self):
+        return {**self.__dict__, "_stacks": {}}
+
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        self.stack_experts()
 
     def _on_device(self, x: torch.Tensor) -> bool:
         """Whether csrc/moe.hip takes the routing of x."""
