@@ -71,7 +71,7 @@ class Fp8Linear(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if (
             x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16
-            and x.is_contiguous() and ops.aligned(x)
+            and x.is_contiguous() and not ops.observed(x) and ops.aligned(x)
             and x.shape[1] % 8 == 0 and x.shape[1] <= 32768
         ):
             return self.forward_quantized(*ops.quant_fp8(x))

@@ -342,10 +342,11 @@ class MoEMLP(nn.Module):
             and x.stride(0) == x.shape[1]  # (of a single row it may be anything)
             and x.shape[1] % 8 == 0
             and self.gate.weight.is_contiguous()
+            and not torch.is_grad_enabled()
+            and not ops.observed(x)
             and ops.aligned(x, self.gate.weight)
             and self.n_experts <= 32
             and self.top_k <= min(8, self.n_experts)
-            and not torch.is_grad_enabled()
         )
 
     def _sorted(self, x: torch.Tensor) -> torch.Tensor:

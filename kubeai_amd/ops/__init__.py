@@ -209,6 +209,26 @@ class ProductSums:
         return self.part, self.x_scale, self.w_scale
 
 
+_PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
+
+
+def observed(*tensors) -> bool:
+    """Whether something follows the tensors' operations that a kernel launch
+    would pass by: autograd, forward mode, vmap, a trace or dispatch mode,
+    autocast, a tensor subclass. Where the library's own operation stood before,
+    it still does then."""
+    grad = torch.is_grad_enabled()
+    return (
+        torch.compiler.is_compiling()
+        or torch._C._get_tracing_state() is not None
+        or torch._C._functorch.peek_interpreter_stack() is not None
+        or torch._C._len_torch_dispatch_stack() > 0
+        or torch.autograd.forward_ad._current_level >= 0
+        or torch.is_autocast_enabled("cuda")
+        or any(type(t) not in _PLAIN_TENSORS or grad and t.requires_grad for t in tensors)
+    )
+
+
 def aligned(*tensors) -> bool:
     """Whether kernels may read the tensors' storage 16 bytes at a time. (A slice
     that counts as contiguous can begin anywhere.)"""
@@ -228,12 +248,12 @@ def _skinny_operands(x, weight) -> bool:
         and weight.is_contiguous()
         # (the stride of a single row may be anything)
         and x.stride(0) == x.shape[1]
-        and aligned(x, weight)
         # (the library refuses fp8 columns that are no multiple of 16)
         and weight.shape[0] % (8 if x.dtype == torch.bfloat16 else 16) == 0
         and weight.shape[1] * weight.element_size() % 64 == 0
         and weight.device == x.device
-        and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
+        and not observed(x, weight)
+        and aligned(x, weight)
     )
 
 
@@ -423,8 +443,8 @@ def grouped_linear_takes(x, w) -> bool:
         and 0 < w.shape[0] < 65536
         and x.stride(0) * es % 16 == w.stride(0) * es % 16 == w.stride(1) * es % 16 == 0
         and x.stride(0) >= w.shape[2] <= w.stride(1)
+        and not observed(x, w)
         and aligned(x, w)
-        and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
     )
 
 

@@ -206,3 +206,39 @@ def test_products_of_operands_that_begin_anywhere():
     x = wide[:1, 1 : K + 1]
     lin = Fp8Linear(w)
     torch.testing.assert_close(lin(x).float(), lin(x.clone()).float(), atol=2e-2, rtol=2.0 ** -6)
+
+
+def test_products_under_transforms():
+    """What follows operations sees the product: forward mode, vmap, a trace,
+    autocast, a dispatch mode, and gradients of the input."""
+    import torch.autograd.forward_ad as fwd
+    from torch.utils.flop_counter import FlopCounterMode
+
+    torch.manual_seed(4)
+    N, K = 20480, 256  # a width that few rows go through the streaming kernel at
+    w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) * K ** -0.5
+    x, t = _x(4, K), _x(4, K) * 0.5
+    want, slope = torch.nn.functional.linear(x, w), torch.nn.functional.linear(t, w)
+
+    def near(a, b):
+        torch.testing.assert_close(a.float(), b.float(), atol=2e-3, rtol=2.0 ** -6)
+
+    with fwd.dual_level():
+        y = fwd.unpack_dual(ops.linear(fwd.make_dual(x, t), w))
+        near(y.primal, want)
+        assert y.tangent is not None
+        near(y.tangent, slope)
+    near(torch.func.jvp(lambda v: ops.linear(v, w), (x,), (t,))[1], slope)
+    near(torch.func.vmap(lambda v: ops.linear(v, w))(torch.stack([x, t]))[1], slope)
+    traced = torch.jit.trace(lambda v: ops.linear(v, w), (x,))
+    near(traced(t), slope)
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert ops.linear(x, w).dtype == torch.float16
+    with FlopCounterMode(display=False) as flops:
+        ops.linear(x, w)
+    assert flops.get_total_flops() == 2 * 4 * N * K
+    v = x.clone().requires_grad_()
+    ops.linear(v, w).float().sum().backward()
+    near(v.grad, w.float().sum(0).expand(4, K))
+    lin = Fp8Linear(w)
+    assert lin(v).requires_grad and not lin(x).requires_grad
