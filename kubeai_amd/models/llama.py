@@ -40,14 +40,36 @@ class EngineLinear(nn.Linear):
         return None if self.bias is not None else ops.product_sums(x, self.weight)
 
 
+def _hooked(module: nn.Module) -> bool:
+    """Whether someone waits for the module's call and its tensors."""
+    return bool(
+        module._forward_hooks or module._forward_pre_hooks
+        or torch.nn.modules.module._has_any_global_hook()
+    )
+
+
 def _project(linear, x, as_sums: bool):
     """linear(x), x a tensor or an (fp8 rows, scales) pair. as_sums: what reads
     the result takes ops.ProductSums, so it may be that."""
     if isinstance(x, tuple):
         y = linear.sums_quantized(*x) if as_sums else None
         return linear.forward_quantized(*x) if y is None else y
-    y = linear.sums(x) if as_sums and isinstance(linear, EngineLinear) else None
+    y = None
+    if as_sums and type(linear) is EngineLinear and not _hooked(linear):
+        y = linear.sums(x)
     return linear(x) if y is None else y
+
+
+def _call(module, *args):
+    return module(*args)
+
+
+def _branch(module, *args):
+    """The attention or feed-forward module's result, ops.ProductSums where it
+    is one that can give them and nobody else sees what it returns."""
+    if type(module) in (Attention, MLP, MoEMLP) and not _hooked(module):
+        return module(*args, as_sums=True)
+    return module(*args)
 
 
 def _rms_head(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
@@ -332,6 +354,20 @@ class MoEMLP(nn.Module):
         super().__setstate__(state)
         self.stack_experts()
 
+    def _own_experts(self) -> bool:
+        """Whether the experts are the modules made here (or their fp8 forms) and
+        nobody waits for their calls: their weights may be used beside them."""
+        for e in self.experts:
+            if type(e) is not MLP or _hooked(e):
+                return False
+            for proj in ("gate_up_proj", "down_proj"):
+                lin = e._modules[proj]
+                if _hooked(lin) or not (
+                    type(lin) is EngineLinear or "weight_fp8" in lin._buffers
+                ):
+                    return False
+        return True
+
     def _on_device(self, x: torch.Tensor) -> bool:
         """Whether csrc/moe.hip takes the routing of x."""
         return (
@@ -347,6 +383,7 @@ class MoEMLP(nn.Module):
             and ops.aligned(x, self.gate.weight)
             and self.n_experts <= 32
             and self.top_k <= min(8, self.n_experts)
+            and self._own_experts()
         )
 
     def _sorted(self, x: torch.Tensor) -> torch.Tensor:
@@ -500,21 +537,23 @@ class DecoderLayer(nn.Module):
                 torch.ones(cfg.hidden_size)
             )
 
-    def forward(self, x, residual, fb, kv_cache, cos_sin):
+    def forward(self, x, residual, fb, kv_cache, cos_sin, as_sums: bool = False):
+        """as_sums: the caller takes the branch as ops.ProductSums too (x may be
+        that in any case)."""
+        last = _branch if as_sums else _call
         if self.post_norms:
             # incoming invariant: hidden = x + residual (residual None at
             # layer 0); outgoing (m_normed, hidden_after_attn) keeps it,
             # so the model-level final fused_add_rmsnorm still applies
             hidden = x if residual is None else x + residual
-            a = self.self_attn(
-                ops.rmsnorm(hidden, self.input_layernorm, self.eps),
-                fb, kv_cache, cos_sin, as_sums=True,
+            a = _branch(
+                self.self_attn, ops.rmsnorm(hidden, self.input_layernorm, self.eps),
+                fb, kv_cache, cos_sin,
             )
             a = ops.rmsnorm(a, self.post_attention_layernorm, self.eps)
             h2 = hidden + a
-            mm = self.mlp(
-                ops.rmsnorm(h2, self.pre_feedforward_layernorm, self.eps), fb,
-                as_sums=True,
+            mm = _branch(
+                self.mlp, ops.rmsnorm(h2, self.pre_feedforward_layernorm, self.eps), fb
             )
             mm = ops.rmsnorm(mm, self.post_feedforward_layernorm, self.eps)
             return mm, h2
@@ -533,7 +572,7 @@ class DecoderLayer(nn.Module):
                 xq, xs = ops.fused_add_rmsnorm_fp8(
                     x, residual, self.input_layernorm, self.eps
                 )
-            x = self.self_attn((xq, xs), fb, kv_cache, cos_sin, as_sums=True)
+            x = _branch(self.self_attn, (xq, xs), fb, kv_cache, cos_sin)
             if isinstance(self.mlp, MoEMLP):
                 # router consumes bf16; MoEMLP quantizes once internally
                 x, residual = ops.fused_add_rmsnorm(
@@ -544,7 +583,7 @@ class DecoderLayer(nn.Module):
                 xq, xs = ops.fused_add_rmsnorm_fp8(
                     x, residual, self.post_attention_layernorm, self.eps
                 )
-                x = self.mlp((xq, xs), as_sums=True)
+                x = last(self.mlp, (xq, xs))
             return x, residual
         if residual is None:
             residual = x
@@ -554,13 +593,13 @@ class DecoderLayer(nn.Module):
                 x, residual, self.input_layernorm, self.eps
             )
         plain = self.res_mult == 1.0  # the next norm reads the branch as it is
-        x = self.self_attn(x, fb, kv_cache, cos_sin, as_sums=plain)
+        x = (_branch if plain else _call)(self.self_attn, x, fb, kv_cache, cos_sin)
         if self.res_mult != 1.0:
             x = x * self.res_mult
         x, residual = ops.fused_add_rmsnorm(
             x, residual, self.post_attention_layernorm, self.eps
         )
-        x = self.mlp(x, fb, as_sums=plain)
+        x = (last if plain else _call)(self.mlp, x, fb)
         if self.res_mult != 1.0:
             x = x * self.res_mult
         return x, residual
@@ -634,8 +673,13 @@ class LlamaForCausalLM(nn.Module):
             # image-placeholder positions take the vision-tower embeddings
             x = x.index_copy(0, fb.mm_idx, fb.mm_embeds.to(x.dtype))
         residual = None
+        n = len(self.layers)
+        # layers that nobody else looks at hand on products that the next one's
+        # (or the final) norm adds up
+        own = [type(layer) is DecoderLayer and not _hooked(layer) for layer in self.layers]
         for i, layer in enumerate(self.layers):
-            x, residual = layer(x, residual, fb, self.kv_caches[i], cs)
+            kw = {"as_sums": True} if own[i] and (i + 1 == n or own[i + 1]) else {}
+            x, residual = layer(x, residual, fb, self.kv_caches[i], cs, **kw)
         x, _ = ops.fused_add_rmsnorm(x, residual, self.norm, self.cfg.rms_norm_eps)
         return x
 
