@@ -32,8 +32,12 @@
 //   8 rows of 3584                                    48 ->  31
 //   1 row of 3000 and 7 idle ones                     32 ->  14
 //   heads 64/8 x 128, 32 rows of 1000-3000           165 ->  60
-//   heads 8/4 x 256, cap, 40 rows of 300-900          55 ->  45
-// At head size 256 a tile is one block (two would need 512 registers).
+//   heads 8/4 x 256, cap, 40 rows of 100-700          42 ->  22
+//     96 rows of 2000, no cap                         222 -> 143
+//   heads 4/4 x 256, 96 rows of 2000                  188 -> 142
+// At head size 256 a tile is one block (two would need 512 registers), and over
+// a bf16 cache the query lies in LDS: with it in registers 25 were spilled, and
+// the reloads waited for the loads in flight (the last two 236 us).
 #include <torch/extension.h>
 
 #include <type_traits>
@@ -112,14 +116,32 @@ __launch_bounds__(kBlockThreads, 2) __global__ void paged_decode_kernel(
   __shared__ float merge_ml[kWaves][kMaxG][2];
   char* vt = smem + wave * kVTile * 2;
 
-  bf16x8 q_frag[NC];
-  {
-    const ushort* qp = q + (int64_t)b * q_stride +
-                       (int64_t)(kh * G + min(col, G - 1)) * HD + grp * 8;
+  // Head size 256 over a bf16 cache: two tiles of K and V and the sums leave no
+  // registers for the query; it lies in LDS, 16-byte units XORed with the head.
+  constexpr bool kQLds = HD == 256 && sizeof(CT) == 2;
+  __shared__ __attribute__((aligned(16))) ushort q_lds[kQLds ? kMaxG * HD : 8];
+  bf16x8 q_frag[kQLds ? 1 : NC];
+  const ushort* qp = q + (int64_t)b * q_stride + (int64_t)kh * G * HD;
+  const int q_head = min(col, G - 1);
+  if constexpr (kQLds) {
+    for (int i = threadIdx.x; i < G * (HD / 8); i += kBlockThreads) {
+      const int g = i / (HD / 8), u = i % (HD / 8);
+      *reinterpret_cast<bf16x8*>(&q_lds[g * HD + ((u ^ g) << 3)]) =
+          *reinterpret_cast<const bf16x8*>(qp + i * 8);
+    }
+    __syncthreads();
+  } else {
 #pragma unroll
     for (int c = 0; c < NC; ++c)
-      q_frag[c] = *reinterpret_cast<const bf16x8*>(qp + c * 32);
+      q_frag[c] = *reinterpret_cast<const bf16x8*>(qp + q_head * HD + grp * 8 + c * 32);
   }
+  auto query = [&](int c) -> bf16x8 {
+    if constexpr (kQLds)
+      return *reinterpret_cast<const bf16x8*>(
+          &q_lds[q_head * HD + (((c * 4 + grp) ^ q_head) << 3)]);
+    else
+      return q_frag[c];
+  };
   const float c2 = CAP ? scale : scale * kLog2e;
   const float inv_cap = CAP ? 1.0f / softcap : 0.f;
 
@@ -184,7 +206,7 @@ __launch_bounds__(kBlockThreads, 2) __global__ void paged_decode_kernel(
 #pragma unroll
       for (int c = 0; c < NC; ++c)
         s[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            to_bf16(kf[set][j][c]), q_frag[c], s[j], 0, 0, 0);
+            to_bf16(kf[set][j][c]), query(c), s[j], 0, 0, 0);
     }
     float tmax = -INFINITY;
 #pragma unroll
@@ -360,6 +382,29 @@ __global__ void decode_merge_kernel(
 
 }  // namespace
 
+// How often a row's keys are split: until there are 512 workgroups (two a CU).
+// The lengths are not known here; more splits cost in the merge, and a row that
+// is much longer than the others is worked through by its own splits alone. At
+// head size 256, whose workgroups read a row at half the rate of those at 128,
+// many rows are split once more for that (576). Head size 128: 40 rows of
+// 100-700 keys, 8 kv heads 23.0 us at 512, 25.6 at 1536; one row of 3000 among 7
+// idle ones 13.6 at 512, 17.0 at 1536. Head size 256: 128 rows of 300 but one
+// of 8000, 4 kv heads 224 us at 512, 122 at 576, 87 at 1536; 8 rows of 3500, e5m2
+// cache, 8 kv heads 33 at 512, 42 at 576; 40 rows of 100-700, e5m2 cache, 4 kv
+// heads 19.3 at 512 and 576, 22 at 768, 25 at 1536. A split has at least one
+// tile of the widest row. KUBEAI_DECODE_SPLIT_TARGET overrides for tuning sweeps.
+int paged_decode_splits(int rows, int n_kv, int hd, int max_blocks) {
+  static const int forced = []() {
+    const char* e = getenv("KUBEAI_DECODE_SPLIT_TARGET");
+    return e ? atoi(e) : 0;
+  }();
+  const int64_t wgs = (int64_t)rows * n_kv;
+  const int target = forced > 0 ? forced : hd == 256 && wgs > 64 ? 576 : 512;
+  const int tiles = hd == 256 ? max_blocks : (max_blocks + 1) / 2;
+  return (int)std::max<int64_t>(
+      1, std::min({(int64_t)kMaxSplits, (int64_t)tiles, (target + wgs - 1) / wgs}));
+}
+
 void paged_attention_decode(torch::Tensor out, torch::Tensor q,
                             torch::Tensor k_cache, torch::Tensor v_cache,
                             torch::Tensor block_tables, torch::Tensor seq_lens,
@@ -383,18 +428,7 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
   if (B == 0) return;
   TORCH_CHECK(G == 1 || G == 2 || G == 4 || G == 5 || G == 6 || G == 8,
               "unsupported GQA group size ", G);
-  // The keys are split until 512 workgroups (two a CU) are there; the lengths
-  // are not known here, and more splits cost in the merge: 40 rows of 100-700
-  // keys, 8 kv heads 23.0 us at 512, 25.6 at 1536; one row of 3000 among 7 idle
-  // ones 13.6 at 512, 17.0 at 1536, 16.7 at 256. KUBEAI_DECODE_SPLIT_TARGET overrides for tuning sweeps.
-  static const int split_target = []() {
-    const char* e = getenv("KUBEAI_DECODE_SPLIT_TARGET");
-    const int v = e ? atoi(e) : 512;
-    return v > 0 ? v : 512;
-  }();
-  const int64_t base_wgs = (int64_t)B * n_kv;
-  const int n_splits = (int)std::max<int64_t>(
-      1, std::min<int64_t>(kMaxSplits, (split_target + base_wgs - 1) / base_wgs));
+  const int n_splits = paged_decode_splits(B, n_kv, hd, max_blocks);
   torch::Tensor part_o, part_ml;
   float *part_o_ptr = nullptr, *part_ml_ptr = nullptr;
   if (n_splits > 1) {
@@ -405,7 +439,7 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
     part_o_ptr = part_o.data_ptr<float>();
     part_ml_ptr = part_ml.data_ptr<float>();
   }
-  const dim3 grid((uint32_t)(base_wgs * n_splits)), block(kBlockThreads);
+  const dim3 grid((uint32_t)((int64_t)B * n_kv * n_splits)), block(kBlockThreads);
   auto stream = c10::hip::getCurrentHIPStream().stream();
   auto launch = [&](auto hdv, auto ct, auto cap) {
     using CT = decltype(ct);

@@ -30,6 +30,7 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
                             torch::Tensor k_cache, torch::Tensor v_cache,
                             torch::Tensor block_tables, torch::Tensor seq_lens,
                             double scale, int64_t window, double softcap);
+int paged_decode_splits(int rows, int n_kv, int hd, int max_blocks);
 void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
                              torch::Tensor k_cache, torch::Tensor v_cache,
                              torch::Tensor block_tables,
@@ -102,6 +103,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "paged KV cache write, fp8 e5m2 cache");
   m.def("paged_attention_decode", &paged_attention_decode,
         "paged attention, one query token per seq");
+  m.def("paged_decode_splits", &paged_decode_splits,
+        "splits of a decode row's keys (rows, kv heads, head size, table width)");
   m.def("paged_attention_prefill", &paged_attention_prefill,
         "paged causal flash attention over cached KV");
   m.def("gelu_and_mul", &gelu_and_mul, "GeGLU tanh-gelu(gate)*up");

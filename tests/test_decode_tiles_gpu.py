@@ -120,3 +120,27 @@ def test_values_that_are_not_finite(hd, cache, L):
         want = ref.paged_attention_decode(q.float(), kc.float(), vc.float(), bt, total, scale)
         assert want[0, 0, 3] == float("inf") and want[0, 1, 9] == -float("inf")
         torch.testing.assert_close(got, want, atol=1e-4, rtol=2.0 ** -8, equal_nan=True)
+
+
+@pytest.mark.parametrize("hd", [128, 256])
+@pytest.mark.parametrize("rows,n_kv,blocks", [(1, 1, 1), (1, 8, 4), (3, 4, 600), (32, 4, 250),
+                                              (64, 4, 400), (128, 4, 500), (700, 2, 40)])
+def test_splits(hd, rows, n_kv, blocks):
+    """Two workgroups a CU where the rows allow it, never more splits than 16 or
+    than a row can have tiles; many rows of head size 256 are split even where
+    they fill the chip (a longer one among them would be worked through alone)."""
+    from kubeai_amd import _C
+
+    n = _C.paged_decode_splits(rows, n_kv, hd, blocks)
+    tiles = blocks if hd == 256 else (blocks + 1) // 2
+    assert 1 <= n <= min(16, tiles)
+    assert n == min(16, tiles) or rows * n_kv * n >= 512
+    assert n == 1 or rows * n_kv * (n - 1) < 576
+    if hd == 256 and rows * n_kv == 512:
+        assert n == 2
+
+
+@pytest.mark.parametrize("group", [1, 2, 8])
+@pytest.mark.parametrize("cache", [torch.bfloat16, torch.float8_e5m2])
+def test_one_long_row_among_short_ones(group, cache):
+    _run([3000] + [9] * 70, 2 * group, 2, 256, 0.06, fp8=cache != torch.bfloat16)
