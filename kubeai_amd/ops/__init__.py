@@ -271,25 +271,36 @@ def product_sums(x, weight, x_scale=None, w_scale=None):
     return ProductSums(_C.skinny_sums(x, weight), x_scale, w_scale)
 
 
-def _streams_better(M: int, N: int, K: int) -> bool:
+def _streams_better(M: int, N: int, K: int, fp8: bool) -> bool:
     """Whether the weight-streaming product beats the library's where it has to
     add its parts itself. Few rows and a width that fills the chip uncut (us,
-    library / this): 8 rows bf16 4096 -> 28672 65 / 50, 2304 -> 18432 51 / 24,
-    2048 -> 32256 33 / 30, fp8 4096 -> 28672 34 / 29; at 32 rows 57 / 56 and
-    21 / 31, at 128256 columns 192 / 198. Very long rows, which the library does
-    not cut: 32256 -> 2048 83 / 36 at 8 rows, 127 / 61 at 96; 14336 -> 4096 at 8
-    rows 27 / 29."""
-    return (M <= 16 and 16384 <= N <= 65536) or (K >= 8 * N and K >= 16384)
+    weights out of cache, library / this, 8 rows): bf16 4096 -> 28672 59.9 / 47.6,
+    2304 -> 18432 50.8 / 25.2, 2048 -> 32256 34.5 / 31.4, 4096 -> 65536 123 / 107,
+    but 4096 -> 16384 33.4 / 34.8, 8192 -> 24576 83.8 / 91.8, 6144 -> 24576 at 16
+    rows 68.5 / 73.8; fp8 4096 -> 16384 27.9 / 20.3, 4096 -> 28672 33.8 / 28.0,
+    8192 -> 30720 65 / 58; beyond two passes of workgroups over the chip only
+    whole passes (8192 -> 36864 fp8 72 / 81), and not for rows under 256 bytes (128
+    -> 65536 fp8 5.6 / 6.7). At 32 rows 53.5 / 53.4 and 21 / 30, at 128256 columns
+    192 / 198. Very long rows, which the library does not cut: 32256 -> 2048 83 /
+    38 at 8 rows, 127 / 60 at 96; it does at 16384 (-> 1024 20.4 / 19.4 at 8 rows,
+    21.0 / 28.7 at 48; fp8 20.2 / 12.9, 20.1 / 21.4 at 96)."""
+    if K >= 8 * N and K >= 16384:
+        return K > 16384 or M <= (64 if fp8 else 32)
+    if M > 16 or N > 65536 or (N > 32768 and N % 16384) or K * (1 if fp8 else 2) < 256:
+        return False
+    if fp8:
+        return N >= 16384 and K <= 8192
+    return N >= 16384 and K <= 1024 or N > 16384 and K <= (6144 if M <= 8 else 4096)
 
 
 def linear(x, weight):
     """x weight^T. Few rows against a wide or a very long weight go through the
     weight-streaming kernel (csrc/skinny_gemm.hip), the rest to the library."""
     if (
-        x.is_cuda
-        and x.dim() == weight.dim() == 2
+        x.dim() == weight.dim() == 2
         and x.shape[0] <= 96
-        and _streams_better(x.shape[0], *weight.shape)
+        and x.is_cuda
+        and _streams_better(x.shape[0], *weight.shape, fp8=False)
         and x.dtype == torch.bfloat16
         and _skinny_operands(x, weight)
     ):
@@ -306,7 +317,7 @@ def linear_fp8(xq, x_scale, weight, w_scale, bias=None, out=None):
     [N, K] e4m3, x_scale [M], w_scale [1, N]; into `out` (dense rows) if given."""
     if (
         xq.shape[0] <= 96
-        and _streams_better(xq.shape[0], *weight.shape)
+        and _streams_better(xq.shape[0], *weight.shape, fp8=True)
         and _skinny_operands(xq, weight)
         and (out is None or out.is_contiguous())
     ):
