@@ -60,13 +60,18 @@ class Fp8Linear(nn.Module):
             xq, x_scale, self.weight_fp8, self.weight_scale, self.bias
         )
 
-    def sums_quantized(self, xq: torch.Tensor, x_scale: torch.Tensor):
-        """forward_quantized as ops.ProductSums, or None (library product)."""
-        if self.bias is not None:
+    def sums_quantized(
+        self, xq: torch.Tensor, x_scale: torch.Tensor, rope: bool = False,
+        eager: bool = False,
+    ):
+        """forward_quantized as ops.ProductSums, for a norm or (rope) the rotation,
+        or None (library product)."""
+        w = self.weight_fp8
+        if self.bias is not None or xq.shape[0] > 96 or not ops.sums_better(
+            xq.shape[0], *w.shape, fp8=True, rope=rope, eager=eager
+        ):
             return None
-        return ops.product_sums(
-            xq, self.weight_fp8, x_scale, self.weight_scale.view(-1)
-        )
+        return ops.product_sums(xq, w, x_scale, self.weight_scale.view(-1))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if (

@@ -35,28 +35,40 @@ class EngineLinear(nn.Linear):
             y = y + self.bias
         return y
 
-    def sums(self, x: torch.Tensor):
-        """The product as ops.ProductSums, or None (library product, bias)."""
-        return None if self.bias is not None else ops.product_sums(x, self.weight)
+    def sums(self, x: torch.Tensor, rope: bool = False, eager: bool = False):
+        """The product as ops.ProductSums, for a norm or (rope) the rotation, or
+        None (library product, bias)."""
+        w = self.weight
+        if self.bias is not None or x.shape[0] > 96 or not ops.sums_better(
+            x.shape[0], *w.shape, fp8=False, rope=rope, eager=eager
+        ):
+            return None
+        return ops.product_sums(x, w)
+
+
+_EVERY_MODULES_HOOKS = torch.nn.modules.module._global_forward_hooks
+_EVERY_MODULES_PRE_HOOKS = torch.nn.modules.module._global_forward_pre_hooks
 
 
 def _hooked(module: nn.Module) -> bool:
     """Whether someone waits for the module's call and its tensors."""
     return bool(
         module._forward_hooks or module._forward_pre_hooks
-        or torch.nn.modules.module._has_any_global_hook()
+        or _EVERY_MODULES_HOOKS or _EVERY_MODULES_PRE_HOOKS
     )
 
 
-def _project(linear, x, as_sums: bool):
+def _project(linear, x, as_sums: bool, fb: ForwardBatch | None, rope: bool = False):
     """linear(x), x a tensor or an (fp8 rows, scales) pair. as_sums: what reads
-    the result takes ops.ProductSums, so it may be that."""
+    the result, a norm or (rope) the rotation, takes ops.ProductSums, so it may
+    be that. Steps with prompt portions are never recorded in a graph."""
+    eager = fb is not None and fb.n_prefill > 0
     if isinstance(x, tuple):
-        y = linear.sums_quantized(*x) if as_sums else None
+        y = linear.sums_quantized(*x, rope, eager) if as_sums else None
         return linear.forward_quantized(*x) if y is None else y
     y = None
     if as_sums and type(linear) is EngineLinear and not _hooked(linear):
-        y = linear.sums(x)
+        y = linear.sums(x, rope, eager)
     return linear(x) if y is None else y
 
 
@@ -141,6 +153,7 @@ class Attention(nn.Module):
             self.qkv_proj, x,
             not lora_live and not self.qk_norm
             and ops.rope_takes_sums(k_cache, v_cache),
+            fb, rope=True,
         )
         if lora_live:
             lm.apply(self.layer_idx, "qkv", x, qkv, fb.lora_ids)
@@ -201,8 +214,8 @@ class Attention(nn.Module):
             )
         attn_flat = out.view(T, -1)
         if fp8_in:
-            return _project(self.o_proj, ops.quant_fp8(attn_flat), as_sums)
-        result = _project(self.o_proj, attn_flat, as_sums and not lora_live)
+            return _project(self.o_proj, ops.quant_fp8(attn_flat), as_sums, fb)
+        result = _project(self.o_proj, attn_flat, as_sums and not lora_live, fb)
         if lora_live:
             lm.apply(self.layer_idx, "o", attn_flat, result, fb.lora_ids)
         return result
@@ -226,7 +239,7 @@ class MLP(nn.Module):
         """as_sums: the caller takes the result as ops.ProductSums too."""
         if isinstance(x, tuple):  # fused fp8 path (never active with LoRA)
             h = self.gate_up_proj.forward_quantized(*x)
-            return _project(self.down_proj, ops.silu_and_mul_fp8(h), as_sums)
+            return _project(self.down_proj, ops.silu_and_mul_fp8(h), as_sums, fb)
         h = self.gate_up_proj(x)
         lm = getattr(self, "_lora_manager", None)
         lora_live = (
@@ -236,7 +249,7 @@ class MLP(nn.Module):
         if lora_live:
             lm.apply(self.layer_idx, "gate_up", x, h, fb.lora_ids)
         a = ops.gelu_and_mul(h) if self.gelu else ops.silu_and_mul(h)
-        y = _project(self.down_proj, a, as_sums and not lora_live)
+        y = _project(self.down_proj, a, as_sums and not lora_live, fb)
         if lora_live:
             lm.apply(self.layer_idx, "down", a, y, fb.lora_ids)
         return y
@@ -379,7 +392,6 @@ class MoEMLP(nn.Module):
             and x.shape[1] % 8 == 0
             and self.gate.weight.is_contiguous()
             and not torch.is_grad_enabled()
-            and not ops.observed(x)
             and ops.aligned(x, self.gate.weight)
             and self.n_experts <= 32
             and self.top_k <= min(8, self.n_experts)
@@ -583,7 +595,7 @@ class DecoderLayer(nn.Module):
                 xq, xs = ops.fused_add_rmsnorm_fp8(
                     x, residual, self.post_attention_layernorm, self.eps
                 )
-                x = last(self.mlp, (xq, xs))
+                x = last(self.mlp, (xq, xs), fb)
             return x, residual
         if residual is None:
             residual = x

@@ -209,24 +209,28 @@ class ProductSums:
         return self.part, self.x_scale, self.w_scale
 
 
+_forward_ad = torch.autograd.forward_ad
 _PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
 
 
 def observed(*tensors) -> bool:
     """Whether something follows the tensors' operations that a kernel launch
     would pass by: autograd, forward mode, vmap, a trace or dispatch mode,
-    autocast, a tensor subclass. Where the library's own operation stood before,
-    it still does then."""
-    grad = torch.is_grad_enabled()
-    return (
-        torch.compiler.is_compiling()
-        or torch._C._get_tracing_state() is not None
+    autocast, a tensor subclass. Where the library's own operation stood by
+    itself before, it still does then."""
+    if (
+        torch._C._len_torch_dispatch_stack()
+        or _forward_ad._current_level >= 0
         or torch._C._functorch.peek_interpreter_stack() is not None
-        or torch._C._len_torch_dispatch_stack() > 0
-        or torch.autograd.forward_ad._current_level >= 0
+        or torch._C._get_tracing_state() is not None
         or torch.is_autocast_enabled("cuda")
-        or any(type(t) not in _PLAIN_TENSORS or grad and t.requires_grad for t in tensors)
-    )
+    ):
+        return True
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if type(t) not in _PLAIN_TENSORS or grad and t.requires_grad:
+            return True
+    return False
 
 
 def aligned(*tensors) -> bool:
@@ -252,23 +256,77 @@ def _skinny_operands(x, weight) -> bool:
         and weight.shape[0] % (8 if x.dtype == torch.bfloat16 else 16) == 0
         and weight.shape[1] * weight.element_size() % 64 == 0
         and weight.device == x.device
-        and not observed(x, weight)
-        and aligned(x, weight)
+        and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
+        and x.data_ptr() % 16 == weight.data_ptr() % 16 == 0
     )
 
 
 def product_sums(x, weight, x_scale=None, w_scale=None):
-    """x weight^T as ProductSums for a consumer that takes them, or None where
-    the library's product is the better one: from 16384 columns on the product
-    fills the chip without being cut, and above 96 rows it is no longer the
-    weights that bound it. (Per product and consumer, us, library -> this: 40
-    rows fp8 4096 -> 6144 18.4 -> 16.5, 14336 -> 4096 28.1 -> 23.8; 96 rows bf16
-    14336 -> 4096 59.6 -> 41.8, 4096 -> 4096 27.5 -> 22.)"""
+    """x weight^T as ProductSums for a consumer that takes them, or None for
+    operands that the kernel does not take (from 16384 columns on the product
+    fills the chip without being cut). Whether it is the better form:
+    sums_better."""
     if not (
         x.shape[0] <= 96 and weight.shape[0] < 16384 and _skinny_operands(x, weight)
     ):
         return None
     return ProductSums(_C.skinny_sums(x, weight), x_scale, w_scale)
+
+
+def sums_better(
+    M: int, N: int, K: int, fp8: bool, rope: bool = False, eager: bool = False
+) -> bool:
+    """Whether a product as ProductSums and the norm that adds them (rope: the
+    rotation and cache write) beat the library's product and its reader. The
+    reader's cost grows with parts x M x N, so wide products of many rows are the
+    library's, and so are those that it cuts along K itself; eight-bit weights
+    are read in half the time and leave less to gain. (In a whole decode step of 40
+    rows in fp8 the sums of the products around attention gain 3 us a layer that
+    pairs timed by themselves do not show.) us, weights out of cache,
+    library / this: bf16 4096 -> 4096 8 rows 18.9 / 13.5, 96 rows 25.3 / 19.3;
+    14336 -> 4096 8 rows 30.4 / 31.0, 40 rows 39.4 / 32.1; 4096 -> 6144 8 rows 18.4
+    / 16.2 (rotation), 64 rows 20.4 / 21.2; 8192 -> 8192 34.7 / 41.4; 8192 -> 1024
+    8 rows 14.6 / 12.3, 40 rows 15.1 / 17.1. fp8 4096 -> 4096 16 rows 15.8 / 13.3,
+    64 rows 16.4 / 18.3; 14336 -> 4096 40 rows 25.1 / 22.8; 8192 -> 8192 8 rows
+    47.5 / 26.6, 16 rows 20.6 / 27.2; 512 -> 4096 8.2 / 8.8. Over 3576 and 1656
+    products of 512 to 28672 columns and rows with either reader the chosen ones
+    take 0.72 and 0.80 of the library's time, the worst 1.2.
+    eager: the step is not replayed from a graph, so the host's launches bound it
+    while the weights are small, and the library's call takes 10 us of the host
+    more (80 tokens of a prompt on 8 layers of 4096: 1796 us / 1493)."""
+    if eager and N * K * (1 if fp8 else 2) < 2**26:
+        return True
+    if K > 16384 and N <= 6144:  # (there the library is two to four times slower)
+        return True
+    if fp8:
+        if rope and (K < 2048 or M > 48 or M > 16 and 2048 < K < 4096):
+            return False
+        if K < 2048:
+            return M <= 40 and N <= 2304 if K >= 1024 and M > 32 else (
+                M <= 32 and N <= (2304 if K < 1024 else 5120)
+            )
+        if M <= 12:
+            return N <= 4096 or K <= 4096 or N >= 8192
+        if N > 4096:
+            return N <= 6144 and K <= 4096 if rope else (
+                M <= 32 and K <= 2048 and N <= 8192
+            )
+        if M <= 48:
+            return True
+        return (N <= 3072 or K > 4096) if M <= 64 else K >= 12288
+    if K <= 1024:
+        return (N <= 6144 or M <= 48) and not (rope and K < 1024 and 1024 < N <= 4096)
+    if N > 6144:
+        return False
+    if K <= 4096:
+        if N > 4096:
+            if rope and (M <= 16 or 32 < M <= 48):
+                return True
+            return M <= (48 if K <= 2048 else 8)
+        return M <= 64 or min(N, K) >= 3072
+    if M <= 16:
+        return N <= 2048 or K >= 12288 and N <= 4096
+    return N <= 4096 if M <= 32 else N >= 2048
 
 
 def _streams_better(M: int, N: int, K: int, fp8: bool) -> bool:
@@ -302,6 +360,7 @@ def linear(x, weight):
         and x.is_cuda
         and _streams_better(x.shape[0], *weight.shape, fp8=False)
         and x.dtype == torch.bfloat16
+        and not observed(x, weight)
         and _skinny_operands(x, weight)
     ):
         y = torch.empty(
@@ -454,7 +513,7 @@ def grouped_linear_takes(x, w) -> bool:
         and 0 < w.shape[0] < 65536
         and x.stride(0) * es % 16 == w.stride(0) * es % 16 == w.stride(1) * es % 16 == 0
         and x.stride(0) >= w.shape[2] <= w.stride(1)
-        and not observed(x, w)
+        and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
         and aligned(x, w)
     )
 
