@@ -67,8 +67,12 @@ class Fp8Linear(nn.Module):
         """forward_quantized as ops.ProductSums, for a norm or (rope) the rotation,
         or None (library product)."""
         w = self.weight_fp8
-        if self.bias is not None or xq.shape[0] > 96 or not ops.sums_better(
-            xq.shape[0], *w.shape, fp8=True, rope=rope, eager=eager
+        if (
+            self.bias is not None or xq.shape[0] > 96
+            or type(self).forward_quantized is not Fp8Linear.forward_quantized
+            or not ops.sums_better(
+                xq.shape[0], *w.shape, fp8=True, rope=rope, eager=eager
+            )
         ):
             return None
         return ops.product_sums(xq, w, x_scale, self.weight_scale.view(-1))

@@ -64,7 +64,8 @@ def _project(linear, x, as_sums: bool, fb: ForwardBatch | None, rope: bool = Fal
     be that. Steps with prompt portions are never recorded in a graph."""
     eager = fb is not None and fb.n_prefill > 0
     if isinstance(x, tuple):
-        y = linear.sums_quantized(*x, rope, eager) if as_sums else None
+        sums = getattr(linear, "sums_quantized", None) if as_sums else None
+        y = sums(*x, rope, eager) if sums is not None else None
         return linear.forward_quantized(*x) if y is None else y
     y = None
     if as_sums and type(linear) is EngineLinear and not _hooked(linear):
@@ -72,15 +73,16 @@ def _project(linear, x, as_sums: bool, fb: ForwardBatch | None, rope: bool = Fal
     return linear(x) if y is None else y
 
 
-def _call(module, *args):
+def _call(module, *args, **own):
     return module(*args)
 
 
-def _branch(module, *args):
+def _branch(module, *args, **own):
     """The attention or feed-forward module's result, ops.ProductSums where it
-    is one that can give them and nobody else sees what it returns."""
+    is one that can give them and nobody else sees what it returns. own: what
+    only the modules of this file take."""
     if type(module) in (Attention, MLP, MoEMLP) and not _hooked(module):
-        return module(*args, as_sums=True)
+        return module(*args, **own, as_sums=True)
     return module(*args)
 
 
@@ -595,7 +597,7 @@ class DecoderLayer(nn.Module):
                 xq, xs = ops.fused_add_rmsnorm_fp8(
                     x, residual, self.post_attention_layernorm, self.eps
                 )
-                x = last(self.mlp, (xq, xs), fb)
+                x = last(self.mlp, (xq, xs), fb=fb)
             return x, residual
         if residual is None:
             residual = x

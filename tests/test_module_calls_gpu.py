@@ -6,7 +6,7 @@ import torch
 import kubeai_amd.ops as ops
 from kubeai_amd.engine import EngineConfig, LLMEngine
 from kubeai_amd.engine.batch import ForwardBatch
-from kubeai_amd.engine.quant import convert_to_fp8
+from kubeai_amd.engine.quant import Fp8Linear, convert_to_fp8
 from kubeai_amd.models.config import PRESETS
 from kubeai_amd.models.llama import MoEMLP
 
@@ -65,6 +65,47 @@ def test_a_layer_called_by_itself_returns_tensors(fp8):
         assert all(type(t) is torch.Tensor for t in out)
         layer.register_forward_hook(lambda m, args, o: None)
         model(fb)
+
+
+def test_fp8_modules_put_in_by_others():
+    """They get the calls that Fp8Linear and MLP got: forward_quantized(rows,
+    scales) for a projection, one argument for a feed-forward module."""
+    model, fb = _step("llama-tiny", True)
+    with torch.inference_mode():
+        want = model(fb).float()
+        layer = model.layers[0]
+        calls = []
+
+        class Watched(Fp8Linear):
+            def forward_quantized(self, xq, x_scale):
+                calls.append("derived")
+                return super().forward_quantized(xq, x_scale)
+
+        class Other(torch.nn.Module):
+            def __init__(self, lin):
+                super().__init__()
+                self.lin = lin
+
+            def forward_quantized(self, xq, x_scale):
+                calls.append("other")
+                return self.lin.forward_quantized(xq, x_scale)
+
+        class Feed(torch.nn.Module):
+            def __init__(self, mlp):
+                super().__init__()
+                self.mlp = mlp
+
+            def forward(self, x):
+                calls.append("feed")
+                return self.mlp(x)
+
+        layer.mlp.down_proj.__class__ = Watched
+        layer.self_attn.o_proj = Other(layer.self_attn.o_proj)
+        layer.mlp = Feed(layer.mlp)
+        got = model(fb).float()
+    assert calls == ["other", "feed", "derived"]
+    # sums of another product's parts: one rounding here and there
+    assert (got - want).norm() < 0.02 * want.norm()
 
 
 def test_expert_hooks():
