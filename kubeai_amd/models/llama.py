@@ -269,7 +269,7 @@ def _restack_after_load(module: "MoEMLP", _) -> None:
 class MoEMLP(nn.Module):
     """Mixtral-style sparse MoE block (token-level top-k routing).
 
-    On GPU, steps of up to GROUPED_MAX_TOKENS tokens route on the device
+    On GPU, small steps route on the device
     (csrc/moe.hip) and run all experts' rows in one weight-streaming product
     per projection (csrc/skinny_gemm.hip): shapes do not depend on the routing,
     so decode steps can be recorded in a graph, and every expert's weights are
@@ -280,13 +280,26 @@ class MoEMLP(nn.Module):
     slower one, the library's on each expert's slice, after one look at the
     experts' row counts."""
 
-    #: one pass of 8 experts of 14336, us, weight-streaming / tiled / every
-    #: expert's tokens asked for one after the other: fp8 128 tokens
-    #: 358/387/722, 256 447/411/743, 512 819/470/1361, 2048 2413/1015/2006;
-    #: bf16 128 617/690/1159, 256 734/731/1221, 512 1397/871/1614, 2048
-    #: 4223/1708/2488 (streaming reads an expert's weights again for every 96
-    #: of its rows). Up to 256 tokens any routing may be recorded in a graph.
+    #: one pass of 8 experts of 14336 x 4096, us, weight-streaming / tiled /
+    #: every expert's tokens asked for one after the other: fp8 128 tokens
+    #: 353/383/722, 512 819/470/1361, 2048 2413/1015/2006; bf16 128
+    #: 602/684/1159, 512 1397/871/1614, 2048 4223/1708/2488 (streaming reads
+    #: an expert's weights again for every 96 of its rows). Up to 256 tokens any
+    #: routing may be recorded in a graph, so no row counts come to the host.
     GROUPED_MAX_TOKENS = 256
+
+    #: Above these the tiled product has the step where it takes both
+    #: projections. us, streaming / tiled, tokens spread evenly (half of them
+    #: alike): fp8 160 tokens 364/389 (478/416), 192 416/393 (549/421), 256
+    #: 443/404 (593/418); 8 x 7168 x 2048 160 140/160 (188/167), 192 160/158
+    #: (209/171); 16 x 6400 x 4096 192 333/319 (401/328); 32 x 1408 x 2048, 4 a
+    #: token, 192 115/118 (133/124); 4 x 3584 x 1024 160 71/78 (93/81), 192 90/80
+    #: (99/77). bf16 192 681/704 (936/752), 224 704/711 (970/739), 256 723/719
+    #: (1017/741); 8 x 7168 x 2048 224 257/266 (365/294), 256 268/270 (371/298);
+    #: 16 x 6400 x 4096 256 591/570 (802/655); 32 x 1408 x 2048 256 176/179
+    #: (236/203).
+    TILED_ABOVE_FP8 = 160
+    TILED_ABOVE_BF16 = 224
 
     def __init__(self, cfg: ModelArchConfig):
         super().__init__()
@@ -449,6 +462,22 @@ class MoEMLP(nn.Module):
             a = ops.gelu_and_mul(h) if self.gelu else ops.silu_and_mul(h)
         return ops.moe_combine(products(a, "down_proj", x.shape[1]), place, weight)
 
+    def _tiled_has(self, tokens: int) -> bool:
+        """Whether a step of up to GROUPED_MAX_TOKENS is the tiled product's."""
+        fp8 = ("down_proj", "weight_fp8") in self._stacks
+        if tokens <= (self.TILED_ABOVE_FP8 if fp8 else self.TILED_ABOVE_BF16):
+            return False
+        for proj in ("gate_up_proj", "down_proj"):
+            w = self._stack(proj, "weight_fp8" if fp8 else "weight")
+            if (
+                w is None or (fp8 and self._stack(proj, "weight_scale") is None)
+                or w.shape[2] * w.element_size() % 128 or w.shape[1] % 16
+                or not ops.aligned(w)
+                or not ops.grouped_linear_better(tokens * self.top_k, w)
+            ):
+                return False
+        return not (fp8 and self.gelu)
+
     def _grouped(self, x: torch.Tensor):
         """All experts' rows at once; None where the kernels do not take it."""
         if not (self._on_device(x) and x.shape[0] <= self.GROUPED_MAX_TOKENS):
@@ -472,11 +501,14 @@ class MoEMLP(nn.Module):
     def forward(
         self, x: torch.Tensor, fb: ForwardBatch | None = None, as_sums: bool = False
     ) -> torch.Tensor:
+        if (
+            x.shape[0] > self.TILED_ABOVE_FP8 and self._on_device(x)
+            and (x.shape[0] > self.GROUPED_MAX_TOKENS or self._tiled_has(x.shape[0]))
+        ):
+            return self._sorted(x)
         out = self._grouped(x)
         if out is not None:
             return out
-        if x.shape[0] > 256 and self._on_device(x):
-            return self._sorted(x)
         T, H = x.shape
         router = F.linear(x.float(), self.gate.weight.float())  # [T, E]
         weights, selected = torch.topk(router, self.top_k, dim=-1)

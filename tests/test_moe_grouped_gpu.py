@@ -53,6 +53,19 @@ def test_skinny_linear(M, N, K):
     _close(y, _mm(x8.float(), w8.float()) * sx[:, None] * sw + b.float())
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 6144, 4096), (33, 4096, 4096), (7, 4096, 14336),
+                                   (64, 4096, 14336), (16, 128256, 4096)])
+def test_skinny_linear_large(M, N, K):
+    from kubeai_amd import _C
+
+    torch.manual_seed(M + N + K)
+    x = torch.randn(M, K, device=DEV, dtype=torch.bfloat16)
+    w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16)
+    y = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    _C.skinny_linear(y, x, w, None, None, None)
+    _close(y, _mm(x, w))
+
+
 def _experts(E, I, H):
     gu = torch.randn(E, 2 * I, H, device=DEV, dtype=torch.bfloat16) * H ** -0.5
     dn = torch.randn(E, H, I, device=DEV, dtype=torch.bfloat16) * I ** -0.5
@@ -129,6 +142,54 @@ def test_module_routes():
         many, few = m(big)[:37].float(), m(big[:37].contiguous()).float()
         assert (many - few).norm() < 0.02 * few.norm()  # sorted, and per expert
     assert PRESETS["mixtral-8x7b"].num_local_experts <= 32
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("I", [192, 256])
+def test_which_product(fp8, I):
+    """The tiled product from 161 (fp8) or 225 tokens on where it takes rows of
+    both widths, with the streaming one's results, also from a graph."""
+    cfg = ModelArchConfig(architecture="mixtral", hidden_size=256, intermediate_size=I,
+                          num_local_experts=8, num_experts_per_tok=2)
+    torch.manual_seed(I)
+    with torch.device(DEV):
+        m = MoEMLP(cfg).bfloat16()
+    if fp8:
+        for e in m.experts:
+            e.gate_up_proj = Fp8Linear(e.gate_up_proj.weight)
+            e.down_proj = Fp8Linear(e.down_proj.weight)
+    m.stack_experts()
+    calls = []
+    ordered = m._sorted
+    m._sorted = lambda x: calls.append(x.shape[0]) or ordered(x)
+    takes = not fp8 or I % 128 == 0
+    with torch.inference_mode():
+        for T in (160, 161, 224, 225, 256, 257):
+            x = torch.randn(T, 256, device=DEV, dtype=torch.bfloat16)
+            got = m(x)
+            tiled = T > 256 or takes and T > (160 if fp8 else 224)
+            assert calls == ([T] if tiled else [])
+            calls.clear()
+            if T > m.GROUPED_MAX_TOKENS:
+                continue
+            want = m._grouped(x)
+            if fp8:
+                # an activation row whose largest value lands one bf16 step away
+                # is scaled, and rounded, anew: by up to 2^-4 of each value
+                assert (got - want).float().norm() < 2.0 ** -5 * want.float().norm()
+            else:
+                _close(got, want)
+        x = torch.randn(256, 256, device=DEV, dtype=torch.bfloat16)
+        m(x)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            out = m(x)
+        for _ in range(3):
+            x.copy_(torch.randn_like(x))
+            x[: 128] = x[0]  # other row counts than the recorded step's
+            g.replay()
+            assert torch.equal(out, m(x))
 
 
 def test_rows_that_begin_anywhere():
