@@ -143,7 +143,7 @@ __launch_bounds__(kBlockThreads, 2) __global__ void paged_decode_kernel(
       return q_frag[c];
   };
   const float c2 = CAP ? scale : scale * kLog2e;
-  const float inv_cap = CAP ? 1.0f / softcap : 0.f;
+  const SoftCap cap(CAP ? softcap : 1.0f);
 
   f32x4 o_acc[ND];
 #pragma unroll
@@ -208,13 +208,13 @@ __launch_bounds__(kBlockThreads, 2) __global__ void paged_decode_kernel(
         s[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
             to_bf16(kf[set][j][c]), query(c), s[j], 0, 0, 0);
     }
+    if constexpr (CAP) cap.apply(s, c2);
     float tmax = -INFINITY;
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        float x = s[j][i] * c2;
-        if constexpr (CAP) x = soft_cap(x, softcap, inv_cap) * kLog2e;
+        float x = s[j][i] * (CAP ? kLog2e : c2);
         const int tok = tok0 + j * kBS + grp * 4 + i;
         if (!whole && (tok >= L || tok < w0)) x = -INFINITY;
         s[j][i] = x;

@@ -44,7 +44,7 @@
 //   512 new tokens behind 3584                          414 -> 100
 //   six turns of 62-100 behind 365-587, 4 padding runs   72 ->  23
 //   heads 64/8 x 128, 4096                              927 -> 360
-//   heads 8/4 x 256, 3029 + 2145, cap, window 4096     1574 -> 273 (207 TF/s)
+//   heads 8/4 x 256, 3029 + 2145, cap, window 4096     1574 -> 268 (211 TF/s)
 // Head size 256 holds 128 accumulator registers of O, so one wave a SIMD
 // and 32-key tiles (a 64-key tile's two buffers would need 128 KB).
 //
@@ -163,7 +163,7 @@ void paged_prefill_kernel(
   }
   // (never 0: a masked score is -inf times this)
   const float c2 = fmaxf(fabsf(scale) * (CAP ? 1.0f : kLog2e), 1e-30f);
-  const float inv_cap = CAP ? 1.0f / softcap : 0.f;
+  const SoftCap cap(CAP ? softcap : 1.0f);
   const int qpos = ctx + wrow0 + ln31;
   const int row_pos_lo = ctx + wrow0;                        // wave's rows
   const int row_pos_hi = ctx + min(wrow0 + kQB, q_len) - 1;  // (may be empty)
@@ -277,14 +277,22 @@ void paged_prefill_kernel(
                                                            s[sub], 0, 0, 0);
         }
 
-      // ---- mask, running maximum -----------------------------------------
-      if constexpr (CAP) {
+      // one wave a SIMD has nobody to cover a read of K: four are kept ahead
+      // (heads 8/4 x 256, 3029 + 2145: 255 -> 235 us, each read waited for
+      // before; two waves a SIMD, at head size 128, cover it themselves)
+      if constexpr (HD == 256) {
+        constexpr int kMfma = 0x008, kLdsRead = 0x100, kAhead = 4;
+        __builtin_amdgcn_sched_group_barrier(kLdsRead, kAhead, 0);
 #pragma unroll
-        for (int sub = 0; sub < NSUB; ++sub)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            s[sub][r] = soft_cap(s[sub][r] * c2, softcap, inv_cap);
+        for (int c = 0; c < NC - kAhead; ++c) {
+          __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(kLdsRead, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(kMfma, kAhead, 0);
       }
+
+      // ---- mask, running maximum -----------------------------------------
+      if constexpr (CAP) cap.apply(s, c2);
       const bool inside = kv_start + KVB - 1 <= row_pos_lo &&
                           (!WIN || kv_start > row_pos_hi - window);
       if (!inside) {

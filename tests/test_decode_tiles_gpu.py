@@ -144,3 +144,10 @@ def test_splits(hd, rows, n_kv, blocks):
 @pytest.mark.parametrize("cache", [torch.bfloat16, torch.float8_e5m2])
 def test_one_long_row_among_short_ones(group, cache):
     _run([3000] + [9] * 70, 2 * group, 2, 256, 0.06, fp8=cache != torch.bfloat16)
+
+
+@pytest.mark.parametrize("hd", [128, 256])
+@pytest.mark.parametrize("spread", [0.2, 0.7, 2.5])
+def test_softcap_on_both_sides_of_its_forms(hd, spread):
+    """Scores about and on both sides of 0.7 of the cap, where the form changes."""
+    _run([70, 33], 4, 2, hd, spread * 20.0 * hd ** -0.5, softcap=20.0)

@@ -64,6 +64,13 @@ def test_eight_bit_cache(hd):
     _run([70, 5], [33, 100], 8, 2, hd, hd ** -0.5, fp8=True)
 
 
+@pytest.mark.parametrize("hd", [128, 256])
+@pytest.mark.parametrize("spread", [0.2, 0.7, 2.5])
+def test_softcap_on_both_sides_of_its_forms(hd, spread):
+    """Scores about and on both sides of 0.7 of the cap, where the form changes."""
+    _run([70], [33], 4, 2, hd, spread * 20.0 * hd ** -0.5, softcap=20.0)
+
+
 def test_softcap_small_and_large_scores():
     _run([80], [40], 4, 1, 256, 1e-4, softcap=50.0)
     _run([80], [40], 4, 1, 256, 2.0, softcap=30.0)
