@@ -76,10 +76,6 @@ DEV_INLINE float e5m2_to_f32(unsigned char b) {
   return c.f;
 }
 
-// native 2 x f32 vector, the result type of the packed bf8->f32 convert
-// (v_cvt_pk_f32_bf8: one instruction turns 2 e5m2 bytes into 2 floats)
-typedef float floatx2 __attribute__((ext_vector_type(2)));
-
 // 8 packed e5m2 bytes -> 8 bf16 values (one staging unit).
 //
 // Route: e5m2 is bit-identical to the TOP BYTE of an IEEE fp16, so
@@ -91,8 +87,7 @@ typedef float floatx2 __attribute__((ext_vector_type(2)));
 // truncation: this toolchain mis-simplifies bit manipulation of that
 // intrinsic's result (low mantissa bit folded to zero — 129/256 byte
 // values corrupt, device-verified in scripts/dbg_cvt.hip; an opaque
-// asm barrier does not stop it). Arithmetic (fadd/fma) consumers of
-// cvt_pk_f32_bf8 are fine — the decode kernel keeps using it.
+// asm barrier does not stop it).
 DEV_INLINE ushort8 e5m2x8_to_bf16x8(uint64_t raw) {
   ushort8 out;
 #pragma unroll

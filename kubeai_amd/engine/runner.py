@@ -420,8 +420,9 @@ class ModelRunner:
             lora_ids = torch.tensor(ids, dtype=torch.int32, device=self.device)
 
         # ---- pad the token stream to a bucket size --------------------
-        # Keeps GEMM M-shapes on a small fixed set (TunableOp algo table +
-        # future hipGraph capture). Pad tokens form a throwaway prefill
+        # Keeps the products' row counts on a small fixed set up to 1024
+        # tokens (algorithm table, decode graphs), above that on multiples
+        # of 256. Pad tokens form a throwaway prefill
         # sequence over cache block 0: slot -1 (no KV write), row-local
         # compute only (GEMMs/norms are row-independent), never sampled.
         T = len(input_ids)

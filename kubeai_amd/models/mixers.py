@@ -745,8 +745,9 @@ class RoutedGatedMoE(nn.Module):
     (decode) run two GEMMs over every expert with the routing weight (0 for
     experts a token did not choose) folded into the activation, so the
     weighted sum happens inside the second GEMM's fp32 accumulation and the
-    step has no data-dependent shapes. Large steps gather each expert's
-    tokens and run its slice.
+    step has no data-dependent shapes. Large steps put the tokens in expert
+    order and multiply all experts' rows in one launch a projection, or each
+    expert's by its slice where the library does that sooner (ExpertRows).
 
     extra_out > 0 appends that many rows (with a bias) to the stacked input
     matrix for a projection of the same input that the caller owns (a

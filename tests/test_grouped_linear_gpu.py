@@ -1,5 +1,5 @@
 """All experts' products of a large step in one launch, at the edges of its
-tiles (128 or 256 rows, 256 columns, 128 bytes of K): empty experts, one row,
+tiles (128, 192 or 256 rows, 256 columns, 128 bytes of K): empty experts, one row,
 one more than a tile, more experts than a wave has lanes, strided weights and
 gathered rows, and what it leaves to the library.
 
