@@ -153,7 +153,7 @@ class Attention(nn.Module):
         lora_live = lm is not None and lm.active and fb.lora_ids is not None
         qkv = _project(
             self.qkv_proj, x,
-            not lora_live and not self.qk_norm
+            T <= 96 and not lora_live and not self.qk_norm
             and ops.rope_takes_sums(k_cache, v_cache),
             fb, rope=True,
         )
@@ -586,19 +586,21 @@ class DecoderLayer(nn.Module):
     def forward(self, x, residual, fb, kv_cache, cos_sin, as_sums: bool = False):
         """as_sums: the caller takes the branch as ops.ProductSums too (x may be
         that in any case)."""
-        last = _branch if as_sums else _call
+        # products are handed on as sums in steps of up to 96 rows only
+        branch = _branch if x.shape[0] <= 96 else _call
+        last = branch if as_sums else _call
         if self.post_norms:
             # incoming invariant: hidden = x + residual (residual None at
             # layer 0); outgoing (m_normed, hidden_after_attn) keeps it,
             # so the model-level final fused_add_rmsnorm still applies
             hidden = x if residual is None else x + residual
-            a = _branch(
+            a = branch(
                 self.self_attn, ops.rmsnorm(hidden, self.input_layernorm, self.eps),
                 fb, kv_cache, cos_sin,
             )
             a = ops.rmsnorm(a, self.post_attention_layernorm, self.eps)
             h2 = hidden + a
-            mm = _branch(
+            mm = branch(
                 self.mlp, ops.rmsnorm(h2, self.pre_feedforward_layernorm, self.eps), fb
             )
             mm = ops.rmsnorm(mm, self.post_feedforward_layernorm, self.eps)
@@ -618,7 +620,7 @@ class DecoderLayer(nn.Module):
                 xq, xs = ops.fused_add_rmsnorm_fp8(
                     x, residual, self.input_layernorm, self.eps
                 )
-            x = _branch(self.self_attn, (xq, xs), fb, kv_cache, cos_sin)
+            x = branch(self.self_attn, (xq, xs), fb, kv_cache, cos_sin)
             if isinstance(self.mlp, MoEMLP):
                 # router consumes bf16; MoEMLP quantizes once internally
                 x, residual = ops.fused_add_rmsnorm(
@@ -639,7 +641,7 @@ class DecoderLayer(nn.Module):
                 x, residual, self.input_layernorm, self.eps
             )
         plain = self.res_mult == 1.0  # the next norm reads the branch as it is
-        x = (_branch if plain else _call)(self.self_attn, x, fb, kv_cache, cos_sin)
+        x = (branch if plain else _call)(self.self_attn, x, fb, kv_cache, cos_sin)
         if self.res_mult != 1.0:
             x = x * self.res_mult
         x, residual = ops.fused_add_rmsnorm(
@@ -722,7 +724,9 @@ class LlamaForCausalLM(nn.Module):
         n = len(self.layers)
         # layers that nobody else looks at hand on products that the next one's
         # (or the final) norm adds up
-        own = [type(layer) is DecoderLayer and not _hooked(layer) for layer in self.layers]
+        few = x.shape[0] <= 96
+        own = [few and type(layer) is DecoderLayer and not _hooked(layer)
+               for layer in self.layers]
         for i, layer in enumerate(self.layers):
             kw = {"as_sums": True} if own[i] and (i + 1 == n or own[i + 1]) else {}
             x, residual = layer(x, residual, fb, self.kv_caches[i], cs, **kw)
