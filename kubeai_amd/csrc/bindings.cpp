@@ -51,7 +51,11 @@ void grouped_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                     c10::optional<torch::Tensor> sx,
                     c10::optional<torch::Tensor> sw, torch::Tensor bounds,
                     c10::optional<torch::Tensor> src,
-                    c10::optional<torch::Tensor> square);
+                    c10::optional<torch::Tensor> square, int64_t act);
+void tiled_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
+                  c10::optional<torch::Tensor> sx,
+                  c10::optional<torch::Tensor> sw, int64_t act);
+torch::Tensor tiled_sums(torch::Tensor x, torch::Tensor w);
 void moe_route(torch::Tensor index, torch::Tensor weight, torch::Tensor begin,
                torch::Tensor src, torch::Tensor place, torch::Tensor x,
                torch::Tensor w);
@@ -114,6 +118,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "weight-streaming product of each expert's rows");
   m.def("grouped_linear", &grouped_linear,
         "all experts' products of a large step, bf16 or fp8 e4m3");
+  m.def("tiled_linear", &tiled_linear, "product of many rows, bf16 or scaled fp8");
+  m.def("tiled_sums", &tiled_sums, "fp32 part sums of a product of many rows");
   m.def("skinny_sums", &skinny_sums, "fp32 part sums of a skinny product");
   m.def("quant_fp8_rows", &quant_fp8_rows, "gathered bf16 rows -> fp8");
   m.def("rmsnorm_sums", &rmsnorm_sums, "norm of a product's part sums");

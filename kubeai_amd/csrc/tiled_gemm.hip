@@ -1,0 +1,237 @@
+// What the tiled products (tiled_gemm.h) are given: checks, the tile shape, the
+// parts of K.
+#include <torch/extension.h>
+
+#include <cmath>
+
+#include "tiled_gemm.h"
+
+namespace tiled {
+namespace {
+
+// A launch takes passes over the CUs x (steps x step + tile) + rest, us. One
+// matrix: fitted to 1100 products (128 to 4096 rows, 4096 to 28672 columns, K 4096
+// and 14336, whole and in 2 to 8 parts; 10 % off in the mean, and the shape with
+// the least at most 6 % slower than the best one). With parts, what reads the
+// sums adds their bytes at 4.5 TB/s. Experts, whose weights are used by few row
+// tiles and come from memory: 8 of 3584 x 2048 to 28672 x 4096, 24 to 1024 rows
+// each; there the choice is 2 % slower than the best in the mean.
+struct Cost {
+  float step, tile, rest;
+};
+constexpr Cost kFp8[kNumShapes] = {
+    {0.965f, 21.2f, -7.9f}, {0.779f, 14.4f, -2.7f}, {0.800f, 18.0f, -7.3f},
+    {0.660f, 12.3f, -3.3f}, {0.664f, 9.3f, -0.6f},  {0.520f, 6.2f, 0.6f},
+    {0.444f, 4.3f, 0.7f},   {0.355f, 0.7f, 1.8f}};
+constexpr Cost kBf16[kNumShapes] = {
+    {0.973f, 37.8f, -23.3f}, {0.794f, 24.4f, -11.6f}, {0.777f, 28.6f, -16.3f},
+    {0.668f, 16.7f, -6.3f},  {0.724f, 9.5f, 0.2f},    {0.557f, 6.7f, 1.6f},
+    {0.490f, 2.6f, 4.1f},    {0.387f, -1.1f, 5.8f}};
+constexpr Cost kExpertsFp8[kNumShapes] = {
+    {1.427f, 20.3f, -5.7f}, {1.113f, 17.9f, 5.0f},  {1.126f, 16.1f, 1.4f},
+    {0.859f, 15.5f, 10.2f}, {0.758f, 15.6f, 22.5f}, {0.720f, 8.8f, 11.5f},
+    {0.520f, 8.0f, 22.1f},  {0.383f, 5.8f, 33.1f}};
+constexpr Cost kExpertsBf16[kNumShapes] = {
+    {1.577f, 26.2f, -16.1f}, {1.293f, 16.7f, -9.4f}, {1.285f, 15.9f, -6.7f},
+    {1.074f, 10.7f, -4.6f},  {1.043f, 10.3f, -4.4f}, {0.883f, 4.6f, 0.8f},
+    {0.680f, 3.6f, 3.8f},    {0.503f, 2.5f, 6.3f}};
+constexpr int kMaxParts = 8;
+
+struct Plan {
+  int shape, parts;
+  double us;
+};
+
+// R rows of E experts against cols columns of the result (halves: a tile has
+// half as many)
+Plan plan(bool fp8, int64_t R, int64_t E, int64_t cols, int64_t KB, bool halves, bool sums) {
+  Plan best{-1, 1, 0.};
+  for (int i = 0; i < kNumShapes; i++) {
+    const Shape s = kShapes[i];
+    if (halves && s.wn % 2) continue;
+    const Cost c = E > 1 ? (fp8 ? kExpertsFp8[i] : kExpertsBf16[i]) : (fp8 ? kFp8[i] : kBf16[i]);
+    const int64_t bn = s.cols() / (halves ? 2 : 1), nt = (cols + bn - 1) / bn;
+    double row_tiles = (R + s.rows() - 1) / s.rows();
+    if (E > 1) {  // the mean over row counts within 30 % of an even split
+      row_tiles = 0.;
+      for (int k = -3; k <= 3; k++) {
+        row_tiles += std::ceil((double)R / E * (1. + 0.1 * k) / s.rows()) * E / 7.;
+      }
+    }
+    for (int parts = 1; parts <= (sums ? kMaxParts : 1); parts++) {
+      const int64_t all = KB / kStep, steps = (all + parts - 1) / parts;
+      if (parts > 1 && (steps < 4 || (all + steps - 1) / steps != parts)) continue;
+      const double passes = std::ceil(row_tiles * nt * parts / (256 * s.per_cu()));
+      const double us = passes * (steps * c.step + c.tile) + c.rest +
+                        (sums ? parts * R * cols * 4 / 4.5e6 : 0.);
+      if (best.shape < 0 || us < best.us) best = {i, parts, us};
+    }
+  }
+  return best;
+}
+
+struct Operands {
+  bool fp8;
+  torch::Tensor x, w;  // x [*, K], w [E, N, K]
+  Args a;
+};
+
+// Offsets within a tile are 32 bits: rows under 8 MB apart (others are copied).
+torch::Tensor near_rows(const torch::Tensor& t) {
+  const int64_t es = t.element_size(), far = (int64_t)1 << 23;
+  const int d = t.dim() - 2;
+  return t.stride(d) * es < far ? t : t.contiguous();
+}
+
+Operands operands(const torch::Tensor& x0, const torch::Tensor& w0,
+                  const c10::optional<torch::Tensor>& sx,
+                  const c10::optional<torch::Tensor>& sw, bool raw) {
+  const bool fp8 = w0.scalar_type() == torch::kFloat8_e4m3fn;
+  TORCH_CHECK(fp8 || w0.scalar_type() == torch::kBFloat16);
+  TORCH_CHECK(x0.scalar_type() == w0.scalar_type() && x0.is_cuda() && w0.is_cuda());
+  TORCH_CHECK(x0.dim() == 2 && w0.dim() == 3 && x0.size(1) == w0.size(2));
+  TORCH_CHECK(x0.stride(1) == 1 && w0.stride(2) == 1);
+  Operands o{fp8, near_rows(x0), near_rows(w0), {}};
+  const auto &x = o.x, &w = o.w;
+  const int es = fp8 ? 1 : 2;
+  const int64_t E = w.size(0), N = w.size(1), KB = w.size(2) * es;
+  const int64_t ldx = x.stride(0) * es, ldw = w.stride(1) * es, ew = w.stride(0) * es;
+  TORCH_CHECK(KB >= kStep && KB % kStep == 0 && KB < (int64_t)1 << 23);
+  TORCH_CHECK(N >= 4 && N % 4 == 0 && N < (int64_t)1 << 30 && E >= 1 && E < 65536);
+  TORCH_CHECK((x.size(0) < 2 || ldx >= KB) && ldx % 16 == 0 && ldw >= KB && ldw % 16 == 0 &&
+                  ew >= 0 && ew % 16 == 0 && ((uintptr_t)x.data_ptr() & 15) == 0 &&
+                  ((uintptr_t)w.data_ptr() & 15) == 0,
+              "16-byte aligned rows");
+  TORCH_CHECK(raw || fp8 == (sx.has_value() && sw.has_value()));
+  Args& a = o.a;
+  if (fp8 && !raw) {
+    TORCH_CHECK(sx->scalar_type() == torch::kFloat32 && sx->is_contiguous() &&
+                sx->is_cuda() && sx->numel() == x.size(0) &&
+                sw->scalar_type() == torch::kFloat32 && sw->is_contiguous() &&
+                sw->is_cuda() && sw->numel() == E * N &&
+                ((uintptr_t)sw->data_ptr() & 15) == 0);
+    a.sx = sx->data_ptr<float>();
+    a.sw = sw->data_ptr<float>();
+  }
+  a.x = (const char*)x.data_ptr();
+  a.w = (const char*)w.data_ptr();
+  a.E = (int)E;
+  a.N = (int)N;
+  a.KB = a.k_part = (int)KB;
+  a.ldx = ldx;
+  a.ldw = ldw;
+  a.ew = ew;
+  return o;
+}
+
+void check_result(const torch::Tensor& y, int64_t cols, Args& a) {
+  TORCH_CHECK(y.scalar_type() == torch::kBFloat16 && y.is_contiguous() && y.is_cuda() &&
+              y.dim() == 2 && y.size(1) == cols && y.size(0) < (int64_t)1 << 30);
+  a.R = (int)y.size(0);
+  a.y = (ushort*)y.data_ptr();
+  a.wide = cols % 8 == 0 && ((uintptr_t)y.data_ptr() & 15) == 0;
+}
+
+Epilogue epilogue_of(int64_t act, const Args& a) {
+  TORCH_CHECK(act >= 0 && act <= 2, "0: none, 1: silu, 2: gelu");
+  if (act == 0) return kRows;
+  TORCH_CHECK(a.N % 16 == 0 && a.N * a.ldw < (int64_t)1 << 31, "gate and up columns");
+  return act == 1 ? kSilu : kGelu;
+}
+
+void run(const Operands& o, Epilogue epi, int shape, int64_t grid) {
+  TORCH_CHECK(grid < (int64_t)1 << 30);
+  if (o.fp8) launch_fp8(shape, epi, o.a, (int)grid);
+  else launch_bf16(shape, epi, o.a, (int)grid);
+}
+
+}  // namespace
+}  // namespace tiled
+
+using namespace tiled;
+
+// y [R, N] = rows of x [*, K] times w[e]^T, w [E, N, K] with any strides of e
+// and n; bounds int32: E row counts or E + 1 offsets; src int32 [R] the rows
+// of x, or none; fp8: sx fp32 [rows of x], sw fp32 [E, N]; square fp32 [R]:
+// y = relu(product)^2 * square. act 1 or 2: y [R, N / 2] = silu or tanh-gelu of
+// the first N / 2 columns times the others.
+void grouped_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
+                    c10::optional<torch::Tensor> sx,
+                    c10::optional<torch::Tensor> sw, torch::Tensor bounds,
+                    c10::optional<torch::Tensor> src,
+                    c10::optional<torch::Tensor> square, int64_t act) {
+  const int64_t R = y.size(0);
+  if (src.has_value()) {
+    TORCH_CHECK(src->scalar_type() == torch::kInt32 && src->is_contiguous() &&
+                src->is_cuda() && src->numel() == R);
+    if (x.dim() == 2 && x.size(0) * x.stride(0) * x.element_size() >= (int64_t)1 << 31) {
+      // offsets of gathered rows are 32 bits
+      if (sx.has_value()) sx = sx->reshape(-1).index_select(0, *src);
+      x = x.view(torch::kUInt8).index_select(0, *src).view(x.scalar_type());
+      src = c10::nullopt;
+    }
+  }
+  Operands o = operands(x, w, sx, sw, false);
+  Args& a = o.a;
+  const int64_t E = a.E;
+  TORCH_CHECK(bounds.scalar_type() == torch::kInt32 && bounds.is_contiguous() &&
+              bounds.is_cuda() && (bounds.numel() == E || bounds.numel() == E + 1));
+  Epilogue epi = epilogue_of(act, a);
+  const int64_t cols = epi == kRows ? a.N : a.N / 2;
+  check_result(y, cols, a);
+  if (!src.has_value()) TORCH_CHECK(o.x.size(0) == R);
+  if (square.has_value()) {
+    TORCH_CHECK(!o.fp8 && act == 0 && square->scalar_type() == torch::kFloat32 &&
+                square->is_contiguous() && square->is_cuda() && square->numel() == R);
+    a.row_weight = square->data_ptr<float>();
+    epi = kSquare;
+  }
+  TORCH_CHECK(!(o.fp8 && epi == kGelu), "gelu: bf16");
+  if (R == 0) return;
+  a.bounds = bounds.data_ptr<int32_t>();
+  a.offsets = bounds.numel() == E + 1;
+  a.src = src.has_value() ? src->data_ptr<int32_t>() : nullptr;
+  a.xbytes = (o.x.size(0) - 1) * a.ldx + a.KB;
+  const bool halves = epi == kSilu || epi == kGelu;
+  const Plan p = plan(o.fp8, R, E, cols, a.KB, halves, false);
+  const Shape s = kShapes[p.shape];
+  const int64_t bn = s.cols() / (halves ? 2 : 1);
+  run(o, epi, p.shape, (R / s.rows() + std::min(E, R)) * ((cols + bn - 1) / bn));
+}
+
+// y [M, N] = x [M, K] w [N, K]^T with the operands, scales and act of
+// grouped_linear
+void tiled_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
+                  c10::optional<torch::Tensor> sx, c10::optional<torch::Tensor> sw,
+                  int64_t act) {
+  Operands o = operands(x, w.unsqueeze(0), sx, sw, false);
+  Args& a = o.a;
+  const Epilogue epi = epilogue_of(act, a);
+  const int64_t cols = epi == kRows ? a.N : a.N / 2;
+  check_result(y, cols, a);
+  TORCH_CHECK(o.x.size(0) == a.R && !(o.fp8 && epi == kGelu));
+  if (a.R == 0) return;
+  const Plan p = plan(o.fp8, a.R, 1, cols, a.KB, epi != kRows, false);
+  const Shape s = kShapes[p.shape];
+  const int64_t bn = s.cols() / (epi != kRows ? 2 : 1);
+  run(o, epi, p.shape, (a.R + s.rows() - 1) / s.rows() * ((cols + bn - 1) / bn));
+}
+
+// the fp32 sums of x w^T alone, [parts, M, N], for a consumer that adds the
+// parts itself (and applies an fp8 product's scales)
+torch::Tensor tiled_sums(torch::Tensor x, torch::Tensor w) {
+  Operands o = operands(x, w.unsqueeze(0), c10::nullopt, c10::nullopt, true);
+  Args& a = o.a;
+  TORCH_CHECK(o.x.size(0) < (int64_t)1 << 30);
+  a.R = (int)o.x.size(0);
+  const Plan p = plan(o.fp8, a.R, 1, a.N, a.KB, false, true);
+  auto part = torch::empty({p.parts, a.R, a.N}, x.options().dtype(torch::kFloat32));
+  if (a.R == 0) return part;
+  const int steps = a.KB / kStep;
+  a.k_part = (steps + p.parts - 1) / p.parts * kStep;
+  a.part = part.data_ptr<float>();
+  const Shape s = kShapes[p.shape];
+  run(o, kSums, p.shape,
+      (int64_t)(a.R + s.rows() - 1) / s.rows() * ((a.N + s.cols() - 1) / s.cols()) * p.parts);
+  return part;
+}

@@ -276,7 +276,7 @@ class MoEMLP(nn.Module):
     read once, for its own rows only. The experts' weights lie behind one
     another in one tensor for that; the modules' parameters are views of it.
     Larger steps sort the rows by expert on the device; a projection is one
-    tiled product for all experts (csrc/grouped_gemm.hip) or, where that is the
+    tiled product for all experts (csrc/tiled_gemm.h) or, where that is the
     slower one, the library's on each expert's slice, after one look at the
     experts' row counts."""
 

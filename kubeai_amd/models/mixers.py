@@ -654,7 +654,7 @@ class ExpertRows:
     """The tokens of a large step in expert order: rows of one buffer, so that
     each product and each pass between them is one launch for all experts, and
     the row counts stay on the device. Where the products are the library's
-    (types and sizes that csrc/grouped_gemm.hip does not take or is slower for)
+    (types and sizes that csrc/tiled_gemm.h does not take or is slower for)
     there is one per expert, and the counts come to the host: they need shapes."""
 
     def __init__(self, h, index, weights, experts: int):

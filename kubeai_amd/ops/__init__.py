@@ -509,6 +509,7 @@ def grouped_linear_takes(x, w) -> bool:
         and x.dtype in (torch.bfloat16, torch.float8_e4m3fn)
         and x.stride(1) == w.stride(2) == 1
         and w.shape[2] * es % 128 == 0
+        and w.shape[2] * es < 2**23
         and w.shape[1] % 4 == 0
         and 0 < w.shape[0] < 65536
         and x.stride(0) * es % 16 == w.stride(0) * es % 16 == w.stride(1) * es % 16 == 0
@@ -541,7 +542,7 @@ def grouped_linear(x, w, bounds, src=None, scales=None, square=None):
     _require_ext()
     n = x.shape[0] if src is None else src.shape[0]
     y = torch.empty((n, w.shape[1]), dtype=torch.bfloat16, device=x.device)
-    _C.grouped_linear(y, x, w, *(scales or (None, None)), bounds, src, square)
+    _C.grouped_linear(y, x, w, *(scales or (None, None)), bounds, src, square, 0)
     return y
 
 
