@@ -30,9 +30,10 @@
 //    accumulators, 13000 now; the loop takes 83000).
 //  - an XCD's tiles are consecutive, up to 8 row tiles down one column, then the
 //    next column: they read the same rows of w from its L2.
-// us, library / this: fp8 28672 x 4096 512 rows 59 / 53, 640 rows 110 / 76, 2048
-// rows 219 / 199, 4096 rows 375 / 365; 4096 x 14336 2048 rows 108 / 96; bf16 28672 x
-// 4096 2048 rows 329 / 376 (the library stays).
+// us, weights out of cache, library / this: fp8 28672 x 4096 384 rows 60 / 45, 2048
+// rows 228 / 211, 8192 rows 764 / 743; 4096 x 4096 384 rows 14.9 / 12.0; 4096 x 14336
+// 4480 rows 264 / 233; bf16 28672 x 4096 384 rows 83 / 84, 2048 rows 333 / 391 (1.65
+// GHz; the library stays); 128256 x 4096 96 rows 225 / 207.
 #pragma once
 
 #include <algorithm>
@@ -172,10 +173,7 @@ DEV_INLINE Work find_tile(const Args& a, int nt) {
       int row, col;
       place(id - (tiles0 + __shfl(tiles - t, f)) * nt, mine, nt, &row, &col);
       row = first + row * BM;
-      return {__builtin_amdgcn_readfirstlane(base + f),
-              __builtin_amdgcn_readfirstlane(row),
-              __builtin_amdgcn_readfirstlane(max(0, min(BM, end - row))),
-              __builtin_amdgcn_readfirstlane(col), 0};
+      return {base + f, row, max(0, min(BM, end - row)), col, 0};
     }
     tiles0 += __shfl(tiles, 63);
     rows0 += __shfl(rows, 63);
@@ -199,7 +197,13 @@ __global__ __launch_bounds__(256, kShapes[SHAPE].per_cu()) void tiled_kernel(con
   __shared__ __attribute__((aligned(16))) char lds[kBytes];
 
   const int N = a.N, cols = kHalves ? N / 2 : N;  // of the result
-  const Work work = find_tile<BM>(a, (cols + OUT - 1) / OUT);
+  Work work = find_tile<BM>(a, (cols + OUT - 1) / OUT);
+  // the same in every lane: buffers are described in scalar registers
+  work.expert = __builtin_amdgcn_readfirstlane(work.expert);
+  work.row = __builtin_amdgcn_readfirstlane(work.row);
+  work.rows = __builtin_amdgcn_readfirstlane(work.rows);
+  work.col = __builtin_amdgcn_readfirstlane(work.col);
+  work.part = __builtin_amdgcn_readfirstlane(work.part);
   if (work.rows <= 0) return;
   const int m0 = work.row, rows = work.rows, n0 = work.col * OUT;
   const int k0 = work.part * a.k_part;

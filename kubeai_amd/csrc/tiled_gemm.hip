@@ -9,32 +9,35 @@
 namespace tiled {
 namespace {
 
-// A launch takes passes over the CUs x (steps x step + tile) + rest, us. One
-// matrix: fitted to 1100 products (128 to 4096 rows, 4096 to 28672 columns, K 4096
-// and 14336, whole and in 2 to 8 parts; 10 % off in the mean, and the shape with
-// the least at most 6 % slower than the best one). With parts, what reads the
-// sums adds their bytes at 4.5 TB/s. Experts, whose weights are used by few row
-// tiles and come from memory: 8 of 3584 x 2048 to 28672 x 4096, 24 to 1024 rows
-// each; there the choice is 2 % slower than the best in the mean.
+// A launch takes passes over the CUs x (steps x step + tile) + rest us, and mb us
+// for each MB of sums. One matrix: fitted to 225 products of each shape and type (40
+// to 8192 rows, 1024 to 32000 columns, K 512 to 14336, weights out of cache), 8 to 15 %
+// off in the mean; the shape with the least is 0.1 % slower than the best one in
+// the mean, 15 % at worst. Sums: the same products in 1 to 8 parts; what reads
+// them adds their bytes at 4.5 TB/s (0.9 %, 20 %). Experts, whose weights are
+// used by few row tiles and come from memory: 8 of 3584 x 2048 to 28672 x 4096, 24 to
+// 1024 rows each (1.8 %, 17 %).
 struct Cost {
-  float step, tile, rest;
+  float step, tile, rest, mb;
 };
-constexpr Cost kFp8[kNumShapes] = {
-    {0.965f, 21.2f, -7.9f}, {0.779f, 14.4f, -2.7f}, {0.800f, 18.0f, -7.3f},
-    {0.660f, 12.3f, -3.3f}, {0.664f, 9.3f, -0.6f},  {0.520f, 6.2f, 0.6f},
-    {0.444f, 4.3f, 0.7f},   {0.355f, 0.7f, 1.8f}};
-constexpr Cost kBf16[kNumShapes] = {
-    {0.973f, 37.8f, -23.3f}, {0.794f, 24.4f, -11.6f}, {0.777f, 28.6f, -16.3f},
-    {0.668f, 16.7f, -6.3f},  {0.724f, 9.5f, 0.2f},    {0.557f, 6.7f, 1.6f},
-    {0.490f, 2.6f, 4.1f},    {0.387f, -1.1f, 5.8f}};
-constexpr Cost kExpertsFp8[kNumShapes] = {
-    {1.427f, 20.3f, -5.7f}, {1.113f, 17.9f, 5.0f},  {1.126f, 16.1f, 1.4f},
-    {0.859f, 15.5f, 10.2f}, {0.758f, 15.6f, 22.5f}, {0.720f, 8.8f, 11.5f},
-    {0.520f, 8.0f, 22.1f},  {0.383f, 5.8f, 33.1f}};
-constexpr Cost kExpertsBf16[kNumShapes] = {
-    {1.577f, 26.2f, -16.1f}, {1.293f, 16.7f, -9.4f}, {1.285f, 15.9f, -6.7f},
-    {1.074f, 10.7f, -4.6f},  {1.043f, 10.3f, -4.4f}, {0.883f, 4.6f, 0.8f},
-    {0.680f, 3.6f, 3.8f},    {0.503f, 2.5f, 6.3f}};
+constexpr Cost kOne[2][kNumShapes] = {
+    {{1.083f, 8.7f, 0.f}, {0.869f, 6.7f, 0.f}, {0.878f, 7.1f, 0.f}, {0.724f, 5.5f, 0.f},
+     {0.752f, 4.1f, 0.f}, {0.577f, 3.7f, 0.f}, {0.484f, 2.6f, 0.f}, {0.357f, 1.3f, 1.1f}},
+    {{1.058f, 10.8f, 0.f}, {0.874f, 9.1f, 0.f}, {0.877f, 10.9f, 0.f}, {0.710f, 9.0f, 0.f},
+     {0.676f, 6.7f, 0.f}, {0.518f, 5.6f, 0.f}, {0.404f, 4.4f, 0.f}, {0.292f, 2.5f, 1.2f}}};
+constexpr Cost kParts[2][kNumShapes] = {
+    {{1.081f, 2.5f, 5.2f, 0.21f}, {0.857f, 0.8f, 5.3f, 0.25f}, {0.869f, 1.3f, 5.1f, 0.23f},
+     {0.701f, 1.0f, 4.3f, 0.25f}, {0.742f, 0.f, 4.4f, 0.27f},  {0.568f, 0.6f, 3.3f, 0.28f},
+     {0.480f, 0.4f, 2.6f, 0.31f}, {0.365f, 1.0f, 1.9f, 0.27f}},
+    {{1.036f, 2.7f, 5.4f, 0.20f}, {0.835f, 1.5f, 5.5f, 0.23f}, {0.852f, 2.7f, 4.5f, 0.20f},
+     {0.662f, 2.3f, 4.0f, 0.22f}, {0.660f, 0.8f, 4.6f, 0.24f}, {0.475f, 0.7f, 3.7f, 0.27f},
+     {0.379f, 0.9f, 3.1f, 0.28f}, {0.277f, 1.2f, 2.3f, 0.28f}}};
+constexpr Cost kExperts[2][kNumShapes] = {
+    {{1.219f, 11.4f, 0.f}, {1.037f, 7.7f, 0.f}, {1.012f, 8.6f, 0.f}, {0.825f, 7.8f, 0.f},
+     {0.907f, 5.8f, 0.f}, {0.720f, 4.4f, 0.2f}, {0.618f, 2.0f, 3.3f}, {0.444f, 0.f, 9.5f}},
+    {{1.169f, 20.2f, 0.f}, {0.983f, 15.6f, 0.9f}, {0.963f, 14.9f, 0.f}, {0.701f, 14.9f, 10.7f},
+     {0.685f, 13.0f, 26.8f}, {0.634f, 6.7f, 11.9f}, {0.513f, 6.2f, 22.3f}, {0.356f, 4.5f, 36.5f}}};
+constexpr double kReadMb = 1. / 4.5;
 constexpr int kMaxParts = 8;
 
 struct Plan {
@@ -49,7 +52,7 @@ Plan plan(bool fp8, int64_t R, int64_t E, int64_t cols, int64_t KB, bool halves,
   for (int i = 0; i < kNumShapes; i++) {
     const Shape s = kShapes[i];
     if (halves && s.wn % 2) continue;
-    const Cost c = E > 1 ? (fp8 ? kExpertsFp8[i] : kExpertsBf16[i]) : (fp8 ? kFp8[i] : kBf16[i]);
+    const Cost c = (E > 1 ? kExperts : sums ? kParts : kOne)[fp8][i];
     const int64_t bn = s.cols() / (halves ? 2 : 1), nt = (cols + bn - 1) / bn;
     double row_tiles = (R + s.rows() - 1) / s.rows();
     if (E > 1) {  // the mean over row counts within 30 % of an even split
@@ -63,7 +66,7 @@ Plan plan(bool fp8, int64_t R, int64_t E, int64_t cols, int64_t KB, bool halves,
       if (parts > 1 && (steps < 4 || (all + steps - 1) / steps != parts)) continue;
       const double passes = std::ceil(row_tiles * nt * parts / (256 * s.per_cu()));
       const double us = passes * (steps * c.step + c.tile) + c.rest +
-                        (sums ? parts * R * cols * 4 / 4.5e6 : 0.);
+                        (sums ? parts * R * cols * 4e-6 * (c.mb + kReadMb) : 0.);
       if (best.shape < 0 || us < best.us) best = {i, parts, us};
     }
   }
