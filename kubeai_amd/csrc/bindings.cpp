@@ -56,6 +56,8 @@ void tiled_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                   c10::optional<torch::Tensor> sx,
                   c10::optional<torch::Tensor> sw, int64_t act);
 torch::Tensor tiled_sums(torch::Tensor x, torch::Tensor w);
+std::tuple<int64_t, int64_t, double> tiled_plan(int64_t M, int64_t N, int64_t KB,
+                                                bool fp8, bool sums);
 void moe_route(torch::Tensor index, torch::Tensor weight, torch::Tensor begin,
                torch::Tensor src, torch::Tensor place, torch::Tensor x,
                torch::Tensor w);
@@ -119,6 +121,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("grouped_linear", &grouped_linear,
         "all experts' products of a large step, bf16 or fp8 e4m3");
   m.def("tiled_linear", &tiled_linear, "product of many rows, bf16 or scaled fp8");
+  m.def("tiled_plan", &tiled_plan,
+        "tile shape, parts and us of a tiled product, whole or as sums");
   m.def("tiled_sums", &tiled_sums, "fp32 part sums of a product of many rows");
   m.def("skinny_sums", &skinny_sums, "fp32 part sums of a skinny product");
   m.def("quant_fp8_rows", &quant_fp8_rows, "gathered bf16 rows -> fp8");

@@ -238,3 +238,12 @@ torch::Tensor tiled_sums(torch::Tensor x, torch::Tensor w) {
       (int64_t)(a.R + s.rows() - 1) / s.rows() * ((a.N + s.cols() - 1) / s.cols()) * p.parts);
   return part;
 }
+
+// How a product is planned, whole or as its sums: tile shape, parts of K, us (with
+// the reading of the sums)
+std::tuple<int64_t, int64_t, double> tiled_plan(int64_t M, int64_t N, int64_t KB, bool fp8,
+                                                bool sums) {
+  TORCH_CHECK(M >= 1 && N >= 1 && KB >= kStep && KB % kStep == 0);
+  const Plan p = plan(fp8, M, 1, N, KB, false, sums);
+  return {p.shape, p.parts, p.us};
+}

@@ -3,8 +3,8 @@
 MI355X-first: gfx950's fp8 MFMA peak is ~2x bf16 and — what actually
 matters for skinny decode GEMMs — fp8 weights halve the HBM bytes per
 step. The BASELINE headline config is Llama-3.1-8B-Instruct-FP8, so this
-is the config-faithful serving mode. GEMMs go through torch._scaled_mm
-(hipBLASLt fp8 path); gfx950 uses OCP e4m3fn, not the MI300X fnuz variant.
+is the config-faithful serving mode. Products go through ops.linear_fp8
+(streaming or tiled kernels, torch._scaled_mm for the rest); gfx950 uses OCP e4m3fn, not the MI300X fnuz variant.
 
 Scheme: W8A8 dynamic — per-output-channel weight scales, per-token
 activation scales (amax/448), bf16 output.
@@ -68,12 +68,16 @@ class Fp8Linear(nn.Module):
         or None (library product)."""
         w = self.weight_fp8
         if (
-            self.bias is not None or xq.shape[0] > 96
+            self.bias is not None
             or type(self).forward_quantized is not Fp8Linear.forward_quantized
-            or not ops.sums_better(
-                xq.shape[0], *w.shape, fp8=True, rope=rope, eager=eager
-            )
         ):
+            return None
+        if xq.shape[0] > 96:
+            better = not rope and ops.tiled_sums_better(xq.shape[0], *w.shape, fp8=True)
+            return ops.tiled_sums(
+                xq, w, x_scale, self.weight_scale.view(-1)
+            ) if better else None
+        if not ops.sums_better(xq.shape[0], *w.shape, fp8=True, rope=rope, eager=eager):
             return None
         return ops.product_sums(xq, w, x_scale, self.weight_scale.view(-1))
 

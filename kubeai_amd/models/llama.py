@@ -39,7 +39,12 @@ class EngineLinear(nn.Linear):
         """The product as ops.ProductSums, for a norm or (rope) the rotation, or
         None (library product, bias)."""
         w = self.weight
-        if self.bias is not None or x.shape[0] > 96 or not ops.sums_better(
+        if self.bias is not None:
+            return None
+        if x.shape[0] > 96:
+            better = not rope and ops.tiled_sums_better(x.shape[0], *w.shape, fp8=False)
+            return ops.tiled_sums(x, w) if better else None
+        if not ops.sums_better(
             x.shape[0], *w.shape, fp8=False, rope=rope, eager=eager
         ):
             return None
@@ -586,8 +591,8 @@ class DecoderLayer(nn.Module):
     def forward(self, x, residual, fb, kv_cache, cos_sin, as_sums: bool = False):
         """as_sums: the caller takes the branch as ops.ProductSums too (x may be
         that in any case)."""
-        # products are handed on as sums in steps of up to 96 rows only
-        branch = _branch if x.shape[0] <= 96 else _call
+        # products are handed on as sums in steps of few rows only
+        branch = _branch if x.shape[0] <= ops.MAX_SUM_ROWS else _call
         last = branch if as_sums else _call
         if self.post_norms:
             # incoming invariant: hidden = x + residual (residual None at
@@ -724,7 +729,7 @@ class LlamaForCausalLM(nn.Module):
         n = len(self.layers)
         # layers that nobody else looks at hand on products that the next one's
         # (or the final) norm adds up
-        few = x.shape[0] <= 96
+        few = x.shape[0] <= ops.MAX_SUM_ROWS
         own = [few and type(layer) is DecoderLayer and not _hooked(layer)
                for layer in self.layers]
         for i, layer in enumerate(self.layers):

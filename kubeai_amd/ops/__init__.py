@@ -7,6 +7,8 @@ reference implementations (ref.py) so the engine logic is testable anywhere.
 """
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from . import ref
@@ -351,9 +353,87 @@ def _streams_better(M: int, N: int, K: int, fp8: bool) -> bool:
     return N >= 16384 and K <= 1024 or N > 16384 and K <= (6144 if M <= 8 else 4096)
 
 
+def _tiled_operands(x, weight) -> bool:
+    """Operands that the tiled product takes (and the library, which refuses fp8
+    columns that are no multiple of 16)."""
+    es = x.element_size()
+    return (
+        _C is not None
+        and x.is_cuda
+        and weight.device == x.device
+        and x.dtype == weight.dtype
+        and x.dtype in (torch.bfloat16, torch.float8_e4m3fn)
+        and x.dim() == weight.dim() == 2
+        and x.shape[0] >= 1
+        and x.shape[1] == weight.shape[1]
+        and x.is_contiguous()
+        and weight.is_contiguous()
+        and weight.shape[1] * es % 128 == 0
+        and weight.shape[1] * es < 2**23
+        and weight.shape[0] % 16 == 0
+        and not observed(x, weight)
+        and aligned(x, weight)
+    )
+
+
+def _tiled_better(M: int, N: int, K: int, fp8: bool) -> bool:
+    """Whether the tiled product (csrc/tiled_gemm.h) beats the library's. fp8: from
+    97 rows on, unless K is short, where the stores count (us, weights out of
+    cache, library / this: 16384 x 512 8192 rows 104 / 127, 1024 x 1024 4.8 / 5.8) or
+    so long that the tiles of few columns leave CUs idle while few rows are
+    multiplied (4096 x 14336 256 rows 34 / 49, 2304 x 9216 160 rows 16 / 22; 640 rows
+    72 / 63 and 29 / 28). Over 137 others (97 to 8192 rows, 2048 to 32000 columns) it
+    takes 0.87 of the library's time, 1.06 at worst. Logits of few rows: 128256 x
+    4096 fp8 40 rows 129 / 107, 96 rows 121 / 118, bf16 40 rows 203 / 192, 160
+    rows 246 / 213, 384 rows 437 / 339, 1024 rows 853 / 838; 57344 x 8192 fp8 40 rows
+    121 / 103. Other bf16 products stay (28672 x 4096 2048 rows 333 / 391)."""
+    if N >= 49152 and K >= 2048:
+        return M > 16 and (fp8 or M <= 1024 and N >= 98304)
+    return fp8 and M > 96 and K >= 2048 and (K <= 2 * N or M > 512)
+
+
+def _tiled_linear(x, weight, x_scale=None, w_scale=None, out=None):
+    if out is None:
+        out = torch.empty(
+            (x.shape[0], weight.shape[0]), dtype=torch.bfloat16, device=x.device
+        )
+    _C.tiled_linear(out, x, weight, x_scale, w_scale, 0)
+    return out
+
+
+#: Products of more rows are not handed on as sums: whole ones fill the chip.
+MAX_SUM_ROWS = 2048
+
+
+@functools.lru_cache(maxsize=4096)
+def tiled_sums_better(M: int, N: int, K: int, fp8: bool) -> bool:
+    """Whether a product of more than 96 rows as ProductSums of a tiled product
+    that is cut along K and the norm that adds them beat the product as a whole
+    and its norm: where its tiles alone leave CUs idle. By the costs of both
+    (csrc/tiled_gemm.hip); against the library in bf16, which is about as fast
+    as a whole tiled product, better over 50 of 50 chosen products of 160 to 2048
+    rows but four (0.95 at worst; 1.6 in the mean), us with the norm's reading:
+    4096 x 14336 160 rows fp8 49.2 / 29.1, bf16 86.4 / 38.0; 384 rows 53.5 / 41.0, 81.8 /
+    58.5; 1024 rows bf16 138 / 117; 4096 x 4096 160 rows bf16 30.7 / 19."""
+    es = 1 if fp8 else 2
+    if _C is None or not 96 < M <= MAX_SUM_ROWS or N > 16384 or K * es % 128:
+        return False
+    whole = _C.tiled_plan(M, N, K * es, fp8, False)[2]
+    return _C.tiled_plan(M, N, K * es, fp8, True)[2] < 0.95 * whole
+
+
+def tiled_sums(x, weight, x_scale=None, w_scale=None):
+    """x weight^T as ProductSums of the tiled product, cut along K so that it
+    fills the chip, or None for operands that it does not take."""
+    if not _tiled_operands(x, weight):
+        return None
+    return ProductSums(_C.tiled_sums(x, weight), x_scale, w_scale)
+
+
 def linear(x, weight):
     """x weight^T. Few rows against a wide or a very long weight go through the
-    weight-streaming kernel (csrc/skinny_gemm.hip), the rest to the library."""
+    weight-streaming kernel (csrc/skinny_gemm.hip), logits through the tiled one
+    (csrc/tiled_gemm.h), the rest to the library."""
     if (
         x.dim() == weight.dim() == 2
         and x.shape[0] <= 96
@@ -368,6 +448,14 @@ def linear(x, weight):
         )
         _C.skinny_linear(y, x, weight, None, None, None)
         return y
+    if (
+        x.is_cuda
+        and x.dim() == weight.dim() == 2
+        and x.dtype == torch.bfloat16
+        and _tiled_better(x.shape[0], *weight.shape, fp8=False)
+        and _tiled_operands(x, weight)
+    ):
+        return _tiled_linear(x, weight)
     return torch.nn.functional.linear(x, weight)
 
 
@@ -386,6 +474,13 @@ def linear_fp8(xq, x_scale, weight, w_scale, bias=None, out=None):
             )
         _C.skinny_linear(out, xq, weight, x_scale.reshape(-1), w_scale.reshape(-1), bias)
         return out
+    if (
+        bias is None
+        and _tiled_better(xq.shape[0], *weight.shape, fp8=True)
+        and _tiled_operands(xq, weight)
+        and (out is None or out.is_contiguous() and out.dtype == torch.bfloat16)
+    ):
+        return _tiled_linear(xq, weight, x_scale.reshape(-1), w_scale.reshape(-1), out)
     kw = {} if out is None else {"out": out}
     return torch._scaled_mm(
         xq, weight.t(), scale_a=x_scale.view(-1, 1), scale_b=w_scale, bias=bias,
