@@ -51,10 +51,10 @@ void grouped_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                     c10::optional<torch::Tensor> sx,
                     c10::optional<torch::Tensor> sw, torch::Tensor bounds,
                     c10::optional<torch::Tensor> src,
-                    c10::optional<torch::Tensor> square, int64_t act);
+                    c10::optional<torch::Tensor> square, bool silu);
 void tiled_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                   c10::optional<torch::Tensor> sx,
-                  c10::optional<torch::Tensor> sw, int64_t act);
+                  c10::optional<torch::Tensor> sw, bool silu);
 torch::Tensor tiled_sums(torch::Tensor x, torch::Tensor w);
 std::tuple<int64_t, int64_t, double> tiled_plan(int64_t M, int64_t N, int64_t KB,
                                                 bool fp8, bool sums);

@@ -1,8 +1,8 @@
 // Products of many rows: y[i] = x[i] w^T, or for the rows of every expert e of a
 // mixture y[i] = x[src[i]] w[e]^T in one launch; bf16 or fp8 e4m3 (W8A8 with row
 // and column scales), fp32 accumulation. What the epilogue makes of them: bf16
-// rows, fp32 sums of a part of K, silu or tanh-gelu(gate) * up of stacked gate
-// and up columns, or relu(.)^2 times a weight per row.
+// rows, fp32 sums of a part of K, silu(gate) * up of stacked gate and up columns
+// (in fp32, rounded once), or relu(.)^2 times a weight per row.
 //
 // Bound by the matrix cores (and the power they draw: dense bf16 runs at 1.65
 // GHz here), as long as nothing keeps them waiting. What it takes:
@@ -33,7 +33,9 @@
 // us, weights out of cache, library / this: fp8 28672 x 4096 384 rows 60 / 45, 2048
 // rows 228 / 211, 8192 rows 764 / 743; 4096 x 4096 384 rows 14.9 / 12.0; 4096 x 14336
 // 4480 rows 264 / 233; bf16 28672 x 4096 384 rows 83 / 84, 2048 rows 333 / 391 (1.65
-// GHz; the library stays); 128256 x 4096 96 rows 225 / 207.
+// GHz; the library stays); 128256 x 4096 96 rows 225 / 207. 28672 x 4096 with silu
+// and up, as two launches / here (fp8: and the conversion of what comes out): fp8
+// 384 rows 57.0 / 54.9, 8192 rows 923 / 858; bf16 384 rows 92 / 89.
 #pragma once
 
 #include <algorithm>
@@ -43,7 +45,7 @@
 
 namespace tiled {
 
-enum Epilogue { kRows, kSums, kSilu, kGelu, kSquare };
+enum Epilogue { kRows, kSums, kSilu, kSquare };
 
 struct Args {
   ushort* y;        // [R, columns]
@@ -187,7 +189,7 @@ __global__ __launch_bounds__(256, kShapes[SHAPE].per_cu()) void tiled_kernel(con
   constexpr int WM = S.wm, WN = S.wn, NA = S.na, NB = S.nb;
   static_assert(NA >= 2 && (NB == NA || (NA == 2 && NB == 3)));
   constexpr int BM = S.rows(), BN = S.cols();
-  constexpr bool kHalves = EPI == kSilu || EPI == kGelu;  // gate | up columns
+  constexpr bool kHalves = EPI == kSilu;  // gate | up columns
   static_assert(!kHalves || WN % 2 == 0);
   constexpr int OUT = kHalves ? BN / 2 : BN;  // columns of the result
   constexpr int AC = BM / 32, BC = BN / 32, L = AC + BC;  // loads per wave and step
@@ -432,12 +434,7 @@ __global__ __launch_bounds__(256, kShapes[SHAPE].per_cu()) void tiled_kernel(con
 #pragma unroll
           for (int t = 0; t < 4; t++) {
             const float g = v[h][t];
-            if constexpr (EPI == kSilu) {
-              v[h][t] = g / (1.0f + __expf(-g)) * up[h][t];
-            } else {  // sqrt(2 / pi)
-              const float th = tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g));
-              v[h][t] = 0.5f * g * (1.0f + th) * up[h][t];
-            }
+            v[h][t] = g / (1.0f + __expf(-g)) * up[h][t];
           }
         }
         bf4 b = __builtin_convertvector(v[h], bf4);
@@ -469,7 +466,7 @@ void launch(int shape, const Args& a, int grid) {
   auto stream = c10::hip::getCurrentHIPStream().stream();
   auto go = [&](auto s) {
     constexpr int i = decltype(s)::value;
-    if constexpr ((EPI != kSilu && EPI != kGelu) || kShapes[i].wn % 2 == 0) {
+    if constexpr (EPI != kSilu || kShapes[i].wn % 2 == 0) {
       hipLaunchKernelGGL((tiled_kernel<FP8, i, EPI>), dim3(grid), dim3(256), 0, stream, a);
     } else {
       TORCH_CHECK(false, "no such tile");

@@ -135,11 +135,10 @@ void check_result(const torch::Tensor& y, int64_t cols, Args& a) {
   a.wide = cols % 8 == 0 && ((uintptr_t)y.data_ptr() & 15) == 0;
 }
 
-Epilogue epilogue_of(int64_t act, const Args& a) {
-  TORCH_CHECK(act >= 0 && act <= 2, "0: none, 1: silu, 2: gelu");
-  if (act == 0) return kRows;
+Epilogue epilogue_of(bool silu, const Args& a) {
+  if (!silu) return kRows;
   TORCH_CHECK(a.N % 16 == 0 && a.N * a.ldw < (int64_t)1 << 31, "gate and up columns");
-  return act == 1 ? kSilu : kGelu;
+  return kSilu;
 }
 
 void run(const Operands& o, Epilogue epi, int shape, int64_t grid) {
@@ -156,13 +155,13 @@ using namespace tiled;
 // y [R, N] = rows of x [*, K] times w[e]^T, w [E, N, K] with any strides of e
 // and n; bounds int32: E row counts or E + 1 offsets; src int32 [R] the rows
 // of x, or none; fp8: sx fp32 [rows of x], sw fp32 [E, N]; square fp32 [R]:
-// y = relu(product)^2 * square. act 1 or 2: y [R, N / 2] = silu or tanh-gelu of
-// the first N / 2 columns times the others.
+// y = relu(product)^2 * square. silu: y [R, N / 2] = silu of the first N / 2 columns
+// times the others.
 void grouped_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                     c10::optional<torch::Tensor> sx,
                     c10::optional<torch::Tensor> sw, torch::Tensor bounds,
                     c10::optional<torch::Tensor> src,
-                    c10::optional<torch::Tensor> square, int64_t act) {
+                    c10::optional<torch::Tensor> square, bool silu) {
   const int64_t R = y.size(0);
   if (src.has_value()) {
     TORCH_CHECK(src->scalar_type() == torch::kInt32 && src->is_contiguous() &&
@@ -179,44 +178,42 @@ void grouped_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   const int64_t E = a.E;
   TORCH_CHECK(bounds.scalar_type() == torch::kInt32 && bounds.is_contiguous() &&
               bounds.is_cuda() && (bounds.numel() == E || bounds.numel() == E + 1));
-  Epilogue epi = epilogue_of(act, a);
-  const int64_t cols = epi == kRows ? a.N : a.N / 2;
+  Epilogue epi = epilogue_of(silu, a);
+  const int64_t cols = silu ? a.N / 2 : a.N;
   check_result(y, cols, a);
   if (!src.has_value()) TORCH_CHECK(o.x.size(0) == R);
   if (square.has_value()) {
-    TORCH_CHECK(!o.fp8 && act == 0 && square->scalar_type() == torch::kFloat32 &&
+    TORCH_CHECK(!o.fp8 && !silu && square->scalar_type() == torch::kFloat32 &&
                 square->is_contiguous() && square->is_cuda() && square->numel() == R);
     a.row_weight = square->data_ptr<float>();
     epi = kSquare;
   }
-  TORCH_CHECK(!(o.fp8 && epi == kGelu), "gelu: bf16");
   if (R == 0) return;
   a.bounds = bounds.data_ptr<int32_t>();
   a.offsets = bounds.numel() == E + 1;
   a.src = src.has_value() ? src->data_ptr<int32_t>() : nullptr;
   a.xbytes = (o.x.size(0) - 1) * a.ldx + a.KB;
-  const bool halves = epi == kSilu || epi == kGelu;
-  const Plan p = plan(o.fp8, R, E, cols, a.KB, halves, false);
+  const Plan p = plan(o.fp8, R, E, cols, a.KB, silu, false);
   const Shape s = kShapes[p.shape];
-  const int64_t bn = s.cols() / (halves ? 2 : 1);
+  const int64_t bn = s.cols() / (silu ? 2 : 1);
   run(o, epi, p.shape, (R / s.rows() + std::min(E, R)) * ((cols + bn - 1) / bn));
 }
 
-// y [M, N] = x [M, K] w [N, K]^T with the operands, scales and act of
+// y [M, N] = x [M, K] w [N, K]^T with the operands, scales and silu of
 // grouped_linear
 void tiled_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                   c10::optional<torch::Tensor> sx, c10::optional<torch::Tensor> sw,
-                  int64_t act) {
+                  bool silu) {
   Operands o = operands(x, w.unsqueeze(0), sx, sw, false);
   Args& a = o.a;
-  const Epilogue epi = epilogue_of(act, a);
-  const int64_t cols = epi == kRows ? a.N : a.N / 2;
+  const Epilogue epi = epilogue_of(silu, a);
+  const int64_t cols = silu ? a.N / 2 : a.N;
   check_result(y, cols, a);
-  TORCH_CHECK(o.x.size(0) == a.R && !(o.fp8 && epi == kGelu));
+  TORCH_CHECK(o.x.size(0) == a.R);
   if (a.R == 0) return;
-  const Plan p = plan(o.fp8, a.R, 1, cols, a.KB, epi != kRows, false);
+  const Plan p = plan(o.fp8, a.R, 1, cols, a.KB, silu, false);
   const Shape s = kShapes[p.shape];
-  const int64_t bn = s.cols() / (epi != kRows ? 2 : 1);
+  const int64_t bn = s.cols() / (silu ? 2 : 1);
   run(o, epi, p.shape, (a.R + s.rows() - 1) / s.rows() * ((cols + bn - 1) / bn));
 }
 

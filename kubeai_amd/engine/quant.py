@@ -60,6 +60,18 @@ class Fp8Linear(nn.Module):
             xq, x_scale, self.weight_fp8, self.weight_scale, self.bias
         )
 
+    def swiglu_quantized(self, xq: torch.Tensor, x_scale: torch.Tensor):
+        """silu(gate) * up of forward_quantized (gate columns, then up columns) in
+        bf16, or None (the product is to be made as a whole)."""
+        if (
+            self.bias is not None or not xq.is_cuda
+            or type(self).forward_quantized is not Fp8Linear.forward_quantized
+        ):
+            return None
+        return ops.tiled_swiglu(
+            xq, self.weight_fp8, x_scale, self.weight_scale.view(-1)
+        )
+
     def sums_quantized(
         self, xq: torch.Tensor, x_scale: torch.Tensor, rope: bool = False,
         eager: bool = False,

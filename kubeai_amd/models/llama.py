@@ -245,17 +245,30 @@ class MLP(nn.Module):
     ) -> torch.Tensor:
         """as_sums: the caller takes the result as ops.ProductSums too."""
         if isinstance(x, tuple):  # fused fp8 path (never active with LoRA)
-            h = self.gate_up_proj.forward_quantized(*x)
-            return _project(self.down_proj, ops.silu_and_mul_fp8(h), as_sums, fb)
-        h = self.gate_up_proj(x)
+            fused = getattr(self.gate_up_proj, "swiglu_quantized", None)
+            a = fused(*x) if fused is not None else None
+            if a is not None:
+                a = ops.quant_fp8(a)
+            else:
+                a = ops.silu_and_mul_fp8(self.gate_up_proj.forward_quantized(*x))
+            return _project(self.down_proj, a, as_sums, fb)
         lm = getattr(self, "_lora_manager", None)
         lora_live = (
             lm is not None and lm.active and fb is not None
             and fb.lora_ids is not None and self.layer_idx is not None
         )
-        if lora_live:
-            lm.apply(self.layer_idx, "gate_up", x, h, fb.lora_ids)
-        a = ops.gelu_and_mul(h) if self.gelu else ops.silu_and_mul(h)
+        a = None
+        if not (
+            lora_live or self.gelu or x.dim() != 2 or x.shape[0] <= 96
+            or type(self.gate_up_proj) is not EngineLinear or _hooked(self.gate_up_proj)
+            or self.gate_up_proj.bias is not None
+        ):
+            a = ops.tiled_swiglu(x, self.gate_up_proj.weight)
+        if a is None:
+            h = self.gate_up_proj(x)
+            if lora_live:
+                lm.apply(self.layer_idx, "gate_up", x, h, fb.lora_ids)
+            a = ops.gelu_and_mul(h) if self.gelu else ops.silu_and_mul(h)
         y = _project(self.down_proj, a, as_sums and not lora_live, fb)
         if lora_live:
             lm.apply(self.layer_idx, "down", a, y, fb.lora_ids)
@@ -427,7 +440,9 @@ class MoEMLP(nn.Module):
         fp8 = hasattr(first.gate_up_proj, "forward_quantized")
         ends = None
 
-        def products(rows, proj, width, src=None):
+        def products(rows, proj, width, src=None, silu=False):
+            """silu: of gate and up rows; the result has half the width then, or
+            the whole where the activation is still to be done."""
             nonlocal ends
             rows, scale = rows if fp8 else (rows, None)
             w = self._stack(proj, "weight_fp8" if fp8 else "weight")
@@ -436,8 +451,13 @@ class MoEMLP(nn.Module):
                 w is not None and (ws is not None) == fp8
                 and ops.grouped_linear_takes(rows, w) and ops.grouped_linear_better(n, w)
             ):
+                silu = silu and (
+                    w.shape[1] % 16 == 0
+                    and w.shape[1] * w.stride(1) * w.element_size() < 2**31
+                )
                 return ops.grouped_linear(
-                    rows, w, begin, src=src, scales=(scale, ws) if fp8 else None
+                    rows, w, begin, src=src, scales=(scale, ws) if fp8 else None,
+                    silu=silu,
                 )
             if src is not None:
                 rows = rows.index_select(0, src)
@@ -460,11 +480,12 @@ class MoEMLP(nn.Module):
 
         width = 2 * first.down_proj.in_features
         if fp8:
-            h = products(ops.quant_fp8_rows(x, src), "gate_up_proj", width)
-            a = ops.silu_and_mul_fp8(h)
+            h = products(ops.quant_fp8_rows(x, src), "gate_up_proj", width, silu=True)
+            a = ops.silu_and_mul_fp8(h) if h.shape[1] == width else ops.quant_fp8(h)
         else:
-            h = products(x, "gate_up_proj", width, src)
-            a = ops.gelu_and_mul(h) if self.gelu else ops.silu_and_mul(h)
+            a = products(x, "gate_up_proj", width, src, silu=not self.gelu)
+            if a.shape[1] == width:
+                a = ops.gelu_and_mul(a) if self.gelu else ops.silu_and_mul(a)
         return ops.moe_combine(products(a, "down_proj", x.shape[1]), place, weight)
 
     def _tiled_has(self, tokens: int) -> bool:
