@@ -78,20 +78,14 @@ class Fp8Linear(nn.Module):
     ):
         """forward_quantized as ops.ProductSums, for a norm or (rope) the rotation,
         or None (library product)."""
-        w = self.weight_fp8
         if (
             self.bias is not None
             or type(self).forward_quantized is not Fp8Linear.forward_quantized
         ):
             return None
-        if xq.shape[0] > 96:
-            better = not rope and ops.tiled_sums_better(xq.shape[0], *w.shape, fp8=True)
-            return ops.tiled_sums(
-                xq, w, x_scale, self.weight_scale.view(-1)
-            ) if better else None
-        if not ops.sums_better(xq.shape[0], *w.shape, fp8=True, rope=rope, eager=eager):
-            return None
-        return ops.product_sums(xq, w, x_scale, self.weight_scale.view(-1))
+        return ops.sums_for_reader(
+            xq, self.weight_fp8, x_scale, self.weight_scale.view(-1), rope, eager
+        )
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if (

@@ -38,17 +38,9 @@ class EngineLinear(nn.Linear):
     def sums(self, x: torch.Tensor, rope: bool = False, eager: bool = False):
         """The product as ops.ProductSums, for a norm or (rope) the rotation, or
         None (library product, bias)."""
-        w = self.weight
         if self.bias is not None:
             return None
-        if x.shape[0] > 96:
-            better = not rope and ops.tiled_sums_better(x.shape[0], *w.shape, fp8=False)
-            return ops.tiled_sums(x, w) if better else None
-        if not ops.sums_better(
-            x.shape[0], *w.shape, fp8=False, rope=rope, eager=eager
-        ):
-            return None
-        return ops.product_sums(x, w)
+        return ops.sums_for_reader(x, self.weight, rope=rope, eager=eager)
 
 
 _EVERY_MODULES_HOOKS = torch.nn.modules.module._global_forward_hooks
@@ -158,7 +150,7 @@ class Attention(nn.Module):
         lora_live = lm is not None and lm.active and fb.lora_ids is not None
         qkv = _project(
             self.qkv_proj, x,
-            T <= 96 and not lora_live and not self.qk_norm
+            T <= ops.MAX_SUM_ROWS and not lora_live and not self.qk_norm
             and ops.rope_takes_sums(k_cache, v_cache),
             fb, rope=True,
         )

@@ -429,18 +429,46 @@ MAX_SUM_ROWS = 2048
 @functools.lru_cache(maxsize=4096)
 def tiled_sums_better(M: int, N: int, K: int, fp8: bool) -> bool:
     """Whether a product of more than 96 rows as ProductSums of a tiled product
-    that is cut along K and the norm that adds them beat the product as a whole
-    and its norm: where its tiles alone leave CUs idle. By the costs of both
-    (csrc/tiled_gemm.hip); against the library in bf16, which is about as fast
-    as a whole tiled product, better over 50 of 50 chosen products of 160 to 2048
-    rows but four (0.95 at worst; 1.6 in the mean), us with the norm's reading:
-    4096 x 14336 160 rows fp8 49.2 / 29.1, bf16 86.4 / 38.0; 384 rows 53.5 / 41.0, 81.8 /
-    58.5; 1024 rows bf16 138 / 117; 4096 x 4096 160 rows bf16 30.7 / 19."""
+    that is cut along K, and the norm or rotation that adds them, beat the product
+    as a whole and its reader: where its tiles alone leave CUs idle. By the costs
+    of both (csrc/tiled_gemm.hip) and 3.5 us that a reader of few rows takes longer.
+    Over 50 products (128 to 1024 rows, 1024 to 10240 columns, K 1024 to 28672) of each
+    type, against the tiled product in fp8 and the library in bf16, with either
+    reader, the chosen ones gain 1.5 and 1.35 in the mean, 0.93 at worst (us with the
+    norm: 4096 x 14336 128 rows fp8 51 / 26, bf16 76 / 35; 512 rows 53 / 49, 92 / 70; 1024
+    rows bf16 139 / 116; 4096 x 4096 128 rows bf16 28 / 19, fp8 15.5 / 16.7: whole)."""
     es = 1 if fp8 else 2
     if _C is None or not 96 < M <= MAX_SUM_ROWS or N > 16384 or K * es % 128:
         return False
     whole = _C.tiled_plan(M, N, K * es, fp8, False)[2]
-    return _C.tiled_plan(M, N, K * es, fp8, True)[2] < 0.95 * whole
+    return _C.tiled_plan(M, N, K * es, fp8, True)[2] + 3.5 < 0.95 * whole
+
+
+def few_tiled_better(M: int, N: int, K: int, fp8: bool, rope: bool, sums: bool) -> bool:
+    """Whether a product of 17 to 96 rows is best read as the sums of the tiled
+    product. sums: the streaming product's sums beat the library's (sums_better);
+    there the streaming kernel is the slower one where K is long or the rows are
+    many (us with the norm, streaming / tiled: fp8 4096 x 14336 24 rows 23.3 / 20.7,
+    96 rows 28.9 / 24.0; 4096 x 4096 24 rows 13.8 / 14.2, 40 rows 15.4 / 13.4; 2048 x
+    2048 24 rows 8.8 / 9.8, 96 rows 12.0 / 11.2; bf16 4096 x 14336 96 rows 39.9 / 31.8).
+    Else the library's product and reader / this: fp8 3072 x 8192 40 rows 17.1 / 16.0
+    (rotation 16.9 / 17.0), 96 rows 25.4 / 17.8; 8192 x 28672 40 rows 74 / 52; 8192 x
+    8192 40 rows 22.6 / 24.7; bf16 6144 x 4096 40 rows 20.4 / 17.9, 96 rows 25.9 / 20.7;
+    10240 x 8192 24 rows 41.1 / 40.7, 96 rows 54.9 / 42.9; 2304 x 2048 80 rows 12.0 /
+    12.6. Over 78 products with either reader a step of these rows takes 0.93 (fp8) and
+    0.92 (bf16) of the time that it took with the streaming product alone."""
+    if sums:
+        return K >= 8192 or K >= 4096 and (M >= 32 or N > 4096) or K >= 2048 and M >= 80
+    if K >= 16384:
+        return True
+    if fp8:
+        return K >= 8192 and (
+            N <= 2304 and M <= 64 or N <= 4096 and (M >= 24 and not rope or K >= 12288)
+            or N > 8192 and M >= 40
+        )
+    return K >= 4096 and N <= 6144 or K >= 8192 and M >= 40 and N > 8192 or (
+        K >= 2304 and M >= 80 and 2304 < N <= 4096
+    )
 
 
 def tiled_sums(x, weight, x_scale=None, w_scale=None):
@@ -449,6 +477,22 @@ def tiled_sums(x, weight, x_scale=None, w_scale=None):
     if not _tiled_operands(x, weight):
         return None
     return ProductSums(_C.tiled_sums(x, weight), x_scale, w_scale)
+
+
+def sums_for_reader(x, weight, x_scale=None, w_scale=None, rope=False, eager=False):
+    """x weight^T (fp8 with the scales of both) as ProductSums where that and the
+    norm, or (rope) the rotation, that reads it are the fastest form, or None: the
+    product as a whole. eager: see sums_better."""
+    M, (N, K), fp8 = x.shape[0], weight.shape, x_scale is not None
+    if M > 96:
+        better = tiled_sums_better(M, N, K, fp8)
+        return tiled_sums(x, weight, x_scale, w_scale) if better else None
+    sums = sums_better(M, N, K, fp8=fp8, rope=rope, eager=eager)
+    if M > 16 and N < 16384 and few_tiled_better(M, N, K, fp8, rope, sums):
+        got = tiled_sums(x, weight, x_scale, w_scale)
+        if got is not None:
+            return got
+    return product_sums(x, weight, x_scale, w_scale) if sums else None
 
 
 def linear(x, weight):
