@@ -10,11 +10,13 @@ from __future__ import annotations
 import os
 from typing import Optional
 
+import numpy as np
 import torch
 
 from kubeai_amd import ops
 from kubeai_amd.models.config import ModelArchConfig
 from kubeai_amd.models.registry import model_class
+from kubeai_amd.ops.seq import SeqMeta
 
 from .batch import ForwardBatch
 from .scheduler import SchedulerOutput
@@ -331,49 +333,51 @@ class ModelRunner:
                 if req.images and req.mm_embeds is None:
                     pixels = torch.stack([im.float() for im in req.images])
                     req.mm_embeds = self.vision.encode(pixels)
-        input_ids: list[int] = []
-        positions: list[int] = []
-        slots: list[int] = []
+        all_seqs = out.all_seqs
+        lens = [1] * len(out.decode) + [ss.chunk_len for ss in out.prefill]
+        # ---- pad the token stream to a bucket size --------------------
+        # Keeps the products' row counts on a small fixed set up to 1024
+        # tokens (algorithm table, decode graphs), above that on multiples
+        # of 256. Pad tokens form a throwaway prefill
+        # sequence over cache block 0: slot -1 (no KV write), row-local
+        # compute only (GEMMs/norms are row-independent), never sampled.
+        T = sum(lens)
+        T_pad = _bucket(T)
+        pad = T_pad - T
+        # padding is split into <=block_size mini-seqs so the throwaway
+        # causal attention stays O(pad * bs), not O(pad^2)
+        pads = [min(bs, pad - at) for at in range(0, pad, bs)]
+        input_ids = np.zeros(T_pad, dtype=np.int32)
+        positions = np.empty(T_pad, dtype=np.int32)
+        slots = np.full(T_pad, -1, dtype=np.int64)
+        max_bt = max([len(ss.req.block_table) for ss in all_seqs], default=1)
+        max_bt = max(max_bt, 1)
+        tables = np.zeros((len(all_seqs) + len(pads), max_bt), dtype=np.int32)
+        nd_tok = len(out.decode)  # decode tokens precede prefill tokens
+        at = 0
+        for i, (ss, n) in enumerate(zip(all_seqs, lens)):
+            req, start = ss.req, ss.chunk_start
+            table = req.block_table
+            tables[i, : len(table)] = table
+            if n == 1:
+                input_ids[at] = req.tokens[start]
+                positions[at] = start
+                slots[at] = table[start // bs] * bs + start % bs
+            else:
+                idx = np.arange(start, start + n)
+                input_ids[at : at + n] = req.tokens[start : start + n]
+                positions[at : at + n] = idx
+                blocks = np.asarray(table, dtype=np.int64)
+                slots[at : at + n] = blocks[idx // bs] * bs + idx % bs
+            at += n
+        for n in pads:
+            positions[at : at + n] = range(n)
+            at += n
 
-        def emit(req, start: int, length: int) -> None:
-            if length > 64:
-                # vectorize long prefill chunks (a pure-Python per-token loop
-                # costs ~1 ms per 8k-token chunk)
-                import numpy as np
-
-                idx = np.arange(start, start + length)
-                input_ids.extend(req.tokens[start : start + length])
-                positions.extend(idx.tolist())
-                table = np.asarray(req.block_table, dtype=np.int64)
-                slots.extend((table[idx // bs] * bs + idx % bs).tolist())
-                return
-            for i in range(start, start + length):
-                input_ids.append(req.tokens[i])
-                positions.append(i)
-                table_idx = i // bs
-                slots.append(req.block_table[table_idx] * bs + i % bs)
-
-        max_bt = 1
-        for ss in out.all_seqs:
-            max_bt = max(max_bt, len(ss.req.block_table))
-
-        dec_tables: list[list[int]] = []
-        dec_lens: list[int] = []
-        for ss in out.decode:
-            emit(ss.req, ss.chunk_start, 1)
-            dec_tables.append(self._pad(ss.req.block_table, max_bt))
-            dec_lens.append(ss.chunk_start + 1)
-
-        pre_tables: list[list[int]] = []
-        pre_lens: list[int] = []
         mm_idx: list[int] = []
         mm_rows: list[torch.Tensor] = []
-        nd_tok = len(input_ids)  # decode tokens precede prefill tokens
         qsl = [0]
         for ss in out.prefill:
-            emit(ss.req, ss.chunk_start, ss.chunk_len)
-            pre_tables.append(self._pad(ss.req.block_table, max_bt))
-            pre_lens.append(ss.chunk_start + ss.chunk_len)
             # image-placeholder positions inside this chunk -> splice rows
             if ss.req.mm_embeds is not None:
                 c0, c1 = ss.chunk_start, ss.chunk_start + ss.chunk_len
@@ -406,83 +410,85 @@ class ModelRunner:
             for j, ss in enumerate(out.prefill):
                 if ss.samples:
                     logit_idx.append(nd + qsl[j + 1] - 1)
-        # runs of the stream with their state slots, in packing order;
-        # bucket padding below appends slot-less runs
+        # runs of the stream with their state slots, in packing order; those of
+        # the padding have none
         runs: list[tuple[int, int]] = [
-            (ss.chunk_len, ss.req.state_slot) for ss in out.all_seqs
+            (n, ss.req.state_slot) for ss, n in zip(all_seqs, lens)
         ]
 
         lora_ids = None
         if getattr(self, "lora_manager", None) is not None and self.lora_manager.active:
-            ids: list[int] = []
-            for ss in out.all_seqs:
-                ids.extend([ss.req.lora_id] * ss.chunk_len)
-            lora_ids = torch.tensor(ids, dtype=torch.int32, device=self.device)
+            ids = [ss.req.lora_id for ss in all_seqs] + [0] * len(pads)
+            lora_ids = np.repeat(np.asarray(ids, dtype=np.int32), lens + pads)
 
-        # ---- pad the token stream to a bucket size --------------------
-        # Keeps the products' row counts on a small fixed set up to 1024
-        # tokens (algorithm table, decode graphs), above that on multiples
-        # of 256. Pad tokens form a throwaway prefill
-        # sequence over cache block 0: slot -1 (no KV write), row-local
-        # compute only (GEMMs/norms are row-independent), never sampled.
-        T = len(input_ids)
-        T_pad = _bucket(T)
-        if T_pad > T:
-            pad = T_pad - T
-            input_ids.extend([0] * pad)
-            slots.extend([-1] * pad)
-            # split padding into <=block_size mini-seqs so the throwaway
-            # causal attention stays O(pad * bs), not O(pad^2)
-            left = pad
-            while left > 0:
-                c = min(left, bs)
-                positions.extend(range(c))
-                runs.append((c, -1))
-                pre_tables.append([0] * max_bt)
-                pre_lens.append(c)
-                qsl.append(qsl[-1] + c)
-                left -= c
-            if lora_ids is not None:
-                lora_ids = torch.cat(
-                    [lora_ids, torch.zeros(pad, dtype=torch.int32, device=self.device)]
-                )
-
-        dev = self.device
-        t32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)
-        n_prefill = len(pre_lens)
-        seq = None
-        pos_t = t32(positions)
+        for n in pads:
+            runs.append((n, -1))
+            qsl.append(qsl[-1] + n)
+        seq_lens = np.asarray(
+            [ss.chunk_start + n for ss, n in zip(all_seqs, lens)] + pads, dtype=np.int32
+        )
+        n_prefill = len(qsl) - 1
+        host = {
+            "input_ids": input_ids, "positions": positions, "slots": slots,
+            "tables": tables, "seq_lens": seq_lens,
+            "qsl": np.asarray(qsl, dtype=np.int32),
+            "logits": np.asarray(logit_idx, dtype=np.int64),
+        }
+        if lora_ids is not None:
+            host["lora_ids"] = lora_ids
+        if mm_idx:
+            host["mm_idx"] = np.asarray(mm_idx, dtype=np.int64)
         if self.uses_seq_meta:
-            from kubeai_amd.ops.seq import SeqMeta
-
-            seq = SeqMeta.build(
-                runs, pos_t, dev, block_tables=t32(dec_tables + pre_tables)
+            host["start"], host["state"], host["token"], longest = SeqMeta.arrays(runs)
+        on = self._upload(host)
+        seq = None
+        if self.uses_seq_meta:
+            seq = SeqMeta(
+                start_loc=on["start"], slots=on["state"], token_seq=on["token"],
+                positions=on["positions"], block_tables=on["tables"],
+                n_seq=len(runs), max_len=longest,
             )
         return ForwardBatch(
             seq=seq,
-            mm_idx=(
-                torch.tensor(mm_idx, dtype=torch.int64, device=dev)
-                if mm_idx
-                else None
-            ),
-            mm_embeds=torch.cat(mm_rows).to(dev) if mm_rows else None,
-            lora_ids=lora_ids,
-            input_ids=t32(input_ids),
-            positions=pos_t,
-            slot_mapping=torch.tensor(slots, dtype=torch.int64, device=dev),
+            mm_idx=on.get("mm_idx"),
+            mm_embeds=torch.cat(mm_rows).to(self.device) if mm_rows else None,
+            lora_ids=on.get("lora_ids"),
+            input_ids=on["input_ids"],
+            positions=on["positions"],
+            slot_mapping=on["slots"],
             n_decode=nd,
-            decode_block_tables=t32(dec_tables) if dec_tables else None,
-            decode_seq_lens=t32(dec_lens) if dec_lens else None,
+            decode_block_tables=on["tables"][:nd] if nd else None,
+            decode_seq_lens=on["seq_lens"][:nd] if nd else None,
             n_prefill=n_prefill,
-            prefill_query_start_loc=t32(qsl) if n_prefill else None,
-            prefill_seq_lens=t32(pre_lens) if pre_lens else None,
-            prefill_block_tables=t32(pre_tables) if pre_tables else None,
-            logits_indices=torch.tensor(logit_idx, dtype=torch.int64, device=dev),
+            prefill_query_start_loc=on["qsl"] if n_prefill else None,
+            prefill_seq_lens=on["seq_lens"][nd:] if n_prefill else None,
+            prefill_block_tables=on["tables"][nd:] if n_prefill else None,
+            logits_indices=on["logits"],
         )
 
-    @staticmethod
-    def _pad(table: list[int], n: int) -> list[int]:
-        return table + [0] * (n - len(table))
+    def _upload(self, host: dict) -> dict:
+        """The arrays as tensors on the device. On a GPU all of them go in one
+        copy out of pinned memory that the host does not wait for (a copy of
+        pageable memory each, as torch.tensor makes them, waits for the work
+        before it: 9 of those kept the GPU idle for 0.3 ms a step). The pinned
+        block goes back to torch's allocator, which hands it out again after
+        the copy. Tensors begin on 64 bytes."""
+        if self.device.type != "cuda":
+            return {k: torch.from_numpy(a).to(self.device) for k, a in host.items()}
+        at, total = {}, 0
+        for k, a in host.items():
+            at[k] = total
+            total += (a.nbytes + 63) // 64 * 64
+        block = torch.empty(max(total, 64), dtype=torch.uint8, pin_memory=True)
+        raw = block.numpy()
+        for k, a in host.items():
+            raw[at[k] : at[k] + a.nbytes] = a.reshape(-1).view(np.uint8)
+        block = block.to(self.device, non_blocking=True)
+        kinds = {"int32": torch.int32, "int64": torch.int64}
+        return {
+            k: block[at[k] : at[k] + a.nbytes].view(kinds[a.dtype.name]).view(a.shape)
+            for k, a in host.items()
+        }
 
     # ------------------------------------------------------------------
     def _execute_graph(self, out: SchedulerOutput):
@@ -519,8 +525,6 @@ class ModelRunner:
             self._graphs[b_pad] = g
         bs = self.block_size
         ids, pos, slots, lens = [], [], [], []
-        import numpy as np
-
         tables = np.zeros((b, g.bt_max), dtype=np.int32)
         for i, ss in enumerate(out.decode):
             req = ss.req

@@ -73,22 +73,30 @@ class SeqMeta:
                 yield s0, n, slots[i], int(pos[s0])
 
     @staticmethod
-    def build(runs, positions, device, block_tables=None) -> "SeqMeta":
-        """runs: list of (length, slot). positions: int32 tensor [T]."""
+    def arrays(runs):
+        """runs: list of (length, slot). Host arrays of start_loc, slots and
+        token_seq, and the longest length."""
         import numpy as np
 
         lens = np.asarray([r[0] for r in runs], dtype=np.int64)
         start = np.zeros(len(runs) + 1, dtype=np.int32)
         np.cumsum(lens, out=start[1:])
+        slots = np.asarray([r[1] for r in runs], dtype=np.int32)
         tok = np.repeat(np.arange(len(runs), dtype=np.int32), lens)
+        return start, slots, tok, int(lens.max()) if len(runs) else 0
+
+    @staticmethod
+    def build(runs, positions, device, block_tables=None) -> "SeqMeta":
+        """runs: list of (length, slot). positions: int32 tensor [T]."""
+        start, slots, tok, longest = SeqMeta.arrays(runs)
         return SeqMeta(
             start_loc=torch.from_numpy(start).to(device),
-            slots=torch.tensor([r[1] for r in runs], dtype=torch.int32, device=device),
+            slots=torch.from_numpy(slots).to(device),
             token_seq=torch.from_numpy(tok).to(device),
             positions=positions,
             block_tables=block_tables,
             n_seq=len(runs),
-            max_len=int(lens.max()) if len(runs) else 0,
+            max_len=longest,
         )
 
 
