@@ -21,6 +21,11 @@ void rmsnorm_sums(torch::Tensor out, c10::optional<torch::Tensor> out_scale,
                   c10::optional<torch::Tensor> sw,
                   c10::optional<torch::Tensor> residual, torch::Tensor weight,
                   double eps);
+void norm_add_norm(torch::Tensor out, torch::Tensor hidden,
+                   c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> part,
+                   c10::optional<torch::Tensor> sx, c10::optional<torch::Tensor> sw,
+                   torch::Tensor residual, c10::optional<torch::Tensor> w1,
+                   torch::Tensor w2, double eps);
 void reshape_and_cache_fp8(torch::Tensor k, torch::Tensor v,
                            torch::Tensor k_cache, torch::Tensor v_cache,
                            torch::Tensor slot_mapping);
@@ -51,10 +56,10 @@ void grouped_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                     c10::optional<torch::Tensor> sx,
                     c10::optional<torch::Tensor> sw, torch::Tensor bounds,
                     c10::optional<torch::Tensor> src,
-                    c10::optional<torch::Tensor> square, bool silu);
+                    c10::optional<torch::Tensor> square, int64_t act);
 void tiled_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                   c10::optional<torch::Tensor> sx,
-                  c10::optional<torch::Tensor> sw, bool silu);
+                  c10::optional<torch::Tensor> sw, int64_t act);
 torch::Tensor tiled_sums(torch::Tensor x, torch::Tensor w);
 std::tuple<int64_t, int64_t, double> tiled_plan(int64_t M, int64_t N, int64_t KB,
                                                 bool fp8, bool sums);
@@ -127,6 +132,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_sums", &skinny_sums, "fp32 part sums of a skinny product");
   m.def("quant_fp8_rows", &quant_fp8_rows, "gathered bf16 rows -> fp8");
   m.def("rmsnorm_sums", &rmsnorm_sums, "norm of a product's part sums");
+  m.def("norm_add_norm", &norm_add_norm,
+        "norm of a branch, residual add and the next norm, or the last two");
   m.def("moe_route", &moe_route,
         "router scores, top-k weights and tokens in expert order");
   m.def("moe_combine", &moe_combine, "weighted sum of the experts' rows");

@@ -1,8 +1,8 @@
 // Products of many rows: y[i] = x[i] w^T, or for the rows of every expert e of a
 // mixture y[i] = x[src[i]] w[e]^T in one launch; bf16 or fp8 e4m3 (W8A8 with row
 // and column scales), fp32 accumulation. What the epilogue makes of them: bf16
-// rows, fp32 sums of a part of K, silu(gate) * up of stacked gate and up columns
-// (in fp32, rounded once), or relu(.)^2 times a weight per row.
+// rows, fp32 sums of a part of K, silu or tanh-gelu(gate) * up of stacked gate and
+// up columns (in fp32, rounded once), or relu(.)^2 times a weight per row.
 //
 // Bound by the matrix cores (and the power they draw: dense bf16 runs at 1.65
 // GHz here), as long as nothing keeps them waiting. What it takes:
@@ -45,7 +45,7 @@
 
 namespace tiled {
 
-enum Epilogue { kRows, kSums, kSilu, kSquare };
+enum Epilogue { kRows, kSums, kSilu, kGelu, kSquare };
 
 struct Args {
   ushort* y;        // [R, columns]
@@ -189,7 +189,7 @@ __global__ __launch_bounds__(256, kShapes[SHAPE].per_cu()) void tiled_kernel(con
   constexpr int WM = S.wm, WN = S.wn, NA = S.na, NB = S.nb;
   static_assert(NA >= 2 && (NB == NA || (NA == 2 && NB == 3)));
   constexpr int BM = S.rows(), BN = S.cols();
-  constexpr bool kHalves = EPI == kSilu;  // gate | up columns
+  constexpr bool kHalves = EPI == kSilu || EPI == kGelu;  // gate | up columns
   static_assert(!kHalves || WN % 2 == 0);
   constexpr int OUT = kHalves ? BN / 2 : BN;  // columns of the result
   constexpr int AC = BM / 32, BC = BN / 32, L = AC + BC;  // loads per wave and step
@@ -434,7 +434,9 @@ __global__ __launch_bounds__(256, kShapes[SHAPE].per_cu()) void tiled_kernel(con
 #pragma unroll
           for (int t = 0; t < 4; t++) {
             const float g = v[h][t];
-            v[h][t] = g / (1.0f + __expf(-g)) * up[h][t];
+            float z = g;  // gelu: 0.5 (1 + tanh y) = 1 / (1 + e^-2y)
+            if constexpr (EPI == kGelu) z = 1.5957691216057308f * (g + 0.044715f * g * g * g);
+            v[h][t] = g / (1.0f + __expf(-z)) * up[h][t];
           }
         }
         bf4 b = __builtin_convertvector(v[h], bf4);
@@ -466,7 +468,7 @@ void launch(int shape, const Args& a, int grid) {
   auto stream = c10::hip::getCurrentHIPStream().stream();
   auto go = [&](auto s) {
     constexpr int i = decltype(s)::value;
-    if constexpr (EPI != kSilu || kShapes[i].wn % 2 == 0) {
+    if constexpr ((EPI != kSilu && EPI != kGelu) || kShapes[i].wn % 2 == 0) {
       hipLaunchKernelGGL((tiled_kernel<FP8, i, EPI>), dim3(grid), dim3(256), 0, stream, a);
     } else {
       TORCH_CHECK(false, "no such tile");

@@ -64,7 +64,12 @@ Plan plan(bool fp8, int64_t R, int64_t E, int64_t cols, int64_t KB, bool halves,
     for (int parts = 1; parts <= (sums ? kMaxParts : 1); parts++) {
       const int64_t all = KB / kStep, steps = (all + parts - 1) / parts;
       if (parts > 1 && (steps < 4 || (all + steps - 1) / steps != parts)) continue;
-      const double passes = std::ceil(row_tiles * nt * parts / (256 * s.per_cu()));
+      const double full = row_tiles * nt * parts / (256 * s.per_cu());
+      double passes = std::ceil(full);
+      if (E > 1) {  // a few tiles more may begin another pass
+        passes = 0.;
+        for (int k = -2; k <= 2; k++) passes += std::ceil(full * (1. + 0.05 * k)) / 5.;
+      }
       const double us = passes * (steps * c.step + c.tile) + c.rest +
                         (sums ? parts * R * cols * 4e-6 * (c.mb + kReadMb) : 0.);
       if (best.shape < 0 || us < best.us) best = {i, parts, us};
@@ -135,10 +140,12 @@ void check_result(const torch::Tensor& y, int64_t cols, Args& a) {
   a.wide = cols % 8 == 0 && ((uintptr_t)y.data_ptr() & 15) == 0;
 }
 
-Epilogue epilogue_of(bool silu, const Args& a) {
-  if (!silu) return kRows;
-  TORCH_CHECK(a.N % 16 == 0 && a.N * a.ldw < (int64_t)1 << 31, "gate and up columns");
-  return kSilu;
+Epilogue epilogue_of(int64_t act, const Operands& o) {
+  TORCH_CHECK(act >= 0 && act <= 2, "0: none, 1: silu, 2: gelu");
+  if (act == 0) return kRows;
+  TORCH_CHECK(o.a.N % 16 == 0 && o.a.N * o.a.ldw < (int64_t)1 << 31, "gate and up columns");
+  TORCH_CHECK(act == 1 || !o.fp8, "gelu: bf16");
+  return act == 1 ? kSilu : kGelu;
 }
 
 void run(const Operands& o, Epilogue epi, int shape, int64_t grid) {
@@ -155,13 +162,13 @@ using namespace tiled;
 // y [R, N] = rows of x [*, K] times w[e]^T, w [E, N, K] with any strides of e
 // and n; bounds int32: E row counts or E + 1 offsets; src int32 [R] the rows
 // of x, or none; fp8: sx fp32 [rows of x], sw fp32 [E, N]; square fp32 [R]:
-// y = relu(product)^2 * square. silu: y [R, N / 2] = silu of the first N / 2 columns
-// times the others.
+// y = relu(product)^2 * square. act 1 or 2: y [R, N / 2] = silu or tanh-gelu of the
+// first N / 2 columns times the others.
 void grouped_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                     c10::optional<torch::Tensor> sx,
                     c10::optional<torch::Tensor> sw, torch::Tensor bounds,
                     c10::optional<torch::Tensor> src,
-                    c10::optional<torch::Tensor> square, bool silu) {
+                    c10::optional<torch::Tensor> square, int64_t act) {
   const int64_t R = y.size(0);
   if (src.has_value()) {
     TORCH_CHECK(src->scalar_type() == torch::kInt32 && src->is_contiguous() &&
@@ -178,12 +185,12 @@ void grouped_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   const int64_t E = a.E;
   TORCH_CHECK(bounds.scalar_type() == torch::kInt32 && bounds.is_contiguous() &&
               bounds.is_cuda() && (bounds.numel() == E || bounds.numel() == E + 1));
-  Epilogue epi = epilogue_of(silu, a);
-  const int64_t cols = silu ? a.N / 2 : a.N;
+  Epilogue epi = epilogue_of(act, o);
+  const int64_t cols = act ? a.N / 2 : a.N;
   check_result(y, cols, a);
   if (!src.has_value()) TORCH_CHECK(o.x.size(0) == R);
   if (square.has_value()) {
-    TORCH_CHECK(!o.fp8 && !silu && square->scalar_type() == torch::kFloat32 &&
+    TORCH_CHECK(!o.fp8 && act == 0 && square->scalar_type() == torch::kFloat32 &&
                 square->is_contiguous() && square->is_cuda() && square->numel() == R);
     a.row_weight = square->data_ptr<float>();
     epi = kSquare;
@@ -193,27 +200,27 @@ void grouped_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   a.offsets = bounds.numel() == E + 1;
   a.src = src.has_value() ? src->data_ptr<int32_t>() : nullptr;
   a.xbytes = (o.x.size(0) - 1) * a.ldx + a.KB;
-  const Plan p = plan(o.fp8, R, E, cols, a.KB, silu, false);
+  const Plan p = plan(o.fp8, R, E, cols, a.KB, act != 0, false);
   const Shape s = kShapes[p.shape];
-  const int64_t bn = s.cols() / (silu ? 2 : 1);
+  const int64_t bn = s.cols() / (act ? 2 : 1);
   run(o, epi, p.shape, (R / s.rows() + std::min(E, R)) * ((cols + bn - 1) / bn));
 }
 
-// y [M, N] = x [M, K] w [N, K]^T with the operands, scales and silu of
+// y [M, N] = x [M, K] w [N, K]^T with the operands, scales and act of
 // grouped_linear
 void tiled_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                   c10::optional<torch::Tensor> sx, c10::optional<torch::Tensor> sw,
-                  bool silu) {
+                  int64_t act) {
   Operands o = operands(x, w.unsqueeze(0), sx, sw, false);
   Args& a = o.a;
-  const Epilogue epi = epilogue_of(silu, a);
-  const int64_t cols = silu ? a.N / 2 : a.N;
+  const Epilogue epi = epilogue_of(act, o);
+  const int64_t cols = act ? a.N / 2 : a.N;
   check_result(y, cols, a);
   TORCH_CHECK(o.x.size(0) == a.R);
   if (a.R == 0) return;
-  const Plan p = plan(o.fp8, a.R, 1, cols, a.KB, silu, false);
+  const Plan p = plan(o.fp8, a.R, 1, cols, a.KB, act != 0, false);
   const Shape s = kShapes[p.shape];
-  const int64_t bn = s.cols() / (silu ? 2 : 1);
+  const int64_t bn = s.cols() / (act ? 2 : 1);
   run(o, epi, p.shape, (a.R + s.rows() - 1) / s.rows() * ((cols + bn - 1) / bn));
 }
 

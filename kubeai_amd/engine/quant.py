@@ -68,7 +68,7 @@ class Fp8Linear(nn.Module):
             or type(self).forward_quantized is not Fp8Linear.forward_quantized
         ):
             return None
-        return ops.tiled_swiglu(
+        return ops.tiled_gated(
             xq, self.weight_fp8, x_scale, self.weight_scale.view(-1)
         )
 

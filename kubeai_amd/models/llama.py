@@ -251,11 +251,11 @@ class MLP(nn.Module):
         )
         a = None
         if not (
-            lora_live or self.gelu or x.dim() != 2 or x.shape[0] <= 96
+            lora_live or x.dim() != 2 or x.shape[0] <= 96
             or type(self.gate_up_proj) is not EngineLinear or _hooked(self.gate_up_proj)
             or self.gate_up_proj.bias is not None
         ):
-            a = ops.tiled_swiglu(x, self.gate_up_proj.weight)
+            a = ops.tiled_gated(x, self.gate_up_proj.weight, gelu=self.gelu)
         if a is None:
             h = self.gate_up_proj(x)
             if lora_live:
@@ -432,8 +432,8 @@ class MoEMLP(nn.Module):
         fp8 = hasattr(first.gate_up_proj, "forward_quantized")
         ends = None
 
-        def products(rows, proj, width, src=None, silu=False):
-            """silu: of gate and up rows; the result has half the width then, or
+        def products(rows, proj, width, src=None, act=0):
+            """act: of gate and up rows; the result has half the width then, or
             the whole where the activation is still to be done."""
             nonlocal ends
             rows, scale = rows if fp8 else (rows, None)
@@ -443,13 +443,11 @@ class MoEMLP(nn.Module):
                 w is not None and (ws is not None) == fp8
                 and ops.grouped_linear_takes(rows, w) and ops.grouped_linear_better(n, w)
             ):
-                silu = silu and (
-                    w.shape[1] % 16 == 0
-                    and w.shape[1] * w.stride(1) * w.element_size() < 2**31
-                )
+                if w.shape[1] % 16 or w.shape[1] * w.stride(1) * w.element_size() >= 2**31:
+                    act = 0
                 return ops.grouped_linear(
                     rows, w, begin, src=src, scales=(scale, ws) if fp8 else None,
-                    silu=silu,
+                    act=act,
                 )
             if src is not None:
                 rows = rows.index_select(0, src)
@@ -472,10 +470,10 @@ class MoEMLP(nn.Module):
 
         width = 2 * first.down_proj.in_features
         if fp8:
-            h = products(ops.quant_fp8_rows(x, src), "gate_up_proj", width, silu=True)
+            h = products(ops.quant_fp8_rows(x, src), "gate_up_proj", width, act=1)
             a = ops.silu_and_mul_fp8(h) if h.shape[1] == width else ops.quant_fp8(h)
         else:
-            a = products(x, "gate_up_proj", width, src, silu=not self.gelu)
+            a = products(x, "gate_up_proj", width, src, act=2 if self.gelu else 1)
             if a.shape[1] == width:
                 a = ops.gelu_and_mul(a) if self.gelu else ops.silu_and_mul(a)
         return ops.moe_combine(products(a, "down_proj", x.shape[1]), place, weight)
@@ -602,8 +600,8 @@ class DecoderLayer(nn.Module):
             )
 
     def forward(self, x, residual, fb, kv_cache, cos_sin, as_sums: bool = False):
-        """as_sums: the caller takes the branch as ops.ProductSums too (x may be
-        that in any case)."""
+        """as_sums: the caller takes the branch as ops.ProductSums too, or with
+        post norms as ops.BranchNorm (x may be that in any case)."""
         # products are handed on as sums in steps of few rows only
         branch = _branch if x.shape[0] <= ops.MAX_SUM_ROWS else _call
         last = branch if as_sums else _call
@@ -611,18 +609,19 @@ class DecoderLayer(nn.Module):
             # incoming invariant: hidden = x + residual (residual None at
             # layer 0); outgoing (m_normed, hidden_after_attn) keeps it,
             # so the model-level final fused_add_rmsnorm still applies
-            hidden = x if residual is None else x + residual
-            a = branch(
-                self.self_attn, ops.rmsnorm(hidden, self.input_layernorm, self.eps),
-                fb, kv_cache, cos_sin,
+            if residual is None:
+                hidden, x = x, ops.rmsnorm(x, self.input_layernorm, self.eps)
+            else:
+                x, hidden = ops.add_and_norm(x, residual, self.input_layernorm, self.eps)
+            a = branch(self.self_attn, x, fb, kv_cache, cos_sin)
+            x, h2 = ops.add_and_norm(
+                ops.BranchNorm(a, self.post_attention_layernorm, self.eps), hidden,
+                self.pre_feedforward_layernorm, self.eps,
             )
-            a = ops.rmsnorm(a, self.post_attention_layernorm, self.eps)
-            h2 = hidden + a
-            mm = branch(
-                self.mlp, ops.rmsnorm(h2, self.pre_feedforward_layernorm, self.eps), fb
-            )
-            mm = ops.rmsnorm(mm, self.post_feedforward_layernorm, self.eps)
-            return mm, h2
+            mm = branch(self.mlp, x, fb)
+            if as_sums:  # the next layer's (or the final) norm takes this one too
+                return ops.BranchNorm(mm, self.post_feedforward_layernorm, self.eps), h2
+            return ops.rmsnorm(mm, self.post_feedforward_layernorm, self.eps), h2
         if (
             getattr(self, "_fp8_fused", False)
             and x.is_cuda
@@ -742,12 +741,14 @@ class LlamaForCausalLM(nn.Module):
         n = len(self.layers)
         # layers that nobody else looks at hand on products that the next one's
         # (or the final) norm adds up
-        few = x.shape[0] <= ops.MAX_SUM_ROWS
+        few = x.shape[0] <= ops.MAX_SUM_ROWS or self.cfg.post_norms
         own = [few and type(layer) is DecoderLayer and not _hooked(layer)
                for layer in self.layers]
         for i, layer in enumerate(self.layers):
             kw = {"as_sums": True} if own[i] and (i + 1 == n or own[i + 1]) else {}
             x, residual = layer(x, residual, fb, self.kv_caches[i], cs, **kw)
+        if isinstance(x, ops.BranchNorm):  # (sums in fp32, as fused_add_rmsnorm's)
+            x = ops.rmsnorm(x.x, x.weight, x.eps)
         x, _ = ops.fused_add_rmsnorm(x, residual, self.norm, self.cfg.rms_norm_eps)
         return x
 

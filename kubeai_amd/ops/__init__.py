@@ -392,34 +392,38 @@ def _tiled_better(M: int, N: int, K: int, fp8: bool) -> bool:
     return fp8 and M > 96 and K >= 2048 and (K <= 2 * N or M > 512)
 
 
-def _tiled_linear(x, weight, x_scale=None, w_scale=None, out=None, silu=False):
+def _tiled_linear(x, weight, x_scale=None, w_scale=None, out=None, act=0):
     if out is None:
         out = torch.empty(
-            (x.shape[0], weight.shape[0] // (2 if silu else 1)), dtype=torch.bfloat16,
+            (x.shape[0], weight.shape[0] // (2 if act else 1)), dtype=torch.bfloat16,
             device=x.device,
         )
-    _C.tiled_linear(out, x, weight, x_scale, w_scale, silu)
+    _C.tiled_linear(out, x, weight, x_scale, w_scale, act)
     return out
 
 
-def tiled_swiglu(x, weight, x_scale=None, w_scale=None):
-    """silu_and_mul of x weight^T (weight: gate rows, then up rows) in one launch,
-    the activation in fp32 and rounded once; None where the product is not a tiled
-    one or two launches are faster. fp8: where the product is tiled anyway; bf16:
-    up to 512 rows (us, library and activation / this: 28672 x 4096 128 rows 58.0 /
-    54.9, 384 rows 92 / 89, 640 rows 150 / 160, 2048 rows 381 / 408; 22016 x 4096 640
-    rows 125 / 121, 1024 rows 173 / 191; 18432 x 2304 384 rows 45.2 / 40.8)."""
+def tiled_gated(x, weight, x_scale=None, w_scale=None, gelu=False):
+    """silu_and_mul (gelu: gelu_and_mul) of x weight^T (weight: gate rows, then up
+    rows) in one launch, the activation in fp32 and rounded once; None where the
+    product is not a tiled one or two launches are faster. fp8 (silu): where the
+    product is tiled anyway; bf16: up to 512 rows, with K up to 2560 up to 1024 (us,
+    library and activation / this: 28672 x 4096 128 rows 58.0 / 54.9, 384 rows 92 /
+    89, 640 rows 150 / 160, 2048 rows 381 / 408; 22016 x 4096 640 rows 125 / 121, 1024
+    rows 173 / 191; 18432 x 2304 gelu 384 rows 45.9 / 41.4, 1024 rows 102 / 94, 2048
+    rows 172 / 181, 5376 rows 399 / 382 alone but 379 / 385 in a model)."""
     (M, K), N = x.shape, weight.shape[0]
     if x_scale is not None:
-        better = M > 96 and _tiled_better(M, N, K, fp8=True)
+        better = M > 96 and not gelu and _tiled_better(M, N, K, fp8=True)
     else:
-        better = 96 < M <= 512 and N >= 8192 and K >= 2048
+        better = 96 < M and N >= 8192 and K >= 2048 and (
+            M <= 512 or K <= 2560 and M <= 1024
+        )
     if not (
         better and weight.dim() == 2 and N * weight.stride(0) * weight.element_size() < 2**31
         and _tiled_operands(x, weight)
     ):
         return None
-    return _tiled_linear(x, weight, x_scale, w_scale, silu=True)
+    return _tiled_linear(x, weight, x_scale, w_scale, act=2 if gelu else 1)
 
 
 #: Products of more rows are not handed on as sums: whole ones fill the chip.
@@ -586,6 +590,53 @@ def _norm_sums(x: ProductSums, residual, weight, eps: float, fp8: bool):
     return (out, scale) if fp8 else out
 
 
+class BranchNorm:
+    """A branch whose norm is still to be taken, by norm_add_norm of what reads it
+    next (add_and_norm)."""
+
+    def __init__(self, x, weight, eps: float):
+        self.x, self.weight, self.eps = x, weight, eps
+        self.shape = x.shape
+
+
+def _norm_add_norm_takes(x, residual, w1, w2) -> bool:
+    tensors = [residual, w2] + [t for t in (w1, x) if isinstance(t, torch.Tensor)]
+    return (
+        residual.is_cuda
+        and residual.dim() == 2
+        and x.shape == residual.shape
+        and residual.shape[1] % 8 == 0
+        and residual.shape[1] <= 16384
+        and all(t.dtype == torch.bfloat16 and t.is_contiguous() for t in tensors)
+        and all(w is None or w.shape == residual.shape[1:] for w in (w1, w2))
+        and aligned(*tensors)
+        and not observed(*tensors)
+    )
+
+
+def add_and_norm(x, residual, weight, eps: float):
+    """hidden = x + residual in bf16 and its norm; returns (norm, hidden). x may be
+    ProductSums or a BranchNorm (then its norm is added). On GPU one launch, with the
+    bits of rmsnorm, the addition and rmsnorm after one another."""
+    w1 = None
+    if isinstance(x, BranchNorm):
+        if x.eps == eps and _norm_add_norm_takes(x.x, residual, x.weight, weight):
+            x, w1 = x.x, x.weight
+        else:
+            x = rmsnorm(x.x, x.weight, x.eps)
+    if not (w1 is not None or _norm_add_norm_takes(x, residual, None, weight)):
+        if isinstance(x, ProductSums):
+            raise RuntimeError("a product's sums beside a residual that is not dense bf16")
+        hidden = x + residual
+        return rmsnorm(hidden, weight, eps), hidden
+    _require_ext()
+    hidden, out = torch.empty_like(residual), torch.empty_like(residual)
+    sums = x.args() if isinstance(x, ProductSums) else (None, None, None)
+    _C.norm_add_norm(out, hidden, None if sums[0] is not None else x, *sums, residual,
+                     w1, weight, eps)
+    return out, hidden
+
+
 def silu_and_mul_fp8(x):
     if not x.is_cuda:
         return ref.quant_fp8(ref.silu_and_mul(x))
@@ -682,29 +733,28 @@ def grouped_linear_takes(x, w) -> bool:
 def grouped_linear_better(n: int, w) -> bool:
     """Whether n rows of w's experts are better multiplied by grouped_linear than
     by a library product per expert. fp8: always (8 experts, 512 rows each, us,
-    grouped / library: 28672 x 4096 609/686, 4096 x 14336 354/474; 2048 rows
-    1963/1892 and 1016/1127, without the look at the routing from the host). bf16: unless
-    every expert's product fills the chip by itself (3584 x 2048, 768 rows
-    107/171, 2048 rows 260/283; 4096 x 14336, 1024 rows 1063/1106, 2048 rows
-    2144/1857; 28672 x 4096, 64 rows 398/428, 128 rows 551/468, 512 1139/955)."""
-    mean, cols = n / w.shape[0], w.shape[1] / 256
-    return w.element_size() == 1 or mean <= 96 or (
-        cols <= 64 and (mean / 256) * cols < 120
-    )
+    grouped / library: 28672 x 4096 539/686, 4096 x 14336 284/474, without the look at
+    the routing from the host). bf16: unless every expert's product fills the chip
+    by itself (28672 x 4096 64 rows 364/431, 256 rows 576/596, 1024 rows 1666/1664, 2048
+    rows 3233/2907; 12800 x 4096 2048 rows 2858/2730; 4096 x 14336 512 rows 540/803, 2048
+    rows 1781/2260; 3584 x 2048 1024 rows 121/193, 2048 rows 249/275, 4096 rows
+    467/388)."""
+    mean = n / w.shape[0]
+    return w.element_size() == 1 or mean <= 1024 or mean <= 3072 and w.shape[1] <= 8192
 
 
-def grouped_linear(x, w, bounds, src=None, scales=None, square=None, silu=False):
+def grouped_linear(x, w, bounds, src=None, scales=None, square=None, act=0):
     """GPU-only: rows of x [*, K] in expert order times their expert's matrix,
     w [E, N, K] (any strides of e and n), all experts in one launch. bounds int32:
     the experts' row counts [E] or offsets [E + 1]; src int32: the rows of x
     (all, in order). fp8 x and w: scales = (fp32 per row of x, [E, N]). square
-    (fp32 per row): relu(product)^2 * square instead of the product. silu: w is
-    gate rows, then up rows; silu(gate) * up [n, N / 2] instead of the product."""
+    (fp32 per row): relu(product)^2 * square instead of the product. act: w is gate
+    rows, then up rows; silu (1) or, in bf16, gelu (2) of gate times up [n, N / 2]."""
     _require_ext()
     n = x.shape[0] if src is None else src.shape[0]
-    width = w.shape[1] // 2 if silu else w.shape[1]
+    width = w.shape[1] // 2 if act else w.shape[1]
     y = torch.empty((n, width), dtype=torch.bfloat16, device=x.device)
-    _C.grouped_linear(y, x, w, *(scales or (None, None)), bounds, src, square, silu)
+    _C.grouped_linear(y, x, w, *(scales or (None, None)), bounds, src, square, act)
     return y
 
 

@@ -145,6 +145,42 @@ def test_norms_of_product_sums(M, fp8, N, K):
     assert torch.equal(r1, r2)
 
 
+@pytest.mark.parametrize("M", [1, 40, 1030])
+@pytest.mark.parametrize("N", [8, 520, 2304, 16384])
+def test_branch_norm_add_and_norm(M, N):
+    """One launch has the bits of the three that it replaces, but for products in
+    fp32 that may be contracted either way (one step of bf16 now and then)."""
+    x, r = _x(M, N), _x(M, N)
+    w1, w2 = (torch.randn(N, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    kept = r.clone()
+
+    def near(a, b):
+        a, b = a.float(), b.float()
+        assert (a != b).sum().item() <= 2 + a.numel() // 100
+        torch.testing.assert_close(a, b, atol=2.0 ** -8, rtol=2.0 ** -7)
+
+    out, hidden = ops.add_and_norm(x, r, w2, 1e-5)
+    assert torch.equal(hidden, x + r) and torch.equal(r, kept)
+    near(out, ops.rmsnorm(x + r, w2, 1e-5))
+    out, hidden = ops.add_and_norm(ops.BranchNorm(x, w1, 1e-5), r, w2, 1e-5)
+    want = r + ops.rmsnorm(x, w1, 1e-5)
+    near(hidden, want)
+    near(out, ops.rmsnorm(hidden, w2, 1e-5))
+    # forms that the launch does not take go one by one
+    wide = torch.cat([r, r], 1)[:, :N]
+    out2, hidden2 = ops.add_and_norm(x, wide, w2, 1e-5) if N == 8 else (out, hidden)
+    if N == 8:
+        assert torch.equal(hidden2, x + r)
+        near(out2, ops.rmsnorm(hidden2, w2, 1e-5))
+    if M <= 96 and 512 <= N <= 4096 and N % 16 == 0:
+        a, w = _x(M, 1024), _x(N, 1024) * 0.05
+        y = ops.rmsnorm(ops.product_sums(a, w), w1, 1e-5)
+        out, hidden = ops.add_and_norm(
+            ops.BranchNorm(ops.product_sums(a, w), w1, 1e-5), r, w2, 1e-5)
+        near(hidden, r + y)
+        near(out, ops.rmsnorm(hidden, w2, 1e-5))
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("cache", [torch.bfloat16, torch.float8_e5m2])
 def test_rope_of_product_sums(fp8, cache):
