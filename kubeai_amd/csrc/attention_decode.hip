@@ -344,8 +344,35 @@ __launch_bounds__(kBlockThreads, 2) __global__ void paged_decode_kernel(
   }
 }
 
-// Merge the splits' results: one wave per (sequence, query head). The lanes
-// read all splits' (m, l) at once and the rows of O are independent loads.
+// Merged values of one query head, 2 or 4 a lane, rounded to bf16. The lanes read
+// all splits' (m, l) at once and the rows of O are independent loads.
+template <int HD>
+struct Merged {
+  static constexpr int EPL = HD / 64;
+  ushort v[EPL];
+  DEV_INLINE Merged(const float* part_o, const float* part_ml, int n_splits, int64_t bh) {
+    typedef __attribute__((ext_vector_type(EPL))) float vec;
+    const int lane = threadIdx.x % WAVE_SIZE;
+    const float* pml = part_ml + bh * n_splits * 2;
+    const vec* po = reinterpret_cast<const vec*>(part_o + bh * n_splits * HD) + lane;
+    const int s = min(lane, n_splits - 1);
+    const float ms = pml[2 * s], ls = lane < n_splits ? pml[2 * s + 1] : 0.f;
+    const float m_star = wave_reduce_max(ms);
+    const float c = __builtin_amdgcn_exp2f(ms - (m_star == -INFINITY ? 0.f : m_star));
+    const float l_star = wave_reduce_sum(ls * c);
+    vec o;
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) o[e] = 0.f;
+#pragma unroll 4
+    for (int k = 0; k < n_splits; ++k)
+      o += po[k * 64] * __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(c), k));
+    const float inv_l = 1.0f / l_star;
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) v[e] = f32_to_bf16(o[e] * inv_l);
+  }
+};
+
+// Merge the splits' results: one wave per (sequence, query head).
 template <int HD>
 __global__ void decode_merge_kernel(
     ushort* __restrict__ out,             // [B, n_q, hd]
@@ -353,31 +380,68 @@ __global__ void decode_merge_kernel(
     const float* __restrict__ part_ml,    // [B, n_q, n_splits, 2]
     const int n_splits, const int64_t n_bh) {
   constexpr int EPL = HD / 64;
-  typedef __attribute__((ext_vector_type(EPL))) float vec;
   const int64_t bh = (int64_t)blockIdx.x * (blockDim.x / WAVE_SIZE) +
                      threadIdx.x / WAVE_SIZE;
   if (bh >= n_bh) return;
-  const int lane = threadIdx.x % WAVE_SIZE;
-  const float* pml = part_ml + bh * n_splits * 2;
-  const vec* po = reinterpret_cast<const vec*>(part_o + bh * n_splits * HD) + lane;
-  const int s = min(lane, n_splits - 1);
-  const float ms = pml[2 * s], ls = lane < n_splits ? pml[2 * s + 1] : 0.f;
-  const float m_star = wave_reduce_max(ms);
-  const float c = __builtin_amdgcn_exp2f(ms - (m_star == -INFINITY ? 0.f : m_star));
-  const float l_star = wave_reduce_sum(ls * c);
-  vec o;
-#pragma unroll
-  for (int e = 0; e < EPL; ++e) o[e] = 0.f;
-#pragma unroll 4
-  for (int k = 0; k < n_splits; ++k)
-    o += po[k * 64] * __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(c), k));
-  const float inv_l = 1.0f / l_star;
-  ushort* oh = out + bh * HD + EPL * lane;
+  const Merged<HD> m(part_o, part_ml, n_splits, bh);
+  ushort* oh = out + bh * HD + EPL * (threadIdx.x % WAVE_SIZE);
 #pragma unroll
   for (int e = 0; e < EPL; e += 2)
-    *reinterpret_cast<uint32_t*>(oh + e) =
-        ((uint32_t)f32_to_bf16(o[e + 1] * inv_l) << 16) |
-        f32_to_bf16(o[e] * inv_l);
+    *reinterpret_cast<uint32_t*>(oh + e) = ((uint32_t)m.v[e + 1] << 16) | m.v[e];
+}
+
+// The same, and the row (all heads of a sequence) to fp8 with one scale, as the
+// conversion of the merged bf16 row has it: one workgroup of 16 waves per row,
+// HPW heads a wave. Bound by its launch: 40 rows of 32 x 128 in 13 splits, merge
+// and conversion 9.6 us, this 5.1.
+template <int HD, int HPW>
+__launch_bounds__(16 * WAVE_SIZE) __global__ void decode_merge_fp8_kernel(
+    unsigned char* __restrict__ out,      // [B, n_q * hd]
+    float* __restrict__ out_scale,        // [B]
+    const float* __restrict__ part_o, const float* __restrict__ part_ml,
+    const int n_splits, const int n_q) {
+  constexpr int EPL = HD / 64;
+  const int wave = threadIdx.x / WAVE_SIZE, lane = threadIdx.x % WAVE_SIZE;
+  const int64_t row = blockIdx.x;
+  __shared__ float red[16];
+  float vals[HPW][EPL];
+  float amax = 0.f;
+#pragma unroll
+  for (int h = 0; h < HPW; ++h) {
+    const int head = h * 16 + wave;
+    if (head < n_q) {  // the same in every lane
+      const Merged<HD> m(part_o, part_ml, n_splits, row * n_q + head);
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) {
+        vals[h][e] = bf16_to_f32(m.v[e]);
+        amax = fmaxf(amax, fabsf(vals[h][e]));
+      }
+    }
+  }
+  amax = wave_reduce_max(amax);
+  if (lane == 0) red[wave] = amax;
+  __syncthreads();
+  float gmax = 1e-6f;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) gmax = fmaxf(gmax, red[w]);
+  if (threadIdx.x == 0) out_scale[row] = gmax / 448.0f;
+  const float inv_scale = 448.0f / gmax;
+#pragma unroll
+  for (int h = 0; h < HPW; ++h) {
+    const int head = h * 16 + wave;
+    if (head < n_q) {
+      unsigned char* to = out + (row * n_q + head) * HD + EPL * lane;
+      int w = __builtin_amdgcn_cvt_pk_fp8_f32(vals[h][0] * inv_scale,
+                                              vals[h][1] * inv_scale, 0, false);
+      if constexpr (EPL == 4) {
+        w = __builtin_amdgcn_cvt_pk_fp8_f32(vals[h][2] * inv_scale,
+                                            vals[h][3] * inv_scale, w, true);
+        *reinterpret_cast<uint32_t*>(to) = (uint32_t)w;
+      } else {
+        *reinterpret_cast<ushort*>(to) = (ushort)w;
+      }
+    }
+  }
 }
 
 }  // namespace
@@ -405,12 +469,14 @@ int paged_decode_splits(int rows, int n_kv, int hd, int max_blocks) {
       1, std::min({(int64_t)kMaxSplits, (int64_t)tiles, (target + wgs - 1) / wgs}));
 }
 
+// out [B, n_q, hd] bf16, or with out_scale [B] fp8 rows with a scale each
 void paged_attention_decode(torch::Tensor out, torch::Tensor q,
                             torch::Tensor k_cache, torch::Tensor v_cache,
                             torch::Tensor block_tables, torch::Tensor seq_lens,
-                            double scale, int64_t window, double softcap) {
+                            double scale, int64_t window, double softcap,
+                            c10::optional<torch::Tensor> out_scale) {
   TORCH_CHECK(q.stride(2) == 1 && q.stride(1) == q.size(2));
-  TORCH_CHECK(out.is_contiguous());
+  TORCH_CHECK(out.is_contiguous() && out.numel() == q.numel());
   TORCH_CHECK(k_cache.is_contiguous() && v_cache.is_contiguous());
   TORCH_CHECK(q.scalar_type() == torch::kBFloat16);
   TORCH_CHECK(k_cache.scalar_type() == torch::kBFloat16 ||
@@ -429,6 +495,12 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
   TORCH_CHECK(G == 1 || G == 2 || G == 4 || G == 5 || G == 6 || G == 8,
               "unsupported GQA group size ", G);
   const int n_splits = paged_decode_splits(B, n_kv, hd, max_blocks);
+  const bool fp8 = out_scale.has_value();
+  TORCH_CHECK(out.scalar_type() == (fp8 ? torch::kFloat8_e4m3fn : torch::kBFloat16));
+  if (fp8)
+    TORCH_CHECK(n_splits > 1 && n_q <= 128 && out_scale->is_contiguous() &&
+                    out_scale->scalar_type() == torch::kFloat32 && out_scale->numel() == B,
+                "fp8 rows come from the merge of up to 128 heads");
   torch::Tensor part_o, part_ml;
   float *part_o_ptr = nullptr, *part_ml_ptr = nullptr;
   if (n_splits > 1) {
@@ -463,7 +535,23 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
   if (k_cache.scalar_type() == torch::kFloat8_e5m2) with_hd((unsigned char)0);
   else with_hd((ushort)0);
   HIP_CHECK_KERNEL();
-  if (n_splits > 1) {
+  if (fp8) {
+    auto merge = [&](auto hdv, auto hpw) {
+      hipLaunchKernelGGL(
+          (decode_merge_fp8_kernel<decltype(hdv)::value, decltype(hpw)::value>), dim3(B),
+          dim3(16 * WAVE_SIZE), 0, stream, (unsigned char*)out.data_ptr(),
+          out_scale->data_ptr<float>(), part_o_ptr, part_ml_ptr, n_splits, n_q);
+    };
+    auto heads = [&](auto hdv) {
+      if (n_q <= 16) merge(hdv, std::integral_constant<int, 1>{});
+      else if (n_q <= 32) merge(hdv, std::integral_constant<int, 2>{});
+      else if (n_q <= 64) merge(hdv, std::integral_constant<int, 4>{});
+      else merge(hdv, std::integral_constant<int, 8>{});
+    };
+    if (hd == 256) heads(std::integral_constant<int, 256>{});
+    else heads(std::integral_constant<int, 128>{});
+    HIP_CHECK_KERNEL();
+  } else if (n_splits > 1) {
     const int64_t n_bh = (int64_t)B * n_q;
     const int wpb = 4;
     const dim3 mgrid((uint32_t)((n_bh + wpb - 1) / wpb)), mblock(wpb * WAVE_SIZE);

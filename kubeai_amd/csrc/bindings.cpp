@@ -34,7 +34,8 @@ void reshape_and_cache(torch::Tensor k, torch::Tensor v, torch::Tensor k_cache,
 void paged_attention_decode(torch::Tensor out, torch::Tensor q,
                             torch::Tensor k_cache, torch::Tensor v_cache,
                             torch::Tensor block_tables, torch::Tensor seq_lens,
-                            double scale, int64_t window, double softcap);
+                            double scale, int64_t window, double softcap,
+                            c10::optional<torch::Tensor> out_scale);
 int paged_decode_splits(int rows, int n_kv, int hd, int max_blocks);
 void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
                              torch::Tensor k_cache, torch::Tensor v_cache,

@@ -182,10 +182,19 @@ class Attention(nn.Module):
                 fb.slot_mapping,
             )
 
+        nd = fb.n_decode
+        if fp8_in and nd == T and fb.n_prefill == 0:
+            return _project(
+                self.o_proj,
+                ops.paged_attention_decode_fp8(
+                    q, k_cache, v_cache, fb.decode_block_tables, fb.decode_seq_lens,
+                    self.scale, window=self.window, softcap=self.softcap,
+                ),
+                as_sums, fb,
+            )
         out = torch.empty(
             (T, self.n_q, self.hd), dtype=q.dtype, device=q.device
         )
-        nd = fb.n_decode
         if nd > 0:
             ops.paged_attention_decode(
                 q[:nd],

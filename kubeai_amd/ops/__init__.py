@@ -138,7 +138,7 @@ def paged_attention_decode(
             out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
         _C.paged_attention_decode(
             out, q, k_cache, v_cache, block_tables, seq_lens, scale, window,
-            softcap
+            softcap, None
         )
         return out
     res = ref.paged_attention_decode(
@@ -149,6 +149,26 @@ def paged_attention_decode(
         out.copy_(res)
         return out
     return res
+
+
+def paged_attention_decode_fp8(
+    q, k_cache, v_cache, block_tables, seq_lens, scale: float, window: int = 0,
+    softcap: float = 0.0,
+):
+    """quant_fp8 of paged_attention_decode's rows [B, n_q * hd]. On GPU the merge of
+    a row's splits converts them, where there is more than one."""
+    B, n_q, hd = q.shape
+    if not q.is_cuda or n_q > 128 or B == 0 or (
+        _C.paged_decode_splits(B, k_cache.shape[1], hd, block_tables.shape[1]) == 1
+    ):
+        out = paged_attention_decode(q, k_cache, v_cache, block_tables, seq_lens, scale,
+                                     window=window, softcap=softcap)
+        return quant_fp8(out.view(B, n_q * hd))
+    out = torch.empty((B, n_q * hd), dtype=torch.float8_e4m3fn, device=q.device)
+    out_scale = torch.empty(B, dtype=torch.float32, device=q.device)
+    _C.paged_attention_decode(out, q, k_cache, v_cache, block_tables, seq_lens, scale,
+                              window, softcap, out_scale)
+    return out, out_scale
 
 
 def paged_attention_prefill(

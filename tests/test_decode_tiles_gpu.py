@@ -151,3 +151,26 @@ def test_one_long_row_among_short_ones(group, cache):
 def test_softcap_on_both_sides_of_its_forms(hd, spread):
     """Scores about and on both sides of 0.7 of the cap, where the form changes."""
     _run([70, 33], 4, 2, hd, spread * 20.0 * hd ** -0.5, softcap=20.0)
+
+
+@pytest.mark.parametrize("rows,n_q,n_kv,hd", [
+    (1, 8, 8, 128), (3, 32, 8, 128), (40, 32, 8, 128), (9, 40, 8, 128), (5, 128, 16, 128),
+    (2, 136, 17, 128), (7, 8, 4, 256), (4, 16, 16, 256), (96, 32, 8, 128),
+])
+def test_fp8_rows_are_the_converted_bf16_rows(rows, n_q, n_kv, hd):
+    """Merged and converted in one launch (up to 128 heads, more than one split) or
+    in two: the same bytes and scales."""
+    torch.manual_seed(rows + n_q)
+    lens = [int(x) for x in torch.randint(1, 900, (rows,))]
+    lens[0] = 900
+    width = (max(lens) + 15) // 16
+    nb = rows * width + 1
+    kc, vc = (torch.randn(nb, n_kv, 16, hd, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    bt = (torch.randperm(nb - 1)[: rows * width] + 1).int().view(rows, width).to(DEV)
+    total = torch.tensor(lens, device=DEV, dtype=torch.int32)
+    q = torch.randn(rows, n_q, hd, device=DEV, dtype=torch.bfloat16)
+    got, scale = ops.paged_attention_decode_fp8(q, kc, vc, bt, total, hd ** -0.5)
+    out = ops.paged_attention_decode(q, kc, vc, bt, total, hd ** -0.5)
+    want, want_scale = ops.quant_fp8(out.view(rows, -1))
+    assert torch.equal(scale, want_scale)
+    assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
