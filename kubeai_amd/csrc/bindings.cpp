@@ -77,7 +77,8 @@ void gumbel_sample(torch::Tensor out, torch::Tensor logits,
 void sgmv(torch::Tensor y, torch::Tensor x, torch::Tensor A, torch::Tensor B,
           torch::Tensor idx, double scale);
 void lora_apply(torch::Tensor y, torch::Tensor x, torch::Tensor table,
-                torch::Tensor ids, int64_t max_rank);
+                torch::Tensor ids, int64_t max_rank,
+                std::optional<torch::Tensor> z);
 void register_chwbl(pybind11::module_& m);
 // one-shot fused all-reduce over xGMI (allreduce.hip)
 pybind11::bytes xgmi_alloc();
@@ -159,6 +160,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("xgmi_shutdown", &xgmi_shutdown, "free/close comm buffers");
   m.def("sgmv", &sgmv, "segmented gather LoRA apply (one adapter segment)");
   m.def("lora_apply", &lora_apply,
-        "LoRA apply over a batch of tokens with mixed adapters");
+        "LoRA apply over a batch of tokens with mixed adapters",
+        py::arg("y"), py::arg("x"), py::arg("table"), py::arg("ids"),
+        py::arg("max_rank"), py::arg("z") = py::none());
   register_chwbl(m);
 }

@@ -58,8 +58,8 @@ def _hooked(module: nn.Module) -> bool:
 def _project(linear, x, as_sums: bool, fb: ForwardBatch | None, rope: bool = False):
     """linear(x), x a tensor or an (fp8 rows, scales) pair. as_sums: what reads
     the result, a norm or (rope) the rotation, takes ops.ProductSums, so it may
-    be that. Steps with prompt portions are never recorded in a graph."""
-    eager = fb is not None and fb.n_prefill > 0
+    be that. Steps with prompt portions or adapters are never recorded in a graph."""
+    eager = fb is not None and (fb.n_prefill > 0 or fb.lora_ids is not None)
     if isinstance(x, tuple):
         sums = getattr(linear, "sums_quantized", None) if as_sums else None
         y = sums(*x, rope, eager) if sums is not None else None
@@ -68,6 +68,20 @@ def _project(linear, x, as_sums: bool, fb: ForwardBatch | None, rope: bool = Fal
     if as_sums and type(linear) is EngineLinear and not _hooked(linear):
         y = linear.sums(x, rope, eager)
     return linear(x) if y is None else y
+
+
+def _project_adapted(linear, x, as_sums: bool, fb, lm, layer_idx, target, rope=False):
+    """_project with the adapters' products of x added: to the first part of the
+    sums, where the adapters go in one batch."""
+    batch = None
+    if as_sums and isinstance(linear, nn.Linear):
+        batch = lm.batch(layer_idx, target, x, fb.lora_ids, linear.out_features)
+    y = _project(linear, x, batch is not None, fb, rope)
+    if isinstance(y, ops.ProductSums):
+        lm.apply_batch(batch, x, y.part[0], fb.lora_ids)
+    else:
+        lm.apply(layer_idx, target, x, y, fb.lora_ids)
+    return y
 
 
 def _call(module, *args, **own):
@@ -148,14 +162,16 @@ class Attention(nn.Module):
         T = (x[0] if fp8_in else x).shape[0]
         lm = None if fp8_in else getattr(self, "_lora_manager", None)
         lora_live = lm is not None and lm.active and fb.lora_ids is not None
-        qkv = _project(
-            self.qkv_proj, x,
-            T <= ops.MAX_SUM_ROWS and not lora_live and not self.qk_norm
-            and ops.rope_takes_sums(k_cache, v_cache),
-            fb, rope=True,
+        qkv_sums = (
+            T <= ops.MAX_SUM_ROWS and not self.qk_norm
+            and ops.rope_takes_sums(k_cache, v_cache)
         )
         if lora_live:
-            lm.apply(self.layer_idx, "qkv", x, qkv, fb.lora_ids)
+            qkv = _project_adapted(
+                self.qkv_proj, x, qkv_sums, fb, lm, self.layer_idx, "qkv", rope=True
+            )
+        else:
+            qkv = _project(self.qkv_proj, x, qkv_sums, fb, rope=True)
         if isinstance(cos_sin, tuple):
             # (global, local) caches — gemma3 dual rope bases
             cos_sin = cos_sin[0] if self.is_global else cos_sin[1]
@@ -223,10 +239,11 @@ class Attention(nn.Module):
         attn_flat = out.view(T, -1)
         if fp8_in:
             return _project(self.o_proj, ops.quant_fp8(attn_flat), as_sums, fb)
-        result = _project(self.o_proj, attn_flat, as_sums and not lora_live, fb)
         if lora_live:
-            lm.apply(self.layer_idx, "o", attn_flat, result, fb.lora_ids)
-        return result
+            return _project_adapted(
+                self.o_proj, attn_flat, as_sums, fb, lm, self.layer_idx, "o"
+            )
+        return _project(self.o_proj, attn_flat, as_sums, fb)
 
 
 class MLP(nn.Module):
@@ -268,12 +285,17 @@ class MLP(nn.Module):
         if a is None:
             h = self.gate_up_proj(x)
             if lora_live:
-                lm.apply(self.layer_idx, "gate_up", x, h, fb.lora_ids)
-            a = ops.gelu_and_mul(h) if self.gelu else ops.silu_and_mul(h)
-        y = _project(self.down_proj, a, as_sums and not lora_live, fb)
+                if not self.gelu:
+                    a = lm.gated(self.layer_idx, x, h, fb.lora_ids)
+                if a is None:
+                    lm.apply(self.layer_idx, "gate_up", x, h, fb.lora_ids)
+            if a is None:
+                a = ops.gelu_and_mul(h) if self.gelu else ops.silu_and_mul(h)
         if lora_live:
-            lm.apply(self.layer_idx, "down", a, y, fb.lora_ids)
-        return y
+            return _project_adapted(
+                self.down_proj, a, as_sums, fb, lm, self.layer_idx, "down"
+            )
+        return _project(self.down_proj, a, as_sums, fb)
 
 
 def _own_tensor(module: nn.Module, name: str):

@@ -165,3 +165,106 @@ def test_infinite_weights_reach_the_output(rank):
     _C.lora_apply(y, x, table, torch.ones(4, dtype=torch.int32, device=DEV), rank)
     assert want[0, 3] == float("inf") and want[1, 3] == -float("inf") and want[2, 3].isnan()
     torch.testing.assert_close(y.double(), want, atol=1e-4, rtol=2.0 ** -8, equal_nan=True)
+
+
+@pytest.mark.parametrize("T,out", [(1, 512), (17, 514), (50, 36), (97, 6144)])
+def test_sums_take_the_adapters_in_their_first_part(T, out):
+    """fp32 rows: nothing is rounded, so they are within the error of the fp32
+    sums (1024 + 16 terms; 2^-14 of the magnitudes is above 1040 * 2^-24)."""
+    from kubeai_amd import _C
+
+    torch.manual_seed(T)
+    ids = [(0, 3, 9, 5)[t * 7 % 4] for t in range(T)]
+    x = torch.randn(T, 1024, device=DEV, dtype=torch.bfloat16)
+    part = torch.randn(3, T, out, device=DEV)
+    sets = {lid: (torch.randn(r, 1024, device=DEV, dtype=torch.bfloat16) * 0.1,
+                  torch.randn(out, r, device=DEV, dtype=torch.bfloat16), 2.0 / r)
+            for lid, r in ((3, 16), (9, 5))}
+    table = torch.tensor([[A.data_ptr(), B.data_ptr(), _two_words(A.shape[0], lid), _float_word(s)]
+                          for lid, (A, B, s) in sets.items()], dtype=torch.int64, device=DEV)
+    want, size = part.double(), part.double().abs()
+    for t, lid in enumerate(ids):
+        if lid in sets:
+            A, B, s = sets[lid]
+            want[0, t] += (B.double() @ (A.double() @ x[t].double())) * s
+            size[0, t] += (B.double().abs() @ (A.double().abs() @ x[t].double().abs())) * s
+    _C.lora_apply(part[0], x, table, torch.tensor(ids, dtype=torch.int32, device=DEV), 16)
+    assert ((part.double() - want).abs() <= size * 2.0 ** -14).all()
+    assert torch.equal(part[1:].double(), want[1:])
+
+
+def test_sums_of_a_product_with_adapters_equal_the_whole_one():
+    """A projection as sums with the adapters in, against the product of bf16 rows
+    with them added (rounded twice: 2^-8 of the larger of product and result)."""
+    from kubeai_amd import ops
+    from kubeai_amd.models.llama import EngineLinear, _project_adapted
+
+    torch.manual_seed(0)
+    m = LoRAManager(_Model(), DEV, torch.bfloat16)
+    for lid in (4, 7):
+        m.load(lid, None)
+    fb = type("Batch", (), {})()
+    fb.n_prefill = 1
+    fb.lora_ids = torch.tensor([4, 0, 7, 7, 4, 1] * 20, dtype=torch.int32, device=DEV)
+    lin = EngineLinear(256, 128, bias=False).to(DEV, torch.bfloat16).requires_grad_(False)
+    x = torch.randn(120, 256, device=DEV, dtype=torch.bfloat16)
+    for rows in (6, 24, 120):
+        ids, fb.lora_ids = fb.lora_ids, fb.lora_ids[:rows].contiguous()
+        whole = _project_adapted(lin, x[:rows], False, fb, m, 1, "down")
+        as_sums = _project_adapted(lin, x[:rows], True, fb, m, 1, "down")
+        fb.lora_ids = ids
+        got = as_sums.part.sum(0) if isinstance(as_sums, ops.ProductSums) else as_sums
+        assert rows > 96 or isinstance(as_sums, ops.ProductSums)
+        size = 2.0 ** -8 * (whole.float().abs() + lin(x[:rows]).float().abs())
+        assert ((got.float() - whole.float()).abs() <= size + 1e-4).all()
+
+
+@pytest.mark.parametrize("T,inner", [(1, 8), (16, 248), (17, 264), (50, 1032)])
+def test_gated_outputs(T, inner):
+    """silu(gate) * up with the adapters in: one rounding to bf16 (2^-9 of the
+    result); the kernel's exponential and quotient stay within 2^-20 of the value,
+    the fp32 sums within 2^-14 of their magnitudes, which gate and up pass on with
+    factors up to |up| * 1.1 and |silu(gate)|."""
+    from kubeai_amd import _C
+
+    torch.manual_seed(T)
+    ids = [(0, 3, 9, 5)[t * 7 % 4] for t in range(T)]
+    x = torch.randn(T, 264, device=DEV, dtype=torch.bfloat16)
+    y = torch.randn(T, 2 * inner, device=DEV, dtype=torch.bfloat16)
+    sets = {lid: (torch.randn(r, 264, device=DEV, dtype=torch.bfloat16) * 0.1,
+                  torch.randn(2 * inner, r, device=DEV, dtype=torch.bfloat16), 2.0 / r)
+            for lid, r in ((3, 16), (9, 5))}
+    table = torch.tensor([[A.data_ptr(), B.data_ptr(), _two_words(A.shape[0], lid), _float_word(s)]
+                          for lid, (A, B, s) in sets.items()], dtype=torch.int64, device=DEV)
+    h, size, was = y.double(), y.double().abs(), y.clone()
+    for t, lid in enumerate(ids):
+        if lid in sets:
+            A, B, s = sets[lid]
+            h[t] += (B.double() @ (A.double() @ x[t].double())) * s
+            size[t] += (B.double().abs() @ (A.double().abs() @ x[t].double().abs())) * s
+    z = torch.empty(T, inner, device=DEV, dtype=torch.bfloat16)
+    _C.lora_apply(y, x, table, torch.tensor(ids, dtype=torch.int32, device=DEV), 16, z)
+    gate, up = h[:, :inner], h[:, inner:]
+    silu = gate * torch.sigmoid(gate)
+    want = silu * up
+    bound = want.abs() * 2.0 ** -8 + 2.0 ** -14 * (
+        1.1 * up.abs() * size[:, :inner] + silu.abs() * size[:, inner:]
+    ) + 1e-6
+    assert ((z.double() - want).abs() <= bound).all()
+    assert torch.equal(y, was)
+
+
+def test_gated_manager_equals_the_two_steps():
+    """Against apply() and the activation, which round gate and up to bf16 first
+    (2^-9 each, and 2^-9 of the result in both)."""
+    from kubeai_amd import ops
+
+    m = LoRAManager(_Model(), DEV, torch.bfloat16)
+    m.load(4, None)
+    ids = torch.tensor([4, 0, 1, 4, 4, 0], dtype=torch.int32, device=DEV)
+    x = torch.randn(6, 128, device=DEV, dtype=torch.bfloat16)
+    y = torch.randn(6, 512, device=DEV, dtype=torch.bfloat16)
+    z = m.gated(1, x, y, ids)
+    m.apply(1, "gate_up", x, y, ids)
+    torch.testing.assert_close(z, ops.silu_and_mul(y), atol=1e-4, rtol=2.0 ** -6)
+    assert m.gated(1, x, y[:, 1:], ids) is None
