@@ -143,6 +143,98 @@ __global__ __launch_bounds__(256) void qknorm_rope_half_cache_kernel(
   }
 }
 
+// The same where half, D and Dv are whole 16-byte units and everything is aligned: a
+// token's q and k are read once, summed in the order of the form above (so the
+// results are the same to the last bit) and kept in LDS, from which pairs are turned
+// a unit at a time; sine and cosine are taken once a token, not once a head. Bound
+// by latency, then by memory (q twice, k and v twice). 3072 tokens, 16 heads and 4
+// of 128: 38 -> 27 us (17 with vectors in registers, summed in another order).
+template <typename T>
+__global__ __launch_bounds__(256) void qknorm_rope_half_rows_kernel(
+    T* __restrict__ q, int64_t q_stride, const T* __restrict__ k,
+    int64_t k_stride, const T* __restrict__ v, int64_t v_stride,
+    const float* __restrict__ qw, const float* __restrict__ kw, float eps,
+    const int* __restrict__ positions, const float* __restrict__ inv_freq,
+    int half, T* __restrict__ k_cache, T* __restrict__ v_cache,
+    const int64_t* __restrict__ slot_mapping, int H, int G, int D, int Dv,
+    int bs) {
+  constexpr int N = Vec16<T>::N;
+  extern __shared__ __attribute__((aligned(16))) float qk_rows[];
+  float* rows = qk_rows;              // [(H + G) D] q, then k
+  float* turn = rows + (H + G) * D;   // [half] cos, [half] sin
+  __shared__ float red0[16], red1[16];
+  const int t = blockIdx.x;
+  const int64_t slot = slot_mapping[t];
+  T* qr = q + (size_t)t * q_stride;
+  const T* kr = k + (size_t)t * k_stride;
+  float sq = 0.f, sk = 0.f;
+#pragma unroll 8
+  for (int i = threadIdx.x; i < H * D; i += 256) {
+    const float x = ldf(qr + i);
+    rows[i] = x;
+    sq += x * x;
+  }
+#pragma unroll 2
+  for (int i = threadIdx.x; i < G * D; i += 256) {
+    const float x = ldf(kr + i);
+    rows[H * D + i] = x;
+    sk += x * x;
+  }
+  const float pos = (float)positions[t];
+  for (int i = threadIdx.x; i < half; i += 256) {
+    float sn, cs;
+    sincosf(pos * inv_freq[i], &sn, &cs);
+    turn[i] = cs;
+    turn[half + i] = sn;
+  }
+  const int64_t blk = slot >= 0 ? slot / bs : 0;
+  const int off = slot >= 0 ? (int)(slot % bs) : 0;
+  if (slot >= 0)
+    for (int e = threadIdx.x * N; e < G * Dv; e += 256 * N)
+      *(uint4*)(v_cache + (((size_t)blk * G + e / Dv) * bs + off) * Dv + e % Dv) =
+          *(const uint4*)(v + (size_t)t * v_stride + e);
+  float rq = 1.f, rk = 1.f;
+  if (qw != nullptr) {
+    rq = 1.0f / sqrtf(block_sum(sq, red0) / (float)(H * D) + eps);
+    rk = 1.0f / sqrtf(block_sum(sk, red1) / (float)(G * D) + eps);
+  }
+  __syncthreads();
+  const int pairs = half / N, uph = (D - half) / N;  // units per head, pairs first
+  const int heads = slot >= 0 ? H + G : H;
+  for (int u = threadIdx.x; u < heads * uph; u += 256) {
+    const int hd = u / uph, i = u % uph;
+    const bool is_q = hd < H;
+    const int h = is_q ? hd : hd - H, at = i < pairs ? i * N : half + i * N;
+    const float r = is_q ? rq : rk;
+    const float* w = qw == nullptr ? nullptr : (is_q ? qw : kw) + h * D + at;
+    const float* src = rows + hd * D + at;
+    T* dst = (is_q ? qr + h * D : k_cache + (((size_t)blk * G + h) * bs + off) * D) + at;
+    float a[N], b[N], x[N], y[N];
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      a[e] = src[e] * r;
+      if (w != nullptr) a[e] *= w[e];
+    }
+    if (i < pairs) {
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        b[e] = src[half + e] * r;
+        if (w != nullptr) b[e] *= w[half + e];
+      }
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        const float cs = turn[at + e], sn = turn[half + at + e];
+        x[e] = a[e] * cs - b[e] * sn;
+        y[e] = b[e] * cs + a[e] * sn;
+      }
+      Vec16<T>::store(dst, x);
+      Vec16<T>::store(dst + half, y);
+    } else {
+      Vec16<T>::store(dst, a);
+    }
+  }
+}
+
 // grid (T). Whole-row RMS norms of q and k when a cached row is key and value:
 // q <- q / rms(q) * w in place; k's row goes to the cache as it is and
 // 1 / rms(k) to key_scale. kVec: 16-byte accesses (rows and heads of whole,
@@ -868,18 +960,30 @@ void qknorm_rope_half_and_cache(torch::Tensor q, torch::Tensor k, torch::Tensor 
               k_cache.scalar_type() == q.scalar_type() &&
               v_cache.scalar_type() == q.scalar_type());
   if (T == 0) return;
+  auto al16 = [](const torch::Tensor& t) { return (size_t)t.data_ptr() % 16 == 0; };
+  const bool aligned =
+      al16(q) && al16(k) && al16(v) && al16(k_cache) && al16(v_cache) &&
+      (!q_weight.has_value() || (al16(*q_weight) && al16(*k_weight)));
   SEQ_DISPATCH_ACT(q, {
-    hipLaunchKernelGGL((qknorm_rope_half_cache_kernel<act_t>), dim3(T), dim3(256), 0,
-                       SEQ_STREAM(), (act_t*)q.data_ptr(), q.stride(0),
-                       (const act_t*)k.data_ptr(), k.stride(0),
-                       (const act_t*)v.data_ptr(), v.stride(0),
-                       q_weight.has_value() ? (const float*)q_weight->data_ptr() : nullptr,
-                       k_weight.has_value() ? (const float*)k_weight->data_ptr() : nullptr,
-                       (float)eps, (const int*)positions.data_ptr(),
-                       (const float*)inv_freq.data_ptr(), half,
-                       (act_t*)k_cache.data_ptr(), (act_t*)v_cache.data_ptr(),
-                       (const int64_t*)slot_mapping.data_ptr(), H, G, D, Dv,
-                       (int)k_cache.size(2));
+    constexpr int N = Vec16<act_t>::N;
+    auto go = [&](auto kernel, size_t lds) {
+      hipLaunchKernelGGL(
+          kernel, dim3(T), dim3(256), lds, SEQ_STREAM(), (act_t*)q.data_ptr(),
+          q.stride(0), (const act_t*)k.data_ptr(), k.stride(0),
+          (const act_t*)v.data_ptr(), v.stride(0),
+          q_weight.has_value() ? (const float*)q_weight->data_ptr() : nullptr,
+          k_weight.has_value() ? (const float*)k_weight->data_ptr() : nullptr, (float)eps,
+          (const int*)positions.data_ptr(), (const float*)inv_freq.data_ptr(), half,
+          (act_t*)k_cache.data_ptr(), (act_t*)v_cache.data_ptr(),
+          (const int64_t*)slot_mapping.data_ptr(), H, G, D, Dv, (int)k_cache.size(2));
+    };
+    const size_t lds = sizeof(float) * ((size_t)(H + G) * D + 2 * half);
+    if (aligned && half % N == 0 && D % N == 0 && Dv % N == 0 && q.stride(0) % N == 0 &&
+        k.stride(0) % N == 0 && v.stride(0) % N == 0 && lds <= 48 * 1024) {
+      go(qknorm_rope_half_rows_kernel<act_t>, lds);
+    } else {
+      go(qknorm_rope_half_cache_kernel<act_t>, 0);
+    }
   });
   SEQ_CHECK_LAUNCH();
 }

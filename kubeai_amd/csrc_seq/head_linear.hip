@@ -77,6 +77,81 @@ __global__ __launch_bounds__(kHlWaves * WAVE) void head_linear_mfma_kernel(
   }
 }
 
+// The same where A is kSteps * 16, B a multiple of 32 and y's (and a gate's) rows are
+// whole 16-byte units: NT * 16 tokens a wave share every byte of W[h], and a lane ends
+// up with 8 neighbouring channels of a token, which it writes at once: two tiles of
+// 16 channels are made together, row m of tile j being channel 8 (m >> 2) + 4 j +
+// (m & 3). Same steps of the sum, so the same bits. Bound by memory where tokens are
+// many (x, gate and y once each). 3072 tokens x 16 heads of 128 -> 128 with a gate:
+// 36 -> 30 us (38 MB; 21 with 16-byte loads of x and W, whose other order of the sum
+// moves a routed token to another expert now and then).
+template <int kSteps, int NT>
+__global__ __launch_bounds__(kHlWaves * WAVE) void head_linear_wide_kernel(
+    bf16raw* __restrict__ y, int64_t y_stride, int64_t y_hs,
+    const bf16raw* __restrict__ x, int64_t x_stride, int64_t x_hs,
+    const bf16raw* __restrict__ w, const bf16raw* __restrict__ gate,
+    int64_t gate_stride, int gate_per_head, int T, int H, int, int B, int b_per) {
+  constexpr int A = kSteps * 16;
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const int col = lane & 15, grp = lane >> 4;
+  const int t0 = (blockIdx.x * kHlWaves + wave) * 16 * NT;
+  if (t0 >= T) return;
+  const int h = blockIdx.y;
+  bf16x4 xf[NT][kSteps];
+  float hg[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    const size_t t = min(t0 + n * 16 + col, T - 1);
+    const bf16raw* xr = x + t * x_stride + (size_t)h * x_hs + grp * 4;
+#pragma unroll
+    for (int ks = 0; ks < kSteps; ++ks) xf[n][ks] = *(const bf16x4*)(xr + ks * 16);
+    hg[n] = gate != nullptr && gate_per_head
+                ? sigmoid_f(bf16_to_f32(gate[t * gate_stride + h])) : 1.f;
+  }
+  const bool per_channel = gate != nullptr && !gate_per_head;
+  const bf16raw* wl = w + (size_t)h * B * A + grp * 4;
+  const int row = (col >> 2) * 8 + (col & 3);
+  const int b_end = min(B, (int)(blockIdx.z + 1) * b_per);
+  for (int b0 = blockIdx.z * b_per; b0 < b_end; b0 += 32) {
+    const int c = b0 + grp * 8;
+    float g[NT][8];
+    if (per_channel) {
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+        Vec16<bf16raw>::load(
+            gate + (size_t)min(t0 + n * 16 + col, T - 1) * gate_stride + (size_t)h * B + c,
+            g[n]);
+    }
+    f32x4 acc[2][NT];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int n = 0; n < NT; ++n) acc[j][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < kSteps; ++ks)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const bf16x4 wf = *(const bf16x4*)(wl + (size_t)(b0 + row + j * 4) * A + ks * 16);
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+          acc[j][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wf, xf[n][ks], acc[j][n],
+                                                                0, 0, 0);
+      }
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      const int t = t0 + n * 16 + col;
+      float o[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        o[e] = acc[e / 4][n][e % 4] * hg[n];
+        if (per_channel) o[e] *= sigmoid_f(g[n][e]);
+      }
+      if (t < T)
+        Vec16<bf16raw>::store(y + (size_t)t * y_stride + (size_t)h * y_hs + c, o);
+    }
+  }
+}
+
 // Any dtype and size: grid (T, H), the head's input row in LDS, one output
 // channel per thread at a time, fp32 accumulation.
 template <typename T_>
@@ -143,9 +218,18 @@ void head_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
       al8(x.data_ptr(), x.stride(0)) && al8(y.data_ptr(), y.stride(0)) &&
       x_hs % 4 == 0 && y_hs % 4 == 0 && al8(w.data_ptr(), 4) &&
       (gp == nullptr || gph || al8(gp, gs))) {
-    const int tb = (T + 16 * kHlWaves - 1) / (16 * kHlWaves), tiles = B / 16;
+    auto al16 = [](const void* p, int64_t stride) {
+      return ((size_t)p) % 16 == 0 && stride % 8 == 0;
+    };
+    const bool wide = A >= 32 && A <= 512 && (A & (A - 1)) == 0 && B % 32 == 0 &&
+                      al16(y.data_ptr(), y.stride(0)) && y_hs % 8 == 0 &&
+                      (gp == nullptr || gph || al16(gp, gs));
+    // 32 tokens a wave where that leaves a workgroup a CU, and registers for them
+    const bool two = wide && A <= 128 && (int64_t)(T + 127) / 128 * H >= 256;
+    const int per = 16 * kHlWaves * (two ? 2 : 1), unit = wide ? 32 : 16;
+    const int tb = (T + per - 1) / per, tiles = B / unit;
     const int parts = std::max(1, std::min(tiles, 512 / (tb * H)));
-    const int b_per = (tiles + parts - 1) / parts * 16;
+    const int b_per = (tiles + parts - 1) / parts * unit;
     const dim3 grid(tb, H, (B + b_per - 1) / b_per);
     auto launch = [&](auto kern) {
       hipLaunchKernelGGL(kern, grid, dim3(kHlWaves * WAVE), 0, SEQ_STREAM(),
@@ -154,6 +238,20 @@ void head_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                          (const bf16raw*)w.data_ptr(), (const bf16raw*)gp, gs, gph, T,
                          H, A, B, b_per);
     };
+    if (wide) {
+      switch (A) {
+        case 32: two ? launch(head_linear_wide_kernel<2, 2>)
+                     : launch(head_linear_wide_kernel<2, 1>); break;
+        case 64: two ? launch(head_linear_wide_kernel<4, 2>)
+                     : launch(head_linear_wide_kernel<4, 1>); break;
+        case 128: two ? launch(head_linear_wide_kernel<8, 2>)
+                      : launch(head_linear_wide_kernel<8, 1>); break;
+        case 256: launch(head_linear_wide_kernel<16, 1>); break;
+        default: launch(head_linear_wide_kernel<32, 1>);
+      }
+      SEQ_CHECK_LAUNCH();
+      return;
+    }
     if (A <= 128) launch(head_linear_mfma_kernel<8>);
     else launch(head_linear_mfma_kernel<32>);
     SEQ_CHECK_LAUNCH();
