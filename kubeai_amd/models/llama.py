@@ -2,10 +2,11 @@
 
 MI355X-first execution model (one process per GPU):
   - token-packed forward ([T, H], no padding) over the ForwardBatch;
-  - plain GEMMs (qkv/o/gate_up/down/lm_head) go through torch.nn.functional
-    .linear, i.e. hipBLASLt/rocBLAS on ROCm — library GEMMs per the design
-    rules; every fused hot op (rmsnorm, rope, cache write, paged attention,
-    SwiGLU) is a hand-written gfx950 kernel via kubeai_amd.ops;
+  - products (qkv/o/gate_up/down/lm_head) go through ops.linear: the
+    weight-streaming or the tiled kernel where they are the faster ones, as
+    sums that the next norm or rotation adds or with the activation behind
+    them, hipBLASLt for the rest; every other hot op (rmsnorm, rope, cache
+    write, paged attention) is a hand-written gfx950 kernel via kubeai_amd.ops;
   - KV cache is paged [num_blocks, n_kv, block_size, head_dim] bf16, owned by
     the runner and passed in.
 
@@ -500,11 +501,16 @@ class MoEMLP(nn.Module):
             return y
 
         width = 2 * first.down_proj.in_features
+        # Steps that the weight-streaming product may have as well round gate and up
+        # as it does, before the activation; larger ones have it in the tiled product,
+        # which saves these rows' way to memory and back.
+        fused = x.shape[0] > self.GROUPED_MAX_TOKENS
         if fp8:
-            h = products(ops.quant_fp8_rows(x, src), "gate_up_proj", width, act=1)
+            h = products(ops.quant_fp8_rows(x, src), "gate_up_proj", width, act=int(fused))
             a = ops.silu_and_mul_fp8(h) if h.shape[1] == width else ops.quant_fp8(h)
         else:
-            a = products(x, "gate_up_proj", width, src, act=2 if self.gelu else 1)
+            act = 0 if not fused else 2 if self.gelu else 1
+            a = products(x, "gate_up_proj", width, src, act)
             if a.shape[1] == width:
                 a = ops.gelu_and_mul(a) if self.gelu else ops.silu_and_mul(a)
         return ops.moe_combine(products(a, "down_proj", x.shape[1]), place, weight)
