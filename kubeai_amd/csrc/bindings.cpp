@@ -14,6 +14,7 @@ void rope_cache(torch::Tensor qkv, torch::Tensor positions,
                 c10::optional<torch::Tensor> sx,
                 c10::optional<torch::Tensor> sw);
 torch::Tensor skinny_sums(torch::Tensor x, torch::Tensor w);
+void skinny_gated(torch::Tensor y, torch::Tensor x, torch::Tensor w, int64_t act);
 void quant_fp8_rows(torch::Tensor out, torch::Tensor out_scale, torch::Tensor x,
                     torch::Tensor src);
 void rmsnorm_sums(torch::Tensor out, c10::optional<torch::Tensor> out_scale,
@@ -139,6 +140,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("experts") = 1);
   m.def("tiled_sums", &tiled_sums, "fp32 part sums of a product of many rows");
   m.def("skinny_sums", &skinny_sums, "fp32 part sums of a skinny product");
+  m.def("skinny_gated", &skinny_gated, "weight-streaming gate and up, activated");
   m.def("quant_fp8_rows", &quant_fp8_rows, "gathered bf16 rows -> fp8");
   m.def("rmsnorm_sums", &rmsnorm_sums, "norm of a product's part sums");
   m.def("norm_add_norm", &norm_add_norm,

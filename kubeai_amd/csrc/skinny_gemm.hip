@@ -2,40 +2,51 @@
 // M <= 96, bf16 or fp8 e4m3 (W8A8 with row and column scales), bf16 out,
 // fp32 accumulation. Decode batches and the logits of a step's last tokens.
 //
-// Bound by reading W once. What it takes to read it at the card's rate:
+// Bound by reading W once: 6.3 TB/s is what plain reads in order reach here. What it
+// takes to come near that:
 //  - workgroup = 4 waves x 16 rows of W. A wave's lanes read 16 rows x 64
 //    contiguous bytes straight into matrix operands (no LDS for W: each byte
-//    is used by one wave); two of those loads fill a 128-byte line. The next
-//    256 (M <= 32: 512) bytes of every row are in flight while the current
-//    ones are multiplied.
+//    is used by one wave); two of those loads fill a 128-byte line. The steps
+//    are 256 bytes of every row; two of them are in flight behind the one that is
+//    multiplied. Loads past the end are of no bytes instead of in a branch: where
+//    paths of more and of fewer loads meet, the compiler waits for all of them (one
+//    row of 28672 x 4096 bf16: 46.5 us -> 43.4).
 //  - x is what the CUs would re-read: with 16 rows of W per workgroup its
 //    traffic is M / 16 that of W, and past M = 16 that limits (40 rows fp8:
-//    54 us for 28672 x 4096 against 28 with x shared by 64 rows). It is
-//    staged through LDS (double-buffered, one barrier a step, 16-byte units
-//    XOR-swizzled by row) and shared by the four waves.
-//  - few output columns do not fill the chip: K is cut into up to 8 parts
-//    (blockIdx.y), whose fp32 sums lie in a workspace [parts, M, N]; a second
-//    kernel adds them (no atomics: the order of the sum is fixed).
+//    54 us for 28672 x 4096 against 28 with x shared by 64 rows). It goes
+//    straight to LDS (three places, one barrier a step, 16-byte units
+//    XOR-swizzled by row by the choice of source) and is shared by the waves.
+//  - few output columns do not fill the chip: K is cut into up to 8 parts,
+//    whose fp32 sums lie in a workspace [parts, M, N]; a second
+//    kernel adds them (no atomics: the order of the sum is fixed). The parts of
+//    a row lie in neighbouring workgroups: what is read at a time is whole rows
+//    (6144 x 4096 bf16 in 8 parts, read alone: 9.8 us apart, 9.4).
+//  - uncut, the workgroups begin at columns of K apart. At the same columns of rows
+//    of 2^n bytes all of them wait for the same few channels of the memory (read
+//    alone, 28672 x 4096 bf16 41.9 us, 37.6 apart; multiplied, 8 waves, 51.7 / 40.2).
+//  - uncut, up to 16 rows: as many waves a workgroup as share the columns evenly
+//    among the CUs (waves_for).
 // With N columns there are N / 64 workgroups; below 256 of them K is cut so
 // that about 768 result (N = 6144, 40 rows fp8: 8.8 us with 768, 9.7 with
 // 384); from 256 on the second pass costs more than the parts give (28672:
 // 28.2 us whole, 29.8 in two parts).
 // Where a consumer can add the parts itself (skinny_sums; the norm after an
 // attention or feed-forward block, the rotation of q and k) that second pass,
-// about 5 us of launch and drain, is gone.
-// Measured in the decode step, W out of cache, us (library product + what
-// reads it -> this + that):
-//   fp8, 40 rows  4096 -> 6144 and rotation   13.5 + 4.9 ->  9.6 + 6.9
-//                 14336 -> 4096 and norm      23.0 + 5.1 -> 16.4 + 7.4
-//                 4096 -> 4096 and norm       11.8 + 5.1 ->  8.0 + 7.4
-//   bf16, 8 rows  4096 -> 6144 and rotation   15.5 + 4.9 -> 12.1 + 4.8
-//                 14336 -> 4096 and norm      25.6 + 5.2 -> 23.0 + 4.8
-//                 4096 -> 28672               62.9       -> 49.6 (4.7 TB/s)
-//   bf16, 96 rows 14336 -> 4096 and norm      54.1 + 5.5 -> 36.0 + 5.8
+// about 5 us of launch and drain, is gone; so is the activation's launch behind gate
+// and up (skinny_gated).
+// W out of cache, us, with branches and the same first columns -> now:
+//   bf16, 1 row   4096 -> 28672  47.4 -> 41.2 (5.7 TB/s), with silu 49.6 -> 42.0
+//                 4096 -> 6144   12.1 -> 11.5; 4096 -> 4096 9.2 -> 8.6
+//                 14336 -> 4096  24.4 -> 22.5; 2304 -> 18432 23.4 -> 20.3
+//                 4096 -> 128256 200 -> 176
+//   bf16, 96 rows 4096 -> 4096 14.3 -> 14.3; 14336 -> 4096 35.3 -> 35.2
+//   fp8, 8 rows   4096 -> 28672 29.0 -> 24.8; 4096 -> 6144 7.7 -> 7.3; 4096 -> 4096
+//                 5.3 -> 5.4; 14336 -> 4096 15.4 -> 13.4; 2304 -> 18432 16.3 -> 12.5
+//   fp8, 40 rows  4096 -> 6144 9.9 -> 9.8; 4096 -> 4096 7.2 -> 6.7
 // The grouped form multiplies every expert's rows of a mixture in one launch,
-// x rows gathered by index. 8 experts of 4096 x 14336, 40 tokens of 2 experts
-// each, both products with routing and activation: fp8 297 us (4.8 TB/s over
-// the weights), 542 with a library product per expert; bf16 561 and 822.
+// x rows gathered by index. 8 experts, 80 rows, 28672 x 4096 and 4096 x 14336: fp8
+// 184 + 94 us -> 170 + 89 (5.5 and 5.3 TB/s), bf16 359 + 193 -> 320 + 179; 32 experts of
+// 1408 x 2048 bf16 44 -> 40.
 #include <torch/extension.h>
 
 #include <type_traits>
@@ -44,9 +55,12 @@
 
 namespace {
 
-constexpr int kNW = 4;         // waves per workgroup
+constexpr int kNW = 4;         // waves per workgroup (waves_for: of uncut few rows)
 constexpr int kMaxRows = 96;
 constexpr int kMaxParts = 8;
+constexpr int kStep = 256;     // bytes of K a step
+constexpr int kAhead = 3;      // steps of x in LDS and of w in registers
+constexpr int64_t kFarRows = (int64_t)1 << 23;  // bytes
 
 typedef __attribute__((ext_vector_type(8))) short bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -92,31 +106,77 @@ DEV_INLINE void store4(ushort* y, f32x4 v, const float* sx, const float* sw,
   *reinterpret_cast<ushort4_t*>(y) = o;
 }
 
+// 16 bytes a lane from base + voff + soff, zeros past `size` bytes; to registers or
+// to l + 16 * lane in LDS
+DEV_INLINE i32x4 load16(const char* base, int size, int voff, int soff) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const auto r = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, size, 0x00020000);
+  return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+#else
+  return i32x4{};
+#endif
+}
+DEV_INLINE void load_lds16(const char* base, int size, char* l, int voff, int soff) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const auto r = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, size, 0x00020000);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(
+      r, (__attribute__((address_space(3))) uint32_t*)l, 16, voff, soff, 0, 0);
+#endif
+}
+constexpr int kNowhere = 0x7fffffff;  // past the end of every buffer
+
+// own LDS reads are done, all but the last N loads have landed
+template <int N>
+DEV_INLINE void wait_loads() {
+  static_assert(N < 64);
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x70);
+}
+
+// Nothing moves over it, loads neither: x and w are not __restrict__, so the
+// compiler takes the asm to write what they point to. (wait_loads counts them.)
+DEV_INLINE void in_order() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+DEV_INLINE void barrier() {
+  in_order();
+  __builtin_amdgcn_s_barrier();
+  in_order();
+}
+
 // MT: 16-row tiles of x. part != null: raw sums of this K range.
 // GROUPED: blockIdx.z is the expert; its rows are taken MT * 16 at a time (W
 // is read again for each such pass: the host picks MT so that one is usual).
-template <bool FP8, int MT, bool GROUPED>
-__launch_bounds__(kNW * WAVE_SIZE) __global__ void skinny_kernel(
-    ushort* __restrict__ y,         // [M, N]
-    float* __restrict__ part,       // [parts, M, N]
-    const char* __restrict__ x,     // M rows of KB bytes, ldx apart
-    const char* __restrict__ w,     // N rows of KB bytes
-    const float* __restrict__ sx, const float* __restrict__ sw,
-    const ushort* __restrict__ bias, const int M_all, const int N, const int KB,
-    const int64_t ldx, const int k_part, const Groups grp) {
-  constexpr int KC = MT <= 2 ? 512 : 256;  // bytes of K per step
-  constexpr int CH = KC / 64;
-  constexpr int UPR = KC / 16;
-  constexpr int XU = MT * 16 * UPR;
-  constexpr int NX = XU / (kNW * WAVE_SIZE);  // staged units per thread
-  static_assert(XU % (kNW * WAVE_SIZE) == 0, "whole units per thread");
-  __shared__ __attribute__((aligned(16))) char xs[2][MT * 16 * KC];
+// ACT (bf16): silu (1) or tanh-gelu (2) of column n times column n + N / 2, in fp32,
+// rounded once; a wave has 8 columns of either half.
+template <bool FP8, int MT, bool GROUPED, int ACT, int NW>
+__launch_bounds__(NW * WAVE_SIZE) __global__ void skinny_kernel(
+    ushort* y,         // [M, N], ACT: [M, N / 2]
+    float* part,       // [parts, M, N]
+    const char* x,     // M rows of KB bytes, ldx apart
+    const char* w,     // N rows of KB bytes
+    const float* sx, const float* sw, const ushort* bias, const int M_all,
+    const int N, const int KB, const int ldx, const int xbytes, const int k_part,
+    const int parts, const Groups grp) {
+  constexpr int CH = kStep / 64, UPR = kStep / 16;
+  constexpr int RW = ACT ? 8 : 16;             // columns of the result a wave
+  constexpr int NX = (MT * 16 * UPR - 1) / (NW * WAVE_SIZE) + 1, L = NX + CH;  // loads a step
+  constexpr int PLACE = NX * NW * WAVE_SIZE * 16;  // x of a step in LDS
+  static_assert(!GROUPED || PLACE == MT * 16 * kStep);  // (else M <= 16 MT)
+  __shared__ __attribute__((aligned(16))) char xs[kAhead * PLACE];
 
-  const int wave = threadIdx.x / WAVE_SIZE, lane = threadIdx.x % WAVE_SIZE;
-  const int r = lane & 15, kg = lane >> 4;
-  const int n0 = (blockIdx.x * kNW + wave) * 16;
-  const int k0 = blockIdx.y * k_part, k1 = min(KB, k0 + k_part);
-  const int steps = (k1 - k0 + KC - 1) / KC;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
+  const int lane = threadIdx.x % WAVE_SIZE, r = lane & 15, kg = lane >> 4;
+  const int tile = blockIdx.x / parts, of = blockIdx.x % parts;
+  const int cols = ACT ? N / 2 : N;  // of the result
+  const int n0 = (tile * NW + wave) * RW;
+  const int k0 = of * k_part, k1 = min(KB, k0 + k_part);
+  const int steps = (k1 - k0 + kStep - 1) / kStep;
+  // whole rows of 2^n bytes: workgroups that read the same columns of K at a time
+  // wait for the same few of the memory's channels
+  const int first =
+      parts == 1 ? __builtin_amdgcn_readfirstlane((blockIdx.x >> 3) * 3u % (uint32_t)steps) : 0;
   int m0 = 0, M = M_all;  // this pass's first row and the rows from it on
   int m_end = M_all;
   if constexpr (GROUPED) {
@@ -127,104 +187,113 @@ __launch_bounds__(kNW * WAVE_SIZE) __global__ void skinny_kernel(
     M = m_end - m0;
     if (M <= 0) return;  // whole workgroup
   }
-  const char* wp = w + (int64_t)min(n0 + r, N - 1) * KB + kg * 16;
+  const char* wb = w + (int64_t)n0 * KB;
+  const int left = max(0, min(cols - n0, RW));  // rows of w
+  const int wbytes = left == 0 ? 0 : (ACT ? cols + left : left) * KB;
+  // lane's offsets; xk: within a row's step
+  const int wo = (ACT ? (r & 7) + (r >> 3) * cols : r) * KB + kg * 16;
+  int xo[NX], xk[NX];
 
   f32x4 acc[MT];
-  i32x4 wf[2][CH], xr[NX];
-  int64_t x_off[NX];  // of the staged units' rows
-
-  // loads past the end of the range read its last bytes again; their
-  // products are skipped
-  auto load_w = [&](int b, int s) {
-#pragma unroll
-    for (int c = 0; c < CH; ++c)
-      wf[b][c] = *reinterpret_cast<const i32x4*>(
-          wp + min(k0 + s * KC + c * 64, k1 - 64));
-  };
-  auto load_x = [&](int s) {
-#pragma unroll
-    for (int i = 0; i < NX; ++i) {
-      const int u = threadIdx.x + i * kNW * WAVE_SIZE;
-      xr[i] = *reinterpret_cast<const i32x4*>(
-          x + x_off[i] + min(k0 + s * KC + u % UPR * 16, k1 - 16));
-    }
-  };
-  auto put_x = [&](int b) {
-#pragma unroll
-    for (int i = 0; i < NX; ++i) {
-      const int u = threadIdx.x + i * kNW * WAVE_SIZE;
-      const int row = u / UPR;
-      *reinterpret_cast<i32x4*>(
-          &xs[b][row * KC + (((u % UPR) ^ (row & 7)) << 4)]) = xr[i];
-    }
-  };
-  auto multiply = [&](int b, int s) {
-#pragma unroll
-    for (int c = 0; c < CH; ++c)
-      if (k0 + s * KC + c * 64 < k1)
-#pragma unroll
-        for (int j = 0; j < MT; ++j) {
-          if (GROUPED && j * 16 >= M) break;  // the same in every lane
-          const i32x4 xf = *reinterpret_cast<const i32x4*>(
-              &xs[b][(j * 16 + r) * KC + (((c * 4 + kg) ^ (r & 7)) << 4)]);
-          acc[j] = mfma_64b<FP8>(wf[b][c], xf, acc[j]);
-        }
-  };
-
+  i32x4 wf[kAhead][CH];
   do {
 #pragma unroll
     for (int j = 0; j < MT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < NX; ++i) {
-      int row = min((threadIdx.x + i * kNW * WAVE_SIZE) / UPR, (unsigned)M - 1);
-      if constexpr (GROUPED) {
-        row += m0;
-        if (grp.src) row = grp.src[row];
-      }
-      x_off[i] = (int64_t)row * ldx;
-    }
-    load_x(0);
-    load_w(0, 0);
-    put_x(0);
-    if (steps > 1) load_x(1);
-    __syncthreads();
-    for (int s = 0; s < steps; s += 2) {
-      if (s + 1 < steps) {
-        load_w(1, s + 1);
-        put_x(1);
-        if (s + 2 < steps) load_x(s + 2);
-      }
-      multiply(0, s);
-      __syncthreads();
-      if (s + 1 < steps) {
-        if (s + 2 < steps) {
-          load_w(0, s + 2);
-          put_x(0);
-          if (s + 3 < steps) load_x(s + 3);
+      // 16-byte unit u of row r lies at u ^ (r & 7): made by the choice of source
+      const int at = (wave * NX + i) * WAVE_SIZE + lane, row = at / UPR;
+      xk[i] = ((at % UPR) ^ (row & 7)) * 16;
+      xo[i] = kNowhere;
+      if (row < M) {
+        int from = m0 + row;
+        if constexpr (GROUPED) {
+          if (grp.src) from = grp.src[from];
         }
-        multiply(1, s + 1);
-        __syncthreads();
+        xo[i] = from * ldx + xk[i];
       }
     }
-
-    // accumulator: row (W) 4 kg + e, column (x) r
-    const int n = n0 + kg * 4;
-    if (n < N) {  // N is a multiple of 4
+    int next = first, ahead = 0;  // the step to load and the number loaded
+    auto load = [&](auto place) {
+      constexpr int P = decltype(place)::value;
+      const int k = k0 + next * kStep, on = ahead < steps;
 #pragma unroll
-      for (int j = 0; j < MT; ++j) {
-        const int m = j * 16 + r;
-        if (m >= M) continue;
-        if (part)
-          *reinterpret_cast<f32x4*>(
-              part + ((int64_t)blockIdx.y * M_all + m) * N + n) = acc[j];
-        else
-          store4(y + (int64_t)(m0 + m) * N + n, acc[j], sx, sw, bias,
-                 GROUPED && grp.src ? grp.src[m0 + m] : m0 + m, n);
+      for (int i = 0; i < NX; ++i)
+        load_lds16(x, on ? xbytes : 0, xs + P * PLACE + (wave * NX + i) * 1024,
+                   xk[i] < k1 - k ? xo[i] : kNowhere, k);
+#pragma unroll
+      for (int c = 0; c < CH; ++c)
+        wf[P][c] = load16(wb, on && k + c * 64 < k1 ? wbytes : 0, wo + c * 64, k);
+      next = next + 1 == steps ? 0 : next + 1;
+      ++ahead;
+    };
+    // one step: its loads have landed everywhere, and everyone is done with the
+    // step before it, whose place the next loads take
+    auto step = [&](auto place, auto behind, auto more) {
+      constexpr int P = decltype(place)::value;
+      in_order();
+      wait_loads<decltype(behind)::value * L>();  // so many steps are loaded behind this one
+      barrier();
+      if constexpr (decltype(more)::value) {
+        load(std::integral_constant<int, (P + kAhead - 1) % kAhead>{});
+        in_order();
       }
+#pragma unroll
+      for (int c = 0; c < CH; ++c)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+          if (GROUPED && j * 16 >= M) break;  // the same in every lane
+          const i32x4 xf = *reinterpret_cast<const i32x4*>(
+              xs + P * PLACE + (j * 16 + r) * kStep + (((c * 4 + kg) ^ (r & 7)) << 4));
+          acc[j] = mfma_64b<FP8>(wf[P][c], xf, acc[j]);
+        }
+    };
+    static_assert(kAhead == 3);
+    constexpr std::integral_constant<int, 0> zero;
+    constexpr std::integral_constant<int, 1> one;
+    constexpr std::integral_constant<int, 2> two;
+    in_order();
+    load(zero);
+    in_order();  // wait_loads counts on it
+    load(one);
+    // (a loop that is left in its middle has the compiler wait for all loads)
+    for (int s = steps; s >= kAhead; s -= kAhead) {
+      step(zero, one, one);
+      step(one, one, one);
+      step(two, one, one);
+    }
+    if (steps % kAhead > 0) step(zero, one, zero);
+    if (steps % kAhead > 1) step(one, zero, zero);
+    wait_loads<0>();  // (the last ones, of nothing, write LDS too)
+
+    // accumulator: row (W) 4 kg + e, column (x) r; with ACT the lanes from 32 on have
+    // the other half's
+    const int n = n0 + kg * 4;
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+      f32x4 v = acc[j];
+      if constexpr (ACT != 0) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float up = __shfl_xor(v[e], 32);
+          float z = v[e];  // gelu: 0.5 (1 + tanh y) = 1 / (1 + e^-2y)
+          if constexpr (ACT == 2) z = 1.5957691216057308f * (z + 0.044715f * z * z * z);
+          v[e] = v[e] / (1.0f + __expf(-z)) * up;
+        }
+        if (kg >= 2) continue;
+      }
+      const int m = j * 16 + r;
+      if (m >= M || n >= cols) continue;  // (cols: a multiple of 4)
+      if (part)
+        *reinterpret_cast<f32x4*>(part + ((int64_t)of * M_all + m) * N + n) = v;
+      else
+        store4(y + (int64_t)(m0 + m) * cols + n, v, sx, sw, bias,
+               GROUPED && grp.src ? grp.src[m0 + m] : m0 + m, n);
     }
     if constexpr (GROUPED) {
       m0 += MT * 16;
       M = m_end - m0;
+      if (M > 0) barrier();  // everyone has read the last step
     }
   } while (GROUPED && M > 0);
 }
@@ -262,6 +331,11 @@ struct Shape {
   bool fp8;
 };
 
+// Offsets are 32 bits: rows under 8 MB apart (others are copied).
+torch::Tensor near_rows(const torch::Tensor& x) {
+  return x.dim() == 2 && x.stride(0) * x.element_size() >= kFarRows ? x.contiguous() : x;
+}
+
 Shape check(const torch::Tensor& x, const torch::Tensor& w,
             const c10::optional<torch::Tensor>& sx,
             const c10::optional<torch::Tensor>& sw,
@@ -275,7 +349,7 @@ Shape check(const torch::Tensor& x, const torch::Tensor& w,
   const int es = fp8 ? 1 : 2;
   const Shape s{(int)x.size(0), (int)w.size(0), (int)w.size(1) * es, fp8};
   TORCH_CHECK(s.M >= 1 && s.M <= kMaxRows, "1 to 96 rows");
-  TORCH_CHECK(s.KB >= 64 && s.KB % 64 == 0 && s.N % 4 == 0 &&
+  TORCH_CHECK(s.KB >= 64 && s.KB % 64 == 0 && s.KB < kFarRows && s.N % 4 == 0 &&
               (int64_t)s.M * s.N < (1ll << 31));
   TORCH_CHECK(x.stride(0) * es % 16 == 0 && x.stride(0) >= x.size(1) &&
               ((uintptr_t)x.data_ptr() & 15) == 0 &&
@@ -294,26 +368,64 @@ Shape check(const torch::Tensor& x, const torch::Tensor& w,
   return s;
 }
 
+// Waves of a workgroup of a whole product of up to 16 rows: those with which the CUs
+// have the most even share of the columns' tiles, as many as possible, which share
+// x. us at one row, bf16, 2 / 4 / 8 waves: 28672 x 4096
+// 45.6 / 43.1 / 41.1, 24576 x 4096 35.7 / 42.1 / 37.9, 18432 x 2304 20.3 / 24.5 / 22.5,
+// 16384 x 4096 25.3 / 25.0 / 40.0, 53248 x 4096 83.1 / 87.8 / 86.9.
+int waves_for(int N) {
+  int best = 8, most = 1 << 30;
+  for (int nw = 8; nw >= 2; nw /= 2) {
+    const int wgs = (N + nw * 16 - 1) / (nw * 16), on_one = (wgs + 255) / 256 * nw;
+    if (on_one < most) {
+      best = nw;
+      most = on_one;
+    }
+  }
+  return best;
+}
+
 void launch(ushort* y, float* part, const torch::Tensor& x,
             const torch::Tensor& w, const float* sx, const float* sw,
-            const ushort* bias, const Shape& s, const Cut& cut) {
-  const dim3 grid((s.N + kNW * 16 - 1) / (kNW * 16), cut.parts);
-  const int64_t ldx = x.stride(0) * x.element_size();
+            const ushort* bias, const Shape& s, const Cut& cut, int act = 0) {
+  const int nw = s.M <= 16 && cut.parts == 1 ? waves_for(s.N) : kNW;
+  const dim3 grid((s.N + nw * 16 - 1) / (nw * 16) * cut.parts);
+  const int ldx = x.stride(0) * x.element_size();
+  const int xbytes = (s.M - 1) * ldx + s.KB;
   auto stream = c10::hip::getCurrentHIPStream().stream();
-  auto go = [&](auto fp8, auto mt) {
-    hipLaunchKernelGGL((skinny_kernel<decltype(fp8)::value, decltype(mt)::value, false>),
-                       grid, dim3(kNW * WAVE_SIZE), 0, stream, y, part,
+  auto go = [&](auto fp8, auto mt, auto a, auto waves) {
+    constexpr int NW = decltype(waves)::value;
+    hipLaunchKernelGGL((skinny_kernel<decltype(fp8)::value, decltype(mt)::value, false,
+                                      decltype(a)::value, NW>),
+                       grid, dim3(NW * WAVE_SIZE), 0, stream, y, part,
                        (const char*)x.data_ptr(), (const char*)w.data_ptr(),
-                       sx, sw, bias, s.M, s.N, s.KB, ldx, cut.k_part, Groups{});
+                       sx, sw, bias, s.M, s.N, s.KB, ldx, xbytes, cut.k_part, cut.parts,
+                       Groups{});
   };
+  constexpr std::integral_constant<int, 0> none;
+  constexpr std::integral_constant<int, 1> one;
+  constexpr std::integral_constant<int, 2> two;
+  constexpr std::integral_constant<int, kNW> four;
+  constexpr std::integral_constant<int, 8> eight;
+  auto few = [&](auto fp8, auto a) {
+    if (nw == 8) go(fp8, one, a, eight);
+    else if (nw == 4) go(fp8, one, a, four);
+    else go(fp8, one, a, two);
+  };
+  if (act) {
+    if (act == 1) few(std::false_type{}, one);
+    else few(std::false_type{}, two);
+    HIP_CHECK_KERNEL();
+    return;
+  }
   auto tiles = [&](auto fp8) {
     switch ((s.M + 15) / 16) {
-      case 1: go(fp8, std::integral_constant<int, 1>{}); break;
-      case 2: go(fp8, std::integral_constant<int, 2>{}); break;
-      case 3: go(fp8, std::integral_constant<int, 3>{}); break;
-      case 4: go(fp8, std::integral_constant<int, 4>{}); break;
-      case 5: go(fp8, std::integral_constant<int, 5>{}); break;
-      default: go(fp8, std::integral_constant<int, 6>{}); break;
+      case 1: few(fp8, none); break;
+      case 2: go(fp8, two, none, four); break;
+      case 3: go(fp8, std::integral_constant<int, 3>{}, none, four); break;
+      case 4: go(fp8, four, none, four); break;
+      case 5: go(fp8, std::integral_constant<int, 5>{}, none, four); break;
+      default: go(fp8, std::integral_constant<int, 6>{}, none, four); break;
     }
   };
   if (s.fp8) tiles(std::true_type{});
@@ -328,6 +440,7 @@ void skinny_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                    c10::optional<torch::Tensor> sx,
                    c10::optional<torch::Tensor> sw,
                    c10::optional<torch::Tensor> bias) {
+  x = near_rows(x);
   const Shape s = check(x, w, sx, sw, bias);
   TORCH_CHECK(y.scalar_type() == torch::kBFloat16 && y.is_contiguous() &&
               y.is_cuda() && y.dim() == 2 && y.size(0) == s.M && y.size(1) == s.N);
@@ -352,11 +465,26 @@ void skinny_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
 // parts itself (and applies an fp8 product's scales)
 torch::Tensor skinny_sums(torch::Tensor x, torch::Tensor w) {
   c10::optional<torch::Tensor> none;
+  x = near_rows(x);
   const Shape s = check(x, w, none, none, none, true);
   const Cut cut = cut_for(s.N, s.KB);
   auto part = torch::empty({cut.parts, s.M, s.N}, x.options().dtype(torch::kFloat32));
   launch(nullptr, part.data_ptr<float>(), x, w, nullptr, nullptr, nullptr, s, cut);
   return part;
+}
+
+// y [M, N / 2] = silu (act 1) or tanh-gelu (act 2) of the first N / 2 columns of x w^T
+// times the others; bf16, up to 16 rows
+void skinny_gated(torch::Tensor y, torch::Tensor x, torch::Tensor w, int64_t act) {
+  c10::optional<torch::Tensor> none;
+  x = near_rows(x);
+  const Shape s = check(x, w, none, none, none);
+  TORCH_CHECK(!s.fp8 && s.M <= 16 && s.N % 8 == 0 && (act == 1 || act == 2));
+  TORCH_CHECK((int64_t)s.N * s.KB < (1ll << 31), "gate and up columns");
+  TORCH_CHECK(y.scalar_type() == torch::kBFloat16 && y.is_contiguous() &&
+              y.is_cuda() && y.dim() == 2 && y.size(0) == s.M && y.size(1) == s.N / 2);
+  launch((ushort*)y.data_ptr(), nullptr, x, w, nullptr, nullptr, nullptr, s, {1, s.KB},
+         (int)act);
 }
 
 // y[i] = x[src[i]] w[e]^T for the rows i of expert e, scaled as above; w
@@ -373,7 +501,8 @@ void skinny_experts(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   TORCH_CHECK(x.stride(1) == 1 && w.is_contiguous());
   const int es = fp8 ? 1 : 2;
   const int E = w.size(0), N = w.size(1), KB = (int)w.size(2) * es;
-  TORCH_CHECK(KB >= 64 && KB % 64 == 0 && N % 4 == 0 && E >= 1 && E <= 65535);
+  TORCH_CHECK(KB >= 64 && KB % 64 == 0 && KB < kFarRows && N % 4 == 0 && E >= 1 &&
+              E <= 65535);
   TORCH_CHECK(x.stride(0) * es % 16 == 0 && x.stride(0) >= x.size(1) &&
               ((uintptr_t)x.data_ptr() & 15) == 0 &&
               ((uintptr_t)w.data_ptr() & 15) == 0,
@@ -397,19 +526,28 @@ void skinny_experts(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   }
   const int R = y.size(0);
   if (R == 0) return;
+  if (x.size(0) * x.stride(0) * es >= (1ll << 31)) {  // offsets are 32 bits
+    if (src.has_value()) {
+      if (fp8) sx = sx->reshape(-1).index_select(0, *src);
+      x = x.view(torch::kUInt8).index_select(0, *src).view(x.scalar_type());
+      src = c10::nullopt;
+    }
+    x = x.contiguous();
+    TORCH_CHECK(x.numel() * es < (1ll << 31));
+  }
   const float* sxp = fp8 ? sx->data_ptr<float>() : nullptr;
   const float* swp = fp8 ? sw->data_ptr<float>() : nullptr;
   const Groups g{begin.data_ptr<int32_t>(),
                  src.has_value() ? src->data_ptr<int32_t>() : nullptr};
   const dim3 grid((N + kNW * 16 - 1) / (kNW * 16), 1, E);
-  const int64_t ldx = x.stride(0) * es;
+  const int ldx = x.stride(0) * es, xbytes = (x.size(0) - 1) * ldx + KB;
   auto stream = c10::hip::getCurrentHIPStream().stream();
   auto go = [&](auto f, auto mt) {
-    hipLaunchKernelGGL((skinny_kernel<decltype(f)::value, decltype(mt)::value, true>),
+    hipLaunchKernelGGL((skinny_kernel<decltype(f)::value, decltype(mt)::value, true, 0, kNW>),
                        grid, dim3(kNW * WAVE_SIZE), 0, stream,
                        (ushort*)y.data_ptr(), nullptr, (const char*)x.data_ptr(),
                        (const char*)w.data_ptr(), sxp, swp, nullptr, R, N, KB,
-                       ldx, KB, g);
+                       ldx, xbytes, KB, 1, g);
   };
   // rows per expert if they are spread evenly; half as many again fit a pass
   const int mean = (R + E - 1) / E;

@@ -233,14 +233,22 @@ __global__ __launch_bounds__(256, 1) void tiled_kernel(const Args a) {
   const char* wb = a.w + work.expert * a.ew + n0 * a.ldw;
   const int xn = a.src ? (int)a.xbytes : (rows - 1) * (int)a.ldx + a.KB;
   const int wn_ = ((kHalves ? N - n0 : min(N - n0, BN)) - 1) * (int)a.ldw + a.KB;
+  // One row tile: the workgroups begin at columns of K apart. At the same ones of
+  // rows of 2^n bytes they wait for the same few of the memory's channels (us, weights
+  // out of cache, all at the first / apart: fp8 28672 x 4096 40 rows 32.0 / 25.9, 65536
+  // x 8192 121 / 101, 128256 x 4096 117 / 108; bf16 28672 x 4096 40 rows 53.6 / 45.5;
+  // 36864 x 4608 47.3 / 47.3). With more row tiles they would lose what they share.
+  const int first = !a.bounds && a.R <= BM && a.k_part == a.KB
+                        ? (int)((blockIdx.x >> 3) * 2u % (uint32_t)steps) : 0;
+  auto column = [&](int s) { return k0 + (s + first < steps ? s + first : s + first - steps) * kStep; };
   // load l of a batch: the AC of step sa of x, then the BC of step sb of w
   auto load = [&](int l, int pa, int sa, int pb, int sb) {
     if (l < AC) {
       load_lds16(xb, sa < steps ? xn : 0, lds + pa * SA + (wave * AC + l) * 1024, ao[l],
-                 k0 + sa * kStep);
+                 column(sa));
     } else {
       load_lds16(wb, sb < steps ? wn_ : 0, lds + NA * SA + pb * SB + (wave * BC + l - AC) * 1024,
-                 bo[l - AC], k0 + sb * kStep);
+                 bo[l - AC], column(sb));
     }
   };
 

@@ -276,11 +276,11 @@ class MLP(nn.Module):
         )
         a = None
         if not (
-            lora_live or x.dim() != 2 or x.shape[0] <= 96
+            lora_live or x.dim() != 2
             or type(self.gate_up_proj) is not EngineLinear or _hooked(self.gate_up_proj)
             or self.gate_up_proj.bias is not None
         ):
-            a = ops.tiled_gated(x, self.gate_up_proj.weight, gelu=self.gelu)
+            a = ops.gated(x, self.gate_up_proj.weight, gelu=self.gelu)
         if a is None:
             h = self.gate_up_proj(x)
             if lora_live:

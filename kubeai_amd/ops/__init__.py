@@ -288,6 +288,7 @@ def _skinny_operands(x, weight) -> bool:
         # (the library refuses fp8 columns that are no multiple of 16)
         and weight.shape[0] % (8 if x.dtype == torch.bfloat16 else 16) == 0
         and weight.shape[1] * weight.element_size() % 64 == 0
+        and weight.shape[1] * weight.element_size() < 2**23
         and weight.device == x.device
         and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
         and x.data_ptr() % 16 == weight.data_ptr() % 16 == 0
@@ -362,19 +363,38 @@ def sums_better(
     return N <= 4096 if M <= 32 else N >= 2048
 
 
+def _even_rows(K: int, fp8: bool) -> bool:
+    """Whether weight rows lie whole 4 KB apart: the same columns of all of them are
+    then the same few channels of the memory. Kernels that begin at columns apart
+    (csrc/skinny_gemm.hip, csrc/tiled_gemm.h) lose less to that than the library's."""
+    return K * (1 if fp8 else 2) % 4096 == 0
+
+
+def _few_rows_better(M: int, N: int, K: int, fp8: bool) -> bool:
+    """Whether the weight-streaming product, uncut, beats the library's: up to 16 rows
+    and a width that fills the chip (us, weights out of cache, library / this, 8 rows):
+    bf16 4096 -> 28672 60.6 / 41.5, 4096 -> 16384 32.1 / 23.7, 4096 -> 128256 183 / 173,
+    8192 -> 57344 172 / 158, 2304 -> 87808 136 / 80; but 1792 -> 56320 38.6 / 39.8, 2304 ->
+    256000 207 / 218, 7680 -> 14848 45 / 52; fp8 4096 -> 28672 31.7 / 23.6, 8192 -> 16384 51
+    / 24, 4096 -> 128256 112 / 94, 6656 -> 9216 38 / 19, but 8192 -> 8192 at 16 rows 16.4 /
+    21.3, 9472 -> 59648 102 / 110, 1536 -> 116992 39 / 41. Not for rows under 256 bytes
+    (128 -> 65536 fp8 5.6 / 6.7). Over 308 products the 200 chosen take 0.74 of the time,
+    1.10 at worst."""
+    if M > 16 or K * (1 if fp8 else 2) < 256:
+        return False
+    if N >= 16384 and _even_rows(K, fp8):
+        return True
+    if fp8:
+        return M <= 12 if 8192 <= N < 16384 else N >= 16384 and (N <= 40000 or K <= 1024)
+    return 16384 <= N <= 40000 or 65536 <= N < 200000
+
+
 def _streams_better(M: int, N: int, K: int, fp8: bool) -> bool:
-    """Whether the weight-streaming product beats the library's where it has to
-    add its parts itself. Few rows and a width that fills the chip uncut (us,
-    weights out of cache, library / this, 8 rows): bf16 4096 -> 28672 59.9 / 47.6,
-    2304 -> 18432 50.8 / 25.2, 2048 -> 32256 34.5 / 31.4, 4096 -> 65536 123 / 107,
-    but 4096 -> 16384 33.4 / 34.8, 8192 -> 24576 83.8 / 91.8, 6144 -> 24576 at 16
-    rows 68.5 / 73.8; fp8 4096 -> 16384 27.9 / 20.3, 4096 -> 28672 33.8 / 28.0,
-    8192 -> 30720 65 / 58; beyond two passes of workgroups over the chip only
-    whole passes (8192 -> 36864 fp8 72 / 81), and not for rows under 256 bytes (128
-    -> 65536 fp8 5.6 / 6.7). At 32 rows 53.5 / 53.4 and 21 / 30, at 128256 columns
-    192 / 198. Very long rows, which the library does not cut: 32256 -> 2048 83 /
-    38 at 8 rows, 127 / 60 at 96; it does at 16384 (-> 1024 20.4 / 19.4 at 8 rows,
-    21.0 / 28.7 at 48; fp8 20.2 / 12.9, 20.1 / 21.4 at 96)."""
+    """Whether the weight-streaming product beats the library's for the length of its
+    rows: very long ones, which the library does not cut (us, library / this): 32256 ->
+    2048 83 / 32 at 8 rows, 127 / 52 at 96; it does at 16384 (-> 1024 20.4 / 16.5 at 8
+    rows, 21.0 / 19 at 48; fp8 20.2 / 11, 20.1 / 15 at 96). And up to 16 rows, uncut, by a
+    rule for where it gains much; _few_rows_better has more of them."""
     if K >= 8 * N and K >= 16384:
         return K > 16384 or M <= (64 if fp8 else 32)
     if M > 16 or N > 65536 or (N > 32768 and N % 16384) or K * (1 if fp8 else 2) < 256:
@@ -382,6 +402,10 @@ def _streams_better(M: int, N: int, K: int, fp8: bool) -> bool:
     if fp8:
         return N >= 16384 and K <= 8192
     return N >= 16384 and K <= 1024 or N > 16384 and K <= (6144 if M <= 8 else 4096)
+
+
+def _streams(M: int, N: int, K: int, fp8: bool) -> bool:
+    return _few_rows_better(M, N, K, fp8) or _streams_better(M, N, K, fp8)
 
 
 def _tiled_operands(x, weight) -> bool:
@@ -435,9 +459,21 @@ def _tiled_better(M: int, N: int, K: int, fp8: bool) -> bool:
     20000) the chosen ones take 0.77 of the library's time, 1.05 at worst. Logits: 128256 x
     4096 fp8 40 rows 129 / 107, 96 rows 121 / 118, bf16 40 rows 203 / 192, 160
     rows 246 / 213, 384 rows 437 / 339, 1024 rows 853 / 838; 57344 x 8192 fp8 40 rows
-    121 / 103; over 68 others 0.85, in bf16 above 200 rows 0.82 to 1.10. Other bf16 products stay (28672 x 4096 2048 rows 333 / 391)."""
+    126 / 90; over 68 others 0.85, in bf16 above 200 rows 0.82 to 1.10. 17 to
+    96 rows beside 24576 columns and more of even rows (fp8 28672 x 4096 40 rows 31.6 / 25.7,
+    96 rows 33.1 / 28.9; bf16 57.1 / 45.4 and 58.8 / 49.6, but 57344 x 8192 173 / 163, 16384
+    x 4096 34.8 / 40.5), fp8 of others where the library's tiles do not fill (22016 x 1280 36
+    rows 13.4 / 11.3, 58368 x 2560 43.6 / 34.4, but 35840 x 2048 20.9 / 23.9), bf16 beside
+    65536 columns (96256 x 2304 94 / 86): over 348 products the 152 chosen take 0.83, 1.07
+    at worst. Other bf16 products stay (28672 x 4096 2048 rows 333 / 391)."""
+    if 16 < M <= 96 and N >= 24576 and _even_rows(K, fp8) and (fp8 or K <= 4096):
+        return True
     if N >= 49152 and K >= 2048:
         return M > 16 and (fp8 or M <= 1024 and N >= 98304)
+    if 16 < M <= 96:
+        if fp8:
+            return 18432 <= N < 32768 or N >= 45056 and K >= 1024
+        return 65536 <= N < 200000 and K <= 4096
     tiles = -(-M // 64) * -(-N // 128)
     if K > 16384:
         return fp8 and M > 96 and tiles >= 64
@@ -484,6 +520,30 @@ def tiled_gated(x, weight, gelu=False):
     ):
         return None
     return _tiled_linear(x, weight, act=2 if gelu else 1)
+
+
+def gated(x, weight, gelu=False):
+    """What tiled_gated computes, also up to 96 rows: by the weight-streaming kernel or
+    the tiled one where linear has the product from them (28672 x 4096 one row: product
+    41.2 us, this 42.0, the activation's launch 4.7); None where two launches are
+    faster."""
+    (M, K), N = x.shape, weight.shape[0]
+    if M > 96:
+        return tiled_gated(x, weight, gelu)
+    if x.dtype != torch.bfloat16 or weight.dim() != 2 or N * K * 2 >= 2**31:
+        return None
+    if (
+        N >= 8192
+        and _few_rows_better(M, N, K, fp8=False)
+        and not observed(x, weight)
+        and _skinny_operands(x, weight)
+    ):
+        y = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
+        _C.skinny_gated(y, x, weight, 2 if gelu else 1)
+        return y
+    if _tiled_better(M, N, K, fp8=False) and _tiled_operands(x, weight):
+        return _tiled_linear(x, weight, act=2 if gelu else 1)
+    return None
 
 
 #: Products of more rows are not handed on as sums: whole ones fill the chip.
@@ -577,7 +637,7 @@ def linear(x, weight):
         x.dim() == weight.dim() == 2
         and x.shape[0] <= 96
         and x.is_cuda
-        and _streams_better(x.shape[0], *weight.shape, fp8=False)
+        and _streams(x.shape[0], *weight.shape, fp8=False)
         and x.dtype == torch.bfloat16
         and not observed(x, weight)
         and _skinny_operands(x, weight)
@@ -603,7 +663,7 @@ def linear_fp8(xq, x_scale, weight, w_scale, bias=None, out=None):
     [N, K] e4m3, x_scale [M], w_scale [1, N]; into `out` (dense rows) if given."""
     if (
         xq.shape[0] <= 96
-        and _streams_better(xq.shape[0], *weight.shape, fp8=True)
+        and _streams(xq.shape[0], *weight.shape, fp8=True)
         and _skinny_operands(xq, weight)
         and (out is None or out.is_contiguous())
     ):
