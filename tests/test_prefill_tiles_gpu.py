@@ -134,3 +134,27 @@ def test_keys_that_are_not_finite(hd, softcap):
         torch.testing.assert_close(got, want, atol=bound, rtol=2 * 2.0 ** -9, equal_nan=True)
     else:  # an infinite score outweighs all others or is outweighed
         assert torch.equal(got.isnan(), want.isnan())
+
+
+@pytest.mark.parametrize("window", [0, 50])
+@pytest.mark.parametrize("n,ctx", [(1, 0), (33, 31), (64, 0), (97, 100), (200, 17)])
+def test_maxima_that_grow_with_every_tile(n, ctx, window):
+    """Head size 256, the sums rescaled in most iterations: each key's score is above
+    the last one's, by 2^4 a tile of 32 keys. Odd and even numbers of tiles; windows
+    that begin behind a wave's first tiles."""
+    torch.manual_seed(n)
+    total, hd = n + ctx, 256
+    kc = torch.zeros((total + 15) // 16 + 1, 2, 16, hd, device=DEV, dtype=torch.bfloat16)
+    vc = torch.randn_like(kc)
+    at = torch.arange(total, device=DEV)
+    kc[at // 16 + 1, :, at % 16, 0] = (at // 4 * 0.35)[:, None].bfloat16()
+    bt = torch.arange(1, kc.shape[0], device=DEV, dtype=torch.int32)[None]
+    q = torch.randn(n, 2, hd, device=DEV, dtype=torch.bfloat16)
+    q[:, :, 0] = 1.0
+    start = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    lens = torch.tensor([total], dtype=torch.int32, device=DEV)
+    got = ops.paged_attention_prefill(q, kc, vc, bt, start, lens, 1.0, window=window)
+    want = ref.paged_attention_prefill(q.float(), kc.float(), vc.float(), bt, start, lens, 1.0,
+                                       window=window)
+    torch.testing.assert_close(got.float(), want, rtol=2 * 2.0 ** -9,
+                               atol=2 * 2.0 ** -9 * vc.float().abs().max().item())
