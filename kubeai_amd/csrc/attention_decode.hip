@@ -20,20 +20,22 @@
 //    part that would be 0 is 2^-100 (or the weight, if that is less): times an
 //    infinite value 0 would be NaN.
 //  - the next tile's K and V are in flight while this one is computed (two
-//    register sets).
+//    register sets), and the blocks of the one after it are being looked up. Past the
+//    last tile the loads are of no bytes: in a branch they had the compiler wait, in
+//    front of each tile, for the next one's loads as well (96 rows of 1500-4000 228 us).
 // Bound by reading the cache. The form before this (scores and weighted sum
 // on the vector ALUs) issued about 150 LDS operations per 16 keys, most of
 // them the lane permutes that passed a weight to every lane; here it is 12.
 // Measured, kernel + merge of the splits, us (before -> this):
 //   heads 32/8 x 128, 40 rows of 100-700 keys         41 ->  23
-//   96 rows of 1500-4000                             364 -> 228 (5.0 TB/s)
-//   64 rows of 1536                                  137 ->  80 (5.1 TB/s)
-//     the same, e5m2 cache                           128 ->  51
+//   96 rows of 1500-4000                             364 -> 205 (5.4 TB/s; in 2 splits 208)
+//   64 rows of 1536                                  137 ->  74 (5.4 TB/s)
+//     the same, e5m2 cache                           128 ->  45
 //   8 rows of 3584                                    48 ->  31
 //   1 row of 3000 and 7 idle ones                     32 ->  14
 //   heads 64/8 x 128, 32 rows of 1000-3000           165 ->  60
-//   heads 8/4 x 256, cap, 40 rows of 100-700          42 ->  22
-//     96 rows of 2000, no cap                         222 -> 143
+//   heads 8/4 x 256, cap, 40 rows of 100-700          42 ->  20
+//     96 rows of 2000, no cap                         222 -> 140
 //   heads 4/4 x 256, 96 rows of 2000                  188 -> 142
 // At head size 256 a tile is one block (two would need 512 registers), and over
 // a bf16 cache the query lies in LDS: with it in registers 25 were spilled, and
@@ -57,6 +59,28 @@ typedef __attribute__((ext_vector_type(4))) short bf16x4;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
 
+// 16 (or 8) bytes a lane from base + at, zeros if size is 0
+template <typename T>
+DEV_INLINE T buffer_load(const void* base, int size, int at) {
+  T v{};
+#ifdef __HIP_DEVICE_COMPILE__
+  const auto r = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, size, 0x00020000);
+  if constexpr (sizeof(T) == 16)
+    v = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0));
+  else
+    v = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, at, 0, 0));
+#endif
+  return v;
+}
+
+// no load moves over it: the caches are not __restrict__, so the compiler takes the
+// asm to write them
+DEV_INLINE void in_order() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 // combine a value over the four 16-lane groups that hold the same column
 template <typename F>
 DEV_INLINE float over_groups(float v, F&& f) {
@@ -70,13 +94,13 @@ DEV_INLINE float over_groups(float v, F&& f) {
 
 // CT = cache element type: ushort (bf16) or unsigned char (fp8 e5m2,
 // converted to bf16 on the way in, exactly). CAP: s = cap * tanh(s / cap)
-// after scaling and before masking.
-template <int HD, typename CT, bool CAP>
+// after scaling and before masking. ONE: no wave has more than one tile.
+template <int HD, typename CT, bool CAP, bool ONE>
 __launch_bounds__(kBlockThreads, 2) __global__ void paged_decode_kernel(
     ushort* __restrict__ out,            // [B, n_q, hd] bf16
     const ushort* __restrict__ q,        // [B, n_q, hd] bf16
-    const CT* __restrict__ k_cache,      // [nb, n_kv, bs, hd]
-    const CT* __restrict__ v_cache,
+    const CT* k_cache,                   // [nb, n_kv, bs, hd]
+    const CT* v_cache,
     const int32_t* __restrict__ block_tables,  // [B, max_blocks]
     const int32_t* __restrict__ seq_lens,      // [B]
     const float scale, const float softcap, const int window,
@@ -157,20 +181,33 @@ __launch_bounds__(kBlockThreads, 2) __global__ void paged_decode_kernel(
     if constexpr (sizeof(CT) == 2) return u;
     else return __builtin_bit_cast(bf16x8, e5m2x8_to_bf16x8(u));
   };
-  auto load_tile = [&](int set, int t) {
+  // the cache blocks of tile t (past the last one: that again)
+  struct Blocks {
+    int at[NB];
+  };
+  auto look_up = [&](int t) {
+    Blocks o;
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+      o.at[j] = bt[min(blk_base + t * NB + j, n_blocks - 1)];
+    return o;
+  };
+  constexpr int kBlockBytes = kBS * HD * sizeof(CT);
+  const int k_at = (col * HD + grp * 8) * sizeof(CT), v_at = lane * 8 * sizeof(CT);
+  // a tile behind the last one: loads of no bytes
+  auto load_tile = [&](int set, int t, const Blocks& blocks) {
+    const int size = t < t_hi ? kBlockBytes : 0;
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-      const int64_t blk = bt[min(blk_base + t * NB + j, n_blocks - 1)];
-      const int64_t base = (blk * n_kv + kh) * (kBS * HD);
-      const CT* kp = k_cache + base + col * HD + grp * 8;
-      const CT* vp = v_cache + base + lane * 8;
+      const int64_t base = ((int64_t)blocks.at[j] * n_kv + kh) * (kBS * HD);
 #pragma unroll
       for (int c = 0; c < NC; ++c)
-        kf[set][j][c] = *reinterpret_cast<const Unit*>(kp + c * 32);
+        kf[set][j][c] =
+            buffer_load<Unit>(k_cache + base, size, k_at + c * 32 * (int)sizeof(CT));
 #pragma unroll
       for (int i = 0; i < NV; ++i)
-        vf[set][j][i] =
-            *reinterpret_cast<const Unit*>(vp + i * WAVE_SIZE * 8);
+        vf[set][j][i] = buffer_load<Unit>(v_cache + base, size,
+                                          v_at + i * WAVE_SIZE * 8 * (int)sizeof(CT));
     }
   };
 
@@ -286,14 +323,26 @@ __launch_bounds__(kBlockThreads, 2) __global__ void paged_decode_kernel(
     __builtin_amdgcn_wave_barrier();
   };
 
+  // (no load in a branch: where paths of more and of fewer loads meet, the compiler
+  // waits for all of them)
   const int first = t_lo + wave;
-  if (first < t_hi) load_tile(0, first);
-  for (int t = first; t < t_hi; t += 2 * kWaves) {
-    if (t + kWaves < t_hi) load_tile(1, t + kWaves);
-    compute(0, t);
-    if (t + kWaves < t_hi) {
-      if (t + 2 * kWaves < t_hi) load_tile(0, t + 2 * kWaves);
-      compute(1, t + kWaves);
+  if (first < t_hi) {
+    load_tile(0, first, look_up(first));
+    if constexpr (ONE) {
+      compute(0, first);
+    } else {
+      Blocks even, odd = look_up(first + kWaves);
+      for (int t = first; t < t_hi; t += 2 * kWaves) {
+        load_tile(1, t + kWaves, odd);
+        even = look_up(t + 2 * kWaves);
+        in_order();
+        compute(0, t);
+        in_order();
+        load_tile(0, t + 2 * kWaves, even);
+        odd = look_up(t + 3 * kWaves);
+        in_order();
+        if (t + kWaves < t_hi) compute(1, t + kWaves);
+      }
     }
   }
 
@@ -514,10 +563,14 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
   }
   const dim3 grid((uint32_t)((int64_t)B * n_kv * n_splits)), block(kBlockThreads);
   auto stream = c10::hip::getCurrentHIPStream().stream();
-  auto launch = [&](auto hdv, auto ct, auto cap) {
+  // (12 rows of 500: 14.9 us with the loop's loads of no bytes, 13.9 without)
+  const int tiles = hd == 256 ? max_blocks : (max_blocks + 1) / 2;
+  const bool few = (tiles + n_splits - 1) / n_splits <= kWaves;
+  auto launch = [&](auto hdv, auto ct, auto cap, auto one) {
     using CT = decltype(ct);
     hipLaunchKernelGGL(
-        (paged_decode_kernel<decltype(hdv)::value, CT, decltype(cap)::value>),
+        (paged_decode_kernel<decltype(hdv)::value, CT, decltype(cap)::value,
+                             decltype(one)::value>),
         grid, block, 0, stream, (ushort*)out.data_ptr(),
         (const ushort*)q.data_ptr(), (const CT*)k_cache.data_ptr(),
         (const CT*)v_cache.data_ptr(), block_tables.data_ptr<int32_t>(),
@@ -526,8 +579,12 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
         part_ml_ptr);
   };
   auto with_cap = [&](auto hdv, auto ct) {
-    if (softcap > 0.0) launch(hdv, ct, std::true_type{});
-    else launch(hdv, ct, std::false_type{});
+    auto with_one = [&](auto capped) {
+      if (few) launch(hdv, ct, capped, std::true_type{});
+      else launch(hdv, ct, capped, std::false_type{});
+    };
+    if (softcap > 0.0) with_one(std::true_type{});
+    else with_one(std::false_type{});
   };
   auto with_hd = [&](auto ct) {
     if (hd == 256) with_cap(std::integral_constant<int, 256>{}, ct);

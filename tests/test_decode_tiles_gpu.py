@@ -186,3 +186,33 @@ def test_rows_of_a_larger_buffer():
     assert ops.paged_attention_decode(q, kc, vc, bt, total, 0.1, out=out) is out
     assert torch.equal(out[:2], ops.paged_attention_decode(q, kc, vc, bt, total, 0.1))
     assert (out[2:] == 7).all()
+
+
+@pytest.mark.parametrize("hd", [128, 256])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_last_tiles_of_a_wave(hd, fp8):
+    """1 to 12 tiles a wave, even and odd, beside waves of none; what lies in the blocks
+    behind a row's last one is not read. (A wave's tiles are every fourth of a split.)"""
+    torch.manual_seed(hd)
+    lens = [1, 16, 17, 32, 33, 63, 65, 127, 129, 191, 255, 257, 300, 400, 500, 700, 1100, 1501]
+    nq, nkv, wide = 8, 2, 100
+    need = [(n + 15) // 16 for n in lens]
+    kc = torch.randn(sum(need) + 1, nkv, 16, hd, device=DEV, dtype=torch.bfloat16)
+    vc = torch.randn_like(kc)
+    kc[0], vc[0] = float("nan"), float("nan")  # the table's other entries
+    if fp8:
+        kc, vc = kc.to(torch.float8_e5m2), vc.to(torch.float8_e5m2)
+    bt = torch.zeros(len(lens), wide, dtype=torch.int32)
+    at = 1
+    for i, n in enumerate(need):
+        bt[i, :n] = torch.arange(at, at + n)
+        at += n
+    for rows in ([len(lens) - 1], range(len(lens)), list(range(len(lens))) * 8):
+        rows = list(rows)
+        q = torch.randn(len(rows), nq, hd, device=DEV, dtype=torch.bfloat16)
+        sl = torch.tensor([lens[i] for i in rows], dtype=torch.int32, device=DEV)
+        args = (bt[rows].to(DEV), sl, hd ** -0.5)
+        got = ops.paged_attention_decode(q, kc, vc, *args)
+        want = ref.paged_attention_decode(q.float(), kc.float(), vc.float(), *args)
+        # fp32 throughout, one rounding
+        torch.testing.assert_close(got.float(), want, rtol=2.0 ** -8, atol=2.0 ** -9)
