@@ -238,9 +238,17 @@ __global__ __launch_bounds__(256, 1) void tiled_kernel(const Args a) {
   // out of cache, all at the first / apart: fp8 28672 x 4096 40 rows 32.0 / 25.9, 65536
   // x 8192 121 / 101, 128256 x 4096 117 / 108; bf16 28672 x 4096 40 rows 53.6 / 45.5;
   // 36864 x 4608 47.3 / 47.3). With more row tiles they would lose what they share.
-  const int first = !a.bounds && a.R <= BM && a.k_part == a.KB
-                        ? (int)((blockIdx.x >> 3) * 2u % (uint32_t)steps) : 0;
-  auto column = [&](int s) { return k0 + (s + first < steps ? s + first : s + first - steps) * kStep; };
+  // (Only in tiles of few rows: in the others it costs 1 % of a large product.)
+  constexpr bool kApart = WM <= 2;
+  int first = 0;
+  if constexpr (kApart) {
+    if (!a.bounds && a.R <= BM && a.k_part == a.KB)
+      first = (int)((blockIdx.x >> 3) * 2u % (uint32_t)steps);
+  }
+  auto column = [&](int s) {
+    if constexpr (!kApart) return k0 + s * kStep;
+    return k0 + (s + first < steps ? s + first : s + first - steps) * kStep;
+  };
   // load l of a batch: the AC of step sa of x, then the BC of step sb of w
   auto load = [&](int l, int pa, int sa, int pb, int sb) {
     if (l < AC) {
