@@ -136,3 +136,23 @@ def test_steps_do_not_share_what_is_still_copied():
                      ss.req.tokens[ss.chunk_start : ss.chunk_start + ss.chunk_len]]))
     for fb, ids in kept:
         assert fb.input_ids[: len(ids)].tolist() == ids
+
+
+@pytest.mark.parametrize("n,size", [(256, 256), (257, 272), (546, 560), (1025, 1040), (5174, 5184),
+                                    (16384, 16384), (20001, 20001), (40, 40), (97, 128)])
+def test_sizes_of_steps_in_eight_bits(n, size):
+    """Models of eight-bit products fill steps of more than 256 tokens up to whole
+    cache blocks; a layer that is not fused keeps the sizes of the library."""
+    from kubeai_amd.engine.runner import ModelRunner
+
+    class Any:
+        pass
+
+    runner, layers = ModelRunner.__new__(ModelRunner), [Any(), Any()]
+    runner.model = Any()
+    assert runner._step_size(n) == _bucket(n)
+    runner.model.layers = layers
+    layers[0]._fp8_fused = True
+    assert runner._step_size(n) == _bucket(n)
+    layers[1]._fp8_fused = True
+    assert runner._step_size(n) == size
