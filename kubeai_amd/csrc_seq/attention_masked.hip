@@ -635,48 +635,81 @@ __global__ __launch_bounds__(WAVE) void masked_prefill_mfma_kernel(
   }
 }
 
-constexpr int kPrefillThreads = 512;
+constexpr int kCUs = 256;
+// elements of a staged row of n, whole 16s: an odd number of 16s, so that eight rows of
+// transposed reads start 8 banks apart
+__host__ __device__ constexpr int staged(int n) { return (n / 16 | 1) * 16; }
+constexpr int prefill_threads(bool exact) { return exact ? 256 : 512; }
+constexpr int prefill_waves(int sub, int d_steps, int dv_tiles) {  // on a SIMD, at least
+  return dv_tiles > 8 ? 2 : sub > 1 || d_steps > 8 ? 3 : 4;
+}
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
 // Prompt portions on the matrix cores with the key / value tiles shared
 // through LDS. A block of HW * QW waves covers QW * 16 consecutive queries of
 // a run for HW query heads of one key/value head (for latent attention all
 // heads share the one cached row, for grouped heads the group does). Per
-// iteration the block stages 32 keys as they lie in the cache (16-byte loads,
-// padded rows): K rows are read back as MFMA operands in 8 or 16-byte pieces,
-// V rows through the transposing LDS read. kTied: the value is the leading
-// part of the key row, so one staged tile serves both. Two LDS buffers: the
-// next tile is loaded into registers before the products of the current one
-// and written to the other buffer after them, one barrier per iteration. P V
-// contracts all 32 keys of a tile in one v_mfma_f32_16x16x32_bf16 per 16 value
+// iteration the block stages 32 kSub keys as they lie in the cache (16-byte
+// loads, rows of an odd number of 32 bytes): K rows are read back as MFMA
+// operands in 8 or 16-byte pieces, V rows through the transposing LDS read.
+// kTied: the value is the leading part of the key row, so one staged tile
+// serves both. Two LDS buffers: the next tile is loaded into registers before
+// the products of the current one and written to the other buffer after them,
+// one barrier per iteration; its cache blocks were looked up an iteration
+// before. P V contracts 32 keys in one v_mfma_f32_16x16x32_bf16 per 16 value
 // dims (a lane's eight contraction slots are keys grp*4 + 0..3 and
 // 16 + grp*4 + 0..3, for P and V alike), and so does K Q^T over 32 key dims
 // when the key size allows (kWideQK). Statistics are fp32, base 2. kExact: the
 // sizes are D = 16 kMaxDSteps, Dv = 16 kMaxDvTiles and the block size is a
-// power of two; otherwise the template sizes are bounds and steps are guarded.
-template <int kMaxDSteps, int kMaxDvTiles, bool kWideQK, bool kTied, bool kExact>
-__global__ __launch_bounds__(kPrefillThreads) void masked_prefill_mfma_shared_kernel(
+// power of two of at least 16; otherwise the template sizes are bounds and
+// steps are guarded.
+// Keys begin at the window of the first of `span` queries (kAligned: at the 16 before
+// the block's own), so the 32 keys after which sums are scaled do not depend on how
+// many waves a block has.
+// Bound by instructions that one wave issues in a row (of the cycles: VALU 0.4,
+// matrix cores 0.25, LDS 0.3) and by the longest tile of queries, so: four waves a
+// block (kExact), which leaves a CU three or four blocks that do not wait for each
+// other; addresses of a piece from scalars; the columns' common maximum and the
+// scaling of the sums only when a lane has a new one. One run of 3000 tokens, 16
+// heads of 128: tied 153 -> 88 us, 4 key heads and a window of 512 41 -> 34; 2048
+// tokens, 16 heads of 64: 79 -> 50, tied 56 -> 35; tied 192 / 128 117 -> 68; sizes that
+// are not kExact: 96 123 -> 92, 128 / 256 211 -> 149; the same to the last bit.
+template <int kMaxDSteps, int kMaxDvTiles, bool kWideQK, bool kTied, bool kExact, int kSub = 1>
+__global__ __launch_bounds__(prefill_threads(kExact), prefill_waves(kSub, kMaxDSteps, kMaxDvTiles)) void masked_prefill_mfma_shared_kernel(
     bf16raw* __restrict__ out, int64_t out_stride, const bf16raw* __restrict__ q,
     int64_t q_stride, const bf16raw* __restrict__ k_cache,
     const bf16raw* __restrict__ v_cache, const int* __restrict__ block_tables,
     int max_blocks, const int* __restrict__ start_loc,
-    const int* __restrict__ positions, int n_seq, int HW, int QW, AttnArgs a) {
+    const int* __restrict__ positions, int n_seq, int HW, int QW, int span, int zb,
+    AttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) bf16raw lds[];
   typedef QkFrag<kWideQK> Frag;
   typedef typename Frag::type frag_t;
   constexpr int kNF = kMaxDSteps * 16 / Frag::kDims;
+  constexpr int kTile = kSub * kKT;
+  constexpr bool kAligned = kExact && kTied;  // tiles begin at multiples of 16 keys
+  constexpr int nthr = prefill_threads(kExact);
   // 16-byte pieces of a tile per thread
-  constexpr int nthr = kPrefillThreads;
-  constexpr int kKVec = (kKT * kMaxDSteps * 2 + nthr - 1) / nthr;
-  constexpr int kVVec = kTied ? 1 : (kKT * kMaxDvTiles * 2 + nthr - 1) / nthr;
+  constexpr int kKVec = (kTile * kMaxDSteps * 2 + nthr - 1) / nthr;
+  constexpr int kVVec = kTied ? 1 : (kTile * kMaxDvTiles * 2 + nthr - 1) / nthr;
+  constexpr bool kWholeK = kExact && kTile * kMaxDSteps * 2 % nthr == 0;
+  constexpr bool kWholeV = kExact && kTile * kMaxDvTiles * 2 % nthr == 0;
   const int G = a.G;
   const int D = kExact ? kMaxDSteps * 16 : a.D, Dv = kExact ? kMaxDvTiles * 16 : a.Dv;
-  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int lane = threadIdx.x % WAVE;
   const int col = lane & 15, grp = lane >> 4;
   const int hw = wave % HW, qw = wave / HW;
+  // The longest tiles first, and in every other round over the CUs from the shortest on:
+  // workgroups that meet on one CU add up to about the same number of keys.
+  const int per = G * zb, n_wg = gridDim.x;
+  const int round0 = blockIdx.x & ~(kCUs - 1);
+  const int rank = blockIdx.x & kCUs ? 2 * round0 + min(kCUs, n_wg - round0) - 1 - blockIdx.x
+                                     : blockIdx.x;
   int tile;
-  const int s = find_tile(start_loc, n_seq, QW * 16, blockIdx.x, &tile);
-  const int g = blockIdx.y, rep = a.H / G;
-  const int hz = blockIdx.z * HW + hw;
+  const int s = find_tile(start_loc, n_seq, QW * 16, (n_wg - 1 - rank) / per, &tile);
+  const int g = rank % per / zb, rep = a.H / G;
+  const int hz = rank % zb * HW + hw;
   const int s0 = start_loc[s], s1 = start_loc[s + 1];
   const int bq0 = s0 + tile * QW * 16;
   if (bq0 >= s1) return;  // the whole block: no barrier is skipped
@@ -692,17 +725,20 @@ __global__ __launch_bounds__(kPrefillThreads) void masked_prefill_mfma_shared_ke
   const int wpos_min = wave_on ? positions[q0] : 0, wpos_max = wpos_min + nq - 1;
   const int lo_q = q_ok ? a.lower(pos_q) : 0;
   const int wlo = a.lower(wpos_min), wlo_max = a.lower(max(wpos_max, 0));
-  const int blo = a.lower(bpos_min);
+  // (from the window of the first query of `span`, whatever the block's part of them)
+  const int blo = kAligned ? a.lower(bpos_min) & ~15
+                           : a.lower(bpos_min - (bq0 - s0) % span);
   // tiles of the kept first tokens, then from the first query's window on
-  const int kept = a.kept(blo), n_kept = (kept + kKT - 1) / kKT;
-  const int n_tiles = n_kept + (bpos_max - blo) / kKT + 1;
+  const int kept = a.kept(blo), n_kept = (kept + kTile - 1) / kTile;
+  const int n_tiles = n_kept + (bpos_max - blo) / kTile + 1;
   const int* bt = block_tables + (size_t)s * max_blocks;
   const int nf = D / Frag::kDims, ndt = Dv / 16;
-  const int krow = D + kRPad, vrow = kTied ? krow : Dv + kRPad;
-  const int k_elems = kKT * krow, v_elems = kTied ? 0 : kKT * vrow;
-  const int buf_elems = k_elems + v_elems + 2 * kKT;  // + key scales (fp32)
+  const int krow = staged(D), vrow = kTied ? krow : staged(Dv);
+  const int k_elems = kTile * krow, v_elems = kTied ? 0 : kTile * vrow;
+  const int buf_elems = k_elems + v_elems + 2 * kTile;  // + key scales (fp32)
   const int kcpr = D / 8, vcpr = Dv / 8;  // 16-byte chunks per cached row
   const ScoreConsts consts(a, h);
+  const bool plain = a.kscale == nullptr && a.slopes == nullptr && a.softcap <= 0.f;
 
   frag_t qf[kNF];
   const bf16raw* qrow = q + (size_t)tq * q_stride + h * D;
@@ -722,44 +758,82 @@ __global__ __launch_bounds__(kPrefillThreads) void masked_prefill_mfma_shared_ke
   for (int dt = 0; dt < kMaxDvTiles; ++dt) oacc[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
 
-  uint4 kreg[kKVec], vreg[kVVec];
-  float kscr = 0.f;
   auto first_key = [&](int it) {
-    return it < n_kept ? it * kKT : blo + (it - n_kept) * kKT;
+    return it < n_kept ? it * kTile : blo + (it - n_kept) * kTile;
   };
   auto last_key = [&](int it) { return it < n_kept ? kept - 1 : bpos_max; };
-  auto cached_at = [&](int j, int64_t* blk, int* off) {
-    *blk = bt[kExact ? j >> a.bs_shift : j / a.bs];
-    *off = kExact ? j & (a.bs - 1) : j % a.bs;
+  // Every load below is of every thread and every tile (past the end the last one
+  // again): a load under a branch would make the compiler wait for all of them.
+  auto key_at = [&](int it, int row) {  // tile `it`'s key of a row, a cached one
+    it = min(it, n_tiles - 1);
+    return min(first_key(it) + min(row, kTile - 1), last_key(it));
+  };
+  const int vper = G / a.kvs * a.bs, vfirst = g / a.kvs * a.bs;
+  u32x4 kreg[kKVec], vreg[kVVec];
+  float kscr = 0.f;
+  // The cache blocks of a tile, a step before its rows. kAligned: blocks hold multiples
+  // of 16 keys, so 16 keys share one: lane i has the block of keys 16 i on, and a wave's
+  // rows of one piece read it into a scalar. Otherwise each thread keeps those of its
+  // rows, and the rows' places in them.
+  constexpr bool kSameRows = kExact && kMaxDSteps == kMaxDvTiles;
+  constexpr int kKOwn = kAligned ? 1 : kKVec, kVOwn = kAligned || kSameRows ? 1 : kVVec;
+  int kblk[kKOwn], vblk[kVOwn], koff[kKOwn], voff[kVOwn], sblk = 0, soff = 0;
+  auto place = [&](int j, int* blk, int* off) {
+    const int b = kExact ? j >> a.bs_shift : j / a.bs;
+    *off = j - b * a.bs;
+    *blk = bt[b];
+  };
+  auto look_up = [&](int it) {
+    if constexpr (kAligned) {
+      kblk[0] = bt[key_at(it, lane * 16) >> a.bs_shift];
+    } else {
+#pragma unroll
+      for (int i = 0; i < kKVec; ++i)
+        place(key_at(it, (i * nthr + (int)threadIdx.x) / kcpr), &kblk[i], &koff[i]);
+      if constexpr (!kTied && !kSameRows) {
+#pragma unroll
+        for (int i = 0; i < kVVec; ++i)
+          place(key_at(it, (i * nthr + (int)threadIdx.x) / vcpr), &vblk[i], &voff[i]);
+      }
+      if (a.kscale != nullptr) place(key_at(it, (int)threadIdx.x), &sblk, &soff);
+    }
+  };
+  // piece i of the rows at `base`, chunks of 8 elements a row, `per` rows a block
+  auto load_piece = [&](const bf16raw* base, int it, int i, int chunks, int blk, int off,
+                        int per, int first, int64_t row_elems) {
+    const int v = i * nthr + threadIdx.x, row = v / chunks, c = v % chunks;
+    if constexpr (kAligned) {
+      off = key_at(it, row) & (a.bs - 1);
+      const bool whole = WAVE % chunks == 0 || chunks % WAVE == 0;  // rows of a wave: a power of 2
+      const int at = (i * nthr + wave * WAVE) / chunks / 16;
+      const int b = whole ? __builtin_amdgcn_readlane(blk, min(at, WAVE - 1))
+                          : __shfl(blk, row / 16, WAVE);
+      const bf16raw* p = base + ((uint64_t)(uint32_t)b * (uint32_t)per + (uint32_t)first) * row_elems;
+      return *(const u32x4*)((const char*)p + (uint32_t)(off * (int)row_elems + c * 8) * 2u);
+    } else {
+      return *(const u32x4*)(base + c * 8 +
+          (int64_t)((uint64_t)(uint32_t)blk * (uint32_t)per + (uint32_t)(first + off)) * row_elems);
+    }
   };
   auto load_tile = [&](int it) {
-    const int j0 = first_key(it), j_end = last_key(it);
-    int64_t blk;
-    int off;
-    if (a.kscale != nullptr && threadIdx.x < kKT) {
-      cached_at(min(j0 + (int)threadIdx.x, j_end), &blk, &off);
-      kscr = a.kscale[blk * a.bs + off];
-    }
 #pragma unroll
-    for (int i = 0; i < kKVec; ++i) {
-      const int v = i * nthr + threadIdx.x;
-      const int row = v / kcpr, c = v % kcpr;
-      if (row < kKT) {
-        cached_at(min(j0 + row, j_end), &blk, &off);
-        kreg[i] = *(const uint4*)(k_cache + ((blk * G + g) * a.bs + off) * D + c * 8);
-      }
-    }
+    for (int i = 0; i < kKVec; ++i)
+      kreg[i] = load_piece(k_cache, it, i, kcpr, kblk[kAligned ? 0 : i],
+                           koff[kAligned ? 0 : i], G * a.bs, g * a.bs, D);
     if constexpr (!kTied) {
 #pragma unroll
-      for (int i = 0; i < kVVec; ++i) {
-        const int v = i * nthr + threadIdx.x;
-        const int row = v / vcpr, c = v % vcpr;
-        if (row < kKT) {
-          cached_at(min(j0 + row, j_end), &blk, &off);
-          vreg[i] = *(const uint4*)(v_cache +
-              ((blk * (G / a.kvs) + g / a.kvs) * a.bs + off) * a.v_rs + c * 8);
-        }
+      for (int i = 0; i < kVVec; ++i)
+        vreg[i] = load_piece(v_cache, it, i, vcpr, kSameRows ? kblk[i] : vblk[i],
+                             kSameRows ? koff[i] : voff[i], vper, vfirst, a.v_rs);
+    }
+    if (a.kscale != nullptr) {
+      int64_t blk = sblk;
+      int off = soff;
+      if constexpr (kAligned) {
+        blk = __shfl(kblk[0], min((int)threadIdx.x / 16, WAVE - 1), WAVE);
+        off = key_at(it, (int)threadIdx.x) & (a.bs - 1);
       }
+      kscr = a.kscale[blk * a.bs + off];
     }
   };
   auto store_tile = [&](int buf) {
@@ -768,7 +842,8 @@ __global__ __launch_bounds__(kPrefillThreads) void masked_prefill_mfma_shared_ke
     for (int i = 0; i < kKVec; ++i) {
       const int v = i * nthr + threadIdx.x;
       const int row = v / kcpr, c = v % kcpr;
-      if (row < kKT) *(uint4*)(ks_ + row * krow + c * 8) = kreg[i];
+      asm volatile("" ::"v"(kreg[i]));  // waited for on every path
+      if (kWholeK || row < kTile) *(u32x4*)(ks_ + row * krow + c * 8) = kreg[i];
     }
     if constexpr (!kTied) {
       bf16raw* vs_ = ks_ + k_elems;
@@ -776,92 +851,136 @@ __global__ __launch_bounds__(kPrefillThreads) void masked_prefill_mfma_shared_ke
       for (int i = 0; i < kVVec; ++i) {
         const int v = i * nthr + threadIdx.x;
         const int row = v / vcpr, c = v % vcpr;
-        if (row < kKT) *(uint4*)(vs_ + row * vrow + c * 8) = vreg[i];
+        asm volatile("" ::"v"(vreg[i]));
+        if (kWholeV || row < kTile) *(u32x4*)(vs_ + row * vrow + c * 8) = vreg[i];
       }
     }
-    if (a.kscale != nullptr && threadIdx.x < kKT)
+    if (a.kscale != nullptr && threadIdx.x < kTile)
       ((float*)(ks_ + k_elems + v_elems))[threadIdx.x] = kscr;
   };
 
+  look_up(0);
   load_tile(0);
+  look_up(1);
   store_tile(0);
   __syncthreads();
-  int buf = 0;
-  for (int it = 0; it < n_tiles; ++it, buf ^= 1) {
-    const bool more = it + 1 < n_tiles;
-    if (more) load_tile(it + 1);
+  for (int it = 0, buf = 0;; ++it, buf ^= 1) {
+    load_tile(it + 1);
+    look_up(it + 2);
     const int j0 = first_key(it);
     const bf16raw* ks_ = lds + buf * buf_elems;
     const bf16raw* vs_ = ks_ + (kTied ? 0 : k_elems);
     const float* kc_ = (const float*)(ks_ + k_elems + v_elems);
     // wave-uniform: something of this tile is visible to the wave's queries
-    if (wave_on && j0 <= wpos_max && (j0 + kKT - 1 >= wlo || j0 < a.keep)) {
-      f32x4 sacc[2];
-      sacc[0] = sacc[1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    if (wave_on && j0 <= wpos_max && (j0 + kTile - 1 >= wlo || j0 < a.keep)) {
+      f32x4 sacc[2 * kSub];
+#pragma unroll
+      for (int i = 0; i < 2 * kSub; ++i) sacc[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
       const bf16raw* kp = ks_ + col * krow + grp * Frag::kElems;
 #pragma unroll
       for (int f = 0; f < kNF; ++f)
         if (kExact || f < nf) {
-          sacc[0] = mfma_qk(*(const frag_t*)(kp + f * Frag::kDims), qf[f], sacc[0]);
-          sacc[1] = mfma_qk(*(const frag_t*)(kp + 16 * krow + f * Frag::kDims), qf[f],
-                            sacc[1]);
+#pragma unroll
+          for (int i = 0; i < 2 * kSub; ++i)
+            sacc[i] = mfma_qk(*(const frag_t*)(kp + i * 16 * krow + f * Frag::kDims), qf[f],
+                              sacc[i]);
         }
-      // this lane: query `col`, keys j0 + sub * 16 + grp * 4 + i
-      float sc[8];
-      base2_scores<true>(sacc, consts, (float)(j0 + grp * 4 - pos_q),
-                         a.kscale != nullptr ? kc_ + grp * 4 : nullptr, sc);
+      // this lane: query `col`, keys jl + (e / 4) * 16 + e % 4
+      const int jl = j0 + grp * 4;
+      float sc[8 * kSub];
+      if (plain) {
+#pragma unroll
+        for (int e = 0; e < 8 * kSub; ++e) sc[e] = sacc[e >> 2][e & 3] * consts.mul;
+      } else {
+#pragma unroll
+        for (int u = 0; u < kSub; ++u)
+          base2_scores<true>(sacc + 2 * u, consts, (float)(jl + u * kKT - pos_q),
+                             a.kscale != nullptr ? kc_ + u * kKT + grp * 4 : nullptr,
+                             sc + 8 * u);
+      }
       // wave-uniform: a tile whose keys all queries see needs no mask. (Masks
       // are selects: hipcc 7.2 has lost such an assignment from under a branch.)
-      const int jl = j0 + grp * 4;
       if (it < n_kept) {
-        if (j0 + kKT > kept) {
+        if (j0 + kTile > kept) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e)
+          for (int e = 0; e < 8 * kSub; ++e)
             sc[e] = jl + (e >> 2) * 16 + (e & 3) < kept ? sc[e] : -INFINITY;
         }
-      } else if (nq < 16 || j0 + kKT - 1 > wpos_min || j0 < wlo_max) {
+      } else if (nq < 16 || j0 + kTile - 1 > wpos_min || j0 < wlo_max) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
+        for (int e = 0; e < 8 * kSub; ++e) {
           const int j = jl + (e >> 2) * 16 + (e & 3);
           const bool vis = (j <= pos_q) & ((j >= lo_q) | (j < a.keep));
           sc[e] = vis ? sc[e] : -INFINITY;
         }
       }
-      float mt = sc[0];
+      // 32 keys after 32 as to the largest score and what it scales. Wave-uniform: the
+      // lanes of a query have to agree on it only where a lane has a new one.
+      float mt[kSub], ms[kSub], corr[kSub];
+      bool any = false;
 #pragma unroll
-      for (int e = 1; e < 8; ++e) mt = fmaxf(mt, sc[e]);
-      mt = column_max(mt, lane);
-      const float m_new = fmaxf(m, mt);
-      // no visible key so far: keep everything at zero without forming inf - inf
-      const float m_use = m_new == -INFINITY ? 0.f : m_new;
-      const float corr = __builtin_amdgcn_exp2f(m - m_use);
-      float pv[8];
-      float ps = 0.f;
+      for (int u = 0; u < kSub; ++u) {
+        mt[u] = sc[8 * u];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        pv[e] = __builtin_amdgcn_exp2f(sc[e] - m_use);
-        ps += pv[e];
+        for (int e = 1; e < 8; ++e) mt[u] = fmaxf(mt[u], sc[8 * u + e]);
+        any = any | (mt[u] > m);
+        ms[u] = m;
+        corr[u] = 1.f;
       }
-      union { bf16x8 v; uint32_t u[4]; } pk;
+      if (__builtin_amdgcn_ballot_w64(any) != 0) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) pk.u[e] = cvt_pk_bf16(pv[2 * e], pv[2 * e + 1]);
-      const bf16x8 pb = pk.v;
-      l = l * corr + ps;
-      m = m_new;
+        for (int u = 0; u < kSub; ++u) {
+          ms[u] = fmaxf(m, column_max(mt[u], lane));
+          corr[u] = ms[u] == m ? 1.f : __builtin_amdgcn_exp2f(m - ms[u]);
+          m = ms[u];
+        }
+#pragma unroll
+        for (int dt = 0; dt < kMaxDvTiles; ++dt)
+          if (kExact || dt < ndt) {
+            oacc[dt][0] *= corr[0]; oacc[dt][1] *= corr[0];
+            oacc[dt][2] *= corr[0]; oacc[dt][3] *= corr[0];
+          }
+      }
+      union { bf16x8 v[kSub]; uint32_t u[4 * kSub]; } pk;
+#pragma unroll
+      for (int u = 0; u < kSub; ++u) {
+        // no visible key so far: keep everything at zero without forming inf - inf
+        const float m_use = ms[u] == -INFINITY ? 0.f : ms[u];
+        float ps = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float p0 = __builtin_amdgcn_exp2f(sc[8 * u + 2 * e] - m_use);
+          const float p1 = __builtin_amdgcn_exp2f(sc[8 * u + 2 * e + 1] - m_use);
+          ps += p0;
+          ps += p1;
+          pk.u[4 * u + e] = cvt_pk_bf16(p0, p1);
+        }
+        l = fmaf(l, corr[u], ps);
+      }
       const bf16raw* vp = vs_ + (grp * 4 + (col >> 2)) * vrow + (col & 3) * 4;
 #pragma unroll
-      for (int dt = 0; dt < kMaxDvTiles; ++dt) {
-        if (kExact || dt < ndt) {
-          const bf16x4 v0 = lds_read_transposed(vp + dt * 16);
-          const bf16x4 v1 = lds_read_transposed(vp + dt * 16 + 16 * vrow);
-          const bf16x8 vf = (bf16x8){v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
-          f32x4 o = oacc[dt];
-          o[0] *= corr; o[1] *= corr; o[2] *= corr; o[3] *= corr;
-          oacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pb, o, 0, 0, 0);
+      for (int u = 0; u < kSub; ++u) {
+        if (u > 0 && __builtin_amdgcn_ballot_w64(corr[u] != 1.f) != 0) {
+#pragma unroll
+          for (int dt = 0; dt < kMaxDvTiles; ++dt)
+            if (kExact || dt < ndt) {
+              oacc[dt][0] *= corr[u]; oacc[dt][1] *= corr[u];
+              oacc[dt][2] *= corr[u]; oacc[dt][3] *= corr[u];
+            }
+        }
+#pragma unroll
+        for (int dt = 0; dt < kMaxDvTiles; ++dt) {
+          if (kExact || dt < ndt) {
+            const bf16x4 v0 = lds_read_transposed(vp + u * kKT * vrow + dt * 16);
+            const bf16x4 v1 = lds_read_transposed(vp + (u * kKT + 16) * vrow + dt * 16);
+            const bf16x8 vf = (bf16x8){v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+            oacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pk.v[u], oacc[dt], 0, 0, 0);
+          }
         }
       }
     }
-    if (more) store_tile(buf ^ 1);
+    if (it + 1 == n_tiles) break;
+    store_tile(buf ^ 1);
     __syncthreads();
   }
   l += __shfl_xor(l, 16, WAVE);
@@ -1181,47 +1300,67 @@ void masked_paged_attention(torch::Tensor out, torch::Tensor q,
       // tiles shared through LDS by up to 8 waves: heads of a group first,
       // then neighbouring query tiles
       const int rep = H / G;
-      int HW = 1;
-      while (HW * 2 <= rep && HW < 8) HW *= 2;
-      constexpr int WPB = kPrefillThreads / WAVE;
-      const int QW = WPB / HW;
+      constexpr int kShortRun = 32;
+      auto launch_shared = [&](auto kern, auto is_exact, int sub = 1) {
+      constexpr int WPB = prefill_threads(decltype(is_exact)::value) / WAVE;
+      const int kTile = sub * kKT;
+      int pow2 = 1;
+      while (pow2 * 2 <= rep && pow2 < 8) pow2 *= 2;
+      const int HW = std::min(pow2, WPB);
+      const int QW = WPB / HW, span = std::max(QW, 8 / std::min(pow2, 8)) * 16;
       const int btiles = T / (QW * 16) + n_seq;
       const int zb = (rep + HW - 1) / HW;
-      TORCH_CHECK(G <= 65535 && zb <= 65535);
-      auto launch_shared = [&](auto kern) {
+      TORCH_CHECK((int64_t)btiles * G * zb <= INT32_MAX / (WPB * WAVE));
+      const size_t lds = (size_t)2 * kTile * (staged(D) + (tied ? 0 : staged(Dv)) + 2) *
+                         sizeof(bf16raw);
+      if (lds > 64 * 1024)
+        hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            160 * 1024);
       hipLaunchKernelGGL(kern,
-                         dim3(btiles, G, zb), dim3(WPB * WAVE), lds_shared,
+                         dim3(btiles * G * zb), dim3(WPB * WAVE), lds,
                          SEQ_STREAM(), (bf16raw*)out.data_ptr(), out.stride(0),
                          (const bf16raw*)q.data_ptr(), q.stride(0),
                          (const bf16raw*)k_cache.data_ptr(),
                          (const bf16raw*)v_cache.data_ptr(),
                          (const int*)block_tables.data_ptr(),
                          (int)block_tables.size(1), (const int*)start_loc.data_ptr(),
-                         (const int*)positions.data_ptr(), n_seq, HW, QW, args);
+                         (const int*)positions.data_ptr(), n_seq, HW, QW, span, zb, args);
       };
       auto sized = [&](auto is_tied) {
         constexpr bool kT = decltype(is_tied)::value;
-        const bool shift = args.bs_shift >= 0, wide = D % 32 == 0;
-        if (shift && D == 128 && Dv == 128)
-          launch_shared(masked_prefill_mfma_shared_kernel<8, 8, true, kT, true>);
+        const bool shift = args.bs_shift >= 4 && bs * (int64_t)D <= INT32_MAX / 2;
+        const bool wide = D % 32 == 0;
+        // One row that is key and value: 64 keys at a time, in registers and LDS of three
+        // workgroups a CU, for half the barriers (3000 tokens, 16 heads of 128: 88 us, 32
+        // at a time 97; 10 runs of 100 tokens 9.6 / 10.0); not for runs that end in the
+        // first 32 (40 of 17 tokens: 8.9 / 7.9).
+        const bool two = kT && max_len > kShortRun;
+        if (shift && two && D == 128 && Dv == 128)
+          launch_shared(masked_prefill_mfma_shared_kernel<8, 8, true, true, true, 2>,
+                        std::true_type{}, 2);
+        else if (shift && two && D == 64 && Dv == 64)
+          launch_shared(masked_prefill_mfma_shared_kernel<4, 4, true, true, true, 2>,
+                        std::true_type{}, 2);
+        else if (shift && D == 128 && Dv == 128)
+          launch_shared(masked_prefill_mfma_shared_kernel<8, 8, true, kT, true>, std::true_type{});
         else if (shift && D == 64 && Dv == 64)
-          launch_shared(masked_prefill_mfma_shared_kernel<4, 4, true, kT, true>);
+          launch_shared(masked_prefill_mfma_shared_kernel<4, 4, true, kT, true>, std::true_type{});
         else if (shift && !kT && D == 64 && Dv == 128)
-          launch_shared(masked_prefill_mfma_shared_kernel<4, 8, true, false, true>);
+          launch_shared(masked_prefill_mfma_shared_kernel<4, 8, true, false, true>, std::true_type{});
         else if (shift && kT && D == 192 && Dv == 128)
-          launch_shared(masked_prefill_mfma_shared_kernel<12, 8, true, true, true>);
+          launch_shared(masked_prefill_mfma_shared_kernel<12, 8, true, true, true>, std::true_type{});
         else if (D <= 128 && Dv <= 128 && wide)
-          launch_shared(masked_prefill_mfma_shared_kernel<8, 8, true, kT, false>);
+          launch_shared(masked_prefill_mfma_shared_kernel<8, 8, true, kT, false>, std::false_type{});
         else if (D <= 128 && Dv <= 128)
-          launch_shared(masked_prefill_mfma_shared_kernel<8, 8, false, kT, false>);
+          launch_shared(masked_prefill_mfma_shared_kernel<8, 8, false, kT, false>, std::false_type{});
         // larger keys (a latent with a rotated part behind it) or values keep
         // more fragments in registers
         else if (D <= 128 && wide)
-          launch_shared(masked_prefill_mfma_shared_kernel<8, 16, true, kT, false>);
+          launch_shared(masked_prefill_mfma_shared_kernel<8, 16, true, kT, false>, std::false_type{});
         else if (wide)
-          launch_shared(masked_prefill_mfma_shared_kernel<16, 16, true, kT, false>);
+          launch_shared(masked_prefill_mfma_shared_kernel<16, 16, true, kT, false>, std::false_type{});
         else
-          launch_shared(masked_prefill_mfma_shared_kernel<16, 16, false, kT, false>);
+          launch_shared(masked_prefill_mfma_shared_kernel<16, 16, false, kT, false>, std::false_type{});
       };
       if (tied) sized(std::true_type{});
       else sized(std::false_type{});

@@ -339,8 +339,9 @@ class ModelRunner:
         # Keeps the products' row counts on a small fixed set up to 1024
         # tokens (algorithm table, decode graphs), above that on multiples
         # of 256; closer where the library has no part in them (_step_size).
-        # Pad tokens form a throwaway prefill sequence over cache block 0: slot -1 (no KV write), row-local
-        # compute only (GEMMs/norms are row-independent), never sampled.
+        # Pad tokens form a throwaway prefill sequence over cache block 0:
+        # slot -1 (no KV write), row-local compute only (GEMMs/norms are
+        # row-independent), never sampled.
         T = sum(lens)
         T_pad = self._step_size(T)
         pad = T_pad - T
