@@ -197,45 +197,80 @@ struct ProductSums {
   int N;
 };
 
-// Sum of PARTS parts of 8 neighbouring columns; every load is issued before
+// The scales of N times 8 neighbouring columns n[i].. of row m, asked for before the
+// parts: loads in any case (of something else without sx, and not used then), since
+// a load under a branch is waited for by itself.
+template <int N>
+struct SumScales {
+  float sx, sw[N][8];
+  DEV_INLINE SumScales(const ProductSums& p, int64_t m, const int (&n)[N]) {
+    const float* rows = p.sx ? p.sx + m : p.part;
+    const float* cols = p.sx ? p.sw : p.part;
+    sx = *rows;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sw[i][j] = cols[n[i] + j];
+  }
+};
+
+// Sum of PARTS parts of N times 8 neighbouring columns; every load is issued before
 // the first addition (a chain of eight would cost eight latencies).
-template <int PARTS>
-DEV_INLINE void add_parts8(const float* a, int64_t stride, float4_t* v) {
-  float4_t t[PARTS][2];
+template <int PARTS, int N>
+DEV_INLINE void add_parts8(const float* const (&a)[N], int64_t first, int64_t stride,
+                           float4_t (&v)[N][2]) {
+  float4_t t[PARTS][N][2];
 #pragma unroll
-  for (int s = 0; s < PARTS; ++s) {
-    const float4_t* b = reinterpret_cast<const float4_t*>(a + s * stride);
-    t[s][0] = b[0];
-    t[s][1] = b[1];
-  }
+  for (int s = 0; s < PARTS; ++s)
 #pragma unroll
-  for (int s = 0; s < PARTS; ++s) {
-    v[0] += t[s][0];
-    v[1] += t[s][1];
-  }
+    for (int i = 0; i < N; ++i) {
+      const float4_t* b = reinterpret_cast<const float4_t*>(a[i] + (first + s) * stride);
+      t[s][i][0] = b[0];
+      t[s][i][1] = b[1];
+    }
+#pragma unroll
+  for (int s = 0; s < PARTS; ++s)
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      v[i][0] += t[s][i][0];
+      v[i][1] += t[s][i][1];
+    }
 }
 
-// 8 neighbouring columns n.. of row m, as the bf16 values a stored product
-// would have (the parts are added in order, whatever their number)
-DEV_INLINE ushort8 read_sums8(const ProductSums& p, int64_t m, int n) {
-  const float* a = p.part + m * p.N + n;
-  float4_t v[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-  int s = 0;
-  for (; s + 8 <= p.parts; s += 8) add_parts8<8>(a + s * p.stride, p.stride, v);
-  if (s + 4 <= p.parts) {
-    add_parts8<4>(a + s * p.stride, p.stride, v);
-    s += 4;
-  }
-  for (; s < p.parts; ++s) add_parts8<1>(a + s * p.stride, p.stride, v);
-  ushort8 o;
-  const float sx = p.sx ? p.sx[m] : 1.0f;
+// N times 8 neighbouring columns n[i].. of row m, as the bf16 values a stored product
+// would have (the parts are added in order, whatever their number; what is left of
+// the eights at once too: 7 parts one by one cost four latencies)
+template <int N>
+DEV_INLINE void read_sums8(const ProductSums& p, int64_t m, const int (&n)[N],
+                           const SumScales<N>& by, ushort8 (&o)[N]) {
+  const float* a[N];
+  float4_t v[N][2];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    float f = v[j / 4][j % 4];
-    if (p.sx) f = f * sx * p.sw[n + j];
-    o[j] = f32_to_bf16(f);
+  for (int i = 0; i < N; ++i) {
+    a[i] = p.part + m * p.N + n[i];
+    v[i][0] = v[i][1] = float4_t{0.f, 0.f, 0.f, 0.f};
   }
-  return o;
+  // (16 at once are more than the compiler gives registers to)
+  constexpr int kAtOnce = N > 1 ? 4 : 8;
+  int s = 0;
+  for (; s + kAtOnce <= p.parts; s += kAtOnce) add_parts8<kAtOnce>(a, s, p.stride, v);
+  switch (p.parts - s) {
+    case 1: add_parts8<1>(a, s, p.stride, v); break;
+    case 2: add_parts8<2>(a, s, p.stride, v); break;
+    case 3: add_parts8<3>(a, s, p.stride, v); break;
+    case 4: add_parts8<4>(a, s, p.stride, v); break;
+    case 5: add_parts8<5>(a, s, p.stride, v); break;
+    case 6: add_parts8<6>(a, s, p.stride, v); break;
+    case 7: add_parts8<7>(a, s, p.stride, v); break;
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float f = v[i][j / 4][j % 4];
+      if (p.sx) f = f * by.sx * by.sw[i][j];
+      o[i][j] = f32_to_bf16(f);
+    }
 }
 
 // ---------------- wave reductions (64-wide) ----------------

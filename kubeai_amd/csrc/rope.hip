@@ -66,6 +66,9 @@ DEV_INLINE void put_row8(CT* dst, const ushort8& v) {
 }
 
 // SUMS: the projection is a product's parts; q goes to its own rows.
+// A chain of latencies at few tokens: slot and position at once, then angles, scales
+// and the parts of both halves at once; no division in 64 bits where 32 will do. 40
+// tokens, 32/8 heads of 128: 6.4 us with each behind the one before, now 4.7.
 template <typename CT, bool SUMS>
 __launch_bounds__(256) __global__ void rope_cache_kernel(
     ushort* __restrict__ qkv,  // [T, (n_q + 2 n_kv) hd], rows strided; SUMS:
@@ -82,20 +85,39 @@ __launch_bounds__(256) __global__ void rope_cache_kernel(
   const int n_rot = (n_q + n_kv) * ppu;
   const int n_item = n_rot + n_kv * (hd / 8);
   const int64_t flat = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t tok = flat / n_item;
+  // (a division in 64 bits takes longer than the whole item)
+  const bool small = n_tok * n_item + 256 <= UINT32_MAX;
+  const int64_t tok = small ? (uint32_t)flat / (uint32_t)n_item : flat / n_item;
   if (tok >= n_tok) return;
   const int item = (int)(flat - tok * n_item);
   ushort* row = qkv + tok * stride;
   if (item < n_rot) {
     const int head = item / ppu, p = item % ppu * 8;
     ushort* base = row + (int64_t)head * hd + p;
-    const int64_t slot = head < n_q ? 0 : slot_mapping[tok];
+    int64_t slot = slot_mapping[tok];
+    int pos = positions[tok];
+    asm volatile("" : "+v"(slot), "+v"(pos));  // both on their way before either is used
+    if (head < n_q) slot = 0;
     if (slot < 0) return;  // a padding token's key goes nowhere
-    const float* cs = cos_sin + (int64_t)positions[tok] * hd + p;
+    const float* cs = cos_sin + (int64_t)pos * hd + p;
+    float cv[8], sv[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      cv[j] = cs[j];
+      sv[j] = cs[half + j];
+    }
     ushort8 a, b;
     if constexpr (SUMS) {
-      a = read_sums8(sums, tok, head * hd + p);
-      b = read_sums8(sums, tok, head * hd + p + half);
+      // both halves' parts at once
+      const int cols[2] = {head * hd + p, head * hd + p + half};
+      const SumScales<2> by(sums, tok, cols);
+      asm volatile("" ::: "memory");  // (or the angles' loads move behind the parts')
+      ushort8 ab[2];
+      read_sums8<2>(sums, tok, cols, by, ab);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(cv[j]), "+v"(sv[j]));
+      a = ab[0];
+      b = ab[1];
     } else {
       a = *reinterpret_cast<const ushort8*>(base);
       b = *reinterpret_cast<const ushort8*>(base + half);
@@ -103,7 +125,7 @@ __launch_bounds__(256) __global__ void rope_cache_kernel(
     ushort8 oa, ob;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const float c = cs[j], s = cs[half + j];
+      const float c = cv[j], s = sv[j];
       const float x1 = bf16_to_f32(a[j]), x2 = bf16_to_f32(b[j]);
       oa[j] = f32_to_bf16(x1 * c - x2 * s);
       ob[j] = f32_to_bf16(x2 * c + x1 * s);
@@ -123,11 +145,16 @@ __launch_bounds__(256) __global__ void rope_cache_kernel(
     const int upr = hd / 8;
     const int head = (item - n_rot) / upr, u = (item - n_rot) % upr * 8;
     ushort8 v;
-    if constexpr (SUMS)
-      v = read_sums8(sums, tok, (n_q + n_kv + head) * hd + u);
-    else
+    if constexpr (SUMS) {
+      const int cols[1] = {(n_q + n_kv + head) * hd + u};
+      const SumScales<1> by(sums, tok, cols);
+      ushort8 one[1];
+      read_sums8<1>(sums, tok, cols, by, one);
+      v = one[0];
+    } else {
       v = *reinterpret_cast<const ushort8*>(
           row + (int64_t)(n_q + n_kv + head) * hd + u);
+    }
     put_row8(v_cache + (((slot / bs) * n_kv + head) * bs + slot % bs) * hd + u, v);
   }
 }

@@ -271,3 +271,40 @@ def test_products_under_transforms():
     near(v.grad, w.float().sum(0).expand(4, K))
     lin = Fp8Linear(w)
     assert lin(v).requires_grad and not lin(x).requires_grad
+
+
+@pytest.mark.parametrize("parts", [1, 2, 3, 4, 5, 6, 7, 8, 9, 12, 15, 17])
+@pytest.mark.parametrize("N,scaled", [(520, True), (4096, False), (8200, True)])
+def test_any_number_of_parts(parts, N, scaled):
+    """Whatever is left of the eights that are added at once, and with scales or none:
+    the bits of the parts added in order in fp32, scaled by row and column, rounded."""
+    T, hd = 19, 8
+    torch.manual_seed(parts)
+    part = torch.randn(parts, T, N, device=DEV)
+    sx = torch.rand(T, device=DEV) + 0.5 if scaled else None
+    sw = (torch.rand(N + 1, device=DEV) + 0.5)[1:] if scaled else None  # 4 bytes off
+    y = torch.zeros(T, N, device=DEV)
+    for p in part:
+        y = y + p
+    y = (y * sx[:, None] * sw if scaled else y).to(torch.bfloat16)
+    w, r = torch.randn(N, device=DEV, dtype=torch.bfloat16), _x(T, N)
+    got, res = ops.fused_add_rmsnorm(ops.ProductSums(part, sx, sw), r.clone(), w, 1e-5)
+    want, kept = ops.fused_add_rmsnorm(y.clone(), r.clone(), w, 1e-5)
+    assert torch.equal(res, kept) and torch.equal(res, y + r)
+    torch.testing.assert_close(got, want, atol=0, rtol=2.0 ** -7)  # a step: contractions
+    _, hidden = ops.add_and_norm(
+        ops.BranchNorm(ops.ProductSums(part, sx, sw), w, 1e-5), r, w, 1e-5)
+    torch.testing.assert_close(hidden, r + ops.rmsnorm(y, w, 1e-5), atol=2.0 ** -7, rtol=2.0 ** -7)
+    # heads of 16: 8 columns a half and whole value rows
+    hd = 16
+    heads = N // hd - 2
+    width = (heads + 2) * hd
+    cache = [torch.zeros(2, 1, 16, hd, device=DEV, dtype=torch.bfloat16) for _ in range(4)]
+    pos, slots = torch.arange(T, device=DEV, dtype=torch.int32), torch.randperm(32, device=DEV)[:T]
+    cs = ref.make_cos_sin_cache(hd, 32).to(DEV)
+    own = ops.ProductSums(part[..., :width].contiguous(), sx, sw[:width] if scaled else None)
+    q = ops.rope_and_cache(own, heads, pos, cs, *cache[:2], slots)
+    q2 = ops.rope_and_cache(y[:, :width].contiguous(), heads, pos, cs, *cache[2:], slots)
+    assert torch.equal(cache[1], cache[3])
+    for a, b in ((q, q2), (cache[0], cache[2])):
+        torch.testing.assert_close(a.float(), b.float(), atol=2.0 ** -20, rtol=2.0 ** -7)
