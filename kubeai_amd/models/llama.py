@@ -320,7 +320,8 @@ class MoEMLP(nn.Module):
     slower one, the library's on each expert's slice, after one look at the
     experts' row counts."""
 
-    #: one pass of 8 experts of 14336 x 4096, us, weight-streaming / tiled /
+    #: one pass of 8 experts of 14336 x 4096, us, weight-streaming (before its loads
+    #: went without branches: 4 % of a decode step of 40 tokens since) / tiled /
     #: every expert's tokens asked for one after the other: fp8 128 tokens
     #: 353/383/722, 512 819/470/1361, 2048 2413/1015/2006; bf16 128
     #: 602/684/1159, 512 1397/871/1614, 2048 4223/1708/2488 (streaming reads
