@@ -673,7 +673,8 @@ typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 // scaling of the sums only when a lane has a new one. One run of 3000 tokens, 16
 // heads of 128: tied 153 -> 88 us, 4 key heads and a window of 512 41 -> 34; 2048
 // tokens, 16 heads of 64: 79 -> 50, tied 56 -> 35; tied 192 / 128 117 -> 68; sizes that
-// are not kExact: 96 123 -> 92, 128 / 256 211 -> 149; the same to the last bit.
+// are not kExact: 96 123 -> 92, 128 / 256 211 -> 149; the same to the last bit (a window
+// or chunk on tied rows: to a rounding of the probabilities, as tiles begin elsewhere).
 template <int kMaxDSteps, int kMaxDvTiles, bool kWideQK, bool kTied, bool kExact, int kSub = 1>
 __global__ __launch_bounds__(prefill_threads(kExact), prefill_waves(kSub, kMaxDSteps, kMaxDvTiles)) void masked_prefill_mfma_shared_kernel(
     bf16raw* __restrict__ out, int64_t out_stride, const bf16raw* __restrict__ q,
