@@ -174,9 +174,10 @@ __launch_bounds__(NW * WAVE_SIZE) __global__ void skinny_kernel(
   const int k0 = of * k_part, k1 = min(KB, k0 + k_part);
   const int steps = (k1 - k0 + kStep - 1) / kStep;
   // whole rows of 2^n bytes: workgroups that read the same columns of K at a time
-  // wait for the same few of the memory's channels
+  // wait for the same few of the memory's channels. Not those of experts: in a routed
+  // model a sum in another order moves tokens whose scores all but tie.
   const int first =
-      parts == 1 ? __builtin_amdgcn_readfirstlane((blockIdx.x >> 3) * 3u % (uint32_t)steps) : 0;
+      !GROUPED && parts == 1 ? __builtin_amdgcn_readfirstlane((blockIdx.x >> 3) * 3u % (uint32_t)steps) : 0;
   int m0 = 0, M = M_all;  // this pass's first row and the rows from it on
   int m_end = M_all;
   if constexpr (GROUPED) {
