@@ -360,11 +360,12 @@ Shape check(const torch::Tensor& x, const torch::Tensor& w,
               "fp8 operands come with their scales, bf16 ones without");
   if (fp8 && !raw) {
     TORCH_CHECK(sx->scalar_type() == torch::kFloat32 && sx->is_contiguous() &&
-                sx->numel() == s.M && sw->scalar_type() == torch::kFloat32 &&
-                sw->is_contiguous() && sw->numel() == s.N);
+                sx->is_cuda() && sx->numel() == s.M &&
+                sw->scalar_type() == torch::kFloat32 && sw->is_contiguous() &&
+                sw->is_cuda() && sw->numel() == s.N);
   }
   if (bias.has_value())
-    TORCH_CHECK(bias->scalar_type() == torch::kBFloat16 &&
+    TORCH_CHECK(bias->scalar_type() == torch::kBFloat16 && bias->is_cuda() &&
                 bias->is_contiguous() && bias->numel() == s.N);
   return s;
 }
@@ -521,9 +522,9 @@ void skinny_experts(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   }
   if (fp8) {
     TORCH_CHECK(sx->scalar_type() == torch::kFloat32 && sx->is_contiguous() &&
-                sx->numel() == x.size(0) &&
+                sx->is_cuda() && sx->numel() == x.size(0) &&
                 sw->scalar_type() == torch::kFloat32 && sw->is_contiguous() &&
-                sw->numel() == (int64_t)E * N);
+                sw->is_cuda() && sw->numel() == (int64_t)E * N);
   }
   const int R = y.size(0);
   if (R == 0) return;

@@ -433,18 +433,43 @@ def _tiled_operands(x, weight) -> bool:
     )
 
 
-def _tiled_scales(x, weight, x_scale, w_scale) -> bool:
-    """Scales that the tiled product reads: one per row and column, dense fp32,
-    the columns' four at a time. (The library takes one for all as well.)"""
+def _row_and_column_scales(x, weight, x_scale, w_scale) -> bool:
+    """Scales of fp8 operands that the kernels read: one per row and column, dense
+    fp32. (The library takes one for all as well.)"""
     return (
         x_scale.dtype == w_scale.dtype == torch.float32
         and x_scale.device == w_scale.device == x.device
         and x_scale.numel() == x.shape[0]
         and x_scale.is_contiguous()
-        and w_scale.shape == (1, weight.shape[0])
+        and w_scale.numel() == weight.shape[0]
         and w_scale.is_contiguous()
-        and aligned(w_scale)
         and not observed(x_scale, w_scale)
+    )
+
+
+def _tiled_scales(x, weight, x_scale, w_scale) -> bool:
+    """Scales that the tiled product reads, the columns' four at a time."""
+    return (
+        _row_and_column_scales(x, weight, x_scale, w_scale)
+        and w_scale.shape == (1, weight.shape[0])
+        and aligned(w_scale)
+    )
+
+
+def _kernel_writes(out, x, weight) -> bool:
+    """Whether a kernel writes the product into `out` (None: a new tensor). (The
+    library fits one of another shape to the result.)"""
+    return out is None or (
+        out.shape == (x.shape[0], weight.shape[0]) and out.is_contiguous()
+        and out.dtype == torch.bfloat16 and out.device == x.device
+    )
+
+
+def _kernel_adds(bias, weight) -> bool:
+    return bias is None or (
+        bias.dtype == torch.bfloat16 and bias.device == weight.device
+        and bias.numel() == weight.shape[0] and bias.is_contiguous()
+        and not observed(bias)
     )
 
 
@@ -666,25 +691,24 @@ def linear_fp8(xq, x_scale, weight, w_scale, bias=None, out=None):
     if (
         xq.shape[0] <= 96
         and _streams(xq.shape[0], *weight.shape, fp8=True)
+        and not observed(xq, weight)
         and _skinny_operands(xq, weight)
-        and (out is None or out.is_contiguous())
+        and _row_and_column_scales(xq, weight, x_scale, w_scale)
+        and _kernel_adds(bias, weight)
+        and _kernel_writes(out, xq, weight)
     ):
         if out is None:
             out = torch.empty(
                 (xq.shape[0], weight.shape[0]), dtype=torch.bfloat16, device=xq.device
             )
-        _C.skinny_linear(out, xq, weight, x_scale.reshape(-1), w_scale.reshape(-1), bias)
+        _C.skinny_linear(out, xq, weight, x_scale.view(-1), w_scale.view(-1), bias)
         return out
     if (
         bias is None
         and _tiled_better(xq.shape[0], *weight.shape, fp8=True)
         and _tiled_operands(xq, weight)
         and _tiled_scales(xq, weight, x_scale, w_scale)
-        and (
-            out is None  # (the library fits one of another shape to the result)
-            or out.shape == (xq.shape[0], weight.shape[0]) and out.is_contiguous()
-            and out.dtype == torch.bfloat16 and out.device == xq.device
-        )
+        and _kernel_writes(out, xq, weight)
     ):
         return _tiled_linear(xq, weight, x_scale.view(-1), w_scale.view(-1), out)
     kw = {} if out is None else {"out": out}

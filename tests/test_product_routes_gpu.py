@@ -106,6 +106,66 @@ def test_fp8_results_of_another_shape_go_to_the_library():
         _near(out, x, w, sx, sw)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (8, 8192, 512),   # (cut along K)
+    (12, 16384, 512),
+    (1, 65536, 4096),
+    (16, 28672, 4096),
+    (40, 1024, 16384),  # long rows
+])
+def test_what_the_streaming_product_does_not_take_goes_to_the_library(M, N, K, monkeypatch):
+    """The forms of scales, bias and result that it has no part in give what the
+    library gives for them; the usual ones are its own."""
+    x, w, sx, sw = _fp8_product(M, N, K)
+    assert ops._streams(M, N, K, fp8=True)
+    calls = []
+    own = ops._C.skinny_linear
+    monkeypatch.setattr(ops._C, "skinny_linear", lambda *a: calls.append(a) or own(*a))
+    out = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    assert ops.linear_fp8(x, sx, w, sw.view(1, -1), out=out) is out
+    _near(out, x, w, sx, sw)
+    bias = torch.randn(N, device=DEV, dtype=torch.bfloat16)
+    got = ops.linear_fp8(x, sx, w, sw.view(1, -1), bias)
+    assert len(calls) == 2
+    assert ((got.double() - out.double() - bias.double()).abs()
+            <= 2.0 ** -7 * (out.double().abs() + bias.double().abs())).all()
+    # one scale for all, as the library takes it
+    one = torch.full((1,), 0.5, device=DEV)
+    _near(ops.linear_fp8(x, one, w, one.view(1, 1)), x, w, one, one)
+    # a result of another shape is fitted
+    for rows in (0, M + 3):
+        other = torch.empty(rows, N, device=DEV, dtype=torch.bfloat16)
+        assert ops.linear_fp8(x, sx, w, sw.view(1, -1), out=other) is other
+        assert other.shape == (M, N)
+        _near(other, x, w, sx, sw)
+    # what follows the operation sees it
+    assert ops.linear_fp8(x, sx.clone().requires_grad_(), w, sw.view(1, -1)).requires_grad
+
+    class Seen(torch.utils._python_dispatch.TorchDispatchMode):
+        names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(func._schema.name)
+            return func(*args, **(kwargs or {}))
+
+    with Seen() as seen:
+        ops.linear_fp8(x, sx, w, sw.view(1, -1))
+    assert "aten::_scaled_mm" in seen.names
+    assert len(calls) == 2
+    with pytest.raises(RuntimeError):
+        ops.linear_fp8(x, sx, w, sw.double().view(1, -1))
+
+
+def test_the_streaming_product_refuses_scales_and_bias_in_host_memory():
+    x, w, sx, sw = _fp8_product(8, 64, 512)
+    y, bias = (torch.empty(n, 64, device=DEV, dtype=torch.bfloat16) for n in (8, 1))
+    ops._C.skinny_linear(y, x, w, sx, sw, bias.zero_())
+    _near(y, x, w, sx, sw)
+    for args in ((sx.cpu(), sw, bias), (sx, sw.cpu(), bias), (sx, sw, bias.cpu())):
+        with pytest.raises(RuntimeError):
+            ops._C.skinny_linear(y, x, w, *args)
+
+
 class _Rows(torch.nn.Module):
     """Keeps the rows that it is given."""
 
