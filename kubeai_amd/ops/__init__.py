@@ -489,24 +489,28 @@ def _tiled_better(M: int, N: int, K: int, fp8: bool) -> bool:
     126 / 90; over 68 others 0.85, in bf16 above 200 rows 0.82 to 1.10. 17 to
     96 rows beside 24576 columns and more of even rows (fp8 28672 x 4096 40 rows 31.6 / 25.7,
     96 rows 33.1 / 28.9; bf16 57.1 / 45.4 and 58.8 / 49.6, but 57344 x 8192 173 / 163, 16384
-    x 4096 34.8 / 40.5), fp8 of others where the library's tiles do not fill (22016 x 1280 36
-    rows 13.4 / 11.3, 58368 x 2560 43.6 / 34.4, but 35840 x 2048 20.9 / 23.9), bf16 beside
-    65536 columns (96256 x 2304 94 / 86): over 348 products the 152 chosen take 0.83, 1.07
-    at worst. Other bf16 products stay (28672 x 4096 2048 rows 333 / 391)."""
-    if 16 < M <= 96 and N >= 24576 and _even_rows(K, fp8) and (fp8 or K <= 4096):
-        return True
-    if N >= 49152 and K >= 2048:
-        return M > 16 and (fp8 or M <= 1024 and N >= 98304)
-    if 16 < M <= 96:
+    x 4096 34.8 / 40.5). fp8 rows of other lengths where the library's tiles do not fill:
+    18432 to 32767 columns however short they are (22016 x 1280 36 rows 11.7 / 10.2, 18432 x
+    128 40 rows 5.2 / 4.8, 32000 x 256 8.5 / 5.7; over 117 products 0.83, 1.06 at worst) and
+    from 45056 on (58368 x 2560 43.6 / 34.4; over 25 with K from 1024 0.75, 1.14 at
+    worst), but 35840 x 2048 21.1 / 23.8. bf16 beside 65536 columns (96256 x 2304 36 rows
+    95 / 86, 91392 x 3264 132 / 124; over 41 products 0.79, 1.02 at worst), but 49920 to 65152
+    columns 0.89 to 1.10. Other bf16 products stay (28672 x 4096 2048 rows 333 / 391)."""
+    if M <= 16:
+        return False
+    if M <= 96:
+        even = N >= 24576 and _even_rows(K, fp8)
         if fp8:
-            return 18432 <= N < 32768 or N >= 45056 and K >= 1024
-        return 65536 <= N < 200000 and K <= 4096
+            return even or 18432 <= N < 32768 or N >= 45056 and K >= 1024
+        if N >= 98304 and K >= 2048:
+            return True
+        return K <= 4096 and (even or 65536 <= N < 200000)
+    if N >= 49152 and K >= 2048:
+        return fp8 or M <= 1024 and N >= 98304
     tiles = -(-M // 64) * -(-N // 128)
     if K > 16384:
-        return fp8 and M > 96 and tiles >= 64
-    return fp8 and M > 96 and K >= 2048 and tiles >= 160 and not (
-        192 < M <= 256 and N >= 16384
-    )
+        return fp8 and tiles >= 64
+    return fp8 and K >= 2048 and tiles >= 160 and not (192 < M <= 256 and N >= 16384)
 
 
 def _tiled_linear(x, weight, x_scale=None, w_scale=None, out=None, act=0):

@@ -78,6 +78,26 @@ def test_few_rows_of_the_tiled_product(M, fp8):
     assert ((y.double() - want).abs() <= tol).all()
 
 
+@pytest.mark.parametrize("N,K,fp8", [(18432, 128, True), (18448, 256, True), (24592, 384, True),
+                                     (32752, 1408, True), (65536, 64, False),
+                                     (65552, 192, False), (65536, 2112, False)])
+@pytest.mark.parametrize("M", [17, 96])
+def test_few_rows_of_few_steps(M, N, K, fp8):
+    """The tiled product of fewer steps of K than its first columns are apart, through
+    the calls that choose it."""
+    assert ops._tiled_better(M, N, K, fp8)
+    x, w = _operands(M, N, K, M)
+    if fp8:
+        (x, sx), (w, sw) = ops.quant_fp8(x), ops.quant_fp8(w)
+        y = ops.linear_fp8(x, sx, w, sw.view(1, -1))
+        x, w = x.double() * sx[:, None].double(), w.double() * sw[:, None].double()
+    else:
+        y = ops.linear(x, w)
+    want = x.double() @ w.double().T
+    tol = 2.0 ** -8 * want.abs() + 2.0 ** -13 * (x.double().abs() @ w.double().abs().T)
+    assert ((y.double() - want).abs() <= tol).all()
+
+
 @pytest.mark.parametrize("T", [1, 16, 17, 40, 96])
 @pytest.mark.parametrize("gelu", [False, True])
 def test_activation_goes_with_few_rows(T, gelu):

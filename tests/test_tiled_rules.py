@@ -34,6 +34,18 @@ import kubeai_amd.ops as ops
     (96, 128256, 4096, False, True),   # 225 / 207
     (2048, 28672, 4096, False, False),  # 333 / 391
     (2048, 128256, 4096, False, False),
+    # few rows beside wide weights whose rows are no whole 4 KB
+    (36, 96256, 2304, False, True),    # 95 / 86
+    (67, 91392, 3264, False, True),    # 132 / 124
+    (61, 57984, 1856, False, False),   # 42.9 / 45.5
+    (29, 67072, 8000, False, False),
+    (37, 98624, 640, False, True),     # 50 / 36
+    (36, 22016, 1280, True, True),     # 11.7 / 10.2
+    (40, 18432, 128, True, True),      # 5.2 / 4.8
+    (40, 35840, 2048, True, False),    # 21.1 / 23.8
+    (41, 33408, 1536, True, False),    # 18.1 / 19.7
+    (72, 58816, 1024, True, True),     # 36.7 / 20.7
+    (39, 54272, 256, True, False),     # 8.7 / 9.9
 ])
 def test_whole_products(M, N, K, fp8, better):
     assert ops._tiled_better(M, N, K, fp8) is better
