@@ -729,9 +729,12 @@ __global__ __launch_bounds__(prefill_threads(kExact), prefill_waves(kSub, kMaxDS
   // (from the window of the first query of `span`, whatever the block's part of them)
   const int blo = kAligned ? a.lower(bpos_min) & ~15
                            : a.lower(bpos_min - (bq0 - s0) % span);
+  // rows [hidden_lo, hidden) of the first tile from there lie in front of the window
+  const int hidden_lo = max(0, a.keep - blo), hidden = a.lower(bpos_min) - blo;
   // tiles of the kept first tokens, then from the first query's window on
   const int kept = a.kept(blo), n_kept = (kept + kTile - 1) / kTile;
   const int n_tiles = n_kept + (bpos_max - blo) / kTile + 1;
+  const int hiding = hidden > hidden_lo ? n_kept : -1;  // that tile
   const int* bt = block_tables + (size_t)s * max_blocks;
   const int nf = D / Frag::kDims, ndt = Dv / 16;
   const int krow = staged(D), vrow = kTied ? krow : staged(Dv);
@@ -837,7 +840,7 @@ __global__ __launch_bounds__(prefill_threads(kExact), prefill_waves(kSub, kMaxDS
       kscr = a.kscale[blk * a.bs + off];
     }
   };
-  auto store_tile = [&](int buf) {
+  auto store_tile = [&](int buf, int it) {
     bf16raw* ks_ = lds + buf * buf_elems;
 #pragma unroll
     for (int i = 0; i < kKVec; ++i) {
@@ -845,6 +848,18 @@ __global__ __launch_bounds__(prefill_threads(kExact), prefill_waves(kSub, kMaxDS
       const int row = v / kcpr, c = v % kcpr;
       asm volatile("" ::"v"(kreg[i]));  // waited for on every path
       if (kWholeK || row < kTile) *(u32x4*)(ks_ + row * krow + c * 8) = kreg[i];
+    }
+    if constexpr (kAligned) {
+      // no query sees these rows, but 0 times a value that is not finite is not 0
+      if (it == hiding) {
+#pragma unroll
+        for (int i = 0; i < kKVec; ++i) {
+          const int v = i * nthr + threadIdx.x;
+          const int row = v / kcpr, c = v % kcpr;
+          if (row >= hidden_lo && row < hidden)
+            *(u32x4*)(ks_ + row * krow + c * 8) = (u32x4){0u, 0u, 0u, 0u};
+        }
+      }
     }
     if constexpr (!kTied) {
       bf16raw* vs_ = ks_ + k_elems;
@@ -863,7 +878,7 @@ __global__ __launch_bounds__(prefill_threads(kExact), prefill_waves(kSub, kMaxDS
   look_up(0);
   load_tile(0);
   look_up(1);
-  store_tile(0);
+  store_tile(0, 0);
   __syncthreads();
   for (int it = 0, buf = 0;; ++it, buf ^= 1) {
     load_tile(it + 1);
@@ -981,7 +996,7 @@ __global__ __launch_bounds__(prefill_threads(kExact), prefill_waves(kSub, kMaxDS
       }
     }
     if (it + 1 == n_tiles) break;
-    store_tile(buf ^ 1);
+    store_tile(buf ^ 1, it + 1);
     __syncthreads();
   }
   l += __shfl_xor(l, 16, WAVE);

@@ -1,7 +1,8 @@
 """Masked attention of prompt portions in bf16, at the edges of its tiles of keys and
 queries: runs that end at and beside 16, 32 and 64 keys, portions that continue, windows
 and chunks that begin inside 16 keys, cache blocks of 8 to 32, sizes with kernels of
-their own and others. Cached rows that no query may see hold NaN: none is read."""
+their own and others. Cached rows that no query may see hold NaN, in hidden blocks and
+beside visible rows: none reaches a result."""
 import pytest
 import torch
 
@@ -41,6 +42,9 @@ def test_prompt_tiles(H, G, D, Dv, tied, bs, short, mask):
             seen = min(bs, p + n - b * bs)
             kc[at, :, :seen] = torch.randn(G, seen, D).bfloat16()
             vc[at, :, :seen] = torch.randn(G, seen, Dv).bfloat16()
+            gone = [j % bs for j in range(b * bs, min((b + 1) * bs, low))
+                    if j >= opts.get("keep_first", 0)]
+            kc[at, :, gone] = vc[at, :, gone] = float("nan")
     if tied:
         vc = kc[..., :Dv]
     q = torch.randn(sum(n for n, _ in runs), H, D).bfloat16()
