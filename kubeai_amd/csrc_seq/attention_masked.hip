@@ -1307,40 +1307,42 @@ void masked_paged_attention(torch::Tensor out, torch::Tensor q,
                          (int)block_tables.size(1), (const int*)start_loc.data_ptr(),
                          (const int*)positions.data_ptr(), n_seq, args);
     };
-    const size_t lds_shared =
-        (size_t)2 * (kKT * (D + kRPad) + (tied ? 0 : kKT * (Dv + kRPad)) + 2 * kKT) *
-        sizeof(bf16raw);
     const bool cache_al16 = ((size_t)k_cache.data_ptr()) % 16 == 0 &&
                             ((size_t)v_cache.data_ptr()) % 16 == 0;
-    if (D <= 256 && Dv <= 256 && lds_shared <= 64 * 1024 && cache_al16) {
-      // tiles shared through LDS by up to 8 waves: heads of a group first,
-      // then neighbouring query tiles
+    if (D <= 256 && Dv <= 256 && cache_al16) {
+      // tiles shared through LDS by 4 (the template's sizes) or 8 waves: heads of a
+      // group first, then neighbouring query tiles
+      // (one wave by itself / this, us: 2048 tokens, 16 heads, 4 of keys, 256 / 256 1196 / 186,
+      // 10 runs of 100 57.6 / 19.4, 4 of 17 43.5 / 20.5)
       const int rep = H / G;
       constexpr int kShortRun = 32;
       auto launch_shared = [&](auto kern, auto is_exact, int sub = 1) {
-      constexpr int WPB = prefill_threads(decltype(is_exact)::value) / WAVE;
-      const int kTile = sub * kKT;
-      int pow2 = 1;
-      while (pow2 * 2 <= rep && pow2 < 8) pow2 *= 2;
-      const int HW = std::min(pow2, WPB);
-      const int QW = WPB / HW, span = std::max(QW, 8 / std::min(pow2, 8)) * 16;
-      const int btiles = T / (QW * 16) + n_seq;
-      const int zb = (rep + HW - 1) / HW;
-      TORCH_CHECK((int64_t)btiles * G * zb <= INT32_MAX / (WPB * WAVE));
-      const size_t lds = (size_t)2 * kTile * (staged(D) + (tied ? 0 : staged(Dv)) + 2) *
-                         sizeof(bf16raw);
-      if (lds > 64 * 1024)
-        hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            160 * 1024);
-      hipLaunchKernelGGL(kern,
-                         dim3(btiles * G * zb), dim3(WPB * WAVE), lds,
-                         SEQ_STREAM(), (bf16raw*)out.data_ptr(), out.stride(0),
-                         (const bf16raw*)q.data_ptr(), q.stride(0),
-                         (const bf16raw*)k_cache.data_ptr(),
-                         (const bf16raw*)v_cache.data_ptr(),
-                         (const int*)block_tables.data_ptr(),
-                         (int)block_tables.size(1), (const int*)start_loc.data_ptr(),
-                         (const int*)positions.data_ptr(), n_seq, HW, QW, span, zb, args);
+        constexpr int WPB = prefill_threads(decltype(is_exact)::value) / WAVE;
+        const int kTile = sub * kKT;
+        int pow2 = 1;
+        while (pow2 * 2 <= rep && pow2 < 8) pow2 *= 2;
+        const int HW = std::min(pow2, WPB);
+        const int QW = WPB / HW, span = std::max(QW, 8 / std::min(pow2, 8)) * 16;
+        const int btiles = T / (QW * 16) + n_seq;
+        const int zb = (rep + HW - 1) / HW;
+        TORCH_CHECK((int64_t)btiles * G * zb <= INT32_MAX / (WPB * WAVE));
+        // (two buffers of rows and key scales: 68 KB at the largest sizes)
+        const size_t lds = (size_t)2 * kTile * (staged(D) + (tied ? 0 : staged(Dv)) + 2) *
+                           sizeof(bf16raw);
+        if (lds > 64 * 1024) {  // (the same limit whatever the sizes: threads share it)
+          const hipError_t e = hipFuncSetAttribute(
+              (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+          TORCH_CHECK(e == hipSuccess, "masked attention: ", hipGetErrorString(e));
+        }
+        hipLaunchKernelGGL(kern,
+                           dim3(btiles * G * zb), dim3(WPB * WAVE), lds,
+                           SEQ_STREAM(), (bf16raw*)out.data_ptr(), out.stride(0),
+                           (const bf16raw*)q.data_ptr(), q.stride(0),
+                           (const bf16raw*)k_cache.data_ptr(),
+                           (const bf16raw*)v_cache.data_ptr(),
+                           (const int*)block_tables.data_ptr(),
+                           (int)block_tables.size(1), (const int*)start_loc.data_ptr(),
+                           (const int*)positions.data_ptr(), n_seq, HW, QW, span, zb, args);
       };
       auto sized = [&](auto is_tied) {
         constexpr bool kT = decltype(is_tied)::value;

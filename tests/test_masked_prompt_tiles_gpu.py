@@ -16,7 +16,8 @@ MASKS = [dict(), dict(window=37), dict(window=37, keep_first=20), dict(chunk=40,
 @pytest.mark.parametrize("H,G,D,Dv,tied", [
     (6, 1, 128, 128, True), (4, 2, 128, 128, False), (3, 1, 64, 64, True),
     (4, 4, 64, 64, False), (4, 2, 64, 128, False), (5, 1, 192, 128, True),
-    (4, 1, 48, 48, False), (2, 1, 128, 256, False),
+    (4, 1, 48, 48, False), (2, 1, 128, 256, False), (2, 1, 256, 256, False),
+    (2, 2, 256, 240, False), (2, 1, 256, 256, True),
     (2, 1, 256, 224, False)])  # (more than 64 KB of LDS)
 @pytest.mark.parametrize("bs", [8, 16, 32])
 @pytest.mark.parametrize("short", [True, False])
