@@ -107,6 +107,7 @@ def convert_to_fp8(model: nn.Module) -> int:
     Dense decoder layers additionally get the FUSED activation-quant path
     (llama.DecoderLayer checks _fp8_fused): producer kernels emit fp8 +
     per-row scales, so per-linear dynamic quantization disappears.
+    _fp8_widths: the sizes by which a step's size is chosen (ModelRunner).
     """
     n = _swap_linears(model)
     for layer in getattr(model, "layers", []):
@@ -114,6 +115,7 @@ def convert_to_fp8(model: nn.Module) -> int:
         mlp = getattr(layer, "mlp", None)
         if attn is None or not isinstance(getattr(attn, "qkv_proj", None), Fp8Linear):
             continue
+        layer._fp8_widths = _row_product_sizes(attn, mlp)
         if isinstance(getattr(mlp, "gate_up_proj", None), Fp8Linear):
             layer._fp8_fused = True  # dense: norms/activations emit fp8
         elif hasattr(mlp, "experts"):
@@ -121,6 +123,23 @@ def convert_to_fp8(model: nn.Module) -> int:
             # bf16 (router needs it) and MoEMLP quantizes once itself
             layer._fp8_fused = True
     return n
+
+
+def _row_product_sizes(attn: nn.Module, mlp: nn.Module):
+    """(N, K) of the eight-bit products that all rows of a layer's step go through, or
+    None where the library has others or has these whatever their sizes: projections
+    with a bias or in bf16, experts that are not multiplied in one launch."""
+    names = ("qkv_proj", "o_proj"), ("gate_up_proj", "down_proj")
+    linears = [getattr(attn, n, None) for n in names[0]]
+    if hasattr(mlp, "experts"):
+        here = getattr(mlp, "sorts_here", None)
+        if here is None or not here():
+            return None
+    else:
+        linears += [getattr(mlp, n, None) for n in names[1]]
+    if not all(type(m) is Fp8Linear and m.bias is None for m in linears):
+        return None
+    return tuple((m.out_features, m.in_features) for m in linears)
 
 
 def _swap_linears(mod: nn.Module) -> int:

@@ -338,7 +338,7 @@ class ModelRunner:
         # ---- pad the token stream to a bucket size --------------------
         # Keeps the products' row counts on a small fixed set up to 1024
         # tokens (algorithm table, decode graphs), above that on multiples
-        # of 256; closer where the library has no part in them (_step_size).
+        # of 256; closer where no product of the step is the library's (_step_size).
         # Pad tokens form a throwaway prefill sequence over cache block 0:
         # slot -1 (no KV write), row-local compute only (GEMMs/norms are
         # row-independent), never sampled.
@@ -468,15 +468,23 @@ class ModelRunner:
         )
 
     def _step_size(self, n: int) -> int:
-        """The token count that a step of n tokens runs as. In eight bits the steps of
-        more than 256 tokens have products, norms and attention from kernels here, whose
-        tiles take any number of rows: they are filled up to whole cache blocks only
-        (546 tokens of Llama-3 8B, 8 layers, 2282 us as 640, 2193 as 560)."""
-        layers = getattr(self.model, "layers", None)
-        if 256 < n <= _BUCKET_MAX and layers and all(
-            getattr(layer, "_fp8_fused", False) for layer in layers
+        """The token count that a step of n tokens runs as: one of the sizes that the
+        library is kept on (_bucket), unless all products of the step's rows are the
+        tiled kernel's, which takes any number of rows (eight bits, and widths at which
+        ops has them from it): then the step is filled up to whole cache blocks only.
+        us, the library's size / whole blocks, 8 layers of Llama-3 8B (4 of Mixtral
+        8x7B): 270 tokens 1426 / 1387 (1760 / 1651), 400 1710 / 1603 (2041 / 1904), 546
+        2053 / 1964 (2181 / 2062), 1300 3509 / 3335 (3533 / 3033), 3100 6878 / 6823 (6227
+        / 6035), 5000 10925 / 10890; none of 21 slower."""
+        if not 256 < n <= _BUCKET_MAX:
+            return _bucket(n)
+        rows = -(-n // 16) * 16
+        sizes = {getattr(layer, "_fp8_widths", None)
+                 for layer in getattr(self.model, "layers", None) or [None]}
+        if None not in sizes and all(
+            ops.fp8_product_tiled(rows, N, K) for of in sizes for N, K in of
         ):
-            return -(-n // 16) * 16
+            return rows
         return _bucket(n)
 
     def _upload(self, host: dict) -> dict:

@@ -437,21 +437,44 @@ class MoEMLP(nn.Module):
                     return False
         return True
 
+    def _routes(self) -> bool:
+        """Whether csrc/moe.hip takes the routing of such rows as _on_device asks for."""
+        gate = self.gate.weight
+        return (
+            gate.dtype == torch.bfloat16
+            and gate.shape[1] % 8 == 0
+            and gate.is_contiguous()
+            and ops.aligned(gate)
+            and self.n_experts <= 32
+            and self.top_k <= min(8, self.n_experts)
+            and self._own_experts()
+        )
+
+    def sorts_here(self) -> bool:
+        """Whether steps of more than GROUPED_MAX_TOKENS have their routing and, for
+        all experts, both projections from kernels here, whatever their size. (In bf16
+        that depends on the rows.)"""
+        if not self._routes():
+            return False
+        for proj in ("gate_up_proj", "down_proj"):
+            w = self._stack(proj, "weight_fp8")
+            if w is None or self._stack(proj, "weight_scale") is None or (
+                not ops.grouped_linear_takes(w[0], w)
+            ):
+                return False
+        return True
+
     def _on_device(self, x: torch.Tensor) -> bool:
         """Whether csrc/moe.hip takes the routing of x."""
         return (
             x.is_cuda
-            and x.dtype == self.gate.weight.dtype == torch.bfloat16
+            and x.dtype == torch.bfloat16
             and x.is_contiguous()
             and x.shape[0] >= 1
             and x.stride(0) == x.shape[1]  # (of a single row it may be anything)
-            and x.shape[1] % 8 == 0
-            and self.gate.weight.is_contiguous()
             and not torch.is_grad_enabled()
-            and ops.aligned(x, self.gate.weight)
-            and self.n_experts <= 32
-            and self.top_k <= min(8, self.n_experts)
-            and self._own_experts()
+            and ops.aligned(x)
+            and self._routes()
         )
 
     def _sorted(self, x: torch.Tensor) -> torch.Tensor:

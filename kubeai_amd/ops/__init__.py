@@ -513,6 +513,12 @@ def _tiled_better(M: int, N: int, K: int, fp8: bool) -> bool:
     return fp8 and K >= 2048 and tiles >= 160 and not (192 < M <= 256 and N >= 16384)
 
 
+def fp8_product_tiled(M: int, N: int, K: int) -> bool:
+    """Whether linear_fp8 has a product of these sizes, without a bias, from the tiled
+    kernel and not from the library."""
+    return N % 16 == 0 and K % 128 == 0 and K < 2**23 and _tiled_better(M, N, K, fp8=True)
+
+
 def _tiled_linear(x, weight, x_scale=None, w_scale=None, out=None, act=0):
     if out is None:
         out = torch.empty(

@@ -138,21 +138,77 @@ def test_steps_do_not_share_what_is_still_copied():
         assert fb.input_ids[: len(ids)].tolist() == ids
 
 
+def _runner(hidden, ff, heads, kv_heads, preset="llama-3-8b", shards=1, **other):
+    """A runner over an eight-bit model of these widths, without memory for it."""
+    import dataclasses
+
+    from kubeai_amd.engine.quant import convert_to_fp8
+    from kubeai_amd.engine.runner import ModelRunner
+    from kubeai_amd.models.config import PRESETS
+    from kubeai_amd.models.llama import LlamaForCausalLM
+
+    # a shard of a tensor-parallel model has a part of the heads and of the inner width
+    cfg = dataclasses.replace(
+        PRESETS[preset], hidden_size=hidden, intermediate_size=ff // shards,
+        num_attention_heads=heads // shards, num_key_value_heads=kv_heads // shards,
+        num_hidden_layers=2, vocab_size=64, **other)
+    runner = ModelRunner.__new__(ModelRunner)
+    runner.model = LlamaForCausalLM(cfg, device="meta")
+    convert_to_fp8(runner.model)
+    return runner
+
+
 @pytest.mark.parametrize("n,size", [(256, 256), (257, 272), (546, 560), (1025, 1040), (5174, 5184),
                                     (16384, 16384), (20001, 20001), (40, 40), (97, 128)])
 def test_sizes_of_steps_in_eight_bits(n, size):
-    """Models of eight-bit products fill steps of more than 256 tokens up to whole
-    cache blocks; a layer that is not fused keeps the sizes of the library."""
-    from kubeai_amd.engine.runner import ModelRunner
-
-    class Any:
-        pass
-
-    runner, layers = ModelRunner.__new__(ModelRunner), [Any(), Any()]
-    runner.model = Any()
-    assert runner._step_size(n) == _bucket(n)
-    runner.model.layers = layers
-    layers[0]._fp8_fused = True
-    assert runner._step_size(n) == _bucket(n)
-    layers[1]._fp8_fused = True
+    """Where all products of a step's rows are the tiled kernel's, steps of more than
+    256 tokens are filled up to whole cache blocks."""
+    runner = _runner(4096, 14336, 32, 8)
     assert runner._step_size(n) == size
+    # a layer that is not in eight bits keeps the sizes of the library
+    del runner.model.layers[1]._fp8_widths
+    assert runner._step_size(n) == _bucket(n)
+
+
+@pytest.mark.parametrize("n", [272, 320, 546, 700, 1025, 2000, 3088, 5174, 16000])
+@pytest.mark.parametrize("widths", [
+    dict(hidden=1536, ff=8960, heads=12, kv_heads=2),              # K below 2048
+    dict(hidden=896, ff=4864, heads=7, kv_heads=1),
+    dict(hidden=4096, ff=14336, heads=32, kv_heads=8, shards=4),   # o_proj: K 1024
+    dict(hidden=4096, ff=14336, heads=32, kv_heads=8, shards=8),
+    dict(hidden=4096, ff=14336, heads=32, kv_heads=8, attention_bias=True),
+    # (experts on a device where they are not multiplied in one launch)
+    dict(hidden=4096, ff=256, heads=32, kv_heads=8, preset="mixtral-8x7b"),
+])
+def test_steps_with_products_of_the_library_keep_its_sizes(n, widths):
+    assert _runner(**widths)._step_size(n) == _bucket(n)
+
+
+@pytest.mark.parametrize("n,size", [(272, 320), (570, 640), (609, 624), (642, 656), (1030, 1040)])
+def test_step_sizes_go_by_the_products_of_their_rows(n, size):
+    """2048 x 2048 is the tiled kernel's from 160 tiles of 64 x 128 on: 577 rows."""
+    from kubeai_amd import ops
+
+    runner = _runner(2048, 8192, 16, 8)
+    assert runner._step_size(n) == size
+    assert ops.fp8_product_tiled(577, 2048, 2048) and not ops.fp8_product_tiled(576, 2048, 2048)
+    for off in ((600, 2056, 2048), (600, 2048, 2080)):
+        assert not ops.fp8_product_tiled(*off)
+
+
+@pytest.mark.gpu
+def test_experts_in_one_launch_are_no_products_of_the_library():
+    import dataclasses
+
+    from kubeai_amd.engine.quant import convert_to_fp8
+    from kubeai_amd.models.config import PRESETS
+    from kubeai_amd.models.llama import LlamaForCausalLM
+
+    for experts, here in ((4, True), (40, False)):  # (40: routed by the library)
+        cfg = dataclasses.replace(PRESETS["mixtral-tiny"], num_local_experts=experts)
+        model = LlamaForCausalLM(cfg, device="cuda")
+        layer = model.layers[0]
+        assert not layer.mlp.sorts_here()  # bf16: by the rows
+        convert_to_fp8(model)
+        assert layer.mlp.sorts_here() is here
+        assert layer._fp8_widths == (((512, 256), (256, 256)) if here else None)
