@@ -372,42 +372,37 @@ def _even_rows(K: int, fp8: bool) -> bool:
     return K * (1 if fp8 else 2) % 4096 == 0
 
 
-def _few_rows_better(M: int, N: int, K: int, fp8: bool) -> bool:
-    """Whether the weight-streaming product, uncut, beats the library's: up to 16 rows
-    and a width that fills the chip (us, weights out of cache, library / this, 8 rows):
-    bf16 4096 -> 28672 60.6 / 41.5, 4096 -> 16384 32.1 / 23.7, 4096 -> 128256 183 / 173,
-    8192 -> 57344 172 / 158, 2304 -> 87808 136 / 80; but 1792 -> 56320 38.6 / 39.8, 2304 ->
-    256000 207 / 218, 7680 -> 14848 45 / 52; fp8 4096 -> 28672 31.7 / 23.6, 8192 -> 16384 51
-    / 24, 4096 -> 128256 112 / 94, 6656 -> 9216 38 / 19, but 8192 -> 8192 at 16 rows 16.4 /
-    21.3, 9472 -> 59648 102 / 110, 1536 -> 116992 39 / 41. Not for rows under 256 bytes
-    (128 -> 65536 fp8 5.6 / 6.7). Over 308 products the 200 chosen take 0.74 of the time,
-    1.10 at worst."""
-    if M > 16 or K * (1 if fp8 else 2) < 256:
-        return False
-    if N >= 16384 and _even_rows(K, fp8):
-        return True
-    if fp8:
-        return M <= 12 if 8192 <= N < 16384 else N >= 16384 and (N <= 40000 or K <= 1024)
-    return 16384 <= N <= 40000 or 65536 <= N < 200000
-
-
 def _streams_better(M: int, N: int, K: int, fp8: bool) -> bool:
-    """Whether the weight-streaming product beats the library's for the length of its
-    rows: very long ones, which the library does not cut (us, library / this): 32256 ->
-    2048 83 / 32 at 8 rows, 127 / 52 at 96; it does at 16384 (-> 1024 20.4 / 16.5 at 8
-    rows, 21.0 / 19 at 48; fp8 20.2 / 11, 20.1 / 15 at 96). And up to 16 rows, uncut, by a
-    rule for where it gains much; _few_rows_better has more of them."""
+    """Whether the weight-streaming product beats the library's. us, weights out of
+    cache, library / this. Up to 16 rows and a width that fills the chip, uncut (8 rows):
+    bf16 4096 -> 28672 60.2 / 41.0, 4096 -> 16384 32.1 / 23.5, 8192 -> 24576 82 / 71, 4096 ->
+    128256 187 / 173, 8192 -> 57344 172 / 158, 2304 -> 87808 136 / 80; but 1792 -> 56320 38.6
+    / 39.8, 2304 -> 256000 207 / 218; fp8 4096 -> 28672 31.7 / 23.6, 4096 -> 16384 26.4 /
+    14.0, 4096 -> 128256 112 / 94, but 9472 -> 59648 102 / 110, 1536 -> 116992 39 / 41.
+    Beyond 40000 columns only where rows lie whole 4 KB apart, or the CUs have even
+    shares of the columns' tiles (bf16 2304 -> 49152 48.9 / 43.7, but 49536 at 13 rows 43.3 /
+    50.8; fp8 1920 -> 49152 20.6 / 20.0, 53504 21.7 / 23.1), or they are so many that the last
+    share counts little. Over 308 products the 200 chosen took 0.74 of the time, 1.10 at
+    worst; of 130 others beside 49152 and 65536 columns 0.87, 1.13 at worst.
+    fp8 from 8192 columns on up to 12 rows, cut along K (6656 -> 9216 38 / 19, 8192 -> 8192
+    16 rows 16.4 / 21.3); bf16 of such widths not (7680 -> 14848 45 / 52). Rows
+    under 256 bytes stay: one launch against another (128 -> 65536 fp8 5.4 / 5.1).
+    Very long rows, which the library does not cut: 32256 -> 2048 83 / 32 at 8 rows, 127 /
+    52 at 96. It does at 16384, where the line lies by a kernel that took a third longer
+    (-> 1024 bf16 16 rows 21.0 / 16.4, fp8 64 rows 26.4 / 14.5; left to the library: bf16 48
+    rows 21.3 / 19.2, -> 2048 fp8 96 rows 21.6 / 17.5)."""
     if K >= 8 * N and K >= 16384:
         return K > 16384 or M <= (64 if fp8 else 32)
-    if M > 16 or N > 65536 or (N > 32768 and N % 16384) or K * (1 if fp8 else 2) < 256:
+    if M > 16 or K * (1 if fp8 else 2) < 256:
         return False
+    if N < 16384:
+        return fp8 and N >= 8192 and M <= 12
+    if N <= 40000 or _even_rows(K, fp8):
+        return True
+    even_shares = N % 16384 == 0 and N <= 65536
     if fp8:
-        return N >= 16384 and K <= 8192
-    return N >= 16384 and K <= 1024 or N > 16384 and K <= (6144 if M <= 8 else 4096)
-
-
-def _streams(M: int, N: int, K: int, fp8: bool) -> bool:
-    return _few_rows_better(M, N, K, fp8) or _streams_better(M, N, K, fp8)
+        return K <= 1024 or even_shares and K <= 8192
+    return 65536 <= N < 200000 or even_shares and K <= (6144 if M <= 8 else 4096)
 
 
 def _tiled_operands(x, weight) -> bool:
@@ -561,17 +556,17 @@ def tiled_gated(x, weight, gelu=False):
 
 def gated(x, weight, gelu=False):
     """What tiled_gated computes, also up to 96 rows: by the weight-streaming kernel or
-    the tiled one where linear has the product from them (28672 x 4096 one row: product
-    41.2 us, this 42.0, the activation's launch 4.7); None where two launches are
-    faster."""
+    the tiled one where linear has the product, uncut, from them (28672 x 4096 one row:
+    product 41.2 us, this 42.0, the activation's launch 4.7); None where two launches
+    are faster."""
     (M, K), N = x.shape, weight.shape[0]
     if M > 96:
         return tiled_gated(x, weight, gelu)
     if x.dtype != torch.bfloat16 or weight.dim() != 2 or N * K * 2 >= 2**31:
         return None
     if (
-        N >= 8192
-        and _few_rows_better(M, N, K, fp8=False)
+        M <= 16 and N >= 16384  # (uncut)
+        and _streams_better(M, N, K, fp8=False)
         and not observed(x, weight)
         and _skinny_operands(x, weight)
     ):
@@ -674,7 +669,7 @@ def linear(x, weight):
         x.dim() == weight.dim() == 2
         and x.shape[0] <= 96
         and x.is_cuda
-        and _streams(x.shape[0], *weight.shape, fp8=False)
+        and _streams_better(x.shape[0], *weight.shape, fp8=False)
         and x.dtype == torch.bfloat16
         and not observed(x, weight)
         and _skinny_operands(x, weight)
@@ -700,7 +695,7 @@ def linear_fp8(xq, x_scale, weight, w_scale, bias=None, out=None):
     [N, K] e4m3, x_scale [M], w_scale [1, N]; into `out` (dense rows) if given."""
     if (
         xq.shape[0] <= 96
-        and _streams(xq.shape[0], *weight.shape, fp8=True)
+        and _streams_better(xq.shape[0], *weight.shape, fp8=True)
         and not observed(xq, weight)
         and _skinny_operands(xq, weight)
         and _row_and_column_scales(xq, weight, x_scale, w_scale)

@@ -117,7 +117,7 @@ def test_what_the_streaming_product_does_not_take_goes_to_the_library(M, N, K, m
     """The forms of scales, bias and result that it has no part in give what the
     library gives for them; the usual ones are its own."""
     x, w, sx, sw = _fp8_product(M, N, K)
-    assert ops._streams(M, N, K, fp8=True)
+    assert ops._streams_better(M, N, K, fp8=True)
     calls = []
     own = ops._C.skinny_linear
     monkeypatch.setattr(ops._C, "skinny_linear", lambda *a: calls.append(a) or own(*a))

@@ -7,32 +7,46 @@ from kubeai_amd.ops import _streams_better, sums_better
 
 @pytest.mark.parametrize("M,N,K,fp8,better", [
     # wide weights: library / streaming, us
-    (8, 28672, 4096, False, True),    # 59.9 / 47.6
-    (16, 18432, 2304, False, True),   # 50.6 / 25.7
-    (8, 32256, 2048, False, True),    # 34.5 / 31.4
-    (1, 16384, 512, False, True),     # 11.5 / 6.5
-    (8, 16384, 4096, False, False),   # 33.4 / 34.8
-    (1, 16384, 8192, False, False),   # 64.7 / 67.7
-    (8, 24576, 8192, False, False),   # 83.8 / 91.8
-    (16, 22528, 6144, False, False),  # 67.4 / 75.5
-    (8, 20480, 6144, False, True),    # 104 / 64
-    (8, 36864, 8192, False, False),   # 145 / 160
-    (8, 65536, 4096, False, True),    # 123 / 107
-    (8, 16384, 4096, True, True),     # 27.9 / 20.3
-    (16, 30720, 8192, True, True),    # 66 / 57
-    (8, 36864, 4096, True, False),    # 41.4 / 42.7
-    (8, 65536, 128, True, False),     # 5.6 / 6.7
-    (17, 28672, 4096, True, False),   # 29.4 / 30.7
-    (8, 128256, 4096, False, False),  # 192 / 198
+    (8, 28672, 4096, False, True),    # 60.2 / 41.0
+    (16, 18432, 2304, False, True),   # 50.4 / 22.3
+    (8, 32256, 2048, False, True),    # 32.5 / 25.0
+    (1, 16384, 512, False, True),     # 11.5 / 5.8
+    (8, 16384, 4096, False, True),    # 32.1 / 23.5
+    (1, 16384, 8192, False, True),    # 61.2 / 46.9
+    (8, 24576, 8192, False, True),    # 81.9 / 70.6
+    (16, 22528, 6144, False, True),   # 64.2 / 60.3
+    (8, 20480, 6144, False, True),    # 103 / 53
+    (8, 36864, 8192, False, True),    # 132 / 116
+    (8, 65536, 4096, False, True),    # 125 / 91
+    (8, 16384, 4096, True, True),     # 26.4 / 14.0
+    (16, 30720, 8192, True, True),    # 61.5 / 44.4
+    (8, 36864, 4096, True, True),     # 38.2 / 32.5
+    (8, 65536, 128, True, False),     # 5.4 / 5.1
+    (17, 28672, 4096, True, False),   # (the tiled product's)
+    (8, 128256, 4096, False, True),   # 187 / 173
+    (8, 256000, 2304, False, False),  # 207 / 218
+    # even shares of the columns, and beside them
+    (8, 49152, 1280, False, True),    # 31.7 / 26.3
+    (8, 49152, 2304, False, True),    # 48.9 / 43.7
+    (13, 49536, 2304, False, False),  # 43.3 / 50.8
+    (10, 49152, 4320, False, False),
+    (8, 49152, 5120, True, True),     # 49.2 / 48.5
+    (13, 53504, 1920, True, False),   # 21.7 / 23.1
+    (8, 81920, 2304, True, False),
+    (12, 51008, 704, True, True),     # 19.4 / 10.9
+    # cut along K
+    (8, 9216, 6656, True, True),      # 38 / 19
+    (16, 8192, 8192, True, False),    # 16.4 / 21.3
+    (8, 14848, 7680, False, False),   # 45 / 52
     # long rows
-    (32, 2048, 32256, False, True),   # 111 / 38
-    (96, 4096, 40960, True, True),    # 140 / 58
-    (16, 1024, 16384, False, True),   # 21.1 / 19.4
-    (48, 1024, 16384, False, False),  # 21.0 / 28.7
-    (33, 512, 16384, False, False),   # 19.0 / 27.7
-    (64, 1024, 16384, True, True),    # 26.2 / 19.9
-    (96, 2048, 16384, True, False),   # 21.2 / 22.2
-    (8, 4096, 14336, False, False),   # 27 / 29
+    (32, 2048, 32256, False, True),   # 111 / 32
+    (96, 4096, 40960, True, True),    # 139 / 55
+    (16, 1024, 16384, False, True),   # 21.0 / 16.4
+    (48, 1024, 16384, False, False),  # 21.3 / 19.2
+    (33, 512, 16384, False, False),   # 18.7 / 16.8
+    (64, 1024, 16384, True, True),    # 26.4 / 14.5
+    (96, 2048, 16384, True, False),   # 21.6 / 17.5
+    (8, 4096, 14336, False, False),   # 25.8 / 27.2
 ])
 def test_streaming_products(M, N, K, fp8, better):
     assert _streams_better(M, N, K, fp8) is better

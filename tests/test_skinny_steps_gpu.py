@@ -109,6 +109,16 @@ def test_activation_goes_with_few_rows(T, gelu):
         assert ops.gated(x.requires_grad_(), w, gelu) is None
 
 
+def test_activation_goes_where_linear_streams():
+    for N, K, here in ((49152, 1280, True), (16384, 8192, True), (16384 - 16, 2048, False)):
+        assert ops._streams_better(8, N, K, fp8=False) is here
+        x, w = _operands(8, N, K, N)
+        y = ops.gated(x, w)
+        assert (y is not None) is here
+        if here:
+            _near_gated(y, x, w, False)
+
+
 @pytest.mark.parametrize("M,N,K,fp8,better", [
     # us, library / streaming
     (8, 16384, 4096, False, True),     # 32.1 / 23.7
@@ -123,4 +133,4 @@ def test_activation_goes_with_few_rows(T, gelu):
     (17, 28672, 4096, True, False),    # (the tiled product's)
 ])
 def test_rule(M, N, K, fp8, better):
-    assert ops._few_rows_better(M, N, K, fp8) is better
+    assert ops._streams_better(M, N, K, fp8) is better
