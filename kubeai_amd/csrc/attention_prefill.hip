@@ -45,7 +45,7 @@
 //   512 new tokens behind 3584                          414 -> 100
 //   six turns of 62-100 behind 365-587, 4 padding runs   72 ->  23
 //   heads 64/8 x 128, 4096                              927 -> 360
-//   heads 8/4 x 256, 3029 + 2145, cap, window 4096     1574 -> 148 (380 TF/s)
+//   heads 8/4 x 256, 3029 + 2145, cap, window 4096     1574 -> 146 (385 TF/s)
 //
 // Fragment layouts:
 //   A[M=32][K=16]: lane l holds A[l&31][(l>>5)*8 + j], j=0..7
@@ -411,7 +411,8 @@ DEV_INLINE void each(const F& f) {
 // reads of V, then of the next K, into registers; the softmax, no step of which waits for
 // another of its slot; registers to LDS (three places for K and V each), the next
 // tiles' loads and the blocks after them.
-//   heads 8/4 x 256, 3029 + 2145: 231 us -> 115, capped 262 -> 143; 500 capped 41 -> 32
+//   heads 8/4 x 256, 3029 + 2145: 231 us -> 115, capped, no window 262 -> 141; 500 capped
+// 41 -> 32
 // The same at head size 128, 64 rows a wave: 8192 as long as with two waves a SIMD and
 // half the rows (611 us, 606: more clocks at a higher rate; the card's power), shorter
 // prompts 1.3 times.

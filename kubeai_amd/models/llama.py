@@ -320,25 +320,28 @@ class MoEMLP(nn.Module):
     slower one, the library's on each expert's slice, after one look at the
     experts' row counts."""
 
-    #: one pass of 8 experts of 14336 x 4096, us, weight-streaming (before its loads
-    #: went without branches: 4 % of a decode step of 40 tokens since) / tiled /
-    #: every expert's tokens asked for one after the other: fp8 128 tokens
-    #: 353/383/722, 512 819/470/1361, 2048 2413/1015/2006; bf16 128
-    #: 602/684/1159, 512 1397/871/1614, 2048 4223/1708/2488 (streaming reads
-    #: an expert's weights again for every 96 of its rows). Up to 256 tokens any
+    #: one pass of 8 experts of 14336 x 4096, us, weight-streaming / tiled: fp8 128
+    #: tokens 360/305, 256 445/335; bf16 627/548, 715/582; every expert's tokens
+    #: asked for one after the other took 722 and 1159 at 128. (Streaming reads an
+    #: expert's weights again for every 96 of its rows.) Up to 256 tokens any
     #: routing may be recorded in a graph, so no row counts come to the host.
     GROUPED_MAX_TOKENS = 256
 
     #: Above these the tiled product has the step where it takes both
     #: projections. us, streaming / tiled, tokens spread evenly (half of them
-    #: alike): fp8 160 tokens 364/389 (478/416), 192 416/393 (549/421), 256
-    #: 443/404 (593/418); 8 x 7168 x 2048 160 140/160 (188/167), 192 160/158
-    #: (209/171); 16 x 6400 x 4096 192 333/319 (401/328); 32 x 1408 x 2048, 4 a
-    #: token, 192 115/118 (133/124); 4 x 3584 x 1024 160 71/78 (93/81), 192 90/80
-    #: (99/77). bf16 192 681/704 (936/752), 224 704/711 (970/739), 256 723/719
-    #: (1017/741); 8 x 7168 x 2048 224 257/266 (365/294), 256 268/270 (371/298);
-    #: 16 x 6400 x 4096 256 591/570 (802/655); 32 x 1408 x 2048 256 176/179
-    #: (236/203).
+    #: alike): fp8 8 x 14336 x 4096 160 tokens 371/319 (436/356), 192 413/321
+    #: (521/375), 256 445/335 (519/395); 8 x 7168 x 2048 160 121/116 (160/122), 192
+    #: 137/116 (180/124); 16 x 6400 x 4096 160 301/304 (380/325), 192 313/305
+    #: (368/325); 32 x 1408 x 2048, 4 a token, 160 104/105 (133/115), 192 108/107
+    #: (123/117); 4 x 3584 x 1024 160 64/46 (81/47), 192 76/47 (87/54). bf16 8 x 14336 x
+    #: 4096 224 688/574 (840/714), 256 715/582 (864/692); 8 x 7168 x 2048 224 209/194
+    #: (268/207), 256 214/198 (286/210); 16 x 6400 x 4096 224 553/507 (614/528), 256
+    #: 568/505 (673/526); 32 x 1408 x 2048 224 163/164 (208/177), 256 165/165
+    #: (200/174). The lines are where the two met before experts' tiles went by the
+    #: costs of one matrix. The tiled kernel is the faster one from fewer tokens on
+    #: now, down to 128 at most of these sizes; the lines have not been moved since.
+    #: (The kernels need not round alike, and in a routed model that can move a token
+    #: whose scores all but tie.)
     TILED_ABOVE_FP8 = 160
     TILED_ABOVE_BF16 = 224
 

@@ -317,16 +317,19 @@ def sums_better(
     are read in half the time and leave less to gain. (In a whole decode step of 40
     rows in fp8 the sums of the products around attention gain 3 us a layer that
     pairs timed by themselves do not show.) us, weights out of cache,
-    library / this: bf16 4096 -> 4096 8 rows 18.7 / 12.8, 96 rows 25.3 / 19.7;
-    14336 -> 4096 8 rows 30.2 / 28.8, 40 rows 43.0 / 35.2; 4096 -> 6144 8 rows 18.8
-    / 16.3 (rotation), 64 rows 21.3 / 21.9; 8192 -> 8192 34.9 / 38.3; 8192 -> 1024
-    8 rows 14.7 / 10.9, 40 rows 15.0 / 12.3. fp8 4096 -> 4096 16 rows 15.8 / 10.9,
-    64 rows 16.3 / 15.1; 14336 -> 4096 40 rows 26.9 / 21.2; 8192 -> 8192 8 rows
-    47.3 / 23.2, 16 rows 21.6 / 24.2; 512 -> 4096 8.3 / 6.9. (The line was drawn where
-    this form and its reader were 1 to 4 us slower: a few products that it leaves to the
-    library, as 8192 -> 1024 of 40 rows, are this one's now. Over 3576 and 1656
-    products of 512 to 28672 columns and rows with either reader the chosen ones took
-    0.72 and 0.80 of the library's time then, the worst 1.2.)
+    library / this: bf16 4096 -> 4096 8 rows 18.8 / 13.0, 96 rows 25.5 / 19.6;
+    14336 -> 4096 8 rows 29.3 / 28.0, 40 rows 39.8 / 33.0; 4096 -> 6144 8 rows 17.5
+    / 16.0 (rotation), 64 rows 21.0 / 21.9; 8192 -> 8192 33.5 / 39.4; 8192 -> 1024
+    8 rows 14.8 / 10.7. fp8 4096 -> 4096 16 rows 16.1 / 11.0; 14336 -> 4096 40 rows
+    24.9 / 21.4; 8192 -> 8192 8 rows 47.0 / 23.8, 16 rows 20.7 / 24.2.
+    The line was drawn where this form and its reader were 1 to 4 us slower than they
+    are, so it is a cautious one: of 22943 products at random (1 to 96 rows, 512 to
+    12288 columns, K 512 to 28672, either reader) the 13496 that this rule and
+    few_tiled_better choose take 0.52 of the library's time, 1.29 at worst (174 of them
+    more than 1.05), and of the other 9447 two thirds would be 5 % or more faster as
+    sums, 0.83 of the time in all: fp8 4096 -> 4096 64 rows 16.6 / 15.4, 512 -> 4096 8 rows
+    8.6 / 7.2. (bf16 8192 -> 1024 of 40 rows, not this rule's either, few_tiled_better
+    has: 15.3, streaming 12.4, tiled 14.3.)
     eager: the step is not replayed from a graph, so the host's launches bound it
     while the weights are small, and the library's call takes 10 us of the host
     more (80 tokens of a prompt on 8 layers of 4096: 1796 us / 1493)."""

@@ -58,19 +58,19 @@ def test_streaming_products(M, N, K, fp8, better):
     (96, 4096, 4096, False, False, True),    # 25.3 / 19.3
     (40, 4096, 14336, False, False, True),   # 39.4 / 32.1
     (8, 1024, 8192, False, False, True),     # 14.6 / 12.3
-    (40, 1024, 8192, False, False, False),   # 15.1 / 17.1
+    (40, 1024, 8192, False, False, False),   # 15.3 / 12.4: the tiled product's sums
     (8, 8192, 8192, False, False, False),    # 34.7 / 41.4
     (17, 12288, 8192, False, False, False),  # 45.8 / 55.1
     (96, 5120, 2048, False, False, False),   # 17.2 / 19.6
     (8, 10240, 1024, False, False, True),    # 0.93 of the library's
     (8, 4608, 28672, False, False, True),    # 0.47
     (16, 4096, 4096, True, False, True),     # 15.8 / 13.3
-    (64, 4096, 4096, True, False, False),    # 16.4 / 18.3
+    (64, 4096, 4096, True, False, False),    # 16.6 / 15.4: a cautious line
     (40, 4096, 14336, True, False, True),    # 25.1 / 22.8
     (8, 8192, 8192, True, False, True),      # 47.5 / 26.6
     (16, 8192, 8192, True, False, False),    # 20.6 / 27.2
     (40, 8192, 8192, True, False, False),    # 22.9 / 28.5
-    (8, 4096, 512, True, False, False),      # 8.2 / 8.8
+    (8, 4096, 512, True, False, False),      # 8.6 / 7.2: the same
     (96, 2048, 2048, True, False, False),    # 11.7 / 11.5
     (40, 2304, 9216, True, False, True),     # 0.98
     # with the rotation and cache write
