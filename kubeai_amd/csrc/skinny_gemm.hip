@@ -200,6 +200,10 @@ __launch_bounds__(NW * WAVE_SIZE) __global__ void skinny_kernel(
   do {
 #pragma unroll
     for (int j = 0; j < MT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // offsets are 32 bits: where experts' rows lie in order, from this pass's first on
+    const bool in_rows = GROUPED && !grp.src;
+    const char* xb = in_rows ? x + (int64_t)m0 * ldx : x;
+    const int xn = in_rows ? (min(M, MT * 16) - 1) * ldx + KB : xbytes;
 #pragma unroll
     for (int i = 0; i < NX; ++i) {
       // 16-byte unit u of row r lies at u ^ (r & 7): made by the choice of source
@@ -207,9 +211,9 @@ __launch_bounds__(NW * WAVE_SIZE) __global__ void skinny_kernel(
       xk[i] = ((at % UPR) ^ (row & 7)) * 16;
       xo[i] = kNowhere;
       if (row < M) {
-        int from = m0 + row;
+        int from = row;
         if constexpr (GROUPED) {
-          if (grp.src) from = grp.src[from];
+          if (!in_rows) from = grp.src[m0 + row];
         }
         xo[i] = from * ldx + xk[i];
       }
@@ -220,7 +224,7 @@ __launch_bounds__(NW * WAVE_SIZE) __global__ void skinny_kernel(
       const int k = k0 + next * kStep, on = ahead < steps;
 #pragma unroll
       for (int i = 0; i < NX; ++i)
-        load_lds16(x, on ? xbytes : 0, xs + P * PLACE + (wave * NX + i) * 1024,
+        load_lds16(xb, on ? xn : 0, xs + P * PLACE + (wave * NX + i) * 1024,
                    xk[i] < k1 - k ? xo[i] : kNowhere, k);
 #pragma unroll
       for (int c = 0; c < CH; ++c)
@@ -528,21 +532,20 @@ void skinny_experts(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   }
   const int R = y.size(0);
   if (R == 0) return;
-  if (x.size(0) * x.stride(0) * es >= (1ll << 31)) {  // offsets are 32 bits
-    if (src.has_value()) {
-      if (fp8) sx = sx->reshape(-1).index_select(0, *src);
-      x = x.view(torch::kUInt8).index_select(0, *src).view(x.scalar_type());
-      src = c10::nullopt;
-    }
-    x = x.contiguous();
-    TORCH_CHECK(x.numel() * es < (1ll << 31));
+  if (src.has_value() && x.size(0) * x.stride(0) * es >= (1ll << 31)) {
+    // offsets are 32 bits: the rows in the order of the experts
+    if (fp8) sx = sx->reshape(-1).index_select(0, *src);
+    x = x.view(torch::kUInt8).index_select(0, *src).view(x.scalar_type());
+    src = c10::nullopt;
   }
+  if (!src.has_value()) x = near_rows(x);
   const float* sxp = fp8 ? sx->data_ptr<float>() : nullptr;
   const float* swp = fp8 ? sw->data_ptr<float>() : nullptr;
   const Groups g{begin.data_ptr<int32_t>(),
                  src.has_value() ? src->data_ptr<int32_t>() : nullptr};
   const dim3 grid((N + kNW * 16 - 1) / (kNW * 16), 1, E);
-  const int ldx = x.stride(0) * es, xbytes = (x.size(0) - 1) * ldx + KB;
+  const int ldx = x.stride(0) * es;
+  const int xbytes = src.has_value() ? (x.size(0) - 1) * ldx + KB : 0;  // (else by the pass)
   auto stream = c10::hip::getCurrentHIPStream().stream();
   auto go = [&](auto f, auto mt) {
     hipLaunchKernelGGL((skinny_kernel<decltype(f)::value, decltype(mt)::value, true, 0, kNW>),

@@ -243,3 +243,32 @@ def test_a_router_that_is_not_finite_reaches_the_output():
             x = torch.randn(T, 128, device=DEV, dtype=torch.bfloat16)
             assert m._grouped(x) is not None or T > m.GROUPED_MAX_TOKENS
             assert m(x).isnan().all()
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("gathered", [False, True])
+def test_experts_over_more_than_2_gib_of_rows(fp8, gathered):
+    rows, N, K = 270_000, 64, 8192 if fp8 else 4096
+    torch.manual_seed(3)
+    x = torch.empty(rows, K, device=DEV, dtype=torch.bfloat16).normal_()
+    w = torch.randn(2, N, K, device=DEV, dtype=torch.bfloat16)
+    sx = sw = None
+    if fp8:
+        x, w = x.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn)
+        sx, sw = torch.rand(rows, device=DEV) + 0.5, torch.rand(2, N, device=DEV) + 0.5
+    if gathered:
+        src = torch.tensor([rows - 1, 0, 5, rows - 2, 131_072] * 30, device=DEV, dtype=torch.int32)
+        begin, at = (0, 70, 150), src.long()
+    else:
+        src, begin, at = None, (0, 97, rows), torch.arange(rows, device=DEV)
+    y = torch.empty(begin[-1], N, device=DEV, dtype=torch.bfloat16)
+    ops._C.skinny_experts(y, x, w, sx, sw,
+                          torch.tensor(begin, dtype=torch.int32, device=DEV), src)
+    for e in range(2):
+        lo, hi = begin[e], begin[e + 1]
+        for part in (slice(lo, min(lo + 200, hi)), slice(max(lo, hi - 200), hi)):
+            a, b = x[at[part]].double(), w[e].double()
+            s = sx[at[part], None].double() * sw[e].double() if fp8 else 1.0
+            want, size = (a @ b.T) * s, (a.abs() @ b.abs().T) * s
+            # one rounding to bf16; fp32 sums
+            assert ((y[part].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * size).all()
