@@ -44,11 +44,15 @@
 //                 5.3 -> 5.4; 14336 -> 4096 15.4 -> 13.4; 2304 -> 18432 16.3 -> 12.5
 //   fp8, 40 rows  4096 -> 6144 9.9 -> 9.8; 4096 -> 4096 7.2 -> 6.7
 // The grouped form multiplies every expert's rows of a mixture in one launch,
-// x rows gathered by index. 8 experts, 80 rows, 28672 x 4096 and 4096 x 14336: fp8
-// 184 + 94 us -> 170 + 89 (5.5 and 5.3 TB/s), bf16 359 + 193 -> 320 + 179; 32 experts of
-// 1408 x 2048 bf16 44 -> 40.
+// x rows gathered by index, its columns in order (below). 8 experts, 80 rows, 28672 x 4096
+// and 4096 x 14336: fp8 183 + 93 us -> 177 + 89, bf16 353 + 198 -> 354 + 194. The experts
+// that have rows are counted off by the workgroups: with a place for every expert, and
+// all workgroups in place at once, some CUs had two to four of them and others none (16
+// experts of 4096 x 6400, bf16, 4 rows 88 -> 44 us, 16 rows 136 -> 115; 32 of 2816 x 2048 16
+// rows 53 -> 41).
 #include <torch/extension.h>
 
+#include <cmath>
 #include <type_traits>
 
 #include "common.h"
@@ -145,9 +149,27 @@ DEV_INLINE void barrier() {
   in_order();
 }
 
+// the n-th of the experts that have rows, -1 if there are fewer
+DEV_INLINE int expert_with_rows(const int32_t* begin, int experts, int n, int lane) {
+  for (int at = 0; at < experts; at += WAVE_SIZE) {
+    const int i = min(at + lane, experts - 1);
+    const bool has = at + lane < experts && begin[i + 1] > begin[i];
+    const uint64_t mask = __builtin_amdgcn_ballot_w64(has);
+    const int count = __builtin_popcountll(mask);
+    if (n < count) {
+      const int before = __builtin_amdgcn_mbcnt_hi(
+          (uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+      return at + __builtin_ctzll(__builtin_amdgcn_ballot_w64(has && before == n));
+    }
+    n -= count;
+  }
+  return -1;
+}
+
 // MT: 16-row tiles of x. part != null: raw sums of this K range.
-// GROUPED: blockIdx.z is the expert; its rows are taken MT * 16 at a time (W
-// is read again for each such pass: the host picks MT so that one is usual).
+// GROUPED: blockIdx.z is the place among the experts with rows; an expert's rows are
+// taken MT * 16 at a time (W is read again for each such pass: the host picks MT so
+// that one is usual).
 // ACT (bf16): silu (1) or tanh-gelu (2) of column n times column n + N / 2, in fp32,
 // rounded once; a wave has 8 columns of either half.
 template <bool FP8, int MT, bool GROUPED, int ACT, int NW>
@@ -181,12 +203,13 @@ __launch_bounds__(NW * WAVE_SIZE) __global__ void skinny_kernel(
   int m0 = 0, M = M_all;  // this pass's first row and the rows from it on
   int m_end = M_all;
   if constexpr (GROUPED) {
-    m0 = grp.begin[blockIdx.z];
-    m_end = grp.begin[blockIdx.z + 1];
-    w += (int64_t)blockIdx.z * N * KB;
-    if (sw) sw += (int64_t)blockIdx.z * N;
+    const int e = expert_with_rows(grp.begin, gridDim.z, blockIdx.z, lane);
+    if (e < 0) return;  // whole workgroup
+    m0 = grp.begin[e];
+    m_end = grp.begin[e + 1];
+    w += (int64_t)e * N * KB;
+    if (sw) sw += (int64_t)e * N;
     M = m_end - m0;
-    if (M <= 0) return;  // whole workgroup
   }
   const char* wb = w + (int64_t)n0 * KB;
   const int left = max(0, min(cols - n0, RW));  // rows of w
@@ -543,24 +566,38 @@ void skinny_experts(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   const float* swp = fp8 ? sw->data_ptr<float>() : nullptr;
   const Groups g{begin.data_ptr<int32_t>(),
                  src.has_value() ? src->data_ptr<int32_t>() : nullptr};
-  const dim3 grid((N + kNW * 16 - 1) / (kNW * 16), 1, E);
   const int ldx = x.stride(0) * es;
   const int xbytes = src.has_value() ? (x.size(0) - 1) * ldx + KB : 0;  // (else by the pass)
   auto stream = c10::hip::getCurrentHIPStream().stream();
-  auto go = [&](auto f, auto mt) {
-    hipLaunchKernelGGL((skinny_kernel<decltype(f)::value, decltype(mt)::value, true, 0, kNW>),
-                       grid, dim3(kNW * WAVE_SIZE), 0, stream,
+  auto go = [&](auto f, auto mt, auto waves) {
+    constexpr int NW = decltype(waves)::value;
+    const dim3 grid((N + NW * 16 - 1) / (NW * 16), 1, E);
+    hipLaunchKernelGGL((skinny_kernel<decltype(f)::value, decltype(mt)::value, true, 0, NW>),
+                       grid, dim3(NW * WAVE_SIZE), 0, stream,
                        (ushort*)y.data_ptr(), nullptr, (const char*)x.data_ptr(),
                        (const char*)w.data_ptr(), sxp, swp, nullptr, R, N, KB,
                        ldx, xbytes, KB, 1, g);
   };
   // rows per expert if they are spread evenly; half as many again fit a pass
   const int mean = (R + E - 1) / E;
+  // Few rows whose experts (as many as R rows at random reach) have fewer than four
+  // workgroups a CU: two waves each, so that the CUs' shares are more even. us, with
+  // branches in the loop and four waves / four / two: 8 of 4096 x 14336 bf16 8 rows 134 /
+  // 164 / 132, 16 rows 171 / 189 / 176, fp8 8 rows 68 / 78 / 65; but 8 of 28672 x 4096
+  // bf16 16 rows 350 / 348 / 359. Over 883 products (up to 64 experts) of under four a
+  // CU 1.27 times as fast as with branches, 0.88 at worst (four waves 1.16), over 342 of
+  // more 1.02 (four 1.04).
+  const double reached = E * (1.0 - std::pow(1.0 - 1.0 / E, R));
+  const bool thin = reached * ((N + kNW * 16 - 1) / (kNW * 16)) < 4 * 256;
+  constexpr std::integral_constant<int, 2> two;
+  constexpr std::integral_constant<int, kNW> four;
   auto tiles = [&](auto f) {
-    if (mean <= 8) go(f, std::integral_constant<int, 1>{});
-    else if (mean <= 22) go(f, std::integral_constant<int, 2>{});
-    else if (mean <= 44) go(f, std::integral_constant<int, 4>{});
-    else go(f, std::integral_constant<int, 6>{});
+    constexpr std::integral_constant<int, 1> one;
+    if (mean <= 8 && thin) go(f, one, two);
+    else if (mean <= 8) go(f, one, four);
+    else if (mean <= 22) go(f, two, four);
+    else if (mean <= 44) go(f, four, four);
+    else go(f, std::integral_constant<int, 6>{}, four);
   };
   if (fp8) tiles(std::true_type{});
   else tiles(std::false_type{});

@@ -272,3 +272,35 @@ def test_experts_over_more_than_2_gib_of_rows(fp8, gathered):
             want, size = (a @ b.T) * s, (a.abs() @ b.abs().T) * s
             # one rounding to bf16; fp32 sums
             assert ((y[part].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * size).all()
+
+
+@pytest.mark.parametrize("E,R,N", [(1, 3, 20), (5, 4, 100), (8, 24, 28672), (64, 9, 68),
+                                   (65, 200, 36), (130, 40, 260), (130, 1, 16), (8, 300, 132)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_experts_without_rows(E, R, N, fp8):
+    """Whichever experts have rows, two waves a workgroup and four, more experts than a
+    wave has lanes; rows behind the last expert's stay as they are."""
+    K = 192
+    torch.manual_seed(E + R)
+    w = torch.randn(E, N, K, device=DEV, dtype=torch.bfloat16)
+    x = torch.randn(R + 2, K, device=DEV, dtype=torch.bfloat16)
+    sx = sw = None
+    if fp8:
+        x, w = x.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn)
+        sx, sw = torch.rand(R + 2, device=DEV) + 0.5, torch.rand(E, N, device=DEV) + 0.5
+    for own in (range(E), [0], [E - 1], [E // 2, E - 1], [i for i in (0, 63, 64) if i < E]):
+        own = list(own)
+        counts = torch.bincount(
+            torch.tensor(own)[torch.randint(len(own), (R,))], minlength=E)
+        begin = [0] + counts.cumsum(0).tolist()
+        y = torch.full((R + 2, N), 7.0, device=DEV, dtype=torch.bfloat16)
+        ops._C.skinny_experts(y, x, w, sx, sw,
+                              torch.tensor(begin, dtype=torch.int32, device=DEV), None)
+        assert (y[R:] == 7).all()
+        for e in range(E):
+            rows = slice(begin[e], begin[e + 1])
+            a, b = x[rows].double(), w[e].double()
+            s = sx[rows, None].double() * sw[e].double() if fp8 else 1.0
+            want, size = (a @ b.T) * s, (a.abs() @ b.abs().T) * s
+            # one rounding to bf16; fp32 sums
+            assert ((y[rows].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * size).all()
