@@ -23,7 +23,7 @@
 //    16-lane transposing read fall in disjoint banks.
 //  - head size 128: LDS is double-buffered, the next tile's global loads issue
 //    before this tile's compute; its cache blocks are looked up one tile earlier
-//    with scalar loads. Head size 256: paged_prefill_wide_kernel.
+//    with scalar loads. Head size 256 of more than a few keys: paged_prefill_wide_kernel.
 //  - the grid numbers the query tiles of the whole packed step (find_tile),
 //    kv head fastest: a step of one long prompt and many padding runs
 //    launches no empty rows of blocks, and with 8 kv heads each XCD works on
@@ -64,6 +64,12 @@ namespace {
 constexpr int kBS = 16;  // cache block size (tokens)
 constexpr int kQB = 32;  // query rows per wave
 constexpr int kNW = 4;   // waves per workgroup
+// Head size 256, at most so many keys a workgroup: one tile after the other instead of
+// three under way at a time, whose beginning and end take longer (us, that / one after the
+// other: 4 tokens 10.4 / 6.2, 20 10.8 / 7.1, 52 + 64 15.5 / 13.6). Over 399 steps of 1 to 40
+// runs one after the other takes 0.64 of the time up to 32 keys, 0.85 up to 96, 0.96 up
+// to 160, 0.99 up to 192, 1.04 up to 288 and 1.28 above 600.
+constexpr int kFewKeys = 192;
 
 typedef __attribute__((ext_vector_type(8))) short bf16x8;
 typedef __attribute__((ext_vector_type(4))) short bf16x4;
@@ -89,11 +95,11 @@ DEV_INLINE int find_tile(const int32_t* start, int n_seq, int size, int n,
   return lo;
 }
 
-// Head size 128. CT = cache element type: ushort (bf16) or unsigned char (fp8 e5m2,
-// converted to bf16 while staging). CAP: capped scores. WIN: keys in
-// (pos - window, pos] only.
-template <int GB, typename CT, bool WIN, bool CAP>
-__launch_bounds__(kNW * WAVE_SIZE, 2) __global__
+// Head size 128, and 256 where no row has many keys (kFewKeys). CT = cache element
+// type: ushort (bf16) or unsigned char (fp8 e5m2, converted to bf16 while staging). CAP:
+// capped scores. WIN: keys in (pos - window, pos] only.
+template <int HD, int GB, typename CT, bool WIN, bool CAP>
+__launch_bounds__(kNW * WAVE_SIZE, HD == 128 ? 2 : 1) __global__
 void paged_prefill_kernel(
     ushort* __restrict__ out,          // [Tq, n_q, HD]
     const ushort* __restrict__ q,      // [Tq, n_q, HD], rows strided
@@ -105,8 +111,7 @@ void paged_prefill_kernel(
     const float scale, const float softcap, const int window,
     const int n_kv, const int G, const int n_seq, const int max_blocks,
     const int64_t q_stride, const int n_tiles_q) {
-  constexpr int HD = 128;
-  constexpr int KVB = 64;                   // keys per staged tile
+  constexpr int KVB = HD == 128 ? 64 : 32;  // keys per staged tile
   constexpr int NSUB = KVB / 32;
   constexpr int NBK = KVB / kBS;            // cache blocks per tile
   constexpr int RS = kNW / GB;              // row subtiles per workgroup
@@ -178,7 +183,7 @@ void paged_prefill_kernel(
   float m_run = -INFINITY, l_run = 0.f;  // l_run: this lane's half of the keys
 
   // ---- staging: thread's unit i is row (tid / UPR) + i * rows_per_pass ----
-  constexpr int RPP = kNW * WAVE_SIZE / UPR;  // rows per pass: 16
+  constexpr int RPP = kNW * WAVE_SIZE / UPR;  // rows per pass: 16 or 8
   const int st_row = threadIdx.x / UPR;
   const int st_unit = threadIdx.x % UPR;
   const int32_t* bt = block_tables + (int64_t)b * max_blocks;
@@ -278,6 +283,18 @@ void paged_prefill_kernel(
           s[sub] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k_frag, q_frag[c],
                                                            s[sub], 0, 0, 0);
         }
+
+      // one wave a SIMD has nobody to cover a read of K: four are kept ahead
+      if constexpr (HD == 256) {
+        constexpr int kMfma = 0x008, kLdsRead = 0x100, kAhead = 4;
+        __builtin_amdgcn_sched_group_barrier(kLdsRead, kAhead, 0);
+#pragma unroll
+        for (int c = 0; c < NC - kAhead; ++c) {
+          __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(kLdsRead, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(kMfma, kAhead, 0);
+      }
 
       // ---- mask, running maximum -----------------------------------------
       if constexpr (CAP) cap.apply(s, c2);
@@ -873,6 +890,9 @@ void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
   const int qr = kNW / GB * kQB;
   const int n_tiles_q = Tq / qr + B;  // see find_tile
   const int64_t blocks = (int64_t)n_tiles_q * (G / GB) * n_kv;
+  // at most, of a workgroup's rows
+  const int64_t keys =
+      std::min((int64_t)max_blocks * kBS, window > 0 ? window + qr : INT64_MAX);
   auto stream = c10::hip::getCurrentHIPStream().stream();
   const bool fp8_cache = k_cache.scalar_type() == torch::kFloat8_e5m2;
   auto launch = [&](auto kernel, auto ct, auto... more) {
@@ -898,15 +918,19 @@ void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
     using CT = decltype(ct);
     masks([&](auto win, auto cap) {
       constexpr bool W = decltype(win)::value, C = decltype(cap)::value;
-      if (hd == 256) {
+      auto heads = [&](auto hdv) {
+        constexpr int HD = decltype(hdv)::value;
+        if (GB == 1) launch(paged_prefill_kernel<HD, 1, CT, W, C>, ct);
+        else if (GB == 2) launch(paged_prefill_kernel<HD, 2, CT, W, C>, ct);
+        else launch(paged_prefill_kernel<HD, 4, CT, W, C>, ct);
+      };
+      if (hd == 128) {
+        heads(std::integral_constant<int, 128>{});
+      } else if (keys <= kFewKeys) {
+        heads(std::integral_constant<int, 256>{});
+      } else {
         const int rs_bits = GB == 4 ? 0 : GB == 2 ? 1 : 2;
         launch(paged_prefill_wide_kernel<CT, W, C>, ct, rs_bits);
-      } else if (GB == 1) {
-        launch(paged_prefill_kernel<1, CT, W, C>, ct);
-      } else if (GB == 2) {
-        launch(paged_prefill_kernel<2, CT, W, C>, ct);
-      } else {
-        launch(paged_prefill_kernel<4, CT, W, C>, ct);
       }
     });
   };

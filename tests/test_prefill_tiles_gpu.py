@@ -59,6 +59,19 @@ def test_windows(hd, window, softcap):
     _run([3, 100, 40], [130, 0, 64], 4, 2, hd, hd ** -0.5, window=window, softcap=softcap)
 
 
+@pytest.mark.parametrize("group", [1, 2, 8])
+@pytest.mark.parametrize("window", [0, 64, 65, 129, 161, 200, 300])
+@pytest.mark.parametrize("softcap,fp8", [(0.0, False), (20.0, False), (0.0, True)])
+def test_head_size_256_on_both_sides_of_192_keys(group, window, softcap, fp8):
+    """Up to 192 keys a workgroup (a window and the 32 to 128 rows behind it count as its
+    most) have a kernel of their own: the same from tables of 12 blocks, and of more."""
+    for lens, ctxs in [([64, 3, 33], [128, 189, 0]), ([65, 1], [128, 500]),
+                       ([3, 100, 130], [330, 0, 264])]:
+        _run(lens, ctxs, 2 * group, 2, 256, 0.07, window=window, softcap=softcap, fp8=fp8)
+    _run([40, 17], [0, 3], 2 * group, 2, 256, 0.07, window=window, softcap=softcap, fp8=fp8,
+         spare_blocks=13)
+
+
 @pytest.mark.parametrize("hd", [128, 256])
 def test_eight_bit_cache(hd):
     _run([70, 5], [33, 100], 8, 2, hd, hd ** -0.5, fp8=True)
@@ -136,8 +149,9 @@ def test_keys_that_are_not_finite(hd, softcap):
         assert torch.equal(got.isnan(), want.isnan())
 
 
-@pytest.mark.parametrize("window", [0, 50])
-@pytest.mark.parametrize("n,ctx", [(1, 0), (33, 31), (64, 0), (97, 100), (200, 17)])
+@pytest.mark.parametrize("window", [0, 50, 90])
+@pytest.mark.parametrize("n,ctx", [(1, 0), (33, 31), (64, 0), (97, 100), (200, 17), (97, 132),
+                                   (170, 251)])
 def test_maxima_that_grow_with_every_tile(n, ctx, window):
     """Head size 256, the sums rescaled in most iterations: each key's score is above
     the last one's, by 2^4 a tile of 32 keys. Odd and even numbers of tiles; windows
