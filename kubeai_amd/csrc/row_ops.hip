@@ -28,6 +28,7 @@
 
 namespace {
 
+constexpr int kCUs = 256;
 constexpr int kMaxH = 16384;     // bf16 norms
 constexpr int kMaxHFp8 = 32768;  // fp8 outputs
 
@@ -182,7 +183,8 @@ __launch_bounds__(VPT == 8 ? 512 : 1024) __global__ void rmsnorm_kernel(
 // hidden = residual + branch, out = norm of hidden, where branch is x or (FIRST)
 // the norm of x: what lies between two sublayers whose outputs are normed too.
 // Every step rounds to bf16 as the launches that it replaces did, so the bits
-// are the same. SUMS as above.
+// are the same (but for 257 to 1023 rows of more than 4096 values out of sums: the last
+// norm by itself adds its squares over more threads there). SUMS as above.
 // A row is read once, in place of two passes over it (norm; add and norm); us in a
 // model, separate launches / this: 5376 x 2304 35.1 / 20.9 (weights
 // asked for behind the sums 22.3).
@@ -308,12 +310,16 @@ __launch_bounds__(VPT == 8 ? 512 : 1024) __global__ void to_fp8_kernel(
 struct Split {
   int threads, vpt;
 };
-Split split_for(int64_t T, int H) {
+Split split_for(int64_t T, int H, bool sums = false) {
   const int nvec = H / 8;
   // from about four rows a CU on the chip is full with 256 threads a row;
-  // longer rows take 512, so that a thread's registers do not limit the waves
+  // longer rows take 512, so that a thread's registers do not limit the waves.
+  // Out of sums, whose threads have about 100 registers, two rows of more than 512
+  // threads do not fit a CU (us, 1024 / 512 threads: 370 rows of 8192, one part, 9.0 / 7.1,
+  // 849 of two 22.9 / 16.9; norm, sum and norm, 789 of six, 37.9 / 30.4).
+  const int most = sums && T > kCUs ? 512 : 1024;
   const int threads = T >= 1024 ? (nvec <= 1024 ? 256 : 512)
-                                : std::min(1024, (nvec + 63) / 64 * 64);
+                                : std::min(most, (nvec + 63) / 64 * 64);
   return {threads, (nvec + threads - 1) / threads};
 }
 
@@ -337,7 +343,7 @@ template <bool ADD, bool FP8, bool SUMS = false>
 void launch_norm(void* out, float* out_scale, const ushort* x, int64_t T, int H,
                  ushort* residual, const torch::Tensor& weight, double eps,
                  const ProductSums& sums = {}) {
-  const Split s = split_for(T, H);
+  const Split s = split_for(T, H, SUMS);
   with_vpt(s.vpt, [&](auto vpt) {
     hipLaunchKernelGGL((rmsnorm_kernel<ADD, FP8, SUMS, decltype(vpt)::value>),
                        dim3((uint32_t)T), dim3(s.threads), 0,
@@ -501,7 +507,7 @@ void norm_add_norm(torch::Tensor out, torch::Tensor hidden,
   for (const auto& w : {w1.has_value() ? *w1 : w2, w2})
     TORCH_CHECK(w.scalar_type() == torch::kBFloat16 && w.numel() == H && w.is_contiguous());
   if (T == 0) return;
-  const Split s = split_for(T, H);
+  const Split s = split_for(T, H, part.has_value());
   auto go = [&](auto first, auto sums, auto vpt) {
     hipLaunchKernelGGL((norm_add_norm_kernel<decltype(first)::value, decltype(sums)::value,
                                              decltype(vpt)::value>),

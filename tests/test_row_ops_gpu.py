@@ -145,6 +145,31 @@ def test_norms_of_product_sums(M, fp8, N, K):
     assert torch.equal(r1, r2)
 
 
+@pytest.mark.parametrize("T", [256, 257, 1023, 1024])
+@pytest.mark.parametrize("H", [4096, 4104, 8192, 16384])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_norms_of_sums_of_many_rows(T, H, fp8):
+    """On both sides of 256 and 1024 rows, where the threads of a row change: the row is
+    the parts' sum in bf16, whatever they are."""
+    torch.manual_seed(T + H)
+    part = torch.randn(3, T, H, device=DEV)
+    sx, sw = torch.rand(T, device=DEV) + 0.5, torch.rand(H, device=DEV) + 0.5
+    weight = torch.randn(H, device=DEV, dtype=torch.bfloat16)
+    r = _x(T, H)
+    h = part[0] + part[1] + part[2]
+    if fp8:
+        h = h * sx[:, None] * sw
+    want, total = ref.fused_add_rmsnorm(h.bfloat16().float(), r.float(), weight.float(), 1e-5)
+    sums = ops.ProductSums(part, *((sx, sw) if fp8 else (None, None)))
+    if fp8:
+        (q, s), res = ops.fused_add_rmsnorm_fp8(sums, r, weight, 1e-5), r
+        _close_fp8(q, s, want)
+    else:
+        out, res = ops.fused_add_rmsnorm(sums, r, weight, 1e-5)
+        torch.testing.assert_close(out.float(), want, atol=1e-6, rtol=2.0 ** -8)
+    assert torch.equal(res, total.bfloat16())
+
+
 @pytest.mark.parametrize("M", [1, 40, 1030])
 @pytest.mark.parametrize("N", [8, 520, 2304, 16384])
 def test_branch_norm_add_and_norm(M, N):
