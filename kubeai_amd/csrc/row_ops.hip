@@ -101,17 +101,16 @@ __launch_bounds__(VPT == 8 ? 512 : 1024) __global__ void rmsnorm_kernel(
   __shared__ float red[2][16];
   float vals[VPT][8];
   float ssum = 0.f;
-  // Of few rows: bound by one latency after the other, so what does not wait for
-  // anything is asked for first (SUMS: before the parts). us, 40 rows of 4096 out of
-  // a product's sums into fp8 7.1 -> 5.1, 560 rows 13.8 -> 10.0; 2000 rows of bf16
-  // 12.8 -> 12.1.
-  constexpr bool kEarly = SUMS || VPT <= 2;
-  ushort8 early_r[SUMS ? VPT : 1], early_w[kEarly ? VPT : 1];
-  if constexpr (kEarly) {
+  // Out of sums: bound by one latency after the other, so what does not wait for
+  // anything is asked for before the parts. us, 40 rows of 4096 into fp8 7.1 -> 5.1, 560
+  // rows 13.8 -> 10.0. (Not of a bf16 row: it would wait for the weights too. Rows in cache,
+  // weights out of it, 40 x 2048 2.8 us with, 2.6 without.)
+  ushort8 early_r[SUMS ? VPT : 1], early_w[SUMS ? VPT : 1];
+  if constexpr (SUMS) {
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
       const int i = min((int)(threadIdx.x + k * blockDim.x), nvec - 1);
-      if constexpr (SUMS && ADD)
+      if constexpr (ADD)
         early_r[k] = reinterpret_cast<const ushort8*>(residual + row * H)[i];
       early_w[k] = reinterpret_cast<const ushort8*>(w)[i];
     }
@@ -149,7 +148,7 @@ __launch_bounds__(VPT == 8 ? 512 : 1024) __global__ void rmsnorm_kernel(
 #pragma unroll
       for (int j = 0; j < 8; ++j) ssum += vals[k][j] * vals[k][j];
     }
-    if constexpr (kEarly) asm volatile("" : "+v"(early_w[k]));
+    if constexpr (SUMS) asm volatile("" : "+v"(early_w[k]));
   }
   const float total = block_reduce_sum(ssum, red[0]);
   const float inv_rms = rsqrtf(total / (float)H + eps);
@@ -159,7 +158,7 @@ __launch_bounds__(VPT == 8 ? 512 : 1024) __global__ void rmsnorm_kernel(
     const int i = threadIdx.x + k * blockDim.x;
     if (i < nvec) {
       ushort8 wv;
-      if constexpr (kEarly) wv = early_w[k];
+      if constexpr (SUMS) wv = early_w[k];
       else wv = reinterpret_cast<const ushort8*>(w)[i];
       if constexpr (FP8) {
 #pragma unroll
@@ -188,7 +187,8 @@ __launch_bounds__(VPT == 8 ? 512 : 1024) __global__ void rmsnorm_kernel(
 // A row is read once, in place of two passes over it (norm; add and norm); us in a
 // model, separate launches / this: 5376 x 2304 35.1 / 20.9 (weights
 // asked for behind the sums 22.3).
-template <bool FIRST, bool SUMS, int VPT>
+// EARLY: the weights are asked for before the branch.
+template <bool FIRST, bool SUMS, int VPT, bool EARLY>
 __launch_bounds__(VPT == 8 ? 512 : 1024) __global__ void norm_add_norm_kernel(
     ushort* __restrict__ out, ushort* __restrict__ hidden,
     const ushort* __restrict__ x, const ushort* __restrict__ residual,
@@ -200,7 +200,7 @@ __launch_bounds__(VPT == 8 ? 512 : 1024) __global__ void norm_add_norm_kernel(
   float vals[VPT][8];
   ushort8 res[VPT];
   float ssum = 0.f;
-  constexpr bool kEarly = VPT <= 2;  // as above
+  constexpr bool kEarly = EARLY && VPT <= 2;
   ushort8 early1[kEarly && FIRST ? VPT : 1], early2[kEarly ? VPT : 1];
 #pragma unroll
   for (int k = 0; k < VPT; ++k) {
@@ -508,9 +508,9 @@ void norm_add_norm(torch::Tensor out, torch::Tensor hidden,
     TORCH_CHECK(w.scalar_type() == torch::kBFloat16 && w.numel() == H && w.is_contiguous());
   if (T == 0) return;
   const Split s = split_for(T, H, part.has_value());
-  auto go = [&](auto first, auto sums, auto vpt) {
+  auto launch = [&](auto first, auto sums, auto vpt, auto early) {
     hipLaunchKernelGGL((norm_add_norm_kernel<decltype(first)::value, decltype(sums)::value,
-                                             decltype(vpt)::value>),
+                                             decltype(vpt)::value, decltype(early)::value>),
                        dim3((uint32_t)T), dim3(s.threads), 0,
                        c10::hip::getCurrentHIPStream().stream(), (ushort*)out.data_ptr(),
                        (ushort*)hidden.data_ptr(),
@@ -519,9 +519,15 @@ void norm_add_norm(torch::Tensor out, torch::Tensor hidden,
                        w1.has_value() ? (const ushort*)w1->data_ptr() : nullptr,
                        (const ushort*)w2.data_ptr(), (float)eps, H, p);
   };
+  using Yes = std::true_type;
+  using No = std::false_type;
+  // Registers for the weights: not in rows of 1024 threads, of which two share a CU then
+  // (1000 x 16384 33 us with, 27 without; 8 x 8192 4.7 / 4.6; 40 x 2304 gains as above).
+  auto go = [&](auto first, auto sums, auto vpt) {
+    if (decltype(sums)::value || s.threads < 1024) launch(first, sums, vpt, Yes{});
+    else launch(first, sums, vpt, No{});
+  };
   with_vpt(s.vpt, [&](auto vpt) {
-    using Yes = std::true_type;
-    using No = std::false_type;
     if (part.has_value()) go(Yes{}, Yes{}, vpt);
     else if (w1.has_value()) go(Yes{}, No{}, vpt);
     else go(No{}, No{}, vpt);
