@@ -7,7 +7,7 @@
 //  - workgroup = 4 waves x 16 rows of W. A wave's lanes read 16 rows x 64
 //    contiguous bytes straight into matrix operands (no LDS for W: each byte
 //    is used by one wave); two of those loads fill a 128-byte line. The steps
-//    are 256 bytes of every row; two of them are in flight behind the one that is
+//    are 256 bytes of every row (step_bytes); two of them are in flight behind the one that is
 //    multiplied. Loads past the end are of no bytes instead of in a branch: where
 //    paths of more and of fewer loads meet, the compiler waits for all of them (one
 //    row of 28672 x 4096 bf16: 46.5 us -> 43.4).
@@ -62,7 +62,12 @@ namespace {
 constexpr int kNW = 4;         // waves per workgroup (waves_for: of uncut few rows)
 constexpr int kMaxRows = 96;
 constexpr int kMaxParts = 8;
-constexpr int kStep = 256;     // bytes of K a step
+// Bytes of K a step. Experts of many fp8 rows: x of three steps of 256 would leave a CU two
+// or three workgroups (16-row tiles 6: 7168 x 1024, 4 experts, 391 rows 23.8 us, 21.4; in bf16 the
+// shorter steps lose, 4096 x 14336, 8 experts, 206 rows 197 us, 204).
+constexpr int step_bytes(bool fp8, int mt, bool grouped) {
+  return fp8 && grouped && mt >= 4 ? 128 : 256;
+}
 constexpr int kAhead = 3;      // steps of x in LDS and of w in registers
 constexpr int64_t kFarRows = (int64_t)1 << 23;  // bytes
 
@@ -181,7 +186,7 @@ __launch_bounds__(NW * WAVE_SIZE) __global__ void skinny_kernel(
     const float* sx, const float* sw, const ushort* bias, const int M_all,
     const int N, const int KB, const int ldx, const int xbytes, const int k_part,
     const int parts, const Groups grp) {
-  constexpr int CH = kStep / 64, UPR = kStep / 16;
+  constexpr int kStep = step_bytes(FP8, MT, GROUPED), CH = kStep / 64, UPR = kStep / 16;
   constexpr int RW = ACT ? 8 : 16;             // columns of the result a wave
   constexpr int NX = (MT * 16 * UPR - 1) / (NW * WAVE_SIZE) + 1, L = NX + CH;  // loads a step
   constexpr int PLACE = NX * NW * WAVE_SIZE * 16;  // x of a step in LDS
