@@ -594,10 +594,20 @@ void skinny_experts(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   // more 1.02 (four 1.04).
   const double reached = E * (1.0 - std::pow(1.0 - 1.0 / E, R));
   const bool thin = reached * ((N + kNW * 16 - 1) / (kNW * 16)) < 4 * 256;
+  // Many bf16 rows, of which a workgroup reads as many bytes as of the weights: eight waves
+  // where those are just one workgroup a CU (us, four / eight: 8 of 4096 x 14336 206 rows 198
+  // / 178, 376 rows 216 / 196; but 16 of 12800 x 4096 416 rows 336 / 356, more than one a CU).
+  const double eights = reached * ((N + 127) / 128);
+  const bool one_each = eights > 192 && eights <= 256;
   constexpr std::integral_constant<int, 2> two;
   constexpr std::integral_constant<int, kNW> four;
   auto tiles = [&](auto f) {
     constexpr std::integral_constant<int, 1> one;
+    if constexpr (!decltype(f)::value) {
+      constexpr std::integral_constant<int, 8> eight;
+      if (mean > 44 && one_each) return go(f, std::integral_constant<int, 6>{}, eight);
+      if (mean > 22 && one_each) return go(f, four, eight);
+    }
     if (mean <= 8 && thin) go(f, one, two);
     else if (mean <= 8) go(f, one, four);
     else if (mean <= 22) go(f, two, four);

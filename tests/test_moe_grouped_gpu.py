@@ -306,13 +306,15 @@ def test_experts_without_rows(E, R, N, fp8):
             assert ((y[rows].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * size).all()
 
 
-@pytest.mark.parametrize("R", [69, 132, 133, 300])
+@pytest.mark.parametrize("R,N", [(69, 68), (132, 68), (133, 68), (300, 68), (69, 9000),
+                                 (133, 9000)])
 @pytest.mark.parametrize("K", [64, 128, 192, 320, 448, 1088])
 @pytest.mark.parametrize("fp8", [False, True])
-def test_experts_of_many_rows(R, K, fp8):
+def test_experts_of_many_rows(R, N, K, fp8):
     """64 and 96 rows a pass, steps of 128 and 256 bytes: one to more than are under way,
-    whole ones and not; several passes (all rows of one expert), gathered rows."""
-    E, N = 3, 68
+    whole ones and not; several passes (all rows of one expert), gathered rows; four waves a
+    workgroup and eight (bf16 of 9000 columns)."""
+    E = 3
     torch.manual_seed(R + K)
     w = torch.randn(E, N, K, device=DEV, dtype=torch.bfloat16)
     x = torch.randn(R, K, device=DEV, dtype=torch.bfloat16)
@@ -327,10 +329,11 @@ def test_experts_of_many_rows(R, K, fp8):
             ops._C.skinny_experts(y, x, w, sx, sw,
                                   torch.tensor(begin, dtype=torch.int32, device=DEV), rows)
             at = torch.arange(R, device=DEV) if rows is None else rows.long()
-            of = torch.bucketize(torch.arange(R), torch.tensor(begin[1:]), right=True).to(DEV)
-            a, b = x[at].double(), w.double()[of]
-            s = sx[at, None].double() * sw[of].double() if fp8 else 1.0
-            want = (a[:, None] * b).sum(-1) * s
-            size = (a[:, None] * b).abs().sum(-1) * s
-            # one rounding to bf16; fp32 sums
-            assert ((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * size).all()
+            for e in range(E):
+                part = slice(begin[e], begin[e + 1])
+                a, b = x[at[part]].double(), w[e].double()
+                s = sx[at[part], None].double() * sw[e].double() if fp8 else 1.0
+                want, size = (a @ b.T) * s, (a.abs() @ b.abs().T) * s
+                # one rounding to bf16; fp32 sums
+                off = (y[part].double() - want).abs()
+                assert (off <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * size).all()
