@@ -62,11 +62,12 @@ namespace {
 constexpr int kNW = 4;         // waves per workgroup (waves_for: of uncut few rows)
 constexpr int kMaxRows = 96;
 constexpr int kMaxParts = 8;
-// Bytes of K a step. Experts of many fp8 rows: x of three steps of 256 would leave a CU two
-// or three workgroups (16-row tiles 6: 7168 x 1024, 4 experts, 391 rows 23.8 us, 21.4; in bf16 the
-// shorter steps lose, 4096 x 14336, 8 experts, 206 rows 197 us, 204).
+// Bytes of K a step. Experts of many fp8 rows: x of three steps of 256 in passes of 96 rows
+// would leave a CU two workgroups (7168 x 1024, 4 experts, 391 rows 23.8 us, 21.4). Passes of
+// 64 rows lose by the shorter steps (28672 x 4096, 8 experts, 3 to 5 %), and so does bf16
+// (4096 x 14336, 8 experts, 206 rows 197 us, 204).
 constexpr int step_bytes(bool fp8, int mt, bool grouped) {
-  return fp8 && grouped && mt >= 4 ? 128 : 256;
+  return fp8 && grouped && mt > 4 ? 128 : 256;
 }
 constexpr int kAhead = 3;      // steps of x in LDS and of w in registers
 constexpr int64_t kFarRows = (int64_t)1 << 23;  // bytes
