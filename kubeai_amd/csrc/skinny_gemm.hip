@@ -597,7 +597,9 @@ void skinny_experts(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   const bool thin = reached * ((N + kNW * 16 - 1) / (kNW * 16)) < 4 * 256;
   // Many bf16 rows, of which a workgroup reads as many bytes as of the weights: eight waves
   // where those are just one workgroup a CU (us, four / eight: 8 of 4096 x 14336 206 rows 198
-  // / 178, 376 rows 216 / 196; but 16 of 12800 x 4096 416 rows 336 / 356, more than one a CU).
+  // / 178, 376 rows 216 / 196; but 16 of 12800 x 4096 416 rows 336 / 356, more than one a CU.
+  // Where half the rows are one expert's, its passes lie on fewer CUs: both products of a
+  // mixture of 128 tokens 788 / 802, 224 899 / 910; spread evenly 647 / 643, 689 / 681).
   const double eights = reached * ((N + 127) / 128);
   const bool one_each = eights > 192 && eights <= 256;
   constexpr std::integral_constant<int, 2> two;

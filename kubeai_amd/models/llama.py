@@ -321,7 +321,7 @@ class MoEMLP(nn.Module):
     experts' row counts."""
 
     #: one pass of 8 experts of 14336 x 4096, us, weight-streaming / tiled: fp8 128
-    #: tokens 360/305, 256 445/335; bf16 627/548, 715/582; every expert's tokens
+    #: tokens 355/302, 256 405/325; bf16 643/557, 704/572; every expert's tokens
     #: asked for one after the other took 722 and 1159 at 128. (Streaming reads an
     #: expert's weights again for every 96 of its rows.) Up to 256 tokens any
     #: routing may be recorded in a graph, so no row counts come to the host.
@@ -329,15 +329,15 @@ class MoEMLP(nn.Module):
 
     #: Above these the tiled product has the step where it takes both
     #: projections. us, streaming / tiled, tokens spread evenly (half of them
-    #: alike): fp8 8 x 14336 x 4096 160 tokens 371/319 (436/356), 192 413/321
-    #: (521/375), 256 445/335 (519/395); 8 x 7168 x 2048 160 121/116 (160/122), 192
-    #: 137/116 (180/124); 16 x 6400 x 4096 160 301/304 (380/325), 192 313/305
-    #: (368/325); 32 x 1408 x 2048, 4 a token, 160 104/105 (133/115), 192 108/107
-    #: (123/117); 4 x 3584 x 1024 160 64/46 (81/47), 192 76/47 (87/54). bf16 8 x 14336 x
-    #: 4096 224 688/574 (840/714), 256 715/582 (864/692); 8 x 7168 x 2048 224 209/194
-    #: (268/207), 256 214/198 (286/210); 16 x 6400 x 4096 224 553/507 (614/528), 256
-    #: 568/505 (673/526); 32 x 1408 x 2048 224 163/164 (208/177), 256 165/165
-    #: (200/174). The lines are where the two met before experts' tiles went by the
+    #: alike): fp8 8 x 14336 x 4096 160 tokens 371/308 (428/343), 192 382/334
+    #: (465/358), 256 405/325 (500/378); 8 x 7168 x 2048 160 129/120 (155/124), 192
+    #: 131/121 (166/128); 16 x 6400 x 4096 160 302/288 (359/308), 192 316/290
+    #: (348/309); 32 x 1408 x 2048, 4 a token, 160 112/111 (138/121), 192 118/112
+    #: (141/123); 4 x 3584 x 1024 160 62/49 (77/50), 192 76/50 (84/57). bf16 8 x 14336 x
+    #: 4096 224 681/565 (910/676), 256 704/572 (958/674); 8 x 7168 x 2048 224 215/201
+    #: (282/211), 256 220/200 (304/210); 16 x 6400 x 4096 224 573/504 (659/550), 256
+    #: 569/491 (721/523); 32 x 1408 x 2048 224 170/168 (204/182), 256 173/169
+    #: (223/180). The lines are where the two met before experts' tiles went by the
     #: costs of one matrix. The tiled kernel is the faster one from fewer tokens on
     #: now, down to 128 at most of these sizes; the lines have not been moved since.
     #: (The kernels need not round alike, and in a routed model that can move a token
