@@ -1,5 +1,5 @@
 """Device-side routing and grouped expert products at the edges of their tiles
-(16-row tiles, 64 columns a workgroup, 256/512-byte steps of K, several passes
+(16-row tiles, 64 columns a workgroup, 128/256-byte steps of K, several passes
 for an expert with many rows) and skinny products at theirs.
 
 The reference rounds where the kernels do (each product and the activation to
