@@ -1,6 +1,8 @@
 // Python bindings for the kubeai_amd gfx950 HIP kernels.
 #include <torch/extension.h>
 
+#include <algorithm>
+
 void rmsnorm(torch::Tensor out, torch::Tensor x, torch::Tensor weight,
              double eps);
 void fused_add_rmsnorm(torch::Tensor x, torch::Tensor residual,
@@ -71,10 +73,10 @@ void moe_route(torch::Tensor index, torch::Tensor weight, torch::Tensor begin,
 void moe_combine(torch::Tensor out, torch::Tensor y, torch::Tensor place,
                  torch::Tensor weight);
 void skinny_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w);
-void greedy_sample(torch::Tensor out, torch::Tensor logits);
-void gumbel_sample(torch::Tensor out, torch::Tensor logits,
-                   torch::Tensor temperature, torch::Tensor seeds,
-                   int64_t step);
+void greedy_sample(torch::Tensor out, torch::Tensor logits,
+                   c10::optional<torch::Tensor> logprob);
+void gumbel_sample(torch::Tensor out, torch::Tensor logits, torch::Tensor temperature,
+                   torch::Tensor seeds, int64_t step, c10::optional<torch::Tensor> logprob);
 void sgmv(torch::Tensor y, torch::Tensor x, torch::Tensor A, torch::Tensor B,
           torch::Tensor idx, double scale);
 void lora_apply(torch::Tensor y, torch::Tensor x, torch::Tensor table,
@@ -104,6 +106,28 @@ void nucleus_accept(torch::Tensor ok, torch::Tensor logits,
                     torch::Tensor cand, torch::Tensor m, torch::Tensor z,
                     torch::Tensor temps, torch::Tensor top_ps,
                     torch::Tensor top_ks);
+
+// out [R, C] int32 on the host: row i takes rows[i], zeros elsewhere
+static void fill_rows(torch::Tensor out, const py::list& rows) {
+  TORCH_CHECK(out.device().is_cpu() && out.scalar_type() == torch::kInt32 &&
+              out.dim() == 2 && out.is_contiguous());
+  const int64_t R = out.size(0), C = out.size(1), n = (int64_t)rows.size();
+  TORCH_CHECK(n <= R, n, " lists for ", R, " rows");
+  int32_t* to = out.data_ptr<int32_t>();
+  std::fill(to, to + R * C, 0);
+  for (int64_t i = 0; i < n; ++i, to += C) {
+    PyObject* row = PyList_GET_ITEM(rows.ptr(), i);
+    TORCH_CHECK(PyList_Check(row), "rows are lists");
+    const int64_t k = PyList_GET_SIZE(row);
+    TORCH_CHECK(k <= C, "a list of ", k, " for a row of ", C);
+    for (int64_t j = 0; j < k; ++j) {
+      const long v = PyLong_AsLong(PyList_GET_ITEM(row, j));
+      if (v == -1 && PyErr_Occurred()) throw py::error_already_set();
+      TORCH_CHECK(v >= INT32_MIN && v <= INT32_MAX, "32-bit values");
+      to[j] = (int32_t)v;
+    }
+  }
+}
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm", &rmsnorm, "RMSNorm (bf16, fp32 accum)");
@@ -150,8 +174,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_combine", &moe_combine, "weighted sum of the experts' rows");
   m.def("skinny_linear", &skinny_linear,
         "weight-streaming product of up to 96 rows, bf16 or scaled fp8");
-  m.def("greedy_sample", &greedy_sample, "argmax sampling");
-  m.def("gumbel_sample", &gumbel_sample, "temperature sampling (hash RNG)");
+  m.def("fill_rows", &fill_rows, "lists of numbers to rows of a host tensor");
+  m.def("greedy_sample", &greedy_sample, "argmax sampling", py::arg("out"),
+        py::arg("logits"), py::arg("logprob") = py::none());
+  m.def("gumbel_sample", &gumbel_sample, "temperature sampling (hash RNG)",
+        py::arg("out"), py::arg("logits"), py::arg("temperature"),
+        py::arg("seeds"), py::arg("step"),
+        py::arg("logprob") = py::none());
   m.def("rmsnorm_fp8", &rmsnorm_fp8, "rmsnorm with fused fp8 row quant");
   m.def("fused_add_rmsnorm_fp8", &fused_add_rmsnorm_fp8,
         "residual add + rmsnorm with fused fp8 row quant");

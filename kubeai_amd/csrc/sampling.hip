@@ -9,6 +9,12 @@
 // Stage 1 splits each vocab row into kSplits chunks (B*kSplits workgroups
 // keep all 256 CUs busy even at decode batch ~32); stage 2 is one wave per
 // row reducing the partials.
+//
+// With log-probabilities the same pass has the sum of exp(x - max) as well: a thread
+// holds 16 values at a time, their maximum moves its sum once, so a value costs one
+// exponential. Bound by reading the logits once and by two launches: 40 rows of 128256
+// 11.6 us (tokens alone 7.4; torch's logsumexp, gather and difference behind that
+// 72), one row 7.6 (5.7 and 49), 96 rows 22.5 (15.2 and 89).
 #include <torch/extension.h>
 
 #include "common.h"
@@ -17,19 +23,55 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kSplits = 32;
+constexpr int kUnits = 4;  // of 4 values, a thread at a time
 
-template <bool kGumbel>
-__global__ void sample_stage1(
-    float* __restrict__ part_val,          // [B, kSplits]
-    int32_t* __restrict__ part_idx,        // [B, kSplits]
+// a chunk's best value (with its noise) and where, that place's logit, and with
+// log-probabilities the largest logit and the sum of exp(logit - it)
+struct Part {
+  float best;
+  int32_t idx;
+  float raw, m, z;
+};
+
+DEV_INLINE void keep_best(Part& p, float v, int32_t i, float raw) {
+  if (v > p.best || (v == p.best && i < p.idx)) {
+    p.best = v;
+    p.idx = i;
+    p.raw = raw;
+  }
+}
+// (a maximum of -inf has only zeros behind it)
+DEV_INLINE float finite_or_0(float m) { return m == -INFINITY ? 0.f : m; }
+DEV_INLINE void keep_sum(Part& p, float m, float z) {
+  const float most = fmaxf(p.m, m), use = finite_or_0(most);
+  p.z = p.z * expf(p.m - use) + z * expf(m - use);
+  p.m = most;
+}
+template <bool kLogprob>
+DEV_INLINE void over_lanes(Part& p) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const float v = __shfl_xor(p.best, off), raw = __shfl_xor(p.raw, off);
+    const int32_t i = __shfl_xor(p.idx, off);
+    keep_best(p, v, i, raw);
+    if constexpr (kLogprob) {
+      const float m = __shfl_xor(p.m, off), z = __shfl_xor(p.z, off);
+      keep_sum(p, m, z);
+    }
+  }
+}
+
+template <bool kGumbel, bool kLogprob>
+__launch_bounds__(kBlock) __global__ void sample_stage1(
+    Part* __restrict__ part,               // [B, kSplits]
     const float* __restrict__ logits,      // [B, V]
     const float* __restrict__ temperature,  // [B]
     const int64_t* __restrict__ seeds,      // [B]
-    const int64_t step, const int V) {
+    const int64_t step, const int V, const bool wide) {
   const int b = blockIdx.x;
   const int split = blockIdx.y;
-  const int chunk = (V + kSplits - 1) / kSplits;
-  const int lo = split * chunk;
+  const int chunk = ((V + kSplits - 1) / kSplits + 3) / 4 * 4;
+  const int lo = min(V, split * chunk);
   const int hi = min(V, lo + chunk);
   const float* row = logits + (int64_t)b * V;
   float temp = 1.0f;
@@ -41,106 +83,134 @@ __global__ void sample_stage1(
     key = (uint64_t)seeds[b] * 1000003ull + (uint64_t)step;
   }
 
-  float best = -INFINITY;
-  int best_idx = V;
-  for (int v = lo + threadIdx.x; v < hi; v += kBlock) {
-    float val = row[v];
-    if (!greedy) {
-      float u = hash_uniform(key, (uint64_t)v);
-      val = val / temp + (-__logf(-__logf(u)));
-    }
-    if (val > best || (val == best && v < best_idx)) {
-      best = val;
-      best_idx = v;
-    }
-  }
+  Part p{-INFINITY, V, -INFINITY, -INFINITY, 0.f};
+  for (int base = lo; base < hi; base += kBlock * 4 * kUnits) {
+    float4_t x[kUnits];
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    float ov = __shfl_xor(best, off, 64);
-    int oi = __shfl_xor(best_idx, off, 64);
-    if (ov > best || (ov == best && oi < best_idx)) {
-      best = ov;
-      best_idx = oi;
+    for (int j = 0; j < kUnits; ++j) {
+      const int v = base + (j * kBlock + threadIdx.x) * 4;
+      x[j] = float4_t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      if (wide) {  // (then hi is a multiple of 4 too)
+        if (v < hi) x[j] = *reinterpret_cast<const float4_t*>(row + v);
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (v + k < hi) x[j][k] = row[v + k];
+      }
+    }
+    float most = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < kUnits; ++j) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int v = base + (j * kBlock + threadIdx.x) * 4 + k;
+        float val = x[j][k];
+        if (v < hi) {
+          if (!greedy) {
+            const float u = hash_uniform(key, (uint64_t)v);
+            val = val / temp + (-__logf(-__logf(u)));
+          }
+          keep_best(p, val, v, x[j][k]);
+        }
+        if constexpr (kLogprob) most = fmaxf(most, x[j][k]);
+      }
+    }
+    if constexpr (kLogprob) {
+      most = fmaxf(most, p.m);
+      const float use = finite_or_0(most);
+      float z = p.z * expf(p.m - use);
+#pragma unroll
+      for (int j = 0; j < kUnits; ++j) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) z += expf(x[j][k] - use);
+      }
+      p.m = most;
+      p.z = z;
     }
   }
-  __shared__ float sval[4];
-  __shared__ int sidx[4];
+  over_lanes<kLogprob>(p);
+  __shared__ Part waves[kBlock / WAVE_SIZE];
   const int wave = threadIdx.x / WAVE_SIZE;
-  if (threadIdx.x % WAVE_SIZE == 0) {
-    sval[wave] = best;
-    sidx[wave] = best_idx;
-  }
+  if (threadIdx.x % WAVE_SIZE == 0) waves[wave] = p;
   __syncthreads();
   if (threadIdx.x == 0) {
 #pragma unroll
     for (int w = 1; w < kBlock / WAVE_SIZE; ++w) {
-      if (sval[w] > best || (sval[w] == best && sidx[w] < best_idx)) {
-        best = sval[w];
-        best_idx = sidx[w];
-      }
+      const Part o = waves[w];
+      keep_best(p, o.best, o.idx, o.raw);
+      if constexpr (kLogprob) keep_sum(p, o.m, o.z);
     }
-    part_val[b * kSplits + split] = best;
-    part_idx[b * kSplits + split] = best_idx;
+    part[b * kSplits + split] = p;
   }
 }
 
-__global__ void sample_stage2(int64_t* __restrict__ out,
-                              const float* __restrict__ part_val,
-                              const int32_t* __restrict__ part_idx) {
+template <bool kLogprob>
+__global__ void sample_stage2(int64_t* __restrict__ out, float* __restrict__ logprob,
+                              const Part* __restrict__ part, const int V) {
   const int b = blockIdx.x;
   const int lane = threadIdx.x;
-  float best = (lane < kSplits) ? part_val[b * kSplits + lane] : -INFINITY;
-  int best_idx = (lane < kSplits) ? part_idx[b * kSplits + lane] : INT32_MAX;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    float ov = __shfl_xor(best, off, 64);
-    int oi = __shfl_xor(best_idx, off, 64);
-    if (ov > best || (ov == best && oi < best_idx)) {
-      best = ov;
-      best_idx = oi;
-    }
+  Part p{-INFINITY, INT32_MAX, -INFINITY, -INFINITY, 0.f};
+  if (lane < kSplits) p = part[b * kSplits + lane];
+  over_lanes<kLogprob>(p);
+  if (lane == 0) {
+    out[b] = p.idx;
+    if constexpr (kLogprob) logprob[b] = p.raw - (finite_or_0(p.m) + logf(p.z));
   }
-  if (lane == 0) out[b] = best_idx;
 }
 
-template <bool kGumbel>
-void launch_sample(torch::Tensor out, torch::Tensor logits,
+template <bool kGumbel, bool kLogprob>
+void launch_sample(torch::Tensor out, float* logprob, torch::Tensor logits,
                    const float* temp_ptr, const int64_t* seed_ptr,
                    int64_t step) {
   const int B = logits.size(0), V = logits.size(1);
   if (B == 0) return;
-  auto opts = torch::TensorOptions().device(logits.device());
-  auto part_val = torch::empty({B, kSplits}, opts.dtype(torch::kFloat32));
-  auto part_idx = torch::empty({B, kSplits}, opts.dtype(torch::kInt32));
+  auto part = torch::empty({B, kSplits, (int64_t)sizeof(Part)},
+                           torch::TensorOptions().device(logits.device()).dtype(torch::kUInt8));
+  auto* pp = reinterpret_cast<Part*>(part.data_ptr());
+  const bool wide = V % 4 == 0 && ((uintptr_t)logits.data_ptr() & 15) == 0;
   auto stream = c10::hip::getCurrentHIPStream().stream();
-  hipLaunchKernelGGL((sample_stage1<kGumbel>), dim3(B, kSplits), dim3(kBlock),
-                     0, stream, part_val.data_ptr<float>(),
-                     part_idx.data_ptr<int32_t>(), logits.data_ptr<float>(),
-                     temp_ptr, seed_ptr, step, V);
+  hipLaunchKernelGGL((sample_stage1<kGumbel, kLogprob>), dim3(B, kSplits), dim3(kBlock),
+                     0, stream, pp, logits.data_ptr<float>(), temp_ptr, seed_ptr, step, V,
+                     wide);
   HIP_CHECK_KERNEL();
-  hipLaunchKernelGGL(sample_stage2, dim3(B), dim3(WAVE_SIZE), 0, stream,
-                     out.data_ptr<int64_t>(), part_val.data_ptr<float>(),
-                     part_idx.data_ptr<int32_t>());
+  hipLaunchKernelGGL((sample_stage2<kLogprob>), dim3(B), dim3(WAVE_SIZE), 0, stream,
+                     out.data_ptr<int64_t>(), logprob, pp, V);
   HIP_CHECK_KERNEL();
+}
+
+template <bool kGumbel>
+void launch_sample(torch::Tensor out, const c10::optional<torch::Tensor>& logprob,
+                   torch::Tensor logits, const float* temp_ptr, const int64_t* seed_ptr,
+                   int64_t step) {
+  if (!logprob.has_value()) {
+    launch_sample<kGumbel, false>(out, nullptr, logits, temp_ptr, seed_ptr, step);
+    return;
+  }
+  TORCH_CHECK(logprob->scalar_type() == torch::kFloat32 && logprob->is_contiguous() &&
+              logprob->is_cuda() && logprob->numel() == logits.size(0));
+  launch_sample<kGumbel, true>(out, logprob->data_ptr<float>(), logits, temp_ptr, seed_ptr,
+                               step);
 }
 
 }  // namespace
 
-void greedy_sample(torch::Tensor out, torch::Tensor logits) {
+// logprob (fp32 [B], or none): the sampled token's logit - log(sum(exp(row)))
+void greedy_sample(torch::Tensor out, torch::Tensor logits,
+                   c10::optional<torch::Tensor> logprob) {
   TORCH_CHECK(logits.is_contiguous());
   TORCH_CHECK(logits.scalar_type() == torch::kFloat32,
               "sampling expects fp32 logits");
-  launch_sample<false>(out, logits, nullptr, nullptr, 0);
+  launch_sample<false>(out, logprob, logits, nullptr, nullptr, 0);
 }
 
 void gumbel_sample(torch::Tensor out, torch::Tensor logits,
                    torch::Tensor temperature, torch::Tensor seeds,
-                   int64_t step) {
+                   int64_t step, c10::optional<torch::Tensor> logprob) {
   TORCH_CHECK(logits.is_contiguous());
   TORCH_CHECK(logits.scalar_type() == torch::kFloat32);
   TORCH_CHECK(temperature.scalar_type() == torch::kFloat32);
   TORCH_CHECK(seeds.scalar_type() == torch::kInt64);
-  launch_sample<true>(out, logits, temperature.data_ptr<float>(),
+  launch_sample<true>(out, logprob, logits, temperature.data_ptr<float>(),
                       seeds.data_ptr<int64_t>(), step);
 }
 

@@ -22,6 +22,9 @@ from .batch import ForwardBatch
 from .scheduler import SchedulerOutput
 
 
+_NUMPY = {torch.int32: np.int32, torch.int64: np.int64}
+
+
 class _DecodeGraph:
     """hipGraph-captured pure-decode step for one padded batch size.
 
@@ -35,75 +38,95 @@ class _DecodeGraph:
         dev = runner.device
         self.b_pad = b_pad
         self.bt_max = bt_max
-        self.input_ids = torch.zeros(b_pad, dtype=torch.int32, device=dev)
-        self.positions = torch.zeros(b_pad, dtype=torch.int32, device=dev)
-        self.slots = torch.full((b_pad,), -1, dtype=torch.int64, device=dev)
-        self.block_tables = torch.zeros(
-            (b_pad, bt_max), dtype=torch.int32, device=dev
-        )
-        self.seq_lens = torch.ones(b_pad, dtype=torch.int32, device=dev)
-        logits_idx = torch.arange(b_pad, dtype=torch.int64, device=dev)
-        # models with per-sequence state: every row is a one-token run; the
-        # rows' state slots are one more refreshed input (-1 on pad rows)
-        self.state_slots = None
+        self.block_size = runner.block_size
+        # all inputs lie behind one another, so that a step's are one copy
+        kinds = {
+            "slots": ((b_pad,), torch.int64),
+            "input_ids": ((b_pad,), torch.int32),
+            "positions": ((b_pad,), torch.int32),
+            "seq_lens": ((b_pad,), torch.int32),
+            "state_slots": ((b_pad,), torch.int32),
+            "tables": ((b_pad, bt_max), torch.int32),
+        }
+        self.layout, total = {}, 0  # name -> (bytes, shape, type)
+        for name, (shape, kind) in kinds.items():
+            n = int(np.prod(shape)) * kind.itemsize
+            self.layout[name] = (slice(total, total + n), shape, kind)
+            total += (n + 63) // 64 * 64
+        self.inputs = torch.zeros(total, dtype=torch.uint8, device=dev)
+
+        def view(name):
+            at, shape, kind = self.layout[name]
+            return self.inputs[at].view(kind).view(shape)
+
+        positions, tables = view("positions"), view("tables")
+        # rows of padding, as all are while the graph is recorded
+        view("slots").fill_(-1)
+        view("state_slots").fill_(-1)
+        view("seq_lens").fill_(1)
+        # models with per-sequence state: every row is a one-token run with its
+        # state slot (-1 on pad rows)
         seq = None
         if runner.uses_seq_meta:
             from kubeai_amd.ops.seq import SeqMeta
 
-            self.state_slots = torch.full((b_pad,), -1, dtype=torch.int32, device=dev)
             seq = SeqMeta(
                 start_loc=torch.arange(b_pad + 1, dtype=torch.int32, device=dev),
-                slots=self.state_slots,
+                slots=view("state_slots"),
                 token_seq=torch.arange(b_pad, dtype=torch.int32, device=dev),
-                positions=self.positions,
-                block_tables=self.block_tables,
+                positions=positions,
+                block_tables=tables,
                 n_seq=b_pad,
                 max_len=1,
             )
         self.fb = ForwardBatch(
             seq=seq,
-            input_ids=self.input_ids,
-            positions=self.positions,
-            slot_mapping=self.slots,
+            input_ids=view("input_ids"),
+            positions=positions,
+            slot_mapping=view("slots"),
             n_decode=b_pad,
-            decode_block_tables=self.block_tables,
-            decode_seq_lens=self.seq_lens,
+            decode_block_tables=tables,
+            decode_seq_lens=view("seq_lens"),
             n_prefill=0,
             prefill_query_start_loc=None,
             prefill_seq_lens=None,
             prefill_block_tables=None,
-            logits_indices=logits_idx,
+            logits_indices=torch.arange(b_pad, dtype=torch.int64, device=dev),  # (all rows)
         )
         # warmup outside capture (allocator, hipBLASLt workspace)
         torch.cuda.synchronize()
         for _ in range(2):
-            h = runner.model(self.fb)
-            runner.model.compute_logits(h[logits_idx])
+            runner.model.compute_logits(runner.model(self.fb))
         torch.cuda.synchronize()
         self.graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(self.graph):
-            h = runner.model(self.fb)
-            self.logits = runner.model.compute_logits(h[logits_idx])
+            self.logits = runner.model.compute_logits(runner.model(self.fb))
 
-    def run(self, input_ids, positions, slots, tables, seq_lens,
-            state_slots=None) -> torch.Tensor:
-        b = len(input_ids)
-        if self.state_slots is not None:
-            self.state_slots[:b].copy_(state_slots, non_blocking=True)
-            if b < self.b_pad:
-                self.state_slots[b:].fill_(-1)
-                self.positions[b:].fill_(0)
-        self.input_ids[:b].copy_(input_ids, non_blocking=True)
-        self.positions[:b].copy_(positions, non_blocking=True)
-        self.slots[:b].copy_(slots, non_blocking=True)
-        if b < self.b_pad:
-            self.slots[b:].fill_(-1)
-            self.seq_lens[b:].fill_(1)
-            self.block_tables[b:].fill_(0)
-        self.block_tables[:b, : tables.shape[1]].copy_(tables, non_blocking=True)
-        if tables.shape[1] < self.bt_max:
-            self.block_tables[:b, tables.shape[1] :].fill_(0)
-        self.seq_lens[:b].copy_(seq_lens, non_blocking=True)
+    def run(self, seqs) -> torch.Tensor:
+        """One step of these sequences; fp32 logits, valid until the next one. The
+        inputs go in one copy out of pinned memory, which torch's allocator hands
+        out again after the copy (as _upload; a copy each and fills of the rows of
+        padding took 0.1 ms of a step)."""
+        block = torch.empty(self.inputs.numel(), dtype=torch.uint8,
+                            pin_memory=self.inputs.is_cuda)
+        raw = block.numpy()
+        b, bs = len(seqs), self.block_size
+        tables = [ss.req.block_table for ss in seqs]
+        at, shape, kind = self.layout["tables"]
+        ops.fill_rows(block[at].view(kind).view(shape), tables)
+        positions = [ss.chunk_start for ss in seqs]
+        slots = [bt[t // bs] * bs + t % bs for bt, t in zip(tables, positions)]
+        ids = [ss.req.tokens[t] for ss, t in zip(seqs, positions)]
+        for name, rows, rest in (
+            ("slots", slots, -1), ("input_ids", ids, 0), ("positions", positions, 0),
+            ("seq_lens", [t + 1 for t in positions], 1),
+            ("state_slots", [ss.req.state_slot for ss in seqs], -1),
+        ):
+            at, _, kind = self.layout[name]
+            of = raw[at].view(_NUMPY[kind])
+            of[:b] = rows
+            of[b:] = rest
+        self.inputs.copy_(block, non_blocking=True)
         self.graph.replay()
         return self.logits[:b]
 
@@ -544,32 +567,7 @@ class ModelRunner:
                 self.enable_graphs = False
                 return None
             self._graphs[b_pad] = g
-        bs = self.block_size
-        ids, pos, slots, lens = [], [], [], []
-        tables = np.zeros((b, g.bt_max), dtype=np.int32)
-        for i, ss in enumerate(out.decode):
-            req = ss.req
-            t = ss.chunk_start
-            ids.append(req.tokens[t])
-            pos.append(t)
-            slots.append(req.block_table[t // bs] * bs + t % bs)
-            lens.append(t + 1)
-            bt = req.block_table
-            tables[i, : len(bt)] = bt
-        return g.run(
-            torch.tensor(ids, dtype=torch.int32),
-            torch.tensor(pos, dtype=torch.int32),
-            torch.tensor(slots, dtype=torch.int64),
-            torch.from_numpy(tables),
-            torch.tensor(lens, dtype=torch.int32),
-            state_slots=(
-                torch.tensor(
-                    [ss.req.state_slot for ss in out.decode], dtype=torch.int32
-                )
-                if self.uses_seq_meta
-                else None
-            ),
-        )
+        return g.run(out.decode)
 
     @torch.inference_mode()
     def forward_logits(self, out: SchedulerOutput, want) -> torch.Tensor:
@@ -656,8 +654,10 @@ class ModelRunner:
                 0, flat, torch.tensor(vals, dtype=logits.dtype, device=dev_l)
             )
         temps = [r.params.temperature for r in sample_reqs]
+        logits = logits.contiguous()
+        block = tokens = None  # tokens with log-probabilities, or tokens alone
         if all(t <= 0.0 for t in temps):
-            tokens = ops.greedy_sample(logits.contiguous())
+            block = ops.sample_with_logprobs(logits)
         else:
             needs_topk = any(
                 (r.params.top_p < 1.0 or r.params.top_k > 0)
@@ -687,21 +687,29 @@ class ModelRunner:
                     cache=self._sampling_cache,
                 ).to(dev)
             else:
-                tokens = ops.gumbel_sample(logits.contiguous(), t_t, seeds, step)
-        tokens = tokens.cpu().tolist()
+                block = ops.sample_with_logprobs(logits, t_t, seeds, step)
+        logprobs = lse = None
+        if block is not None:
+            tokens, logprobs = ops.sampled_to_host(block)
+        else:
+            tokens = tokens.cpu().tolist()
+        if max(tokens) >= V:  # no value of a row compares
+            raise RuntimeError("logits without a number in them")
         if any(r.params.json_mode for r in sample_reqs):
-            tokens = self._constrain_json(sample_reqs, tokens, logits)
-        tokens_t = torch.tensor(tokens, dtype=torch.int64, device=logits.device)
-        # logprob of the chosen token: logit - logsumexp(row)
-        lse = torch.logsumexp(logits, dim=-1)
-        chosen = logits.gather(1, tokens_t.view(-1, 1)).squeeze(1)
-        logprobs = (chosen - lse).cpu().tolist()
+            tokens, logprobs = self._constrain_json(sample_reqs, tokens, logits), None
+        want = max((r.params.logprobs for r in sample_reqs), default=0)
+        if logprobs is None or want > 0:
+            lse = torch.logsumexp(logits, dim=-1)
+        if logprobs is None:
+            # logprob of the chosen token: logit - logsumexp(row)
+            tokens_t = torch.tensor(tokens, dtype=torch.int64, device=logits.device)
+            chosen = logits.gather(1, tokens_t.view(-1, 1)).squeeze(1)
+            logprobs = (chosen - lse).cpu().tolist()
         self.last_logprobs = {
             r.request_id: float(lp) for r, lp in zip(sample_reqs, logprobs)
         }
         # top-alternative logprobs, only when some request asked for them
         self.last_top_logprobs = {}
-        want = max((r.params.logprobs for r in sample_reqs), default=0)
         if want > 0:
             k = min(want, logits.shape[-1])
             tv, ti = (logits - lse.unsqueeze(1)).topk(k, dim=-1)
