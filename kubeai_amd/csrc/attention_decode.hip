@@ -3,9 +3,14 @@
 // Semantics: kubeai_amd/ops/ref.py::paged_attention_decode.
 //
 // Structure:
-//  - workgroup = (sequence, kv head, split of the keys); 4 waves take tiles of
-//    NB cache blocks in turn (32 keys at head size 128, 16 at 256), each with
-//    its own softmax state; the G query heads of the group share every key.
+//  - workgroup = (sequence, kv head, split of the keys); the waves of a row's splits
+//    take tiles in turn, each with its own softmax state; the G query heads of the
+//    group share every key. A tile is one cache block (32 keys over an e5m2 cache at
+//    head size 128): 145 registers and three waves a SIMD, where tiles of 32 keys take
+//    209 and leave room for two (28 rows of 100-700 in 3 splits 17.9 us, 15.9). The first
+//    look-up in the block table does not wait for the row's length.
+//  - which splits there are, and in which order, is worked out on the device once a
+//    step (decode_plan_kernel below), by the rows' lengths.
 //  - S^T = K.Q^T on v_mfma_f32_16x16x32_bf16: a lane reads 16 bytes of one
 //    key straight into the operand (16 keys x 64 contiguous bytes per load,
 //    no LDS), the query heads are columns (lane & 15; those past G repeat the
@@ -26,18 +31,20 @@
 // Bound by reading the cache. The form before this (scores and weighted sum
 // on the vector ALUs) issued about 150 LDS operations per 16 keys, most of
 // them the lane permutes that passed a weight to every lane; here it is 12.
-// Measured, kernel + merge of the splits, us (before -> this):
-//   heads 32/8 x 128, 40 rows of 100-700 keys         41 ->  23
-//   96 rows of 1500-4000                             364 -> 205 (5.4 TB/s; in 2 splits 208)
-//   64 rows of 1536                                  137 ->  74 (5.4 TB/s)
-//     the same, e5m2 cache                           128 ->  45
-//   8 rows of 3584                                    48 ->  31
-//   1 row of 3000 and 7 idle ones                     32 ->  14
-//   heads 64/8 x 128, 32 rows of 1000-3000           165 ->  60
-//   heads 8/4 x 256, cap, 40 rows of 100-700          42 ->  20
-//     96 rows of 2000, no cap                         222 -> 140
-//   heads 4/4 x 256, 96 rows of 2000                  188 -> 142
-// At head size 256 a tile is one block (two would need 512 registers), and over
+// Measured, kernel + merge of the splits, us (the same number of splits for every row
+// and tiles of 32 keys -> planned):
+//   heads 32/8 x 128, 40 rows of 100-700 keys         23.2 -> 18.8, to fp8 25.3 -> 20.1
+//   96 rows of 1500-4000                             209 -> 195 (5.8 TB/s)
+//   64 rows of 100-2000                              60.9 -> 53.4
+//   40 rows of 200, one of 4000                      34.9 -> 15.8, to fp8 37.1 -> 19.6
+//   8 rows of 3584                                    28.8 -> 25.6
+//   1 row of 3000 and 7 idle ones                     12.6 -> 8.7
+//   12 rows of 500                                    13.2 -> 10.5
+//   96 rows of 100-300, one split each                20.5 -> 19.8 (unplanned 18.8)
+//   heads 8/4 x 256, 40 rows of 100-700               21.9 -> 18.4
+//     64 rows of 100-2000                             65.1 -> 60.3
+//     96 rows of 2000                                 139 -> 139.5
+// At head size 256, over
 // a bf16 cache the query lies in LDS: with it in registers 25 were spilled, and
 // the reloads waited for the loads in flight (the last two 236 us).
 #include <torch/extension.h>
@@ -53,11 +60,28 @@ constexpr int kBlockThreads = kWaves * WAVE_SIZE;
 constexpr int kBS = 16;      // cache block size (tokens)
 constexpr int kMaxSplits = 16;
 constexpr int kMaxG = 8;
+constexpr int kCUs = 256;
 
 typedef __attribute__((ext_vector_type(8))) short bf16x8;
 typedef __attribute__((ext_vector_type(4))) short bf16x4;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+
+// One split of a row; a row's splits, which lie behind one another.
+struct alignas(16) Item {
+  int row, len;  // row < 0: none
+  uint16_t split, splits;
+  int part;      // where its results go
+};
+struct alignas(8) Splits {
+  int first, n;
+};
+
+// Cache blocks of a tile.
+constexpr int blocks_per_tile(int hd, int element) { return hd == 128 && element == 1 ? 2 : 1; }
+
+// Waves a SIMD holds: 145 registers at head size 128, 256 at 256.
+constexpr int waves_per_simd(int hd) { return hd == 128 ? 3 : 2; }
 
 // 16 (or 8) bytes a lane from base + at, zeros if size is 0
 template <typename T>
@@ -96,8 +120,8 @@ DEV_INLINE float over_groups(float v, F&& f) {
 // converted to bf16 on the way in, exactly). CAP: s = cap * tanh(s / cap)
 // after scaling and before masking. ONE: no wave has more than one tile.
 template <int HD, typename CT, bool CAP, bool ONE>
-__launch_bounds__(kBlockThreads, 2) __global__ void paged_decode_kernel(
-    ushort* __restrict__ out,            // [B, n_q, hd] bf16
+__launch_bounds__(kBlockThreads, waves_per_simd(HD)) __global__ void paged_decode_kernel(
+    ushort* __restrict__ out,            // [B, n_q, hd] bf16, or null: parts of all rows
     const ushort* __restrict__ q,        // [B, n_q, hd] bf16
     const CT* k_cache,                   // [nb, n_kv, bs, hd]
     const CT* v_cache,
@@ -105,31 +129,45 @@ __launch_bounds__(kBlockThreads, 2) __global__ void paged_decode_kernel(
     const int32_t* __restrict__ seq_lens,      // [B]
     const float scale, const float softcap, const int window,
     const int n_kv, const int G, const int max_blocks,
-    const int64_t q_stride, const int n_splits,
-    float* __restrict__ part_o,    // [B, n_q, n_splits, hd]
-    float* __restrict__ part_ml) { // [B, n_q, n_splits, 2]
-  constexpr int NB = HD == 128 ? 2 : 1;  // cache blocks per tile
+    const int64_t q_stride, const int row_splits,
+    const Item* __restrict__ plan,  // or null: row_splits splits of every row
+    float* __restrict__ part_o,    // [splits of all rows, n_q, hd]
+    float* __restrict__ part_ml) { // [splits of all rows, n_q, 2]
+  constexpr int NB = blocks_per_tile(HD, sizeof(CT));
   constexpr int NC = HD / 32;            // contraction steps of S
   constexpr int ND = HD / 16;            // row blocks of O^T
   constexpr int NV = HD / 32;            // 16-byte V units per lane and block
-  const int b = blockIdx.x / (n_kv * n_splits);
-  const int rem = blockIdx.x % (n_kv * n_splits);
-  const int kh = rem / n_splits;
-  const int split = rem % n_splits;
+  const int item = blockIdx.x / n_kv, kh = blockIdx.x % n_kv;
+  int b, split, n_splits, L, part_row = item;
+  if (plan) {
+    const Item it = plan[item];
+    if (it.row < 0) return;
+    b = it.row;
+    split = it.split;
+    n_splits = it.splits;
+    L = it.len;
+    part_row = it.part;
+  } else {
+    b = item / row_splits;
+    split = item % row_splits;
+    n_splits = row_splits;
+    L = seq_lens[b];
+  }
   const int n_q = n_kv * G;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
   const int lane = threadIdx.x % WAVE_SIZE;
   const int col = lane & 15, grp = lane >> 4;
-  const int L = seq_lens[b];
   const int n_blocks = (L + kBS - 1) / kBS;
   // sliding window: the query (position L-1) attends keys in
   // (L-1-window, L-1]; splits divide the visible blocks only
-  const int w0 = (window > 0) ? max(0, L - window) : 0;
-  const int blk_base = w0 / kBS;
+  int w0 = 0, blk_base = 0;
+  if (window > 0) {
+    w0 = max(0, L - window);
+    blk_base = w0 / kBS;
+  }
   const int n_units = (n_blocks - blk_base + NB - 1) / NB;  // tiles
-  const int chunk = (n_units + n_splits - 1) / n_splits;
-  const int t_lo = split * chunk;
-  const int t_hi = min(n_units, t_lo + chunk);
+  // the waves of all splits take tiles in turn
+  const int turn = kWaves * n_splits;
 
   constexpr int kVTile = NB * kBS * HD;  // elements of a wave's V tile
   constexpr size_t kSmem = sizeof(ushort) * kWaves * kVTile >
@@ -181,7 +219,8 @@ __launch_bounds__(kBlockThreads, 2) __global__ void paged_decode_kernel(
     if constexpr (sizeof(CT) == 2) return u;
     else return __builtin_bit_cast(bf16x8, e5m2x8_to_bf16x8(u));
   };
-  // the cache blocks of tile t (past the last one: that again)
+  // the cache blocks of tile t (past the last one: any entry of the table, not used).
+  // Without a window the first look-up does not wait for the row's length.
   struct Blocks {
     int at[NB];
   };
@@ -189,16 +228,16 @@ __launch_bounds__(kBlockThreads, 2) __global__ void paged_decode_kernel(
     Blocks o;
 #pragma unroll
     for (int j = 0; j < NB; ++j)
-      o.at[j] = bt[min(blk_base + t * NB + j, n_blocks - 1)];
+      o.at[j] = bt[min(blk_base + t * NB + j, max_blocks - 1)];
     return o;
   };
   constexpr int kBlockBytes = kBS * HD * sizeof(CT);
   const int k_at = (col * HD + grp * 8) * sizeof(CT), v_at = lane * 8 * sizeof(CT);
-  // a tile behind the last one: loads of no bytes
+  // blocks behind the last one: loads of no bytes
   auto load_tile = [&](int set, int t, const Blocks& blocks) {
-    const int size = t < t_hi ? kBlockBytes : 0;
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
+      const int size = blk_base + t * NB + j < n_blocks ? kBlockBytes : 0;
       const int64_t base = ((int64_t)blocks.at[j] * n_kv + kh) * (kBS * HD);
 #pragma unroll
       for (int c = 0; c < NC; ++c)
@@ -325,23 +364,24 @@ __launch_bounds__(kBlockThreads, 2) __global__ void paged_decode_kernel(
 
   // (no load in a branch: where paths of more and of fewer loads meet, the compiler
   // waits for all of them)
-  const int first = t_lo + wave;
-  if (first < t_hi) {
-    load_tile(0, first, look_up(first));
+  const int first = split * kWaves + wave;
+  const Blocks start = look_up(first);
+  if (first < n_units) {
+    load_tile(0, first, start);
     if constexpr (ONE) {
       compute(0, first);
     } else {
-      Blocks even, odd = look_up(first + kWaves);
-      for (int t = first; t < t_hi; t += 2 * kWaves) {
-        load_tile(1, t + kWaves, odd);
-        even = look_up(t + 2 * kWaves);
+      Blocks even, odd = look_up(first + turn);
+      for (int t = first; t < n_units; t += 2 * turn) {
+        load_tile(1, t + turn, odd);
+        even = look_up(t + 2 * turn);
         in_order();
         compute(0, t);
         in_order();
-        load_tile(0, t + 2 * kWaves, even);
-        odd = look_up(t + 3 * kWaves);
+        load_tile(0, t + 2 * turn, even);
+        odd = look_up(t + 3 * turn);
         in_order();
-        if (t + kWaves < t_hi) compute(1, t + kWaves);
+        if (t + turn < n_units) compute(1, t + turn);
       }
     }
   }
@@ -376,7 +416,8 @@ __launch_bounds__(kBlockThreads, 2) __global__ void paged_decode_kernel(
       o += *reinterpret_cast<const f32x4*>(merge_o + (w * G + g) * HD + e) * c;
     }
     const int64_t head = (int64_t)b * n_q + kh * G + g;
-    if (n_splits == 1) {
+    const int64_t part = (int64_t)part_row * n_q + kh * G + g;
+    if (n_splits == 1 && out) {
       const float inv_l = 1.0f / l_star;
       ushort4_t r;
 #pragma unroll
@@ -384,55 +425,88 @@ __launch_bounds__(kBlockThreads, 2) __global__ void paged_decode_kernel(
       *reinterpret_cast<ushort4_t*>(out + head * HD + e) = r;
     } else {
       // partial results (an empty split writes m = -inf, l = 0, o = 0)
-      *reinterpret_cast<f32x4*>(part_o + (head * n_splits + split) * HD + e) = o;
+      *reinterpret_cast<f32x4*>(part_o + part * HD + e) = o;
       if (e == 0) {
-        part_ml[(head * n_splits + split) * 2] = m_star;
-        part_ml[(head * n_splits + split) * 2 + 1] = l_star;
+        part_ml[part * 2] = m_star;
+        part_ml[part * 2 + 1] = l_star;
       }
     }
   }
 }
 
 // Merged values of one query head, 2 or 4 a lane, rounded to bf16. The lanes read
-// all splits' (m, l) at once and the rows of O are independent loads.
+// all splits' (m, l) at once; the rows of O are on their way before those are used, up
+// to 16 at a time (as many as a row has splits), 4 where there are no more.
 template <int HD>
 struct Merged {
   static constexpr int EPL = HD / 64;
+  typedef __attribute__((ext_vector_type(EPL))) float vec;
   ushort v[EPL];
-  DEV_INLINE Merged(const float* part_o, const float* part_ml, int n_splits, int64_t bh) {
-    typedef __attribute__((ext_vector_type(EPL))) float vec;
+  float ms, ls;
+  const vec* po;
+  int64_t step;
+  int n;
+  vec o[kMaxSplits];
+
+  // the head's parts lie n_q apart, at first + head and on
+  template <int MOST>
+  DEV_INLINE void load(const float* part_o, const float* part_ml, Splits of, int n_q,
+                       int head) {
     const int lane = threadIdx.x % WAVE_SIZE;
-    const float* pml = part_ml + bh * n_splits * 2;
-    const vec* po = reinterpret_cast<const vec*>(part_o + bh * n_splits * HD) + lane;
-    const int s = min(lane, n_splits - 1);
-    const float ms = pml[2 * s], ls = lane < n_splits ? pml[2 * s + 1] : 0.f;
+    const int64_t first = (int64_t)of.first * n_q + head;
+    n = of.n;
+    step = (int64_t)n_q * 64;
+    const float* pml = part_ml + (first + (int64_t)min(lane, n - 1) * n_q) * 2;
+    po = reinterpret_cast<const vec*>(part_o + first * HD) + lane;
+    ms = pml[0];
+    ls = pml[1];
+#pragma unroll
+    for (int k = 0; k < MOST; ++k) o[k] = po[min(k, n - 1) * step];
+  }
+  template <int MOST>
+  DEV_INLINE void finish() {
+    const int lane = threadIdx.x % WAVE_SIZE;
     const float m_star = wave_reduce_max(ms);
     const float c = __builtin_amdgcn_exp2f(ms - (m_star == -INFINITY ? 0.f : m_star));
-    const float l_star = wave_reduce_sum(ls * c);
-    vec o;
+    const float l_star = wave_reduce_sum(lane < n ? ls * c : 0.f);
+    vec sum;
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) o[e] = 0.f;
-#pragma unroll 4
-    for (int k = 0; k < n_splits; ++k)
-      o += po[k * 64] * __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(c), k));
+    for (int e = 0; e < EPL; ++e) sum[e] = 0.f;
+#pragma unroll
+    for (int k = 0; k < MOST; ++k)
+      if (k < n) sum += o[k] * __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(c), k));
     const float inv_l = 1.0f / l_star;
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) v[e] = f32_to_bf16(o[e] * inv_l);
+    for (int e = 0; e < EPL; ++e) v[e] = f32_to_bf16(sum[e] * inv_l);
   }
 };
 
-// Merge the splits' results: one wave per (sequence, query head).
+// a row's splits, from the plan or the same number for all
+DEV_INLINE Splits splits_of(const Splits* plan, int n, int row) {
+  return plan ? plan[row] : Splits{row * n, n};
+}
+
+// Merge the splits' results: one wave per (sequence, query head). A planned row that
+// was not split has its result.
 template <int HD>
 __global__ void decode_merge_kernel(
     ushort* __restrict__ out,             // [B, n_q, hd]
-    const float* __restrict__ part_o,     // [B, n_q, n_splits, hd]
-    const float* __restrict__ part_ml,    // [B, n_q, n_splits, 2]
-    const int n_splits, const int64_t n_bh) {
+    const float* __restrict__ part_o, const float* __restrict__ part_ml,
+    const Splits* __restrict__ plan, const int n_splits, const int n_q,
+    const int64_t n_bh) {
   constexpr int EPL = HD / 64;
   const int64_t bh = (int64_t)blockIdx.x * (blockDim.x / WAVE_SIZE) +
                      threadIdx.x / WAVE_SIZE;
   if (bh >= n_bh) return;
-  const Merged<HD> m(part_o, part_ml, n_splits, bh);
+  const Splits of = splits_of(plan, n_splits, (int)(bh / n_q));
+  if (of.n == 1) return;
+  Merged<HD> m;
+  auto merge = [&](auto most) {
+    m.template load<decltype(most)::value>(part_o, part_ml, of, n_q, (int)(bh % n_q));
+    m.template finish<decltype(most)::value>();
+  };
+  if (of.n <= 4) merge(std::integral_constant<int, 4>{});
+  else merge(std::integral_constant<int, kMaxSplits>{});
   ushort* oh = out + bh * HD + EPL * (threadIdx.x % WAVE_SIZE);
 #pragma unroll
   for (int e = 0; e < EPL; e += 2)
@@ -449,25 +523,32 @@ __launch_bounds__(16 * WAVE_SIZE) __global__ void decode_merge_fp8_kernel(
     unsigned char* __restrict__ out,      // [B, n_q * hd]
     float* __restrict__ out_scale,        // [B]
     const float* __restrict__ part_o, const float* __restrict__ part_ml,
-    const int n_splits, const int n_q) {
+    const Splits* __restrict__ plan, const int n_splits, const int n_q) {
   constexpr int EPL = HD / 64;
   const int wave = threadIdx.x / WAVE_SIZE, lane = threadIdx.x % WAVE_SIZE;
   const int64_t row = blockIdx.x;
+  const Splits of = splits_of(plan, n_splits, (int)row);
   __shared__ float red[16];
   float vals[HPW][EPL];
   float amax = 0.f;
+  Merged<HD> m[HPW];
+  auto merge = [&](auto most) {
+    constexpr int MOST = decltype(most)::value;
 #pragma unroll
-  for (int h = 0; h < HPW; ++h) {
-    const int head = h * 16 + wave;
-    if (head < n_q) {  // the same in every lane
-      const Merged<HD> m(part_o, part_ml, n_splits, row * n_q + head);
+    for (int h = 0; h < HPW; ++h)  // (past the last head: that again)
+      m[h].template load<MOST>(part_o, part_ml, of, n_q, min(h * 16 + wave, n_q - 1));
+#pragma unroll
+    for (int h = 0; h < HPW; ++h) {
+      m[h].template finish<MOST>();
 #pragma unroll
       for (int e = 0; e < EPL; ++e) {
-        vals[h][e] = bf16_to_f32(m.v[e]);
+        vals[h][e] = bf16_to_f32(m[h].v[e]);
         amax = fmaxf(amax, fabsf(vals[h][e]));
       }
     }
-  }
+  };
+  if (of.n <= 4) merge(std::integral_constant<int, 4>{});
+  else merge(std::integral_constant<int, kMaxSplits>{});
   amax = wave_reduce_max(amax);
   if (lane == 0) red[wave] = amax;
   __syncthreads();
@@ -494,9 +575,138 @@ __launch_bounds__(16 * WAVE_SIZE) __global__ void decode_merge_fp8_kernel(
   }
 }
 
+
+// How the rows of a step are split, and in which order the splits are worked through.
+// One workgroup; threads 8 c + r weigh candidate c over every eighth row.
+//
+// A CU reads at most about 56 GB/s (3000 keys of one head in one workgroup of 4, 6 or
+// 12 waves: 33 us all of them), so a step takes as long as the CU with the most keys.
+// M = CUs / kv heads splits fill the chip once. A candidate is a largest number of
+// tiles to a split; it costs, in tiles, its largest split or that many rounds of the
+// mean one, and kSplitCost a round for what a split costs beside its tiles. Splits go to
+// the CUs in turn, so they are ordered largest first, and every second round backwards:
+// each CU's share is about the same, and CUs with a split less than the others get the
+// largest.
+constexpr int kPlanThreads = 256, kCandidates = 32, kPlanRows = 1024;
+constexpr float kSplitCost = 6.f;  // tiles
+constexpr int kLeastTiles = 8;     // that a split is cut to
+
+DEV_INLINE int all_sum(int v) {
+#pragma unroll
+  for (int d = 1; d < 64; d *= 2) v += __shfl_xor(v, d);
+  return v;
+}
+
+__global__ void __launch_bounds__(kPlanThreads) decode_plan_kernel(
+    Item* __restrict__ items, Splits* __restrict__ rows, const int32_t* __restrict__ seq_lens,
+    const int B, const int n_items, const int M, const int window, const int tile_keys) {
+  // a row's tiles, then its splits and their size (from the front, padded with none)
+  __shared__ __attribute__((aligned(16))) int tiles[kPlanRows], sizes[kPlanRows];
+  __shared__ int lens[kPlanRows];
+  __shared__ int total[kPlanThreads / 64];
+  __shared__ float best_cost[kPlanThreads / 64];
+  __shared__ int best_limit[kPlanThreads / 64];
+  const int t = threadIdx.x, padded = (B + 7) / 8 * 8;
+  int mine = 0;
+  for (int i = t; i < padded; i += kPlanThreads) {
+    int n = 0;
+    if (i < B) {
+      lens[i] = seq_lens[i];
+      const int L = max(1, lens[i]);
+      const int first = window > 0 ? max(0, L - window) / kBS * kBS : 0;
+      n = (L - first + tile_keys - 1) / tile_keys;
+    }
+    tiles[i] = n;
+    mine += n;
+  }
+  mine = all_sum(mine);
+  if (t % 64 == 0) total[t / 64] = mine;
+  __syncthreads();
+  float all = 0.f;
+#pragma unroll
+  for (int w = 0; w < kPlanThreads / 64; ++w) all += (float)total[w];
+  // candidate c: splits of at most all / (3 M 0.9^c) tiles
+  const int c = t / 8;
+  const int limit =
+      max(kLeastTiles, (int)ceilf(all / (3.f * M * __builtin_amdgcn_exp2f(-0.152003f * c))));
+  float n = 0.f, large = 0.f;
+  const float inv = 1.f / limit;
+  for (int i = t % 8; i < padded; i += 8) {
+    const float x = (float)tiles[i], k = fminf(ceilf(x * inv), (float)kMaxSplits);
+    n += k;
+    large = fmaxf(large, k > 0.f ? x * __builtin_amdgcn_rcpf(k) : 0.f);
+  }
+#pragma unroll
+  for (int d = 1; d < 8; d *= 2) {
+    n += __shfl_xor(n, d);
+    large = fmaxf(large, __shfl_xor(large, d));
+  }
+  float cost = fmaxf(large, ceilf(n / M) * all / n) + kSplitCost * n / M;
+  int of = limit;
+#pragma unroll
+  for (int d = 8; d < 64; d *= 2) {
+    const float other = __shfl_xor(cost, d);
+    const int l = __shfl_xor(of, d);
+    if (other < cost || (other == cost && l > of)) {
+      cost = other;
+      of = l;
+    }
+  }
+  if (t % 64 == 0) {
+    best_cost[t / 64] = cost;
+    best_limit[t / 64] = of;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kPlanThreads / 64; ++w) {
+    if (best_cost[w] < cost || (best_cost[w] == cost && best_limit[w] > of)) {
+      cost = best_cost[w];
+      of = best_limit[w];
+    }
+  }
+  for (int i = t; i < padded; i += kPlanThreads) {
+    const int x = tiles[i], k = min(kMaxSplits, (x + of - 1) / of);
+    // size in front: rows by it, their splits (up to 16) below
+    sizes[i] = k ? ((x + k - 1) / k) << 5 | k : 0;
+  }
+  __syncthreads();
+  for (int i = t; i < B; i += kPlanThreads) {
+    const int own = sizes[i] >> 5, k_own = sizes[i] & 31;
+    int first = 0, N = 0;
+#pragma unroll 4
+    for (int j = 0; j < padded; j += 4) {
+      const int4 four = *reinterpret_cast<const int4*>(sizes + j);
+      const int e[4] = {four.x, four.y, four.z, four.w};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int size = e[q] >> 5, k = e[q] & 31;
+        N += k;
+        if (size > own || (size == own && j + q < i)) first += k;
+      }
+    }
+    rows[i] = {first, k_own};
+    const int rounds = (N + M - 1) / M, rest = N - (rounds - 1) * M;  // CUs of the last one
+    const int L = lens[i];
+    int round = first / M, x = first - round * M;
+    for (int k = 0; k < k_own; ++k) {
+      int cu;
+      if (round == rounds - 1) cu = round % 2 ? rest - 1 - x : x;
+      else if (round % 2) cu = x < rest ? rest - 1 - x : M - 1 - (x - rest);
+      else cu = x < M - rest ? rest + x : x - (M - rest);
+      items[round * M + cu] = {i, L, (uint16_t)k, (uint16_t)k_own, first + k};
+      if (++x == M) {
+        x = 0;
+        ++round;
+      }
+    }
+    if (i == 0) total[0] = N;
+  }
+  __syncthreads();
+  for (int i = total[0] + t; i < n_items; i += kPlanThreads) items[i] = {-1, 0, 0, 0, 0};
+}
 }  // namespace
 
-// How often a row's keys are split: until there are 512 workgroups (two a CU).
+// How often a row's keys are split without a plan: until there are 512 workgroups (two a CU).
 // The lengths are not known here; more splits cost in the merge, and a row that
 // is much longer than the others is worked through by its own splits alone. At
 // head size 256, whose workgroups read a row at half the rate of those at 128,
@@ -505,8 +715,8 @@ __launch_bounds__(16 * WAVE_SIZE) __global__ void decode_merge_fp8_kernel(
 // idle ones 13.6 at 512, 17.0 at 1536. Head size 256: 128 rows of 300 but one
 // of 8000, 4 kv heads 224 us at 512, 122 at 576, 87 at 1536; 8 rows of 3500, e5m2
 // cache, 8 kv heads 33 at 512, 42 at 576; 40 rows of 100-700, e5m2 cache, 4 kv
-// heads 19.3 at 512 and 576, 22 at 768, 25 at 1536. A split has at least one
-// tile of the widest row. KUBEAI_DECODE_SPLIT_TARGET overrides for tuning sweeps.
+// heads 19.3 at 512 and 576, 22 at 768, 25 at 1536. (Measured with tiles of 32 keys.) A
+// split has at least 32 keys of the widest row, 16 at head size 256. KUBEAI_DECODE_SPLIT_TARGET overrides for tuning sweeps.
 int paged_decode_splits(int rows, int n_kv, int hd, int max_blocks) {
   static const int forced = []() {
     const char* e = getenv("KUBEAI_DECODE_SPLIT_TARGET");
@@ -519,12 +729,36 @@ int paged_decode_splits(int rows, int n_kv, int hd, int max_blocks) {
       1, std::min({(int64_t)kMaxSplits, (int64_t)tiles, (target + wgs - 1) / wgs}));
 }
 
+// The splits of a step's rows, for paged_attention_decode over any caches of this many
+// kv heads, head size, element and window while the lengths are these: int32 [4 items +
+// 2 rows], the items in front.
+torch::Tensor paged_decode_plan(torch::Tensor seq_lens, int64_t n_kv, int64_t hd,
+                                int64_t element_size, int64_t window) {
+  TORCH_CHECK(seq_lens.scalar_type() == torch::kInt32 && seq_lens.is_contiguous() &&
+              seq_lens.is_cuda() && seq_lens.dim() == 1);
+  const int B = (int)seq_lens.size(0);
+  TORCH_CHECK(B >= 1 && B <= kPlanRows, "1 to ", kPlanRows, " rows");
+  TORCH_CHECK(n_kv >= 1 && (hd == 128 || hd == 256) && (element_size == 1 || element_size == 2));
+  const int M = std::max<int64_t>(1, kCUs / n_kv);
+  const int64_t n_items = 3 * M + B;  // (what the first candidate may need)
+  auto plan = torch::empty({4 * n_items + 2 * B}, seq_lens.options());
+  auto* items = reinterpret_cast<Item*>(plan.data_ptr());
+  hipLaunchKernelGGL(decode_plan_kernel, dim3(1), dim3(kPlanThreads), 0,
+                     c10::hip::getCurrentHIPStream().stream(), items,
+                     reinterpret_cast<Splits*>(items + n_items), seq_lens.data_ptr<int32_t>(),
+                     B, (int)n_items, M, (int)window,
+                     kBS * blocks_per_tile((int)hd, (int)element_size));
+  HIP_CHECK_KERNEL();
+  return plan;
+}
+
 // out [B, n_q, hd] bf16, or with out_scale [B] fp8 rows with a scale each
 void paged_attention_decode(torch::Tensor out, torch::Tensor q,
                             torch::Tensor k_cache, torch::Tensor v_cache,
                             torch::Tensor block_tables, torch::Tensor seq_lens,
                             double scale, int64_t window, double softcap,
-                            c10::optional<torch::Tensor> out_scale) {
+                            c10::optional<torch::Tensor> out_scale,
+                            c10::optional<torch::Tensor> plan) {
   TORCH_CHECK(q.stride(2) == 1 && q.stride(1) == q.size(2));
   TORCH_CHECK(out.is_contiguous() && out.numel() >= q.numel());
   TORCH_CHECK(k_cache.is_contiguous() && v_cache.is_contiguous());
@@ -545,42 +779,55 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
   TORCH_CHECK(G == 1 || G == 2 || G == 4 || G == 5 || G == 6 || G == 8,
               "unsupported GQA group size ", G);
   const int n_splits = paged_decode_splits(B, n_kv, hd, max_blocks);
+  const Item* items = nullptr;
+  const Splits* row_splits = nullptr;
+  int64_t parts = (int64_t)B * n_splits;
+  if (plan.has_value()) {
+    TORCH_CHECK(plan->scalar_type() == torch::kInt32 && plan->is_contiguous() &&
+                plan->is_cuda() && plan->dim() == 1 && plan->numel() >= 6 * B &&
+                (plan->numel() - 2 * B) % 4 == 0 && ((uintptr_t)plan->data_ptr() & 15) == 0);
+    parts = (plan->numel() - 2 * B) / 4;
+    items = reinterpret_cast<const Item*>(plan->data_ptr());
+    row_splits = reinterpret_cast<const Splits*>(items + parts);
+  }
   const bool fp8 = out_scale.has_value();
   TORCH_CHECK(out.scalar_type() == (fp8 ? torch::kFloat8_e4m3fn : torch::kBFloat16));
   if (fp8)
-    TORCH_CHECK(n_splits > 1 && n_q <= 32 && out_scale->is_contiguous() &&
+    TORCH_CHECK((items || n_splits > 1) && n_q <= 32 && out_scale->is_contiguous() &&
                     out_scale->scalar_type() == torch::kFloat32 && out_scale->numel() == B,
                 "fp8 rows come from the merge of up to 32 heads");
   torch::Tensor part_o, part_ml;
   float *part_o_ptr = nullptr, *part_ml_ptr = nullptr;
-  if (n_splits > 1) {
+  const bool merged = items || n_splits > 1;
+  if (merged) {
     auto opts =
         torch::TensorOptions().device(q.device()).dtype(torch::kFloat32);
-    part_o = torch::empty({B, n_q, n_splits, (int64_t)hd}, opts);
-    part_ml = torch::empty({B, n_q, n_splits, 2}, opts);
+    part_o = torch::empty({parts, n_q, (int64_t)hd}, opts);
+    part_ml = torch::empty({parts, n_q, 2}, opts);
     part_o_ptr = part_o.data_ptr<float>();
     part_ml_ptr = part_ml.data_ptr<float>();
   }
-  const dim3 grid((uint32_t)((int64_t)B * n_kv * n_splits)), block(kBlockThreads);
+  TORCH_CHECK(parts * n_kv < (int64_t)1 << 31);
+  const dim3 grid((uint32_t)(parts * n_kv)), block(kBlockThreads);
   auto stream = c10::hip::getCurrentHIPStream().stream();
-  // (12 rows of 500: 14.9 us with the loop's loads of no bytes, 13.9 without)
-  const int tiles = hd == 256 ? max_blocks : (max_blocks + 1) / 2;
-  const bool few = (tiles + n_splits - 1) / n_splits <= kWaves;
   auto launch = [&](auto hdv, auto ct, auto cap, auto one) {
     using CT = decltype(ct);
     hipLaunchKernelGGL(
         (paged_decode_kernel<decltype(hdv)::value, CT, decltype(cap)::value,
                              decltype(one)::value>),
-        grid, block, 0, stream, (ushort*)out.data_ptr(),
+        grid, block, 0, stream, fp8 ? nullptr : (ushort*)out.data_ptr(),
         (const ushort*)q.data_ptr(), (const CT*)k_cache.data_ptr(),
         (const CT*)v_cache.data_ptr(), block_tables.data_ptr<int32_t>(),
         seq_lens.data_ptr<int32_t>(), (float)scale, (float)softcap,
-        (int)window, n_kv, G, max_blocks, q.stride(0), n_splits, part_o_ptr,
+        (int)window, n_kv, G, max_blocks, q.stride(0), n_splits, items, part_o_ptr,
         part_ml_ptr);
   };
+  // (12 rows of 500: 14.9 us with the loop's loads of no bytes, 13.9 without)
+  const int nb = blocks_per_tile(hd, k_cache.element_size());
+  const bool one = !items && (max_blocks + nb - 1) / nb <= n_splits * kWaves;
   auto with_cap = [&](auto hdv, auto ct) {
     auto with_one = [&](auto capped) {
-      if (few) launch(hdv, ct, capped, std::true_type{});
+      if (one) launch(hdv, ct, capped, std::true_type{});
       else launch(hdv, ct, capped, std::false_type{});
     };
     if (softcap > 0.0) with_one(std::true_type{});
@@ -598,7 +845,7 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
       hipLaunchKernelGGL(
           (decode_merge_fp8_kernel<decltype(hdv)::value, decltype(hpw)::value>), dim3(B),
           dim3(16 * WAVE_SIZE), 0, stream, (unsigned char*)out.data_ptr(),
-          out_scale->data_ptr<float>(), part_o_ptr, part_ml_ptr, n_splits, n_q);
+          out_scale->data_ptr<float>(), part_o_ptr, part_ml_ptr, row_splits, n_splits, n_q);
     };
     auto heads = [&](auto hdv) {
       if (n_q <= 16) merge(hdv, std::integral_constant<int, 1>{});
@@ -607,18 +854,18 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
     if (hd == 256) heads(std::integral_constant<int, 256>{});
     else heads(std::integral_constant<int, 128>{});
     HIP_CHECK_KERNEL();
-  } else if (n_splits > 1) {
+  } else if (merged) {
     const int64_t n_bh = (int64_t)B * n_q;
     const int wpb = 4;
     const dim3 mgrid((uint32_t)((n_bh + wpb - 1) / wpb)), mblock(wpb * WAVE_SIZE);
     if (hd == 256)
       hipLaunchKernelGGL((decode_merge_kernel<256>), mgrid, mblock, 0, stream,
                          (ushort*)out.data_ptr(), part_o_ptr, part_ml_ptr,
-                         n_splits, n_bh);
+                         row_splits, n_splits, n_q, n_bh);
     else
       hipLaunchKernelGGL((decode_merge_kernel<128>), mgrid, mblock, 0, stream,
                          (ushort*)out.data_ptr(), part_o_ptr, part_ml_ptr,
-                         n_splits, n_bh);
+                         row_splits, n_splits, n_q, n_bh);
     HIP_CHECK_KERNEL();
   }
 }

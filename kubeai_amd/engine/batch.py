@@ -46,6 +46,10 @@ class ForwardBatch:
     # built only for models that carry per-sequence state
     seq: "object | None" = None
 
+    # how the decode rows are split over workgroups (ops.decode_plan), by kind of cache;
+    # a dict while a model's forward runs, whose layers share it
+    decode_plans: dict | None = None
+
     @property
     def n_tokens(self) -> int:
         return self.input_ids.shape[0]

@@ -201,12 +201,15 @@ class Attention(nn.Module):
             )
 
         nd = fb.n_decode
+        plan = ops.decode_plan(
+            fb.decode_plans, fb.decode_seq_lens, fb.decode_block_tables, k_cache, self.window
+        ) if nd > 0 else None
         if fp8_in and nd == T and fb.n_prefill == 0:
             return _project(
                 self.o_proj,
                 ops.paged_attention_decode_fp8(
                     q, k_cache, v_cache, fb.decode_block_tables, fb.decode_seq_lens,
-                    self.scale, window=self.window, softcap=self.softcap,
+                    self.scale, window=self.window, softcap=self.softcap, plan=plan,
                 ),
                 as_sums, fb,
             )
@@ -224,6 +227,7 @@ class Attention(nn.Module):
                 out=out[:nd],
                 window=self.window,
                 softcap=self.softcap,
+                plan=plan,
             )
         if fb.n_prefill > 0:
             ops.paged_attention_prefill(
@@ -800,6 +804,13 @@ class LlamaForCausalLM(nn.Module):
         if fb.mm_embeds is not None:
             # image-placeholder positions take the vision-tower embeddings
             x = x.index_copy(0, fb.mm_idx, fb.mm_embeds.to(x.dtype))
+        fb.decode_plans = {}
+        try:
+            return self._run_layers(x, fb, cs)
+        finally:
+            fb.decode_plans = None
+
+    def _run_layers(self, x, fb, cs):
         residual = None
         n = len(self.layers)
         # layers that nobody else looks at hand on products that the next one's

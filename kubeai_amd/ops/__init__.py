@@ -124,21 +124,39 @@ def rope_and_cache(qkv, n_q: int, positions, cos_sin, k_cache, v_cache, slot_map
     return q
 
 
+def decode_plan(plans, seq_lens, block_tables, k_cache, window: int = 0):
+    """How paged_attention_decode best splits rows of these lengths over caches like
+    k_cache, worked out on the GPU once for all layers of a step: `plans` is the step's
+    dict, which must not outlive it (None: no plan). A plan holds for the lengths that
+    seq_lens had when it was made; recorded in a graph it is made again by each replay."""
+    if plans is None or not seq_lens.is_cuda or not 1 <= seq_lens.shape[0] <= 1024:
+        return None
+    n_kv, bs, hd = k_cache.shape[1:]
+    if window >= block_tables.shape[1] * bs:
+        window = 0  # no row is longer
+    key = (n_kv, hd, k_cache.element_size(), window)
+    if key not in plans:
+        _require_ext()
+        plans[key] = _C.paged_decode_plan(seq_lens, *key)
+    return plans[key]
+
+
 def paged_attention_decode(
     q, k_cache, v_cache, block_tables, seq_lens, scale: float, out=None,
-    window: int = 0, softcap: float = 0.0,
+    window: int = 0, softcap: float = 0.0, plan=None,
 ):
     """q may be a row-strided view (fused qkv output); out must be
     contiguous (allocated here if not supplied). window > 0 enables
     sliding-window attention (Mistral/Gemma2 style: keys in
-    (pos-window, pos])."""
+    (pos-window, pos]). plan: decode_plan of these lengths (another order of the
+    sums)."""
     if q.is_cuda:
         _require_ext()
         if out is None:
             out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
         _C.paged_attention_decode(
             out, q, k_cache, v_cache, block_tables, seq_lens, scale, window,
-            softcap
+            softcap, None, plan
         )
         return out
     res = ref.paged_attention_decode(
@@ -153,32 +171,35 @@ def paged_attention_decode(
 
 def decode_fp8_merges(n_q: int, splits: int) -> bool:
     """Whether the merge of a decode row's splits best converts the row to fp8 as
-    well. One workgroup has the row then, and a wave of it merges a head for each 16
-    of the row, one behind the other, where the merge by itself has a wave per head (us
-    with the attention, two launches / one: 16 heads 4 rows in 16 splits 16.0 / 14.3,
-    72 rows in 2 13.2 / 10.9; 32 heads 38 rows in 2 splits 13.9 / 13.1, 7 rows in 4
-    10.7 / 10.9, 7 in 10 14.2 / 15.9, 2 in 16 13.9 / 17.8; 64 heads 25 rows in 2 12.1 /
-    14.0, 2 in 12 13.7 / 24.7)."""
+    well, where all rows have this many. One workgroup has the row then, and a wave of it
+    merges a head for each 16 of the row, where the merge by itself has a wave per head
+    (us with the attention, two launches / one: 16 heads 4 rows in 16 splits 16.0 / 14.3,
+    72 rows in 2 13.2 / 10.9; 32 heads 38 rows of 400 in 2 splits 19.6 / 18.8, 7 rows of
+    900 in 10 13.6 / 15.5, in 16 12.4 / 13.5; 64 heads 25 rows in 2 12.1 / 14.0, 2 in 12
+    13.7 / 24.7). Planned splits are merged so up to 32 heads: most rows have one or two
+    (the same 38 rows 20.1 / 19.0, the 7 11.7 / 10.9)."""
     return splits > 1 and (n_q <= 16 or n_q <= 32 and splits <= 4)
 
 
 def paged_attention_decode_fp8(
     q, k_cache, v_cache, block_tables, seq_lens, scale: float, window: int = 0,
-    softcap: float = 0.0,
+    softcap: float = 0.0, plan=None,
 ):
     """quant_fp8 of paged_attention_decode's rows [B, n_q * hd]. On GPU the merge of
     a row's splits converts them, where that is the faster form."""
     B, n_q, hd = q.shape
-    if not q.is_cuda or B == 0 or not decode_fp8_merges(
-        n_q, _C.paged_decode_splits(B, k_cache.shape[1], hd, block_tables.shape[1])
+    if not q.is_cuda or B == 0 or not (
+        n_q <= 32 if plan is not None else decode_fp8_merges(
+            n_q, _C.paged_decode_splits(B, k_cache.shape[1], hd, block_tables.shape[1])
+        )
     ):
         out = paged_attention_decode(q, k_cache, v_cache, block_tables, seq_lens, scale,
-                                     window=window, softcap=softcap)
+                                     window=window, softcap=softcap, plan=plan)
         return quant_fp8(out.view(B, n_q * hd))
     out = torch.empty((B, n_q * hd), dtype=torch.float8_e4m3fn, device=q.device)
     out_scale = torch.empty(B, dtype=torch.float32, device=q.device)
     _C.paged_attention_decode(out, q, k_cache, v_cache, block_tables, seq_lens, scale,
-                              window, softcap, out_scale)
+                              window, softcap, out_scale, plan)
     return out, out_scale
 
 

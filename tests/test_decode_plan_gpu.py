@@ -1,0 +1,105 @@
+"""Decode attention over planned splits against the reference, and what a plan holds."""
+import random
+
+import pytest
+import torch
+
+from kubeai_amd import ops
+from kubeai_amd.ops import ref
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+BS = 16
+
+
+def _caches(lens, n_kv, hd, dtype, seed):
+    need = [max(1, -(-n // BS)) for n in lens]
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    kc, vc = (torch.randn(sum(need) + 1, n_kv, BS, hd, device=DEV, generator=g).to(dtype)
+              for _ in range(2))
+    ids = list(range(1, sum(need) + 1))
+    random.Random(seed).shuffle(ids)
+    bt = torch.zeros(len(lens), max(need), dtype=torch.int32)
+    for i, n in enumerate(need):
+        bt[i, :n] = torch.tensor([ids.pop() for _ in range(n)])
+    return kc, vc, bt.to(DEV), torch.tensor(lens, dtype=torch.int32, device=DEV)
+
+
+LENGTHS = {
+    "one": [1], "one long": [5003], "one of many": [37] * 9 + [3000] + [200] * 14,
+    "edges": [1, 15, 16, 17, 31, 32, 33, 127, 128, 129, 255, 256, 257, 2048, 2049],
+    "even": [512] * 32, "many": [1 + 7 * i % 400 for i in range(130)],
+}
+
+
+@pytest.mark.parametrize("lens", LENGTHS.values(), ids=LENGTHS.keys())
+@pytest.mark.parametrize("n_kv,tile,window", [(8, 16, 0), (1, 32, 0), (4, 16, 100), (300, 16, 0)])
+def test_plan_names_every_split_once(lens, n_kv, tile, window):
+    sl = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    plan = ops._C.paged_decode_plan(sl, n_kv, 128, 2 if tile == 16 else 1, window).cpu()
+    B, M = len(lens), max(1, 256 // n_kv)
+    n = 3 * M + B
+    items, rows = plan[: 4 * n].view(n, 4).tolist(), plan[4 * n :].view(B, 2).tolist()
+    used = sum(k for _, k in rows)
+    assert sorted(i for at, k in rows for i in range(at, at + k)) == list(range(used))
+    got = {}
+    for row, length, packed, part in items[:used]:
+        split, splits = packed & 0xFFFF, packed >> 16
+        at, k = rows[row]
+        assert length == lens[row] and splits == k and part == at + split and 0 <= split < k
+        got.setdefault(row, set()).add(split)
+    assert all(got[i] == set(range(rows[i][1])) for i in range(B))
+    assert all(it[0] == -1 for it in items[used:])
+    assert all(1 <= k <= 16 for _, k in rows)
+
+
+@pytest.mark.parametrize("lens", LENGTHS.values(), ids=LENGTHS.keys())
+@pytest.mark.parametrize("n_q,n_kv,hd,dtype,window,cap", [
+    (32, 8, 128, torch.bfloat16, 0, 0.0),
+    (8, 1, 128, torch.float8_e5m2, 0, 0.0),
+    (8, 4, 256, torch.bfloat16, 100, 30.0),
+    (40, 8, 128, torch.bfloat16, 700, 0.0),
+])
+def test_planned_attention(lens, n_q, n_kv, hd, dtype, window, cap):
+    kc, vc, bt, sl = _caches(lens, n_kv, hd, dtype, n_q + len(lens))
+    q = torch.randn(len(lens), n_q, hd, device=DEV).bfloat16()
+    plans = {}
+    plan = ops.decode_plan(plans, sl, bt, kc, window)
+    assert ops.decode_plan(plans, sl, bt, kc, window) is plan  # one a step
+    kw = dict(window=window, softcap=cap)
+    got = ops.paged_attention_decode(q, kc, vc, bt, sl, hd**-0.5, plan=plan, **kw)
+    want = ref.paged_attention_decode(q.float(), kc.float(), vc.float(), bt, sl, hd**-0.5, **kw)
+    # rounded once to bf16 (half a unit, 2^-9), fp32 within
+    err = (got.float() - want).abs()
+    assert torch.all(err <= 2.0**-8 * want.abs() + 1e-4)
+    f8, scale = ops.paged_attention_decode_fp8(q, kc, vc, bt, sl, hd**-0.5, plan=plan, **kw)
+    w8, wscale = ops.quant_fp8(got.view(len(lens), -1))
+    assert torch.equal(f8.view(torch.uint8), w8.view(torch.uint8))
+    assert torch.equal(scale, wscale.view(-1))
+
+
+def test_no_plan():
+    kc, vc, bt, sl = _caches([20, 30], 2, 128, torch.bfloat16, 0)
+    assert ops.decode_plan(None, sl, bt, kc) is None
+    assert ops.decode_plan({}, sl.cpu(), bt.cpu(), kc) is None
+    assert ops.decode_plan({}, sl.expand(600, 2).reshape(-1), bt, kc) is None
+
+
+def test_a_recorded_plan_follows_the_lengths():
+    kc, vc, bt, sl = _caches([700, 90, 333], 8, 128, torch.bfloat16, 1)
+    q = torch.randn(3, 32, 128, device=DEV).bfloat16()
+
+    def step():
+        plan = ops.decode_plan({}, sl, bt, kc)
+        return ops.paged_attention_decode(q, kc, vc, bt, sl, 0.1, plan=plan)
+
+    step()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    for lens in ([700, 90, 333], [1, 80, 5], [650, 1, 320], [16, 17, 200]):
+        sl.copy_(torch.tensor(lens, dtype=torch.int32))
+        graph.replay()
+        want = ref.paged_attention_decode(q.float(), kc.float(), vc.float(), bt, sl, 0.1)
+        assert torch.all((out.float() - want).abs() <= 2.0**-8 * want.abs() + 1e-4)
