@@ -77,6 +77,14 @@ struct alignas(8) Splits {
   int first, n;
 };
 
+// Rows that are still sums (common.h: ProductSums, [parts, B, (n_q + 2 n_kv) hd]).
+struct NewRows {
+  ProductSums sums;
+  const int32_t* positions;  // [B]
+  const float* cos_sin;      // [max_pos, hd]
+  const int64_t* slots;      // [B]; < 0: the row's key is in the cache or nowhere
+};
+
 // Cache blocks of a tile.
 constexpr int blocks_per_tile(int hd, int element) { return hd == 128 && element == 1 ? 2 : 1; }
 
@@ -119,18 +127,26 @@ DEV_INLINE float over_groups(float v, F&& f) {
 // CT = cache element type: ushort (bf16) or unsigned char (fp8 e5m2,
 // converted to bf16 on the way in, exactly). CAP: s = cap * tanh(s / cap)
 // after scaling and before masking. ONE: no wave has more than one tile.
-template <int HD, typename CT, bool CAP, bool ONE>
+// NEW: the rows' queries, keys and values are a product's sums still, of up to so many
+// parts. Every workgroup adds and rotates its own query heads and the key, a unit of 8
+// columns a thread, with the first tile's loads on their way behind the sums'; the one
+// that has the row's last tile writes key and value to the cache, and takes them from
+// LDS for that tile. us with the merge, rotation as a
+// launch before / here: 40 rows of 100-700, sums in 4 parts, to fp8 25.0 / 22.2, bf16 23.5 /
+// 21.0; 8 rows, sums in 8 parts 18.2 / 14.8, 14.9 / 11.6.
+template <int HD, typename CT, bool CAP, bool ONE, int NEW>
 __launch_bounds__(kBlockThreads, waves_per_simd(HD)) __global__ void paged_decode_kernel(
     ushort* __restrict__ out,            // [B, n_q, hd] bf16, or null: parts of all rows
     const ushort* __restrict__ q,        // [B, n_q, hd] bf16
-    const CT* k_cache,                   // [nb, n_kv, bs, hd]
-    const CT* v_cache,
+    CT* k_cache,                         // [nb, n_kv, bs, hd]
+    CT* v_cache,
     const int32_t* __restrict__ block_tables,  // [B, max_blocks]
     const int32_t* __restrict__ seq_lens,      // [B]
     const float scale, const float softcap, const int window,
     const int n_kv, const int G, const int max_blocks,
     const int64_t q_stride, const int row_splits,
     const Item* __restrict__ plan,  // or null: row_splits splits of every row
+    const NewRows fresh,
     float* __restrict__ part_o,    // [splits of all rows, n_q, hd]
     float* __restrict__ part_ml) { // [splits of all rows, n_q, 2]
   constexpr int NB = blocks_per_tile(HD, sizeof(CT));
@@ -181,11 +197,15 @@ __launch_bounds__(kBlockThreads, waves_per_simd(HD)) __global__ void paged_decod
   // Head size 256 over a bf16 cache: two tiles of K and V and the sums leave no
   // registers for the query; it lies in LDS, 16-byte units XORed with the head.
   constexpr bool kQLds = HD == 256 && sizeof(CT) == 2;
-  __shared__ __attribute__((aligned(16))) ushort q_lds[kQLds ? kMaxG * HD : 8];
+  __shared__ __attribute__((aligned(16))) ushort q_lds[kQLds || NEW > 0 ? kMaxG * HD : 8];
+  static_assert(NEW == 0 || sizeof(CT) == 2);  // (over an e5m2 cache 116 registers were spilled)
+  __shared__ __attribute__((aligned(16))) CT new_kv[2][NEW > 0 ? HD : 16];
   bf16x8 q_frag[kQLds ? 1 : NC];
   const ushort* qp = q + (int64_t)b * q_stride + (int64_t)kh * G * HD;
   const int q_head = min(col, G - 1);
-  if constexpr (kQLds) {
+  if constexpr (NEW > 0) {
+    // (below, behind the first tile's loads)
+  } else if constexpr (kQLds) {
     for (int i = threadIdx.x; i < G * (HD / 8); i += kBlockThreads) {
       const int g = i / (HD / 8), u = i % (HD / 8);
       *reinterpret_cast<bf16x8*>(&q_lds[g * HD + ((u ^ g) << 3)]) =
@@ -258,9 +278,28 @@ __launch_bounds__(kBlockThreads, waves_per_simd(HD)) __global__ void paged_decod
   const int tr_u = (lane & 3) >> 1;  // unit within the 32 bytes
   const char* tr_base = vt + tr_row * HD * 2 + (lane & 1) * 8;
 
+  int new_tile = -1;  // the tile whose last key is still in LDS
   auto compute = [&](int set, int t) {
     const int tok0 = (blk_base + t * NB) * kBS;
     const bool whole = tok0 >= w0 && tok0 + NB * kBS <= L;
+    if constexpr (NEW > 0) {
+      if (t == new_tile) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          const int row = L - 1 - tok0 - j * kBS;  // (in this block or not)
+#pragma unroll
+          for (int c = 0; c < NC; ++c)
+            if (col == row)
+              kf[set][j][c] = *reinterpret_cast<const Unit*>(&new_kv[0][c * 32 + grp * 8]);
+#pragma unroll
+          for (int i = 0; i < NV; ++i) {
+            const int e = lane + i * WAVE_SIZE;
+            if (e / (HD / 8) == row)
+              vf[set][j][i] = *reinterpret_cast<const Unit*>(&new_kv[1][e % (HD / 8) * 8]);
+          }
+        }
+      }
+    }
     // ---- V to LDS ------------------------------------------------------
 #pragma unroll
     for (int j = 0; j < NB; ++j)
@@ -366,8 +405,82 @@ __launch_bounds__(kBlockThreads, waves_per_simd(HD)) __global__ void paged_decod
   // waits for all of them)
   const int first = split * kWaves + wave;
   const Blocks start = look_up(first);
-  if (first < n_units) {
+  if constexpr (NEW > 0) {
+    constexpr int HALF = HD / 2, UPH = HD / 8;  // units a head
+    // the lanes 2 i and 2 i + 1 have units half a head apart; all threads load (past
+    // the last unit: that again), none in a branch
+    const int at_unit = min((int)threadIdx.x, (G + 2) * UPH - 2 + (int)(threadIdx.x & 1));
+    const int head = at_unit / UPH, half = at_unit & 1;  // G: the key, G + 1: the value
+    const int u = at_unit % UPH / 2 * 8;                 // the pair's column in a half
+    const int col0 = (head < G ? kh * G + head : head == G ? n_q + kh : n_q + n_kv + kh) * HD +
+                     u + half * HALF;
+    const ProductSums& sums = fresh.sums;
+    const int at = max(0, L - 1);  // the new key's place in the row
+    const int64_t slot = fresh.slots[b];
+    const float* cs = fresh.cos_sin + (int64_t)fresh.positions[b] * HD + u;
+    const int last = bt[min(at / kBS, max_blocks - 1)];
+    f32x4 part[NEW][2];
+    const float* row = sums.part + (int64_t)b * sums.N + col0;
+#pragma unroll
+    for (int k = 0; k < NEW; ++k) {
+      const auto* from =
+          reinterpret_cast<const f32x4*>(row + min(k, sums.parts - 1) * sums.stride);
+      part[k][0] = from[0];
+      part[k][1] = from[1];
+    }
+    const int cols[1] = {col0};
+    const SumScales<1> by(sums, b, cols);
+    f32x4 cv[2], sv[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      cv[i] = reinterpret_cast<const f32x4*>(cs)[i];
+      sv[i] = reinterpret_cast<const f32x4*>(cs + HALF)[i];
+    }
+    in_order();
     load_tile(0, first, start);
+    in_order();
+    f32x4 x[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int k = 0; k < NEW; ++k)
+        if (k < sums.parts) x[i] += part[k][i];
+    ushort8 o;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float f = x[j / 4][j % 4];
+      if (sums.sx) f = f * by.sx * by.sw[0][j];
+      o[j] = f32_to_bf16(f);
+      const float own = bf16_to_f32(o[j]), other = __shfl_xor(own, 1);
+      const float c = cv[j / 4][j % 4], s = sv[j / 4][j % 4];
+      if (head <= G) o[j] = f32_to_bf16(half ? own * c + other * s : own * c - other * s);
+    }
+    // the waves' turns go on over the splits
+    const bool owner = (max(n_units, 1) - 1) / kWaves % n_splits == split;
+    if (threadIdx.x < (G + 2) * UPH) {
+      const int unit = u / 8 + half * (UPH / 2);
+      if (head < G) {
+        *reinterpret_cast<ushort8*>(&q_lds[head * HD + ((unit ^ head) << 3)]) = o;
+      } else {
+        *reinterpret_cast<ushort8*>(&new_kv[head - G][unit * 8]) = o;
+        if (owner && slot >= 0) {
+          CT* cache = head == G ? k_cache : v_cache;
+          *reinterpret_cast<ushort8*>(
+              cache + ((slot / kBS * n_kv + kh) * kBS + slot % kBS) * HD + unit * 8) = o;
+        }
+      }
+    }
+    new_tile = slot >= 0 && slot == (int64_t)last * kBS + at % kBS ? n_units - 1 : -1;
+    __syncthreads();
+    if constexpr (!kQLds) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        q_frag[c] = *reinterpret_cast<const bf16x8*>(
+            &q_lds[q_head * HD + (((c * 4 + grp) ^ q_head) << 3)]);
+    }
+  }
+  if (first < n_units) {
+    if constexpr (NEW == 0) load_tile(0, first, start);
     if constexpr (ONE) {
       compute(0, first);
     } else {
@@ -753,21 +866,18 @@ torch::Tensor paged_decode_plan(torch::Tensor seq_lens, int64_t n_kv, int64_t hd
 }
 
 // out [B, n_q, hd] bf16, or with out_scale [B] fp8 rows with a scale each
-void paged_attention_decode(torch::Tensor out, torch::Tensor q,
-                            torch::Tensor k_cache, torch::Tensor v_cache,
-                            torch::Tensor block_tables, torch::Tensor seq_lens,
-                            double scale, int64_t window, double softcap,
-                            c10::optional<torch::Tensor> out_scale,
-                            c10::optional<torch::Tensor> plan) {
-  TORCH_CHECK(q.stride(2) == 1 && q.stride(1) == q.size(2));
-  TORCH_CHECK(out.is_contiguous() && out.numel() >= q.numel());
+static void attend(torch::Tensor out, const ushort* q, int64_t q_stride, const NewRows* fresh,
+                   int B, int n_q, torch::Tensor k_cache, torch::Tensor v_cache,
+                   torch::Tensor block_tables, torch::Tensor seq_lens, double scale,
+                   int64_t window, double softcap, c10::optional<torch::Tensor> out_scale,
+                   c10::optional<torch::Tensor> plan) {
+  const int hd = k_cache.size(3);
+  TORCH_CHECK(out.is_contiguous() && out.numel() >= (int64_t)B * n_q * hd);
   TORCH_CHECK(k_cache.is_contiguous() && v_cache.is_contiguous());
-  TORCH_CHECK(q.scalar_type() == torch::kBFloat16);
   TORCH_CHECK(k_cache.scalar_type() == torch::kBFloat16 ||
               k_cache.scalar_type() == torch::kFloat8_e5m2);
   TORCH_CHECK(block_tables.scalar_type() == torch::kInt32);
   TORCH_CHECK(seq_lens.scalar_type() == torch::kInt32);
-  const int B = q.size(0), n_q = q.size(1), hd = q.size(2);
   const int n_kv = k_cache.size(1);
   const int max_blocks = block_tables.size(1);
   TORCH_CHECK(hd == 128 || hd == 256,
@@ -801,7 +911,7 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
   const bool merged = items || n_splits > 1;
   if (merged) {
     auto opts =
-        torch::TensorOptions().device(q.device()).dtype(torch::kFloat32);
+        torch::TensorOptions().device(k_cache.device()).dtype(torch::kFloat32);
     part_o = torch::empty({parts, n_q, (int64_t)hd}, opts);
     part_ml = torch::empty({parts, n_q, 2}, opts);
     part_o_ptr = part_o.data_ptr<float>();
@@ -810,17 +920,24 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
   TORCH_CHECK(parts * n_kv < (int64_t)1 << 31);
   const dim3 grid((uint32_t)(parts * n_kv)), block(kBlockThreads);
   auto stream = c10::hip::getCurrentHIPStream().stream();
-  auto launch = [&](auto hdv, auto ct, auto cap, auto one) {
+  auto with_new = [&](auto hdv, auto ct, auto cap, auto one, auto fresh_v) {
     using CT = decltype(ct);
     hipLaunchKernelGGL(
         (paged_decode_kernel<decltype(hdv)::value, CT, decltype(cap)::value,
-                             decltype(one)::value>),
-        grid, block, 0, stream, fp8 ? nullptr : (ushort*)out.data_ptr(),
-        (const ushort*)q.data_ptr(), (const CT*)k_cache.data_ptr(),
-        (const CT*)v_cache.data_ptr(), block_tables.data_ptr<int32_t>(),
+                             decltype(one)::value, decltype(fresh_v)::value>),
+        grid, block, 0, stream, fp8 ? nullptr : (ushort*)out.data_ptr(), q,
+        (CT*)k_cache.data_ptr(), (CT*)v_cache.data_ptr(), block_tables.data_ptr<int32_t>(),
         seq_lens.data_ptr<int32_t>(), (float)scale, (float)softcap,
-        (int)window, n_kv, G, max_blocks, q.stride(0), n_splits, items, part_o_ptr,
-        part_ml_ptr);
+        (int)window, n_kv, G, max_blocks, q_stride, n_splits, items,
+        fresh ? *fresh : NewRows{}, part_o_ptr, part_ml_ptr);
+  };
+  auto launch = [&](auto hdv, auto ct, auto cap, auto one) {
+    if constexpr (sizeof(ct) == 2) {
+      if (fresh && fresh->sums.parts <= 4)
+        return with_new(hdv, ct, cap, one, std::integral_constant<int, 4>{});
+      if (fresh) return with_new(hdv, ct, cap, one, std::integral_constant<int, 8>{});
+    }
+    with_new(hdv, ct, cap, one, std::integral_constant<int, 0>{});
   };
   // (12 rows of 500: 14.9 us with the loop's loads of no bytes, 13.9 without)
   const int nb = blocks_per_tile(hd, k_cache.element_size());
@@ -868,4 +985,60 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
                          row_splits, n_splits, n_q, n_bh);
     HIP_CHECK_KERNEL();
   }
+}
+
+void paged_attention_decode(torch::Tensor out, torch::Tensor q,
+                            torch::Tensor k_cache, torch::Tensor v_cache,
+                            torch::Tensor block_tables, torch::Tensor seq_lens,
+                            double scale, int64_t window, double softcap,
+                            c10::optional<torch::Tensor> out_scale,
+                            c10::optional<torch::Tensor> plan) {
+  TORCH_CHECK(q.stride(2) == 1 && q.stride(1) == q.size(2) && k_cache.dim() == 4 &&
+              k_cache.size(3) == q.size(2));
+  TORCH_CHECK(q.scalar_type() == torch::kBFloat16);
+  attend(out, (const ushort*)q.data_ptr(), q.stride(0), nullptr, q.size(0), q.size(1), k_cache,
+         v_cache, block_tables, seq_lens, scale, window, softcap, out_scale, plan);
+}
+
+// The same for rows whose queries, keys and values are a product's sums `part` (with
+// the scales of fp8 operands), [parts, B, (n_q + 2 n_kv) hd]: rotated by positions, keys
+// and values written to slots, which name the places of the rows' last keys (or < 0).
+void paged_attention_decode_sums(torch::Tensor out, torch::Tensor part,
+                                 c10::optional<torch::Tensor> sx,
+                                 c10::optional<torch::Tensor> sw, int64_t n_q,
+                                 torch::Tensor positions, torch::Tensor cos_sin,
+                                 torch::Tensor slots, torch::Tensor k_cache,
+                                 torch::Tensor v_cache, torch::Tensor block_tables,
+                                 torch::Tensor seq_lens, double scale, int64_t window,
+                                 double softcap, c10::optional<torch::Tensor> out_scale,
+                                 c10::optional<torch::Tensor> plan) {
+  TORCH_CHECK(k_cache.dim() == 4 && v_cache.sizes() == k_cache.sizes() &&
+              v_cache.scalar_type() == torch::kBFloat16 &&
+              k_cache.scalar_type() == torch::kBFloat16);
+  const int64_t n_kv = k_cache.size(1), hd = k_cache.size(3), width = (n_q + 2 * n_kv) * hd;
+  TORCH_CHECK(part.scalar_type() == torch::kFloat32 && part.is_contiguous() &&
+              part.is_cuda() && part.dim() == 3 && part.size(0) >= 1 && part.size(0) <= 8 &&
+              part.size(2) == width && ((uintptr_t)part.data_ptr() & 15) == 0);
+  TORCH_CHECK((n_q / n_kv + 2) * hd / 8 <= kBlockThreads, "a thread has 8 columns");
+  const int64_t B = part.size(1);
+  TORCH_CHECK(seq_lens.numel() == B && block_tables.size(0) == B);
+  TORCH_CHECK(positions.scalar_type() == torch::kInt32 && positions.numel() >= B &&
+              positions.is_contiguous() && slots.scalar_type() == torch::kInt64 &&
+              slots.numel() >= B && slots.is_contiguous());
+  TORCH_CHECK(cos_sin.scalar_type() == torch::kFloat32 && cos_sin.is_contiguous() &&
+              cos_sin.size(1) == hd && ((uintptr_t)cos_sin.data_ptr() & 15) == 0);
+  TORCH_CHECK(sx.has_value() == sw.has_value());
+  NewRows fresh{{part.data_ptr<float>(), nullptr, nullptr, (int)part.size(0), B * width,
+                 (int)width},
+                positions.data_ptr<int32_t>(), cos_sin.data_ptr<float>(),
+                slots.data_ptr<int64_t>()};
+  if (sx.has_value()) {
+    TORCH_CHECK(sx->scalar_type() == torch::kFloat32 && sx->is_contiguous() &&
+                sx->numel() == B && sw->scalar_type() == torch::kFloat32 &&
+                sw->is_contiguous() && sw->numel() == width);
+    fresh.sums.sx = sx->data_ptr<float>();
+    fresh.sums.sw = sw->data_ptr<float>();
+  }
+  attend(out, nullptr, 0, &fresh, (int)B, (int)n_q, k_cache, v_cache, block_tables, seq_lens,
+         scale, window, softcap, out_scale, plan);
 }

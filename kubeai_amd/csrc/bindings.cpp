@@ -40,6 +40,15 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
                             double scale, int64_t window, double softcap,
                             c10::optional<torch::Tensor> out_scale,
                             c10::optional<torch::Tensor> plan);
+void paged_attention_decode_sums(torch::Tensor out, torch::Tensor part,
+                                 c10::optional<torch::Tensor> sx,
+                                 c10::optional<torch::Tensor> sw, int64_t n_q,
+                                 torch::Tensor positions, torch::Tensor cos_sin,
+                                 torch::Tensor slots, torch::Tensor k_cache,
+                                 torch::Tensor v_cache, torch::Tensor block_tables,
+                                 torch::Tensor seq_lens, double scale, int64_t window,
+                                 double softcap, c10::optional<torch::Tensor> out_scale,
+                                 c10::optional<torch::Tensor> plan);
 torch::Tensor paged_decode_plan(torch::Tensor seq_lens, int64_t n_kv, int64_t hd,
                                 int64_t element_size, int64_t window);
 int paged_decode_splits(int rows, int n_kv, int hd, int max_blocks);
@@ -147,6 +156,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),
         py::arg("seq_lens"), py::arg("scale"), py::arg("window"), py::arg("softcap"),
         py::arg("out_scale") = py::none(), py::arg("plan") = py::none());
+  m.def("paged_attention_decode_sums", &paged_attention_decode_sums,
+        "paged decode attention of rows that are a product's sums");
   m.def("paged_decode_plan", &paged_decode_plan,
         "splits of all rows of a decode step (lengths, kv heads, head size, bytes of an "
         "element, window)");

@@ -177,6 +177,25 @@ class Attention(nn.Module):
         if isinstance(cos_sin, tuple):
             # (global, local) caches — gemma3 dual rope bases
             cos_sin = cos_sin[0] if self.is_global else cos_sin[1]
+        nd = fb.n_decode
+        plan = ops.decode_plan(
+            fb.decode_plans, fb.decode_seq_lens, fb.decode_block_tables, k_cache, self.window
+        ) if nd > 0 else None
+        if nd == T and fb.n_prefill == 0 and ops.decode_takes_sums(
+            qkv, self.n_q, cos_sin, k_cache, v_cache
+        ):
+            out = ops.paged_attention_decode_sums(
+                qkv, self.n_q, fb.positions, cos_sin, fb.slot_mapping, k_cache, v_cache,
+                fb.decode_block_tables, fb.decode_seq_lens, self.scale,
+                window=self.window, softcap=self.softcap, plan=plan, fp8=fp8_in,
+            )
+            if not fp8_in:
+                out = out.view(T, -1)
+            if lora_live:
+                return _project_adapted(
+                    self.o_proj, out, as_sums, fb, lm, self.layer_idx, "o"
+                )
+            return _project(self.o_proj, out, as_sums, fb)
         if self.qk_norm:
             # gemma3: per-head RMSNorm ((1+w) stored as w) before rope;
             # fp32 math, contiguous bf16 out. v follows to contiguous —
@@ -200,10 +219,6 @@ class Attention(nn.Module):
                 fb.slot_mapping,
             )
 
-        nd = fb.n_decode
-        plan = ops.decode_plan(
-            fb.decode_plans, fb.decode_seq_lens, fb.decode_block_tables, k_cache, self.window
-        ) if nd > 0 else None
         if fp8_in and nd == T and fb.n_prefill == 0:
             return _project(
                 self.o_proj,

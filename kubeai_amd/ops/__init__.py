@@ -203,6 +203,50 @@ def paged_attention_decode_fp8(
     return out, out_scale
 
 
+def decode_takes_sums(qkv, n_q: int, cos_sin, k_cache, v_cache) -> bool:
+    """Whether paged_attention_decode_sums takes these."""
+    return (
+        isinstance(qkv, ProductSums)
+        and k_cache.dtype == v_cache.dtype == torch.bfloat16
+        and k_cache.shape == v_cache.shape
+        and k_cache.shape[2] == 16
+        and k_cache.shape[3] in (128, 256)
+        and n_q % k_cache.shape[1] == 0
+        and n_q // k_cache.shape[1] in (1, 2, 4, 5, 6, 8)
+        and (n_q // k_cache.shape[1] + 2) * k_cache.shape[3] <= 2048
+        and qkv.part.shape[0] <= 8
+        and cos_sin.dtype == torch.float32
+        and cos_sin.is_contiguous()
+        and aligned(cos_sin)
+    )
+
+
+def paged_attention_decode_sums(
+    qkv, n_q: int, positions, cos_sin, slot_mapping, k_cache, v_cache, block_tables, seq_lens,
+    scale: float, window: int = 0, softcap: float = 0.0, plan=None, fp8: bool = False,
+):
+    """rope_and_cache and paged_attention_decode in one launch (GPU only), for rows whose
+    q | k | v is a product's sums: [B, n_q, hd] bf16, or (fp8) quant_fp8 of its rows. Every
+    row's slot is the place of its last key (negative: nothing is written, and the cache
+    has the key), and no other row reads that place."""
+    B, (n_kv, _, hd) = qkv.shape[0], k_cache.shape[1:]
+    merges = fp8 and (
+        n_q <= 32 if plan is not None
+        else decode_fp8_merges(n_q, _C.paged_decode_splits(B, n_kv, hd, block_tables.shape[1]))
+    )
+    dev = k_cache.device
+    out = torch.empty((B, n_q, hd), device=dev,
+                      dtype=torch.float8_e4m3fn if merges else torch.bfloat16)
+    out_scale = torch.empty(B, dtype=torch.float32, device=dev) if merges else None
+    _C.paged_attention_decode_sums(
+        out, *qkv.args(), n_q, positions, cos_sin, slot_mapping, k_cache, v_cache,
+        block_tables, seq_lens, scale, window, softcap, out_scale, plan)
+    if not fp8:
+        return out
+    flat = out.view(B, n_q * hd)
+    return (flat, out_scale) if merges else quant_fp8(flat)
+
+
 def paged_attention_prefill(
     q, k_cache, v_cache, block_tables, query_start_loc, seq_lens, scale: float,
     out=None, window: int = 0, softcap: float = 0.0,

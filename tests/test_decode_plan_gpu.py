@@ -103,3 +103,55 @@ def test_a_recorded_plan_follows_the_lengths():
         graph.replay()
         want = ref.paged_attention_decode(q.float(), kc.float(), vc.float(), bt, sl, 0.1)
         assert torch.all((out.float() - want).abs() <= 2.0**-8 * want.abs() + 1e-4)
+
+
+@pytest.mark.parametrize("planned", [True, False])
+@pytest.mark.parametrize("lens", [LENGTHS[k] for k in ("one", "one long", "edges", "even")],
+                         ids=["one", "one long", "edges", "even"])
+@pytest.mark.parametrize("n_q,n_kv,hd,window,cap,parts,scaled", [
+    (32, 8, 128, 0, 0.0, 4, True),
+    (8, 1, 128, 0, 0.0, 7, False),
+    (8, 4, 256, 100, 30.0, 1, True),
+    (12, 2, 256, 0, 0.0, 8, False),
+    (2, 2, 128, 33, 20.0, 3, True),
+])
+def test_from_sums(lens, n_q, n_kv, hd, window, cap, parts, scaled, planned):
+    """One launch against rotation, cache write and attention after one another: the
+    same bits in the caches (angles are powers of 2: a product is exact, so it does not
+    matter which of two the compiler fuses with the sum), and results that differ by a
+    rounding here and there (sums in fp32 may be fused differently, 2^-24 of them, which is
+    the other side of a rounding to 2^-9 once in some ten thousand). A row without a slot
+    keeps its key from the cache."""
+    B, width = len(lens), (n_q + 2 * n_kv) * hd
+    kc, vc, bt, sl = _caches(lens, n_kv, hd, torch.bfloat16, parts)
+    g = torch.Generator(device=DEV).manual_seed(7)
+    part = torch.randn(parts, B, width, device=DEV, generator=g) * parts**-0.5
+    scales = (torch.rand(B, device=DEV) + 0.5, torch.rand(width, device=DEV) + 0.5)
+    qkv = ops.ProductSums(part, *(scales if scaled else (None, None)))
+    pos = sl - 1
+    angle = pos.max().item() + 1
+    cos_sin = 2.0 ** -torch.randint(0, 4, (angle, hd), device=DEV, generator=g).float()
+    cos_sin[:, ::3] *= -1.0
+    at = (sl - 1).long()
+    slots = bt.gather(1, (at // BS)[:, None]).long()[:, 0] * BS + at % BS
+    if B > 2:
+        slots[1] = -1
+    plan = ops.decode_plan({}, sl, bt, kc, window) if planned else None
+    one, two = (kc.clone(), vc.clone()), (kc.clone(), vc.clone())
+    q = ops.rope_and_cache(qkv, n_q, pos, cos_sin, *one, slots)
+    kw = dict(window=window, softcap=cap, plan=plan)
+    want = ops.paged_attention_decode(q, *one, bt, sl, hd**-0.5, **kw)
+    assert ops.decode_takes_sums(qkv, n_q, cos_sin, *two)
+    got = ops.paged_attention_decode_sums(qkv, n_q, pos, cos_sin, slots, *two, bt, sl,
+                                          hd**-0.5, **kw)
+    assert torch.equal(one[0], two[0]) and torch.equal(one[1], two[1])
+    diff = (got.float() - want.float()).abs()
+    assert torch.all(diff <= 2.0**-7 * want.float().abs() + 2.0**-21)
+    assert (diff > 0).float().mean() < 2e-3
+    two = (kc.clone(), vc.clone())
+    f8, scale = ops.paged_attention_decode_sums(qkv, n_q, pos, cos_sin, slots, *two, bt, sl,
+                                                hd**-0.5, fp8=True, **kw)
+    w8, wscale = ops.quant_fp8(got.view(B, -1))
+    assert torch.equal(f8.view(torch.uint8), w8.view(torch.uint8))
+    assert torch.equal(scale.view(-1), wscale.view(-1))
+    assert torch.equal(one[0], two[0]) and torch.equal(one[1], two[1])
