@@ -141,12 +141,22 @@ constexpr int kSB = 1024;  // threads of a sorting block
 // grid (E): block e places the pairs of expert e. Its first place is the
 // number of pairs of lower experts; a pair's rank is the number of earlier
 // pairs of the same expert (block-wide prefix sums over slices of the list).
+// every: one more block and expert E, which all tokens use with weight 1, in order.
 __global__ __launch_bounds__(kSB) void expert_order_kernel(
     const int* __restrict__ index, const float* __restrict__ weights,
     int* __restrict__ tok, float* __restrict__ wrow, int* __restrict__ place,
-    int* __restrict__ counts, int N, int top) {
+    int* __restrict__ counts, int N, int top, int every) {
   __shared__ int part[kSB / WAVE + 1], total_s;
-  const int e = blockIdx.x;
+  const int e = blockIdx.x, places = top + every;  // of a token
+  if (every && e == (int)gridDim.x - 1) {
+    for (int t = threadIdx.x; t < N / top; t += kSB) {
+      tok[N + t] = t;
+      wrow[N + t] = 1.f;
+      place[t * places + top] = N + t;
+    }
+    if (threadIdx.x == 0) counts[e] = N / top;
+    return;  // the whole block
+  }
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
   int below = 0;
   for (int i = threadIdx.x; i < N; i += kSB) below += index[i] < e ? 1 : 0;
@@ -178,7 +188,7 @@ __global__ __launch_bounds__(kSB) void expert_order_kernel(
       const int p = at + before + __popcll(b & ((1ull << lane) - 1));
       tok[p] = i / top;
       wrow[p] = weights[i];
-      place[i] = p;
+      place[i / top * places + i % top] = p;
     }
     at += all;
   }
@@ -279,14 +289,16 @@ void expert_order(torch::Tensor index, torch::Tensor weights, torch::Tensor tok,
   check_i32(place, "place");
   check_i32(counts, "counts");
   TORCH_CHECK(index.dim() == 2);
-  const int64_t N = index.numel();
-  TORCH_CHECK(weights.numel() == N && tok.numel() == N && wrow.numel() == N &&
-              place.numel() == N && N < (int64_t)1 << 30 && counts.numel() >= 1);
+  const int64_t N = index.numel(), T = index.size(0);
+  const int64_t rows = place.numel();  // T more than N: one expert has every token
+  TORCH_CHECK(weights.numel() == N && tok.numel() == rows && wrow.numel() == rows &&
+              (rows == N || rows == N + T) && rows < (int64_t)1 << 30 &&
+              counts.numel() >= (rows == N ? 1 : 2));
   if (N == 0) return;
   hipLaunchKernelGGL(expert_order_kernel, dim3(counts.numel()), dim3(kSB), 0, SEQ_STREAM(),
                      (const int*)index.data_ptr(), (const float*)weights.data_ptr(),
                      (int*)tok.data_ptr(), (float*)wrow.data_ptr(), (int*)place.data_ptr(),
-                     (int*)counts.data_ptr(), (int)N, (int)index.size(1));
+                     (int*)counts.data_ptr(), (int)N, (int)index.size(1), rows != N);
   SEQ_CHECK_LAUNCH();
 }
 

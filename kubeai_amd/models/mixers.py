@@ -655,12 +655,13 @@ class ExpertRows:
     each product and each pass between them is one launch for all experts, and
     the row counts stay on the device. Where the products are the library's
     (types and sizes that csrc/tiled_gemm.h does not take or is slower for)
-    there is one per expert, and the counts come to the host: they need shapes."""
+    there is one per expert, and the counts come to the host: they need shapes.
+    every: one more expert has the rows of all tokens."""
 
-    def __init__(self, h, index, weights, experts: int):
+    def __init__(self, h, index, weights, experts: int, every: bool = False):
         self.h = h
         self.token, self.weight, self.place, self.counts = sops.expert_order(
-            index, weights, experts)
+            index, weights, experts, every)
 
     def products(self, x, w, square: bool = False):
         """Every expert's rows (of the tokens if x is None, else of x) times its
@@ -696,6 +697,7 @@ class RoutedSquaredReluMoE(nn.Module):
     order and multiply each expert's by its slice of the stacked matrices."""
 
     DENSE_MAX_TOKENS = 256
+    TOGETHER_MAX = 3072 * 7168  # tokens x columns (see forward)
 
     def __init__(self, width, experts, top, ff, shared_ff=0):
         super().__init__()
@@ -715,11 +717,27 @@ class RoutedSquaredReluMoE(nn.Module):
         if T <= self.DENSE_MAX_TOKENS:
             a = sops.relu_squared_weighted(self.up(h), dense, ff)
             return self.down(a)
-        rows = ExpertRows(h, idx, w, E)
-        a = rows.products(None, self.up.weight[: E * ff].unflatten(0, (E, ff)), square=True)
-        y = rows.products(a, self.down.weight[:, : E * ff].unflatten(1, (E, ff)).transpose(0, 1))
+        # A shared expert of the others' size lies behind them as one of them: its tiles
+        # fill the launches' last passes over the CUs, and two library products and the
+        # squared ReLU between them are gone. The layer, us, apart / together: 8 experts of
+        # 3584 x 2048, 260 tokens 132 / 112, 700 156 / 130, 2048 261 / 219, 4400 456 / 448;
+        # of 1792 x 1024, 260 71 / 51, 3072 154 / 125; 16 of 1408 x 2048, 4 a token, 1000
+        # 152 / 129. Not where each of the two fills the chip several times by itself:
+        # of 7168 x 4096, 260 302 / 279, 1500 638 / 566, but 3072 1077 / 1076, 4400 1415 / 1462
+        every = self.shared_ff == ff and T * ff <= self.TOGETHER_MAX
+        n = E + every
+        up = self.up.weight[: n * ff].unflatten(0, (n, ff))
+        down = self.down.weight[:, : n * ff].unflatten(1, (n, ff)).transpose(0, 1)
+        if every and not all(
+            ops.grouped_linear_takes(x, m) and ops.grouped_linear_better(T * (self.top + 1), m)
+            for x, m in ((h, up), (up.new_empty((0, ff)), down))
+        ):
+            every, up, down = False, up[:E], down[:E]
+        rows = ExpertRows(h, idx, w, E, every)
+        a = rows.products(None, up, square=True)
+        y = rows.products(a, down)
         shared = None
-        if self.shared_ff:
+        if self.shared_ff and not every:
             u = F.linear(h, self.up.weight[E * ff :])
             shared = F.linear(sops.relu_squared(u), self.down.weight[:, E * ff :])
         return sops.combine_expert_rows(y, rows.place, shared)

@@ -794,21 +794,26 @@ def route_tokens(h, router, experts: int, top: int, bias=None, scale: float = 1.
     return dense, w, idx, logits[:, experts:] if n else None
 
 
-def expert_order(index, weights, experts: int):
+def expert_order(index, weights, experts: int, every: bool = False):
     """(token, choice) pairs sorted by expert, stably. index int32 and weights
     fp32 [T, top] -> (token int32 [N] of every sorted row, its weight fp32
     [N, 1], place int32 [T, top] of every pair among the sorted rows, counts
-    int32 [experts]), N = T * top."""
+    int32 [experts]), N = T * top. every: as if all tokens had chosen one more
+    expert, the last one, with weight 1 (top and experts are one more in the results)."""
     T, top = index.shape
-    N = T * top
+    N = T * (top + every)
     if index.is_cuda:
         _require_ext()
         i32 = dict(dtype=torch.int32, device=index.device)
-        tok, place = torch.empty(N, **i32), torch.empty((T, top), **i32)
-        counts = torch.empty(experts, **i32)
+        tok, place = torch.empty(N, **i32), torch.empty((T, top + every), **i32)
+        counts = torch.empty(experts + every, **i32)
         wrow = torch.empty((N, 1), dtype=torch.float32, device=index.device)
         _C.expert_order(index, weights, tok, wrow, place, counts)
         return tok, wrow, place, counts
+    if every:
+        index = torch.cat([index, torch.full_like(index[:, :1], experts)], 1)
+        weights = torch.cat([weights, torch.ones_like(weights[:, :1])], 1)
+        top, experts = top + 1, experts + 1
     flat = index.flatten().long()
     order = torch.argsort(flat, stable=True)
     place = torch.empty(N, dtype=torch.int32)
