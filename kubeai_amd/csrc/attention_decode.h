@@ -1,0 +1,737 @@
+// Paged-attention decode (one new token per sequence) for gfx950: the kernels.
+//
+// Semantics: kubeai_amd/ops/ref.py::paged_attention_decode.
+//
+// Structure:
+//  - workgroup = (sequence, kv head, split of the keys); the waves of a row's splits
+//    take tiles in turn, each with its own softmax state; the G query heads of the
+//    group share every key. A tile is one cache block (32 keys over an e5m2 cache at
+//    head size 128): 145 registers and three waves a SIMD, where tiles of 32 keys take
+//    209 and leave room for two (28 rows of 100-700 in 3 splits 17.9 us, 15.9). The first
+//    look-up in the block table does not wait for the row's length.
+//  - which splits there are, and in which order, is worked out on the device once a
+//    step (attention_decode.hip), by the rows' lengths.
+//  - S^T = K.Q^T on v_mfma_f32_16x16x32_bf16: a lane reads 16 bytes of one
+//    key straight into the operand (16 keys x 64 contiguous bytes per load,
+//    no LDS), the query heads are columns (lane & 15; those past G repeat the
+//    last head). Scores of 4 keys per block lie in the lane, a maximum is two
+//    lane swaps, the sum stays per lane until the end.
+//  - O^T += V^T.P^T: the score registers are the second product's operand as
+//    they stand. V needs its keys along a lane: it goes through a
+//    wave-private LDS tile (row-major, 16-byte units XOR-swizzled, no
+//    barriers) and comes back through ds_read_b64_tr_b16.
+//  - the weights keep their 24 bits: they are cut into three bf16 parts of 8
+//    bits that are multiplied one after the other into the same fp32 sum. A
+//    part that would be 0 is 2^-100 (or the weight, if that is less): times an
+//    infinite value 0 would be NaN.
+//  - the next tile's K and V are in flight while this one is computed (two
+//    register sets), and the blocks of the one after it are being looked up. Past the
+//    last tile the loads are of no bytes: in a branch they had the compiler wait, in
+//    front of each tile, for the next one's loads as well (96 rows of 1500-4000 228 us).
+// Bound by reading the cache. The form before this (scores and weighted sum
+// on the vector ALUs) issued about 150 LDS operations per 16 keys, most of
+// them the lane permutes that passed a weight to every lane; here it is 12.
+// Measured, kernel + merge of the splits, us (the same number of splits for every row
+// and tiles of 32 keys -> planned):
+//   heads 32/8 x 128, 40 rows of 100-700 keys         23.2 -> 18.8, to fp8 25.3 -> 20.1
+//   96 rows of 1500-4000                             209 -> 195 (5.8 TB/s)
+//   64 rows of 100-2000                              60.9 -> 53.4
+//   40 rows of 200, one of 4000                      34.9 -> 15.8, to fp8 37.1 -> 19.6
+//   8 rows of 3584                                    28.8 -> 25.6
+//   1 row of 3000 and 7 idle ones                     12.6 -> 8.7
+//   12 rows of 500                                    13.2 -> 10.5
+//   96 rows of 100-300, one split each                20.5 -> 19.8 (unplanned 18.8)
+//   heads 8/4 x 256, 40 rows of 100-700               21.9 -> 18.4
+//     64 rows of 100-2000                             65.1 -> 60.3
+//     96 rows of 2000                                 139 -> 139.5
+// At head size 256, over
+// a bf16 cache the query lies in LDS: with it in registers 25 were spilled, and
+// the reloads waited for the loads in flight (the last two 236 us).
+#pragma once
+
+#include <type_traits>
+
+#include "common.h"
+
+namespace decode {
+namespace {
+
+constexpr int kWaves = 4;
+constexpr int kBlockThreads = kWaves * WAVE_SIZE;
+constexpr int kBS = 16;      // cache block size (tokens)
+constexpr int kMaxSplits = 16;
+constexpr int kMaxG = 8;
+constexpr int kCUs = 256;
+
+typedef __attribute__((ext_vector_type(8))) short bf16x8;
+typedef __attribute__((ext_vector_type(4))) short bf16x4;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+
+// One split of a row; a row's splits, which lie behind one another.
+struct alignas(16) Item {
+  int row, len;  // row < 0: none
+  uint16_t split, splits;
+  int part;      // where its results go
+};
+struct alignas(8) Splits {
+  int first, n;
+};
+
+// Rows that are still sums (common.h: ProductSums, [parts, B, (n_q + 2 n_kv) hd]).
+struct NewRows {
+  ProductSums sums;
+  const int32_t* positions;  // [B]
+  const float* cos_sin;      // [max_pos, hd]
+  const int64_t* slots;      // [B]; < 0: the row's key is in the cache or nowhere
+};
+
+// Cache blocks of a tile.
+constexpr int blocks_per_tile(int hd, int element) { return hd == 128 && element == 1 ? 2 : 1; }
+
+// Waves a SIMD holds: 145 registers at head size 128, 256 at 256.
+constexpr int waves_per_simd(int hd) { return hd == 128 ? 3 : 2; }
+
+// 16 (or 8) bytes a lane from base + at, zeros if size is 0
+template <typename T>
+DEV_INLINE T buffer_load(const void* base, int size, int at) {
+  T v{};
+#ifdef __HIP_DEVICE_COMPILE__
+  const auto r = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, size, 0x00020000);
+  if constexpr (sizeof(T) == 16)
+    v = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0));
+  else
+    v = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, at, 0, 0));
+#endif
+  return v;
+}
+
+// no load moves over it: the caches are not __restrict__, so the compiler takes the
+// asm to write them
+DEV_INLINE void in_order() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// combine a value over the four 16-lane groups that hold the same column
+template <typename F>
+DEV_INLINE float over_groups(float v, F&& f) {
+  const auto a = __builtin_amdgcn_permlane32_swap(
+      __float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane16_swap(
+      __float_as_uint(v), __float_as_uint(v), false, false);
+  return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+// CT = cache element type: ushort (bf16) or unsigned char (fp8 e5m2,
+// converted to bf16 on the way in, exactly). CAP: s = cap * tanh(s / cap)
+// after scaling and before masking. ONE: no wave has more than one tile.
+// NEW: the rows' queries, keys and values are a product's sums still, of up to so many
+// parts. Every workgroup adds and rotates its own query heads and the key, a unit of 8
+// columns a thread, with the first tile's loads on their way behind the sums'; the one
+// that has the row's last tile writes key and value to the cache, and takes them from
+// LDS for that tile. us with the merge, rotation as a
+// launch before / here: 40 rows of 100-700, sums in 4 parts, to fp8 25.0 / 22.2, bf16 23.5 /
+// 21.0; 8 rows, sums in 8 parts 18.2 / 14.8, 14.9 / 11.6.
+template <int HD, typename CT, int NEW>
+struct alignas(16) Lds {
+  // Head size 256 over a bf16 cache: two tiles of K and V and the sums leave no
+  // registers for the query; it lies in LDS, 16-byte units XORed with the head.
+  static constexpr bool kQuery = HD == 256 && sizeof(CT) == 2;
+  static constexpr int kVTile = blocks_per_tile(HD, sizeof(CT)) * kBS * HD;  // elements a wave
+  static constexpr size_t kTiles = sizeof(ushort) * kWaves * kVTile >
+                                           sizeof(float) * kWaves * kMaxG * HD
+                                       ? sizeof(ushort) * kWaves * kVTile
+                                       : sizeof(float) * kWaves * kMaxG * HD;
+  alignas(16) char tiles[kTiles];  // of V, then the waves' results
+  alignas(16) ushort query[kQuery || NEW > 0 ? kMaxG * HD : 8];
+  alignas(16) CT new_kv[2][NEW > 0 ? HD : 16];
+  float merge_ml[kWaves][kMaxG][2];
+};
+
+template <int HD, typename CT, bool CAP, bool ONE, int NEW>
+DEV_INLINE void attend_split(
+    Lds<HD, CT, NEW>& mem, const int block,
+    ushort* __restrict__ out,            // [B, n_q, hd] bf16, or null: parts of all rows
+    const ushort* __restrict__ q,        // [B, n_q, hd] bf16
+    CT* k_cache,                         // [nb, n_kv, bs, hd]
+    CT* v_cache,
+    const int32_t* __restrict__ block_tables,  // [B, max_blocks]
+    const int32_t* __restrict__ seq_lens,      // [B]
+    const float scale, const float softcap, const int window,
+    const int n_kv, const int G, const int max_blocks,
+    const int64_t q_stride, const int row_splits,
+    const Item* __restrict__ plan,  // or null: row_splits splits of every row
+    const NewRows fresh,
+    float* __restrict__ part_o,    // [splits of all rows, n_q, hd]
+    float* __restrict__ part_ml) { // [splits of all rows, n_q, 2]
+  constexpr int NB = blocks_per_tile(HD, sizeof(CT));
+  constexpr int NC = HD / 32;            // contraction steps of S
+  constexpr int ND = HD / 16;            // row blocks of O^T
+  constexpr int NV = HD / 32;            // 16-byte V units per lane and block
+  const int item = block / n_kv, kh = block % n_kv;
+  int b, split, n_splits, L, part_row = item;
+  if (plan) {
+    const Item it = plan[item];
+    if (it.row < 0) return;
+    b = it.row;
+    split = it.split;
+    n_splits = it.splits;
+    L = it.len;
+    part_row = it.part;
+  } else {
+    b = item / row_splits;
+    split = item % row_splits;
+    n_splits = row_splits;
+    L = seq_lens[b];
+  }
+  const int n_q = n_kv * G;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
+  const int lane = threadIdx.x % WAVE_SIZE;
+  const int col = lane & 15, grp = lane >> 4;
+  const int n_blocks = (L + kBS - 1) / kBS;
+  // sliding window: the query (position L-1) attends keys in
+  // (L-1-window, L-1]; splits divide the visible blocks only
+  int w0 = 0, blk_base = 0;
+  if (window > 0) {
+    w0 = max(0, L - window);
+    blk_base = w0 / kBS;
+  }
+  const int n_units = (n_blocks - blk_base + NB - 1) / NB;  // tiles
+  // the waves of all splits take tiles in turn
+  const int turn = kWaves * n_splits;
+
+  constexpr int kVTile = Lds<HD, CT, NEW>::kVTile;
+  constexpr bool kQLds = Lds<HD, CT, NEW>::kQuery;
+  auto& smem = mem.tiles;
+  auto& q_lds = mem.query;
+  auto& new_kv = mem.new_kv;
+  auto& merge_ml = mem.merge_ml;
+  char* vt = smem + wave * kVTile * 2;
+  static_assert(NEW == 0 || sizeof(CT) == 2);  // (over an e5m2 cache 116 registers were spilled)
+  bf16x8 q_frag[kQLds ? 1 : NC];
+  const ushort* qp = q + (int64_t)b * q_stride + (int64_t)kh * G * HD;
+  const int q_head = min(col, G - 1);
+  if constexpr (NEW > 0) {
+    // (below, behind the first tile's loads)
+  } else if constexpr (kQLds) {
+    for (int i = threadIdx.x; i < G * (HD / 8); i += kBlockThreads) {
+      const int g = i / (HD / 8), u = i % (HD / 8);
+      *reinterpret_cast<bf16x8*>(&q_lds[g * HD + ((u ^ g) << 3)]) =
+          *reinterpret_cast<const bf16x8*>(qp + i * 8);
+    }
+    __syncthreads();
+  } else {
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      q_frag[c] = *reinterpret_cast<const bf16x8*>(qp + q_head * HD + grp * 8 + c * 32);
+  }
+  auto query = [&](int c) -> bf16x8 {
+    if constexpr (kQLds)
+      return *reinterpret_cast<const bf16x8*>(
+          &q_lds[q_head * HD + (((c * 4 + grp) ^ q_head) << 3)]);
+    else
+      return q_frag[c];
+  };
+  const float c2 = CAP ? scale : scale * kLog2e;
+  const SoftCap cap(CAP ? softcap : 1.0f);
+
+  f32x4 o_acc[ND];
+#pragma unroll
+  for (int d = 0; d < ND; ++d) o_acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;  // l_run: this lane's keys
+
+  const int32_t* bt = block_tables + (int64_t)b * max_blocks;
+  using Unit = std::conditional_t<sizeof(CT) == 2, bf16x8, uint64_t>;
+  Unit kf[2][NB][NC], vf[2][NB][NV];
+  auto to_bf16 = [](const Unit& u) -> bf16x8 {
+    if constexpr (sizeof(CT) == 2) return u;
+    else return __builtin_bit_cast(bf16x8, e5m2x8_to_bf16x8(u));
+  };
+  // the cache blocks of tile t (past the last one: any entry of the table, not used).
+  // Without a window the first look-up does not wait for the row's length.
+  struct Blocks {
+    int at[NB];
+  };
+  auto look_up = [&](int t) {
+    Blocks o;
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+      o.at[j] = bt[min(blk_base + t * NB + j, max_blocks - 1)];
+    return o;
+  };
+  constexpr int kBlockBytes = kBS * HD * sizeof(CT);
+  const int k_at = (col * HD + grp * 8) * sizeof(CT), v_at = lane * 8 * sizeof(CT);
+  // blocks behind the last one: loads of no bytes
+  auto load_tile = [&](int set, int t, const Blocks& blocks) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int size = blk_base + t * NB + j < n_blocks ? kBlockBytes : 0;
+      const int64_t base = ((int64_t)blocks.at[j] * n_kv + kh) * (kBS * HD);
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        kf[set][j][c] =
+            buffer_load<Unit>(k_cache + base, size, k_at + c * 32 * (int)sizeof(CT));
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        vf[set][j][i] = buffer_load<Unit>(v_cache + base, size,
+                                          v_at + i * WAVE_SIZE * 8 * (int)sizeof(CT));
+    }
+  };
+
+  // LDS offsets of the transposing reads: keys 4 grp + (lane >> 2 & 3) of a
+  // block, columns 16 d + 4 (lane & 3); units of rows r are XORed with
+  // 2 (r & 3), which spreads the four rows of a 16-lane read over the banks
+  const int tr_row = 4 * grp + ((lane >> 2) & 3);
+  const int tr_x = ((lane >> 2) & 3) << 1;
+  const int tr_u = (lane & 3) >> 1;  // unit within the 32 bytes
+  const char* tr_base = vt + tr_row * HD * 2 + (lane & 1) * 8;
+
+  int new_tile = -1;  // the tile whose last key is still in LDS
+  auto compute = [&](int set, int t) {
+    const int tok0 = (blk_base + t * NB) * kBS;
+    const bool whole = tok0 >= w0 && tok0 + NB * kBS <= L;
+    if constexpr (NEW > 0) {
+      if (t == new_tile) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          const int row = L - 1 - tok0 - j * kBS;  // (in this block or not)
+#pragma unroll
+          for (int c = 0; c < NC; ++c)
+            if (col == row)
+              kf[set][j][c] = *reinterpret_cast<const Unit*>(&new_kv[0][c * 32 + grp * 8]);
+#pragma unroll
+          for (int i = 0; i < NV; ++i) {
+            const int e = lane + i * WAVE_SIZE;
+            if (e / (HD / 8) == row)
+              vf[set][j][i] = *reinterpret_cast<const Unit*>(&new_kv[1][e % (HD / 8) * 8]);
+          }
+        }
+      }
+    }
+    // ---- V to LDS ------------------------------------------------------
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const int e = lane + i * WAVE_SIZE;  // 16-byte unit of the block
+        const int row = e / (HD / 8), un = e % (HD / 8);
+        bf16x8 v = to_bf16(vf[set][j][i]);
+        // rows past the end: their weight is 0, but 0 * stale NaN is not
+        if (!whole && tok0 + j * kBS + row >= L) v = bf16x8{};
+        *reinterpret_cast<bf16x8*>(
+            vt + (j * kBS + row) * HD * 2 + ((un ^ ((row & 3) << 1)) << 4)) = v;
+      }
+    // ---- scores ----------------------------------------------------------
+    f32x4 s[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      s[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        s[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            to_bf16(kf[set][j][c]), query(c), s[j], 0, 0, 0);
+    }
+    if constexpr (CAP) cap.apply(s, c2);
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float x = s[j][i] * (CAP ? kLog2e : c2);
+        const int tok = tok0 + j * kBS + grp * 4 + i;
+        if (!whole && (tok >= L || tok < w0)) x = -INFINITY;
+        s[j][i] = x;
+        tmax = fmaxf(tmax, x);
+      }
+    tmax = over_groups(tmax, [](float a, float c) { return fmaxf(a, c); });
+    // the maximum may lag by 2^11 before everything is rescaled
+    if (!__all(tmax <= m_run + 11.0f)) {
+      const float m_new = fmaxf(m_run, tmax);
+      const float corr =
+          __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.f : m_new));
+      l_run *= corr;
+#pragma unroll
+      for (int d = 0; d < ND; ++d) o_acc[d] *= corr;
+      m_run = m_new;
+    }
+    const float m_use = (m_run == -INFINITY) ? 0.f : m_run;
+    // ---- weights, in three bf16 parts --------------------------------------
+    short p_part[3][NB * 4];
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float p = __builtin_amdgcn_exp2f(s[j][i] - m_use);
+        l_run += p;
+        const float least = fminf(p, 0x1p-100f);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const uint32_t top = __float_as_uint(p) & 0xffff0000u;
+          p_part[k][j * 4 + i] = (short)(top >> 16);
+          p = fmaxf(p - __uint_as_float(top), least);
+        }
+      }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // ---- O^T += V^T . P^T ------------------------------------------------
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+      const char* a = tr_base + (((2 * d + tr_u) ^ tr_x) << 4);
+      const bf16x4 v0 =
+          __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4*)(a));
+      if constexpr (NB == 2) {
+        const bf16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_bf16x4*)(a + kBS * HD * 2));
+        const bf16x8 v =
+            __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          bf16x8 p;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) p[i] = p_part[k][i];
+          o_acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, p, o_acc[d],
+                                                             0, 0, 0);
+        }
+      } else {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          bf16x4 p;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) p[i] = p_part[k][i];
+          o_acc[d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v0, p, o_acc[d],
+                                                               0, 0, 0);
+        }
+      }
+    }
+    // the next tile's V is stored after these reads (LDS operations of a
+    // wave run in order)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+
+  // (no load in a branch: where paths of more and of fewer loads meet, the compiler
+  // waits for all of them)
+  const int first = split * kWaves + wave;
+  const Blocks start = look_up(first);
+  if constexpr (NEW > 0) {
+    constexpr int HALF = HD / 2, UPH = HD / 8;  // units a head
+    // the lanes 2 i and 2 i + 1 have units half a head apart; all threads load (past
+    // the last unit: that again), none in a branch
+    const int at_unit = min((int)threadIdx.x, (G + 2) * UPH - 2 + (int)(threadIdx.x & 1));
+    const int head = at_unit / UPH, half = at_unit & 1;  // G: the key, G + 1: the value
+    const int u = at_unit % UPH / 2 * 8;                 // the pair's column in a half
+    const int col0 = (head < G ? kh * G + head : head == G ? n_q + kh : n_q + n_kv + kh) * HD +
+                     u + half * HALF;
+    const ProductSums& sums = fresh.sums;
+    const int at = max(0, L - 1);  // the new key's place in the row
+    const int64_t slot = fresh.slots[b];
+    const float* cs = fresh.cos_sin + (int64_t)fresh.positions[b] * HD + u;
+    const int last = bt[min(at / kBS, max_blocks - 1)];
+    f32x4 part[NEW][2];
+    const float* row = sums.part + (int64_t)b * sums.N + col0;
+#pragma unroll
+    for (int k = 0; k < NEW; ++k) {
+      const auto* from =
+          reinterpret_cast<const f32x4*>(row + min(k, sums.parts - 1) * sums.stride);
+      part[k][0] = from[0];
+      part[k][1] = from[1];
+    }
+    const int cols[1] = {col0};
+    const SumScales<1> by(sums, b, cols);
+    f32x4 cv[2], sv[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      cv[i] = reinterpret_cast<const f32x4*>(cs)[i];
+      sv[i] = reinterpret_cast<const f32x4*>(cs + HALF)[i];
+    }
+    in_order();
+    load_tile(0, first, start);
+    in_order();
+    f32x4 x[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int k = 0; k < NEW; ++k)
+        if (k < sums.parts) x[i] += part[k][i];
+    ushort8 o;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float f = x[j / 4][j % 4];
+      if (sums.sx) f = f * by.sx * by.sw[0][j];
+      o[j] = f32_to_bf16(f);
+      const float own = bf16_to_f32(o[j]), other = __shfl_xor(own, 1);
+      const float c = cv[j / 4][j % 4], s = sv[j / 4][j % 4];
+      if (head <= G) o[j] = f32_to_bf16(half ? own * c + other * s : own * c - other * s);
+    }
+    // the waves' turns go on over the splits
+    const bool owner = (max(n_units, 1) - 1) / kWaves % n_splits == split;
+    if (threadIdx.x < (G + 2) * UPH) {
+      const int unit = u / 8 + half * (UPH / 2);
+      if (head < G) {
+        *reinterpret_cast<ushort8*>(&q_lds[head * HD + ((unit ^ head) << 3)]) = o;
+      } else {
+        *reinterpret_cast<ushort8*>(&new_kv[head - G][unit * 8]) = o;
+        if (owner && slot >= 0) {
+          CT* cache = head == G ? k_cache : v_cache;
+          *reinterpret_cast<ushort8*>(
+              cache + ((slot / kBS * n_kv + kh) * kBS + slot % kBS) * HD + unit * 8) = o;
+        }
+      }
+    }
+    new_tile = slot >= 0 && slot == (int64_t)last * kBS + at % kBS ? n_units - 1 : -1;
+    __syncthreads();
+    if constexpr (!kQLds) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        q_frag[c] = *reinterpret_cast<const bf16x8*>(
+            &q_lds[q_head * HD + (((c * 4 + grp) ^ q_head) << 3)]);
+    }
+  }
+  if (first < n_units) {
+    if constexpr (NEW == 0) load_tile(0, first, start);
+    if constexpr (ONE) {
+      compute(0, first);
+    } else {
+      Blocks even, odd = look_up(first + turn);
+      for (int t = first; t < n_units; t += 2 * turn) {
+        load_tile(1, t + turn, odd);
+        even = look_up(t + 2 * turn);
+        in_order();
+        compute(0, t);
+        in_order();
+        load_tile(0, t + 2 * turn, even);
+        odd = look_up(t + 3 * turn);
+        in_order();
+        if (t + turn < n_units) compute(1, t + turn);
+      }
+    }
+  }
+
+  // ---- merge the waves -----------------------------------------------------
+  l_run = over_groups(l_run, [](float a, float c) { return a + c; });
+  __syncthreads();  // the V tiles are free
+  float* merge_o = reinterpret_cast<float*>(smem);  // [wave][G][HD]
+  if (col < G) {
+    float* mo = merge_o + (wave * G + col) * HD + grp * 4;
+#pragma unroll
+    for (int d = 0; d < ND; ++d)
+      *reinterpret_cast<f32x4*>(mo + d * 16) = o_acc[d];
+    if (grp == 0) {
+      merge_ml[wave][col][0] = m_run;
+      merge_ml[wave][col][1] = l_run;
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < G * (HD / 4); i += kBlockThreads) {
+    const int g = i / (HD / 4), e = i % (HD / 4) * 4;
+    float m_star = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) m_star = fmaxf(m_star, merge_ml[w][g][0]);
+    const float m_use = (m_star == -INFINITY) ? 0.f : m_star;
+    float l_star = 0.f;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const float c = __builtin_amdgcn_exp2f(merge_ml[w][g][0] - m_use);
+      l_star += merge_ml[w][g][1] * c;
+      o += *reinterpret_cast<const f32x4*>(merge_o + (w * G + g) * HD + e) * c;
+    }
+    const int64_t head = (int64_t)b * n_q + kh * G + g;
+    const int64_t part = (int64_t)part_row * n_q + kh * G + g;
+    if (n_splits == 1 && out) {
+      const float inv_l = 1.0f / l_star;
+      ushort4_t r;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) r[k] = f32_to_bf16(o[k] * inv_l);
+      *reinterpret_cast<ushort4_t*>(out + head * HD + e) = r;
+    } else {
+      // partial results (an empty split writes m = -inf, l = 0, o = 0)
+      *reinterpret_cast<f32x4*>(part_o + part * HD + e) = o;
+      if (e == 0) {
+        part_ml[part * 2] = m_star;
+        part_ml[part * 2 + 1] = l_star;
+      }
+    }
+  }
+}
+
+template <int HD, typename CT, bool CAP, bool ONE, int NEW>
+__launch_bounds__(kBlockThreads, waves_per_simd(HD)) __global__ void paged_decode_kernel(
+    ushort* __restrict__ out, const ushort* __restrict__ q, CT* k_cache, CT* v_cache,
+    const int32_t* __restrict__ block_tables, const int32_t* __restrict__ seq_lens,
+    const float scale, const float softcap, const int window, const int n_kv, const int G,
+    const int max_blocks, const int64_t q_stride, const int row_splits,
+    const Item* __restrict__ plan, const NewRows fresh, float* __restrict__ part_o,
+    float* __restrict__ part_ml) {
+  __shared__ Lds<HD, CT, NEW> mem;
+  attend_split<HD, CT, CAP, ONE, NEW>(mem, blockIdx.x, out, q, k_cache, v_cache, block_tables,
+                                      seq_lens, scale, softcap, window, n_kv, G, max_blocks,
+                                      q_stride, row_splits, plan, fresh, part_o, part_ml);
+}
+
+// Merged values of one query head, 2 or 4 a lane, rounded to bf16. The lanes read
+// all splits' (m, l) at once; the rows of O are on their way before those are used, up
+// to 16 at a time (as many as a row has splits), 4 where there are no more.
+template <int HD>
+struct Merged {
+  static constexpr int EPL = HD / 64;
+  typedef __attribute__((ext_vector_type(EPL))) float vec;
+  ushort v[EPL];
+  float ms, ls;
+  const vec* po;
+  int64_t step;
+  int n;
+  vec o[kMaxSplits];
+
+  // the head's parts lie n_q apart, at first + head and on
+  template <int MOST>
+  DEV_INLINE void load(const float* part_o, const float* part_ml, Splits of, int n_q,
+                       int head) {
+    const int lane = threadIdx.x % WAVE_SIZE;
+    const int64_t first = (int64_t)of.first * n_q + head;
+    n = of.n;
+    step = (int64_t)n_q * 64;
+    const float* pml = part_ml + (first + (int64_t)min(lane, n - 1) * n_q) * 2;
+    po = reinterpret_cast<const vec*>(part_o + first * HD) + lane;
+    ms = pml[0];
+    ls = pml[1];
+#pragma unroll
+    for (int k = 0; k < MOST; ++k) o[k] = po[min(k, n - 1) * step];
+  }
+  template <int MOST>
+  DEV_INLINE void finish() {
+    const int lane = threadIdx.x % WAVE_SIZE;
+    const float m_star = wave_reduce_max(ms);
+    const float c = __builtin_amdgcn_exp2f(ms - (m_star == -INFINITY ? 0.f : m_star));
+    const float l_star = wave_reduce_sum(lane < n ? ls * c : 0.f);
+    vec sum;
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) sum[e] = 0.f;
+#pragma unroll
+    for (int k = 0; k < MOST; ++k)
+      if (k < n) sum += o[k] * __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(c), k));
+    const float inv_l = 1.0f / l_star;
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) v[e] = f32_to_bf16(sum[e] * inv_l);
+  }
+};
+
+// a row's splits, from the plan or the same number for all
+DEV_INLINE Splits splits_of(const Splits* plan, int n, int row) {
+  return plan ? plan[row] : Splits{row * n, n};
+}
+
+// Merge the splits' results: one wave per (sequence, query head). A planned row that
+// was not split has its result.
+template <int HD>
+__global__ void decode_merge_kernel(
+    ushort* __restrict__ out,             // [B, n_q, hd]
+    const float* __restrict__ part_o, const float* __restrict__ part_ml,
+    const Splits* __restrict__ plan, const int n_splits, const int n_q,
+    const int64_t n_bh) {
+  constexpr int EPL = HD / 64;
+  const int64_t bh = (int64_t)blockIdx.x * (blockDim.x / WAVE_SIZE) +
+                     threadIdx.x / WAVE_SIZE;
+  if (bh >= n_bh) return;
+  const Splits of = splits_of(plan, n_splits, (int)(bh / n_q));
+  if (of.n == 1) return;
+  Merged<HD> m;
+  auto merge = [&](auto most) {
+    m.template load<decltype(most)::value>(part_o, part_ml, of, n_q, (int)(bh % n_q));
+    m.template finish<decltype(most)::value>();
+  };
+  if (of.n <= 4) merge(std::integral_constant<int, 4>{});
+  else merge(std::integral_constant<int, kMaxSplits>{});
+  ushort* oh = out + bh * HD + EPL * (threadIdx.x % WAVE_SIZE);
+#pragma unroll
+  for (int e = 0; e < EPL; e += 2)
+    *reinterpret_cast<uint32_t*>(oh + e) = ((uint32_t)m.v[e + 1] << 16) | m.v[e];
+}
+
+// The same, and the row (all heads of a sequence) to fp8 with one scale, as the
+// conversion of the merged bf16 row has it: one workgroup of 16 waves per row,
+// HPW heads a wave, one after the other: a chain of loads each, so only for few of
+// them (ops.decode_fp8_merges). Bound by its launch: 40 rows of 32 x 128 in 2 splits,
+// merge and conversion 9.6 us, this 5.1 (in a profile; beside the attention 1 less).
+// Rows from n_split on are no splits but bf16 rows of `whole`, to be converted.
+template <int HD, int HPW>
+__launch_bounds__(16 * WAVE_SIZE) __global__ void decode_merge_fp8_kernel(
+    unsigned char* __restrict__ out,      // [rows, n_q * hd]
+    float* __restrict__ out_scale,        // [rows]
+    const ushort* __restrict__ whole,     // [rows, n_q * hd], the first n_split not read
+    const int n_split,
+    const float* __restrict__ part_o, const float* __restrict__ part_ml,
+    const Splits* __restrict__ plan, const int n_splits, const int n_q) {
+  constexpr int EPL = HD / 64;
+  const int wave = threadIdx.x / WAVE_SIZE, lane = threadIdx.x % WAVE_SIZE;
+  const int64_t row = blockIdx.x;
+  __shared__ float red[16];
+  float vals[HPW][EPL];
+  float amax = 0.f;
+  Merged<HD> m[HPW];
+  Splits of{0, 1};
+  auto merge = [&](auto most) {
+    constexpr int MOST = decltype(most)::value;
+#pragma unroll
+    for (int h = 0; h < HPW; ++h)  // (past the last head: that again)
+      m[h].template load<MOST>(part_o, part_ml, of, n_q, min(h * 16 + wave, n_q - 1));
+#pragma unroll
+    for (int h = 0; h < HPW; ++h) {
+      m[h].template finish<MOST>();
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) {
+        vals[h][e] = bf16_to_f32(m[h].v[e]);
+        amax = fmaxf(amax, fabsf(vals[h][e]));
+      }
+    }
+  };
+  if (row < n_split) {
+    of = splits_of(plan, n_splits, (int)row);
+    if (of.n <= 4) merge(std::integral_constant<int, 4>{});
+    else merge(std::integral_constant<int, kMaxSplits>{});
+  } else {
+    typedef __attribute__((ext_vector_type(EPL))) ushort values;
+    values from[HPW];
+#pragma unroll
+    for (int h = 0; h < HPW; ++h)  // (past the last head: that again)
+      from[h] = *reinterpret_cast<const values*>(
+          whole + (row * n_q + min(h * 16 + wave, n_q - 1)) * HD + EPL * lane);
+#pragma unroll
+    for (int h = 0; h < HPW; ++h)
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) {
+        vals[h][e] = bf16_to_f32(from[h][e]);
+        amax = fmaxf(amax, fabsf(vals[h][e]));
+      }
+  }
+  amax = wave_reduce_max(amax);
+  if (lane == 0) red[wave] = amax;
+  __syncthreads();
+  float gmax = 1e-6f;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) gmax = fmaxf(gmax, red[w]);
+  if (threadIdx.x == 0) out_scale[row] = gmax / 448.0f;
+  const float inv_scale = 448.0f / gmax;
+#pragma unroll
+  for (int h = 0; h < HPW; ++h) {
+    const int head = h * 16 + wave;
+    if (head < n_q) {
+      unsigned char* to = out + (row * n_q + head) * HD + EPL * lane;
+      int w = __builtin_amdgcn_cvt_pk_fp8_f32(vals[h][0] * inv_scale,
+                                              vals[h][1] * inv_scale, 0, false);
+      if constexpr (EPL == 4) {
+        w = __builtin_amdgcn_cvt_pk_fp8_f32(vals[h][2] * inv_scale,
+                                            vals[h][3] * inv_scale, w, true);
+        *reinterpret_cast<uint32_t*>(to) = (uint32_t)w;
+      } else {
+        *reinterpret_cast<ushort*>(to) = (ushort)w;
+      }
+    }
+  }
+}
+
+}  // namespace
+}  // namespace decode

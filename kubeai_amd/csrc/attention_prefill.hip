@@ -55,8 +55,10 @@
 //   from the 8 bytes addressed by lane 4j + (l>>2), element l&3
 #include <torch/extension.h>
 
+#include <algorithm>
 #include <type_traits>
 
+#include "attention_decode.h"
 #include "common.h"
 
 namespace {
@@ -98,9 +100,13 @@ DEV_INLINE int find_tile(const int32_t* start, int n_seq, int size, int n,
 // Head size 128, and 256 where no row has many keys (kFewKeys). CT = cache element
 // type: ushort (bf16) or unsigned char (fp8 e5m2, converted to bf16 while staging). CAP:
 // capped scores. WIN: keys in (pos - window, pos] only.
+constexpr int tile_keys(int hd) { return hd == 128 ? 64 : 32; }
+template <int HD>
+using Tiles = char[2][2][tile_keys(HD) * HD * 2];  // places, K and V
+
 template <int HD, int GB, typename CT, bool WIN, bool CAP>
-__launch_bounds__(kNW * WAVE_SIZE, HD == 128 ? 2 : 1) __global__
-void paged_prefill_kernel(
+DEV_INLINE void attend_rows(
+    Tiles<HD>& lds, const int block,
     ushort* __restrict__ out,          // [Tq, n_q, HD]
     const ushort* __restrict__ q,      // [Tq, n_q, HD], rows strided
     const CT* __restrict__ k_cache,    // [nb, n_kv, 16, HD]
@@ -111,7 +117,7 @@ void paged_prefill_kernel(
     const float scale, const float softcap, const int window,
     const int n_kv, const int G, const int n_seq, const int max_blocks,
     const int64_t q_stride, const int n_tiles_q) {
-  constexpr int KVB = HD == 128 ? 64 : 32;  // keys per staged tile
+  constexpr int KVB = tile_keys(HD);  // keys per staged tile
   constexpr int NSUB = KVB / 32;
   constexpr int NBK = KVB / kBS;            // cache blocks per tile
   constexpr int RS = kNW / GB;              // row subtiles per workgroup
@@ -122,8 +128,8 @@ void paged_prefill_kernel(
   constexpr int ND = HD / 32;               // column blocks of O
 
   const int hg_n = G / GB;
-  const int kh = blockIdx.x % n_kv;
-  const int rest = blockIdx.x / n_kv;
+  const int kh = block % n_kv;
+  const int rest = block / n_kv;
   const int hg = rest % hg_n;
   int tile;
   const int b = __builtin_amdgcn_readfirstlane(
@@ -148,8 +154,6 @@ void paged_prefill_kernel(
   const int n_tiles = (kv_limit + KVB - 1) / KVB;
   const int kt0 = WIN ? max(0, ctx + row_lo - window + 1) / KVB : 0;
   const int last_blk = (kv_limit - 1) / kBS;
-
-  __shared__ __attribute__((aligned(16))) char lds[2][2][KVB * HD * 2];
 
   // ---- queries in registers, B operand per 16-wide step ------------------
   // (a negative scale turns the signs here, so that the largest product is
@@ -399,6 +403,57 @@ void paged_prefill_kernel(
           o[j] = f32_to_bf16(o_acc[d][rq * 4 + j] * inv_l);
         *reinterpret_cast<ushort4_t*>(op + d * 32 + rq * 8) = o;
       }
+  }
+}
+
+template <int HD, int GB, typename CT, bool WIN, bool CAP>
+__launch_bounds__(kNW * WAVE_SIZE, HD == 128 ? 2 : 1) __global__
+void paged_prefill_kernel(
+    ushort* __restrict__ out, const ushort* __restrict__ q, const CT* __restrict__ k_cache,
+    const CT* __restrict__ v_cache, const int32_t* __restrict__ block_tables,
+    const int32_t* __restrict__ query_start_loc, const int32_t* __restrict__ seq_lens,
+    const float scale, const float softcap, const int window, const int n_kv, const int G,
+    const int n_seq, const int max_blocks, const int64_t q_stride, const int n_tiles_q) {
+  __shared__ __attribute__((aligned(16))) Tiles<HD> lds;
+  attend_rows<HD, GB, CT, WIN, CAP>(lds, blockIdx.x, out, q, k_cache, v_cache, block_tables,
+                                    query_start_loc, seq_lens, scale, softcap, window, n_kv, G,
+                                    n_seq, max_blocks, q_stride, n_tiles_q);
+}
+
+// A step's prompt portions and its decode rows (head size 128, planned splits) in one
+// launch: neither fills the chip by itself, and each is a chain of latencies. The first
+// workgroups are the prompts', the longest of them first; the decode splits go where
+// there is room beside and behind them, two workgroups a CU by the prompts' registers.
+// us, two launches / this, each with the merge (heads 32/8): 32 rows of 100-700 and six
+// turns of 48-112 behind 300-600 43.0 / 36.7, to fp8 46.0 / 38.8; 28 rows and four prompts
+// of 20-120 25.4 / 18.7; 40 rows of 50-1000 and 17 tokens 30.1 / 22.1, 300 tokens 37.1 /
+// 27.0, 2000 tokens 91.9 / 82.7, 6000 tokens 372 / 366; 96 of 1500-4000 and 100 tokens
+// 208 / 199; one row and 20 tokens 13.4 / 9.1. The results are the same bits.
+template <int GB, typename CT, bool WIN, bool CAP>
+__launch_bounds__(kNW * WAVE_SIZE, 2) __global__ void step_attention_kernel(
+    ushort* __restrict__ out,  // [T, n_q, 128], the decode rows first
+    ushort* __restrict__ decode_out,  // the same, or null: parts of all decode rows
+    const ushort* __restrict__ q, CT* k_cache, CT* v_cache,
+    const int32_t* __restrict__ prompt_tables, const int32_t* __restrict__ query_start_loc,
+    const int32_t* __restrict__ prompt_lens, const int32_t* __restrict__ decode_tables,
+    const int32_t* __restrict__ decode_lens, const float scale, const float softcap,
+    const int window, const int n_kv, const int G, const int n_seq, const int prompt_blocks,
+    const int decode_blocks, const int64_t q_stride, const int n_tiles_q, const int n_decode,
+    const int prompt_wgs, const decode::Item* __restrict__ plan, float* __restrict__ part_o,
+    float* __restrict__ part_ml) {
+  static_assert(kNW == decode::kWaves);
+  using Own = decode::Lds<128, CT, 0>;
+  __shared__ __attribute__((aligned(16))) char mem[std::max(sizeof(Tiles<128>), sizeof(Own))];
+  if ((int)blockIdx.x < prompt_wgs) {
+    attend_rows<128, GB, CT, WIN, CAP>(
+        *reinterpret_cast<Tiles<128>*>(mem), blockIdx.x, out + (int64_t)n_decode * n_kv * G * 128,
+        q + n_decode * q_stride, k_cache, v_cache, prompt_tables, query_start_loc, prompt_lens,
+        scale, softcap, window, n_kv, G, n_seq, prompt_blocks, q_stride, n_tiles_q);
+  } else {
+    decode::attend_split<128, CT, CAP, false, 0>(
+        *reinterpret_cast<Own*>(mem), blockIdx.x - prompt_wgs, decode_out, q, k_cache, v_cache,
+        decode_tables, decode_lens, scale, softcap, window, n_kv, G, decode_blocks, q_stride, 1,
+        plan, decode::NewRows{}, part_o, part_ml);
   }
 }
 
@@ -936,5 +991,105 @@ void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
   };
   if (fp8_cache) sizes((unsigned char)0);
   else sizes((ushort)0);
+  HIP_CHECK_KERNEL();
+}
+
+// paged_attention_prefill of rows n_decode.. of q [T, n_q, 128] and paged_attention_decode
+// of those before, by a plan, in one launch and the merge of the decode rows' splits. out
+// [T, n_q, 128] bf16, or (out_scale fp32 [T]) [T, n_q * 128] fp8 rows with a scale each,
+// which the merge makes of up to 32 heads.
+void paged_attention_step(torch::Tensor out, c10::optional<torch::Tensor> out_scale,
+                          torch::Tensor q, int64_t n_decode, torch::Tensor k_cache,
+                          torch::Tensor v_cache, torch::Tensor decode_tables,
+                          torch::Tensor decode_lens, torch::Tensor plan,
+                          torch::Tensor prompt_tables, torch::Tensor query_start_loc,
+                          torch::Tensor prompt_lens, double scale, int64_t window,
+                          double softcap) {
+  TORCH_CHECK(q.dim() == 3 && q.stride(2) == 1 && q.stride(1) == 128 && q.size(2) == 128 &&
+              q.scalar_type() == torch::kBFloat16 && q.is_cuda());
+  TORCH_CHECK(k_cache.is_contiguous() && v_cache.is_contiguous() && k_cache.dim() == 4 &&
+              v_cache.sizes() == k_cache.sizes() && k_cache.size(2) == kBS &&
+              k_cache.size(3) == 128 && v_cache.scalar_type() == k_cache.scalar_type());
+  TORCH_CHECK(k_cache.scalar_type() == torch::kBFloat16 ||
+              k_cache.scalar_type() == torch::kFloat8_e5m2);
+  for (const auto& t : {decode_tables, decode_lens, plan, prompt_tables, query_start_loc,
+                        prompt_lens})
+    TORCH_CHECK(t.scalar_type() == torch::kInt32 && t.is_contiguous() && t.is_cuda());
+  const int64_t T = q.size(0), n_q = q.size(1);
+  const int n_kv = k_cache.size(1), G = n_q / n_kv, B = prompt_lens.numel();
+  const int64_t D = n_decode, Tq = T - D;
+  TORCH_CHECK(n_q % n_kv == 0 && (G == 1 || G == 2 || G == 4 || G == 8),
+              "unsupported GQA group size ", G);
+  TORCH_CHECK(D >= 1 && Tq >= 1 && B >= 1 && decode_lens.numel() == D &&
+              decode_tables.dim() == 2 && decode_tables.size(0) == D &&
+              prompt_tables.dim() == 2 && prompt_tables.size(0) == B &&
+              query_start_loc.numel() == B + 1);
+  TORCH_CHECK(plan.dim() == 1 && plan.numel() >= 6 * D && (plan.numel() - 2 * D) % 4 == 0 &&
+              ((uintptr_t)plan.data_ptr() & 15) == 0);
+  const bool fp8 = out_scale.has_value();
+  TORCH_CHECK(out.is_contiguous() && out.is_cuda() && out.numel() == T * n_q * 128 &&
+              out.scalar_type() == (fp8 ? torch::kFloat8_e4m3fn : torch::kBFloat16));
+  if (fp8)
+    TORCH_CHECK(n_q <= 32 && out_scale->is_contiguous() && out_scale->is_cuda() &&
+                out_scale->scalar_type() == torch::kFloat32 && out_scale->numel() == T);
+  const int64_t items = (plan.numel() - 2 * D) / 4;
+  const auto* item = reinterpret_cast<const decode::Item*>(plan.data_ptr());
+  const auto* splits = reinterpret_cast<const decode::Splits*>(item + items);
+  const auto opts = q.options().dtype(torch::kFloat32);
+  auto part_o = torch::empty({items, n_q, 128}, opts), part_ml = torch::empty({items, n_q, 2}, opts);
+  auto rows = fp8 ? torch::empty({T, n_q, 128}, q.options()) : out;
+  const int GB = std::min(G, 4), qr = kNW / GB * kQB;
+  const int n_tiles_q = Tq / qr + B;  // see find_tile
+  const int64_t prompt_wgs = (int64_t)n_tiles_q * (G / GB) * n_kv;
+  TORCH_CHECK(prompt_wgs + items * n_kv < (int64_t)1 << 31);
+  auto stream = c10::hip::getCurrentHIPStream().stream();
+  auto launch = [&](auto gb, auto ct, auto win, auto cap) {
+    using CT = decltype(ct);
+    hipLaunchKernelGGL(
+        (step_attention_kernel<decltype(gb)::value, CT, decltype(win)::value,
+                               decltype(cap)::value>),
+        dim3((uint32_t)(prompt_wgs + items * n_kv)), dim3(kNW * WAVE_SIZE), 0, stream,
+        (ushort*)rows.data_ptr(), fp8 ? nullptr : (ushort*)rows.data_ptr(),
+        (const ushort*)q.data_ptr(), (CT*)k_cache.data_ptr(), (CT*)v_cache.data_ptr(),
+        prompt_tables.data_ptr<int32_t>(), query_start_loc.data_ptr<int32_t>(),
+        prompt_lens.data_ptr<int32_t>(), decode_tables.data_ptr<int32_t>(),
+        decode_lens.data_ptr<int32_t>(), (float)scale, (float)softcap, (int)window, n_kv, G, B,
+        (int)prompt_tables.size(1), (int)decode_tables.size(1), q.stride(0), n_tiles_q, (int)D,
+        (int)prompt_wgs, item, part_o.data_ptr<float>(), part_ml.data_ptr<float>());
+  };
+  auto masks = [&](auto gb, auto ct) {
+    if (window > 0) {
+      if (softcap > 0.0) launch(gb, ct, std::true_type{}, std::true_type{});
+      else launch(gb, ct, std::true_type{}, std::false_type{});
+    } else {
+      if (softcap > 0.0) launch(gb, ct, std::false_type{}, std::true_type{});
+      else launch(gb, ct, std::false_type{}, std::false_type{});
+    }
+  };
+  auto heads = [&](auto ct) {
+    if (GB == 1) masks(std::integral_constant<int, 1>{}, ct);
+    else if (GB == 2) masks(std::integral_constant<int, 2>{}, ct);
+    else masks(std::integral_constant<int, 4>{}, ct);
+  };
+  if (k_cache.scalar_type() == torch::kFloat8_e5m2) heads((unsigned char)0);
+  else heads((ushort)0);
+  HIP_CHECK_KERNEL();
+  if (fp8) {
+    auto merge = [&](auto hpw) {
+      hipLaunchKernelGGL((decode::decode_merge_fp8_kernel<128, decltype(hpw)::value>),
+                         dim3((uint32_t)T), dim3(16 * WAVE_SIZE), 0, stream,
+                         (unsigned char*)out.data_ptr(), out_scale->data_ptr<float>(),
+                         (const ushort*)rows.data_ptr(), (int)D, part_o.data_ptr<float>(),
+                         part_ml.data_ptr<float>(), splits, 1, (int)n_q);
+    };
+    if (n_q <= 16) merge(std::integral_constant<int, 1>{});
+    else merge(std::integral_constant<int, 2>{});
+  } else {
+    const int64_t n_bh = D * n_q;
+    hipLaunchKernelGGL((decode::decode_merge_kernel<128>), dim3((uint32_t)((n_bh + 3) / 4)),
+                       dim3(4 * WAVE_SIZE), 0, stream, (ushort*)out.data_ptr(),
+                       part_o.data_ptr<float>(), part_ml.data_ptr<float>(), splits, 1, (int)n_q,
+                       n_bh);
+  }
   HIP_CHECK_KERNEL();
 }

@@ -40,6 +40,13 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
                             double scale, int64_t window, double softcap,
                             c10::optional<torch::Tensor> out_scale,
                             c10::optional<torch::Tensor> plan);
+void paged_attention_step(torch::Tensor out, c10::optional<torch::Tensor> out_scale,
+                          torch::Tensor q, int64_t n_decode, torch::Tensor k_cache,
+                          torch::Tensor v_cache, torch::Tensor decode_tables,
+                          torch::Tensor decode_lens, torch::Tensor plan,
+                          torch::Tensor prompt_tables, torch::Tensor query_start_loc,
+                          torch::Tensor prompt_lens, double scale, int64_t window,
+                          double softcap);
 void paged_attention_decode_sums(torch::Tensor out, torch::Tensor part,
                                  c10::optional<torch::Tensor> sx,
                                  c10::optional<torch::Tensor> sw, int64_t n_q,
@@ -156,6 +163,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),
         py::arg("seq_lens"), py::arg("scale"), py::arg("window"), py::arg("softcap"),
         py::arg("out_scale") = py::none(), py::arg("plan") = py::none());
+  m.def("paged_attention_step", &paged_attention_step,
+        "a step's prompt portions and decode rows in one launch");
   m.def("paged_attention_decode_sums", &paged_attention_decode_sums,
         "paged decode attention of rows that are a product's sums");
   m.def("paged_decode_plan", &paged_decode_plan,

@@ -191,11 +191,7 @@ class Attention(nn.Module):
             )
             if not fp8_in:
                 out = out.view(T, -1)
-            if lora_live:
-                return _project_adapted(
-                    self.o_proj, out, as_sums, fb, lm, self.layer_idx, "o"
-                )
-            return _project(self.o_proj, out, as_sums, fb)
+            return self._out_proj(out, fb, lm if lora_live else None, as_sums)
         if self.qk_norm:
             # gemma3: per-head RMSNorm ((1+w) stored as w) before rope;
             # fp32 math, contiguous bf16 out. v follows to contiguous —
@@ -228,6 +224,15 @@ class Attention(nn.Module):
                 ),
                 as_sums, fb,
             )
+        if fb.n_prefill > 0 and ops.step_attention_takes(q, nd, k_cache, plan):
+            out = ops.paged_attention_step(
+                q, nd, k_cache, v_cache, fb.decode_block_tables, fb.decode_seq_lens,
+                fb.prefill_block_tables, fb.prefill_query_start_loc, fb.prefill_seq_lens,
+                self.scale, window=self.window, softcap=self.softcap, plan=plan, fp8=fp8_in,
+            )
+            if fp8_in:
+                return _project(self.o_proj, out, as_sums, fb)
+            return self._out_proj(out.view(T, -1), fb, lm if lora_live else None, as_sums)
         out = torch.empty(
             (T, self.n_q, self.hd), dtype=q.dtype, device=q.device
         )
@@ -260,11 +265,13 @@ class Attention(nn.Module):
         attn_flat = out.view(T, -1)
         if fp8_in:
             return _project(self.o_proj, ops.quant_fp8(attn_flat), as_sums, fb)
-        if lora_live:
-            return _project_adapted(
-                self.o_proj, attn_flat, as_sums, fb, lm, self.layer_idx, "o"
-            )
-        return _project(self.o_proj, attn_flat, as_sums, fb)
+        return self._out_proj(attn_flat, fb, lm if lora_live else None, as_sums)
+
+    def _out_proj(self, x, fb, lm, as_sums: bool):
+        """lm: the adapters that are live in this step, or None."""
+        if lm is not None:
+            return _project_adapted(self.o_proj, x, as_sums, fb, lm, self.layer_idx, "o")
+        return _project(self.o_proj, x, as_sums, fb)
 
 
 class MLP(nn.Module):

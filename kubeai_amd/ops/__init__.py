@@ -247,6 +247,44 @@ def paged_attention_decode_sums(
     return (flat, out_scale) if merges else quant_fp8(flat)
 
 
+def step_attention_takes(q, n_decode: int, k_cache, plan) -> bool:
+    """Whether paged_attention_step has a step of these queries [T, n_q, hd]."""
+    n_kv = k_cache.shape[1]
+    return (
+        plan is not None  # (on the GPU)
+        and 0 < n_decode < q.shape[0]
+        and q.shape[2] == 128
+        and q.dtype == torch.bfloat16
+        and q.stride(1) == 128 and q.stride(2) == 1
+        and q.shape[1] in (n_kv, 2 * n_kv, 4 * n_kv, 8 * n_kv)
+    )
+
+
+def paged_attention_step(
+    q, n_decode: int, k_cache, v_cache, decode_tables, decode_lens, prompt_tables,
+    query_start_loc, prompt_lens, scale: float, window: int = 0, softcap: float = 0.0,
+    plan=None, fp8: bool = False,
+):
+    """paged_attention_decode of the first n_decode rows and paged_attention_prefill of
+    the others in one launch (step_attention_takes): [T, n_q, hd] bf16, or (fp8)
+    quant_fp8 of its rows. Up to 1024 rows of up to 32 heads the merge of the decode rows'
+    splits converts them; its workgroup a row is the slower conversion of many (us, with
+    the attention, merge and conversion apart / one: 572 rows 41 / 38.8, 1501 rows 62 /
+    62.3, 2008 rows 80 / 86, 6040 rows 371 / 393)."""
+    T, n_q, hd = q.shape
+    merges = fp8 and n_q <= 32 and T <= 1024
+    out = torch.empty((T, n_q, hd), device=q.device,
+                      dtype=torch.float8_e4m3fn if merges else torch.bfloat16)
+    out_scale = torch.empty(T, dtype=torch.float32, device=q.device) if merges else None
+    _C.paged_attention_step(
+        out, out_scale, q, n_decode, k_cache, v_cache, decode_tables, decode_lens, plan,
+        prompt_tables, query_start_loc, prompt_lens, scale, window, softcap)
+    if not fp8:
+        return out
+    flat = out.view(T, n_q * hd)
+    return (flat, out_scale) if merges else quant_fp8(flat)
+
+
 def paged_attention_prefill(
     q, k_cache, v_cache, block_tables, query_start_loc, seq_lens, scale: float,
     out=None, window: int = 0, softcap: float = 0.0,
