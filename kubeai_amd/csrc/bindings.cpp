@@ -84,6 +84,7 @@ void tiled_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                   c10::optional<torch::Tensor> sx,
                   c10::optional<torch::Tensor> sw, int64_t act);
 torch::Tensor tiled_sums(torch::Tensor x, torch::Tensor w);
+torch::Tensor narrow_sums(torch::Tensor x, torch::Tensor w);
 std::tuple<int64_t, int64_t, double> tiled_plan(int64_t M, int64_t N, int64_t KB,
                                                 bool fp8, bool sums, int64_t experts);
 void moe_route(torch::Tensor index, torch::Tensor weight, torch::Tensor begin,
@@ -188,6 +189,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "tile shape, parts and us of a tiled product, whole or as sums",
         py::arg("M"), py::arg("N"), py::arg("KB"), py::arg("fp8"), py::arg("sums"),
         py::arg("experts") = 1);
+  m.def("narrow_sums", &narrow_sums, "sums of up to 64 rows, tiles of 64 columns");
   m.def("tiled_sums", &tiled_sums, "fp32 part sums of a product of many rows");
   m.def("skinny_sums", &skinny_sums, "fp32 part sums of a skinny product");
   m.def("skinny_gated", &skinny_gated, "weight-streaming gate and up, activated");

@@ -67,8 +67,11 @@ struct Shape {
   constexpr int cols() const { return 64 * wn; }
 };
 constexpr Shape kShapes[] = {{4, 4, 2, 3}, {3, 4, 2, 3}, {4, 3, 2, 3}, {3, 3, 3, 3},
-                             {2, 4, 3, 3}, {3, 2, 3, 3}, {2, 2, 4, 4}, {1, 2, 4, 4}};
+                             {2, 4, 3, 3}, {3, 2, 3, 3}, {2, 2, 4, 4}, {1, 2, 4, 4},
+                             {1, 1, 6, 6}};
 constexpr int kNumShapes = sizeof(kShapes) / sizeof(kShapes[0]);
+// the last shape is for the sums of few rows alone (tiled_gemm.hip: narrow_sums)
+constexpr int kNarrow = kNumShapes - 1;
 
 void launch_fp8(int shape, Epilogue epi, const Args& a, int grid);
 void launch_bf16(int shape, Epilogue epi, const Args& a, int grid);
@@ -262,16 +265,24 @@ __global__ __launch_bounds__(256, 1) void tiled_kernel(const Args a) {
     }
   };
 
-  f32x16 acc[WN][WM];
+  constexpr int C = FP8 ? 2 : 4;              // chunks of K a step
+  // A sum for each chunk of a step where there are few parts: the error grows with the
+  // terms that are added one behind the other (bf16 4096 x 14336 in 4 parts 3.7e-7 of the
+  // result, 2.5e-7 in the 8 that other tiles have, 1.7e-7 with these sums).
+  constexpr int SUMS = SHAPE == kNarrow ? C : 1;
+  f32x16 sums[SUMS][WN][WM];
 #pragma unroll
-  for (int i = 0; i < WN; i++) {
+  for (int u = 0; u < SUMS; u++) {
 #pragma unroll
-    for (int j = 0; j < WM; j++) {
+    for (int i = 0; i < WN; i++) {
 #pragma unroll
-      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+      for (int j = 0; j < WM; j++) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) sums[u][i][j][r] = 0.f;
+      }
     }
   }
-  constexpr int C = FP8 ? 2 : 4;              // chunks of K a step
+  auto& acc = sums[0];
   constexpr int MF = WM * WN, RO = WM + WN;   // products, operands a chunk
   typename std::conditional<FP8, i32x8, bf16x8>::type va[2][WM], vb[2][WN];
   // operand o of chunk c: b[0], a[0], the other b, the other a
@@ -292,8 +303,9 @@ __global__ __launch_bounds__(256, 1) void tiled_kernel(const Args a) {
       else va[buf][i] = v;
     }
   };
-  auto multiply = [&](int t, int buf) {
-    const int j = t / WN, i = t % WN;
+  auto multiply = [&](int t, int c) {
+    const int j = t / WN, i = t % WN, buf = c & 1;
+    auto& acc = sums[c % SUMS];
     if constexpr (FP8) {  // block scales of 1
       acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
           vb[buf][i], va[buf][j], acc[i][j], 0, 0, 0, 0x7f7f7f7f, 0, 0x7f7f7f7f);
@@ -365,7 +377,7 @@ __global__ __launch_bounds__(256, 1) void tiled_kernel(const Args a) {
           if (last) read(o, (c + 1) & 1, na, nb, 0);
           else read(o, (c + 1) & 1, pa, pb, c + 1);
         }
-        multiply(t, c & 1);
+        multiply(t, c);
         const int g = last ? t : (c + 1) * MF + t;
         const int end = g == C * MF - 1 ? L : begun(g + 1);
 #pragma unroll
@@ -384,6 +396,17 @@ __global__ __launch_bounds__(256, 1) void tiled_kernel(const Args a) {
   }
   wait_loads<0>();
   barrier();
+#pragma unroll
+  for (int u = SUMS / 2; u > 0; u /= 2) {
+#pragma unroll
+    for (int c = 0; c < u; c++) {
+#pragma unroll
+      for (int i = 0; i < WN; i++) {
+#pragma unroll
+        for (int j = 0; j < WM; j++) sums[c][i][j] += sums[c + u][i][j];
+      }
+    }
+  }
 
   // A lane's sums are row l31 and, four at a time, columns 8 q + 4 hi: all the
   // first halves of 8 columns lie in front of all the second ones.
@@ -478,7 +501,8 @@ void launch(int shape, const Args& a, int grid) {
   auto stream = c10::hip::getCurrentHIPStream().stream();
   auto go = [&](auto s) {
     constexpr int i = decltype(s)::value;
-    if constexpr ((EPI != kSilu && EPI != kGelu) || kShapes[i].wn % 2 == 0) {
+    if constexpr (EPI == kSums ||
+                  (i != kNarrow && ((EPI != kSilu && EPI != kGelu) || kShapes[i].wn % 2 == 0))) {
       hipLaunchKernelGGL((tiled_kernel<FP8, i, EPI>), dim3(grid), dim3(256), 0, stream, a);
     } else {
       TORCH_CHECK(false, "no such tile");
@@ -492,7 +516,9 @@ void launch(int shape, const Args& a, int grid) {
     case 4: go(std::integral_constant<int, 4>{}); break;
     case 5: go(std::integral_constant<int, 5>{}); break;
     case 6: go(std::integral_constant<int, 6>{}); break;
-    default: go(std::integral_constant<int, 7>{}); break;
+    case 7: go(std::integral_constant<int, 7>{}); break;
+    case 8: go(std::integral_constant<int, 8>{}); break;
+    default: TORCH_CHECK(false, "no such tile");
   }
   HIP_CHECK_KERNEL();
 }

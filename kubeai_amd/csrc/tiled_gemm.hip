@@ -23,12 +23,12 @@ namespace {
 struct Cost {
   float step, tile, rest, mb;
 };
-constexpr Cost kOne[2][kNumShapes] = {
+constexpr Cost kOne[2][kNarrow] = {
     {{1.083f, 8.7f, 0.f}, {0.869f, 6.7f, 0.f}, {0.878f, 7.1f, 0.f}, {0.724f, 5.5f, 0.f},
      {0.752f, 4.1f, 0.f}, {0.577f, 3.7f, 0.f}, {0.484f, 2.6f, 0.f}, {0.357f, 1.3f, 1.1f}},
     {{1.058f, 10.8f, 0.f}, {0.874f, 9.1f, 0.f}, {0.877f, 10.9f, 0.f}, {0.710f, 9.0f, 0.f},
      {0.676f, 6.7f, 0.f}, {0.518f, 5.6f, 0.f}, {0.404f, 4.4f, 0.f}, {0.292f, 2.5f, 1.2f}}};
-constexpr Cost kParts[2][kNumShapes] = {
+constexpr Cost kParts[2][kNarrow] = {
     {{1.081f, 2.5f, 5.2f, 0.21f}, {0.857f, 0.8f, 5.3f, 0.25f}, {0.869f, 1.3f, 5.1f, 0.23f},
      {0.701f, 1.0f, 4.3f, 0.25f}, {0.742f, 0.f, 4.4f, 0.27f},  {0.568f, 0.6f, 3.3f, 0.28f},
      {0.480f, 0.4f, 2.6f, 0.31f}, {0.365f, 1.0f, 1.9f, 0.27f}},
@@ -47,7 +47,7 @@ struct Plan {
 // half as many)
 Plan plan(bool fp8, int64_t R, int64_t E, int64_t cols, int64_t KB, bool halves, bool sums) {
   Plan best{-1, 1, 0.};
-  for (int i = 0; i < kNumShapes; i++) {
+  for (int i = 0; i < kNarrow; i++) {
     const Shape s = kShapes[i];
     if (halves && s.wn % 2) continue;
     const Cost c = (sums ? kParts : kOne)[fp8][i];
@@ -222,23 +222,48 @@ void tiled_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   run(o, epi, p.shape, (a.R + s.rows() - 1) / s.rows() * ((cols + bn - 1) / bn));
 }
 
+// x w^T as `parts` sums (none of them empty) in tiles of a shape
+static torch::Tensor sums_of(Operands& o, int shape, int parts) {
+  Args& a = o.a;
+  auto part = torch::empty({parts, a.R, a.N}, o.x.options().dtype(torch::kFloat32));
+  if (a.R == 0) return part;
+  a.k_part = (a.KB / kStep + parts - 1) / parts * kStep;
+  a.part = part.data_ptr<float>();
+  const Shape s = kShapes[shape];
+  run(o, kSums, shape,
+      (int64_t)(a.R + s.rows() - 1) / s.rows() * ((a.N + s.cols() - 1) / s.cols()) * parts);
+  return part;
+}
+
 // the fp32 sums of x w^T alone, [parts, M, N], for a consumer that adds the
 // parts itself (and applies an fp8 product's scales)
 torch::Tensor tiled_sums(torch::Tensor x, torch::Tensor w) {
   Operands o = operands(x, w.unsqueeze(0), c10::nullopt, c10::nullopt, true);
-  Args& a = o.a;
   TORCH_CHECK(o.x.size(0) < (int64_t)1 << 30);
-  a.R = (int)o.x.size(0);
-  const Plan p = plan(o.fp8, a.R, 1, a.N, a.KB, false, true);
-  auto part = torch::empty({p.parts, a.R, a.N}, x.options().dtype(torch::kFloat32));
-  if (a.R == 0) return part;
-  const int steps = a.KB / kStep;
-  a.k_part = (steps + p.parts - 1) / p.parts * kStep;
-  a.part = part.data_ptr<float>();
-  const Shape s = kShapes[p.shape];
-  run(o, kSums, p.shape,
-      (int64_t)(a.R + s.rows() - 1) / s.rows() * ((a.N + s.cols() - 1) / s.cols()) * p.parts);
-  return part;
+  o.a.R = (int)o.x.size(0);
+  const Plan p = plan(o.fp8, o.a.R, 1, o.a.N, o.a.KB, false, true);
+  return sums_of(o, p.shape, p.parts);
+}
+
+// The same of up to 64 rows in tiles of 64 columns, whose workgroups are at most one a
+// CU: half the parts that tiles of 128 columns need to fill the chip, which half the
+// bytes are written and read again by (40 rows of 4096 columns in 8 parts: 5.2 MB, where
+// the fp8 weights of K 4096 are 16.8), and five steps of 16 KB on their way to each CU.
+// us with the norm, weights out of cache, the streaming or wider tiles' sums / these: fp8
+// 4096 x 4096 1 row 10.4 / 10.3, 24 rows 12.2 / 11.4, 40 rows 13.5 / 12.2, 64 rows 14.4 /
+// 13.3; 6144 x 4096 1 row 12.9 / 12.4, 40 rows 15.2 / 14.4; 4096 x 14336 40 rows 20.5 / 19.1;
+// bf16 4096 x 4096 1 row 13.0 / 13.0, 40 rows 15.8 / 14.0; 4096 x 14336 1 row 29.1 / 29.3, 40
+// rows 31.1 / 29.2; 2304 x 9216 40 rows 19.6 / 15.9. With four places instead of six 0.3 to 0.9 less gain where K is long,
+// with eight where it is short.
+torch::Tensor narrow_sums(torch::Tensor x, torch::Tensor w) {
+  Operands o = operands(x, w.unsqueeze(0), c10::nullopt, c10::nullopt, true);
+  constexpr Shape s = kShapes[kNarrow];
+  TORCH_CHECK(o.x.size(0) <= s.rows(), "up to 64 rows");
+  o.a.R = (int)o.x.size(0);
+  const int tiles = (o.a.N + s.cols() - 1) / s.cols(), steps = o.a.KB / kStep;
+  const int most = std::max(1, std::min({kMaxParts, 256 / tiles, steps}));
+  const int per = (steps + most - 1) / most;
+  return sums_of(o, kNarrow, (steps + per - 1) / per);
 }
 
 // How a product (or M rows of that many experts' products) is planned, whole or as

@@ -743,12 +743,36 @@ def few_tiled_better(M: int, N: int, K: int, fp8: bool, rope: bool, sums: bool) 
     )
 
 
+def narrow_better(M: int, N: int, K: int, fp8: bool) -> bool:
+    """Whether a product of up to 64 rows is best read as the sums of tiles of 64 columns
+    (csrc/tiled_gemm.hip: narrow_sums): their workgroups, one a CU at most, leave few CUs
+    idle, and K is more than a few steps for each. Over 96 products (512 to 16000 columns,
+    K 1024 to 24000) whose sums were the streaming or the wider tiles', with the norm, the
+    chosen ones take 0.91 of the time, 1.07 at worst; over 59 that were the library's 0.72,
+    1.07 at worst (us: fp8 6144 x 4096 40 rows 17.8 / 14.3, bf16 2304 x 9216 1 row 20.5 /
+    14.6, 15168 x 12288 78 / 84). Left: bf16 with 192 workgroups (6144 x 4096 40 rows 18.4 /
+    19.8), fewer of them (8256 x 9344 44 rows 39 / 54), few steps (fp8 2048 x 2048 8 rows
+    7.3 / 8.3)."""
+    if type(M) is not int or not 1 <= M <= 64 or N < 1:  # (a trace has tensors)
+        return False
+    tiles, steps = -(-N // 64), K * (1 if fp8 else 2) // 128
+    parts = min(8, 256 // tiles) if tiles <= 256 else 0
+    return (
+        parts > 0
+        and parts * tiles >= (192 if fp8 else 200)
+        and steps >= parts * (5 if M > 16 else 7)
+    )
+
+
 def tiled_sums(x, weight, x_scale=None, w_scale=None):
     """x weight^T as ProductSums of the tiled product, cut along K so that it
-    fills the chip, or None for operands that it does not take."""
+    fills the chip (narrow_better: in tiles of 64 columns), or None for operands that it
+    does not take."""
     if not _tiled_operands(x, weight) or x_scale is not None and observed(x_scale, w_scale):
         return None
-    return ProductSums(_C.tiled_sums(x, weight), x_scale, w_scale)
+    narrow = narrow_better(x.shape[0], *weight.shape, x.element_size() == 1)
+    sums = _C.narrow_sums if narrow else _C.tiled_sums
+    return ProductSums(sums(x, weight), x_scale, w_scale)
 
 
 def sums_for_reader(x, weight, x_scale=None, w_scale=None, rope=False, eager=False):
@@ -760,7 +784,9 @@ def sums_for_reader(x, weight, x_scale=None, w_scale=None, rope=False, eager=Fal
         better = type(M) is int and tiled_sums_better(M, N, K, fp8)
         return tiled_sums(x, weight, x_scale, w_scale) if better else None
     sums = sums_better(M, N, K, fp8=fp8, rope=rope, eager=eager)
-    if M > 16 and N < 16384 and few_tiled_better(M, N, K, fp8, rope, sums):
+    if narrow_better(M, N, K, fp8) or (
+        M > 16 and N < 16384 and few_tiled_better(M, N, K, fp8, rope, sums)
+    ):
         got = tiled_sums(x, weight, x_scale, w_scale)
         if got is not None:
             return got
