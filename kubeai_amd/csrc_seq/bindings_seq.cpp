@@ -63,7 +63,8 @@ void qknorm_rope_half_and_cache(torch::Tensor q, torch::Tensor k, torch::Tensor 
                                 torch::Tensor slot_mapping);
 void sandwich_rmsnorm(torch::Tensor out, c10::optional<torch::Tensor> branch,
                       c10::optional<torch::Tensor> post_weight,
-                      torch::Tensor residual, torch::Tensor pre_weight, double eps);
+                      torch::Tensor residual, torch::Tensor pre_weight, double eps,
+                      c10::optional<torch::Tensor> place);
 void rmsnorm_to_cache(torch::Tensor cache, torch::Tensor x, torch::Tensor weight,
                       torch::Tensor slot_mapping, double eps);
 void sigmoid_gate(torch::Tensor out, torch::Tensor x, torch::Tensor gate);

@@ -55,11 +55,18 @@ __global__ __launch_bounds__(kBlock) void sandwich_rmsnorm_kernel(
 // them every result are the same to the last bit. us, before -> this: 40 x 2048
 // 6.2 -> 4.6, 40 x 4096 9.8 -> 6.5, 3072 x 2048 21.7 -> 15.9, 3072 x 4096 37.0 ->
 // 33.4 (75 and 151 MB).
-template <typename T, typename B, int K>
+// GATHER: the branch's row t is the sum of the rows place[t, :top] (experts' rows, which
+// combine_rows_kernel would add; the same bits), four of them asked for at a time, 16
+// bytes a lane, and handed over in LDS (two bytes a lane: 3072 x 2048 of 3 rows 42 us).
+// Bound by memory too: 3072 x 2048 of 3 rows 101 MB. us, that kernel and this one / here:
+// 3072 x 2048 of 3 rows 33.0 / 21.8, of 5 39.6 / 27.7; 300 x 2048 of 3 9.8 / 6.4; 3072 x 4096
+// of 3 72 / 43.
+template <typename T, typename B, int K, bool GATHER>
 __global__ __launch_bounds__(kBlock) void sandwich_rmsnorm_rows_kernel(
     T* __restrict__ out, const B* __restrict__ branch,
     const float* __restrict__ post_w, float* __restrict__ residual,
-    const float* __restrict__ pre_w, int C, float eps) {
+    const float* __restrict__ pre_w, int C, float eps, const int* __restrict__ place,
+    int top) {
   __shared__ float red0[16], red1[16];
   const size_t base = (size_t)blockIdx.x * C;
   float x[K], b[K], pw[K], qw[K];
@@ -67,10 +74,36 @@ __global__ __launch_bounds__(kBlock) void sandwich_rmsnorm_rows_kernel(
   for (int k = 0; k < K; ++k) {
     const int c = k * kBlock + threadIdx.x;
     const bool in = c < C, both = in && branch != nullptr;
-    b[k] = both ? ldf(branch + base + c) : 0.f;
+    if constexpr (!GATHER) b[k] = both ? ldf(branch + base + c) : 0.f;
     x[k] = in ? residual[base + c] : 0.f;
     pw[k] = both ? post_w[c] : 0.f;
     qw[k] = in ? pre_w[c] : 0.f;
+  }
+  if constexpr (GATHER) {
+    constexpr int N = Vec16<T>::N;
+    __shared__ __attribute__((aligned(16))) T row[K * kBlock];
+    const int* own = place + (size_t)blockIdx.x * top;
+    for (int c = threadIdx.x * N; c < C; c += kBlock * N) {
+      float sum[N], v[4][N];
+#pragma unroll
+      for (int j = 0; j < N; ++j) sum[j] = 0.f;
+      for (int e0 = 0; e0 < top; e0 += 4) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)  // (past the last: that again)
+          Vec16<T>::load(branch + (size_t)own[min(e0 + e, top - 1)] * C + c, v[e]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int j = 0; j < N; ++j) sum[j] = e0 + e < top ? sum[j] + v[e][j] : sum[j];
+      }
+      Vec16<T>::store(row + c, sum);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int c = k * kBlock + threadIdx.x;
+      b[k] = c < C ? ldf(row + c) : 0.f;
+    }
   }
   if (branch != nullptr) {
     float sb = 0.f;
@@ -188,9 +221,11 @@ __global__ void sigmoid_gate_kernel(T* __restrict__ out, int64_t out_stride,
 
 }  // namespace
 
+// place int32 [T, top]: the branch's row t is the sum of its rows place[t, :]
 void sandwich_rmsnorm(torch::Tensor out, c10::optional<torch::Tensor> branch,
                       c10::optional<torch::Tensor> post_weight,
-                      torch::Tensor residual, torch::Tensor pre_weight, double eps) {
+                      torch::Tensor residual, torch::Tensor pre_weight, double eps,
+                      c10::optional<torch::Tensor> place) {
   check_f32(residual, "residual");
   check_f32(pre_weight, "pre_weight");
   TORCH_CHECK(residual.dim() == 2 && out.is_contiguous() && out.is_cuda() &&
@@ -203,35 +238,49 @@ void sandwich_rmsnorm(torch::Tensor out, c10::optional<torch::Tensor> branch,
   if (branch.has_value()) {
     check_f32(*post_weight, "post_weight");
     TORCH_CHECK(post_weight->numel() == C);
-    TORCH_CHECK(branch->is_contiguous() && branch->is_cuda() &&
-                branch->sizes() == residual.sizes());
+    TORCH_CHECK(branch->is_contiguous() && branch->is_cuda() && branch->dim() == 2 &&
+                branch->size(1) == C && (place.has_value() || branch->size(0) == T));
     wide = branch->scalar_type() == torch::kFloat32;
     TORCH_CHECK(wide || branch->scalar_type() == out.scalar_type(),
                 "branch must be fp32 or the output's dtype");
+  }
+  const int* places = nullptr;
+  int top = 0;
+  if (place.has_value()) {
+    check_i32(*place, "place");
+    TORCH_CHECK(branch.has_value() && branch->scalar_type() == out.scalar_type() &&
+                place->dim() == 2 && place->size(0) == T && place->size(1) >= 1 &&
+                C <= 16 * kBlock && C * branch->element_size() % 16 == 0 &&
+                ((size_t)branch->data_ptr()) % 16 == 0,
+                "gathered rows: of the output's dtype, whole 16 bytes, up to 4096 columns");
+    places = (const int*)place->data_ptr();
+    top = place->size(1);
   }
   if (T == 0) return;
   const void* bp = branch.has_value() ? branch->data_ptr() : nullptr;
   const float* pw = branch.has_value() ? (const float*)post_weight->data_ptr() : nullptr;
   SEQ_DISPATCH_ACT(out, {
-    auto rows = [&](auto kernel, auto b, size_t lds) {
+    auto rows = [&](auto kernel, auto b, size_t lds, auto... more) {
       hipLaunchKernelGGL(kernel, dim3(T), dim3(kBlock), lds, SEQ_STREAM(),
                          (act_t*)out.data_ptr(), (decltype(b))bp, pw,
                          (float*)residual.data_ptr(),
-                         (const float*)pre_weight.data_ptr(), C, (float)eps);
+                         (const float*)pre_weight.data_ptr(), C, (float)eps, more...);
     };
-    auto go = [&](auto* b) {
+    auto go = [&](auto* b, auto gather) {
       using B = std::remove_const_t<std::remove_pointer_t<decltype(b)>>;
+      constexpr bool G = decltype(gather)::value;
       if (C <= 4 * kBlock)
-        rows(sandwich_rmsnorm_rows_kernel<act_t, B, 4>, (const B*)b, 0);
+        rows(sandwich_rmsnorm_rows_kernel<act_t, B, 4, G>, (const B*)b, 0, places, top);
       else if (C <= 8 * kBlock)
-        rows(sandwich_rmsnorm_rows_kernel<act_t, B, 8>, (const B*)b, 0);
+        rows(sandwich_rmsnorm_rows_kernel<act_t, B, 8, G>, (const B*)b, 0, places, top);
       else if (C <= 16 * kBlock)
-        rows(sandwich_rmsnorm_rows_kernel<act_t, B, 16>, (const B*)b, 0);
+        rows(sandwich_rmsnorm_rows_kernel<act_t, B, 16, G>, (const B*)b, 0, places, top);
       else
         rows(sandwich_rmsnorm_kernel<act_t, B>, (const B*)b, (size_t)C * 4);
     };
-    if (wide) go((const float*)nullptr);
-    else go((const act_t*)nullptr);
+    if (places) go((const act_t*)nullptr, std::true_type{});
+    else if (wide) go((const float*)nullptr, std::false_type{});
+    else go((const act_t*)nullptr, std::false_type{});
   });
   SEQ_CHECK_LAUNCH();
 }

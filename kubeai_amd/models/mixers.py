@@ -709,7 +709,8 @@ class RoutedSquaredReluMoE(nn.Module):
         self.up = Proj(width, n)
         self.down = Proj(n, width)
 
-    def forward(self, h):
+    def forward(self, h, as_sum=False):
+        """as_sum: the caller takes the result as sops.ExpertSum too."""
         T = h.shape[0]
         E, ff = self.experts, self.ff
         logits = F.linear(h.float(), self.router)
@@ -740,6 +741,8 @@ class RoutedSquaredReluMoE(nn.Module):
         if self.shared_ff and not every:
             u = F.linear(h, self.up.weight[E * ff :])
             shared = F.linear(sops.relu_squared(u), self.down.weight[:, E * ff :])
+        if as_sum and shared is None:
+            return sops.ExpertSum(y, rows.place)
         return sops.combine_expert_rows(y, rows.place, shared)
 
 

@@ -22,6 +22,7 @@ import torch.nn.functional as F
 from kubeai_amd.engine.batch import ForwardBatch
 from kubeai_amd.ops import seq as sops
 from .config import HybridLayerSpec, ModelArchConfig
+from .llama import _hooked
 from .mixers import LatentAttention, RoutedSquaredReluMoE, SinkWindowAttention, _f32
 
 
@@ -139,7 +140,9 @@ class NugopelForCausalLM(nn.Module):
             if layer.mlp is not None:
                 h = sops.sandwich_rmsnorm(y, layer.norm1b, residual, layer.norm2,
                                           self.eps, self.dtype)
-                y = layer.mlp(h)
+                # (who waits for the module's call is to see a tensor)
+                own = type(layer.mlp) is RoutedSquaredReluMoE and not _hooked(layer.mlp)
+                y = layer.mlp(h, as_sum=True) if own else layer.mlp(h)
                 h = sops.sandwich_rmsnorm(y, layer.norm2b, residual, nxt,
                                           self.eps, self.dtype)
             else:

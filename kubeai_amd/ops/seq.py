@@ -534,18 +534,34 @@ def qknorm_rope_half_and_cache(q, k, v, q_weight, k_weight, eps: float, position
 # norms around both sides of a sublayer, cached latents, gates
 # ---------------------------------------------------------------------------
 
+class ExpertSum:
+    """combine_expert_rows(y, place), not yet added (sandwich_rmsnorm adds it)."""
+
+    def __init__(self, y, place):
+        self.y, self.place = y, place
+
+
 def sandwich_rmsnorm(branch, post_weight, residual, pre_weight, eps: float,
                      out_dtype):
     """residual (fp32, in place) += branch / rms(branch) * post_weight, then
     returns residual / rms(residual) * pre_weight in ``out_dtype``. rms(x) =
     sqrt(mean(x^2) + eps). Weights are fp32 multipliers (a checkpoint that
     stores them around zero adds the one when it is loaded). branch (serving
-    dtype or fp32) may be None: only the second norm runs."""
+    dtype or fp32) may be None: only the second norm runs; or ExpertSum."""
+    place = None
+    if isinstance(branch, ExpertSum):
+        y, place = branch.y, branch.place
+        # (the kernel that adds the rows has a row in registers)
+        in_one = (
+            y.is_cuda and y.dtype == out_dtype and y.shape[1] <= 4096
+            and y.shape[1] * y.element_size() % 16 == 0 and y.data_ptr() % 16 == 0
+        )
+        branch, place = (y, place) if in_one else (combine_expert_rows(y, place), None)
     if residual.is_cuda:
         _require_ext()
         out = torch.empty(residual.shape, dtype=out_dtype, device=residual.device)
         _C.sandwich_rmsnorm(out, branch, post_weight if branch is not None else None,
-                            residual, pre_weight, eps)
+                            residual, pre_weight, eps, place)
         return out
     if branch is not None:
         b = branch.float()

@@ -44,3 +44,21 @@ def test_mixture_with_a_shared_expert(T, W, E, top, ff, shared):
     # three roundings to bf16 in a row (2^-9 each, at most), of independent signs
     assert (got - want).norm() / want.norm() < 5e-3
     assert ops.have_hip_ext()
+
+
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("T,C,top", [(1, 8, 1), (3, 1000, 2), (70, 1024, 3), (257, 2048, 3),
+                                     (5, 2052, 4), (9, 4096, 5), (4, 4100, 3)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_norms_of_rows_not_yet_added(device, T, C, top, dtype):
+    """The bits of the sum as a launch of its own: rows in registers and longer ones, as
+    many choices as are asked for at a time and more."""
+    g = torch.Generator().manual_seed(C + top)
+    y = torch.randn(T * top, C, generator=g).to(device, dtype)
+    place = torch.randperm(T * top, generator=g).int().view(T, top).to(device)
+    res = torch.randn(T, C, generator=g).to(device)
+    w = [torch.rand(C, generator=g).to(device) + 0.5 for _ in range(2)]
+    one, two = res.clone(), res.clone()
+    want = sops.sandwich_rmsnorm(sops.combine_expert_rows(y, place), w[0], one, w[1], 1e-5, dtype)
+    got = sops.sandwich_rmsnorm(sops.ExpertSum(y, place), w[0], two, w[1], 1e-5, dtype)
+    assert torch.equal(got, want) and torch.equal(one, two)
