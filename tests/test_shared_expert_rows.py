@@ -11,7 +11,7 @@ DEVICES = ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)]
 
 @pytest.mark.parametrize("device", DEVICES)
 @pytest.mark.parametrize("T,E,top", [(1, 1, 1), (7, 3, 2), (257, 8, 2), (1025, 5, 3),
-                                     (2048, 70, 1)])
+                                     (2048, 70, 1), (4096, 8, 2), (4097, 8, 2), (16385, 3, 1)])
 def test_one_more_expert_has_every_token(device, T, E, top):
     """The same rows, places and counts as when each token chooses it itself."""
     g = torch.Generator().manual_seed(T)
