@@ -743,6 +743,7 @@ def few_tiled_better(M: int, N: int, K: int, fp8: bool, rope: bool, sums: bool) 
     )
 
 
+@functools.lru_cache(maxsize=4096)
 def narrow_better(M: int, N: int, K: int, fp8: bool) -> bool:
     """Whether a product of up to 64 rows is best read as the sums of tiles of 64 columns
     (csrc/tiled_gemm.hip: narrow_sums): their workgroups, one a CU at most, leave few CUs
@@ -753,7 +754,7 @@ def narrow_better(M: int, N: int, K: int, fp8: bool) -> bool:
     14.6, 15168 x 12288 78 / 84). Left: bf16 with 192 workgroups (6144 x 4096 40 rows 18.4 /
     19.8), fewer of them (8256 x 9344 44 rows 39 / 54), few steps (fp8 2048 x 2048 8 rows
     7.3 / 8.3)."""
-    if type(M) is not int or not 1 <= M <= 64 or N < 1:  # (a trace has tensors)
+    if not 1 <= M <= 64 or N < 1:
         return False
     tiles, steps = -(-N // 64), K * (1 if fp8 else 2) // 128
     parts = min(8, 256 // tiles) if tiles <= 256 else 0
@@ -783,10 +784,12 @@ def sums_for_reader(x, weight, x_scale=None, w_scale=None, rope=False, eager=Fal
     if M > 96:  # (in a trace sizes are tensors, which no rule is to keep)
         better = type(M) is int and tiled_sums_better(M, N, K, fp8)
         return tiled_sums(x, weight, x_scale, w_scale) if better else None
+    if type(M) is int and narrow_better(M, N, K, fp8):
+        got = tiled_sums(x, weight, x_scale, w_scale)
+        if got is not None:
+            return got
     sums = sums_better(M, N, K, fp8=fp8, rope=rope, eager=eager)
-    if narrow_better(M, N, K, fp8) or (
-        M > 16 and N < 16384 and few_tiled_better(M, N, K, fp8, rope, sums)
-    ):
+    if M > 16 and N < 16384 and few_tiled_better(M, N, K, fp8, rope, sums):
         got = tiled_sums(x, weight, x_scale, w_scale)
         if got is not None:
             return got
