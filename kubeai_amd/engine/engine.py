@@ -16,7 +16,7 @@ from kubeai_amd.models.config import ModelArchConfig, PRESETS
 
 from .kvcache import BlockManager
 from .runner import ModelRunner
-from .scheduler import Request, SamplingParams, Scheduler
+from .scheduler import NO_TOKEN, Request, SamplingParams, Scheduler
 
 
 class RequestError(ValueError):
@@ -222,21 +222,23 @@ class LLMEngine:
             req = ss.req
             if not ss.samples:
                 continue
-            tok = sampled[req.request_id]
+            rid, tok = req.request_id, sampled[req.request_id]
+            got = tok != NO_TOKEN
             results.append(
                 RequestOutput(
-                    request_id=req.request_id,
-                    new_token_ids=[tok],
-                    finished=req.request_id in finished_ids,
+                    request_id=rid,
+                    new_token_ids=[tok] if got else [],
+                    finished=rid in finished_ids,
                     finish_reason=req.status.value if req.status.finished else None,
                     num_prompt_tokens=req.num_prompt_tokens,
                     num_cached_tokens=req.num_cached_prompt_tokens,
                     output_token_ids=req.output_token_ids,
-                    logprob=getattr(self.runner, "last_logprobs", {}).get(
-                        req.request_id
+                    logprob=(
+                        getattr(self.runner, "last_logprobs", {}).get(rid) if got else None
                     ),
-                    top_logprobs=getattr(self.runner, "last_top_logprobs", {}).get(
-                        req.request_id
+                    top_logprobs=(
+                        getattr(self.runner, "last_top_logprobs", {}).get(rid)
+                        if got else None
                     ),
                 )
             )

@@ -19,7 +19,7 @@ from kubeai_amd.models.registry import model_class
 from kubeai_amd.ops.seq import SeqMeta
 
 from .batch import ForwardBatch
-from .scheduler import SchedulerOutput
+from .scheduler import NO_TOKEN, SchedulerOutput
 
 
 _NUMPY = {torch.int32: np.int32, torch.int64: np.int64}
@@ -583,7 +583,7 @@ class ModelRunner:
 
     @torch.inference_mode()
     def execute(self, out: SchedulerOutput, step: int) -> dict[str, int]:
-        """Run one forward + sampling; returns request_id -> sampled token."""
+        """Run one forward + sampling; returns request_id -> sampled token (or NO_TOKEN)."""
         logits = None
         if (
             self.enable_graphs
@@ -693,8 +693,9 @@ class ModelRunner:
             tokens, logprobs = ops.sampled_to_host(block)
         else:
             tokens = tokens.cpu().tolist()
-        if max(tokens) >= V:  # no value of a row compares
-            raise RuntimeError("logits without a number in them")
+        # (the samplers' sign for a row in which no value compares: a token behind the
+        # vocabulary)
+        tokens = [t if t < V else NO_TOKEN for t in tokens]
         if any(r.params.json_mode for r in sample_reqs):
             tokens, logprobs = self._constrain_json(sample_reqs, tokens, logits), None
         want = max((r.params.logprobs for r in sample_reqs), default=0)
@@ -703,6 +704,7 @@ class ModelRunner:
         if logprobs is None:
             # logprob of the chosen token: logit - logsumexp(row)
             tokens_t = torch.tensor(tokens, dtype=torch.int64, device=logits.device)
+            tokens_t.clamp_(min=0)  # (NO_TOKEN)
             chosen = logits.gather(1, tokens_t.view(-1, 1)).squeeze(1)
             logprobs = (chosen - lse).cpu().tolist()
         self.last_logprobs = {
@@ -723,7 +725,7 @@ class ModelRunner:
         # keep persistent penalty counts current with this step's samples
         upd = [
             (r, t) for r, t in zip(sample_reqs, tokens)
-            if (r.params.presence_penalty or r.params.frequency_penalty)
+            if t != NO_TOKEN and (r.params.presence_penalty or r.params.frequency_penalty)
         ]
         if upd:
             for r, t in upd:
@@ -745,7 +747,7 @@ class ModelRunner:
 
         eos = self.arch.eos_token_id
         for i, r in enumerate(sample_reqs):
-            if not r.params.json_mode:
+            if not r.params.json_mode or tokens[i] == NO_TOKEN:
                 continue
             v = self._json_validators.get(r.request_id)
             if v is None:
@@ -889,7 +891,8 @@ def _sample_topk_topp(logits, top_ps, top_ks, temps, t_t, seeds, step,
     c2, ok2 = draw(1)
     c3, ok3 = draw(2)
     tokens = torch.where(ok1, c1, torch.where(ok2, c2, c3))
-    pending = ~(ok1 | ok2 | ok3)
+    # (a row in which no value compares has no token, however it is masked)
+    pending = ~(ok1 | ok2 | ok3) & (c3 < V)
     if cache is not None:
         cache["calls"] = cache.get("calls", 0) + 1
     if bool(pending.any()):

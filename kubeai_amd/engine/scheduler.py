@@ -15,6 +15,10 @@ from typing import Optional
 
 from .kvcache import BlockManager, NoFreeBlocks
 
+#: the sampled token of a row without one: none of its logits compares (they are not
+#: numbers, from a parameter of the request or a weight that is none)
+NO_TOKEN = -1
+
 
 @dataclasses.dataclass
 class SamplingParams:
@@ -382,7 +386,8 @@ class Scheduler:
         """Commit a step: advance counters, append sampled tokens, seal
         full blocks into the prefix cache, finish/free requests.
 
-        `sampled` maps request_id -> token for every seq with samples=True.
+        `sampled` maps request_id -> token for every seq with samples=True
+        (NO_TOKEN: the request ends as aborted, the others go on).
         Returns requests that finished this step.
         """
         if now is None:
@@ -394,6 +399,11 @@ class Scheduler:
             req.num_computed += ss.chunk_len
             if ss.samples:
                 tok = sampled[req.request_id]
+                if tok == NO_TOKEN:
+                    req.status = RequestStatus.FINISHED_ABORTED
+                    req.finish_time = now
+                    finished.append(req)
+                    continue  # (nor are its blocks sealed for others)
                 if req.first_token_time is None:
                     req.first_token_time = now
                 req.tokens.append(tok)

@@ -17,6 +17,7 @@ from __future__ import annotations
 import argparse
 import asyncio
 import json
+import math
 import os
 import queue
 import re
@@ -32,6 +33,9 @@ import prometheus_client as prom
 from .engine import EngineConfig, LLMEngine
 from .scheduler import SamplingParams
 from .tokenizer import StreamDecoder, apply_chat_template, load_tokenizer
+
+#: a penalty beyond it is infinite in the logits' 32 bits, and 0 times it NaN
+F32_MAX = 2.0**128 - 2.0**104
 
 
 class _StopScanner:
@@ -500,23 +504,28 @@ def build_app(server: EngineServer) -> FastAPI:
             return False, None
         raise RequestError(f"unsupported response_format type {rtype!r}")
 
+    def _number(name: str, value, most: float = math.inf) -> float:
+        v = float(value)
+        if not -most <= v <= most:  # (NaN compares with nothing)
+            raise RequestError(f"{name} {v} is out of range")
+        return v
+
     def _params_from(body: dict) -> SamplingParams:
         mt = body.get("max_tokens") or body.get("max_completion_tokens") or 128
         temp = body.get("temperature")
-        temp = 1.0 if temp is None else float(temp)
         seed = body.get("seed")
         jm, schema = _json_mode_from(body)
         return SamplingParams(
             json_mode=jm,
             json_schema=schema,
             max_tokens=int(mt),
-            temperature=float(temp),
-            top_p=float(body.get("top_p") or 1.0),
+            temperature=_number("temperature", 1.0 if temp is None else temp),
+            top_p=_number("top_p", body.get("top_p") or 1.0),
             top_k=int(body.get("top_k") or 0),
             seed=int(seed) if seed is not None else None,
             ignore_eos=bool(body.get("ignore_eos") or False),
-            presence_penalty=float(body.get("presence_penalty") or 0.0),
-            frequency_penalty=float(body.get("frequency_penalty") or 0.0),
+            presence_penalty=_number("presence_penalty", body.get("presence_penalty") or 0.0, F32_MAX),
+            frequency_penalty=_number("frequency_penalty", body.get("frequency_penalty") or 0.0, F32_MAX),
             priority=int(body.get("priority") or 0),
             logit_bias=_logit_bias_from(body),
         )
