@@ -146,7 +146,7 @@ __launch_bounds__(kBlock) __global__ void sample_stage1(
 
 template <bool kLogprob>
 __global__ void sample_stage2(int64_t* __restrict__ out, float* __restrict__ logprob,
-                              const Part* __restrict__ part, const int V) {
+                              const Part* __restrict__ part) {
   const int b = blockIdx.x;
   const int lane = threadIdx.x;
   Part p{-INFINITY, INT32_MAX, -INFINITY, -INFINITY, 0.f};
@@ -174,7 +174,7 @@ void launch_sample(torch::Tensor out, float* logprob, torch::Tensor logits,
                      wide);
   HIP_CHECK_KERNEL();
   hipLaunchKernelGGL((sample_stage2<kLogprob>), dim3(B), dim3(WAVE_SIZE), 0, stream,
-                     out.data_ptr<int64_t>(), logprob, pp, V);
+                     out.data_ptr<int64_t>(), logprob, pp);
   HIP_CHECK_KERNEL();
 }
 
@@ -264,7 +264,12 @@ __global__ void nucleus_accept_kernel(
     return;
   }
   const float* x = logits + (int64_t)row * V;
-  const float lt = x[cand[row]];
+  const int64_t c = cand[row];
+  if (c < 0 || c >= V) {  // (what the sampler gives for a row in which no value compares)
+    if (threadIdx.x == 0) ok[row] = 0;
+    return;
+  }
+  const float lt = x[c];
   const float t = fmaxf(t0, 1e-6f);
   const float m = m_in[row], z = z_in[row];
   __shared__ float red[16];

@@ -1066,6 +1066,8 @@ def _with_scale(quantized, weight, weight_scale):
 
 
 def greedy_sample(logits):
+    """The place of each row's largest value. On GPU a row in which none compares (all
+    NaN) gives V, one behind the last; gumbel_sample and sample_with_logprobs do too."""
     if logits.is_cuda:
         _require_ext()
         out = torch.empty(logits.shape[0], dtype=torch.int64, device=logits.device)
@@ -1143,7 +1145,8 @@ def nucleus_stats(logits, temps):
 def nucleus_accept(logits, cand, m, z, temps, top_ps, top_ks):
     """uint8 mask: sampled token lies in the top-p/top-k nucleus
     (probability mass strictly above it < top_p, rank < top_k);
-    greedy rows always accept."""
+    greedy rows always accept, and on GPU a candidate outside the
+    vocabulary (see greedy_sample) never does in the others."""
     if logits.is_cuda:
         _require_ext()
         ok = torch.empty(logits.shape[0], dtype=torch.uint8,

@@ -105,3 +105,27 @@ def test_numbers_that_are_none_are_refused(client, body):
 def test_what_was_taken_is_taken(client, body):
     r = client.post("/v1/completions", json={"prompt": "a b", "max_tokens": 2, **body})
     assert r.status_code == 200
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V", [1, 1000, 4099])
+def test_candidates_outside_the_vocabulary(V):
+    """None is in the nucleus, and no logit is read for it (the last row's would lie
+    behind them all); the row beside it draws what it draws alone."""
+    from kubeai_amd.engine.runner import _sample_topk_topp
+
+    x = torch.randn(2, V, device="cuda")
+    x[1] = float("nan")
+    temps = torch.ones(2, device="cuda")
+    m, z = ops.nucleus_stats(x, temps)
+    top_p = torch.full((2,), 0.9, device="cuda")
+    top_k = torch.zeros(2, dtype=torch.int32, device="cuda")
+    best = x[0].argmax().item()
+    for none in (V, -1):
+        cand = torch.tensor([best, none], device="cuda")
+        ok = ops.nucleus_accept(x, cand, m, z, temps, top_p, top_k)
+        assert ok.tolist() == [1, 0]
+    seeds = torch.tensor([4, 5], device="cuda")
+    both = _sample_topk_topp(x, [0.9] * 2, [0] * 2, [1.0] * 2, temps, seeds, 3)
+    one = _sample_topk_topp(x[:1], [0.9], [0], [1.0], temps[:1], seeds[:1], 3)
+    assert both.tolist() == [one.item(), V]
