@@ -49,6 +49,9 @@
 // the reloads waited for the loads in flight (the last two 236 us).
 #pragma once
 
+#include <torch/extension.h>
+
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -77,6 +80,20 @@ struct alignas(16) Item {
 struct alignas(8) Splits {
   int first, n;
 };
+
+// Splits that a plan of B rows has room for: what its first candidate may need
+// (attention_decode.hip).
+inline int64_t plan_items(int64_t B, int64_t n_kv) {
+  return 3 * std::max<int64_t>(1, kCUs / n_kv) + B;
+}
+// A plan is int32 [4 plan_items + 2 B], the items in front: its numbers become indices of
+// rows and parts, so one of other rows than these is refused.
+inline void check_plan(const torch::Tensor& plan, int64_t B, int64_t n_kv) {
+  TORCH_CHECK(plan.scalar_type() == torch::kInt32 && plan.is_contiguous() && plan.is_cuda() &&
+                  plan.dim() == 1 && plan.numel() == 4 * plan_items(B, n_kv) + 2 * B &&
+                  ((uintptr_t)plan.data_ptr() & 15) == 0,
+              "a plan of ", B, " rows over ", n_kv, " kv heads");
+}
 
 // Rows that are still sums (common.h: ProductSums, [parts, B, (n_q + 2 n_kv) hd]).
 struct NewRows {

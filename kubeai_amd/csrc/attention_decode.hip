@@ -164,8 +164,7 @@ int paged_decode_splits(int rows, int n_kv, int hd, int max_blocks) {
 }
 
 // The splits of a step's rows, for paged_attention_decode over any caches of this many
-// kv heads, head size, element and window while the lengths are these: int32 [4 items +
-// 2 rows], the items in front.
+// kv heads, head size, element and window while the lengths are these.
 torch::Tensor paged_decode_plan(torch::Tensor seq_lens, int64_t n_kv, int64_t hd,
                                 int64_t element_size, int64_t window) {
   TORCH_CHECK(seq_lens.scalar_type() == torch::kInt32 && seq_lens.is_contiguous() &&
@@ -174,7 +173,7 @@ torch::Tensor paged_decode_plan(torch::Tensor seq_lens, int64_t n_kv, int64_t hd
   TORCH_CHECK(B >= 1 && B <= kPlanRows, "1 to ", kPlanRows, " rows");
   TORCH_CHECK(n_kv >= 1 && (hd == 128 || hd == 256) && (element_size == 1 || element_size == 2));
   const int M = std::max<int64_t>(1, kCUs / n_kv);
-  const int64_t n_items = 3 * M + B;  // (what the first candidate may need)
+  const int64_t n_items = plan_items(B, n_kv);
   auto plan = torch::empty({4 * n_items + 2 * B}, seq_lens.options());
   auto* items = reinterpret_cast<Item*>(plan.data_ptr());
   hipLaunchKernelGGL(decode_plan_kernel, dim3(1), dim3(kPlanThreads), 0,
@@ -214,10 +213,8 @@ static void attend(torch::Tensor out, const ushort* q, int64_t q_stride, const N
   const Splits* row_splits = nullptr;
   int64_t parts = (int64_t)B * n_splits;
   if (plan.has_value()) {
-    TORCH_CHECK(plan->scalar_type() == torch::kInt32 && plan->is_contiguous() &&
-                plan->is_cuda() && plan->dim() == 1 && plan->numel() >= 6 * B &&
-                (plan->numel() - 2 * B) % 4 == 0 && ((uintptr_t)plan->data_ptr() & 15) == 0);
-    parts = (plan->numel() - 2 * B) / 4;
+    check_plan(*plan, B, n_kv);
+    parts = plan_items(B, n_kv);
     items = reinterpret_cast<const Item*>(plan->data_ptr());
     row_splits = reinterpret_cast<const Splits*>(items + parts);
   }

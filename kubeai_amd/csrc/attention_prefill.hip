@@ -1012,8 +1012,7 @@ void paged_attention_step(torch::Tensor out, c10::optional<torch::Tensor> out_sc
               k_cache.size(3) == 128 && v_cache.scalar_type() == k_cache.scalar_type());
   TORCH_CHECK(k_cache.scalar_type() == torch::kBFloat16 ||
               k_cache.scalar_type() == torch::kFloat8_e5m2);
-  for (const auto& t : {decode_tables, decode_lens, plan, prompt_tables, query_start_loc,
-                        prompt_lens})
+  for (const auto& t : {decode_tables, decode_lens, prompt_tables, query_start_loc, prompt_lens})
     TORCH_CHECK(t.scalar_type() == torch::kInt32 && t.is_contiguous() && t.is_cuda());
   const int64_t T = q.size(0), n_q = q.size(1);
   const int n_kv = k_cache.size(1), G = n_q / n_kv, B = prompt_lens.numel();
@@ -1024,15 +1023,14 @@ void paged_attention_step(torch::Tensor out, c10::optional<torch::Tensor> out_sc
               decode_tables.dim() == 2 && decode_tables.size(0) == D &&
               prompt_tables.dim() == 2 && prompt_tables.size(0) == B &&
               query_start_loc.numel() == B + 1);
-  TORCH_CHECK(plan.dim() == 1 && plan.numel() >= 6 * D && (plan.numel() - 2 * D) % 4 == 0 &&
-              ((uintptr_t)plan.data_ptr() & 15) == 0);
+  decode::check_plan(plan, D, n_kv);
   const bool fp8 = out_scale.has_value();
   TORCH_CHECK(out.is_contiguous() && out.is_cuda() && out.numel() == T * n_q * 128 &&
               out.scalar_type() == (fp8 ? torch::kFloat8_e4m3fn : torch::kBFloat16));
   if (fp8)
     TORCH_CHECK(n_q <= 32 && out_scale->is_contiguous() && out_scale->is_cuda() &&
                 out_scale->scalar_type() == torch::kFloat32 && out_scale->numel() == T);
-  const int64_t items = (plan.numel() - 2 * D) / 4;
+  const int64_t items = decode::plan_items(D, n_kv);
   const auto* item = reinterpret_cast<const decode::Item*>(plan.data_ptr());
   const auto* splits = reinterpret_cast<const decode::Splits*>(item + items);
   const auto opts = q.options().dtype(torch::kFloat32);

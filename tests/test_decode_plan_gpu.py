@@ -155,3 +155,26 @@ def test_from_sums(lens, n_q, n_kv, hd, window, cap, parts, scaled, planned):
     assert torch.equal(f8.view(torch.uint8), w8.view(torch.uint8))
     assert torch.equal(scale.view(-1), wscale.view(-1))
     assert torch.equal(one[0], two[0]) and torch.equal(one[1], two[1])
+
+
+@pytest.mark.parametrize("planned_rows", [1, 7, 9, 40])
+def test_plans_of_other_rows_are_refused(planned_rows):
+    """Their numbers would be taken as rows of q and as parts: nothing is launched."""
+    kc, vc, bt, sl = _caches([30] * 40, 8, 128, torch.bfloat16, 0)
+    plan = ops.decode_plan({}, sl[:planned_rows].contiguous(), bt, kc)
+    q = torch.randn(9, 32, 128, device=DEV).bfloat16()
+    caches = (kc, vc, bt[:8].contiguous(), sl[:8].contiguous())
+    own = ops.decode_plan({}, caches[3], bt, kc)
+    prompt = (bt[8:9].contiguous(), torch.tensor([0, 1], dtype=torch.int32, device=DEV),
+              sl[8:9].contiguous())
+    ops.paged_attention_decode(q[:8], *caches, 0.1, plan=own)
+    ops.paged_attention_step(q, 8, *caches, *prompt, 0.1, plan=own)
+    for wrong in (plan, own[:-1], own[:-6], torch.cat([own, own[:6]])):
+        with pytest.raises(RuntimeError, match="a plan of 8 rows"):
+            ops.paged_attention_decode(q[:8], *caches, 0.1, plan=wrong)
+        with pytest.raises(RuntimeError, match="a plan of 8 rows"):
+            ops.paged_attention_step(q, 8, *caches, *prompt, 0.1, plan=wrong)
+    # of other kv heads than the cache's
+    other = ops._C.paged_decode_plan(caches[3], 4, 128, 2, 0)
+    with pytest.raises(RuntimeError, match="over 8 kv heads"):
+        ops.paged_attention_decode(q[:8], *caches, 0.1, plan=other)
