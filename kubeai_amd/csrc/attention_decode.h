@@ -95,6 +95,12 @@ inline void check_plan(const torch::Tensor& plan, int64_t B, int64_t n_kv) {
               "a plan of ", B, " rows over ", n_kv, " kv heads");
 }
 
+// A table with a column at least: the kernel reads an entry before it knows whether the
+// row has a key (rows of no keys are taken without a table too).
+inline torch::Tensor with_a_column(const torch::Tensor& tables) {
+  return tables.size(1) ? tables : torch::zeros({tables.size(0), 1}, tables.options());
+}
+
 // Rows that are still sums (common.h: ProductSums, [parts, B, (n_q + 2 n_kv) hd]).
 struct NewRows {
   ProductSums sums;

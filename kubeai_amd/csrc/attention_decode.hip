@@ -198,6 +198,7 @@ static void attend(torch::Tensor out, const ushort* q, int64_t q_stride, const N
               k_cache.scalar_type() == torch::kFloat8_e5m2);
   TORCH_CHECK(block_tables.scalar_type() == torch::kInt32);
   TORCH_CHECK(seq_lens.scalar_type() == torch::kInt32);
+  block_tables = with_a_column(block_tables);
   const int n_kv = k_cache.size(1);
   const int max_blocks = block_tables.size(1);
   TORCH_CHECK(hd == 128 || hd == 256,

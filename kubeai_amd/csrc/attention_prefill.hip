@@ -1023,6 +1023,7 @@ void paged_attention_step(torch::Tensor out, c10::optional<torch::Tensor> out_sc
               decode_tables.dim() == 2 && decode_tables.size(0) == D &&
               prompt_tables.dim() == 2 && prompt_tables.size(0) == B &&
               query_start_loc.numel() == B + 1);
+  decode_tables = decode::with_a_column(decode_tables);
   decode::check_plan(plan, D, n_kv);
   const bool fp8 = out_scale.has_value();
   TORCH_CHECK(out.is_contiguous() && out.is_cuda() && out.numel() == T * n_q * 128 &&

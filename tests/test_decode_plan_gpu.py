@@ -178,3 +178,22 @@ def test_plans_of_other_rows_are_refused(planned_rows):
     other = ops._C.paged_decode_plan(caches[3], 4, 128, 2, 0)
     with pytest.raises(RuntimeError, match="over 8 kv heads"):
         ops.paged_attention_decode(q[:8], *caches, 0.1, plan=other)
+
+
+@pytest.mark.parametrize("hd", [128, 256])
+@pytest.mark.parametrize("planned", [True, False])
+def test_rows_of_no_keys_need_no_table(planned, hd):
+    """As with a table whose entries do not count: no number, and nothing read for it."""
+    kc, vc, _, _ = _caches([30], 4, hd, torch.bfloat16, 0)
+    sl = torch.zeros(3, dtype=torch.int32, device=DEV)
+    q = torch.randn(4, 8, hd, device=DEV).bfloat16()
+    prompt = (torch.zeros(1, 1, dtype=torch.int32, device=DEV),
+              torch.tensor([0, 1], dtype=torch.int32, device=DEV), sl[:1] + 1)
+    for columns in (1, 0):
+        bt = torch.zeros(3, columns, dtype=torch.int32, device=DEV)
+        plan = ops.decode_plan({}, sl, bt, kc) if planned else None
+        got = ops.paged_attention_decode(q[:3], kc, vc, bt, sl, 0.1, plan=plan)
+        assert got.isnan().all()
+        if planned and hd == 128:
+            got = ops.paged_attention_step(q, 3, kc, vc, bt, sl, *prompt, 0.1, plan=plan)
+            assert got[:3].isnan().all() and not got[3:].isnan().any()
