@@ -747,22 +747,43 @@ def few_tiled_better(M: int, N: int, K: int, fp8: bool, rope: bool, sums: bool) 
 def narrow_better(M: int, N: int, K: int, fp8: bool) -> bool:
     """Whether a product of up to 64 rows is best read as the sums of tiles of 64 columns
     (csrc/tiled_gemm.hip: narrow_sums): their workgroups, one a CU at most, leave few CUs
-    idle, and K is more than a few steps for each. Over 96 products (512 to 16000 columns,
-    K 1024 to 24000) whose sums were the streaming or the wider tiles', with the norm, the
-    chosen ones take 0.91 of the time, 1.07 at worst; over 59 that were the library's 0.72,
-    1.07 at worst (us: fp8 6144 x 4096 40 rows 17.8 / 14.3, bf16 2304 x 9216 1 row 20.5 /
-    14.6, 15168 x 12288 78 / 84). Left: bf16 with 192 workgroups (6144 x 4096 40 rows 18.4 /
-    19.8), fewer of them (8256 x 9344 44 rows 39 / 54), few steps (fp8 2048 x 2048 8 rows
-    7.3 / 8.3)."""
+    idle, and K is more than a few steps for each. Measured against the form that the rules
+    below have without this one, weights out of cache (us, that form / narrow tiles: fp8
+    6144 x 4096 40 rows with the norm 17.8 / 14.3, bf16 2304 x 9216 1 row 20.5 / 14.6). Left:
+    - bf16 with 192 workgroups (6144 x 4096 40 rows 18.4 / 19.8), fewer of them (8256 x 9344
+      44 rows 39 / 54), few steps (fp8 2048 x 2048 8 rows 7.3 / 8.3).
+    - eight parts, which are no fewer than the streaming product's, up to 32 rows (over 175
+      products with either reader 1.04, 1.13 at worst; bf16 2048 x 4096 3 rows 9.3 / 10.3).
+    - one part, of more than 8192 columns, where the library has tuned products (bf16 14336 x
+      8192 1 row 51.5 / 57.3, 16384 x 8192 64 rows 61 / 71), the streaming one is uncut (fp8
+      16384 x 4096 8 rows 21.6 / 23.7) or wider tiles are taken (fp8 12672 x 20480 55 rows
+      1.22, bf16 13312 x 9216 62 rows 1.17).
+    - long K beside more than 48 rows (fp8 7168 x 22528 51 rows 41.1 / 44.2), up to 16 rows
+      bf16 in two parts with tuned library products (6784 x 12288 1 row 37.9 / 41.8) and fp8
+      rows that all begin in one channel (4096 x 16384 1 row 19.4 / 21.7 with the rotation).
+    Over 1400 products (1 to 64 rows, 512 to 16384 columns, K 640 to 24500) the chosen ones
+    take, with the norm, 0.91 of the time of other sums and 0.80 of the library's product,
+    with the rotation 0.93 and 0.81; 6 of 2329 take more than 1.07 (bf16 with the rotation
+    4096 x 8192 2 rows 1.15, 3712 x 22016 5 rows 1.11). Read by decode attention (which
+    reads them once for each of a row's splits) 0.91 over 90 products, 1.06 at worst (fp8 6144
+    x 4096 1 row 18.1 / 19.0)."""
     if not 1 <= M <= 64 or N < 1:
         return False
     tiles, steps = -(-N // 64), K * (1 if fp8 else 2) // 128
     parts = min(8, 256 // tiles) if tiles <= 256 else 0
-    return (
+    if not (
         parts > 0
         and parts * tiles >= (192 if fp8 else 200)
         and steps >= parts * (5 if M > 16 else 7)
-    )
+    ):
+        return False
+    if parts == 8:
+        return M > 32
+    if parts == 1:
+        return K % 4096 != 0 and (M <= 16 or fp8 and K < 8192)
+    if M <= 16:
+        return K % 16384 != 0 if fp8 else parts > 2 or K % 4096 != 0
+    return M <= 48 or K < 15000
 
 
 def tiled_sums(x, weight, x_scale=None, w_scale=None):

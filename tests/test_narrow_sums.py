@@ -12,7 +12,18 @@ from kubeai_amd import ops
     (40, 6144, 4096, True, True), (40, 6144, 4096, False, False),  # 192 workgroups
     (8, 2048, 2048, True, False),                                 # two steps each
     (16, 4096, 2560, True, False), (17, 4096, 2560, True, True),  # five
-    (8, 8256, 8192, False, False), (8, 16384, 4096, True, True), (8, 16448, 4096, True, False),
+    (8, 8256, 8192, False, False), (8, 16384, 4224, True, True), (8, 16448, 4096, True, False),
+    # eight parts
+    (32, 2048, 8192, True, False), (33, 2048, 8192, True, True), (1, 2048, 4096, False, False),
+    (33, 2048, 4096, False, True), (1, 2112, 4608, False, True),
+    # one part
+    (8, 16384, 4096, True, False), (40, 16384, 4096, True, False), (1, 14336, 8192, False, False),
+    (16, 14336, 9088, False, True), (17, 14336, 9088, False, False), (17, 14336, 8064, True, True),
+    (17, 14336, 8320, True, False), (16, 14336, 8320, True, True), (1, 8192, 4224, False, True),
+    # two to seven
+    (16, 8192, 4096, False, False), (17, 8192, 4096, False, True), (1, 4096, 4096, False, True),
+    (16, 4096, 16384, True, False), (17, 4096, 16384, True, True), (49, 7168, 14976, True, True),
+    (49, 7168, 15104, True, False), (48, 7168, 15104, True, True),
 ])
 def test_where_they_are_taken(M, N, K, fp8, better):
     assert ops.narrow_better(M, N, K, fp8) is better
