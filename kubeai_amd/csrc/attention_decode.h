@@ -675,10 +675,11 @@ __global__ void decode_merge_kernel(
 }
 
 // The same, and the row (all heads of a sequence) to fp8 with one scale, as the
-// conversion of the merged bf16 row has it: one workgroup of 16 waves per row,
-// HPW heads a wave, one after the other: a chain of loads each, so only for few of
-// them (ops.decode_fp8_merges). Bound by its launch: 40 rows of 32 x 128 in 2 splits,
-// merge and conversion 9.6 us, this 5.1 (in a profile; beside the attention 1 less).
+// conversion of the merged bf16 row has it: one workgroup of 16 waves per row, HPW heads
+// a wave, where the merge alone has a wave a head: only for few of them
+// (ops.decode_fp8_merges). Bound by its launch, and by its loads where one row has many
+// splits: 40 rows of 32 x 128 in 2 splits, merge and conversion 9.6 us, this 5.1 (in a
+// profile; beside the attention 1 less).
 // Rows from n_split on are no splits but bf16 rows of `whole`, to be converted.
 template <int HD, int HPW>
 __launch_bounds__(16 * WAVE_SIZE) __global__ void decode_merge_fp8_kernel(
@@ -694,20 +695,28 @@ __launch_bounds__(16 * WAVE_SIZE) __global__ void decode_merge_fp8_kernel(
   __shared__ float red[16];
   float vals[HPW][EPL];
   float amax = 0.f;
-  Merged<HD> m[HPW];
   Splits of{0, 1};
   auto merge = [&](auto most) {
     constexpr int MOST = decltype(most)::value;
+    // A wave's heads are asked for together, but two of 256 columns in 16 splits one
+    // behind the other: together they took 128 registers and spilled 18 (with the
+    // attention, us, together / one behind the other: 20 heads 1 row of 3000 20.8 / 16.7, 16
+    // of 2000-4000 55.2 / 51.7; 32 heads 4 rows of 3000 32.5 / 29.7).
+    constexpr int AHEAD = HD == 256 && MOST > 4 ? 1 : HPW;
+    Merged<HD> m[AHEAD];
 #pragma unroll
-    for (int h = 0; h < HPW; ++h)  // (past the last head: that again)
-      m[h].template load<MOST>(part_o, part_ml, of, n_q, min(h * 16 + wave, n_q - 1));
+    for (int h0 = 0; h0 < HPW; h0 += AHEAD) {
 #pragma unroll
-    for (int h = 0; h < HPW; ++h) {
-      m[h].template finish<MOST>();
+      for (int h = 0; h < AHEAD; ++h)  // (past the last head: that again)
+        m[h].template load<MOST>(part_o, part_ml, of, n_q, min((h0 + h) * 16 + wave, n_q - 1));
 #pragma unroll
-      for (int e = 0; e < EPL; ++e) {
-        vals[h][e] = bf16_to_f32(m[h].v[e]);
-        amax = fmaxf(amax, fabsf(vals[h][e]));
+      for (int h = 0; h < AHEAD; ++h) {
+        m[h].template finish<MOST>();
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) {
+          vals[h0 + h][e] = bf16_to_f32(m[h].v[e]);
+          amax = fmaxf(amax, fabsf(vals[h0 + h][e]));
+        }
       }
     }
   };

@@ -197,3 +197,19 @@ def test_rows_of_no_keys_need_no_table(planned, hd):
         if planned and hd == 128:
             got = ops.paged_attention_step(q, 3, kc, vc, bt, sl, *prompt, 0.1, plan=plan)
             assert got[:3].isnan().all() and not got[3:].isnan().any()
+
+
+@pytest.mark.parametrize("n_q,n_kv", [(16, 4), (20, 4), (32, 8)])
+@pytest.mark.parametrize("lens", [LENGTHS[k] for k in ("one long", "one of many", "edges")],
+                         ids=["one long", "one of many", "edges"])
+def test_heads_of_256_to_eight_bits(lens, n_q, n_kv):
+    """One wave merges one head, or two of which the second may not be there, in up to 16
+    splits: the bits of the merge and the conversion after one another."""
+    kc, vc, bt, sl = _caches(lens, n_kv, 256, torch.bfloat16, n_q)
+    q = torch.randn(len(lens), n_q, 256, device=DEV).bfloat16()
+    plan = ops.decode_plan({}, sl, bt, kc)
+    want = ops.paged_attention_decode(q, kc, vc, bt, sl, 0.06, plan=plan)
+    f8, scale = ops.paged_attention_decode_fp8(q, kc, vc, bt, sl, 0.06, plan=plan)
+    w8, wscale = ops.quant_fp8(want.view(len(lens), -1))
+    assert torch.equal(f8.view(torch.uint8), w8.view(torch.uint8))
+    assert torch.equal(scale, wscale.view(-1))
