@@ -179,7 +179,8 @@ class Attention(nn.Module):
             cos_sin = cos_sin[0] if self.is_global else cos_sin[1]
         nd = fb.n_decode
         plan = ops.decode_plan(
-            fb.decode_plans, fb.decode_seq_lens, fb.decode_block_tables, k_cache, self.window
+            fb.decode_plans, fb.decode_seq_lens, fb.decode_block_tables, k_cache, self.window,
+            alone=fb.n_prefill == 0,
         ) if nd > 0 else None
         if nd == T and fb.n_prefill == 0 and ops.decode_takes_sums(
             qkv, self.n_q, cos_sin, k_cache, v_cache

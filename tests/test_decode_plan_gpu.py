@@ -213,3 +213,20 @@ def test_heads_of_256_to_eight_bits(lens, n_q, n_kv):
     w8, wscale = ops.quant_fp8(want.view(len(lens), -1))
     assert torch.equal(f8.view(torch.uint8), w8.view(torch.uint8))
     assert torch.equal(scale, wscale.view(-1))
+
+
+@pytest.mark.parametrize("rows,columns,n_kv,window,alone,planned", [
+    (8, 8, 8, 0, True, True),      # split without a plan too
+    (64, 8, 8, 0, True, False), (64, 9, 8, 0, True, True), (64, 8, 8, 0, False, True),
+    (1, 1, 8, 0, True, False), (1, 2, 8, 0, True, False), (1, 512, 8, 0, True, True),
+    (64, 512, 8, 128, True, False), (64, 512, 8, 129, True, True),
+    (256, 9, 1, 0, True, True), (257, 512, 1, 0, True, False), (257, 512, 1, 0, False, True),
+    (512, 512, 8, 0, False, True), (513, 512, 8, 0, False, False),
+])
+def test_where_rows_are_planned(rows, columns, n_kv, window, alone, planned):
+    cache = torch.empty(1, n_kv, BS, 128, dtype=torch.bfloat16, device=DEV)
+    sl = torch.ones(rows, dtype=torch.int32, device=DEV)
+    bt = torch.zeros(rows, columns, dtype=torch.int32, device=DEV)
+    plan = ops.decode_plan({}, sl, bt, cache, window, alone=alone)
+    assert (plan is not None) is planned
+    assert ops.decode_plan(None, sl, bt, cache, window, alone=alone) is None
