@@ -13,9 +13,11 @@
 // With log-probabilities the same pass has the sum of exp(x - max) as well: a thread
 // holds 16 values at a time, their maximum moves its sum once, so a value costs one
 // exponential. Bound by reading the logits once and by two launches: 40 rows of 128256
-// 11.6 us (tokens alone 7.4; torch's logsumexp, gather and difference behind that
-// 72), one row 7.6 (5.7 and 49), 96 rows 22.5 (15.2 and 89).
+// 11.6 us (the greedy tokens alone 7.4; torch's logsumexp, gather and difference behind
+// that 72), one row 7.6 (5.7 and 49), 96 rows 22.5 (15.2 and 89).
 #include <torch/extension.h>
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -25,45 +27,61 @@ constexpr int kBlock = 256;
 constexpr int kSplits = 32;
 constexpr int kUnits = 4;  // of 4 values, a thread at a time
 
-// a chunk's best value (with its noise) and where, that place's logit, and with
-// log-probabilities the largest logit and the sum of exp(logit - it)
+// a chunk's best value (with its noise) and where, and with log-probabilities that
+// place's logit, the largest logit and the sum of exp(logit - it)
+template <bool kLogprob>
 struct Part {
+  float best;
+  int32_t idx;
+};
+template <>
+struct Part<true> {
   float best;
   int32_t idx;
   float raw, m, z;
 };
+template <bool kLogprob>
+DEV_INLINE Part<kLogprob> none(int32_t idx) {
+  if constexpr (kLogprob) return {-INFINITY, idx, -INFINITY, -INFINITY, 0.f};
+  else return {-INFINITY, idx};
+}
 
-DEV_INLINE void keep_best(Part& p, float v, int32_t i, float raw) {
+template <bool kLogprob>
+DEV_INLINE void keep_best(Part<kLogprob>& p, float v, int32_t i, float raw) {
   if (v > p.best || (v == p.best && i < p.idx)) {
     p.best = v;
     p.idx = i;
-    p.raw = raw;
+    if constexpr (kLogprob) p.raw = raw;
   }
 }
 // (a maximum of -inf has only zeros behind it)
 DEV_INLINE float finite_or_0(float m) { return m == -INFINITY ? 0.f : m; }
-DEV_INLINE void keep_sum(Part& p, float m, float z) {
+DEV_INLINE void keep_sum(Part<true>& p, float m, float z) {
   const float most = fmaxf(p.m, m), use = finite_or_0(most);
   p.z = p.z * expf(p.m - use) + z * expf(m - use);
   p.m = most;
 }
 template <bool kLogprob>
-DEV_INLINE void over_lanes(Part& p) {
+DEV_INLINE void over_lanes(Part<kLogprob>& p) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
-    const float v = __shfl_xor(p.best, off), raw = __shfl_xor(p.raw, off);
+    const float v = __shfl_xor(p.best, off);
     const int32_t i = __shfl_xor(p.idx, off);
-    keep_best(p, v, i, raw);
     if constexpr (kLogprob) {
-      const float m = __shfl_xor(p.m, off), z = __shfl_xor(p.z, off);
+      const float raw = __shfl_xor(p.raw, off), m = __shfl_xor(p.m, off),
+                  z = __shfl_xor(p.z, off);
+      keep_best(p, v, i, raw);
       keep_sum(p, m, z);
+    } else {
+      keep_best(p, v, i, 0.f);
     }
   }
 }
 
-template <bool kGumbel, bool kLogprob>
+// kMany: a thread takes 16 values at a time, else one
+template <bool kGumbel, bool kLogprob, bool kMany>
 __launch_bounds__(kBlock) __global__ void sample_stage1(
-    Part* __restrict__ part,               // [B, kSplits]
+    Part<kLogprob>* __restrict__ part,     // [B, kSplits]
     const float* __restrict__ logits,      // [B, V]
     const float* __restrict__ temperature,  // [B]
     const int64_t* __restrict__ seeds,      // [B]
@@ -83,8 +101,19 @@ __launch_bounds__(kBlock) __global__ void sample_stage1(
     key = (uint64_t)seeds[b] * 1000003ull + (uint64_t)step;
   }
 
-  Part p{-INFINITY, V, -INFINITY, -INFINITY, 0.f};
-  for (int base = lo; base < hi; base += kBlock * 4 * kUnits) {
+  auto noisy = [&](float val, int v) {
+    if (!greedy) {
+      const float u = hash_uniform(key, (uint64_t)v);
+      val = val / temp + (-__logf(-__logf(u)));
+    }
+    return val;
+  };
+  static_assert(kMany || !kLogprob);
+  Part<kLogprob> p = none<kLogprob>(V);
+  if constexpr (!kMany) {
+    for (int v = lo + threadIdx.x; v < hi; v += kBlock) keep_best(p, noisy(row[v], v), v, 0.f);
+  }
+  for (int base = lo; kMany && base < hi; base += kBlock * 4 * kUnits) {
     float4_t x[kUnits];
 #pragma unroll
     for (int j = 0; j < kUnits; ++j) {
@@ -104,14 +133,7 @@ __launch_bounds__(kBlock) __global__ void sample_stage1(
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const int v = base + (j * kBlock + threadIdx.x) * 4 + k;
-        float val = x[j][k];
-        if (v < hi) {
-          if (!greedy) {
-            const float u = hash_uniform(key, (uint64_t)v);
-            val = val / temp + (-__logf(-__logf(u)));
-          }
-          keep_best(p, val, v, x[j][k]);
-        }
+        if (v < hi) keep_best(p, noisy(x[j][k], v), v, x[j][k]);
         if constexpr (kLogprob) most = fmaxf(most, x[j][k]);
       }
     }
@@ -129,16 +151,20 @@ __launch_bounds__(kBlock) __global__ void sample_stage1(
     }
   }
   over_lanes<kLogprob>(p);
-  __shared__ Part waves[kBlock / WAVE_SIZE];
+  __shared__ Part<kLogprob> waves[kBlock / WAVE_SIZE];
   const int wave = threadIdx.x / WAVE_SIZE;
   if (threadIdx.x % WAVE_SIZE == 0) waves[wave] = p;
   __syncthreads();
   if (threadIdx.x == 0) {
 #pragma unroll
     for (int w = 1; w < kBlock / WAVE_SIZE; ++w) {
-      const Part o = waves[w];
-      keep_best(p, o.best, o.idx, o.raw);
-      if constexpr (kLogprob) keep_sum(p, o.m, o.z);
+      const Part<kLogprob> o = waves[w];
+      if constexpr (kLogprob) {
+        keep_best(p, o.best, o.idx, o.raw);
+        keep_sum(p, o.m, o.z);
+      } else {
+        keep_best(p, o.best, o.idx, 0.f);
+      }
     }
     part[b * kSplits + split] = p;
   }
@@ -146,10 +172,10 @@ __launch_bounds__(kBlock) __global__ void sample_stage1(
 
 template <bool kLogprob>
 __global__ void sample_stage2(int64_t* __restrict__ out, float* __restrict__ logprob,
-                              const Part* __restrict__ part) {
+                              const Part<kLogprob>* __restrict__ part) {
   const int b = blockIdx.x;
   const int lane = threadIdx.x;
-  Part p{-INFINITY, INT32_MAX, -INFINITY, -INFINITY, 0.f};
+  Part<kLogprob> p = none<kLogprob>(INT32_MAX);
   if (lane < kSplits) p = part[b * kSplits + lane];
   over_lanes<kLogprob>(p);
   if (lane == 0) {
@@ -164,14 +190,24 @@ void launch_sample(torch::Tensor out, float* logprob, torch::Tensor logits,
                    int64_t step) {
   const int B = logits.size(0), V = logits.size(1);
   if (B == 0) return;
-  auto part = torch::empty({B, kSplits, (int64_t)sizeof(Part)},
+  auto part = torch::empty({B, kSplits, (int64_t)sizeof(Part<kLogprob>)},
                            torch::TensorOptions().device(logits.device()).dtype(torch::kUInt8));
-  auto* pp = reinterpret_cast<Part*>(part.data_ptr());
+  auto* pp = reinterpret_cast<Part<kLogprob>*>(part.data_ptr());
   const bool wide = V % 4 == 0 && ((uintptr_t)logits.data_ptr() & 15) == 0;
   auto stream = c10::hip::getCurrentHIPStream().stream();
-  hipLaunchKernelGGL((sample_stage1<kGumbel, kLogprob>), dim3(B, kSplits), dim3(kBlock),
-                     0, stream, pp, logits.data_ptr<float>(), temp_ptr, seed_ptr, step, V,
-                     wide);
+  auto stage1 = [&](auto many) {
+    hipLaunchKernelGGL((sample_stage1<kGumbel, kLogprob, decltype(many)::value>),
+                       dim3(B, kSplits), dim3(kBlock), 0, stream, pp, logits.data_ptr<float>(),
+                       temp_ptr, seed_ptr, step, V, wide);
+  };
+  // Tokens alone take a value at a time: the noise hides the loads, and a chunk of a small
+  // vocabulary has no 16 values for each thread (us, at a time one / 16: 278 rows of 3954
+  // greedy 11.2 / 17.2, noise 12.5 / 20.9; 144 of 27950 11.4 / 11.9, 14.4 / 16.7; 109 of 77195
+  // 14.5 / 14.2, 22.3 / 24.6; 198 of 91860 31.4 / 21.4, 41.3 / 41.5; 22 of 188508 14.0 / 9.8,
+  // 17.8 / 17.1).
+  if constexpr (kLogprob) stage1(std::true_type{});
+  else if (!kGumbel && V >= 65536) stage1(std::true_type{});
+  else stage1(std::false_type{});
   HIP_CHECK_KERNEL();
   hipLaunchKernelGGL((sample_stage2<kLogprob>), dim3(B), dim3(WAVE_SIZE), 0, stream,
                      out.data_ptr<int64_t>(), logprob, pp);

@@ -70,3 +70,18 @@ def test_fill_rows():
     for rows in ([[1] * 5], [[1]] * 4):
         with pytest.raises((RuntimeError, IndexError)):
             ops.fill_rows(out, rows)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,V", [(1, 1), (3, 33), (70, 8192), (5, 65535), (5, 65536), (2, 65539)])
+def test_tokens_alone(S, V):
+    """One value at a time and 16 give the tokens of the pass with log-probabilities, the
+    first of equal ones too."""
+    x = _logits(S, V, "cuda")
+    x[:, V // 2 :] = x[:, : V - V // 2]  # every value twice
+    assert ops.greedy_sample(x).tolist() == x.argmax(-1).tolist()
+    assert ops.greedy_sample(x).tolist() == ops.sampled_to_host(ops.sample_with_logprobs(x))[0]
+    temps = torch.rand(S, device="cuda") + 0.2
+    seeds = torch.arange(S, device="cuda")
+    want = ops.sampled_to_host(ops.sample_with_logprobs(x, temps, seeds, 5))[0]
+    assert ops.gumbel_sample(x, temps, seeds, 5).tolist() == want
