@@ -142,35 +142,35 @@ constexpr int kSB = 1024;  // threads of a sorting block
 // number of pairs of lower experts; a pair's rank is the number of earlier
 // pairs of the same expert (block-wide prefix sums over slices of the list).
 // A chain of latencies: S slices are loaded and counted between two barriers. us, one
-// slice at a time / eight, tokens of two choices among 8 experts: 300 3.3 / 4.4, 1024
-// 4.3 / 4.7, 3072 8.0 / 5.7, 8192 17.5 / 10.2; so eight from more than two slices on.
-// every: one more block and expert E, which all tokens use with weight 1, in order.
+// slice at a time / eight, tokens of two choices among 8 experts: 300 3.0 / 4.4, 1024
+// 4.1 / 4.7, 3072 7.8 / 5.4, 8192 17.5 / 10.2; so eight from more than two slices on.
+// last: one more expert and its block, which all tokens use with weight 1, in order; or -1.
 template <int S>
 __global__ __launch_bounds__(kSB) void expert_order_kernel(
     const int* __restrict__ index, const float* __restrict__ weights,
     int* __restrict__ tok, float* __restrict__ wrow, int* __restrict__ place,
-    int* __restrict__ counts, int N, int top, int every) {
+    int* __restrict__ counts, int N, int top, int last) {
   constexpr int NW = kSB / WAVE, NP = S * NW;
   static_assert(S == 1 || NP == 2 * WAVE);
   __shared__ int part[NP + 1], total_s;
-  const int e = blockIdx.x, places = top + every;  // of a token
-  if (every && e == (int)gridDim.x - 1) {
+  const int e = blockIdx.x;
+  if (e == last) {
     for (int t = threadIdx.x; t < N / top; t += kSB) {
       tok[N + t] = t;
       wrow[N + t] = 1.f;
-      place[t * places + top] = N + t;
+      place[t * (top + 1) + top] = N + t;
     }
     if (threadIdx.x == 0) counts[e] = N / top;
     return;  // the whole block
   }
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  int mine[S];  // the thread's entries of the batch, -1 past the end
+  int mine[S];  // the thread's entries of the batch, past the end none's
   auto load = [&](int i0) {
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       const int i = i0 + s * kSB + threadIdx.x;
       const int v = index[min(i, N - 1)];
-      mine[s] = i < N ? v : -1;
+      mine[s] = i < N ? v : INT32_MAX;
     }
   };
   constexpr int kBatch = S * kSB;
@@ -178,17 +178,16 @@ __global__ __launch_bounds__(kSB) void expert_order_kernel(
   for (int i0 = 0; i0 < N; i0 += kBatch) {
     load(i0);
 #pragma unroll
-    for (int s = 0; s < S; ++s) below += mine[s] >= 0 && mine[s] < e ? 1 : 0;
+    for (int s = 0; s < S; ++s) below += mine[s] < e ? 1 : 0;
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) below += __shfl_xor(below, off, WAVE);
   if (lane == 0) part[wave] = below;
   __syncthreads();
-  if (wave == 0) {
-    int s = lane < NW ? part[lane] : 0;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, WAVE);
-    if (lane == 0) total_s = s;
+  if (threadIdx.x == 0) {
+    int s = 0;
+    for (int w = 0; w < NW; ++w) s += part[w];
+    total_s = s;
   }
   __syncthreads();
   const int first = total_s;
@@ -231,9 +230,10 @@ __global__ __launch_bounds__(kSB) void expert_order_kernel(
       if (mine[s] != e) continue;
       const int i = i0 + s * kSB + threadIdx.x;
       const int p = at + (S > 1 ? part[s * NW + wave] : before) + __popcll(b[s] & ((1ull << lane) - 1));
-      tok[p] = i / top;
+      const int t = i / top;
+      tok[p] = t;
       wrow[p] = weights[i];
-      place[i / top * places + i % top] = p;
+      place[last < 0 ? i : i + t] = p;
     }
     at += all;
   }
@@ -344,7 +344,8 @@ void expert_order(torch::Tensor index, torch::Tensor weights, torch::Tensor tok,
   hipLaunchKernelGGL(kernel, dim3(counts.numel()), dim3(kSB), 0, SEQ_STREAM(),
                      (const int*)index.data_ptr(), (const float*)weights.data_ptr(),
                      (int*)tok.data_ptr(), (float*)wrow.data_ptr(), (int*)place.data_ptr(),
-                     (int*)counts.data_ptr(), (int)N, (int)index.size(1), rows != N);
+                     (int*)counts.data_ptr(), (int)N, (int)index.size(1),
+                     rows == N ? -1 : (int)counts.numel() - 1);
   SEQ_CHECK_LAUNCH();
 }
 
