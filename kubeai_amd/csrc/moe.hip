@@ -3,11 +3,11 @@
 // weighted sum of what the experts returned. All of it on the device, with
 // shapes that do not depend on the routing, so that a step can be recorded.
 //
-//  - moe_route: workgroup = token; a wave per expert (up to 16, then in turn), eight
-//    loads of either row on their way at a time, the products of
-//    the bf16 hidden row and router rows summed in fp32 (with
-//    the order, us, four waves and loads / these: 40 x 4096 8 experts 9.2 / 8.1, 32 experts 21.7
-//    / 14.0, 40 x 2048 16 experts 11.6 / 9.5); the largest top_k
+//  - moe_route: workgroup = token; a wave per expert (up to 16, then in turn), the products
+//    of the bf16 hidden row and router rows summed in fp32. A chain of loads: the kernel
+//    has 40 registers, and a unit of either row is waited for before the next ones'
+//    products (with the order, us, four waves / a wave an expert: 40 x 4096 8 experts 9.1 / 7.9,
+//    32 experts 21.2 / 13.4, 40 x 2048 16 experts 10.7 / 8.6); the largest top_k
 //    (ties: the lower expert) and the softmax over them in fp32. NaN is the
 //    largest score, and infinite scores make the weights NaN, as in the library
 //    calls that this stands for: a token whose scores are not finite shows it.
@@ -33,7 +33,6 @@ constexpr int kMaxTop = 8;
 constexpr int kOrderThreads = 256;
 constexpr int kMostRouteWaves = 16;
 
-template <int AHEAD>
 __launch_bounds__(kMostRouteWaves * WAVE_SIZE) __global__ void moe_route_kernel(
     int32_t* __restrict__ index,   // [T, top]
     float* __restrict__ weight,    // [T, top]
@@ -47,7 +46,7 @@ __launch_bounds__(kMostRouteWaves * WAVE_SIZE) __global__ void moe_route_kernel(
   for (int e = wave; e < E; e += blockDim.x / WAVE_SIZE) {
     const ushort8* wr = reinterpret_cast<const ushort8*>(w + (int64_t)e * H);
     float acc = 0.f;
-#pragma unroll AHEAD
+#pragma unroll 4
     for (int i = lane; i < H / 8; i += WAVE_SIZE) {
       const ushort8 a = xr[i], b = wr[i];
 #pragma unroll
@@ -200,12 +199,10 @@ void moe_route(torch::Tensor index, torch::Tensor weight, torch::Tensor begin,
               weight.is_cuda() && weight.numel() == n && n < (1ll << 30));
   if (T == 0) return;
   auto stream = c10::hip::getCurrentHIPStream().stream();
-  // many tokens fill the chip with four waves each and four loads ahead (2048 22.5 us;
-  // eight of either 23.6, of the loads alone 23.3)
-  const bool many = T > 1024;
-  const int waves = many ? 4 : std::min(kMostRouteWaves, std::max(4, E));
-  const auto route = many ? moe_route_kernel<4> : moe_route_kernel<8>;
-  hipLaunchKernelGGL(route, dim3((uint32_t)T), dim3(waves * WAVE_SIZE), 0, stream,
+  // more tokens than two a CU fill the chip with four waves each (us, 16 / 4 waves: 20
+  // experts of 4096 500 tokens 15.0 / 17.0, 600 19.2 / 17.6; 16 of 1024 800 13.6 / 12.2)
+  const int waves = T > 512 ? 4 : std::min(kMostRouteWaves, std::max(4, E));
+  hipLaunchKernelGGL(moe_route_kernel, dim3((uint32_t)T), dim3(waves * WAVE_SIZE), 0, stream,
                      index.data_ptr<int32_t>(), weight.data_ptr<float>(),
                      (const ushort*)x.data_ptr(), (const ushort*)w.data_ptr(),
                      H, E, top);
