@@ -722,10 +722,12 @@ class RoutedSquaredReluMoE(nn.Module):
         # fill the launches' last passes over the CUs, and two library products and the
         # squared ReLU between them are gone. The layer, us, apart / together: 8 experts of
         # 3584 x 2048, 260 tokens 132 / 112, 700 156 / 130, 2048 261 / 219, 4400 456 / 448;
-        # of 1792 x 1024, 260 71 / 51, 3072 154 / 125; 16 of 1408 x 2048, 4 a token, 1000
-        # 152 / 129. Not where each of the two fills the chip several times by itself:
-        # of 7168 x 4096, 260 302 / 279, 1500 638 / 566, but 3072 1077 / 1076, 4400 1415 / 1462
-        every = self.shared_ff == ff and T * ff <= self.TOGETHER_MAX
+        # of 1792 x 1024, 260 71 / 51, 3072 154 / 125. Not where each of the two fills the chip
+        # several times by itself: of 7168 x 4096, 260 302 / 279, 1500 638 / 566, but 3072 1077 / 1076, 4400 1415 / 1462.
+        # Nor beside 16 experts and more, whose tiles may fill their passes to the last: 0.86
+        # of the time over 260 layers, but 14 of them up to 1.12 (16 of 1792 x 1792, 3 a token,
+        # 803 123 / 138; 32 of 3584 x 3584 2584 551 / 606); over 200 of fewer 0.81, 1.03 at most.
+        every = self.shared_ff == ff and E < 16 and T * ff <= self.TOGETHER_MAX
         n = E + every
         up = self.up.weight[: n * ff].unflatten(0, (n, ff))
         down = self.down.weight[:, : n * ff].unflatten(1, (n, ff)).transpose(0, 1)

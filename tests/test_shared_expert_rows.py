@@ -62,3 +62,20 @@ def test_norms_of_rows_not_yet_added(device, T, C, top, dtype):
     want = sops.sandwich_rmsnorm(sops.combine_expert_rows(y, place), w[0], one, w[1], 1e-5, dtype)
     got = sops.sandwich_rmsnorm(sops.ExpertSum(y, place), w[0], two, w[1], 1e-5, dtype)
     assert torch.equal(got, want) and torch.equal(one, two)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,shared,together", [(15, 128, True), (16, 128, False), (4, 64, False)])
+def test_where_the_shared_expert_is_among_the_others(monkeypatch, E, shared, together):
+    seen, real = [], sops.expert_order
+
+    def order(index, weights, experts, every=False):
+        seen.append(every)
+        return real(index, weights, experts, every)
+
+    monkeypatch.setattr(sops, "expert_order", order)
+    moe = RoutedSquaredReluMoE(256, E, 2, 128, shared).to("cuda", torch.bfloat16)
+    moe.router.data = moe.router.data.float()
+    with torch.no_grad():
+        moe(torch.randn(300, 256, device="cuda").bfloat16())
+    assert seen == [together]
