@@ -137,8 +137,10 @@ def decode_plan(plans, seq_lens, block_tables, k_cache, window: int = 0, alone: 
     planned rows saves 5 us a layer and more) not for more than 256, nor where all see at
     most 128 keys and would not be split without a plan: the merge's launch is what a
     plan adds then (us, unplanned / planned: 76 rows of 11-22 4.3 / 5.8, 118 of 26-36 7.7 /
-    10.1, 183 of 16-81 14.8 / 18.6; of 9 to 16 blocks as fast; over 490 other batches of up to
-    400 rows planned ones take 0.79 of the time of the same number of splits each)."""
+    10.1, 183 of 16-81 14.8 / 18.6; of 9 to 16 blocks as fast), or are few, where a plan's
+    splits of eight tiles are too long (12 rows of 76-90 keys of one head of 256 8.4 / 9.5).
+    Over 450 other batches of up to 400 rows planned ones take 0.78 of the time of the same
+    number of splits each."""
     B, cols = seq_lens.shape[0], block_tables.shape[1]
     if plans is None or not seq_lens.is_cuda or not 1 <= B <= (256 if alone else 512):
         return None
@@ -147,7 +149,8 @@ def decode_plan(plans, seq_lens, block_tables, k_cache, window: int = 0, alone: 
         window = 0  # no row is longer
     if alone and min(cols * bs, window or cols * bs) <= 128:
         _require_ext()
-        if _C.paged_decode_splits(B, n_kv, hd, cols) == 1:
+        few = cols * bs <= 128 and B * n_kv <= 64
+        if few or _C.paged_decode_splits(B, n_kv, hd, cols) == 1:
             return None
     key = (n_kv, hd, k_cache.element_size(), window)
     if key not in plans:

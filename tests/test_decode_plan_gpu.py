@@ -216,7 +216,7 @@ def test_heads_of_256_to_eight_bits(lens, n_q, n_kv):
 
 
 @pytest.mark.parametrize("rows,columns,n_kv,window,alone,planned", [
-    (8, 8, 8, 0, True, True),      # split without a plan too
+    (8, 8, 8, 0, True, False), (8, 9, 8, 0, True, True), (9, 8, 8, 0, True, True),
     (64, 8, 8, 0, True, False), (64, 9, 8, 0, True, True), (64, 8, 8, 0, False, True),
     (1, 1, 8, 0, True, False), (1, 2, 8, 0, True, False), (1, 512, 8, 0, True, True),
     (64, 512, 8, 128, True, False), (64, 512, 8, 129, True, True),
