@@ -158,12 +158,12 @@ DEV_INLINE float over_groups(float v, F&& f) {
 // LDS for that tile. us with the merge, rotation as a
 // launch before / here: 40 rows of 100-700, sums in 4 parts, to fp8 25.0 / 22.2, bf16 23.5 /
 // 21.0; 8 rows, sums in 8 parts 18.2 / 14.8, 14.9 / 11.6.
-template <int HD, typename CT, int NEW>
+template <int HD, typename CT, int NEW, int NB = blocks_per_tile(HD, sizeof(CT))>
 struct alignas(16) Lds {
   // Head size 256 over a bf16 cache: two tiles of K and V and the sums leave no
   // registers for the query; it lies in LDS, 16-byte units XORed with the head.
   static constexpr bool kQuery = HD == 256 && sizeof(CT) == 2;
-  static constexpr int kVTile = blocks_per_tile(HD, sizeof(CT)) * kBS * HD;  // elements a wave
+  static constexpr int kVTile = NB * kBS * HD;  // elements a wave
   static constexpr size_t kTiles = sizeof(ushort) * kWaves * kVTile >
                                            sizeof(float) * kWaves * kMaxG * HD
                                        ? sizeof(ushort) * kWaves * kVTile
@@ -174,9 +174,10 @@ struct alignas(16) Lds {
   float merge_ml[kWaves][kMaxG][2];
 };
 
-template <int HD, typename CT, bool CAP, bool ONE, int NEW>
+template <int HD, typename CT, bool CAP, bool ONE, int NEW,
+          int NB = blocks_per_tile(HD, sizeof(CT))>
 DEV_INLINE void attend_split(
-    Lds<HD, CT, NEW>& mem, const int block,
+    Lds<HD, CT, NEW, NB>& mem, const int block,
     ushort* __restrict__ out,            // [B, n_q, hd] bf16, or null: parts of all rows
     const ushort* __restrict__ q,        // [B, n_q, hd] bf16
     CT* k_cache,                         // [nb, n_kv, bs, hd]
@@ -190,7 +191,6 @@ DEV_INLINE void attend_split(
     const NewRows fresh,
     float* __restrict__ part_o,    // [splits of all rows, n_q, hd]
     float* __restrict__ part_ml) { // [splits of all rows, n_q, 2]
-  constexpr int NB = blocks_per_tile(HD, sizeof(CT));
   constexpr int NC = HD / 32;            // contraction steps of S
   constexpr int ND = HD / 16;            // row blocks of O^T
   constexpr int NV = HD / 32;            // 16-byte V units per lane and block
@@ -226,8 +226,8 @@ DEV_INLINE void attend_split(
   // the waves of all splits take tiles in turn
   const int turn = kWaves * n_splits;
 
-  constexpr int kVTile = Lds<HD, CT, NEW>::kVTile;
-  constexpr bool kQLds = Lds<HD, CT, NEW>::kQuery;
+  constexpr int kVTile = Lds<HD, CT, NEW, NB>::kVTile;
+  constexpr bool kQLds = Lds<HD, CT, NEW, NB>::kQuery;
   auto& smem = mem.tiles;
   auto& q_lds = mem.query;
   auto& new_kv = mem.new_kv;
@@ -581,7 +581,7 @@ DEV_INLINE void attend_split(
   }
 }
 
-template <int HD, typename CT, bool CAP, bool ONE, int NEW>
+template <int HD, typename CT, bool CAP, bool ONE, int NEW, int NB>
 __launch_bounds__(kBlockThreads, waves_per_simd(HD)) __global__ void paged_decode_kernel(
     ushort* __restrict__ out, const ushort* __restrict__ q, CT* k_cache, CT* v_cache,
     const int32_t* __restrict__ block_tables, const int32_t* __restrict__ seq_lens,
@@ -589,8 +589,8 @@ __launch_bounds__(kBlockThreads, waves_per_simd(HD)) __global__ void paged_decod
     const int max_blocks, const int64_t q_stride, const int row_splits,
     const Item* __restrict__ plan, const NewRows fresh, float* __restrict__ part_o,
     float* __restrict__ part_ml) {
-  __shared__ Lds<HD, CT, NEW> mem;
-  attend_split<HD, CT, CAP, ONE, NEW>(mem, blockIdx.x, out, q, k_cache, v_cache, block_tables,
+  __shared__ Lds<HD, CT, NEW, NB> mem;
+  attend_split<HD, CT, CAP, ONE, NEW, NB>(mem, blockIdx.x, out, q, k_cache, v_cache, block_tables,
                                       seq_lens, scale, softcap, window, n_kv, G, max_blocks,
                                       q_stride, row_splits, plan, fresh, part_o, part_ml);
 }

@@ -239,31 +239,44 @@ static void attend(torch::Tensor out, const ushort* q, int64_t q_stride, const N
   TORCH_CHECK(parts * n_kv < (int64_t)1 << 31);
   const dim3 grid((uint32_t)(parts * n_kv)), block(kBlockThreads);
   auto stream = c10::hip::getCurrentHIPStream().stream();
-  auto with_new = [&](auto hdv, auto ct, auto cap, auto one, auto fresh_v) {
+  auto with_new = [&](auto hdv, auto ct, auto cap, auto one, auto fresh_v, auto nb) {
     using CT = decltype(ct);
     hipLaunchKernelGGL(
         (paged_decode_kernel<decltype(hdv)::value, CT, decltype(cap)::value,
-                             decltype(one)::value, decltype(fresh_v)::value>),
+                             decltype(one)::value, decltype(fresh_v)::value,
+                             decltype(nb)::value>),
         grid, block, 0, stream, fp8 ? nullptr : (ushort*)out.data_ptr(), q,
         (CT*)k_cache.data_ptr(), (CT*)v_cache.data_ptr(), block_tables.data_ptr<int32_t>(),
         seq_lens.data_ptr<int32_t>(), (float)scale, (float)softcap,
         (int)window, n_kv, G, max_blocks, q_stride, n_splits, items,
         fresh ? *fresh : NewRows{}, part_o_ptr, part_ml_ptr);
   };
+  // No wave has more than one tile (12 rows of 500: 14.9 us with the loop's loads of no
+  // bytes, 13.9 without): of a cache block, or up to twice as many keys of two, which are
+  // faster than a loop of two (111 rows of 29-76 10.1 / 11.4).
+  const int nb = blocks_per_tile(hd, k_cache.element_size());
+  auto fit = [&](int blocks) {
+    return !items && (max_blocks + blocks - 1) / blocks <= n_splits * kWaves;
+  };
+  const bool one = fit(nb), one_of_two = !one && !fresh && hd == 128 && nb == 1 && fit(2);
   auto launch = [&](auto hdv, auto ct, auto cap, auto one) {
+    constexpr int HD = decltype(hdv)::value;
+    const std::integral_constant<int, blocks_per_tile(HD, sizeof(ct))> own{};
     if constexpr (sizeof(ct) == 2) {
       if (fresh && fresh->sums.parts <= 4)
-        return with_new(hdv, ct, cap, one, std::integral_constant<int, 4>{});
-      if (fresh) return with_new(hdv, ct, cap, one, std::integral_constant<int, 8>{});
+        return with_new(hdv, ct, cap, one, std::integral_constant<int, 4>{}, own);
+      if (fresh) return with_new(hdv, ct, cap, one, std::integral_constant<int, 8>{}, own);
     }
-    with_new(hdv, ct, cap, one, std::integral_constant<int, 0>{});
+    const std::integral_constant<int, 0> none{};
+    if constexpr (sizeof(ct) == 2 && HD == 128 && decltype(one)::value) {
+      if (one_of_two)
+        return with_new(hdv, ct, cap, one, none, std::integral_constant<int, 2>{});
+    }
+    with_new(hdv, ct, cap, one, none, own);
   };
-  // (12 rows of 500: 14.9 us with the loop's loads of no bytes, 13.9 without)
-  const int nb = blocks_per_tile(hd, k_cache.element_size());
-  const bool one = !items && (max_blocks + nb - 1) / nb <= n_splits * kWaves;
   auto with_cap = [&](auto hdv, auto ct) {
     auto with_one = [&](auto capped) {
-      if (one) launch(hdv, ct, capped, std::true_type{});
+      if (one || one_of_two) launch(hdv, ct, capped, std::true_type{});
       else launch(hdv, ct, capped, std::false_type{});
     };
     if (softcap > 0.0) with_one(std::true_type{});

@@ -230,3 +230,18 @@ def test_where_rows_are_planned(rows, columns, n_kv, window, alone, planned):
     plan = ops.decode_plan({}, sl, bt, cache, window, alone=alone)
     assert (plan is not None) is planned
     assert ops.decode_plan(None, sl, bt, cache, window, alone=alone) is None
+
+
+@pytest.mark.parametrize("columns", [1, 4, 5, 8, 9])
+@pytest.mark.parametrize("rows,n_kv,window,cap", [(70, 8, 0, 0.0), (3, 2, 0, 20.0), (70, 8, 50, 0.0)])
+def test_one_tile_a_wave(rows, columns, n_kv, window, cap):
+    """Without a plan: tiles of one block, of two where a wave then has one, and a loop."""
+    g = random.Random(columns)
+    lens = [16 * columns - g.randrange(16 * columns) for _ in range(rows)]
+    lens[0] = 16 * columns
+    kc, vc, bt, sl = _caches(lens, n_kv, 128, torch.bfloat16, columns)
+    q = torch.randn(rows, 4 * n_kv, 128, device=DEV).bfloat16()
+    kw = dict(window=window, softcap=cap)
+    got = ops.paged_attention_decode(q, kc, vc, bt, sl, 0.09, **kw)
+    want = ref.paged_attention_decode(q.float(), kc.float(), vc.float(), bt, sl, 0.09, **kw)
+    assert torch.all((got.float() - want).abs() <= 2.0**-8 * want.abs() + 1e-4)
