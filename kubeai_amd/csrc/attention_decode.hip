@@ -253,7 +253,7 @@ static void attend(torch::Tensor out, const ushort* q, int64_t q_stride, const N
   };
   // No wave has more than one tile (12 rows of 500: 14.9 us with the loop's loads of no
   // bytes, 13.9 without): of a cache block, or up to twice as many keys of two, which are
-  // faster than a loop of two (111 rows of 29-76 10.1 / 11.4).
+  // faster than a loop of two (111 rows of 29-76 10.4 / 11.4).
   const int nb = blocks_per_tile(hd, k_cache.element_size());
   auto fit = [&](int blocks) {
     return !items && (max_blocks + blocks - 1) / blocks <= n_splits * kWaves;

@@ -175,10 +175,14 @@ __global__ __launch_bounds__(kSB) void expert_order_kernel(
   };
   constexpr int kBatch = S * kSB;
   int below = 0;
-  for (int i0 = 0; i0 < N; i0 += kBatch) {
-    load(i0);
+  if constexpr (S == 1) {
+    for (int i = threadIdx.x; i < N; i += kSB) below += index[i] < e ? 1 : 0;
+  } else {
+    for (int i0 = 0; i0 < N; i0 += kBatch) {
+      load(i0);
 #pragma unroll
-    for (int s = 0; s < S; ++s) below += mine[s] < e ? 1 : 0;
+      for (int s = 0; s < S; ++s) below += mine[s] < e ? 1 : 0;
+    }
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) below += __shfl_xor(below, off, WAVE);
@@ -193,7 +197,12 @@ __global__ __launch_bounds__(kSB) void expert_order_kernel(
   const int first = total_s;
   int at = first;
   for (int i0 = 0; i0 < N; i0 += kBatch) {
-    if (N > kBatch) load(i0);
+    if constexpr (S == 1) {
+      const int i = i0 + threadIdx.x;
+      mine[0] = i < N ? index[i] : INT32_MAX;
+    } else if (N > kBatch) {
+      load(i0);
+    }
     uint64_t b[S];
 #pragma unroll
     for (int s = 0; s < S; ++s) b[s] = __ballot(mine[s] == e);
