@@ -222,9 +222,14 @@ def paged_attention_decode_fp8(
 
 
 def decode_takes_sums(qkv, n_q: int, cos_sin, k_cache, v_cache) -> bool:
-    """Whether paged_attention_decode_sums takes these."""
+    """Whether paged_attention_decode_sums takes these. Every split of a row adds the row's
+    sums again, so not more than 512 rows, which fill the chip in a rotation of their own
+    (us, that and the attention / one launch: 40/8 heads, 810 rows of 5-75 keys 50.9 / 60.6, 4/1
+    heads 520 of 136-1436 53.9 / 57.7; over 250 steps of up to 512 rows 0.79, 1.03 at
+    most)."""
     return (
         isinstance(qkv, ProductSums)
+        and qkv.part.shape[1] <= 512
         and k_cache.dtype == v_cache.dtype == torch.bfloat16
         and k_cache.shape == v_cache.shape
         and k_cache.shape[2] == 16
