@@ -10,7 +10,8 @@
 //    209 and leave room for two (28 rows of 100-700 in 3 splits 17.9 us, 15.9). The first
 //    look-up in the block table does not wait for the row's length.
 //  - which splits there are, and in which order, is worked out on the device once a
-//    step (attention_decode.hip), by the rows' lengths.
+//    step (attention_decode.hip), by the lengths of all rows: another row's length may
+//    change the order of a row's sums.
 //  - S^T = K.Q^T on v_mfma_f32_16x16x32_bf16: a lane reads 16 bytes of one
 //    key straight into the operand (16 keys x 64 contiguous bytes per load,
 //    no LDS), the query heads are columns (lane & 15; those past G repeat the
@@ -112,7 +113,8 @@ struct NewRows {
 // Cache blocks of a tile.
 constexpr int blocks_per_tile(int hd, int element) { return hd == 128 && element == 1 ? 2 : 1; }
 
-// Waves a SIMD holds: 145 registers at head size 128, 256 at 256.
+// Waves a SIMD holds: at head size 128 145 registers, 156 where the rows are sums still,
+// with a cap 162; at 256 228 to 256, of which the capped bf16 forms spill 1, from sums 5.
 constexpr int waves_per_simd(int hd) { return hd == 128 ? 3 : 2; }
 
 // 16 (or 8) bytes a lane from base + at, zeros if size is 0
@@ -148,16 +150,7 @@ DEV_INLINE float over_groups(float v, F&& f) {
   return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
-// CT = cache element type: ushort (bf16) or unsigned char (fp8 e5m2,
-// converted to bf16 on the way in, exactly). CAP: s = cap * tanh(s / cap)
-// after scaling and before masking. ONE: no wave has more than one tile.
-// NEW: the rows' queries, keys and values are a product's sums still, of up to so many
-// parts. Every workgroup adds and rotates its own query heads and the key, a unit of 8
-// columns a thread, with the first tile's loads on their way behind the sums'; the one
-// that has the row's last tile writes key and value to the cache, and takes them from
-// LDS for that tile. us with the merge, rotation as a
-// launch before / here: 40 rows of 100-700, sums in 4 parts, to fp8 25.0 / 22.2, bf16 23.5 /
-// 21.0; 8 rows, sums in 8 parts 18.2 / 14.8, 14.9 / 11.6.
+// What a workgroup has in LDS (attend_split).
 template <int HD, typename CT, int NEW, int NB = blocks_per_tile(HD, sizeof(CT))>
 struct alignas(16) Lds {
   // Head size 256 over a bf16 cache: two tiles of K and V and the sums leave no
@@ -174,6 +167,17 @@ struct alignas(16) Lds {
   float merge_ml[kWaves][kMaxG][2];
 };
 
+// CT = cache element type: ushort (bf16) or unsigned char (fp8 e5m2,
+// converted to bf16 on the way in, exactly). CAP: s = cap * tanh(s / cap)
+// after scaling and before masking. ONE: no wave has more than one tile. NB: cache blocks
+// of a tile.
+// NEW: the rows' queries, keys and values are a product's sums still, of up to so many
+// parts. Every workgroup adds and rotates its own query heads and the key, a unit of 8
+// columns a thread, with the first tile's loads on their way behind the sums'; the one
+// that has the row's last tile writes key and value to the cache, and takes them from
+// LDS for that tile. us with the merge, rotation as a launch before / here: 40 rows of
+// 100-700, sums in 4 parts, to fp8 25.0 / 22.2, bf16 23.5 / 21.0; 8 rows, sums in 8 parts
+// 18.2 / 14.8, 14.9 / 11.6.
 template <int HD, typename CT, bool CAP, bool ONE, int NEW,
           int NB = blocks_per_tile(HD, sizeof(CT))>
 DEV_INLINE void attend_split(

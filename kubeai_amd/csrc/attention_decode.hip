@@ -21,7 +21,7 @@ namespace {
 // the CUs in turn, so they are ordered largest first, and every second round backwards:
 // each CU's share is about the same, and CUs with a split less than the others get the
 // largest.
-constexpr int kPlanThreads = 256, kCandidates = 32, kPlanRows = 1024;
+constexpr int kCandidates = 32, kPlanThreads = 8 * kCandidates, kPlanRows = 1024;
 constexpr float kSplitCost = 6.f;  // tiles
 constexpr int kLeastTiles = 8;     // that a split is cut to
 
@@ -145,12 +145,13 @@ __global__ void __launch_bounds__(kPlanThreads) decode_plan_kernel(
 // is much longer than the others is worked through by its own splits alone. At
 // head size 256, whose workgroups read a row at half the rate of those at 128,
 // many rows are split once more for that (576). Head size 128: 40 rows of
-// 100-700 keys, 8 kv heads 23.0 us at 512, 25.6 at 1536; one row of 3000 among 7
-// idle ones 13.6 at 512, 17.0 at 1536. Head size 256: 128 rows of 300 but one
-// of 8000, 4 kv heads 224 us at 512, 122 at 576, 87 at 1536; 8 rows of 3500, e5m2
-// cache, 8 kv heads 33 at 512, 42 at 576; 40 rows of 100-700, e5m2 cache, 4 kv
-// heads 19.3 at 512 and 576, 22 at 768, 25 at 1536. (Measured with tiles of 32 keys.) A
-// split has at least 32 keys of the widest row, 16 at head size 256. KUBEAI_DECODE_SPLIT_TARGET overrides for tuning sweeps.
+// 100-700 keys, 8 kv heads 22.4 us at 512, 21.1 at 256, 22.5 at 1536; of 1500-4000 96, 111
+// at 256, 94; one row of 3000 among 7 idle ones 11.3, 14.5 at 256, 10.1; 96 rows of 100-300,
+// 4 kv heads 15.8, 13.2 at 256, 18.9. Head size 256: 128 rows of 300 but one of 8000, 4
+// kv heads 181 at 512, 113 at 576, 90 at 1536; 8 rows of 3500, e5m2 cache, 8 kv heads 31.5
+// at 512, 39 at 576, 36 at 1536; 40 rows of 100-700, e5m2 cache, 4 kv heads 23.8, 24.0 and
+// 27.2. A split has at least 32 keys of the widest row, 16 at head size 256.
+// KUBEAI_DECODE_SPLIT_TARGET overrides it (steps with a plan do not ask).
 int paged_decode_splits(int rows, int n_kv, int hd, int max_blocks) {
   static const int forced = []() {
     const char* e = getenv("KUBEAI_DECODE_SPLIT_TARGET");

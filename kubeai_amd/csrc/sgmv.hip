@@ -24,7 +24,8 @@
 // and a launch each. So the table is searched in registers, one load for all
 // its ids, x, y and the first adapter's B are asked for before v is there, the
 // next adapter's weights while one is multiplied, and no load stands in a branch
-// of its own (each such branch waits for its load).
+// that waits for it (the shrink's loads of x and A are in one each, for inputs past the
+// last, with no wait between them).
 // 4 adapters of rank 16, 28 decode rows and 304 prompt tokens (384 padded), us:
 // shrink 8.5; expand 4096 -> 4096 and 6144 8.0, 14336 -> 4096 into sums 9.9, 4096 ->
 // 28672 with the activation 22.0. With v cut at every product, loads one behind

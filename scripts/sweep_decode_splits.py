@@ -1,6 +1,8 @@
 """Sweep KUBEAI_DECODE_SPLIT_TARGET for the flash-decoding kernel.
 
-The split target is read once per process (static), so run this script
+The target is what steps without a plan of their splits go by (tensor parallel, more
+than 256 rows, few keys); a step that has one (ops.decode_plan) is timed beside it and
+does not depend on the target. It is read once per process (static), so run this script
 once per value:
 
     for t in 192 256 512 1024 2048; do
@@ -47,5 +49,8 @@ for B, L in ((40, 1536), (8, 8192), (256, 2048)):
     us = timeit(lambda: ops.paged_attention_decode(qd, kc, vc, bt, sl, scale))
     kv_bytes = B * L * nkv * hd * 2 * 2
     gbs = kv_bytes / (us * 1e-6) / 1e9
-    print(f"B={B:4d} L={L:5d}  {us:8.1f} us  {gbs:7.0f} GB/s  err={err:.4f}",
-          flush=True)
+    plan = ops.decode_plan({}, sl, bt, kc, alone=True)
+    planned = timeit(
+        lambda: ops.paged_attention_decode(qd, kc, vc, bt, sl, scale, plan=plan))
+    print(f"B={B:4d} L={L:5d}  {us:8.1f} us  {gbs:7.0f} GB/s  err={err:.4f}"
+          f"  planned {planned:8.1f} us", flush=True)
