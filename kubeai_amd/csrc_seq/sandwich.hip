@@ -67,6 +67,9 @@ __global__ __launch_bounds__(kBlock) void sandwich_rmsnorm_rows_kernel(
     const float* __restrict__ post_w, float* __restrict__ residual,
     const float* __restrict__ pre_w, int C, float eps, const int* __restrict__ place,
     int top) {
+  // (a constant: behind this many arguments the launch's own size lies in a cache line of
+  // its own, which both sums waited for: 60 x 2048 in a step 6.6 -> 7.1 us)
+  constexpr int kWaves = kBlock / WAVE;
   __shared__ float red0[16], red1[16];
   const size_t base = (size_t)blockIdx.x * C;
   float x[K], b[K], pw[K], qw[K];
@@ -109,7 +112,7 @@ __global__ __launch_bounds__(kBlock) void sandwich_rmsnorm_rows_kernel(
     float sb = 0.f;
 #pragma unroll
     for (int k = 0; k < K; ++k) sb = fmaf(b[k], b[k], sb);
-    const float rb = 1.0f / sqrtf(block_sum(sb, red0) / (float)C + eps);
+    const float rb = 1.0f / sqrtf(block_sum<kWaves>(sb, red0) / (float)C + eps);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       const int c = k * kBlock + threadIdx.x;
@@ -120,7 +123,7 @@ __global__ __launch_bounds__(kBlock) void sandwich_rmsnorm_rows_kernel(
   float sx = 0.f;
 #pragma unroll
   for (int k = 0; k < K; ++k) sx = fmaf(x[k], x[k], sx);
-  const float rx = 1.0f / sqrtf(block_sum(sx, red1) / (float)C + eps);
+  const float rx = 1.0f / sqrtf(block_sum<kWaves>(sx, red1) / (float)C + eps);
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int c = k * kBlock + threadIdx.x;

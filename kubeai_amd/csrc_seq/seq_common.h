@@ -109,11 +109,12 @@ DEV_INLINE float wave_max(float v) {
   return v;
 }
 
-// Sum over the block (<= 16 waves); every thread gets the total. `smem`
-// holds >= 16 floats and must not be reused before the next barrier.
+// Sum over the block (<= 16 waves; WAVES of them, or 0: as launched); every thread gets
+// the total. `smem` holds >= 16 floats and must not be reused before the next barrier.
+template <int WAVES = 0>
 DEV_INLINE float block_sum(float v, float* smem) {
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  const int n_waves = (blockDim.x + WAVE - 1) / WAVE;
+  const int n_waves = WAVES ? WAVES : (blockDim.x + WAVE - 1) / WAVE;
   v = wave_sum(v);
   if (lane == 0) smem[wave] = v;
   __syncthreads();
