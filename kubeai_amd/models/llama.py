@@ -225,7 +225,9 @@ class Attention(nn.Module):
                 ),
                 as_sums, fb,
             )
-        if fb.n_prefill > 0 and ops.step_attention_takes(q, nd, k_cache, plan):
+        if plan is not None and fb.n_prefill > 0 and ops.step_attention_takes(
+            q, nd, k_cache, plan
+        ):
             out = ops.paged_attention_step(
                 q, nd, k_cache, v_cache, fb.decode_block_tables, fb.decode_seq_lens,
                 fb.prefill_block_tables, fb.prefill_query_start_loc, fb.prefill_seq_lens,
