@@ -701,9 +701,11 @@ __launch_bounds__(16 * WAVE_SIZE) __global__ void decode_merge_fp8_kernel(
   float vals[HPW][EPL];
   float amax = 0.f;
   Splits of{0, 1};
-  // (the same in every lane; waves without a head load nothing: where they loaded the
-  // last one again, 269 rows of 6 heads of 256 and 14-17 keys took 15.4 us, 12.9 so)
-  auto has = [&](int h) { return h * 16 + wave < n_q; };
+  // Waves without a head load nothing (the same in every lane): where they loaded the last
+  // one again, 269 rows of 6 heads of 256 and 14-17 keys took 15.4 us, 13.5 so. A second
+  // head that is not there is the last one again: in a branch its loads wait for the
+  // first one's (40 rows of 32 heads of 128 in a step 4.8 us, 5.5).
+  const bool has = HPW > 1 || wave < n_q;
   auto merge = [&](auto most) {
     constexpr int MOST = decltype(most)::value;
     // A wave's heads are asked for together, but two of 256 columns in 16 splits one
@@ -716,11 +718,11 @@ __launch_bounds__(16 * WAVE_SIZE) __global__ void decode_merge_fp8_kernel(
     for (int h0 = 0; h0 < HPW; h0 += AHEAD) {
 #pragma unroll
       for (int h = 0; h < AHEAD; ++h)
-        if (has(h0 + h))
-          m[h].template load<MOST>(part_o, part_ml, of, n_q, (h0 + h) * 16 + wave);
+        if (has)
+          m[h].template load<MOST>(part_o, part_ml, of, n_q, min((h0 + h) * 16 + wave, n_q - 1));
 #pragma unroll
       for (int h = 0; h < AHEAD; ++h) {
-        if (!has(h0 + h)) continue;
+        if (!has) continue;
         m[h].template finish<MOST>();
 #pragma unroll
         for (int e = 0; e < EPL; ++e) {
@@ -739,13 +741,13 @@ __launch_bounds__(16 * WAVE_SIZE) __global__ void decode_merge_fp8_kernel(
     values from[HPW];
 #pragma unroll
     for (int h = 0; h < HPW; ++h)
-      if (has(h))
+      if (has)
         from[h] = *reinterpret_cast<const values*>(
-            whole + (row * n_q + h * 16 + wave) * HD + EPL * lane);
+            whole + (row * n_q + min(h * 16 + wave, n_q - 1)) * HD + EPL * lane);
 #pragma unroll
     for (int h = 0; h < HPW; ++h)
 #pragma unroll
-      for (int e = 0; has(h) && e < EPL; ++e) {
+      for (int e = 0; has && e < EPL; ++e) {
         vals[h][e] = bf16_to_f32(from[h][e]);
         amax = fmaxf(amax, fabsf(vals[h][e]));
       }
