@@ -114,7 +114,7 @@ struct NewRows {
 constexpr int blocks_per_tile(int hd, int element) { return hd == 128 && element == 1 ? 2 : 1; }
 
 // Waves a SIMD holds: at head size 128 145 registers, 156 where the rows are sums still,
-// with a cap 162; at 256 228 to 256, of which the capped bf16 forms spill 1, from sums 5.
+// with a cap 162; at 256 223 to 256, of which the capped bf16 forms spill 1, from sums 5.
 constexpr int waves_per_simd(int hd) { return hd == 128 ? 3 : 2; }
 
 // 16 (or 8) bytes a lane from base + at, zeros if size is 0

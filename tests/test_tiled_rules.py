@@ -167,3 +167,22 @@ def test_no_rule_keeps_the_sizes_of_a_trace():
     before = ops.tiled_sums_better.cache_info().currsize
     torch.jit.trace(Reader(), torch.randn(128, 14336), check_trace=False)
     assert ops.tiled_sums_better.cache_info().currsize == before
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,taken", [(8, True), (40, True), (64, True), (128, False)])
+def test_no_rule_keeps_them_with_operands_that_tiles_take(rows, taken):
+    class Reader(torch.nn.Module):
+        def forward(self, x):
+            ops.sums_for_reader(x, w)
+            return x + 1
+
+    w = torch.randn(2304, 9216, device="cuda").bfloat16()
+    x = torch.randn(rows, 9216, device="cuda").bfloat16()
+    rules = (ops.narrow_better, ops.tiled_sums_better)
+    ops.sums_for_reader(x, w)
+    before = [rule.cache_info().currsize for rule in rules]
+    for _ in range(2):
+        torch.jit.trace(Reader(), x, check_trace=False)
+    assert [rule.cache_info().currsize for rule in rules] == before
+    assert ops.narrow_better(rows, 2304, 9216, False) is taken
